@@ -14,7 +14,7 @@ FB_MASK_NONE, FB_MASK_VECTOR, FB_MASK_MATRIX = 0, 1, 2
 
 #: every symbol that include/flashbias.h declares
 EXPORTS = ("fb_version", "fb_init", "fb_last_error", "fb_bwd_workspace_bytes", "fb_suggest_bias_grad_group", "fb_check", "fb_fwd", "fb_bwd",
-           "fb_sum_over_batch", "fb_resize_rank",
+           "fb_sum_over_batch", "fb_resize_rank", "fb_alibi_factors", "fb_cosine_workspace_bytes", "fb_cosine_fwd", "fb_cosine_bwd",
            "fb_bwd_preprocess", "fb_bwd_dkv", "fb_bwd_dq", "fb_bwd_static")
 
 
@@ -31,7 +31,7 @@ class FbParams(ctypes.Structure):
                 + [(n, FbTensor) for n in ("q", "k", "v", "q_bias", "k_bias", "mask", "o")]
                 + [("lse", ctypes.c_void_p)]
                 + [(n, FbTensor) for n in ("dout", "dq", "dk", "dv", "dq_bias", "dk_bias")]
-                + [("delta", ctypes.c_void_p), ("bias_grad_group", ctypes.c_int32)])
+                + [("delta", ctypes.c_void_p), ("bias_grad_group", ctypes.c_int32), ("mask_batches", ctypes.c_int32)])
 
 
 class FlashBiasError(RuntimeError):

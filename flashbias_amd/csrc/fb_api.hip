@@ -25,6 +25,10 @@ hipError_t launch_bwd_both_general_f16_2(const BwdArgs &a, hipStream_t stream);
 hipError_t launch_bwd_win_bf16_2(const BwdArgs &a, hipStream_t stream);
 hipError_t launch_bwd_win_f16_2(const BwdArgs &a, hipStream_t stream);
 
+// elementwise part of a cosine-attention window block (fb_cosine.hip)
+hipError_t launch_cosine(const fb_cosine *p, bool backward, hipStream_t stream);
+int64_t cosine_sweep(int64_t tokens, int H, int d);
+
 hipError_t launch_fwd(const FwdArgs &a, bool bf16, hipStream_t stream) {
     switch (nkd_of(a.d)) {
     case 1: return bf16 ? launch_fwd_bf16_1(a, stream) : launch_fwd_f16_1(a, stream);
@@ -118,6 +122,7 @@ fb::MaskDesc dev_mask(const fb_params *p) {
     m.ptr = p->mask_type ? p->mask.ptr : nullptr;
     m.sb = p->mask.stride_b;
     m.sh = p->mask.stride_h;
+    m.batches = p->mask_batches;
     m.sm = p->mask_type == FB_MASK_MATRIX ? p->mask.stride_s : 0;
     m.type = p->mask_type;
     m.is_f32 = p->mask_dtype == FB_F32;
@@ -237,6 +242,58 @@ int fb_resize_rank(const void *in, void *out, int64_t rows, int r_in, int r_out,
     if (rows <= 0 || r_in <= 0 || r_out <= 0 || r_in > 4096 || r_out > 4096 || (rows + 255) / 256 > 0x7fffffff)
         return fb::api_fail(FB_ERR_SHAPE, "fb_resize_rank: rows and both ranks must be positive (ranks up to 4096, rows below 2^39)");
     return launched(fb::launch_resize_rank(in, out, rows, r_in, r_out, static_cast<hipStream_t>(stream)), "fb_resize_rank");
+}
+
+int fb_alibi_factors(void *q_bias, void *k_bias, int dtype, int Lq, int Lk, int H, int r, int reference_sign, void *stream) {
+    fb::api_clear_error();
+    if (!q_bias || !k_bias) return fb::api_fail(FB_ERR_NULL, "fb_alibi_factors: null pointer");
+    if (dtype != FB_F16 && dtype != FB_BF16) return fb::api_fail(FB_ERR_DTYPE, "only fp16 and bf16 are supported");
+    if (Lq <= 0 || Lk <= 0 || Lq > 65536 || Lk > 65536 || H <= 0 || H > (1 << 20) || r < 8 || r > FB_MAX_RANK || r % 8 != 0)
+        return fb::api_fail(FB_ERR_SHAPE, "fb_alibi_factors: up to 65536 positions, a rank of 8, 16, ... 128");
+    if (reinterpret_cast<uintptr_t>(q_bias) % 16 != 0 || reinterpret_cast<uintptr_t>(k_bias) % 16 != 0)
+        return fb::api_fail(FB_ERR_STRIDE, "fb_alibi_factors: factors must be 16-byte aligned");
+    return launched(fb::launch_alibi_factors(q_bias, k_bias, dtype == FB_BF16, Lq, Lk, H, r, reference_sign != 0, static_cast<hipStream_t>(stream)),
+                    "fb_alibi_factors");
+}
+
+static int check_cosine(const fb_cosine *p, bool backward) {
+    fb::api_clear_error();
+    if (!p) return fb::api_fail(FB_ERR_NULL, "fb_cosine: null pointer");
+    if (p->size != sizeof(fb_cosine)) return fb::api_fail(FB_ERR_ABI, "fb_cosine.size does not match this library");
+    if (p->dtype != FB_F16 && p->dtype != FB_BF16) return fb::api_fail(FB_ERR_DTYPE, "only fp16 and bf16 are supported");
+    if (p->in_dtype < FB_F16 || p->in_dtype > FB_F32 || p->scale_dtype < FB_F16 || p->scale_dtype > FB_F32)
+        return fb::api_fail(FB_ERR_DTYPE, "qkv and logit_scale must be fp16, bf16 or fp32");
+    if (p->tokens <= 0 || p->H <= 0 || p->H > (1 << 20) || p->d < 8 || p->d > FB_MAX_HEADDIM || (p->d & (p->d - 1)))
+        return fb::api_fail(FB_ERR_SHAPE, "fb_cosine: tokens and H must be positive, d one of 8, 16, 32, 64, 128");
+    const void *need[] = {p->qkv, p->logit_scale, backward ? p->dq : p->q, backward ? p->dk : p->k, backward ? p->dqkv : p->q};
+    for (const void *x : need)
+        if (!x) return fb::api_fail(FB_ERR_NULL, "fb_cosine: null pointer");
+    const void *rows[] = {p->qkv, p->q, p->k, p->v, p->dq, p->dk, p->dv, p->dqkv};
+    for (const void *x : rows)
+        if (reinterpret_cast<uintptr_t>(x) % 16 != 0) return fb::api_fail(FB_ERR_STRIDE, "fb_cosine: tensors must be 16-byte aligned");
+    if (backward) {
+        if (!p->dlogit_scale || !p->partial) return fb::api_fail(FB_ERR_NULL, "fb_cosine: null pointer");
+        if (p->grad_stride < (int64_t)p->H * p->d || p->grad_stride % 8 != 0)
+            return fb::api_fail(FB_ERR_STRIDE, "fb_cosine: grad_stride must be a multiple of 8 and at least H d");
+    }
+    return FB_OK;
+}
+
+size_t fb_cosine_workspace_bytes(const fb_cosine *p) {
+    if (!p || p->tokens <= 0 || p->H <= 0 || p->d < 8) return 0;
+    return (size_t)fb::cosine_sweep(p->tokens, p->H, p->d) * p->H * sizeof(float);
+}
+
+int fb_cosine_fwd(const fb_cosine *p, void *stream) {
+    const int rc = check_cosine(p, false);
+    if (rc) return rc;
+    return launched(fb::launch_cosine(p, false, static_cast<hipStream_t>(stream)), "fb_cosine_fwd");
+}
+
+int fb_cosine_bwd(const fb_cosine *p, void *stream) {
+    const int rc = check_cosine(p, true);
+    if (rc) return rc;
+    return launched(fb::launch_cosine(p, true, static_cast<hipStream_t>(stream)), "fb_cosine_bwd");
 }
 
 int fb_bwd_static(const fb_params *p, void *stream) {

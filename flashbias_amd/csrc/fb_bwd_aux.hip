@@ -203,6 +203,34 @@ hipError_t launch_resize_rank(const void *in, void *out, int64_t rows, int r_in,
     return hipGetLastError();
 }
 
+// Exact ALiBi factors (include/flashbias.h): one thread per (position, head) row of either factor, the queries' rows
+// first.  The slope in double precision: its value rounded to fp32 and then to the dtype is that of the host's pow.
+template <class T>
+__global__ __launch_bounds__(256) void alibi_factors_kernel(uint16_t *q_bias, uint16_t *k_bias, int64_t rows_q, int64_t rows, int H,
+                                                            int r, float sign) {
+    const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (row >= rows) return;
+    const bool is_k = row >= rows_q;
+    const int64_t at = is_k ? row - rows_q : row;
+    const int pos = (int)(at / H), h = (int)(at % H);
+    const float m = T::to_float(T::from_float((float)exp2(-8.0 * (h + 1) / H)));
+    const float a = (float)(pos >> 8), b = (float)(pos & 255);
+    uint16_t *dst = (is_k ? k_bias : q_bias) + at * r;
+    u32x4_t first = {0u, 0u, 0u, 0u};
+    first[0] = is_k ? T::pack2(-sign * 256.f * m, -sign * m) : T::pack2(a, b);
+    first[1] = is_k ? T::pack2(sign * a, sign * b) : T::pack2(256.f * m, m);
+    *reinterpret_cast<u32x4_t *>(dst) = first;
+    for (int c = 8; c < r; c += 8) *reinterpret_cast<u32x4_t *>(dst + c) = u32x4_t{0u, 0u, 0u, 0u};
+}
+
+hipError_t launch_alibi_factors(void *q_bias, void *k_bias, bool bf16, int Lq, int Lk, int H, int r, bool reference_sign, hipStream_t stream) {
+    const int64_t rows_q = (int64_t)Lq * H, rows = rows_q + (int64_t)Lk * H;
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(bf16 ? alibi_factors_kernel<BF16> : alibi_factors_kernel<F16>, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, stream,
+                       static_cast<uint16_t *>(q_bias), static_cast<uint16_t *>(k_bias), rows_q, rows, H, r, reference_sign ? -1.f : 1.f);
+    return hipGetLastError();
+}
+
 hipError_t launch_bwd_preprocess(const BwdArgs &a, bool bf16, hipStream_t stream) {
     (void)hipGetLastError(); // (an earlier, unrelated error of the process is not this launch's)
     if (bf16)

@@ -350,7 +350,7 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
     const uint8_t *mbase = nullptr;
     if constexpr (C::MASK)
         mbase = reinterpret_cast<const uint8_t *>(a.mask.ptr) +
-                (b * a.mask.sb + h * a.mask.sh) * (a.mask.is_f32 ? 4 : 2);
+                mask_offset(a.mask, b, h) * (a.mask.is_f32 ? 4 : 2);
 
     const float to_log2 = C::FOLD ? a.scale * kLog2e : kLog2e; // the scores are in units of 1 / scale when folded
 

@@ -268,7 +268,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
     const uint8_t *mbase = nullptr;
     if constexpr (C::MASK)
         mbase = reinterpret_cast<const uint8_t *>(a.mask.ptr) +
-                (b * a.mask.sb + h * a.mask.sh) * (a.mask.is_f32 ? 4 : 2);
+                mask_offset(a.mask, b, h) * (a.mask.is_f32 ? 4 : 2);
 
     // ---- query-side operands, resident in registers
     u32x4_t qr[C::QBLK][C::NKD];

@@ -112,6 +112,7 @@ int fb_check(const fb_params *p, int pass) {
         if (p->mask_dtype != p->dtype && p->mask_dtype != FB_F32)
             return fail(FB_ERR_MASK, "mask must have the input dtype or fp32");
         if (!p->mask.ptr) return fail(FB_ERR_NULL, "%s: null pointer", "mask");
+        if (p->mask_batches < 0) return fail(FB_ERR_MASK, "mask_batches must not be negative");
         if (p->mask.stride_b < 0 || p->mask.stride_h < 0 || p->mask.stride_s < 0)
             return fail(FB_ERR_STRIDE, "%s: negative stride", "mask");
     }

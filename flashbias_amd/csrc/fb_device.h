@@ -84,7 +84,13 @@ struct MaskDesc {
     int type;   // 0 none, 1 vector, 2 matrix
     int is_f32; // else same 16-bit type as the inputs
     int vec_ok; // base and strides allow aligned loads of four consecutive keys
+    int batches; // > 0: batch entry b takes the mask of entry b % batches
 };
+
+// Element offset of the mask of one (batch, head).
+__device__ __forceinline__ int64_t mask_offset(const MaskDesc &m, int b, int h) {
+    return (m.batches > 0 ? b % m.batches : b) * m.sb + h * m.sh;
+}
 
 // Eight consecutive channels [col0, col0 + 8) of row `row` of a (rows x ncols) matrix with row
 // stride `ld`; zero beyond ncols and for row >= nrows.  Branch-free: out-of-range lanes read a

@@ -267,7 +267,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs &a) {
     const uint8_t *mbase = nullptr;
     if constexpr (C::MASK)
         mbase = reinterpret_cast<const uint8_t *>(a.mask.ptr) +
-                (b * a.mask.sb + h * a.mask.sh) * (a.mask.is_f32 ? 4 : 2);
+                mask_offset(a.mask, b, h) * (a.mask.is_f32 ? 4 : 2);
 
     // ---- query operands, resident in registers for the whole key loop
     u32x4_t qr[C::QB][C::NKD], qbr[C::QB][C::NKR > 0 ? C::NKR : 1];

@@ -52,6 +52,9 @@ hipError_t launch_sum_over_batch(const void *full, void *out, bool bf16, bool ou
 // out[row][c] = c < min(r_in, r_out) ? in[row][c] : 0: contiguous rows of 16-bit elements.
 hipError_t launch_resize_rank(const void *in, void *out, int64_t rows, int r_in, int r_out, hipStream_t stream);
 
+// The exact rank-4 ALiBi factors, zero-padded to r columns (include/flashbias.h).
+hipError_t launch_alibi_factors(void *q_bias, void *k_bias, bool bf16, int Lq, int Lk, int H, int r, bool reference_sign, hipStream_t stream);
+
 // Compute units of the current device (cached per device; 256 on MI355X).  The launchers pick
 // smaller query tiles when the larger ones would leave compute units without a workgroup.
 inline int num_cus() {

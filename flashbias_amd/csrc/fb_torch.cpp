@@ -11,6 +11,7 @@
 // or none; additive mask (B|1, H|1, 1|Lq, Lk) or none.
 #include <torch/extension.h>
 
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
@@ -38,10 +39,34 @@ int dtype_code(c10::ScalarType t) {
 
 void check(int status) { TORCH_CHECK(status == FB_OK, "flashbias status ", status, ": ", fb_last_error()); }
 
-// The parameter block shared by forward and backward.  `keep` receives the expanded views whose
-// data the block points at.
-fb_params block(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &qb, const Tensor &kb, const Tensor &mask,
-                bool causal, double scale, tensor_list &keep) {
+// A contiguous tensor straight from the caching allocator: a backward makes six of them, and the dispatcher's way
+// to the same call takes a microsecond longer each.
+Tensor fresh(at::IntArrayRef sizes, c10::ScalarType type, c10::Device device) {
+    return Tensor(at::detail::empty_cuda(sizes, type, device, c10::nullopt));
+}
+Tensor fresh_like(const Tensor &x) { return x.is_contiguous() ? fresh(x.sizes(), x.scalar_type(), x.device()) : torch::empty_like(x); }
+
+// The stride of a dimension that may be 1 where `n` is wanted (broadcast: stride 0).
+int64_t broadcast_stride(const Tensor &x, int dim, int64_t n, const char *what) {
+    if (x.size(dim) == n) return x.stride(dim);
+    TORCH_CHECK(x.size(dim) == 1, what, ": dimension ", dim, " must be 1 or ", n, ", got ", x.size(dim));
+    return 0;
+}
+fb_tensor factor(const Tensor &x, int64_t B, int64_t L, int64_t H, const char *what) {
+    return fb_tensor{x.data_ptr(), broadcast_stride(x, 0, B, what), broadcast_stride(x, 2, H, what), broadcast_stride(x, 1, L, what)};
+}
+
+// What one call of the operator is given.  `mask_batches`: the mask's batch entries where they repeat (else 0).
+struct Call {
+    Tensor q, k, v, qb, kb, mask;
+    bool causal;
+    double scale;
+    int mask_batches;
+};
+
+// The parameter block shared by forward and backward.
+fb_params block(const Call &c) {
+    const Tensor &q = c.q, &k = c.k, &v = c.v, &qb = c.qb, &kb = c.kb, &mask = c.mask;
     TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4, "q, k, v must be (batch, seqlen, nheads, headdim)");
     const int64_t B = q.size(0), Lq = q.size(1), H = q.size(2), d = q.size(3), Lk = k.size(1);
     TORCH_CHECK(k.size(0) == B && k.size(2) == H && k.size(3) == d && v.sizes() == k.sizes(), "k, v must be (batch, seqlen_k, nheads, headdim)");
@@ -54,21 +79,17 @@ fb_params block(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor 
     p.size = sizeof(p);
     p.dtype = dtype_code(q.scalar_type());
     p.B = (int32_t)B; p.H = (int32_t)H; p.Lq = (int32_t)Lq; p.Lk = (int32_t)Lk; p.d = (int32_t)d;
-    p.causal = causal ? 1 : 0;
-    p.scale = (float)scale;
+    p.causal = c.causal ? 1 : 0;
+    p.scale = (float)c.scale;
     p.q = t4(q); p.k = t4(k); p.v = t4(v);
     if (qb.defined()) {
         TORCH_CHECK(kb.defined() && qb.scalar_type() == q.scalar_type() && kb.scalar_type() == q.scalar_type() && qb.is_cuda() &&
                         kb.is_cuda() && qb.dim() == 4 && kb.dim() == 4 && qb.size(3) == kb.size(3),
                     "q_bias, k_bias must be GPU tensors of the input dtype and one rank");
-        const int64_t r = qb.size(3);
+        p.r = (int32_t)qb.size(3);
         // stride-0 broadcast over batch / heads (flash_bias_triton.py:1135-1136)
-        const Tensor qe = qb.expand({B, Lq, H, r}), ke = kb.expand({B, Lk, H, r});
-        p.r = (int32_t)r;
-        p.q_bias = t4(qe);
-        p.k_bias = t4(ke);
-        keep.push_back(qe);
-        keep.push_back(ke);
+        p.q_bias = factor(qb, B, Lq, H, "q_bias");
+        p.k_bias = factor(kb, B, Lk, H, "k_bias");
     }
     if (mask.defined()) {
         TORCH_CHECK(mask.dim() == 4 && mask.is_cuda() && (mask.scalar_type() == q.scalar_type() || mask.scalar_type() == torch::kFloat32),
@@ -79,13 +100,15 @@ fb_params block(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor 
             p.mask_type = FB_MASK_MATRIX;
         else
             TORCH_CHECK(false, "Last 2 dimensions of mask must be (1, seqlen_k) or (seqlen_q, seqlen_k)");
-        const Tensor me = mask.expand({B, H, Lq, Lk});
-        p.mask = fb_tensor{me.data_ptr(), me.stride(0), me.stride(1), me.stride(2)};
+        p.mask = fb_tensor{mask.data_ptr(), c.mask_batches ? mask.stride(0) : broadcast_stride(mask, 0, B, "mask"),
+                           broadcast_stride(mask, 1, H, "mask"), mask.size(2) == Lq ? mask.stride(2) : 0};
         p.mask_dtype = dtype_code(mask.scalar_type());
-        keep.push_back(me);
+        p.mask_batches = c.mask_batches;
     }
     return p;
 }
+
+hipStream_t stream_of(const Tensor &x) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.device().index()).stream(); }
 
 // The gradient of `ref` from the full (B, L, H, r) gradient the kernels wrote: summed over the dims in
 // which `ref` was broadcast, in fp32 (over the batch by the library's streaming kernel).
@@ -111,30 +134,64 @@ Tensor reduce_like(Tensor full, const Tensor &ref, hipStream_t stream) {
     return full.is_contiguous() ? full : full.contiguous();
 }
 
+// o and lse of a call.
+std::pair<Tensor, Tensor> attend(const Call &c) {
+    fb_params p = block(c);
+    Tensor o = fresh_like(c.q);
+    Tensor lse = fresh({p.B, p.H, p.Lq}, torch::kFloat32, c.q.device());
+    p.o = t4(o);
+    p.lse = lse.data_ptr<float>();
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(c.q.device()); // (torch on ROCm presents its devices as "cuda")
+    check(fb_fwd(&p, stream_of(c.q)));
+    return {o, lse};
+}
+
+// dq, dk, dv into the tensors given (any strides with contiguous channels); returns the factors' gradients,
+// undefined where nobody asks for them (constant factors; the library then skips them).
+std::pair<Tensor, Tensor> attend_backward(const Call &c, const Tensor &o, const Tensor &lse, const Tensor &dout_in, const Tensor &dq,
+                                          const Tensor &dk, const Tensor &dv, bool factor_grads) {
+    const Tensor dout = channel_contiguous(dout_in);
+    fb_params p = block(c);
+    p.o = t4(o);
+    p.lse = lse.data_ptr<float>();
+    p.dout = t4(dout);
+    p.dq = t4(dq); p.dk = t4(dk); p.dv = t4(dv);
+    Tensor dqb_full, dkb_full;
+    factor_grads = factor_grads && p.r;
+    // factors shared by a large batch of short sequences: a workgroup walks `group` batch entries (it then loads
+    // the factor operand it keeps once), sums their factor gradients itself, and the full-shape tensors shrink by
+    // that factor
+    // (only for factors saved with a batch of one: a factor expanded over the batch by its caller also has batch
+    // stride 0, but autograd wants its gradient in the expanded shape)
+    const bool shared = p.r && c.qb.size(0) == 1 && c.kb.size(0) == 1 && p.B > 1;
+    const int group = p.bias_grad_group = p.r ? (shared ? fb_suggest_bias_grad_group(&p) : 1) : 0;
+    if (factor_grads) {
+        const int64_t rows = ((int64_t)p.B + group - 1) / group;
+        dqb_full = fresh({rows, p.Lq, p.H, p.r}, c.q.scalar_type(), c.q.device());
+        dkb_full = fresh({rows, p.Lk, p.H, p.r}, c.q.scalar_type(), c.q.device());
+        p.dq_bias = t4(dqb_full);
+        p.dk_bias = t4(dkb_full);
+    }
+    // scratch of the backward, sized by the library
+    Tensor scratch = fresh({(int64_t)(fb_bwd_workspace_bytes(&p) / 4)}, torch::kFloat32, c.q.device());
+    p.delta = scratch.data_ptr<float>();
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(c.q.device());
+    const hipStream_t stream = stream_of(c.q);
+    check(fb_bwd(&p, stream));
+    if (!factor_grads) return {Tensor(), Tensor()};
+    return {reduce_like(dqb_full, c.qb, stream), reduce_like(dkb_full, c.kb, stream)};
+}
+
+double scale_or_default(double softmax_scale, const Tensor &q) { return softmax_scale != 0.0 ? softmax_scale : 1.0 / std::sqrt((double)q.size(3)); }
+
+Tensor given(const c10::optional<Tensor> &x) { return x.has_value() && x->defined() ? channel_contiguous(*x) : Tensor(); }
+
 struct FlashBiasFn : public torch::autograd::Function<FlashBiasFn> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &q_in, const Tensor &k_in, const Tensor &v_in,
-                          const c10::optional<Tensor> &qb_in, const c10::optional<Tensor> &kb_in,
-                          const c10::optional<Tensor> &mask_in, bool causal, double softmax_scale) {
-        const Tensor q = channel_contiguous(q_in), k = channel_contiguous(k_in), v = channel_contiguous(v_in);
-        Tensor qb, kb, mask;
-        if (qb_in.has_value() && qb_in->defined()) {
-            TORCH_CHECK(kb_in.has_value() && kb_in->defined(), "q_bias without k_bias");
-            qb = channel_contiguous(*qb_in);
-            kb = channel_contiguous(*kb_in);
-        }
-        if (mask_in.has_value() && mask_in->defined()) mask = channel_contiguous(*mask_in);
-        const double scale = softmax_scale != 0.0 ? softmax_scale : 1.0 / std::sqrt((double)q.size(3));
-        tensor_list keep;
-        fb_params p = block(q, k, v, qb, kb, mask, causal, scale, keep);
-        Tensor o = torch::empty_like(q);
-        Tensor lse = torch::empty({q.size(0), q.size(2), q.size(1)}, q.options().dtype(torch::kFloat32));
-        p.o = t4(o);
-        p.lse = lse.data_ptr<float>();
-        {
-            const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device()); // (torch on ROCm presents its devices as "cuda")
-            check(fb_fwd(&p, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.device().index()).stream()));
-        }
-        ctx->save_for_backward({q, k, v, o, lse, qb, kb, mask});
+    static Tensor forward(AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &qb,
+                          const c10::optional<Tensor> &kb, const c10::optional<Tensor> &mask, bool causal, double scale) {
+        const Call c{q, k, v, qb.value_or(Tensor()), kb.value_or(Tensor()), mask.value_or(Tensor()), causal, scale, 0};
+        const auto [o, lse] = attend(c);
+        ctx->save_for_backward({q, k, v, o, lse, c.qb, c.kb, c.mask});
         ctx->saved_data["causal"] = causal;
         ctx->saved_data["scale"] = scale;
         return o;
@@ -142,55 +199,134 @@ struct FlashBiasFn : public torch::autograd::Function<FlashBiasFn> {
 
     static tensor_list backward(AutogradContext *ctx, tensor_list grads) {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &o = saved[3], &lse = saved[4];
-        const Tensor &qb = saved[5], &kb = saved[6], &mask = saved[7];
+        const Call c{saved[0], saved[1], saved[2], saved[5], saved[6], saved[7], ctx->saved_data["causal"].toBool(), ctx->saved_data["scale"].toDouble(), 0};
         // as the reference, only a backward that is asked for the mask's gradient fails (flash_bias_triton.py:1371).
         // (The graph edges count the tensor arguments that were given: q, k, v, then the factors, then the mask.)
-        if (mask.defined())
-            TORCH_CHECK(!ctx->needs_input_grad(qb.defined() ? 5 : 3), "FlashBias does not support mask gradient yet");
-        const bool causal = ctx->saved_data["causal"].toBool();
-        const double scale = ctx->saved_data["scale"].toDouble();
-        const Tensor dout = channel_contiguous(grads[0]);
-        tensor_list keep;
-        fb_params p = block(q, k, v, qb, kb, mask, causal, scale, keep);
-        Tensor dq = torch::empty_like(q), dk = torch::empty_like(k), dv = torch::empty_like(v);
-        p.o = t4(o);
-        p.lse = lse.data_ptr<float>();
-        p.dout = t4(dout);
-        p.dq = t4(dq); p.dk = t4(dk); p.dv = t4(dv);
-        Tensor dqb_full, dkb_full;
-        // (neither factor asks for its gradient: constant factors; the library then skips them)
-        const bool factor_grads = p.r && (ctx->needs_input_grad(3) || ctx->needs_input_grad(4));
-        // factors shared by a large batch of short sequences: a workgroup walks `group` batch entries (it then loads
-        // the factor operand it keeps once), sums their factor gradients itself, and the full-shape tensors shrink by
-        // that factor
-        // (only for factors saved with a batch of one: a factor expanded over the batch by its caller also has batch
-        // stride 0, but autograd wants its gradient in the expanded shape)
-        const bool shared = p.r && qb.size(0) == 1 && kb.size(0) == 1 && p.B > 1;
-        const int group = p.bias_grad_group = p.r ? (shared ? fb_suggest_bias_grad_group(&p) : 1) : 0;
-        if (factor_grads) {
-            const int64_t rows = ((int64_t)p.B + group - 1) / group;
-            dqb_full = torch::empty({rows, p.Lq, p.H, p.r}, q.options());
-            dkb_full = torch::empty({rows, p.Lk, p.H, p.r}, q.options());
-            p.dq_bias = t4(dqb_full);
-            p.dk_bias = t4(dkb_full);
-        }
-        // scratch of the backward, sized by the library
-        Tensor scratch = torch::empty({(int64_t)(fb_bwd_workspace_bytes(&p) / 4)}, q.options().dtype(torch::kFloat32));
-        p.delta = scratch.data_ptr<float>();
-        Tensor dqb, dkb;
-        {
-            const c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device()); // (torch on ROCm presents its devices as "cuda")
-            const hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.device().index()).stream();
-            check(fb_bwd(&p, stream));
-            if (factor_grads) {
-                dqb = reduce_like(dqb_full, qb, stream);
-                dkb = reduce_like(dkb_full, kb, stream);
-            }
-        }
+        if (c.mask.defined())
+            TORCH_CHECK(!ctx->needs_input_grad(c.qb.defined() ? 5 : 3), "FlashBias does not support mask gradient yet");
+        const Tensor dq = fresh_like(c.q), dk = fresh_like(c.k), dv = fresh_like(c.v);
+        const bool factor_grads = c.qb.defined() && (ctx->needs_input_grad(3) || ctx->needs_input_grad(4));
+        const auto [dqb, dkb] = attend_backward(c, saved[3], saved[4], grads[0], dq, dk, dv, factor_grads);
         return {dq, dk, dv, dqb, dkb, Tensor(), Tensor(), Tensor()};
     }
 };
+
+// The attention core of a cosine-attention window block on its packed projection qkv (windows, n, 3 H d): unit q and
+// k and the logit scale in one pass (fb_cosine_fwd), the operator on them and on v where it lies, and backward the
+// operator's gradients written into the packed gradient, where one more pass (fb_cosine_bwd) turns dq and dk into
+// those of the projection.  (As tensor operations: about 40 passes over tensors of that size, and the split of the
+// packed tensor comes back as three zero-filled copies added up.)  `mask` (nW, n, n) or none, one per window of an image.
+struct WindowFn : public torch::autograd::Function<WindowFn> {
+    static fb_cosine cosine(const Tensor &qkv, const Tensor &logit_scale, int64_t heads, c10::ScalarType type) {
+        fb_cosine a;
+        std::memset(&a, 0, sizeof(a));
+        a.size = sizeof(a);
+        a.dtype = dtype_code(type);
+        a.in_dtype = dtype_code(qkv.scalar_type());
+        a.scale_dtype = dtype_code(logit_scale.scalar_type());
+        a.H = (int32_t)heads;
+        a.d = (int32_t)(qkv.size(2) / (3 * heads));
+        a.tokens = qkv.size(0) * qkv.size(1);
+        a.qkv = qkv.data_ptr();
+        a.logit_scale = logit_scale.data_ptr();
+        return a;
+    }
+    // part `which` of a packed tensor, as (windows, n, H, d)
+    static Tensor part(const Tensor &packed, int64_t which, int64_t heads) {
+        const int64_t B = packed.size(0), n = packed.size(1), dim = packed.size(2) / 3;
+        return packed.as_strided({B, n, heads, dim / heads}, {n * 3 * dim, 3 * dim, dim / heads, 1}, packed.storage_offset() + which * dim);
+    }
+
+    static Tensor forward(AutogradContext *ctx, const Tensor &qkv, const Tensor &logit_scale, const Tensor &qb, const Tensor &kb,
+                          const c10::optional<Tensor> &mask_in, int64_t heads, int64_t dtype) {
+        const auto type = (c10::ScalarType)dtype;
+        TORCH_CHECK(qkv.dim() == 3 && qkv.is_contiguous() && qkv.is_cuda() && qkv.size(2) % (3 * heads) == 0 && logit_scale.is_contiguous() &&
+                        logit_scale.is_cuda() && logit_scale.numel() == heads,
+                    "qkv must be a contiguous (windows, n, 3 * heads * headdim) GPU tensor, logit_scale one value per head");
+        const int64_t B = qkv.size(0), n = qkv.size(1), d = qkv.size(2) / (3 * heads);
+        fb_cosine a = cosine(qkv, logit_scale, heads, type);
+        Call c;
+        c.q = fresh({B, n, heads, d}, type, qkv.device());
+        c.k = fresh({B, n, heads, d}, type, qkv.device());
+        const bool convert = qkv.scalar_type() != type;
+        c.v = convert ? fresh({B, n, heads, d}, type, qkv.device()) : part(qkv, 2, heads);
+        c.qb = qb;
+        c.kb = kb;
+        c.causal = false;
+        c.scale = 1.0;
+        c.mask_batches = 0;
+        if (mask_in.has_value() && mask_in->defined()) {
+            c.mask = channel_contiguous(*mask_in).unsqueeze(1);
+            TORCH_CHECK(c.mask.dim() == 4 && c.mask.size(0) > 0 && B % c.mask.size(0) == 0, "the windows must be a multiple of the mask's");
+            c.mask_batches = (int)c.mask.size(0);
+        }
+        a.q = c.q.data_ptr();
+        a.k = c.k.data_ptr();
+        a.v = convert ? c.v.data_ptr() : nullptr;
+        {
+            const c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
+            check(fb_cosine_fwd(&a, stream_of(qkv)));
+        }
+        const auto [o, lse] = attend(c);
+        ctx->save_for_backward({qkv, logit_scale, c.q, c.k, convert ? c.v : Tensor(), o, lse, qb, kb, c.mask});
+        ctx->saved_data["heads"] = heads;
+        return o;
+    }
+
+    static tensor_list backward(AutogradContext *ctx, tensor_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &qkv = saved[0], &logit_scale = saved[1];
+        const int64_t heads = ctx->saved_data["heads"].toInt();
+        const bool convert = saved[4].defined();
+        Call c{saved[2], saved[3], convert ? saved[4] : part(qkv, 2, heads), saved[7], saved[8], saved[9], false, 1.0, 0};
+        if (c.mask.defined()) c.mask_batches = (int)c.mask.size(0);
+        TORCH_CHECK(!(c.mask.defined() && ctx->needs_input_grad(4)), "FlashBias does not support mask gradient yet");
+        Tensor dqkv = fresh_like(qkv);
+        Tensor dq, dk, dv;
+        if (convert) {
+            dq = fresh_like(c.q);
+            dk = fresh_like(c.k);
+            dv = fresh_like(c.v);
+        } else {
+            dq = part(dqkv, 0, heads);
+            dk = part(dqkv, 1, heads);
+            dv = part(dqkv, 2, heads);
+        }
+        const auto [dqb, dkb] = attend_backward(c, saved[5], saved[6], grads[0], dq, dk, dv, ctx->needs_input_grad(2) || ctx->needs_input_grad(3));
+        fb_cosine a = cosine(qkv, logit_scale, heads, c.q.scalar_type());
+        Tensor dscale = fresh_like(logit_scale);
+        Tensor partial = fresh({(int64_t)(fb_cosine_workspace_bytes(&a) / 4)}, torch::kFloat32, qkv.device());
+        a.dq = dq.data_ptr();
+        a.dk = dk.data_ptr();
+        a.dv = convert ? dv.data_ptr() : nullptr;
+        a.grad_stride = dq.stride(1);
+        a.dqkv = dqkv.data_ptr();
+        a.dlogit_scale = dscale.data_ptr();
+        a.partial = partial.data_ptr<float>();
+        {
+            const c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
+            check(fb_cosine_bwd(&a, stream_of(qkv)));
+        }
+        return {dqkv, dscale, dqb, dkb, Tensor(), Tensor(), Tensor()};
+    }
+};
+
+Tensor window_attention(const Tensor &qkv, const Tensor &logit_scale, const Tensor &qb, const Tensor &kb, const c10::optional<Tensor> &mask,
+                        int64_t heads, py::object dtype) {
+    return WindowFn::apply(qkv, logit_scale, channel_contiguous(qb), channel_contiguous(kb), mask, heads,
+                           (int64_t)torch::python::detail::py_object_to_dtype(dtype));
+}
+
+// (q_bias, k_bias) of fb_alibi_factors, (1, L, H, rank) in the 16-bit dtype of `like`'s device.
+std::pair<Tensor, Tensor> alibi_factors(int64_t Lq, int64_t Lk, int64_t heads, int64_t rank, bool reference_sign, py::object dtype, py::object device) {
+    const auto type = torch::python::detail::py_object_to_dtype(dtype);
+    const auto where = torch::python::detail::py_object_to_device(device);
+    Tensor qb = torch::empty({1, Lq, heads, rank}, torch::TensorOptions().dtype(type).device(where));
+    Tensor kb = torch::empty({1, Lk, heads, rank}, torch::TensorOptions().dtype(type).device(where));
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(qb.device());
+    check(fb_alibi_factors(qb.data_ptr(), kb.data_ptr(), dtype_code(type), (int)Lq, (int)Lk, (int)heads, (int)rank, reference_sign, stream_of(qb)));
+    return {qb, kb};
+}
 
 // x (..., r) with its last dim zero-padded (or cut) to `rank` columns in one launch of the library; the gradient
 // is the same operation the other way.  For contiguous 16-bit GPU tensors (the caller checks).
@@ -215,9 +351,33 @@ struct ResizeRankFn : public torch::autograd::Function<ResizeRankFn> {
 
 Tensor resize_rank(const Tensor &x, int64_t rank) { return ResizeRankFn::apply(x, rank); }
 
-Tensor flash_bias(const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &q_bias,
+Tensor flash_bias(const Tensor &q_in, const Tensor &k_in, const Tensor &v_in, const c10::optional<Tensor> &q_bias,
                   const c10::optional<Tensor> &k_bias, const c10::optional<Tensor> &mask, bool causal, double softmax_scale) {
-    return FlashBiasFn::apply(q, k, v, q_bias, k_bias, mask, causal, softmax_scale);
+    const Tensor q = channel_contiguous(q_in), k = channel_contiguous(k_in), v = channel_contiguous(v_in);
+    const Tensor qb = given(q_bias), kb = given(k_bias), m = given(mask);
+    TORCH_CHECK(!qb.defined() || kb.defined(), "q_bias without k_bias");
+    const double scale = scale_or_default(softmax_scale, q);
+    auto wants = [](const Tensor &x) { return x.defined() && x.requires_grad(); };
+    // nothing to differentiate: no graph node either
+    if (!c10::GradMode::is_enabled() || !(wants(q) || wants(k) || wants(v) || wants(qb) || wants(kb) || wants(m)))
+        return attend(Call{q, k, v, qb, kb, m, causal, scale, 0}).first;
+    auto maybe = [](const Tensor &x) { return x.defined() ? c10::optional<Tensor>(x) : c10::nullopt; };
+    return FlashBiasFn::apply(q, k, v, maybe(qb), maybe(kb), maybe(m), causal, scale);
+}
+
+// The operator on arguments that need no preparation and break no rule, else nothing: the caller then takes its own
+// way through the checks (which say what is wrong) and the preparations.
+c10::optional<Tensor> flash_bias_ready(const Tensor &q, const Tensor &k, const Tensor &v, const c10::optional<Tensor> &q_bias,
+                                       const c10::optional<Tensor> &k_bias, const c10::optional<Tensor> &mask, bool causal,
+                                       c10::optional<double> softmax_scale) {
+    const auto type = q.scalar_type();
+    const bool ready = q.dim() == 4 && k.dim() == 4 && q.is_cuda() && k.is_cuda() && v.is_cuda() && (type == torch::kFloat16 || type == torch::kBFloat16) &&
+                       k.scalar_type() == type && v.scalar_type() == type && k.size(0) == q.size(0) && k.size(2) == q.size(2) &&
+                       k.size(3) == q.size(3) && v.sizes() == k.sizes() && q.size(3) <= FB_MAX_HEADDIM &&
+                       !(q_bias.has_value() && (q_bias->dim() != 4 || q_bias->size(3) % 8 != 0)) &&
+                       !(mask.has_value() && mask->dim() == 4 && mask->size(2) == 1);
+    if (!ready) return c10::nullopt;
+    return flash_bias(q, k, v, q_bias, k_bias, mask, causal, softmax_scale.value_or(0.0));
 }
 
 } // namespace
@@ -226,6 +386,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "flash_bias_func with its autograd function in C++ (kernel-ready inputs; see flashbias_amd/interface.py)";
     // what this module was compiled against: the caller compares both with the library it loaded
     m.def("abi", []() { return std::make_pair((int)FB_VERSION, (int)sizeof(fb_params)); });
+    m.def("flash_bias_ready", &flash_bias_ready, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("q_bias"), py::arg("k_bias"), py::arg("mask"),
+          py::arg("causal"), py::arg("softmax_scale"));
+    m.def("window_attention", &window_attention, py::arg("qkv"), py::arg("logit_scale"), py::arg("q_bias"), py::arg("k_bias"), py::arg("mask"),
+          py::arg("heads"), py::arg("dtype"));
+    m.def("alibi_factors", &alibi_factors, py::arg("seqlen_q"), py::arg("seqlen_k"), py::arg("heads"), py::arg("rank"), py::arg("reference_sign"),
+          py::arg("dtype"), py::arg("device"));
     m.def("resize_rank", &resize_rank, py::arg("x"), py::arg("rank"));
     m.def("flash_bias", &flash_bias, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("q_bias") = py::none(),
           py::arg("k_bias") = py::none(), py::arg("mask") = py::none(), py::arg("causal") = false,

@@ -7,7 +7,7 @@ initialised (no checkpoints ship with either repository)."""
 import torch
 import torch.nn as nn
 
-from . import factors
+from . import factors, interface
 from .interface import flash_bias_func
 
 
@@ -36,8 +36,13 @@ class AttentionWithALiBiBias(nn.Module):
         b, n, _ = x.shape
         split = lambda t: t.view(b, n, self.heads, self.dim_head).to(self.dtype)
         q, k, v = split(self.to_q(x)), split(self.to_k(x)), split(self.to_v(x))
-        q_bias, k_bias = factors.alibi_factors(n, n, self.heads, self.dtype, x.device, exact=True,
-                                               reference_sign=self.reference_sign)
+        ext = interface._extension()
+        if ext is not None and x.is_cuda and n <= 65536:
+            # the same factors in one launch, with the zero columns the operator would append on every call
+            q_bias, k_bias = ext.alibi_factors(n, n, self.heads, 16, self.reference_sign, self.dtype, x.device)
+        else:
+            q_bias, k_bias = factors.alibi_factors(n, n, self.heads, self.dtype, x.device, exact=True,
+                                                   reference_sign=self.reference_sign)
         o = flash_bias_func(q, k, v, q_bias, k_bias, None, True, self.scale)
         return self.to_out(o.reshape(b, n, -1).to(x.dtype))
 
@@ -64,7 +69,15 @@ class WindowAttentionCore(nn.Module):
 
     def forward(self, x, mask=None):
         b_, n, c = x.shape
-        qkv = self.qkv(x).view(b_, n, 3, self.heads, c // self.heads)
+        qkv = self.qkv(x)
+        ext = interface._extension()
+        if ext is not None and qkv.is_cuda and qkv.is_contiguous() and c // self.heads in (8, 16, 32, 64, 128) and self.q_bias_pos.shape[-1] % 8 == 0 \
+                and self.q_bias_pos.dtype == self.dtype:
+            # normalisation, attention and the packed projection's gradient without passes in between (csrc/fb_torch.cpp)
+            o = ext.window_attention(qkv, self.logit_scale, self.q_bias_pos, self.k_bias_pos,
+                                     None if mask is None else mask.to(self.dtype), self.heads, self.dtype)
+            return self.proj(o.reshape(b_, n, c).to(x.dtype))
+        qkv = qkv.view(b_, n, 3, self.heads, c // self.heads)
         q, k, v = qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2]
         scale = torch.clamp(self.logit_scale, max=4.6052).exp().view(1, 1, self.heads, 1)
         q = (torch.nn.functional.normalize(q, dim=-1) * scale).to(self.dtype)

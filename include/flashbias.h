@@ -98,6 +98,9 @@ typedef struct fb_params {
                                    once; the caller reduces the remaining rows.  (The reference accumulates the factor
                                    gradients with atomic adds into fp32 buffers laid out like the factors
                                    themselves, flash_bias_triton.py:1219-1231, :1342.) */
+    int32_t mask_batches;       /* 0: the mask has B batch entries, or one (stride_b = 0).  n > 0: it has n, and batch
+                                   entry b takes b % n: the masks of a shifted-window block, one per window of an image,
+                                   which the reference repeats over the images (swin_transformer_v2.py:190-203) */
 } fb_params;
 
 /* Library / ABI version. */
@@ -186,6 +189,13 @@ int fb_sum_over_batch(const void *full, void *out, int dtype, int out_dtype, int
  * of two of at least 16, with masked loads: flash_bias_triton.py:1137, :195-200). */
 int fb_resize_rank(const void *in, void *out, int64_t rows, int r_in, int r_out, void *stream);
 
+/* The exact ALiBi bias -m_h (i - j) as factors of rank 4, zero-padded to `r` columns (positions below 65536 in two
+ * 8-bit digits, i = 256 a + b, so that every column is a whole number or a slope in 16 bits):
+ *     q_bias[i] = [a_i, b_i, 256 m, m, 0 ...],   k_bias[j] = [-256 m, -m, a_j, b_j, 0 ...],
+ * both (L, H, r) contiguous and 16-byte aligned, r a multiple of 8, m_h = 2^(-8 (h + 1) / H) rounded to the dtype;
+ * reference_sign: +m_h (i - j), what the reference's module builds (attention_with_alibi_bias.py:44-52).  One launch. */
+int fb_alibi_factors(void *q_bias, void *k_bias, int dtype, int Lq, int Lk, int H, int r, int reference_sign, void *stream);
+
 /* The backward in three phases, exported so that a harness can time them separately (call them in
  * this order: the two main kernels read what the preprocess wrote).
  *   fb_bwd_preprocess: delta = rowsum(o * dout)       (_bwd_preprocess_do_o_dot, :358-400); fills the
@@ -200,6 +210,32 @@ int fb_resize_rank(const void *in, void *out, int64_t rows, int r_in, int r_out,
 int fb_bwd_preprocess(const fb_params *p, void *stream);
 int fb_bwd_dkv(const fb_params *p, void *stream);
 int fb_bwd_dq(const fb_params *p, void *stream);
+
+/* The elementwise part of a cosine-attention window block around the operator
+ * (swin_transformer_v2.py:155-207: normalize(q) * exp(min(logit_scale, 4.6052)), normalize(k)), one pass over the
+ * packed projection in each direction.  qkv and dqkv are (tokens, 3, H, d), contiguous and 16-byte aligned;
+ * d is 8, 16, 32, 64 or 128. */
+typedef struct fb_cosine {
+    uint32_t size;        /* sizeof(fb_cosine) as seen by the caller */
+    int32_t dtype;        /* FB_F16 or FB_BF16: q, k, v and their gradients */
+    int32_t in_dtype;     /* fb_dtype of qkv and dqkv */
+    int32_t scale_dtype;  /* fb_dtype of logit_scale and its gradient */
+    int32_t H, d;
+    int64_t tokens;
+    const void *qkv;         /* in */
+    const void *logit_scale; /* in, (H) */
+    void *q, *k, *v;         /* fwd out, (tokens, H, d) contiguous; v NULL: not wanted (it can be read from qkv in place) */
+    const void *dq, *dk, *dv; /* bwd in, rows of H d elements; dv NULL: already in dqkv */
+    int64_t grad_stride;     /* elements from one token's dq (dk, dv) to the next's.  dq and dk may lie where the
+                                gradient of their part of dqkv goes (then in_dtype = dtype, grad_stride = 3 H d) */
+    void *dqkv;              /* bwd out */
+    void *dlogit_scale;      /* bwd out, (H) */
+    float *partial;          /* bwd scratch of fb_cosine_workspace_bytes() bytes */
+} fb_cosine;
+
+size_t fb_cosine_workspace_bytes(const fb_cosine *p);
+int fb_cosine_fwd(const fb_cosine *p, void *stream);
+int fb_cosine_bwd(const fb_cosine *p, void *stream);
 
 #ifdef __cplusplus
 }
