@@ -331,9 +331,13 @@ def flash_bias_func(q, k, v, q_bias=None, k_bias=None, mask=None, causal=False, 
     else the Python FlashBiasFunc above.  The rare preparations (a large vector mask folded into the
     factors, a rank padded to a multiple of 8) are ordinary differentiable tensor operations here,
     so their gradients come from autograd."""
-    ext = _extension()
+    ext = _ext or _extension()
     if ext is None:
         return FlashBiasFunc.apply(q, k, v, q_bias, k_bias, mask, causal, softmax_scale)
+    # (kernel-ready arguments, which is most calls: one call into the extension, nothing else in Python)
+    o = ext.flash_bias_ready(q, k, v, q_bias, k_bias, mask, bool(causal), softmax_scale)
+    if o is not None:
+        return o
     # the launcher's assertions (:1100-1143), as assertions
     assert q.dim() == 4 and k.dim() == 4 and k.shape[0] == q.shape[0] and k.shape[2:] == q.shape[2:] and v.shape == k.shape
     assert q.shape[-1] <= 128, "FlashBias only supports head dimensions up to 128"
