@@ -34,15 +34,19 @@ namespace fb {
 // (the launcher says when that is exact).
 // BG_: also accumulate dk_bias (false: the caller does not want the factor gradients; the accumulator blocks that
 // hold nothing but dk_bias are then left out).
-template <class T, int NKD_, int NKR_, int NDV_, bool VEC_, bool MASK_, int PART_ = 0, bool FOLD_ = false, bool BG_ = true>
+template <class T, int NKD_, int NKR_, int NDV_, bool VEC_, int MASK_, int PART_ = 0, bool FOLD_ = false, bool BG_ = true>
 struct DkvCfg {
     static constexpr bool FOLD = FOLD_;
-    static_assert(!FOLD_ || (VEC_ && !MASK_), "folded scale: direct loader, no additive mask");
+    static constexpr bool VEC = VEC_;
+    // A vector mask is one value per key here, that is per lane: a single register that the FMA of the scale adds.
+    // Its instantiations (VMASK) are the unmasked ones otherwise; XMASK is every other masked one.
+    static constexpr bool MASK = MASK_ != kNoMask, VMASK = MASK_ == kVectorMask, XMASK = MASK_ == kMatrixMask;
+    static_assert(!VMASK || VEC_, "");
+    static_assert(!FOLD_ || (VEC_ && !MASK), "folded scale: direct loader, no additive mask");
     // folded scale with r <= 8: the Q_b columns 8..15 of a step hold a second copy of q_b, the
     // partner of the low parts of k_b / scale in the key operand
     static __device__ __forceinline__ bool low_parts(const BwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
     static constexpr int NKD = NKD_, NKR = NKR_, NDV = NDV_;
-    static constexpr bool VEC = VEC_, MASK = MASK_;
     static constexpr bool DO_DV = PART_ <= 1, DO_DK = PART_ != 1;
     static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES;
     static constexpr int NK = NKD + NKR;
@@ -60,13 +64,13 @@ struct DkvCfg {
     static constexpr int ROWCHO = 2 * NKD <= 8 ? 8 : 16;
     static constexpr int SQ = BMQ * ROWCH * 8, SDO = BMQ * ROWCHO * 8;
     // masked, aligned instantiations also stage the step's 64 x 128 tile of a 16-bit matrix mask
-    static constexpr bool MTILE = VEC_ && MASK_;
+    static constexpr bool MTILE = VEC_ && XMASK;
     static constexpr int MROWCH = BN / 8; // chunks per mask-tile row
     static constexpr int SM = MTILE ? BMQ * BN : 0;
     static constexpr int STAGE_ELEMS = SQ + SDO + 4 * BMQ + SM; // + lse * log2(e), -delta as fp32
     // direct loader: three stages, two steps ahead; with a mask tile (or the element-wise loader) two
     // stages, one step ahead
-    static constexpr int AHEAD = (VEC_ && !MASK_) ? 2 : 1;
+    static constexpr int AHEAD = (VEC_ && !XMASK) ? 2 : 1;
     static constexpr int NSTAGE = AHEAD + 1;
     static constexpr int LDS_BYTES = NSTAGE * STAGE_ELEMS * 2;
     // loader tasks: 8-channel chunks of Q, Q_b and dout, one query row each
@@ -75,10 +79,10 @@ struct DkvCfg {
     static constexpr int PT = (TASKS + NTHREADS - 1) / NTHREADS;
     // one wave per SIMD (512 registers) where two would spill: large head dims in one pass, and
     // masked instantiations beyond the smallest (they also hold a step's mask values)
-    static constexpr bool BIG = MASK_ && PART_ == 0 && (NDV_ >= 2 || NKD_ + NKR_ >= 5);
+    static constexpr bool BIG = XMASK && PART_ == 0 && (NDV_ >= 2 || NKD_ + NKR_ >= 5);
     // (aligned, unmasked, at most four operand steps, head dim <= 32: 164-168 registers, and the third wave is worth
     // more than the few that the allocator would otherwise take beyond 168)
-    static constexpr int WAVES_EU = BIG ? 1 : (VEC_ && !MASK_ && PART_ == 0 && NK <= 4 && NDV == 1) ? 3 : ((NK <= 8 && NDV <= 2) || PART_ != 0) ? 2 : 1;
+    static constexpr int WAVES_EU = BIG ? 1 : (VEC_ && !XMASK && PART_ == 0 && NK <= 4 && NDV == 1) ? 3 : ((NK <= 8 && NDV <= 2) || PART_ != 0) ? 2 : 1;
 };
 
 template <class C>
@@ -390,6 +394,15 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
         }
     }
 
+    float mkey[C::KBW]; // vector mask: the value of this lane's keys
+    if constexpr (C::VMASK) {
+#pragma unroll
+        for (int kb = 0; kb < C::KBW; ++kb) {
+            const int key = min(wk0 + kb * 32 + c, a.Lk - 1);
+            mkey[kb] = a.mask.is_f32 ? reinterpret_cast<const float *>(mbase)[key] : T::to_float(reinterpret_cast<const uint16_t *>(mbase)[key]);
+        }
+    }
+
     // causal: the first query step that can see this key tile (:498)
     const int step0 = a.causal ? n0 / C::BMQ : 0;
     const int nsteps = (a.Lq + C::BMQ - 1) / C::BMQ;
@@ -426,8 +439,8 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
 
     // Additive mask: the values of a step (16 per lane and 32 x 32 block) are requested one step
     // ahead and added by the FMA that applies the softmax scale.
-    f32x16_t mk[C::MASK ? C::QBLK : 1][C::MASK ? C::KBW : 1], mkn[C::MASK ? C::QBLK : 1][C::MASK ? C::KBW : 1];
-    auto load_mask = [&](f32x16_t (&dst)[C::MASK ? C::QBLK : 1][C::MASK ? C::KBW : 1], int m0) {
+    f32x16_t mk[C::XMASK ? C::QBLK : 1][C::XMASK ? C::KBW : 1], mkn[C::XMASK ? C::QBLK : 1][C::XMASK ? C::KBW : 1];
+    auto load_mask = [&](f32x16_t (&dst)[C::XMASK ? C::QBLK : 1][C::XMASK ? C::KBW : 1], int m0) {
 #pragma unroll
         for (int qb = 0; qb < C::QBLK; ++qb)
 #pragma unroll
@@ -435,7 +448,7 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
                 mask_block_queries<T>(a.mask, mbase, m0 + qb * 32, g, wk0 + kb * 32 + c, a.Lq, a.Lk, dst[qb][kb]);
     };
     const bool mtile = C::MTILE && direct.mtile; // else the mask values travel through registers
-    if constexpr (C::MASK) {
+    if constexpr (C::XMASK) {
         if (step0 < nsteps && !mtile) load_mask(mk, step0 * C::BMQ);
     }
 
@@ -444,7 +457,7 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
         const int m0 = step * C::BMQ;
         const bool more = step + 1 < nsteps;
         const int nxt = cur == C::NSTAGE - 1 ? 0 : cur + 1;
-        if constexpr (C::MASK) {
+        if constexpr (C::XMASK) {
             if (more && !mtile) load_mask(mkn, m0 + C::BMQ);
         }
         if constexpr (C::VEC) {
@@ -498,7 +511,7 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
 #pragma unroll
                     for (int t = 0; t < (C::DO_DK ? C::NKD : 0); ++t) dp = T::mfma(da[t], vreg[kb][t], dp);
                     f32x16_t mval; // additive mask of this block, added by the FMA that applies the scale
-                    if constexpr (C::MASK) {
+                    if constexpr (C::XMASK) {
                         if (mtile) { // column `key`, rows in C-layout order: four transposing reads
                             if constexpr (C::MTILE) {
                                 const int col = (wave * C::KBW + kb) * 32 + 16 * (c >> 4) + 4 * (c & 3);
@@ -513,7 +526,7 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
                                 }
                             }
                         } else {
-                            mval = mk[C::MASK ? qb : 0][C::MASK ? kb : 0];
+                            mval = mk[C::XMASK ? qb : 0][C::XMASK ? kb : 0];
                         }
                     }
                     // the softmax scale multiplies the fp32 q k^T accumulator before the bias steps
@@ -521,7 +534,7 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
                     if constexpr (!C::FOLD) {
 #pragma unroll
                         for (int v = 0; v < 16; ++v)
-                            s[v] = C::MASK ? __builtin_fmaf(s[v], a.scale, mval[v]) : s[v] * a.scale;
+                            s[v] = C::XMASK ? __builtin_fmaf(s[v], a.scale, mval[v]) : C::VMASK ? __builtin_fmaf(s[v], a.scale, mkey[kb]) : s[v] * a.scale;
                     }
 #pragma unroll
                     for (int t = C::NKD; t < C::NK; ++t) s = T::mfma(qa[t], kreg[kb][t], s);
@@ -577,7 +590,7 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
             __syncthreads();
         }
         cur = nxt;
-        if constexpr (C::MASK) {
+        if constexpr (C::XMASK) {
 #pragma unroll
             for (int qb = 0; qb < C::QBLK; ++qb)
 #pragma unroll
@@ -604,7 +617,7 @@ bwd_dkv_kernel(const BwdArgs a) {
     bwd_dkv_body<T, C>(a, blockIdx.x);
 }
 
-template <class T, int NKD, int NKR, int NDV, bool VEC, bool MASK, int PART, bool FOLD, bool BG = true>
+template <class T, int NKD, int NKR, int NDV, bool VEC, int MASK, int PART, bool FOLD, bool BG = true>
 static hipError_t launch_dkv_part(const BwdArgs &a0, hipStream_t stream) {
     typedef DkvCfg<T, NKD, NKR, NDV, VEC, MASK, PART, FOLD, BG> C;
     BwdArgs a = a0;
@@ -619,16 +632,16 @@ static hipError_t launch_dkv_part(const BwdArgs &a0, hipStream_t stream) {
 
 // One pass, or (head dims above 64, aligned tensors) two or three passes that each keep a part
 // of the accumulators.
-template <class T, int NKD, int NKR, int NDV, bool VEC, bool MASK, bool FOLD = false>
+template <class T, int NKD, int NKR, int NDV, bool VEC, int MASK, bool FOLD = false>
 static hipError_t launch_dkv_vec(const BwdArgs &a, hipStream_t stream) {
     if constexpr (NKD > 4 && VEC) {
-        if constexpr (NKR <= 2 && !MASK) {
+        if constexpr (NKR <= 2 && MASK != kMatrixMask) {
             // two passes, dv and then all of [dk | dk_bias]: 44 MFMAs per 32 x 32 block (three passes: 61;
             // dv with the lower half of dk, then the upper half: 52, measured 15-24 % slower than this)
             const hipError_t e = launch_dkv_part<T, NKD, NKR, NDV, VEC, MASK, 1, FOLD>(a, stream);
             if (e != hipSuccess) return e;
             return launch_dkv_part<T, NKD, NKR, NDV, VEC, MASK, 2, FOLD>(a, stream);
-        } else { // larger ranks and masked calls: all of dk would spill at 256 registers
+        } else { // larger ranks and matrix masks: all of dk would spill at 256 registers
             hipError_t e = launch_dkv_part<T, NKD, NKR, NDV, VEC, MASK, 1, FOLD>(a, stream);
             if (e != hipSuccess) return e;
             e = launch_dkv_part<T, NKD, NKR, NDV, VEC, MASK, 3, FOLD>(a, stream);
@@ -655,9 +668,10 @@ static hipError_t launch_dkv_cfg(const BwdArgs &a, hipStream_t stream) {
     const bool vec = a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.dout.vec_ok && a.d % 8 == 0 &&
                      (a.r == 0 || (a.qb.vec_ok && a.kb.vec_ok && a.r % 8 == 0)) && a.q.ss < lim && a.dout.ss < lim &&
                      (a.r == 0 || a.qb.ss < lim);
+    if (vec && a.mask.type == kVectorMask) return launch_dkv_vec<T, NKD, NKR, NDV, true, kVectorMask>(a, stream);
     if (a.mask.type)
-        return vec ? launch_dkv_vec<T, NKD, NKR, NDV, true, true>(a, stream)
-                   : launch_dkv_vec<T, NKD, NKR, NDV, false, true>(a, stream);
+        return vec ? launch_dkv_vec<T, NKD, NKR, NDV, true, kMatrixMask>(a, stream)
+                   : launch_dkv_vec<T, NKD, NKR, NDV, false, kMatrixMask>(a, stream);
     if constexpr (NKD == 2 && NKR <= 1 && NDV == 1) {
         // the streamlined kernel: same 128-key workgroups as the general one, and ahead of it at every
         // grid size (measured at B2 H4: 0.019 against 0.023 ms at L=1024, 0.063 against 0.082 at 4096,
@@ -670,10 +684,10 @@ static hipError_t launch_dkv_cfg(const BwdArgs &a, hipStream_t stream) {
         }
     }
     if constexpr (NKR <= 2) {
-        if (vec && fold_scale_ok<T>(a.scale, a.r, a.Lq)) return launch_dkv_vec<T, NKD, NKR, NDV, true, false, true>(a, stream);
+        if (vec && fold_scale_ok<T>(a.scale, a.r, a.Lq)) return launch_dkv_vec<T, NKD, NKR, NDV, true, kNoMask, true>(a, stream);
     }
-    return vec ? launch_dkv_vec<T, NKD, NKR, NDV, true, false>(a, stream)
-               : launch_dkv_vec<T, NKD, NKR, NDV, false, false>(a, stream);
+    return vec ? launch_dkv_vec<T, NKD, NKR, NDV, true, kNoMask>(a, stream)
+               : launch_dkv_vec<T, NKD, NKR, NDV, false, kNoMask>(a, stream);
 }
 
 template <class T, int NKD, int NDV>

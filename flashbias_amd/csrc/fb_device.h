@@ -87,6 +87,10 @@ struct MaskDesc {
     int batches; // > 0: batch entry b takes the mask of entry b % batches
 };
 
+// Instantiations of the forward and dk/dv kernels by mask (kMatrixMask also takes a vector mask where there is no instantiation
+// of its own); the values are those of MaskDesc::type.
+constexpr int kNoMask = 0, kVectorMask = 1, kMatrixMask = 2;
+
 // Element offset of the mask of one (batch, head).
 __device__ __forceinline__ int64_t mask_offset(const MaskDesc &m, int b, int h) {
     return (m.batches > 0 ? b % m.batches : b) * m.sb + h * m.sh;

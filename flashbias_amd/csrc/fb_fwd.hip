@@ -32,20 +32,27 @@
 namespace fb {
 
 // VEC: every streamed tensor is 16-byte aligned (base and strides) and d, r are multiples of 8.
+// MASK_: kNoMask, kMatrixMask (any additive mask) or kVectorMask (aligned tensors; one value per key).
 // QB2_: allow two query blocks per wave (the launcher turns it off for small grids).
 // FOLD_: the scores are scale * (q k^T + (q_b / scale) k_b^T), one MFMA chain and no FMA per
 // score for the scale (see the launcher for when that is exact).
-template <class T, int NKD_, int NKR_, int NDV_, bool VEC_, bool MASK_, bool QB2_ = true, bool FOLD_ = false>
+template <class T, int NKD_, int NKR_, int NDV_, bool VEC_, int MASK_, bool QB2_ = true, bool FOLD_ = false>
 struct FwdCfg {
     static constexpr int NKD = NKD_, NKR = NKR_, NDV = NDV_;
-    static constexpr bool VEC = VEC_, MASK = MASK_, FOLD = FOLD_;
-    static_assert(!FOLD_ || !MASK_, "the additive mask is not divided by the scale");
+    static constexpr bool VEC = VEC_, MASK = MASK_ != kNoMask, FOLD = FOLD_;
+    // a vector mask travels as one fp32 value per key in the stage of its tile: its 16 values of a block come from
+    // LDS straight into the accumulator of the bias chain and cost no conversion and no register of their own, so
+    // these instantiations are the unmasked ones otherwise (the staged 128 x 64 tile that a matrix mask needs held
+    // 64 copies of the same row)
+    static constexpr bool VMASK = MASK_ == kVectorMask, XMASK = MASK_ == kMatrixMask;
+    static_assert(!FOLD_ || !MASK, "the additive mask is not divided by the scale");
+    static_assert(!VMASK || VEC_, "");
     static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES;
     // query blocks (of 32) per wave: two where the registers allow (head dim <= 32, rank <= 32:
     // 219-247 registers at four operand steps), so that every key / value fragment read from LDS
     // feeds two blocks and two waves per SIMD carry four softmax streams (768 x 4 rows of 768
     // tokens at rank 32: 0.77 -> 0.64 ms)
-    static constexpr int QB = (QB2_ && NKD_ + NKR_ <= 4 && NDV_ == 1 && VEC_ && !MASK_) ? 2 : 1;
+    static constexpr int QB = (QB2_ && NKD_ + NKR_ <= 4 && NDV_ == 1 && VEC_ && !XMASK) ? 2 : 1;
     static constexpr int BM = NWAVES * 32 * QB;
     static constexpr int NK = NKD + NKR;
     // A wave computes KBLK * 32 keys at a time; an LDS tile (one barrier) holds SUBS such groups.
@@ -53,7 +60,7 @@ struct FwdCfg {
     // two groups per tile where three workgroups of that size still fit the 160 KB of a CU
     static constexpr int LDS2 = 2 * 2 * (2 * BSUB * (16 * NK + 8) + 32 * NDV_ * (2 * BSUB + 8));
     // (masked, aligned instantiations also stage a BM x BN mask tile: one group per tile)
-    static constexpr bool MTILE = VEC_ && MASK_;
+    static constexpr bool MTILE = VEC_ && XMASK;
     static constexpr int SUBS = (!MTILE && NK <= 4 && NDV_ <= 2 && 3 * LDS2 <= 160 * 1024) ? 2 : 1;
     static constexpr int BN = BSUB * SUBS;
     static constexpr int DKP = 16 * NK + 8; // LDS row of [K | K_b], elements (16 B of padding)
@@ -61,7 +68,8 @@ struct FwdCfg {
     static constexpr int BNP = BN + 8; // LDS row of V^T
     static constexpr int SK_ELEMS = BN * DKP, SV_ELEMS = DV * BNP;
     static constexpr int MROWCH = BN / 8;                    // 16-byte chunks per mask-tile row
-    static constexpr int SM_ELEMS = MTILE ? BM * BN : 0;      // 16-bit matrix mask tile, swizzled chunks
+    // 16-bit matrix mask tile, swizzled chunks; or the tile's fp32 vector mask
+    static constexpr int SM_ELEMS = MTILE ? BM * BN : VMASK ? 2 * BN : 0;
     static constexpr int LDS_BYTES = 2 * (SK_ELEMS + SV_ELEMS + SM_ELEMS) * 2;
     // cooperative loader: 8-channel chunks of K and K_b (one key row each), (4 keys x 4
     // channels) blocks of V.  Consecutive threads take the consecutive chunks of one row, then the
@@ -78,7 +86,7 @@ struct FwdCfg {
     // with head dims up to 64: 158-166; the attribute is a cap the hardware honours, so a kernel that
     // would fit three waves runs two unless it says three), one (512 registers) where the
     // mask values or an unaligned head dim of 128 would spill at 256, else two
-    static constexpr bool BIG = (MASK_ && (NDV_ >= 2 || NKD_ + NKR_ >= 5)) || (!VEC_ && NDV_ == 4) ||
+    static constexpr bool BIG = (XMASK && (NDV_ >= 2 || NKD_ + NKR_ >= 5)) || (!VEC_ && NDV_ == 4) ||
                                 2 * LDS_BYTES > 160 * 1024; // (one workgroup per CU anyway)
     static constexpr int WAVES_EU = QB == 2 ? 2 : BIG ? 1 : (NK <= 6 && NDV <= 2) ? 3 : 2;
     // LDS fragments requested ahead of their use: all key steps of a group when they are few,
@@ -327,15 +335,29 @@ __device__ __forceinline__ void fwd_body(const FwdArgs &a) {
     bool mtile = false;
     if constexpr (C::MTILE) {
         static_assert(C::QB == 1, "one query block per wave in masked instantiations");
-        if (a.mask.vec_ok && !a.mask.is_f32 && a.Lk % 8 == 0 && a.mask.sm % 8 == 0 && // (a vector mask: row stride 0)
+        if (a.mask.vec_ok && !a.mask.is_f32 && a.Lk % 8 == 0 && a.mask.sm % 8 == 0 &&
             a.mask.sm < (1 << 24) && reinterpret_cast<uintptr_t>(mbase) % 16 == 0) {
             mtile = true;
             mdma.init(reinterpret_cast<const uint16_t *>(mbase), a.mask.sm, C::BN, C::MROWCH, nullptr, 0, 0, wave, lane, m0);
             if (C::BN <= a.Lk) mdma.issue_step(lds_addr_of(sMbuf), m0, a.Lq, a.mask.sm, 0, C::MROWCH, 2 * C::BN, 0);
         }
     }
+    // Vector mask: thread `tid` carries the value of key n0 + tid of the tile that follows.
+    static_assert(!C::VMASK || C::BN <= C::NTHREADS, "");
+    float mkey = 0.f;
+    auto load_vmask = [&](int n0) {
+        const int key = min(n0 + (tid & (C::BN - 1)), a.Lk - 1); // (past the end: the score is set to -inf below)
+        mkey = a.mask.is_f32 ? reinterpret_cast<const float *>(mbase)[key] : T::to_float(reinterpret_cast<const uint16_t *>(mbase)[key]);
+    };
+    auto store_vmask = [&](int buf) {
+        if (tid < C::BN) reinterpret_cast<float *>(sMbuf + buf * C::SM_ELEMS)[tid] = mkey;
+    };
     FwdStage<C> st;
     load_tile(st, 0);
+    if constexpr (C::VMASK) {
+        load_vmask(0);
+        store_vmask(0);
+    }
     ld.store(st, sKbuf, sVbuf);
     if constexpr (C::MTILE) wait_vmcnt<0>();
     __syncthreads();
@@ -352,6 +374,9 @@ __device__ __forceinline__ void fwd_body(const FwdArgs &a) {
                                 2 * C::BN, 0);
         }
         if (more) load_tile(st, n0 + C::BN);
+        if constexpr (C::VMASK) {
+            if (more) load_vmask(n0 + C::BN);
+        }
 
         const uint16_t *sK = sKbuf + cur * C::SK_ELEMS;
         const uint16_t *sVt = sVbuf + cur * C::SV_ELEMS;
@@ -391,8 +416,8 @@ __device__ __forceinline__ void fwd_body(const FwdArgs &a) {
                 // ---- S^T = [K | K_b] [scale Q | Q_b]^T
                 f32x16_t s[C::KBLK];
                 // additive mask: requested up front, it is the initial value of the bias chain
-                f32x16_t mk[C::MASK ? C::KBLK : 1];
-                if constexpr (C::MASK) {
+                f32x16_t mk[C::XMASK ? C::KBLK : 1];
+                if constexpr (C::XMASK) {
                     const uint8_t *mrow = mbase + (a.mask.type == 2 ? (int64_t)min(query, a.Lq - 1) * a.mask.sm : 0) *
                                                       (a.mask.is_f32 ? 4 : 2);
                     if (C::MTILE && mtile && n0 + C::BN <= a.Lk) {
@@ -424,7 +449,16 @@ __device__ __forceinline__ void fwd_body(const FwdArgs &a) {
 #pragma unroll
                     for (int v = 0; v < 16; ++v) {
                         acc[v] = 0.f;
-                        accb[v] = C::MASK ? mk[C::MASK ? kb : 0][v] : 0.f;
+                        accb[v] = C::XMASK ? mk[C::XMASK ? kb : 0][v] : 0.f;
+                    }
+                    if constexpr (C::VMASK) {
+                        const float *sM = reinterpret_cast<const float *>(sMbuf + cur * C::SM_ELEMS) + sub * C::BSUB + kb * 32 + 4 * g;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const f32x4_t x = *reinterpret_cast<const f32x4_t *>(sM + 8 * j);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) accb[4 * j + e] = x[e];
+                        }
                     }
 #pragma unroll
                     for (int t = 0; t < C::NK; ++t) {
@@ -504,6 +538,9 @@ __device__ __forceinline__ void fwd_body(const FwdArgs &a) {
                     }
             }
         }
+        if constexpr (C::VMASK) {
+            if (more) store_vmask(cur ^ 1);
+        }
         if (more) ld.store(st, sKbuf + (cur ^ 1) * C::SK_ELEMS, sVbuf + (cur ^ 1) * C::SV_ELEMS);
         if constexpr (C::MTILE) wait_vmcnt<0>(); // the mask tile copies are not known to the compiler
         __syncthreads();
@@ -535,7 +572,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 #include "fb_fwd_lean.h"
 namespace fb {
 
-template <class T, int NKD, int NKR, int NDV, bool VEC, bool MASK, bool QB2, bool FOLD>
+template <class T, int NKD, int NKR, int NDV, bool VEC, int MASK, bool QB2, bool FOLD>
 static hipError_t launch_fwd_qb(const FwdArgs &a0, hipStream_t stream) {
     typedef FwdCfg<T, NKD, NKR, NDV, VEC, MASK, QB2, FOLD> C;
     FwdArgs a = a0;
@@ -557,7 +594,7 @@ static hipError_t launch_fwd_qb(const FwdArgs &a0, hipStream_t stream) {
 // grid was walked head by head the small workgroups stayed ahead up to seven per compute unit).
 // Short sequences whose last 256-query workgroup would be half
 // empty also take the small ones (8192 x 16 windows of 128 tokens: 1.94 -> 1.41 ms).
-template <class T, int NKD, int NKR, int NDV, bool VEC, bool MASK, bool FOLD = false>
+template <class T, int NKD, int NKR, int NDV, bool VEC, int MASK, bool FOLD = false>
 static hipError_t launch_fwd_vec(const FwdArgs &a, hipStream_t stream) {
     if constexpr (FwdCfg<T, NKD, NKR, NDV, VEC, MASK, true>::QB == 2) {
         const int64_t wgs = (int64_t)a.B * a.H * ((a.Lq + 255) / 256);
@@ -574,9 +611,13 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
     const bool vec = a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.o.vec_ok && a.d % 8 == 0 &&
                      (a.r == 0 || (a.qb.vec_ok && a.kb.vec_ok && a.r % 8 == 0)) && a.k.ss < lim && a.v.ss < lim &&
                      (a.r == 0 || a.kb.ss < lim);
+    // A vector mask on aligned tensors, against the general masked instantiation: 384 x 4 rows of 384 tokens, rank 32,
+    // 131 -> 114 us a call; head dim 64, rank 16, 8 x 8 x (1000 x 1500), forward + backward, together with the dk/dv
+    // kernel's: 425 -> 236 us.  The outputs are bit for bit the same there.
+    if (vec && a.mask.type == kVectorMask) return launch_fwd_vec<T, NKD, NKR, NDV, true, kVectorMask>(a, stream);
     if (a.mask.type)
-        return vec ? launch_fwd_vec<T, NKD, NKR, NDV, true, true>(a, stream)
-                   : launch_fwd_vec<T, NKD, NKR, NDV, false, true>(a, stream);
+        return vec ? launch_fwd_vec<T, NKD, NKR, NDV, true, kMatrixMask>(a, stream)
+                   : launch_fwd_vec<T, NKD, NKR, NDV, false, kMatrixMask>(a, stream);
     if constexpr (NKD == 2 && NKR <= 1 && NDV == 1) {
         // The streamlined kernel: 256-query workgroups (two query blocks per wave) where they give every
         // SIMD of the chip a wave, 128-query workgroups (one block per wave) below that.
@@ -591,10 +632,10 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
         }
     }
     if constexpr (NKR <= 2) {
-        if (vec && fold_scale_ok<T>(a.scale, a.r, a.Lk)) return launch_fwd_vec<T, NKD, NKR, NDV, true, false, true>(a, stream);
+        if (vec && fold_scale_ok<T>(a.scale, a.r, a.Lk)) return launch_fwd_vec<T, NKD, NKR, NDV, true, kNoMask, true>(a, stream);
     }
-    return vec ? launch_fwd_vec<T, NKD, NKR, NDV, true, false>(a, stream)
-               : launch_fwd_vec<T, NKD, NKR, NDV, false, false>(a, stream);
+    return vec ? launch_fwd_vec<T, NKD, NKR, NDV, true, kNoMask>(a, stream)
+               : launch_fwd_vec<T, NKD, NKR, NDV, false, kNoMask>(a, stream);
 }
 
 template <class T, int NKD, int NDV>

@@ -191,6 +191,39 @@ def test_vector_mask_folded_into_factors(gpu_device, monkeypatch, r, bmask, hmas
     _gate(got2, ref, torch.bfloat16)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,r,B,Lq,Lk", [
+    (32, 32, 2, 300, 520), (32, 8, 1, 65, 129), (32, 16, 160, 200, 130), (32, 0, 3, 64, 1), (64, 16, 2, 129, 257), (64, 0, 1, 31, 63),
+    (128, 8, 1, 97, 190), (128, 64, 1, 64, 128), (16, 8, 2, 40, 95)])
+def test_vector_mask_equals_its_matrix(gpu_device, monkeypatch, d, r, B, Lq, Lk, dtype):
+    """A vector mask has instantiations of its own in the forward and dk/dv kernels (edges of their tiles, one and two
+    query blocks per wave, 16-bit and fp32 values, a base that is only 2-byte aligned, -inf and the type's lowest
+    value, causal): the same as the mask written out as a matrix, which takes the general ones.  The two add the same
+    values in fp32 at different places of a chain and sum over tiles of other lengths, so results differ in the last
+    bits only: twice the rounding of the outputs (2^-8 bf16, 2^-11 fp16) plus that of P and dS (the same again)."""
+    from flashbias_amd import interface
+    monkeypatch.setattr(interface, "_FOLD_MIN_PAIRS", 1 << 62)
+    H = 4
+    q, k, v, qb, kb, do = make_inputs(B, Lq, Lk, H, d, r, dtype, seed=d + r + Lk)
+    g = torch.Generator().manual_seed(5)
+    eps = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    for mtype, causal, low, offset in ((dtype, False, float("-inf"), 0), (torch.float32, False, torch.finfo(dtype).min, 1),
+                                       (dtype, True, torch.finfo(dtype).min, 1), (torch.float32, True, -1e4, 0)):
+        store = torch.randn(B * Lk + 1, generator=g).to(mtype)
+        mask = store[offset:offset + B * Lk].view(B, 1, 1, Lk)
+        if Lk > 8:
+            mask[..., Lk - Lk // 8:] = low
+            mask[0, ..., 3] = low
+        dev = store.to(gpu_device)[offset:offset + B * Lk].view(B, 1, 1, Lk)
+        vec = run_gpu(flash_bias_func, q, k, v, qb, kb, dev, causal, None, do, gpu_device)
+        mat = run_gpu(flash_bias_func, q, k, v, qb, kb, dev.expand(B, 1, Lq, Lk).contiguous() if Lq > 1 else dev, causal, None, do, gpu_device)
+        for name, x, y in zip(NAMES, vec, mat):
+            if y is None:
+                continue
+            assert torch.isfinite(x).all(), name
+            assert (x - y).abs().max() <= 2 * eps * max(1e-3, float(y.abs().max())), (name, mtype, causal)
+
+
 def test_very_long_sequence_properties(gpu_device):
     """L = 65536 (too long for the dense oracle): the first 1024 rows of a causal problem do not
     depend on anything behind them, so they must equal the L = 1024 result of the same inputs
