@@ -570,6 +570,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 
 } // namespace fb
 #include "fb_fwd_lean.h"
+#include "fb_fwd_wide.h"
 namespace fb {
 
 template <class T, int NKD, int NKR, int NDV, bool VEC, int MASK, bool QB2, bool FOLD>
@@ -611,10 +612,21 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
     const bool vec = a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.o.vec_ok && a.d % 8 == 0 &&
                      (a.r == 0 || (a.qb.vec_ok && a.kb.vec_ok && a.r % 8 == 0)) && a.k.ss < lim && a.v.ss < lim &&
                      (a.r == 0 || a.kb.ss < lim);
-    // A vector mask on aligned tensors, against the general masked instantiation: 384 x 4 rows of 384 tokens, rank 32,
-    // 131 -> 114 us a call; head dim 64, rank 16, 8 x 8 x (1000 x 1500), forward + backward, together with the dk/dv
-    // kernel's: 425 -> 236 us.  The outputs are bit for bit the same there.
-    if (vec && a.mask.type == kVectorMask) return launch_fwd_vec<T, NKD, NKR, NDV, true, kVectorMask>(a, stream);
+    // Head dims above 32, ranks up to 32: fb_fwd_wide.h at every length and grid (against the general kernel: causal
+    // B4 H32 L=4096 d128 r8 848 -> 642 us, B8 H16 L=4096 d64 r16 793 -> 687, B1 H4 L=256 d64 r8 10.0 -> 7.5, B8 H32 L=300
+    // d64 r8 20.0 -> 17.3; fp16 d64 r16 8 x 8 x (1000 x 1500) with a vector mask 117 -> 49); a matrix mask needs its tile
+    // in LDS, larger ranks more registers, and they stay with the general one.
+    constexpr bool WIDE = NKD >= 4 && NKR <= 2;
+    if constexpr (WIDE) {
+        if (vec && a.mask.type == kVectorMask) return launch_fwd_wide<T, NKD, NKR, NDV, kVectorMask, false>(a, stream);
+        if (vec && a.mask.type == kNoMask)
+            return fold_scale_ok<T>(a.scale, a.r, a.Lk) ? launch_fwd_wide<T, NKD, NKR, NDV, kNoMask, true>(a, stream)
+                                                       : launch_fwd_wide<T, NKD, NKR, NDV, kNoMask, false>(a, stream);
+    } else if (vec && a.mask.type == kVectorMask) {
+        // A vector mask on aligned tensors, against the general masked instantiation: 384 x 4 rows of 384 tokens, rank
+        // 32, 131 -> 114 us a call.  The outputs are bit for bit the same.
+        return launch_fwd_vec<T, NKD, NKR, NDV, true, kVectorMask>(a, stream);
+    }
     if (a.mask.type)
         return vec ? launch_fwd_vec<T, NKD, NKR, NDV, true, kMatrixMask>(a, stream)
                    : launch_fwd_vec<T, NKD, NKR, NDV, false, kMatrixMask>(a, stream);
@@ -631,11 +643,13 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
                                                              : launch_fwd_lean<T, NKR, 1>(a, stream);
         }
     }
-    if constexpr (NKR <= 2) {
+    if constexpr (NKR <= 2 && !WIDE) {
         if (vec && fold_scale_ok<T>(a.scale, a.r, a.Lk)) return launch_fwd_vec<T, NKD, NKR, NDV, true, kNoMask, true>(a, stream);
     }
-    return vec ? launch_fwd_vec<T, NKD, NKR, NDV, true, kNoMask>(a, stream)
-               : launch_fwd_vec<T, NKD, NKR, NDV, false, kNoMask>(a, stream);
+    if constexpr (!WIDE) {
+        if (vec) return launch_fwd_vec<T, NKD, NKR, NDV, true, kNoMask>(a, stream);
+    }
+    return launch_fwd_vec<T, NKD, NKR, NDV, false, kNoMask>(a, stream);
 }
 
 template <class T, int NKD, int NDV>

@@ -1,0 +1,277 @@
+// Forward for head dims 33 ... 128 on aligned tensors (rank up to 32, no mask or a vector mask).  Included by fb_fwd.hip
+// after the general kernel, whose arithmetic it shares (one query per lane, S^T = [K | K_b] [Q | Q_b]^T, online softmax
+// against a lagging reference point, O^T += V^T P^T, P from registers).
+//
+// What differs is how tiles reach the matrix cores.  At these head dims the general kernel's loader, which takes K and V
+// through registers and transposes V on the way into LDS, is what a tile's time goes into: the transposing stores meet
+// in few banks, its stage takes about 40 registers (at head dim 128 the kernel spilled at 256), and K fragments are
+// requested one MFMA ahead.  Here global_load_lds copies [K], [K_b] and [V] row-major into two stages, one tile ahead,
+// V^T fragments come from transposing LDS reads, and no register holds a tile.
+#pragma once
+#include "fb_lean_tiles.h"
+
+namespace fb {
+
+template <class T, int NKD_, int NKR_, int NDV_, int MASK_, bool FOLD_>
+struct FwdWideCfg {
+    static constexpr int NKD = NKD_, NKR = NKR_, NDV = NDV_, NK = NKD_ + NKR_;
+    static constexpr bool VMASK = MASK_ == kVectorMask, FOLD = FOLD_;
+    static_assert(MASK_ != kMatrixMask && !(FOLD_ && VMASK), "");
+    static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES;
+    static constexpr int BM = 32 * NWAVES;
+    static constexpr int KBLK = 2, BN = 32 * KBLK;
+    static constexpr int ROWCH = 2 * NKD, CPR = 2 * NKR; // 16-byte chunks per row of K and V, of K_b
+    static constexpr int SK = BN * ROWCH * 8, SKB = BN * CPR * 8, SM = VMASK ? 2 * BN : 0;
+    static constexpr int STAGE = 2 * SK + SKB + SM; // elements: K, V, K_b, fp32 vector mask
+    static constexpr int LDS_BYTES = 2 * STAGE * 2;
+    static constexpr int KBINST = BN * CPR / 64; // copies that fill the K_b region, one per wave
+    static_assert(KBINST <= NWAVES, "");
+    // head dim <= 64: three workgroups per compute unit (168 registers, 3 x 40 KB)
+    static constexpr int WAVES_EU = NKD <= 4 ? 3 : 2;
+    static __device__ __forceinline__ bool low_parts(const FwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
+};
+
+// K_b rows as a dense region (fb_lean_tiles.h), one copy instruction of waves 0 ... KBINST - 1 per tile.
+template <class C>
+struct FwdWideBias {
+    uint32_t off, row;
+    uint64_t lanes;
+    const uint8_t *p;
+    uint32_t pitch;
+    int wave;
+    __device__ __forceinline__ void init(const FwdArgs &a, const uint16_t *kbbase, int wave_, int lane) {
+        wave = wave_;
+        p = reinterpret_cast<const uint8_t *>(kbbase);
+        pitch = (uint32_t)(a.kb.ss * 2);
+        int r, ch;
+        lean_copy_place<C::CPR>(lane, r, ch);
+        row = wave * (64 / C::CPR) + r;
+        if (C::low_parts(a) && ch == 1) ch = 0; // (the partner of the low parts of q_b / scale)
+        lanes = __builtin_amdgcn_ballot_w64(ch * 8 < a.r);
+        off = row * pitch + ch * 16;
+    }
+    __device__ __forceinline__ void issue(uint32_t lds, int n0, int Lk) {
+        if (wave < C::KBINST) {
+            uint32_t o = off;
+            if (n0 + C::BN > Lk) o -= (uint32_t)max(n0 + (int)row - (Lk - 1), 0) * pitch; // (past the end: the last row again)
+            lds_dma16_lanes(o, p, lds + wave * 1024, lanes);
+        }
+        p += (int64_t)C::BN * pitch;
+    }
+};
+
+template <class T, class C>
+__global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::WAVES_EU, C::WAVES_EU))) void fwd_wide_kernel(const FwdArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    uint16_t *stage0 = reinterpret_cast<uint16_t *>(smem);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 31, g = lane >> 5;
+
+    const int total = a.ntiles_m * a.B * a.H;
+    int bh, tile_m;
+    work_order(blockIdx.x, a.ntiles_m, total, a.causal, bh, tile_m);
+    if (a.causal) tile_m = a.ntiles_m - 1 - tile_m; // the last query tile sees the most keys
+    const int b = bh / a.H, h = bh % a.H;
+    const int m0 = tile_m * C::BM, wq0 = m0 + wave * 32;
+    const int query = wq0 + c;
+
+    const uint16_t *qbase = a.q.ptr + b * a.q.sb + h * a.q.sh;
+    const uint16_t *kbase = a.k.ptr + b * a.k.sb + h * a.k.sh;
+    const uint16_t *vbase = a.v.ptr + b * a.v.sb + h * a.v.sh;
+
+    u32x4_t qr[C::NK];
+#pragma unroll
+    for (int t = 0; t < C::NKD; ++t) qr[t] = load_chunk<true>(qbase, a.q.ss, query, a.Lq, 16 * t + 8 * g, a.d);
+    FwdWideBias<C> kbd;
+    if constexpr (C::NKR > 0) {
+        const uint16_t *qbbase = a.qb.ptr + b * a.qb.sb + h * a.qb.sh;
+        const bool low = C::low_parts(a) && g == 1;
+#pragma unroll
+        for (int t = 0; t < C::NKR; ++t) {
+            u32x4_t x = load_chunk<true>(qbbase, a.qb.ss, query, a.Lq, low ? 0 : 16 * t + 8 * g, a.r);
+            if (C::FOLD && a.scale != 1.f) x = fold_scale_chunk<T>(x, 1.f / a.scale, C::low_parts(a), low);
+            qr[C::NKD + t] = x;
+        }
+        kbd.init(a, a.kb.ptr + b * a.kb.sb + h * a.kb.sh, wave, lane);
+    }
+    f32x16_t acc_o[C::NDV];
+#pragma unroll
+    for (int n = 0; n < C::NDV; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc_o[n][v] = 0.f;
+    float m_ref = -INFINITY, m2 = 0.f, l_run = 0.f; // (as in fwd_body)
+    const float to_log2 = C::FOLD ? a.scale * kLog2e : kLog2e;
+    const float lag = 8.0f / to_log2;
+
+    int k_end = a.Lk;
+    if (a.causal && m0 + C::BM < k_end) k_end = m0 + C::BM;
+    const int ntiles = (k_end + C::BN - 1) / C::BN;
+
+    {   // clear the stages once: the zero padding of the channel dimension is never rewritten
+        u32x4_t *z = reinterpret_cast<u32x4_t *>(smem);
+        for (int i = tid; i < C::LDS_BYTES / 16; i += C::NTHREADS) z[i] = u32x4_t{0u, 0u, 0u, 0u};
+    }
+    __syncthreads();
+
+    TileDma<C::BN, C::ROWCH, C::NWAVES, false> kd, vd;
+    kd.init(kbase, a.k.ss, a.d, C::ROWCH, nullptr, 0, 0, wave, lane, 0);
+    vd.init(vbase, a.v.ss, a.d, C::ROWCH, nullptr, 0, 0, wave, lane, 0);
+    auto issue = [&](int buf, int n0) {
+        const uint32_t base = lds_addr_of(stage0 + buf * C::STAGE);
+        kd.issue(base, n0, a.Lk, a.k.ss, 0, C::ROWCH);
+        if constexpr (C::NKR > 0) kbd.issue(base + 4 * C::SK, n0, a.Lk);
+        vd.issue(base + 2 * C::SK, n0, a.Lk, a.v.ss, 0, C::ROWCH);
+    };
+    // Vector mask: thread `tid` carries the value of key n0 + tid of the tile that follows.
+    float mkey = 0.f;
+    auto load_vmask = [&](int n0) {
+        const int key = min(n0 + (tid & (C::BN - 1)), a.Lk - 1); // (past the end: the score is set to -inf below)
+        const uint8_t *mbase = reinterpret_cast<const uint8_t *>(a.mask.ptr) + mask_offset(a.mask, b, h) * (a.mask.is_f32 ? 4 : 2);
+        mkey = a.mask.is_f32 ? reinterpret_cast<const float *>(mbase)[key] : T::to_float(reinterpret_cast<const uint16_t *>(mbase)[key]);
+    };
+    auto store_vmask = [&](int buf) {
+        if (tid < C::BN) reinterpret_cast<float *>(stage0 + buf * C::STAGE + 2 * C::SK + C::SKB)[tid] = mkey;
+    };
+    issue(0, 0);
+    if constexpr (C::VMASK) {
+        load_vmask(0);
+        store_vmask(0);
+    }
+    wait_vmcnt<0>();
+    barrier_lds();
+
+    int turn = __builtin_amdgcn_readfirstlane(cu_slot());
+    for (int it = 0; it < ntiles; ++it) {
+        const int cur = it & 1, n0 = it * C::BN;
+        const bool more = it + 1 < ntiles;
+        take_turn(turn, a.slots);
+        if (more) {
+            issue(cur ^ 1, n0 + C::BN);
+            if constexpr (C::VMASK) load_vmask(n0 + C::BN);
+        }
+        const uint16_t *sK = stage0 + cur * C::STAGE, *sV = sK + C::SK;
+        const uint8_t *sKb = reinterpret_cast<const uint8_t *>(sV + C::SK);
+        // (a tile hidden from every query of this wave: so are all later ones, but the copies and barriers go on)
+        if (!(a.causal && n0 > wq0 + 31) && wq0 < a.Lq) {
+            f32x16_t s[C::KBLK];
+#pragma unroll
+            for (int kb = 0; kb < C::KBLK; ++kb)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) s[kb][v] = 0.f;
+#pragma unroll
+            for (int t = 0; t < C::NKD; ++t)
+#pragma unroll
+                for (int kb = 0; kb < C::KBLK; ++kb) {
+                    const u32x4_t kf = *reinterpret_cast<const u32x4_t *>(sK + swz_off<C::ROWCH>(kb * 32 + c, 2 * t + g));
+                    s[kb] = T::mfma(kf, qr[t], s[kb]);
+                }
+            // the softmax scale multiplies the fp32 q k^T accumulator before the bias steps (:246-256)
+            if constexpr (!C::FOLD) {
+#pragma unroll
+                for (int kb = 0; kb < C::KBLK; ++kb) {
+                    if constexpr (C::VMASK) {
+                        const float *sM = reinterpret_cast<const float *>(sV + C::SK + C::SKB) + kb * 32 + 4 * g;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const f32x4_t x = *reinterpret_cast<const f32x4_t *>(sM + 8 * j);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) s[kb][4 * j + e] = __builtin_fmaf(s[kb][4 * j + e], a.scale, x[e]);
+                        }
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) s[kb][v] *= a.scale;
+                    }
+                }
+            }
+            if constexpr (C::NKR > 0) {
+#pragma unroll
+                for (int t = 0; t < C::NKR; ++t)
+#pragma unroll
+                    for (int kb = 0; kb < C::KBLK; ++kb) {
+                        const u32x4_t kf = *reinterpret_cast<const u32x4_t *>(sKb + lean_row_addr<C::CPR>(c, 2 * t + g) + kb * 32 * C::CPR * 16);
+                        s[kb] = T::mfma(kf, qr[C::NKD + t], s[kb]);
+                    }
+            }
+            // (bitwise on purpose, as in the dq kernel: no scalar block between the last MFMA and the branch)
+            const bool edge = (n0 + C::BN > a.Lk) | ((a.causal != 0) & (n0 + C::BN - 1 > wq0));
+            if (edge) {
+                int key0 = n0 + 4 * g;
+                asm volatile("" : "+v"(key0)); // (computed here, not kept in registers across the loop)
+#pragma unroll
+                for (int kb = 0; kb < C::KBLK; ++kb)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const int key = key0 + kb * 32 + 8 * (v >> 2) + (v & 3);
+                        if (key >= a.Lk || (a.causal && key > query)) s[kb][v] = -INFINITY;
+                    }
+            }
+            float mx = s[0][0];
+#pragma unroll
+            for (int kb = 0; kb < C::KBLK; ++kb)
+#pragma unroll
+                for (int v = (kb == 0 ? 1 : 0); v < 16; ++v) mx = fmaxf(mx, s[kb][v]);
+            mx = half_wave_max(mx);
+            const bool grow = mx > m_ref + lag; // also true for the first finite score of a row
+            if (__any(grow)) {
+                const float m_new = grow ? mx : m_ref;
+                const float alpha = grow ? fast_exp2((m_ref - m_new) * to_log2) : 1.f; // exp2(-inf) = 0
+                l_run *= alpha;
+#pragma unroll
+                for (int n = 0; n < C::NDV; ++n)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc_o[n][v] *= alpha;
+                m_ref = m_new;
+                m2 = (m_new == -INFINITY) ? 0.f : m_new * to_log2;
+            }
+#pragma unroll
+            for (int kb = 0; kb < C::KBLK; ++kb)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    u32x4_t pb;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float p0 = fast_exp2(__builtin_fmaf(s[kb][8 * t + 2 * e], to_log2, -m2));
+                        const float p1 = fast_exp2(__builtin_fmaf(s[kb][8 * t + 2 * e + 1], to_log2, -m2));
+                        pb[e] = T::pack2(p0, p1);
+                        l_run += p0 + p1;
+                    }
+#pragma unroll
+                    for (int n = 0; n < C::NDV; ++n)
+                        acc_o[n] = T::mfma(lds_read_a_tr<C::ROWCH>(sV, kb * 32 + 16 * t, 32 * n, c, g), pb, acc_o[n]);
+                }
+        }
+        if constexpr (C::VMASK) {
+            if (more) store_vmask(cur ^ 1);
+        }
+        wait_vmcnt<0>(); // the next tile has landed
+        barrier_lds();
+    }
+
+    uint16_t *obase = const_cast<uint16_t *>(a.o.ptr) + b * a.o.sb + h * a.o.sh;
+    int q = query;
+    asm volatile("" : "+v"(q)); // (keeps the address arithmetic below the key loop)
+    const float l = l_run + __shfl_xor(l_run, 32, 64);
+    const float inv = 1.f / l;
+    const bool ok = q < a.Lq;
+    if (ok && g == 0) a.lse[(int64_t)bh * a.Lq + q] = m_ref * (C::FOLD ? a.scale : 1.f) + __builtin_amdgcn_logf(l) * kLn2;
+    uint16_t *orow = obase + (int64_t)(ok ? q : 0) * a.o.ss;
+#pragma unroll
+    for (int n = 0; n < C::NDV; ++n) store_acc_rows<T, true>(orow + 32 * n, ok, true, acc_o[n], inv, a.d - 32 * n, g);
+}
+
+template <class T, int NKD, int NKR, int NDV, int MASK, bool FOLD>
+static hipError_t launch_fwd_wide(const FwdArgs &a0, hipStream_t stream) {
+    typedef FwdWideCfg<T, NKD, NKR, NDV, MASK, FOLD> C;
+    FwdArgs a = a0;
+    a.ntiles_m = (a.Lq + C::BM - 1) / C::BM;
+    auto kern = fwd_wide_kernel<T, C>;
+    static KernelOnce once;
+    const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
+    if (e != hipSuccess) return e;
+    const int64_t total = (int64_t)a.ntiles_m * a.B * a.H;
+    a.slots = slots_per_cu(kern, C::NTHREADS, C::LDS_BYTES, total, once);
+    return launch_flat(kern, total, C::NTHREADS, C::LDS_BYTES, stream, a);
+}
+
+} // namespace fb

@@ -224,6 +224,17 @@ def test_vector_mask_equals_its_matrix(gpu_device, monkeypatch, d, r, B, Lq, Lk,
             assert (x - y).abs().max() <= 2 * eps * max(1e-3, float(y.abs().max())), (name, mtype, causal)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,r,Lq,Lk,scale", [
+    (64, 8, 1, 1, None), (64, 16, 127, 63, None), (40, 8, 129, 64, None), (64, 0, 128, 65, None), (56, 24, 200, 600, 0.125),
+    (128, 8, 33, 640, None), (128, 32, 130, 129, 1.0), (72, 16, 257, 127, None), (96, 0, 31, 192, -0.1), (128, 16, 64, 530, 0.0625)])
+def test_wide_heads(gpu_device, d, r, Lq, Lk, scale, dtype):
+    """Forward of head dims above 32 at the edges of its tiles (128 queries, 64 keys), padded head dims and ranks, the
+    scale folded (a power of two, 1, low parts at rank 8) and not, causal, and a gradient through its lse."""
+    for causal in (False, True):
+        _case(gpu_device, 2, Lq, Lk, 3, d, r, dtype, causal, scale=scale, seed=d + r + Lk, o_by_magnitude=True)
+
+
 def test_very_long_sequence_properties(gpu_device):
     """L = 65536 (too long for the dense oracle): the first 1024 rows of a causal problem do not
     depend on anything behind them, so they must equal the L = 1024 result of the same inputs
