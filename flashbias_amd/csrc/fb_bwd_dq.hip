@@ -18,16 +18,18 @@
 // summation order (bit-reproducible).  The softmax scale multiplies the fp32 q k^T accumulator as
 // in the forward; dq is multiplied by the scale in the epilogue, dq_bias is not (:728-732).
 #include "fb_kernels.h"
+#include "fb_lean_tiles.h"
 
 namespace fb {
 
 // QB2_: allow two query blocks per wave (the launcher turns it off for small grids).
 // FOLD_: the scores are scale * (q k^T + (q_b / scale) k_b^T), one MFMA chain and no FMA per
 // score for the scale (the launcher says when that is exact).
-// KB1_: 32-key tiles (half the LDS per stage: two workgroups per CU at head dims above 64).
+// SPLIT_: K_b in a dense region of its own instead of the upper chunks of a padded K row (head dims above 64, aligned,
+// unmasked, rank <= 32: 16 + 2 or 4 chunks against 32), so that 64-key tiles in two stages fit two workgroups per CU.
 // BG_: also accumulate dq_bias (false: the caller does not want the factor gradients; the accumulator blocks that
 // hold nothing but dq_bias are then left out of the products).
-template <class T, int NKD_, int NKR_, bool VEC_, bool MASK_, bool QB2_ = true, bool FOLD_ = false, bool KB1_ = false,
+template <class T, int NKD_, int NKR_, bool VEC_, bool MASK_, bool QB2_ = true, bool FOLD_ = false, bool SPLIT_ = false,
           bool BG_ = true>
 struct DqCfg {
     static constexpr bool FOLD = FOLD_;
@@ -36,6 +38,7 @@ struct DqCfg {
     // partner of the low parts of q_b / scale in the query operand
     static __device__ __forceinline__ bool low_parts(const BwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
     static constexpr int NKD = NKD_, NKR = NKR_;
+    static constexpr bool SPLIT = SPLIT_;
     static constexpr bool VEC = VEC_, MASK = MASK_;
     static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES;
     static constexpr int NK = NKD + NKR;
@@ -43,21 +46,23 @@ struct DqCfg {
     static constexpr int MBE = BG_ ? MB : (NKD + 1) / 2; // ... of which the key loop accumulates the first MBE
     static constexpr int QBLK = (QB2_ && NK <= 3 && !MASK_) ? 2 : 1; // the mask values need the registers of the second block
     static constexpr int BM = NWAVES * QBLK * 32;
-    static constexpr int KBLK = KB1_ ? 1 : 2, BN = 32 * KBLK;
-    static constexpr bool ONECHAIN = KB1_ && !MASK_; // scale between the d steps and the r steps of one MFMA chain
+    static constexpr int KBLK = 2, BN = 32 * KBLK;
+    static constexpr int UNROLL = SPLIT ? 1 : KBLK;
+    static constexpr bool ONECHAIN = SPLIT_ && !MASK_; // scale between the d steps and the r steps of one MFMA chain
     // sK row: [K | K_b] of one key in ROWCH swizzled 16-byte chunks; the one copy is read
     // row-wise for S^T and column-wise for [dQ | dQ_b]^T
-    static constexpr int ROWCH = 2 * NK <= 8 ? 8 : 2 * NK <= 16 ? 16 : 32;
+    static constexpr int ROWCH = SPLIT ? 2 * NKD : 2 * NK <= 8 ? 8 : 2 * NK <= 16 ? 16 : 32;
     static constexpr int ROWCHV = 2 * NKD <= 8 ? 8 : 16; // sV row: V of one key, same chunk swizzle
     static constexpr int SK = BN * ROWCH * 8, SV = BN * ROWCHV * 8;
+    static constexpr int CPR = 2 * (NKR > 0 ? NKR : 1), SKB = SPLIT && NKR > 0 ? BN * CPR * 8 : 0; // (after the V tile)
     // masked, aligned instantiations also stage the tile's BM x BN block of a 16-bit matrix mask
     static constexpr bool MTILE = VEC_ && MASK_;
     static constexpr int MROWCH = BN / 8; // chunks per mask-tile row
     static constexpr int SM = MTILE ? BM * BN : 0;
-    static constexpr int STAGE = SK + SV + SM;
+    static constexpr int STAGE = SK + SV + SKB + SM;
     // direct loader: three stages, two tiles ahead; with a mask tile (or the element-wise loader)
     // two stages, one ahead
-    static constexpr int AHEAD = (VEC_ && !MASK_) ? 2 : 1;
+    static constexpr int AHEAD = (VEC_ && !MASK_ && !SPLIT) ? 2 : 1;
     static constexpr int NSTAGE = AHEAD + 1;
     static constexpr int LDS_BYTES = NSTAGE * STAGE * 2;
     // loader: 8-channel chunks of K, K_b and V, one key row each
@@ -65,7 +70,7 @@ struct DqCfg {
     static constexpr int K_TASKS = BN * (CD + CR), V_TASKS = BN * CD;
     static constexpr int K_PT = (K_TASKS + NTHREADS - 1) / NTHREADS;
     static constexpr int V_PT = (V_TASKS + NTHREADS - 1) / NTHREADS;
-    static constexpr int WAVES_EU = (NK <= (MASK_ ? 6 : 8) || KB1_) ? 2 : 1;
+    static constexpr int WAVES_EU = (NK <= (MASK_ ? 6 : 8) || SPLIT_) ? 2 : 1;
 };
 
 template <class C>
@@ -135,7 +140,8 @@ struct DqLoader {
 // a key tile, copied straight into an LDS stage.
 template <class C>
 struct DqDirect {
-    TileDma<C::BN, C::ROWCH, C::NWAVES, (C::NKR > 0)> k;
+    TileDma<C::BN, C::ROWCH, C::NWAVES, (C::SKB == 0 && C::NKR > 0)> k;
+    DenseCopy<C::BN, C::CPR> kb; // K_b where it has a region of its own
     TileDma<C::BN, C::ROWCHV, C::NWAVES, false> v;
     TileDma<C::BM, C::MROWCH, C::NWAVES, false> m; // mask tile (masked instantiations, 16-bit matrix masks)
     bool mtile = false;
@@ -145,6 +151,7 @@ struct DqDirect {
                                          const uint16_t *vbase, int wave, int lane) {
         k.init(kbase, a.k.ss, a.d, 2 * C::NKD, C::NKR > 0 ? kbbase : nullptr, C::NKR > 0 ? a.kb.ss : 0, a.r, wave, lane, 0,
                C::low_parts(a));
+        if constexpr (C::SKB > 0) kb.init(kbbase, a.kb.ss, a.r, C::low_parts(a), wave, lane, 0);
         v.init(vbase, a.v.ss, a.d, C::ROWCHV, nullptr, 0, 0, wave, lane, 0);
     }
 
@@ -159,6 +166,7 @@ struct DqDirect {
     __device__ __forceinline__ void issue(const BwdArgs &a, uint16_t *stage, int n0, int Lk) {
         const uint32_t base = lds_addr_of(stage);
         k.issue(base, n0, Lk, a.k.ss, C::NKR > 0 ? a.kb.ss : 0, 2 * C::NKD);
+        if constexpr (C::SKB > 0) kb.issue(base + 2 * (C::SK + C::SV), n0, Lk);
         v.issue(base + 2 * C::SK, n0, Lk, a.v.ss, 0, C::ROWCHV);
         if constexpr (C::MTILE) { // full tiles only: a ragged last tile takes the element path
             if (mtile && n0 + C::BN <= Lk)
@@ -276,7 +284,9 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
     float lse2[C::QBLK]; // lse * log2(e) of this lane's queries
     // -delta of this lane's query in all 16 registers of an accumulator block: the initial value
     // of every dP^T chain (lane = query, so it is the same for every key), no add per score
+    // (SPLIT: added per score instead, the 16 registers are needed)
     f32x16_t negd[C::QBLK];
+    float negd1[C::QBLK];
 #pragma unroll
     for (int qb = 0; qb < C::QBLK; ++qb) {
         const int query = wq0 + qb * 32 + c;
@@ -339,7 +349,8 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
         }
         lse2[qb] = l2; // rows past the end: P = exp2(-inf) = 0
 #pragma unroll
-        for (int v = 0; v < 16; ++v) negd[qb][v] = nd;
+        for (int v = 0; v < 16; ++v) negd[qb][v] = C::SPLIT ? 0.f : nd;
+        negd1[qb] = nd;
         // (element v of block n is channel 32 n + 8 (v / 4) + 4 g + v % 4: below 16 NKD it belongs to dq)
 #pragma unroll
         for (int n = 0; n < C::MB; ++n)
@@ -382,7 +393,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
     __syncthreads();
 
     int cur = 0; // stage of the current tile
-    take_turn(turn, a.slots);
+    if (!C::SPLIT) take_turn(turn, a.slots);
     for (int it = 0; it < ntiles_k; ++it) {
         const int n0 = it * C::BN;
         const bool more = it + 1 < ntiles_k;
@@ -395,17 +406,30 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
         }
 
         const uint16_t *sK = stage0 + cur * C::STAGE, *sV = sK + C::SK;
+        const uint8_t *sKb = reinterpret_cast<const uint8_t *>(sV + C::SV);
         const bool visible = !(a.causal && n0 > wq0 + 32 * C::QBLK - 1) && wq0 < a.Lq;
         if (visible) {
-#pragma unroll
+            // (head dims above 64: one block at a time, two at once would spill)
+#pragma unroll C::UNROLL
             for (int kb = 0; kb < C::KBLK; ++kb) {
+                TileAddr16 ta(lds_addr_of(sK) + kb * (32 * 256), c, g); // (SPLIT; the V tile follows at + 2 SK)
+                if constexpr (C::SPLIT) asm volatile("" : "+v"(ta.row), "+v"(ta.tr));
+                if (C::UNROLL == 1 && a.causal && n0 + kb * 32 > wq0 + 31) break; // hidden from every query of this wave
+                // (the wave that feeds the matrix pipe goes first, instead of turns by tile: 994 -> 977 us causal B4 H32 L=4096 d128)
+                if (C::SPLIT) __builtin_amdgcn_s_setprio(1);
                 u32x4_t ka[C::NK], va[C::NKD];
 #pragma unroll
-                for (int t = 0; t < C::NK; ++t)
-                    ka[t] = *reinterpret_cast<const u32x4_t *>(sK + swz_off<C::ROWCH>(kb * 32 + c, 2 * t + g));
+                for (int t = 0; t < C::NK; ++t) {
+                    if (C::SKB > 0 && t >= C::NKD)
+                        ka[t] = *reinterpret_cast<const u32x4_t *>(sKb + kb * 32 * C::CPR * 16 + lean_row_addr<C::CPR>(c, 2 * (t - C::NKD) + g));
+                    else if constexpr (C::SPLIT)
+                        ka[t] = ta.load_row(t, 0);
+                    else
+                        ka[t] = *reinterpret_cast<const u32x4_t *>(sK + swz_off<C::ROWCH>(kb * 32 + c, 2 * t + g));
+                }
 #pragma unroll
                 for (int t = 0; t < C::NKD; ++t)
-                    va[t] = *reinterpret_cast<const u32x4_t *>(sV + swz_off<C::ROWCHV>(kb * 32 + c, 2 * t + g));
+                    va[t] = C::SPLIT ? ta.load_row(t, 2 * C::SK) : *reinterpret_cast<const u32x4_t *>(sV + swz_off<C::ROWCHV>(kb * 32 + c, 2 * t + g));
                 u32x4_t dsp[C::QBLK][2]; // dS^T, packed, per 16-key step
 #pragma unroll
                 for (int qb = 0; qb < C::QBLK; ++qb) {
@@ -469,6 +493,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
                     }
 #pragma unroll
                     for (int t = 0; t < C::NKD; ++t) dp = T::mfma(va[t], dor[qb][t], t == 0 ? negd[qb] : dp);
+                    if (C::SPLIT) __builtin_amdgcn_s_setprio(0);
                     // (bitwise on purpose: a short-circuit evaluation puts a small block of scalar code between the last
                     // MFMA and the branch, which the branch's other edge skips, and the compiler then counts the
                     // wait states between an MFMA and the first reader of its result along the longer path only)
@@ -486,15 +511,25 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
                     for (int v = 0; v < 16; v += 2) {
                         const float p0 = fast_exp2(__builtin_fmaf(s[v], to_log2, -lse2[qb]));
                         const float p1 = fast_exp2(__builtin_fmaf(s[v + 1], to_log2, -lse2[qb]));
-                        dsp[qb][v >> 3][(v & 7) >> 1] = T::pack2(p0 * dp[v], p1 * dp[v + 1]);
+                        if constexpr (C::SPLIT)
+                            dsp[qb][v >> 3][(v & 7) >> 1] = T::pack2(p0 * (dp[v] + negd1[qb]), p1 * (dp[v + 1] + negd1[qb]));
+                        else
+                            dsp[qb][v >> 3][(v & 7) >> 1] = T::pack2(p0 * dp[v], p1 * dp[v + 1]);
                     }
                 }
+                if (C::SPLIT) __builtin_amdgcn_s_setprio(1);
                 // [dQ | dQ_b]^T += [K | K_b]^T dS^T over this block's 32 keys
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
                     for (int n = 0; n < C::MBE; ++n) {
-                        const u32x4_t kt = lds_read_a_tr<C::ROWCH>(sK, kb * 32 + 16 * t, 32 * n, c, g);
+                        u32x4_t kt;
+                        if (C::SKB > 0 && 2 * n >= C::NKD)
+                            kt = dense_read_a_tr<C::CPR>(sKb, kb * 32 + 16 * t, c, g);
+                        else if constexpr (C::SPLIT)
+                            kt = ta.load_tr(n, 16 * 256 * t);
+                        else
+                            kt = lds_read_a_tr<C::ROWCH>(sK, kb * 32 + 16 * t, 32 * n, c, g);
 #pragma unroll
                         for (int qb = 0; qb < C::QBLK; ++qb) acc[qb][n] = T::mfma(kt, dsp[qb][t], acc[qb][n]);
                     }
@@ -511,7 +546,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
             __syncthreads();
         }
         cur = nxt;
-        take_turn(turn, a.slots); // (next to the barrier: the compiler moves nothing across either)
+        if (!C::SPLIT) take_turn(turn, a.slots); // (next to the barrier: the compiler moves nothing across either)
     }
 
     // ---- epilogue of this batch entry: dq = scale * acc rows [0, d)
@@ -535,9 +570,9 @@ bwd_dq_kernel(const BwdArgs a) {
     bwd_dq_body<T, C>(a, blockIdx.x);
 }
 
-template <class T, int NKD, int NKR, bool VEC, bool MASK, bool QB2, bool FOLD, bool KB1, bool BG>
+template <class T, int NKD, int NKR, bool VEC, bool MASK, bool QB2, bool FOLD, bool SPLIT, bool BG>
 static hipError_t launch_dq_qb_bg(const BwdArgs &a0, hipStream_t stream) {
-    typedef DqCfg<T, NKD, NKR, VEC, MASK, QB2, FOLD, KB1, BG> C;
+    typedef DqCfg<T, NKD, NKR, VEC, MASK, QB2, FOLD, SPLIT, BG> C;
     BwdArgs a = a0;
     a.ntiles_m = (a.Lq + C::BM - 1) / C::BM;
     auto kern = bwd_dq_kernel<T, C>;
@@ -550,13 +585,13 @@ static hipError_t launch_dq_qb_bg(const BwdArgs &a0, hipStream_t stream) {
     return launch_flat(kern, total, C::NTHREADS, C::LDS_BYTES, stream, a);
 }
 
-template <class T, int NKD, int NKR, bool VEC, bool MASK, bool QB2, bool FOLD, bool KB1 = false>
+template <class T, int NKD, int NKR, bool VEC, bool MASK, bool QB2, bool FOLD, bool SPLIT = false>
 static hipError_t launch_dq_qb(const BwdArgs &a, hipStream_t stream) {
     // head dim 32, aligned, unmasked, no dq_bias wanted: the instantiation without its products
-    if constexpr (NKD == 2 && NKR > 0 && NKR <= 2 && VEC && !MASK && !KB1) {
-        if (!a.dqb.ptr) return launch_dq_qb_bg<T, NKD, NKR, VEC, MASK, QB2, FOLD, KB1, false>(a, stream);
+    if constexpr (NKD == 2 && NKR > 0 && NKR <= 2 && VEC && !MASK && !SPLIT) {
+        if (!a.dqb.ptr) return launch_dq_qb_bg<T, NKD, NKR, VEC, MASK, QB2, FOLD, SPLIT, false>(a, stream);
     }
-    return launch_dq_qb_bg<T, NKD, NKR, VEC, MASK, QB2, FOLD, KB1, true>(a, stream);
+    return launch_dq_qb_bg<T, NKD, NKR, VEC, MASK, QB2, FOLD, SPLIT, true>(a, stream);
 }
 
 // 256-query workgroups (two blocks per wave) once every compute unit has two of them (three under
@@ -571,9 +606,8 @@ static hipError_t launch_dq_vec(const BwdArgs &a, hipStream_t stream) {
         if (wgs < (int64_t)(a.causal ? 3 : 2) * num_cus() || half_empty_256(a.Lq))
             return launch_dq_qb<T, NKD, NKR, VEC, MASK, false, FOLD>(a, stream);
     }
-    // head dims above 64, aligned, unmasked, rank <= 32: 32-key tiles fit two workgroups per CU
-    // (measured 20-35 % faster without and 35-40 % faster with a causal mask at head dim 128;
-    // larger ranks spill at 256 registers and keep 64-key tiles at one wave per SIMD)
+    // head dims above 64, aligned, unmasked, rank <= 32: two workgroups per CU (larger ranks spill at 256 registers and
+    // keep one wave per SIMD)
     if constexpr (NKD > 4 && NKR <= 2 && VEC && !MASK)
         return launch_dq_qb<T, NKD, NKR, VEC, MASK, true, FOLD, true>(a, stream);
     return launch_dq_qb<T, NKD, NKR, VEC, MASK, true, FOLD>(a, stream);

@@ -24,40 +24,9 @@ struct FwdWideCfg {
     static constexpr int SK = BN * ROWCH * 8, SKB = BN * CPR * 8, SM = VMASK ? 2 * BN : 0;
     static constexpr int STAGE = 2 * SK + SKB + SM; // elements: K, V, K_b, fp32 vector mask
     static constexpr int LDS_BYTES = 2 * STAGE * 2;
-    static constexpr int KBINST = BN * CPR / 64; // copies that fill the K_b region, one per wave
-    static_assert(KBINST <= NWAVES, "");
     // head dim <= 64: three workgroups per compute unit (168 registers, 3 x 40 KB)
     static constexpr int WAVES_EU = NKD <= 4 ? 3 : 2;
     static __device__ __forceinline__ bool low_parts(const FwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
-};
-
-// K_b rows as a dense region (fb_lean_tiles.h), one copy instruction of waves 0 ... KBINST - 1 per tile.
-template <class C>
-struct FwdWideBias {
-    uint32_t off, row;
-    uint64_t lanes;
-    const uint8_t *p;
-    uint32_t pitch;
-    int wave;
-    __device__ __forceinline__ void init(const FwdArgs &a, const uint16_t *kbbase, int wave_, int lane) {
-        wave = wave_;
-        p = reinterpret_cast<const uint8_t *>(kbbase);
-        pitch = (uint32_t)(a.kb.ss * 2);
-        int r, ch;
-        lean_copy_place<C::CPR>(lane, r, ch);
-        row = wave * (64 / C::CPR) + r;
-        if (C::low_parts(a) && ch == 1) ch = 0; // (the partner of the low parts of q_b / scale)
-        lanes = __builtin_amdgcn_ballot_w64(ch * 8 < a.r);
-        off = row * pitch + ch * 16;
-    }
-    __device__ __forceinline__ void issue(uint32_t lds, int n0, int Lk) {
-        if (wave < C::KBINST) {
-            uint32_t o = off;
-            if (n0 + C::BN > Lk) o -= (uint32_t)max(n0 + (int)row - (Lk - 1), 0) * pitch; // (past the end: the last row again)
-            lds_dma16_lanes(o, p, lds + wave * 1024, lanes);
-        }
-        p += (int64_t)C::BN * pitch;
-    }
 };
 
 template <class T, class C>
@@ -83,7 +52,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     u32x4_t qr[C::NK];
 #pragma unroll
     for (int t = 0; t < C::NKD; ++t) qr[t] = load_chunk<true>(qbase, a.q.ss, query, a.Lq, 16 * t + 8 * g, a.d);
-    FwdWideBias<C> kbd;
+    DenseCopy<C::BN, C::NKR ? C::CPR : 2> kbd; // K_b rows, one copy instruction of the first waves per tile
     if constexpr (C::NKR > 0) {
         const uint16_t *qbbase = a.qb.ptr + b * a.qb.sb + h * a.qb.sh;
         const bool low = C::low_parts(a) && g == 1;
@@ -93,7 +62,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             if (C::FOLD && a.scale != 1.f) x = fold_scale_chunk<T>(x, 1.f / a.scale, C::low_parts(a), low);
             qr[C::NKD + t] = x;
         }
-        kbd.init(a, a.kb.ptr + b * a.kb.sb + h * a.kb.sh, wave, lane);
+        kbd.init(a.kb.ptr + b * a.kb.sb + h * a.kb.sh, a.kb.ss, a.r, C::low_parts(a), wave, lane, 0);
     }
     f32x16_t acc_o[C::NDV];
 #pragma unroll
@@ -141,11 +110,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     wait_vmcnt<0>();
     barrier_lds();
 
-    int turn = __builtin_amdgcn_readfirstlane(cu_slot());
     for (int it = 0; it < ntiles; ++it) {
         const int cur = it & 1, n0 = it * C::BN;
         const bool more = it + 1 < ntiles;
-        take_turn(turn, a.slots);
         if (more) {
             issue(cur ^ 1, n0 + C::BN);
             if constexpr (C::VMASK) load_vmask(n0 + C::BN);
@@ -154,6 +121,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         const uint8_t *sKb = reinterpret_cast<const uint8_t *>(sV + C::SK);
         // (a tile hidden from every query of this wave: so are all later ones, but the copies and barriers go on)
         if (!(a.causal && n0 > wq0 + 31) && wq0 < a.Lq) {
+            // (the wave that feeds the matrix pipe goes first, its neighbour's exponentials fill the gaps: 2-3 % over taking
+            // turns by tile, causal B4 H32 L=4096 d128 646 -> 628 us)
+            __builtin_amdgcn_s_setprio(1);
             f32x16_t s[C::KBLK];
 #pragma unroll
             for (int kb = 0; kb < C::KBLK; ++kb)
@@ -206,6 +176,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                         if (key >= a.Lk || (a.causal && key > query)) s[kb][v] = -INFINITY;
                     }
             }
+            __builtin_amdgcn_s_setprio(0);
             float mx = s[0][0];
 #pragma unroll
             for (int kb = 0; kb < C::KBLK; ++kb)
@@ -270,7 +241,6 @@ static hipError_t launch_fwd_wide(const FwdArgs &a0, hipStream_t stream) {
     const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
     if (e != hipSuccess) return e;
     const int64_t total = (int64_t)a.ntiles_m * a.B * a.H;
-    a.slots = slots_per_cu(kern, C::NTHREADS, C::LDS_BYTES, total, once);
     return launch_flat(kern, total, C::NTHREADS, C::LDS_BYTES, stream, a);
 }
 

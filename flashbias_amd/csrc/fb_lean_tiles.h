@@ -147,6 +147,71 @@ struct LeanCopy2 {
 // argument arrives in vector registers, which would make every value loaded through it look
 // divergent (vector loads, no scalar operands for the copy instructions); made wave-uniform again
 // and typed as constant memory it is read with scalar loads like the kernel's own copy.
+// Copies of a dense region of ROWS rows x CPR chunks (CPR = 2 or 4: a factor of rank up to 16 or 32) by the first
+// waves of a workgroup, one instruction each; lanes whose chunk is channel padding stay off (the region is cleared
+// once), and with `twice` chunk 1 is a second copy of chunk 0 (fold_scale_chunk).  Row strides below 2^24 elements.
+template <int ROWS, int CPR>
+struct DenseCopy {
+    static constexpr int NINST = ROWS * CPR / 64;
+    uint32_t off, row, pitch;
+    uint64_t lanes;
+    const uint8_t *p; // first row of the next tile
+    int wave;
+    __device__ __forceinline__ void init(const uint16_t *base, int64_t ld, int ncols, bool twice, int wave_, int lane, int r0) {
+        wave = wave_;
+        pitch = (uint32_t)(ld * 2);
+        p = reinterpret_cast<const uint8_t *>(base) + (int64_t)r0 * pitch;
+        int r, ch;
+        lean_copy_place<CPR>(lane, r, ch);
+        row = wave * (64 / CPR) + r;
+        if (twice && ch == 1) ch = 0;
+        lanes = __builtin_amdgcn_ballot_w64(ch * 8 < ncols);
+        off = row * pitch + ch * 16;
+    }
+    // Rows [r0, r0 + ROWS), past the end the last one again, and on to the tile after them.
+    __device__ __forceinline__ void issue(uint32_t lds, int r0, int nrows) {
+        if (wave < NINST) {
+            uint32_t o = off;
+            if (r0 + ROWS > nrows) o -= (uint32_t)max(r0 + (int)row - (nrows - 1), 0) * pitch;
+            lds_dma16_lanes(o, p, lds + wave * 1024, lanes);
+        }
+        p += (int64_t)ROWS * pitch;
+    }
+};
+
+// Column-wise A operand of a dense region for a B operand in C layout: rows [row0, row0 + 16), columns [0, 32) (CPR = 2:
+// columns 0 ... 15, repeated), lean_tr_addr4 / lean_tr_addr2 for any row0 that is a multiple of 16.
+template <int CPR>
+__device__ __forceinline__ u32x4_t dense_read_a_tr(const uint8_t *region, int row0, int c, int g) {
+    const uint8_t *base = region + (row0 & ~31) * CPR * 16;
+    if constexpr (CPR == 4) {
+        const uint8_t *step = base + (row0 & 16) * 64;
+        return lean_read_tr(step + lean_tr_addr4(c, g, 0), step + lean_tr_addr4(c, g, 1));
+    } else {
+        const int t = (row0 >> 4) & 1;
+        return lean_read_tr(base + lean_tr_addr2(c, g, 0, t), base + lean_tr_addr2(c, g, 1, t));
+    }
+}
+
+// Reads of a swizzled tile with 16 chunks per row (swz_off<16>) from one address register per access pattern: the chunk of
+// contraction step t, or of column block n, differs from the first one's in address bits that are XORed in, one
+// vector instruction a read, where one register for each of the 8 + 8 addresses costs a kernel its last ones (what
+// the compiler keeps if it may; the values are made opaque where they are formed).
+struct TileAddr16 {
+    uint32_t row, tr;
+    __device__ __forceinline__ TileAddr16(uint32_t tile, int c, int g) {
+        const int r = 4 * g + ((c & 15) >> 2), chunk = 2 * (c >> 4) + ((c & 3) >> 1);
+        row = tile + c * 256 + ((g ^ swz_of<16>(c)) << 4);
+        tr = tile + r * 256 + ((chunk ^ swz_of<16>(r)) << 4) + 8 * (c & 1);
+    }
+    // chunk 2 t + g of row c of the 32 rows that start at byte `at` of the tile
+    __device__ __forceinline__ u32x4_t load_row(int t, int at) const { return lds_load16((row ^ (uint32_t)(32 * t)) + at); }
+    // lds_read_a_tr<16> for the 16 rows that start at byte `at`, columns [32 n, 32 n + 32)  (row + 8: swizzle bit 1)
+    __device__ __forceinline__ u32x4_t load_tr(int n, int at) const {
+        return lds_load_tr((tr ^ (uint32_t)(64 * n)) + at, (tr ^ (uint32_t)(64 * n + 32)) + at + 8 * 256);
+    }
+};
+
 template <class A>
 __device__ __forceinline__ A uniform_kernargs(const void *p) {
     static_assert(sizeof(A) % 4 == 0, "");
