@@ -47,7 +47,7 @@ struct DqCfg {
     static constexpr int QBLK = (QB2_ && NK <= 3 && !MASK_) ? 2 : 1; // the mask values need the registers of the second block
     static constexpr int BM = NWAVES * QBLK * 32;
     static constexpr int KBLK = 2, BN = 32 * KBLK;
-    static constexpr int UNROLL = SPLIT ? 1 : KBLK;
+    static constexpr int UNROLL = SPLIT ? 1 : KBLK; // key blocks computed together
     static constexpr bool ONECHAIN = SPLIT_ && !MASK_; // scale between the d steps and the r steps of one MFMA chain
     // sK row: [K | K_b] of one key in ROWCH swizzled 16-byte chunks; the one copy is read
     // row-wise for S^T and column-wise for [dQ | dQ_b]^T
@@ -168,9 +168,11 @@ struct DqDirect {
         k.issue(base, n0, Lk, a.k.ss, C::NKR > 0 ? a.kb.ss : 0, 2 * C::NKD);
         if constexpr (C::SKB > 0) kb.issue(base + 2 * (C::SK + C::SV), n0, Lk);
         v.issue(base + 2 * C::SK, n0, Lk, a.v.ss, 0, C::ROWCHV);
-        if constexpr (C::MTILE) { // full tiles only: a ragged last tile takes the element path
+        if constexpr (C::MTILE) { // (a ragged last tile: the columns that exist; the others' scores are set to -inf)
             if (mtile && n0 + C::BN <= Lk)
                 m.issue_step(base + 2 * (C::SK + C::SV), m0_, a.Lq, a.mask.sm, 0, C::MROWCH, 2 * C::BN, 0);
+            else if (mtile)
+                m.issue_cols(base + 2 * (C::SK + C::SV), m0_, a.Lq, a.mask.sm, Lk - n0);
         }
     }
     int m0_ = 0; // first query of the workgroup (set by init_mask)
@@ -410,8 +412,11 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
         const bool visible = !(a.causal && n0 > wq0 + 32 * C::QBLK - 1) && wq0 < a.Lq;
         if (visible) {
             // (head dims above 64: one block at a time, two at once would spill)
-#pragma unroll C::UNROLL
-            for (int kb = 0; kb < C::KBLK; ++kb) {
+#pragma unroll 1
+            for (int ko = 0; ko < C::KBLK; ko += C::UNROLL)
+#pragma unroll
+            for (int ki = 0; ki < C::UNROLL; ++ki) {
+                const int kb = ko + ki;
                 TileAddr16 ta(lds_addr_of(sK) + kb * (32 * 256), c, g); // (SPLIT; the V tile follows at + 2 SK)
                 if constexpr (C::SPLIT) asm volatile("" : "+v"(ta.row), "+v"(ta.tr));
                 if (C::UNROLL == 1 && a.causal && n0 + kb * 32 > wq0 + 31) break; // hidden from every query of this wave
@@ -443,7 +448,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
                     if constexpr (C::NKR > 0 || C::MASK) {
                         f32x16_t sb;
                         if constexpr (C::MASK) {
-                            if (C::MTILE && direct.mtile && n0 + C::BN <= a.Lk) {
+                            if (C::MTILE && direct.mtile) {
                                 // this lane's query row of the staged tile, keys in C-layout order
                                 const uint16_t *sM = sV + C::SV;
                                 const int row = wave * 32 + c;

@@ -93,7 +93,9 @@ constexpr int kNoMask = 0, kVectorMask = 1, kMatrixMask = 2;
 
 // Element offset of the mask of one (batch, head).
 __device__ __forceinline__ int64_t mask_offset(const MaskDesc &m, int b, int h) {
-    return (m.batches > 0 ? b % m.batches : b) * m.sb + h * m.sh;
+    int e = b; // (wave-uniform; the remainder is computed in vector registers and would take the mask's addresses there)
+    if (m.batches > 0) e = __builtin_amdgcn_readfirstlane(b % m.batches);
+    return e * m.sb + h * m.sh;
 }
 
 // Eight consecutive channels [col0, col0 + 8) of row `row` of a (rows x ncols) matrix with row
@@ -336,6 +338,18 @@ struct TileDma {
     // after it.  lda / ldb as given to init(); all lanes of the wave must be active.
     __device__ __forceinline__ void issue(uint32_t lds_tile, int r0, int nrows, int64_t lda, int64_t ldb, int split) {
         issue_step(lds_tile, r0, nrows, lda, ldb, split, lda * (2 * ROWS), ldb * (2 * ROWS));
+    }
+
+    // A tile of which only the first `cols` channels (a multiple of 8) exist, the last one of a sequence that runs along the
+    // rows of tensor A; the chunks past them are not copied and keep what an earlier tile left there.
+    __device__ __forceinline__ void issue_cols(uint32_t lds_tile, int r0, int nrows, int64_t lda, int cols) {
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            const int p = (wave * NI + j) * 64 + lane;
+            const int r = p / ROWCH, chunk = (p % ROWCH) ^ swz_of<ROWCH>(r);
+            const uint32_t o = off[j] - (uint32_t)max(r0 + r - (nrows - 1), 0) * (uint32_t)(lda * 2);
+            lds_dma16_lanes(o, pa, lds_tile + (wave * NI + j) * 1024, lanes_a[j] & __builtin_amdgcn_ballot_w64(chunk * 8 < cols));
+        }
     }
 
     // The same with the byte distance to the next tile given by the caller (a sequence of tiles

@@ -329,17 +329,26 @@ __device__ __forceinline__ void fwd_body(const FwdArgs &a) {
             ld.load_safe(stg, a, kbase, kbbase, vbase, n0, tid);
     };
     // Masked, aligned instantiations: a 16-bit matrix mask whose rows allow 16-byte copies travels
-    // as a BM x BN tile straight into LDS, one tile ahead like K and V (full key tiles only; a
-    // ragged last tile and every other kind of mask take the loads of mask_block_keys).
+    // as a BM x BN tile straight into LDS, one tile ahead like K and V (every other kind of mask takes the loads of
+    // mask_block_keys).
     TileDma<C::BM, C::MROWCH, C::NWAVES, false> mdma;
     bool mtile = false;
+    // (a ragged last tile has its existing columns copied; the scores of the others are set to -inf below.  While such
+    // tiles took mask_block_keys, windows of 144 tokens cost as much as windows of 256)
+    auto issue_mask = [&](int buf, int n0) {
+        const uint32_t dst = lds_addr_of(sMbuf + buf * C::SM_ELEMS);
+        if (n0 + C::BN <= a.Lk)
+            mdma.issue_step(dst, m0, a.Lq, a.mask.sm, 0, C::MROWCH, 2 * C::BN, 0);
+        else
+            mdma.issue_cols(dst, m0, a.Lq, a.mask.sm, a.Lk - n0);
+    };
     if constexpr (C::MTILE) {
         static_assert(C::QB == 1, "one query block per wave in masked instantiations");
         if (a.mask.vec_ok && !a.mask.is_f32 && a.Lk % 8 == 0 && a.mask.sm % 8 == 0 &&
             a.mask.sm < (1 << 24) && reinterpret_cast<uintptr_t>(mbase) % 16 == 0) {
             mtile = true;
             mdma.init(reinterpret_cast<const uint16_t *>(mbase), a.mask.sm, C::BN, C::MROWCH, nullptr, 0, 0, wave, lane, m0);
-            if (C::BN <= a.Lk) mdma.issue_step(lds_addr_of(sMbuf), m0, a.Lq, a.mask.sm, 0, C::MROWCH, 2 * C::BN, 0);
+            issue_mask(0, 0);
         }
     }
     // Vector mask: thread `tid` carries the value of key n0 + tid of the tile that follows.
@@ -369,9 +378,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs &a) {
         const int n0 = it * C::BN;
         const bool more = it + 1 < ntiles_k;
         if constexpr (C::MTILE) {
-            if (mtile && more && n0 + 2 * C::BN <= a.Lk)
-                mdma.issue_step(lds_addr_of(sMbuf + (cur ^ 1) * C::SM_ELEMS), m0, a.Lq, a.mask.sm, 0, C::MROWCH,
-                                2 * C::BN, 0);
+            if (mtile && more) issue_mask(cur ^ 1, n0 + C::BN);
         }
         if (more) load_tile(st, n0 + C::BN);
         if constexpr (C::VMASK) {
@@ -420,7 +427,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs &a) {
                 if constexpr (C::XMASK) {
                     const uint8_t *mrow = mbase + (a.mask.type == 2 ? (int64_t)min(query, a.Lq - 1) * a.mask.sm : 0) *
                                                       (a.mask.is_f32 ? 4 : 2);
-                    if (C::MTILE && mtile && n0 + C::BN <= a.Lk) {
+                    if (C::MTILE && mtile) {
                         // this lane's query row of the staged tile, keys in C-layout order
                         const uint16_t *sM = sMbuf + cur * C::SM_ELEMS;
                         const int row = wave * 32 + c;
