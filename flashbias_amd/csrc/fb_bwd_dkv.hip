@@ -62,10 +62,10 @@ struct DkvCfg {
     // memory load whose wait also waits for the tile copies in flight.  B2 H8 L=4096 d128 r8, whole backward with the
     // dq kernel's: 652 -> 566 us; causal B4 H32: 2714 -> 2510 us
     static constexpr bool SPLIT = VEC_ && !XMASK && PART_ != 0 && NKR_ <= 2;
-    static constexpr int UNROLL = SPLIT && DO_DK ? 1 : 2;
     static constexpr int KBW = 1; // key blocks per wave
     static constexpr int BN = 32 * KBW * NWAVES;              // keys per workgroup
     static constexpr int QBLK = PART_ == 0 || SPLIT ? 2 : 1, BMQ = 32 * QBLK; // queries per step
+    static constexpr int UNROLL = SPLIT && DO_DK ? 1 : QBLK; // query blocks computed together
     // sQ row: [Q | Q_b] of one query, sdO row: dout of one query, both in swizzled 16-byte
     // chunks; each tile is kept once and read row-wise (S, dP) and column-wise (dK, dV)
     static constexpr int ROWCH = SPLIT ? 2 * NKD : 2 * NK <= 8 ? 8 : 2 * NK <= 16 ? 16 : 32;
@@ -491,8 +491,11 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
         const bool visible = !(a.causal && wk0 > m0 + C::BMQ - 1) && wk0 < a.Lk;
         if (visible) {
             // ([dK | dK_b] at head dims above 64: one block at a time, two at once would spill)
-#pragma unroll C::UNROLL
-            for (int qb = 0; qb < C::QBLK; ++qb) {
+#pragma unroll 1
+            for (int qo = 0; qo < C::QBLK; qo += C::UNROLL)
+#pragma unroll
+            for (int qi = 0; qi < C::UNROLL; ++qi) {
+                const int qb = qo + qi;
                 TileAddr16 ta(lds_addr_of(sQ) + qb * (32 * 256), c, g); // (SPLIT; the dO tile follows at + 2 SQ)
                 if constexpr (C::SPLIT) asm volatile("" : "+v"(ta.row), "+v"(ta.tr));
                 if (C::UNROLL == 1 && C::QBLK > 1 && a.causal && wk0 > m0 + qb * 32 + 31) continue; // hidden from every key of this wave
@@ -539,10 +542,12 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
                     if constexpr (C::XMASK) {
                         if (mtile) { // column `key`, rows in C-layout order: four transposing reads
                             if constexpr (C::MTILE) {
-                                const int col = (wave * C::KBW + kb) * 32 + 16 * (c >> 4) + 4 * (c & 3);
+                                int cm = c; // (the addresses are formed here: kept across the loop they cost the last registers)
+                                asm volatile("" : "+v"(cm));
+                                const int col = (wave * C::KBW + kb) * 32 + 16 * (cm >> 4) + 4 * (cm & 3);
 #pragma unroll
                                 for (int j = 0; j < 4; ++j) {
-                                    const int row = qb * 32 + 8 * j + 4 * g + ((c & 15) >> 2);
+                                    const int row = qb * 32 + 8 * j + 4 * g + ((cm & 15) >> 2);
                                     const u32x2_t x = lds_read_tr4(sM + swz_off<C::MROWCH>(row, col >> 3) + (col & 7));
                                     mval[4 * j + 0] = T::to_float((uint16_t)(x[0] & 0xffffu));
                                     mval[4 * j + 1] = T::to_float((uint16_t)(x[0] >> 16));

@@ -31,9 +31,13 @@
 namespace fb {
 
 // NKR_: 16-wide steps of the rank (0, 1, 2).  FOLD_: the scores are scale * (q k^T + q_b k_b^T), no multiply per
-// score for the scale (no factors, or a scale of exactly 1).  BG_: also form dq_bias and dk_bias.
-template <class T, int NKR_, bool FOLD_, bool BG_>
+// score for the scale (no factors, or a scale of exactly 1).  BG_: also form dq_bias and dk_bias.  MASK_: an additive
+// mask of the 16-bit type.  A vector mask is one value per lane (key).  A matrix mask's 32 x 32 block is read element-wise, lane = key and register = query (a load instruction
+// asks for two 64-byte row pieces, and the heads of a window meet in one L2), requested as soon as the block before it
+// has used its 16 registers: there is no LDS left for a tile, and the copies are 1024 of a window's 34000 cycles.
+template <class T, int NKR_, bool FOLD_, bool BG_, int MASK_>
 struct WinCfg {
+    static constexpr bool MASK = MASK_ == kMatrixMask, VMASK = MASK_ == kVectorMask;
     static constexpr int NKD = 2, NKR = NKR_, NK = NKD + NKR_, NDV = 1, KBW = 1;
     static constexpr bool FOLD = FOLD_, BG = BG_ && NKR_ > 0, VEC = true, DO_DV = true, DO_DK = true;
     static constexpr int NWAVES = 8, NTHREADS = 64 * NWAVES;
@@ -201,6 +205,29 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
         // statistics were requested during the previous window (or above); every wave has left the previous window's
         // [K | K_b] and dS tiles and its statistics (the barrier that ends a step).
         const bool next = bi + 1 < group && b + 1 < a.B;
+        uint16_t mraw[C::MASK ? 16 : 1]; // mask values of the next block
+        const uint8_t *mbase = nullptr;
+        uint32_t moff = 0;
+        auto request_mask = [&](int r0) { // (register v: query r0 + 8 (v / 4) + 4 g + v % 4)
+            if (r0 + 32 <= a.Lq) {
+#pragma unroll
+                for (int v = 0; v < (C::MASK ? 16 : 1); ++v)
+                    mraw[v] = *reinterpret_cast<const uint16_t *>(mbase + (int64_t)(r0 + 8 * (v >> 2) + (v & 3)) * a.mask.sm * 2 + moff);
+            } else { // queries past the end read the last row
+#pragma unroll
+                for (int v = 0; v < (C::MASK ? 16 : 1); ++v)
+                    mraw[v] = *reinterpret_cast<const uint16_t *>(
+                        mbase + ((int64_t)min(r0 + 8 * (v >> 2) + 4 * g + (v & 3), a.Lq - 1) * a.mask.sm + min(key, a.Lk - 1)) * 2);
+            }
+        };
+        float mkey = 0.f; // vector mask: the value of this lane's key
+        if constexpr (C::VMASK)
+            mkey = T::to_float(reinterpret_cast<const uint16_t *>(a.mask.ptr)[mask_offset(a.mask, b, h) + min(key, a.Lk - 1)]);
+        if constexpr (C::MASK) {
+            mbase = reinterpret_cast<const uint8_t *>(a.mask.ptr) + mask_offset(a.mask, b, h) * 2;
+            moff = (uint32_t)(4 * g * a.mask.sm + min(key, a.Lk - 1)) * 2;
+            if (visible) request_mask(0);
+        }
         const int bn = __builtin_amdgcn_readfirstlane(b + 1);
         // Everything requested for this window has landed (what this waits for beyond that are the few stores of the
         // previous window's last step).
@@ -277,14 +304,18 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
                         }
                     }
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) s[v] = 0.f;
+                    for (int v = 0; v < 16; ++v) s[v] = C::FOLD ? (C::MASK ? T::to_float(mraw[C::MASK ? v : 0]) : C::VMASK ? mkey : 0.f) : 0.f;
 #pragma unroll
                     for (int t = 0; t < C::NKD; ++t) s = T::mfma(qa[t], kreg[t], s);
 #pragma unroll
                     for (int t = 0; t < C::NKD; ++t) dp = T::mfma(da[t], vreg[t], dp);
                     if constexpr (!C::FOLD) { // the softmax scale multiplies q k^T only (flash_bias_triton.py:248)
 #pragma unroll
-                        for (int v = 0; v < 16; ++v) s[v] *= a.scale;
+                        for (int v = 0; v < 16; ++v)
+                            s[v] = C::MASK ? __builtin_fmaf(s[v], a.scale, T::to_float(mraw[C::MASK ? v : 0])) : C::VMASK ? __builtin_fmaf(s[v], a.scale, mkey) : s[v] * a.scale;
+                    }
+                    if constexpr (C::MASK) {
+                        if (r0 + 32 < a.Lq) request_mask(r0 + 32);
                     }
 #pragma unroll
                     for (int t = C::NKD; t < C::NK; ++t) s = T::mfma(qa[t], kreg[t], s);
@@ -385,9 +416,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
     }
 }
 
-template <class T, int NKR, bool FOLD, bool BG>
+template <class T, int NKR, bool FOLD, bool BG, int MASK>
 static hipError_t launch_win_cfg(const BwdArgs &a, hipStream_t stream) {
-    typedef WinCfg<T, NKR, FOLD, BG> C;
+    typedef WinCfg<T, NKR, FOLD, BG, MASK> C;
     auto kern = bwd_win_kernel<T, C>;
     static KernelOnce once;
     const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
@@ -404,12 +435,20 @@ static hipError_t launch_win_cfg(const BwdArgs &a, hipStream_t stream) {
     return launch_flat(kern, (int64_t)((a.B + group - 1) / group) * a.H, C::NTHREADS, C::LDS_BYTES, stream, b);
 }
 
+template <class T, int NKR, int MASK>
+static hipError_t launch_win_m(const BwdArgs &a, bool fold, bool bg, hipStream_t stream) {
+    if (fold) return bg ? launch_win_cfg<T, NKR, true, true, MASK>(a, stream) : launch_win_cfg<T, NKR, true, false, MASK>(a, stream);
+    return bg ? launch_win_cfg<T, NKR, false, true, MASK>(a, stream) : launch_win_cfg<T, NKR, false, false, MASK>(a, stream);
+}
+
 template <class T, int NKR>
 static hipError_t launch_win_r(const BwdArgs &a, hipStream_t stream) {
-    const bool fold = a.r == 0 || a.scale == 1.f;
     const bool bg = NKR > 0 && a.dqb.ptr;
-    if (fold) return bg ? launch_win_cfg<T, NKR, true, true>(a, stream) : launch_win_cfg<T, NKR, true, false>(a, stream);
-    return bg ? launch_win_cfg<T, NKR, false, true>(a, stream) : launch_win_cfg<T, NKR, false, false>(a, stream);
+    switch (a.mask.type) {
+    case kNoMask: return launch_win_m<T, NKR, kNoMask>(a, a.r == 0 || a.scale == 1.f, bg, stream);
+    case kVectorMask: return launch_win_m<T, NKR, kVectorMask>(a, a.scale == 1.f, bg, stream); // (the mask is not divided by the scale)
+    default: return launch_win_m<T, NKR, kMatrixMask>(a, a.scale == 1.f, bg, stream);
+    }
 }
 
 // Compiled once per element type for head dim 32 (see Makefile).  When fb_bwd takes this path is decided by

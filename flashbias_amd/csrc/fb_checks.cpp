@@ -78,7 +78,9 @@ int fb_suggest_bias_grad_group(const fb_params *p) {
     // compute unit by itself and pays for every start with an LDS clear and a first window whose loads nothing
     // overlaps (about 4.6 us: 4096 x 16 windows 5.33 ms ungrouped, 4.29 in groups of 8): groups of up to 32 there,
     // as long as four workgroups per compute unit remain.
-    const bool window = p->d == 32 && p->r % 8 == 0 && p->r <= 32 && p->Lq <= 256 && p->Lk <= 256 && !p->causal && p->mask_type == 0;
+    const bool window = p->d == 32 && p->r % 8 == 0 && p->r <= 32 && p->Lq <= 256 && p->Lk <= 256 && !p->causal &&
+                        (p->mask_type == FB_MASK_NONE || p->mask_dtype == p->dtype) &&
+                        (p->Lq > 128 || p->Lk > 128 || p->mask_type == FB_MASK_VECTOR);
     for (int g = window ? 32 : 8; g > 1; g /= 2)
         if (((int64_t)p->B + g - 1) / g * p->H * ((lmin + 255) / 256) >= 1024) return g;
     return 1;

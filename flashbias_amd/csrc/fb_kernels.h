@@ -132,13 +132,18 @@ inline bool mixed_general_backward(const BwdArgs &a0);
 
 // Whether fb_bwd runs the window kernel (fb_bwd_win.hip: one workgroup per (batch, head) forms the per-query
 // statistics and all five gradients, dq summed inside the workgroup) instead of the dq and dk/dv launches: whole
-// sequences of at most 256 positions, head dim 32, rank a multiple of 8 up to 32, aligned tensors, no additive or
-// causal mask, and at least one workgroup per compute unit (a workgroup fills a compute unit by itself).  Such
+// sequences of at most 256 positions, head dim 32, rank a multiple of 8 up to 32, aligned tensors, no causal
+// mask, no fp32 mask (the mask is read element-wise, any strides), and at least one workgroup per compute unit (a workgroup fills a compute unit by itself).  Such
 // sequences are bound by memory traffic, and the two-kernel backward reads q, k, v, o and dO twice.
+// And sequences of more than one 128-row block: up to there the two kernels read nothing twice either, and most of
+// the window kernel's eight waves have no keys (512 x 16 windows, rank 16, two kernels against this one: 170 / 224 us
+// at 64 positions, 248 / 264 at 96, 290 / 303 at 128, 570 / 411 at 144; with a matrix mask 284 / 412, 450 / 481,
+// 442 / 535, 1188 / 713; with a vector mask, whose dq kernel stages it as a tile, 227 / 231, 346 / 274, 354 / 317, 835 / 422).
 inline bool window_backward(const BwdArgs &a) {
     const int64_t lim = (int64_t)1 << 22; // (32-bit byte offsets of 256 tile rows)
     const int group = a.group > 1 ? a.group : 1;
-    return a.mask.type == 0 && !a.causal && a.d == 32 && a.r % 8 == 0 && a.r <= 32 && a.Lq <= 256 && a.Lk <= 256 &&
+    if (a.Lq <= 128 && a.Lk <= 128 && a.mask.type != kVectorMask) return false;
+    return (a.mask.type == 0 || (!a.mask.is_f32 && a.mask.sm < lim)) && !a.causal && a.d == 32 && a.r % 8 == 0 && a.r <= 32 && a.Lq <= 256 && a.Lk <= 256 &&
            a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.o.vec_ok && a.dout.vec_ok && (a.r == 0 || (a.qb.vec_ok && a.kb.vec_ok)) &&
            a.q.ss < lim && a.k.ss < lim && a.dout.ss < lim && (a.r == 0 || (a.qb.ss < lim && a.kb.ss < lim)) &&
            (int64_t)((a.B + group - 1) / group) * a.H >= num_cus();

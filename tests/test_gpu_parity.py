@@ -235,6 +235,31 @@ def test_wide_heads(gpu_device, d, r, Lq, Lk, scale, dtype):
         _case(gpu_device, 2, Lq, Lk, 3, d, r, dtype, causal, scale=scale, seed=d + r + Lk, o_by_magnitude=True)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind,Lq,Lk,r,scale,shared", [
+    ("matrix", 256, 256, 16, 1.0, True), ("matrix", 144, 144, 16, None, True), ("matrix", 129, 200, 32, None, False),
+    ("matrix", 200, 129, 0, None, False), ("matrix", 131, 250, 8, 1.0, False), ("vector", 64, 64, 16, None, True),
+    ("vector", 256, 130, 32, 1.0, False), ("vector", 49, 250, 0, None, False)])
+def test_window_backward_with_a_mask(gpu_device, monkeypatch, kind, Lq, Lk, r, scale, shared, dtype):
+    """The window backward under an additive mask (-100 as in shifted windows, -inf as in padding; lengths and mask
+    pitches that no 16-byte copy allows, a sliced mask, ragged key tiles of the forward) against the oracle."""
+    from flashbias_amd import interface
+    monkeypatch.setattr(interface, "_FOLD_MIN_PAIRS", 1 << 62)
+    B, H = 66, 4  # more workgroups than compute units
+    q, k, v, qb, kb, do = make_inputs(B, Lq, Lk, H, 32, r, dtype, seed=Lq + Lk + r, bq=(shared, False), bk=(shared, False))
+    if scale == 1.0:
+        q = (q.float() / 6).to(dtype)
+    g = torch.Generator().manual_seed(3)
+    mask = torch.randn(B, 1, Lq if kind == "matrix" else 1, Lk, generator=g)
+    mask[..., Lk - Lk // 5:] = -100.0
+    if kind == "matrix":
+        mask[:, :, Lq // 2:, : Lk // 2] = float("-inf")
+    mask = mask.to(dtype)
+    ref = oracle(q, k, v, qb, kb, mask, False, scale, do)
+    got = run_gpu(flash_bias_func, q, k, v, qb, kb, mask, False, scale, do, gpu_device)
+    _gate(got, ref, dtype, o_by_magnitude=True)
+
+
 def test_very_long_sequence_properties(gpu_device):
     """L = 65536 (too long for the dense oracle): the first 1024 rows of a causal problem do not
     depend on anything behind them, so they must equal the L = 1024 result of the same inputs
