@@ -11,6 +11,7 @@
 // or none; additive mask (B|1, H|1, 1|Lq, Lk) or none.
 #include <torch/extension.h>
 
+#include <ATen/FuncTorchTLS.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -357,10 +358,15 @@ Tensor flash_bias(const Tensor &q_in, const Tensor &k_in, const Tensor &v_in, co
     const Tensor qb = given(q_bias), kb = given(k_bias), m = given(mask);
     TORCH_CHECK(!qb.defined() || kb.defined(), "q_bias without k_bias");
     const double scale = scale_or_default(softmax_scale, q);
-    auto wants = [](const Tensor &x) { return x.defined() && x.requires_grad(); };
-    // nothing to differentiate: no graph node either
-    if (!c10::GradMode::is_enabled() || !(wants(q) || wants(k) || wants(v) || wants(qb) || wants(kb) || wants(m)))
+    // Nothing to differentiate: no graph node either.  What the autograd function refuses stays refused: inputs that
+    // carry a forward-mode tangent (they need not require a gradient, and may do so with gradients off; without the
+    // refusal their derivative would come out as zero) and calls under a function transform (torch.func).
+    const bool grad_mode = c10::GradMode::is_enabled();
+    auto differentiated = [&](const Tensor &x) { return x.defined() && ((grad_mode && x.requires_grad()) || x._fw_grad(/*level=*/0).defined()); };
+    if (!(differentiated(q) || differentiated(k) || differentiated(v) || differentiated(qb) || differentiated(kb) || differentiated(m))) {
+        if (const auto &transforms = at::functorch::functorchTLSAccessor()) transforms->checkSupportsCppAutogradFunction();
         return attend(Call{q, k, v, qb, kb, m, causal, scale, 0}).first;
+    }
     auto maybe = [](const Tensor &x) { return x.defined() ? c10::optional<Tensor>(x) : c10::nullopt; };
     return FlashBiasFn::apply(q, k, v, maybe(qb), maybe(kb), maybe(m), causal, scale);
 }
