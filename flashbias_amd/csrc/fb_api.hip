@@ -2,6 +2,7 @@
 // argument blocks and dispatch to the instantiation that covers (dtype, head dim, rank).  The
 // argument checks themselves (fb_check) are plain C++ in fb_checks.cpp.
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -26,7 +27,7 @@ hipError_t launch_bwd_win_bf16_2(const BwdArgs &a, hipStream_t stream);
 hipError_t launch_bwd_win_f16_2(const BwdArgs &a, hipStream_t stream);
 
 // elementwise part of a cosine-attention window block (fb_cosine.hip)
-hipError_t launch_cosine(const fb_cosine *p, bool backward, hipStream_t stream);
+hipError_t launch_cosine(const fb_cosine *p, bool fp32, bool backward, hipStream_t stream);
 int64_t cosine_sweep(int64_t tokens, int H, int d);
 
 hipError_t launch_fwd(const FwdArgs &a, bool bf16, hipStream_t stream) {
@@ -259,7 +260,8 @@ int fb_alibi_factors(void *q_bias, void *k_bias, int dtype, int Lq, int Lk, int 
 static int check_cosine(const fb_cosine *p, bool backward) {
     fb::api_clear_error();
     if (!p) return fb::api_fail(FB_ERR_NULL, "fb_cosine: null pointer");
-    if (p->size != sizeof(fb_cosine)) return fb::api_fail(FB_ERR_ABI, "fb_cosine.size does not match this library");
+    if (p->size != sizeof(fb_cosine) && p->size != offsetof(fb_cosine, fp32))
+        return fb::api_fail(FB_ERR_ABI, "fb_cosine.size does not match this library");
     if (p->dtype != FB_F16 && p->dtype != FB_BF16) return fb::api_fail(FB_ERR_DTYPE, "only fp16 and bf16 are supported");
     if (p->in_dtype < FB_F16 || p->in_dtype > FB_F32 || p->scale_dtype < FB_F16 || p->scale_dtype > FB_F32)
         return fb::api_fail(FB_ERR_DTYPE, "qkv and logit_scale must be fp16, bf16 or fp32");
@@ -279,6 +281,9 @@ static int check_cosine(const fb_cosine *p, bool backward) {
     return FB_OK;
 }
 
+// (a block that ends before the field was there: 0)
+static bool cosine_fp32(const fb_cosine *p) { return p->size > offsetof(fb_cosine, fp32) && p->fp32 != 0; }
+
 size_t fb_cosine_workspace_bytes(const fb_cosine *p) {
     if (!p || p->tokens <= 0 || p->H <= 0 || p->d < 8) return 0;
     return (size_t)fb::cosine_sweep(p->tokens, p->H, p->d) * p->H * sizeof(float);
@@ -287,13 +292,13 @@ size_t fb_cosine_workspace_bytes(const fb_cosine *p) {
 int fb_cosine_fwd(const fb_cosine *p, void *stream) {
     const int rc = check_cosine(p, false);
     if (rc) return rc;
-    return launched(fb::launch_cosine(p, false, static_cast<hipStream_t>(stream)), "fb_cosine_fwd");
+    return launched(fb::launch_cosine(p, cosine_fp32(p), false, static_cast<hipStream_t>(stream)), "fb_cosine_fwd");
 }
 
 int fb_cosine_bwd(const fb_cosine *p, void *stream) {
     const int rc = check_cosine(p, true);
     if (rc) return rc;
-    return launched(fb::launch_cosine(p, true, static_cast<hipStream_t>(stream)), "fb_cosine_bwd");
+    return launched(fb::launch_cosine(p, cosine_fp32(p), true, static_cast<hipStream_t>(stream)), "fb_cosine_bwd");
 }
 
 int fb_bwd_static(const fb_params *p, void *stream) {

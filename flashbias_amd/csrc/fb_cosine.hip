@@ -11,9 +11,12 @@
 // As tensor operations the same work took about 40 passes over tensors of that size (16 x 64 windows of 256 tokens, 16
 // heads of 32 channels, bf16, forward + backward: 7.4 of the module's 12.9 ms).
 //
-// Rounding: the type of the packed projection is also the type that the tensor operations compute in, which round the
-// norm, the quotient and the product to it one after the other; these kernels do the same, so that q and k are those of
-// the tensor operations.  The backward rounds its results only.
+// Rounding (fb_cosine.fp32 == 0): the type of the packed projection is also the type that tensor operations compute in,
+// which round the norm, the quotient and the product to it one after the other; these kernels do the same, so that q and
+// k are those of the tensor operations.  Under autocast (fb_cosine.fp32 != 0) the projection has 16 bits while tensor
+// operations keep norm, quotient, exponential and product in fp32 and round once, and so do these kernels: with the
+// roundings in between, scaled q would be off by 2.9e-3 instead of 1.7e-3 of its norm, on cosines that the scale
+// multiplies by 10 and more.  The backward rounds its results only.
 #include "flashbias.h"
 #include "fb_kernels.h"
 
@@ -79,48 +82,54 @@ __device__ __forceinline__ float sum_over(float x, int lanes) { // over aligned 
     return x;
 }
 
-template <class SC>
+// FP32: nothing is rounded in between (the bound of the clamp stays a number of the parameter's type).
+template <class X, bool FP32>
+__device__ __forceinline__ float step(float x) {
+    return FP32 ? x : Io<X>::round(x);
+}
+
+template <class SC, bool FP32>
 __device__ __forceinline__ float logit_scale_of(const CosineArgs &a, int h) {
     const float l = Io<SC>::load1(a.logit_scale, h);
-    return Io<SC>::round(expf(fminf(l, Io<SC>::round(kLogitMax))));
+    return step<SC, FP32>(expf(fminf(l, Io<SC>::round(kLogitMax))));
 }
 
 // The unit vector of the lane group's row, rounded as the tensor operations round it; returns what it is divided by.
-template <class IN>
+template <class IN, bool FP32>
 __device__ __forceinline__ float normalise(float (&x)[8], int lanes, float &norm) {
     float s = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) s = __builtin_fmaf(x[e], x[e], s);
-    norm = Io<IN>::round(__builtin_sqrtf(sum_over(s, lanes)));
-    const float denom = fmaxf(norm, Io<IN>::round(kNormEps));
+    norm = step<IN, FP32>(__builtin_sqrtf(sum_over(s, lanes)));
+    const float denom = fmaxf(norm, step<IN, FP32>(kNormEps));
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = Io<IN>::round(x[e] / denom);
+    for (int e = 0; e < 8; ++e) x[e] = step<IN, FP32>(x[e] / denom);
     return denom;
 }
 
 // The product with the scale is formed in the wider of the two types.
-template <class IN, class SC>
+template <class IN, class SC, bool FP32>
 __device__ __forceinline__ float times_scale(float x, float s) {
-    return __is_same(IN, SC) ? Io<IN>::round(x * s) : x * s;
+    return __is_same(IN, SC) ? step<IN, FP32>(x * s) : x * s;
 }
 
-template <class IN, class OUT, class SC>
+template <class IN, class OUT, class SC, bool FP32>
 __global__ __launch_bounds__(256) void cosine_fwd_kernel(const CosineArgs a) {
     const int lanes = a.d / 8, chunks = a.H * lanes;
     const int idx = blockIdx.x * 256 + threadIdx.x, col = idx % chunks, first = idx / chunks;
     if (first >= a.sweep) return;
     const int h = col / lanes;
-    const float s = logit_scale_of<SC>(a, h);
+    const float s = logit_scale_of<SC, FP32>(a, h);
     const int64_t row = (int64_t)a.H * a.d;
     for (int64_t t = first; t < a.tokens; t += a.sweep) {
         float q[8], k[8], v[8], norm;
         Io<IN>::load(a.x, 3 * row * t + 8 * col, q);
         Io<IN>::load(a.x, 3 * row * t + row + 8 * col, k);
         if (a.v) Io<IN>::load(a.x, 3 * row * t + 2 * row + 8 * col, v);
-        normalise<IN>(q, lanes, norm);
-        normalise<IN>(k, lanes, norm);
+        normalise<IN, FP32>(q, lanes, norm);
+        normalise<IN, FP32>(k, lanes, norm);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) q[e] = times_scale<IN, SC>(q[e], s);
+        for (int e = 0; e < 8; ++e) q[e] = times_scale<IN, SC, FP32>(q[e], s);
         Io<OUT>::store(a.q, row * t + 8 * col, q);
         Io<OUT>::store(a.k, row * t + 8 * col, k);
         if (a.v) Io<OUT>::store(a.v, row * t + 8 * col, v);
@@ -139,13 +148,13 @@ __device__ __forceinline__ void project(float (&g)[8], const float (&n)[8], int 
     for (int e = 0; e < 8; ++e) g[e] = (g[e] - n[e] * dot) * inv;
 }
 
-template <class IN, class OUT, class SC>
+template <class IN, class OUT, class SC, bool FP32>
 __global__ __launch_bounds__(256) void cosine_bwd_kernel(const CosineArgs a) {
     const int lanes = a.d / 8, chunks = a.H * lanes;
     const int idx = blockIdx.x * 256 + threadIdx.x, col = idx % chunks, first = idx / chunks;
     if (first >= a.sweep) return;
     const int h = col / lanes;
-    const float s = logit_scale_of<SC>(a, h);
+    const float s = logit_scale_of<SC, FP32>(a, h);
     const int64_t row = (int64_t)a.H * a.d;
     float sum = 0.f;
     for (int64_t t = first; t < a.tokens; t += a.sweep) {
@@ -160,7 +169,7 @@ __global__ __launch_bounds__(256) void cosine_bwd_kernel(const CosineArgs a) {
             Io<OUT>::load(a.dv, from, gv);
             Io<IN>::store(a.dx, at + 2 * row, gv);
         }
-        const float dq = normalise<IN>(q, lanes, qn), dk = normalise<IN>(k, lanes, kn);
+        const float dq = normalise<IN, FP32>(q, lanes, qn), dk = normalise<IN, FP32>(k, lanes, kn);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             sum = __builtin_fmaf(gq[e], q[e], sum);
@@ -175,7 +184,7 @@ __global__ __launch_bounds__(256) void cosine_bwd_kernel(const CosineArgs a) {
     if (col % lanes == 0) a.partial[(int64_t)h * a.sweep + first] = sum;
 }
 
-template <class SC>
+template <class SC, bool FP32>
 __global__ __launch_bounds__(256) void cosine_scale_grad_kernel(const CosineArgs a) {
     __shared__ float part[256];
     const int h = blockIdx.x, tid = threadIdx.x;
@@ -188,7 +197,7 @@ __global__ __launch_bounds__(256) void cosine_scale_grad_kernel(const CosineArgs
     }
     if (tid == 0) {
         const bool inside = Io<SC>::load1(a.logit_scale, h) <= Io<SC>::round(kLogitMax);
-        Io<SC>::store1(a.dlogit_scale, h, inside ? part[0] * logit_scale_of<SC>(a, h) : 0.f);
+        Io<SC>::store1(a.dlogit_scale, h, inside ? part[0] * logit_scale_of<SC, FP32>(a, h) : 0.f);
     }
 }
 
@@ -204,25 +213,30 @@ int64_t cosine_sweep(int64_t tokens, int H, int d) {
     return (int64_t)cosine_blocks(tokens, chunks) * 256 / chunks;
 }
 
-template <class IN, class OUT, class SC>
+template <class IN, class OUT, class SC, bool FP32>
 static hipError_t launch_cosine_t(const CosineArgs &a, bool backward, hipStream_t stream) {
     const int blocks = cosine_blocks(a.tokens, a.H * (a.d / 8));
-    if (!backward) return launch_flat(cosine_fwd_kernel<IN, OUT, SC>, blocks, 256, 0, stream, a);
-    const hipError_t e = launch_flat(cosine_bwd_kernel<IN, OUT, SC>, blocks, 256, 0, stream, a);
+    if (!backward) return launch_flat(cosine_fwd_kernel<IN, OUT, SC, FP32>, blocks, 256, 0, stream, a);
+    const hipError_t e = launch_flat(cosine_bwd_kernel<IN, OUT, SC, FP32>, blocks, 256, 0, stream, a);
     if (e != hipSuccess) return e;
-    return launch_flat(cosine_scale_grad_kernel<SC>, a.H, 256, 0, stream, a);
+    return launch_flat(cosine_scale_grad_kernel<SC, FP32>, a.H, 256, 0, stream, a);
+}
+
+template <class IN, class OUT, class SC>
+static hipError_t launch_cosine_p(const CosineArgs &a, bool fp32, bool backward, hipStream_t stream) {
+    return fp32 ? launch_cosine_t<IN, OUT, SC, true>(a, backward, stream) : launch_cosine_t<IN, OUT, SC, false>(a, backward, stream);
 }
 
 template <class IN, class OUT>
-static hipError_t launch_cosine_s(const CosineArgs &a, int scale_type, bool backward, hipStream_t stream) {
+static hipError_t launch_cosine_s(const CosineArgs &a, int scale_type, bool fp32, bool backward, hipStream_t stream) {
     switch (scale_type) {
-    case FB_F16: return launch_cosine_t<IN, OUT, F16>(a, backward, stream);
-    case FB_BF16: return launch_cosine_t<IN, OUT, BF16>(a, backward, stream);
-    default: return launch_cosine_t<IN, OUT, F32>(a, backward, stream);
+    case FB_F16: return launch_cosine_p<IN, OUT, F16>(a, fp32, backward, stream);
+    case FB_BF16: return launch_cosine_p<IN, OUT, BF16>(a, fp32, backward, stream);
+    default: return launch_cosine_p<IN, OUT, F32>(a, fp32, backward, stream);
     }
 }
 
-hipError_t launch_cosine(const fb_cosine *p, bool backward, hipStream_t stream) {
+hipError_t launch_cosine(const fb_cosine *p, bool fp32, bool backward, hipStream_t stream) {
     CosineArgs a;
     a.x = p->qkv;
     a.logit_scale = p->logit_scale;
@@ -242,9 +256,9 @@ hipError_t launch_cosine(const fb_cosine *p, bool backward, hipStream_t stream) 
     a.sweep = (int)cosine_sweep(p->tokens, p->H, p->d);
     const bool bf16 = p->dtype == FB_BF16;
     switch (p->in_dtype) {
-    case FB_F16: return bf16 ? launch_cosine_s<F16, BF16>(a, p->scale_dtype, backward, stream) : launch_cosine_s<F16, F16>(a, p->scale_dtype, backward, stream);
-    case FB_BF16: return bf16 ? launch_cosine_s<BF16, BF16>(a, p->scale_dtype, backward, stream) : launch_cosine_s<BF16, F16>(a, p->scale_dtype, backward, stream);
-    default: return bf16 ? launch_cosine_s<F32, BF16>(a, p->scale_dtype, backward, stream) : launch_cosine_s<F32, F16>(a, p->scale_dtype, backward, stream);
+    case FB_F16: return bf16 ? launch_cosine_s<F16, BF16>(a, p->scale_dtype, fp32, backward, stream) : launch_cosine_s<F16, F16>(a, p->scale_dtype, fp32, backward, stream);
+    case FB_BF16: return bf16 ? launch_cosine_s<BF16, BF16>(a, p->scale_dtype, fp32, backward, stream) : launch_cosine_s<BF16, F16>(a, p->scale_dtype, fp32, backward, stream);
+    default: return bf16 ? launch_cosine_s<F32, BF16>(a, p->scale_dtype, fp32, backward, stream) : launch_cosine_s<F32, F16>(a, p->scale_dtype, fp32, backward, stream);
     }
 }
 

@@ -12,6 +12,7 @@
 #include <torch/extension.h>
 
 #include <ATen/FuncTorchTLS.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -218,7 +219,7 @@ struct FlashBiasFn : public torch::autograd::Function<FlashBiasFn> {
 // those of the projection.  (As tensor operations: about 40 passes over tensors of that size, and the split of the
 // packed tensor comes back as three zero-filled copies added up.)  `mask` (nW, n, n) or none, one per window of an image.
 struct WindowFn : public torch::autograd::Function<WindowFn> {
-    static fb_cosine cosine(const Tensor &qkv, const Tensor &logit_scale, int64_t heads, c10::ScalarType type) {
+    static fb_cosine cosine(const Tensor &qkv, const Tensor &logit_scale, int64_t heads, c10::ScalarType type, bool autocast) {
         fb_cosine a;
         std::memset(&a, 0, sizeof(a));
         a.size = sizeof(a);
@@ -230,6 +231,7 @@ struct WindowFn : public torch::autograd::Function<WindowFn> {
         a.tokens = qkv.size(0) * qkv.size(1);
         a.qkv = qkv.data_ptr();
         a.logit_scale = logit_scale.data_ptr();
+        a.fp32 = autocast;
         return a;
     }
     // part `which` of a packed tensor, as (windows, n, H, d)
@@ -245,7 +247,9 @@ struct WindowFn : public torch::autograd::Function<WindowFn> {
                         logit_scale.is_cuda() && logit_scale.numel() == heads,
                     "qkv must be a contiguous (windows, n, 3 * heads * headdim) GPU tensor, logit_scale one value per head");
         const int64_t B = qkv.size(0), n = qkv.size(1), d = qkv.size(2) / (3 * heads);
-        fb_cosine a = cosine(qkv, logit_scale, heads, type);
+        // (tensor operations would compute the norm, and with it all that follows, in fp32 there)
+        const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
+        fb_cosine a = cosine(qkv, logit_scale, heads, type, autocast);
         Call c;
         c.q = fresh({B, n, heads, d}, type, qkv.device());
         c.k = fresh({B, n, heads, d}, type, qkv.device());
@@ -271,6 +275,7 @@ struct WindowFn : public torch::autograd::Function<WindowFn> {
         const auto [o, lse] = attend(c);
         ctx->save_for_backward({qkv, logit_scale, c.q, c.k, convert ? c.v : Tensor(), o, lse, qb, kb, c.mask});
         ctx->saved_data["heads"] = heads;
+        ctx->saved_data["autocast"] = autocast;
         return o;
     }
 
@@ -294,7 +299,7 @@ struct WindowFn : public torch::autograd::Function<WindowFn> {
             dv = part(dqkv, 2, heads);
         }
         const auto [dqb, dkb] = attend_backward(c, saved[5], saved[6], grads[0], dq, dk, dv, ctx->needs_input_grad(2) || ctx->needs_input_grad(3));
-        fb_cosine a = cosine(qkv, logit_scale, heads, c.q.scalar_type());
+        fb_cosine a = cosine(qkv, logit_scale, heads, c.q.scalar_type(), ctx->saved_data["autocast"].toBool());
         Tensor dscale = fresh_like(logit_scale);
         Tensor partial = fresh({(int64_t)(fb_cosine_workspace_bytes(&a) / 4)}, torch::kFloat32, qkv.device());
         a.dq = dq.data_ptr();

@@ -231,6 +231,10 @@ typedef struct fb_cosine {
     void *dqkv;              /* bwd out */
     void *dlogit_scale;      /* bwd out, (H) */
     float *partial;          /* bwd scratch of fb_cosine_workspace_bytes() bytes */
+    int32_t fp32;            /* 0: norm, quotient, exponential and product are rounded to the type of their tensors one after
+                                the other, as tensor operations do; else they stay in fp32 and only the results are
+                                rounded, as under autocast.  (A block whose size ends before this field is accepted: 0.) */
+    int32_t reserved;        /* 0 */
 } fb_cosine;
 
 size_t fb_cosine_workspace_bytes(const fb_cosine *p);

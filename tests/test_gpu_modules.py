@@ -1,9 +1,11 @@
 """The one-pass kernels of the module drop-ins (csrc/fb_cosine.hip, the ALiBi factor builder) against the tensor
 operations they replace."""
+import ctypes
+
 import pytest
 import torch
 
-from flashbias_amd import factors, interface, modules
+from flashbias_amd import _lib, factors, interface, modules
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +52,123 @@ def test_window_block_against_tensor_operations(gpu_device, monkeypatch, dtype, 
         else:
             assert (g.float() - w.float()).norm() <= bound * w.float().norm(), name
     assert got[2].flatten()[0] == 0
+
+
+class FbCosine(ctypes.Structure):  # fb_cosine of include/flashbias.h
+    _fields_ = ([("size", ctypes.c_uint32)] + [(n, ctypes.c_int32) for n in ("dtype", "in_dtype", "scale_dtype", "H", "d")]
+                + [("tokens", ctypes.c_int64)] + [(n, ctypes.c_void_p) for n in ("qkv", "logit_scale", "q", "k", "v", "dq", "dk", "dv")]
+                + [("grad_stride", ctypes.c_int64)] + [(n, ctypes.c_void_p) for n in ("dqkv", "dlogit_scale", "partial")]
+                + [("fp32", ctypes.c_int32), ("reserved", ctypes.c_int32)])
+
+
+CODES = {torch.float16: _lib.FB_F16, torch.bfloat16: _lib.FB_BF16, torch.float32: _lib.FB_F32}
+
+
+def _cosine_block(qkv, logit_scale, heads, dtype):
+    a = FbCosine()
+    a.size = ctypes.sizeof(FbCosine)
+    a.dtype, a.in_dtype, a.scale_dtype = CODES[dtype], CODES[qkv.dtype], CODES[logit_scale.dtype]
+    a.H, a.d, a.tokens = heads, qkv.shape[1] // (3 * heads), qkv.shape[0]
+    a.qkv, a.logit_scale = qkv.data_ptr(), logit_scale.data_ptr()
+    return a
+
+
+def _cosine_inputs(dev, in_dtype, scale_dtype, heads, d, tokens=333):
+    g = torch.Generator().manual_seed(4)
+    qkv = (torch.randn(tokens, 3 * heads * d, generator=g) * torch.logspace(-3, 3, tokens, dtype=torch.float32)[:, None]).to(in_dtype)
+    qkv[7] = 0  # rows without a direction
+    scale = (torch.randn(heads, generator=g) * 0.5 + 2.3).to(scale_dtype)
+    scale[0] = 7.0  # clamped
+    return qkv.to(dev), scale.to(dev)
+
+
+def _cosine_exact(qkv, logit_scale, heads):
+    """q, k, v of (tokens, 3 H d) as float64 tensor operations; the clamp's bound is a number of the parameter's type."""
+    x = qkv.double().view(qkv.shape[0], 3, heads, -1)
+    top = torch.tensor(4.6052).to(logit_scale.dtype).double().item()
+    s = logit_scale.double().clamp(max=top).exp()[None, :, None]
+    unit = lambda t: torch.nn.functional.normalize(t, dim=-1)
+    return unit(x[:, 0]) * s, unit(x[:, 1]), x[:, 2]
+
+
+COSINE_TYPES = [(torch.bfloat16, torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.bfloat16, torch.float32),
+                (torch.float16, torch.float16, torch.float32), (torch.float16, torch.bfloat16, torch.float32),
+                (torch.float32, torch.bfloat16, torch.float32), (torch.float32, torch.float16, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("in_dtype,dtype,scale_dtype", COSINE_TYPES)
+@pytest.mark.parametrize("heads,d", [(1, 8), (3, 16), (5, 32), (2, 128)])
+def test_cosine_forward_in_fp32_rounds_once(gpu_device, in_dtype, dtype, scale_dtype, heads, d):
+    """Unit q (times the logit scale) and unit k with fp32 steps are the float64 values rounded once to the attention's
+    type, whatever types the projection and the scale have."""
+    lib = _lib.load()
+    qkv, scale = _cosine_inputs(gpu_device, in_dtype, scale_dtype, heads, d)
+    got = [torch.full((qkv.shape[0], heads, d), float("nan"), device=gpu_device, dtype=dtype) for _ in range(3)]
+    a = _cosine_block(qkv, scale, heads, dtype)
+    a.q, a.k, a.v = (t.data_ptr() for t in got)
+    a.fp32 = 1
+    _lib.check_status(lib.fb_cosine_fwd(ctypes.byref(a), ctypes.c_void_p(interface._stream())))
+    torch.cuda.synchronize()
+    # half a unit in the last place of the result's 8 or 11 significant bits (fp16: subnormals below 2^-14) on top of the
+    # fp32 arithmetic: 8 + log2(d / 8) additions halved by the root, the root, the division, the product, 2 units of exp
+    bits, low = (8, -125) if dtype == torch.bfloat16 else (11, -13)
+    for name, g, w in zip("qkv", got, _cosine_exact(qkv, scale, heads)):
+        half = torch.ldexp(torch.ones_like(w), torch.frexp(w).exponent.clamp(min=low) - 1 - bits)
+        excess = (g.double() - w).abs() - half - w.abs() * 12 * 2.0 ** -24
+        assert (excess <= 0).all(), (name, float((excess / half).max()))
+    assert not got[0][7].any() and not got[1][7].any()
+
+
+class Given(torch.nn.Module):
+    """In the place of a projection: its result."""
+
+    def __init__(self, y):
+        super().__init__()
+        self.y = y
+
+    def forward(self, x):
+        return self.y
+
+
+def _window_core_exact(mod, qkv, logit_scale, heads):
+    """Attention of a window block on its projection, in float64 tensor operations."""
+    windows, n, dim = qkv.shape[0], qkv.shape[1], qkv.shape[2] // 3
+    q, k, v = (t.view(windows, n, heads, dim // heads).transpose(1, 2).contiguous()
+               for t in _cosine_exact(qkv.view(windows * n, -1), logit_scale, heads))
+    bias = mod.q_bias_pos.double()[0].transpose(0, 1) @ mod.k_bias_pos.double()[0].permute(1, 2, 0).contiguous()
+    o = torch.softmax(q @ k.transpose(-1, -2).contiguous() + bias, dim=-1) @ v
+    return o.transpose(1, 2).reshape(windows, n, dim)
+
+
+@pytest.mark.parametrize("dtype,autocast", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16), (torch.bfloat16, torch.float16)])
+@pytest.mark.parametrize("param", [torch.float32, torch.bfloat16])
+def test_window_block_under_autocast(gpu_device, monkeypatch, dtype, autocast, param):
+    """Under torch.autocast the projection comes in 16 bits while norm, quotient, exponential and product are computed in
+    fp32: output and the projection's gradient are no further from float64 than the tensor operations'."""
+    torch.manual_seed(2)
+    window, heads, hd, windows = 8, 4, 32, 16
+    n, dim = window * window, heads * hd
+    mod = modules.WindowAttentionCore(dim, window, heads, rank=8, dtype=dtype).to(gpu_device, param)
+    mod.q_bias_pos, mod.k_bias_pos = mod.q_bias_pos.to(dtype), mod.k_bias_pos.to(dtype)
+    x = torch.randn(windows, n, dim, device=gpu_device, dtype=param)
+    dy = torch.randn(windows, n, dim, device=gpu_device, dtype=param)
+    with torch.no_grad(), torch.autocast("cuda", dtype=autocast):
+        qkv = mod.qkv(x)
+    assert qkv.dtype == autocast
+    qkv.requires_grad_(True)
+    mod.qkv, mod.proj = Given(qkv), torch.nn.Identity()  # (the attention itself)
+
+    def run():
+        with torch.autocast("cuda", dtype=autocast):
+            y = mod(x)
+        return [y.detach().double(), torch.autograd.grad(y, qkv, dy)[0].double()]
+    got = run()
+    monkeypatch.setattr(interface, "_ext", None)
+    ops = run()
+    leaf = qkv.detach().double().requires_grad_(True)
+    y = _window_core_exact(mod, leaf, mod.logit_scale.detach().flatten(), heads)
+    exact = [y.detach(), torch.autograd.grad(y, leaf, dy.double())[0]]
+    for name, g, o, w in zip(("y", "dqkv"), got, ops, exact):
+        error = lambda t: float((t - w).norm() / w.norm())
+        # (131072 and 393216 values with roundings of their own: the two errors are measured to less than 2 %)
+        assert error(g) <= 1.05 * error(o), (name, error(g), error(o))
