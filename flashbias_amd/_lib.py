@@ -31,7 +31,8 @@ class FbParams(ctypes.Structure):
                 + [(n, FbTensor) for n in ("q", "k", "v", "q_bias", "k_bias", "mask", "o")]
                 + [("lse", ctypes.c_void_p)]
                 + [(n, FbTensor) for n in ("dout", "dq", "dk", "dv", "dq_bias", "dk_bias")]
-                + [("delta", ctypes.c_void_p), ("bias_grad_group", ctypes.c_int32), ("mask_batches", ctypes.c_int32)])
+                + [("delta", ctypes.c_void_p), ("bias_grad_group", ctypes.c_int32), ("reserved0", ctypes.c_int32),
+                   ("mask_batches", ctypes.c_int32), ("reserved1", ctypes.c_int32 * 3)])
 
 
 class FlashBiasError(RuntimeError):

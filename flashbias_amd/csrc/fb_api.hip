@@ -123,7 +123,7 @@ fb::MaskDesc dev_mask(const fb_params *p) {
     m.ptr = p->mask_type ? p->mask.ptr : nullptr;
     m.sb = p->mask.stride_b;
     m.sh = p->mask.stride_h;
-    m.batches = p->mask_batches;
+    m.batches = fb::mask_batches(p);
     m.sm = p->mask_type == FB_MASK_MATRIX ? p->mask.stride_s : 0;
     m.type = p->mask_type;
     m.is_f32 = p->mask_dtype == FB_F32;
@@ -306,7 +306,7 @@ int fb_bwd_static(const fb_params *p, void *stream) {
     // fb_params.delta (which is ignored): no allocation, here or in anything it calls.
     fb::api_clear_error();
     if (!p) return fb::api_fail(FB_ERR_NULL, "params: null pointer");
-    if (p->size != sizeof(fb_params)) return fb::api_fail(FB_ERR_ABI, "fb_params.size does not match this library");
+    if (!fb::known_size(p)) return fb::api_fail(FB_ERR_ABI, "fb_params.size does not match this library");
     const size_t need = fb_bwd_workspace_bytes(p);
     if (need == 0) return fb::api_fail(FB_ERR_SHAPE, "B, H, Lq, Lk must be positive");
     if (need > (size_t)FB_STATIC_SCRATCH_BYTES)
@@ -314,7 +314,9 @@ int fb_bwd_static(const fb_params *p, void *stream) {
     hipError_t e = hipSuccess;
     void *ptr = static_scratch(&e);
     if (!ptr) return launched(e, "fb_bwd_static (hipGetSymbolAddress)");
-    fb_params q = *p;
+    fb_params q;
+    std::memset(&q, 0, sizeof(q));
+    std::memcpy(&q, p, p->size); // (which may be smaller)
     q.delta = static_cast<float *>(ptr);
     return fb_bwd(&q, stream);
 }

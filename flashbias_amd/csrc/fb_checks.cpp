@@ -89,7 +89,7 @@ int fb_suggest_bias_grad_group(const fb_params *p) {
 int fb_check(const fb_params *p, int pass) {
     g_err[0] = 0;
     if (!p) return fail(FB_ERR_NULL, "params: null pointer");
-    if (p->size != sizeof(fb_params)) return fail(FB_ERR_ABI, "fb_params.size does not match this library");
+    if (!fb::known_size(p)) return fail(FB_ERR_ABI, "fb_params.size does not match this library");
     if (p->dtype != FB_F16 && p->dtype != FB_BF16) return fail(FB_ERR_DTYPE, "only fp16 and bf16 are supported");
     if (p->B <= 0 || p->H <= 0 || p->Lq <= 0 || p->Lk <= 0) return fail(FB_ERR_SHAPE, "B, H, Lq, Lk must be positive");
     if (p->d <= 0 || p->d > FB_MAX_HEADDIM) return fail(FB_ERR_SHAPE, "head dim must be in 1..128");
@@ -114,7 +114,7 @@ int fb_check(const fb_params *p, int pass) {
         if (p->mask_dtype != p->dtype && p->mask_dtype != FB_F32)
             return fail(FB_ERR_MASK, "mask must have the input dtype or fp32");
         if (!p->mask.ptr) return fail(FB_ERR_NULL, "%s: null pointer", "mask");
-        if (p->mask_batches < 0) return fail(FB_ERR_MASK, "mask_batches must not be negative");
+        if (fb::mask_batches(p) < 0) return fail(FB_ERR_MASK, "mask_batches must not be negative");
         if (p->mask.stride_b < 0 || p->mask.stride_h < 0 || p->mask.stride_s < 0)
             return fail(FB_ERR_STRIDE, "%s: negative stride", "mask");
     }

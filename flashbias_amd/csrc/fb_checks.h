@@ -4,6 +4,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "flashbias.h"
+
 #ifdef __HIPCC__
 #define FB_HOST_DEVICE __host__ __device__
 #else
@@ -14,6 +16,10 @@ namespace fb {
 // Stores the formatted text as the calling thread's last error and returns `code`.
 int api_fail(int code, const char *fmt, ...);
 void api_clear_error();
+
+// Sizes a caller's block may have, and its mask_batches (version 3's block has none; what follows it is the caller's).
+inline bool known_size(const fb_params *p) { return p->size == sizeof(fb_params) || p->size == FB_PARAMS_SIZE_3; }
+inline int mask_batches(const fb_params *p) { return p->size > FB_PARAMS_SIZE_3 ? p->mask_batches : 0; }
 
 // Layout of the backward's scratch buffer, in floats from its (16-byte aligned) start: rows =
 // B * H * Lq values of -delta, rows values of lse * log2(e), and from stat_offset(rows) on one

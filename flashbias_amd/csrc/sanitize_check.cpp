@@ -80,6 +80,19 @@ int main() {
         }
     }
     expect(fb_check(nullptr, 0), FB_ERR_NULL, "null block");
+    for (int pass = 0; pass < 2; ++pass) { // version 3's block with nothing after it, its padding not initialised
+        fb_params p = good(pass);
+        p.size = FB_PARAMS_SIZE_3;
+        p.mask_type = FB_MASK_VECTOR;
+        p.mask_dtype = p.dtype;
+        p.mask.ptr = p.q.ptr;
+        p.reserved0 = -1;
+        std::vector<int64_t> old(FB_PARAMS_SIZE_3 / sizeof(int64_t));
+        std::memcpy(old.data(), &p, FB_PARAMS_SIZE_3);
+        const fb_params *q = reinterpret_cast<const fb_params *>(old.data());
+        expect(fb_check(q, pass), FB_OK, "version 3 block");
+        if (fb_bwd_workspace_bytes(q) == 0 || fb_suggest_bias_grad_group(q) != 1) bad = 1;
+    }
     fb_params p = good(1);
     if (fb_bwd_workspace_bytes(&p) != (size_t)2 * 4 * 128 * (2 * sizeof(float) + 16)) bad = 1; // per query row: two floats, one chunk
     p.B = 0;

@@ -32,7 +32,8 @@
 extern "C" {
 #endif
 
-#define FB_VERSION 3
+/* 4: mask_batches at the end of fb_params (blocks of version 3 are accepted), fb_alibi_factors and fb_cosine_* */
+#define FB_VERSION 4
 #define FB_MAX_HEADDIM 128 /* flash_bias_triton.py:1106 */
 #define FB_MAX_RANK 128
 /* Size of the library-owned scratch buffer used by fb_bwd_static (one copy per GPU, held until the
@@ -47,7 +48,7 @@ typedef enum fb_status {
     FB_ERR_STRIDE = -4,     /* stride would alias gradient rows / negative stride */
     FB_ERR_MASK = -5,       /* bad mask type / dtype */
     FB_ERR_RESERVED = -6,
-    FB_ERR_ABI = -7,        /* fb_params.size does not match this library */
+    FB_ERR_ABI = -7,        /* fb_params.size is none that this library knows */
     FB_ERR_LAUNCH = -8,     /* HIP reported a launch error */
     FB_ERR_SCALE = -9       /* softmax scale not finite or zero (negative scales are accepted) */
 } fb_status;
@@ -66,7 +67,7 @@ typedef struct fb_tensor {
 } fb_tensor;
 
 typedef struct fb_params {
-    uint32_t size; /* sizeof(fb_params) as seen by the caller */
+    uint32_t size; /* sizeof(fb_params) as seen by the caller; FB_PARAMS_SIZE_3, the block of version 3, is taken too */
     int32_t dtype; /* fb_dtype of q, k, v, factors, o and all gradients */
     int32_t B, H, Lq, Lk;
     int32_t d;     /* head dim, 1..128 */
@@ -98,10 +99,15 @@ typedef struct fb_params {
                                    once; the caller reduces the remaining rows.  (The reference accumulates the factor
                                    gradients with atomic adds into fp32 buffers laid out like the factors
                                    themselves, flash_bias_triton.py:1219-1231, :1342.) */
+    int32_t reserved0;          /* not read (padding at the end of version 3's block) */
     int32_t mask_batches;       /* 0: the mask has B batch entries, or one (stride_b = 0).  n > 0: it has n, and batch
                                    entry b takes b % n: the masks of a shifted-window block, one per window of an image,
                                    which the reference repeats over the images (swin_transformer_v2.py:190-203) */
+    int32_t reserved1[3];       /* not read */
 } fb_params;
+
+/* The block of version 3 ends before mask_batches, which is then 0. */
+#define FB_PARAMS_SIZE_3 offsetof(fb_params, mask_batches)
 
 /* Library / ABI version. */
 int fb_version(void);

@@ -25,7 +25,7 @@ def test_library_exports_every_declared_symbol():
     assert declared == set(_lib.EXPORTS)
     for name in declared:
         assert hasattr(lib, name), name
-    assert lib.fb_version() == 3
+    assert lib.fb_version() == 4
 
 
 def test_workspace_size_query():
@@ -93,6 +93,37 @@ def test_check_rejects_forward(mutate, code):
     assert lib.fb_check(p, 0) == code
     assert lib.fb_last_error() != b""
     assert lib.fb_fwd(p, None) == code  # rejected before any launch
+
+
+def _version_3(p, left_over):
+    """The block of a caller compiled against version 3: it ends before mask_batches, and what it ends with is padding
+    that nobody initialised.  Given with nothing after it."""
+    size = _lib.FbParams.mask_batches.offset
+    p.size, p.reserved0 = size, left_over
+    block = (ctypes.c_char * size)()
+    ctypes.memmove(block, ctypes.byref(p), size)
+    return ctypes.cast(block, ctypes.POINTER(_lib.FbParams)), block
+
+
+@pytest.mark.parametrize("left_over", [0, 1, 3, -1])
+@pytest.mark.parametrize("pass_", [0, 1])
+def test_check_accepts_the_block_of_version_3(left_over, pass_):
+    lib = _lib.load()
+    assert _lib.FbParams.mask_batches.offset == 488
+    p = _good(pass_)
+    p.mask_type, p.mask_dtype = _lib.FB_MASK_VECTOR, p.dtype
+    p.mask = _lib.FbTensor(0x10000, 128, 0, 0)
+    old, keep = _version_3(p, left_over)
+    assert lib.fb_check(old, pass_) == 0, lib.fb_last_error()
+    assert lib.fb_bwd_workspace_bytes(old) > 0 and lib.fb_suggest_bias_grad_group(old) == 1
+    # of this version's block every size but its own is refused, as is a negative number of masks
+    for size in (480, 487, 489, 496, ctypes.sizeof(_lib.FbParams) + 8):
+        q = _good(pass_)
+        q.size = size
+        assert lib.fb_check(q, pass_) == -7
+    q = _good(pass_)
+    q.mask_type, q.mask_dtype, q.mask, q.mask_batches = p.mask_type, p.mask_dtype, p.mask, -1
+    assert lib.fb_check(q, pass_) == -5
 
 
 @pytest.mark.parametrize("mutate,code", [
