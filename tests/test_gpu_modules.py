@@ -172,3 +172,38 @@ def test_window_block_under_autocast(gpu_device, monkeypatch, dtype, autocast, p
         error = lambda t: float((t - w).norm() / w.norm())
         # (131072 and 393216 values with roundings of their own: the two errors are measured to less than 2 %)
         assert error(g) <= 1.05 * error(o), (name, error(g), error(o))
+
+
+def _both_ways(monkeypatch, mod, x, mask):
+    """Output and input gradient of the module from the one-pass kernels and from the tensor operations; an error in the
+    place of a result that there is none of."""
+    out = []
+    for ext in (interface._extension(), None):
+        with monkeypatch.context() as m:
+            m.setattr(interface, "_ext", ext)
+            try:
+                y = mod(x, mask)
+                out.append([y.detach().double(), torch.autograd.grad(y.double().square().sum(), x)[0].double()])
+            except (RuntimeError, AssertionError) as e:
+                out.append(e)
+    return out
+
+
+# windows of 16 tokens, 8 of them, 4 to an image; what expands to (4, 16, 16), then what does not
+@pytest.mark.parametrize("shape,accepted", [
+    ((4, 16, 16), True), ((4, 16, 1), True), ((4, 1, 16), True), ((4, 1, 1), True), ((8, 16, 1), True), ((1, 16, 16), True),
+    ((1, 16), True), ((1, 1), True), ((1,), True), ((4, 16), False), ((3, 16, 16), False), ((4, 8, 16), False), ((4, 16, 8), False),
+    ((16, 16, 16), False), ((4, 1, 16, 16), False)])
+def test_window_masks_that_broadcast(gpu_device, monkeypatch, shape, accepted):
+    torch.manual_seed(3)
+    mod = modules.WindowAttentionCore(64, 4, 2, rank=8).to(gpu_device)
+    x = torch.randn(8, 16, 64, device=gpu_device, requires_grad=True)
+    mask = torch.randn(shape, device=gpu_device) * 2
+    one, ops = _both_ways(monkeypatch, mod, x, mask)
+    if not accepted:
+        assert isinstance(one, Exception) and isinstance(ops, Exception)
+        return
+    for name, a, b in zip(("y", "dx"), one, ops):
+        # (fp32 projection: q and k differ by the last bit where fp32 sums in another order fall on the other side of a
+        # rounding, P and dS by 2^-9 relative; outputs rounded to bf16)
+        assert (a - b).norm() <= 2.0 ** -7 * b.norm(), name
