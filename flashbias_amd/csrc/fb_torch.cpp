@@ -243,9 +243,6 @@ struct WindowFn : public torch::autograd::Function<WindowFn> {
     static Tensor forward(AutogradContext *ctx, const Tensor &qkv, const Tensor &logit_scale, const Tensor &qb, const Tensor &kb,
                           const c10::optional<Tensor> &mask_in, int64_t heads, int64_t dtype) {
         const auto type = (c10::ScalarType)dtype;
-        TORCH_CHECK(qkv.dim() == 3 && qkv.is_contiguous() && qkv.is_cuda() && qkv.size(2) % (3 * heads) == 0 && logit_scale.is_contiguous() &&
-                        logit_scale.is_cuda() && logit_scale.numel() == heads,
-                    "qkv must be a contiguous (windows, n, 3 * heads * headdim) GPU tensor, logit_scale one value per head");
         const int64_t B = qkv.size(0), n = qkv.size(1), d = qkv.size(2) / (3 * heads);
         // (tensor operations would compute the norm, and with it all that follows, in fp32 there)
         const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
@@ -317,10 +314,20 @@ struct WindowFn : public torch::autograd::Function<WindowFn> {
     }
 };
 
-Tensor window_attention(const Tensor &qkv, const Tensor &logit_scale, const Tensor &qb, const Tensor &kb, const c10::optional<Tensor> &mask,
-                        int64_t heads, py::object dtype) {
-    return WindowFn::apply(qkv, logit_scale, channel_contiguous(qb), channel_contiguous(kb), mask, heads,
-                           (int64_t)torch::python::detail::py_object_to_dtype(dtype));
+// The attention core on what its kernels take, else nothing: the caller then runs the tensor operations, which take the
+// rest (float64 parameters, a projection that is not packed in 16-byte aligned rows, other head dims and ranks) and say
+// what is wrong with what nobody takes.
+c10::optional<Tensor> window_attention(const Tensor &qkv, const Tensor &logit_scale, const Tensor &qb, const Tensor &kb,
+                                       const c10::optional<Tensor> &mask, int64_t heads, py::object dtype) {
+    const auto type = torch::python::detail::py_object_to_dtype(dtype);
+    auto floating = [](const Tensor &x) { return x.scalar_type() == torch::kFloat16 || x.scalar_type() == torch::kBFloat16 || x.scalar_type() == torch::kFloat32; };
+    const int64_t d = heads > 0 && qkv.dim() == 3 && qkv.size(2) % (3 * heads) == 0 ? qkv.size(2) / (3 * heads) : 0;
+    const bool ready = d >= 8 && d <= FB_MAX_HEADDIM && (d & (d - 1)) == 0 && qkv.is_cuda() && qkv.is_contiguous() && floating(qkv) &&
+                       reinterpret_cast<uintptr_t>(qkv.data_ptr()) % 16 == 0 && logit_scale.device() == qkv.device() &&
+                       floating(logit_scale) && logit_scale.numel() == heads && (type == torch::kFloat16 || type == torch::kBFloat16) &&
+                       qb.scalar_type() == type && kb.scalar_type() == type && qb.dim() == 4 && qb.size(3) % 8 == 0;
+    if (!ready) return c10::nullopt;
+    return WindowFn::apply(qkv, logit_scale.contiguous(), channel_contiguous(qb), channel_contiguous(kb), mask, heads, (int64_t)type);
 }
 
 // (q_bias, k_bias) of fb_alibi_factors, (1, L, H, rank) in the 16-bit dtype of `like`'s device.

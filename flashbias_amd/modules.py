@@ -71,15 +71,16 @@ class WindowAttentionCore(nn.Module):
         b_, n, c = x.shape
         qkv = self.qkv(x)
         ext = interface._extension()
-        if ext is not None and qkv.is_cuda and qkv.is_contiguous() and c // self.heads in (8, 16, 32, 64, 128) and self.q_bias_pos.shape[-1] % 8 == 0 \
-                and self.q_bias_pos.dtype == self.dtype:
+        if ext is not None and qkv.is_cuda:
             # normalisation, attention and the packed projection's gradient without passes in between (csrc/fb_torch.cpp)
+            m = mask
             if mask is not None:
-                mask = mask.to(self.dtype)
-                if mask.dim() != 3 or mask.shape[2] != n:  # broadcast over the keys (or the windows), as below
-                    mask = mask[None, :, None].expand(1, mask.shape[0], 1, n, n)[0, :, 0]
-            o = ext.window_attention(qkv, self.logit_scale, self.q_bias_pos, self.k_bias_pos, mask, self.heads, self.dtype)
-            return self.proj(o.reshape(b_, n, c).to(x.dtype))
+                m = mask.to(self.dtype)
+                if m.dim() != 3 or m.shape[2] != n:  # broadcast over the keys (or the windows), as below
+                    m = m[None, :, None].expand(1, m.shape[0], 1, n, n)[0, :, 0]
+            o = ext.window_attention(qkv, self.logit_scale, self.q_bias_pos, self.k_bias_pos, m, self.heads, self.dtype)
+            if o is not None:
+                return self.proj(o.reshape(b_, n, c).to(x.dtype))
         qkv = qkv.view(b_, n, 3, self.heads, c // self.heads)
         q, k, v = qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2]
         scale = torch.clamp(self.logit_scale, max=4.6052).exp().view(1, 1, self.heads, 1)

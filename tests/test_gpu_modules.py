@@ -207,3 +207,38 @@ def test_window_masks_that_broadcast(gpu_device, monkeypatch, shape, accepted):
         # (fp32 projection: q and k differ by the last bit where fp32 sums in another order fall on the other side of a
         # rounding, P and dS by 2^-9 relative; outputs rounded to bf16)
         assert (a - b).norm() <= 2.0 ** -7 * b.norm(), name
+
+
+@pytest.mark.parametrize("what", ["float64", "float64 scale", "strided scale", "flat scale", "misaligned projection", "fp16 in bf16 out",
+                                  "head dim 24", "rank 12"])
+def test_window_block_takes_what_the_tensor_operations_take(gpu_device, monkeypatch, what):
+    """Parameters and projections that the one-pass kernels have no form for, or not the obvious one."""
+    torch.manual_seed(4)
+    hd, rank = 24 if what == "head dim 24" else 32, 12 if what == "rank 12" else 8
+    mod = modules.WindowAttentionCore(2 * hd, 4, 2, rank=rank).to(gpu_device)
+    q_bias, k_bias = mod.q_bias_pos, mod.k_bias_pos
+    mod = mod.to({"float64": torch.float64, "fp16 in bf16 out": torch.float16}.get(what, torch.float32))
+    mod.q_bias_pos, mod.k_bias_pos = q_bias, k_bias  # (bf16 still)
+    if what == "float64 scale":
+        mod.logit_scale = torch.nn.Parameter(mod.logit_scale.double())
+    if what == "strided scale":
+        mod.logit_scale = torch.nn.Parameter(torch.tensor([[2.0, 9.0], [2.5, 9.0]], device=gpu_device)[:, :1, None])
+        assert not mod.logit_scale.is_contiguous()
+    if what == "flat scale":
+        mod.logit_scale = torch.nn.Parameter(torch.tensor([2.0, 2.5], device=gpu_device))
+    x = torch.randn(6, 16, 2 * hd, device=gpu_device, dtype=mod.qkv.weight.dtype, requires_grad=True)
+    if what == "misaligned projection":
+        store = torch.randn(6 * 16 * 6 * hd + 1, device=gpu_device)
+        mod.qkv = Given(store.requires_grad_(True)[1:].view(6, 16, 6 * hd))
+        assert mod.qkv.y.data_ptr() % 16
+        x = x.detach()
+    target = mod.qkv.y if isinstance(mod.qkv, Given) else x
+    results = []
+    for ext in (interface._extension(), None):
+        with monkeypatch.context() as m:
+            m.setattr(interface, "_ext", ext)
+            y = mod(x)
+            results.append([y.detach().double()] + [t.double() for t in torch.autograd.grad(y.double().square().sum(), [target, mod.logit_scale])])
+    for name, a, b in zip(("y", "input", "scale"), *results):
+        # (as test_window_masks_that_broadcast; the scale's gradient is a sum over all scores: as the module's other tests)
+        assert (a - b).norm() <= (3e-2 if name == "scale" else 2.0 ** -7) * b.norm(), name
