@@ -19,14 +19,12 @@ def _args(dev, r, mask):
 
 
 # rank 8 without a vector mask goes straight to the extension, rank 4 and vector masks through the preparations
-@pytest.mark.parametrize("r,mask", [(8, "none"), (8, "matrix"), (8, "vector"), (4, "none"), (0, "none")])
+@pytest.mark.parametrize("r,mask,folded", [(8, "none", False), (8, "matrix", False), (8, "vector", False), (8, "vector", True), (4, "none", False),
+                                           (0, "none", False)])
 @pytest.mark.parametrize("grad_enabled", [True, False])
-@pytest.mark.parametrize("folded", [False, True])
 def test_forward_mode_derivatives_are_refused(gpu_device, monkeypatch, r, mask, grad_enabled, folded):
     assert interface._extension() is not None
     if folded:
-        if mask != "vector":
-            pytest.skip("only vector masks are folded")
         monkeypatch.setattr(interface, "_FOLD_MIN_PAIRS", 1)
     args = _args(gpu_device, r, mask)
     with torch.set_grad_enabled(grad_enabled):

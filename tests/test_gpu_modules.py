@@ -42,7 +42,7 @@ def test_window_block_against_tensor_operations(gpu_device, monkeypatch, dtype, 
     got = grads()
     monkeypatch.setattr(interface, "_ext", None)  # the tensor operations and the Python autograd function
     want = grads()
-    # q and k have the same bits on both ways; what is left is the backward's own rounding (2^-8 per product of
+    # (q and k have the same bits on both ways: test_cosine_forward_has_the_bits_of_tensor_operations)  What is left is the backward's own rounding (2^-8 per product of
     # bf16 tensor operations, of which the fused pass has fewer) and the summation orders
     bound = 3e-2
     for name, g, w in zip(["y", "x"] + [k for k, _ in mod.named_parameters()], got, want):
@@ -119,6 +119,32 @@ def test_cosine_forward_in_fp32_rounds_once(gpu_device, in_dtype, dtype, scale_d
     assert not got[0][7].any() and not got[1][7].any()
 
 
+@pytest.mark.parametrize("in_dtype,dtype,scale_dtype", [t for t in COSINE_TYPES if t[0] != torch.float32])
+@pytest.mark.parametrize("heads,d", [(1, 8), (3, 16), (5, 32), (2, 128)])
+def test_cosine_forward_has_the_bits_of_tensor_operations(gpu_device, in_dtype, dtype, scale_dtype, heads, d):
+    """With steps in the projection's type q and k are those of the tensor operations, also from a block that ends before
+    the field that says so."""
+    lib = _lib.load()
+    qkv, scale = _cosine_inputs(gpu_device, in_dtype, scale_dtype, heads, d)
+    qkv[7] = 1  # (a row of zeros in fp16 is 0 / 0 on both ways)
+    x = qkv.view(qkv.shape[0], 3, heads, d)
+    unit = lambda t: torch.nn.functional.normalize(t, dim=-1)
+    s = torch.clamp(scale, max=4.6052).exp().view(1, heads, 1)
+    want = [(unit(x[:, 0]) * s).to(dtype), unit(x[:, 1]).to(dtype), x[:, 2].to(dtype)]
+    for size in (ctypes.sizeof(FbCosine), FbCosine.fp32.offset):
+        got = [torch.full_like(w, float("nan")) for w in want]
+        a = _cosine_block(qkv, scale, heads, dtype)
+        a.size = size
+        a.q, a.k, a.v = (t.data_ptr() for t in got)
+        _lib.check_status(lib.fb_cosine_fwd(ctypes.byref(a), ctypes.c_void_p(interface._stream())))
+        torch.cuda.synchronize()
+        for name, g, w in zip("qkv", got, want):
+            # (the two sum squares in fp32 in orders of their own: up to 12 x 2^-24 apart, which puts one norm in
+            # 2^12 / 12 (fp16; bf16 2^15 / 12) on the other side of a rounding: at most two of the 333 to 1665 here, twice d elements)
+            assert int((g != w).any(-1).sum()) <= (0 if name == "v" else 2), name
+            assert (g.float() - w.float()).abs().max() <= 2.0 ** -6 * w.float().abs().max(), name
+
+
 class Given(torch.nn.Module):
     """In the place of a projection: its result."""
 
@@ -130,13 +156,14 @@ class Given(torch.nn.Module):
         return self.y
 
 
-def _window_core_exact(mod, qkv, logit_scale, heads):
+def _window_core_exact(mod, qkv, logit_scale, heads, mask=None):
     """Attention of a window block on its projection, in float64 tensor operations."""
     windows, n, dim = qkv.shape[0], qkv.shape[1], qkv.shape[2] // 3
     q, k, v = (t.view(windows, n, heads, dim // heads).transpose(1, 2).contiguous()
                for t in _cosine_exact(qkv.view(windows * n, -1), logit_scale, heads))
     bias = mod.q_bias_pos.double()[0].transpose(0, 1) @ mod.k_bias_pos.double()[0].permute(1, 2, 0).contiguous()
-    o = torch.softmax(q @ k.transpose(-1, -2).contiguous() + bias, dim=-1) @ v
+    logits = q @ k.transpose(-1, -2).contiguous() + bias
+    o = torch.softmax(logits if mask is None else logits + mask[:, None], dim=-1) @ v
     return o.transpose(1, 2).reshape(windows, n, dim)
 
 
@@ -242,3 +269,43 @@ def test_window_block_takes_what_the_tensor_operations_take(gpu_device, monkeypa
     for name, a, b in zip(("y", "input", "scale"), *results):
         # (as test_window_masks_that_broadcast; the scale's gradient is a sum over all scores: as the module's other tests)
         assert (a - b).norm() <= (3e-2 if name == "scale" else 2.0 ** -7) * b.norm(), name
+
+
+@pytest.mark.parametrize("dtype,param", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("window,heads,hd,windows,types", [(8, 2, 32, 6, 3), (7, 3, 128, 4, 0), (16, 8, 32, 64, 4), (12, 4, 32, 66, 6)])
+def test_window_block_against_float64(gpu_device, monkeypatch, dtype, param, window, heads, hd, windows, types):
+    """The module's attention on its projection, forward and backward, against float64, and beside the error that the tensor
+    operations have there (64 x 8 windows of 256 and 66 x 4 of 144: one workgroup per window and head in the backward, masks
+    that repeat over the images)."""
+    torch.manual_seed(5)
+    n, dim = window * window, heads * hd
+    mod = modules.WindowAttentionCore(dim, window, heads, rank=8, dtype=dtype).to(gpu_device, param)
+    mod.q_bias_pos, mod.k_bias_pos = mod.q_bias_pos.to(dtype), mod.k_bias_pos.to(dtype)
+    qkv = torch.randn(windows, n, 3 * dim, device=gpu_device).to(param).requires_grad_(True)
+    mod.qkv, mod.proj = Given(qkv), torch.nn.Identity()
+    x = torch.zeros(windows, n, dim, device=gpu_device, dtype=param)
+    dy = torch.randn(windows, n, dim, device=gpu_device).to(param)
+    mask = (torch.rand(types, n, n, device=gpu_device) < 0.2).float() * -100.0 if types else None
+
+    def run():
+        y = mod(x, mask)
+        return [y.detach()] + list(torch.autograd.grad(y, [qkv, mod.logit_scale], dy))
+    got = run()
+    monkeypatch.setattr(interface, "_ext", None)
+    ops = run()
+    leaf, scale = qkv.detach().double().requires_grad_(True), mod.logit_scale.detach().double().flatten().requires_grad_(True)
+    exact = [[], [], 0]
+    for at in range(0, windows, 8):  # (dense)
+        part = slice(at, min(at + 8, windows))
+        m = None if mask is None else mask[torch.arange(at, part.stop, device=gpu_device) % types].double()
+        y = _window_core_exact(mod, leaf[part], scale, heads, m)
+        g = torch.autograd.grad(y, [leaf, scale], dy[part].double())
+        exact[0].append(y.detach())
+        exact[1].append(g[0][part])
+        exact[2] = exact[2] + g[1]
+    exact = [torch.cat(exact[0]), torch.cat(exact[1]), exact[2].view_as(mod.logit_scale)]
+    for name, g, o, w in zip(("y", "dqkv", "dscale"), got, ops, exact):
+        error = lambda t: float((t.double() - w).norm() / w.norm())
+        # y and dqkv: independent roundings of thousands of values, the two errors are measured to a percent or two; dscale:
+        # `heads` values, each the rest of a sum that cancels, where two errors of one size differ by a factor
+        assert torch.isfinite(g).all() and error(g) <= (3 if name == "dscale" else 1.05) * error(o), (name, error(g), error(o))

@@ -1253,11 +1253,12 @@ def test_modules(gpu_device):
         y = mod(x, **kw)
         gx, = torch.autograd.grad(y.sum(), x)
         M.flash_bias_func = oracle_func
+        ext, M.interface._ext = M.interface._ext, None  # (the window block's one-pass kernels do not ask flash_bias_func)
         try:
             y_ref = mod(x, **kw)
             gx_ref, = torch.autograd.grad(y_ref.sum(), x)
         finally:
-            M.flash_bias_func = real
+            M.flash_bias_func, M.interface._ext = real, ext
         assert (y - y_ref).abs().max() <= 2e-2 * max(1.0, y_ref.abs().max().item())
         assert (gx - gx_ref).abs().max() <= 5e-2 * gx_ref.abs().max()
 

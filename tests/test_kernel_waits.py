@@ -1,7 +1,8 @@
 """The static check of MFMA wait states (flashbias_amd/csrc/check_mfma_waits.py): on hand-made instruction
 sequences, and on the compiled code of the two units in which the compiler's own count fell short before
 (the window backward, whose first version read a score block across a loop branch after two slots, and the
-general dq kernel, where a short-circuit condition gave the block after the last MFMA two ways out)."""
+general dq kernel, where a short-circuit condition gave the block after the last MFMA two ways out) and of the
+units of head dim 128 (the wide forward, dq and dk/dv with factors in a region of their own)."""
 import importlib.util
 import os
 import shutil
@@ -55,8 +56,8 @@ def test_every_path_counts():
 
 @pytest.mark.skipif(shutil.which("hipcc") is None or shutil.which("make") is None, reason="needs hipcc and make")
 def test_compiled_kernels():
-    units = ["build/asm/fb_bwd_win_bf16_2.s", "build/asm/fb_bwd_dq_bf16_2.s"]
-    subprocess.run(["make", "-j2"] + units, cwd=CSRC, check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    units = [f"build/asm/fb_{unit}.s" for unit in ("bwd_dkv_bf16_8", "bwd_win_bf16_2", "bwd_dq_bf16_8", "fwd_bf16_8", "bwd_dq_bf16_2")]
+    subprocess.run(["make", "-j4"] + units, cwd=CSRC, check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
     for unit in units:
         with open(os.path.join(CSRC, unit)) as f:
             text = f.read()
