@@ -613,9 +613,8 @@ static hipError_t launch_dq_vec(const BwdArgs &a, hipStream_t stream) {
     }
     // head dims above 64, aligned, unmasked, rank <= 32: two workgroups per CU (larger ranks spill at 256 registers and
     // keep one wave per SIMD)
-    if constexpr (NKD > 4 && NKR <= 2 && VEC && !MASK)
-        return launch_dq_qb<T, NKD, NKR, VEC, MASK, true, FOLD, true>(a, stream);
-    return launch_dq_qb<T, NKD, NKR, VEC, MASK, true, FOLD>(a, stream);
+    constexpr bool SPLIT = NKD > 4 && NKR <= 2 && VEC && !MASK;
+    return launch_dq_qb<T, NKD, NKR, VEC, MASK, true, FOLD, SPLIT>(a, stream);
 }
 
 } // namespace fb

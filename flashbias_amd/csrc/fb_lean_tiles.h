@@ -143,10 +143,6 @@ struct LeanCopy2 {
     __device__ __forceinline__ static int count(int wave) { return (ROWS < 128 && wave >= ROWS / 32) ? 0 : 1; }
 };
 
-// The kernel arguments as a function called by the kernel may read them: a function's pointer
-// argument arrives in vector registers, which would make every value loaded through it look
-// divergent (vector loads, no scalar operands for the copy instructions); made wave-uniform again
-// and typed as constant memory it is read with scalar loads like the kernel's own copy.
 // Copies of a dense region of ROWS rows x CPR chunks (CPR = 2 or 4: a factor of rank up to 16 or 32) by the first
 // waves of a workgroup, one instruction each; lanes whose chunk is channel padding stay off (the region is cleared
 // once), and with `twice` chunk 1 is a second copy of chunk 0 (fold_scale_chunk).  Row strides below 2^24 elements.
@@ -212,6 +208,10 @@ struct TileAddr16 {
     }
 };
 
+// The kernel arguments as a function called by the kernel may read them: a function's pointer
+// argument arrives in vector registers, which would make every value loaded through it look
+// divergent (vector loads, no scalar operands for the copy instructions); made wave-uniform again
+// and typed as constant memory it is read with scalar loads like the kernel's own copy.
 template <class A>
 __device__ __forceinline__ A uniform_kernargs(const void *p) {
     static_assert(sizeof(A) % 4 == 0, "");
