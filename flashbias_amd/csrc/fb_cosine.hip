@@ -9,7 +9,7 @@
 // keeps its head and channels for all the tokens it walks, so the scale is read once and the logit scale's gradient
 // is one running sum per thread; its last step is a small kernel of one workgroup per head, in a fixed order.
 // As tensor operations the same work took about 40 passes over tensors of that size (16 x 64 windows of 256 tokens, 16
-// heads of 32 channels, bf16, forward + backward: 7.4 of the module's 12.9 ms).
+// heads of 32 channels, bf16, forward + backward: 7.4 of the module's 12.7 ms).
 //
 // Rounding (fb_cosine.fp32 == 0): the type of the packed projection is also the type that tensor operations compute in,
 // which round the norm, the quotient and the product to it one after the other; these kernels do the same, so that q and

@@ -38,8 +38,13 @@ def _last_dim_contiguous(x):
 
 
 # A vector mask on a problem of at least this many (batch, head, query, key) pairs is folded into
-# the factors (below that the extra tensor operations cost more than the kernels gain: measured
-# at B2 H4 d32 r8, 2.09 against 2.96 ms fwd+bwd at L=16384, 0.38 against 0.32 ms at L=4096).
+# the factors.  Forward + backward, folded against the kernels' own vector masks, in ms: B2 H4
+# L=16384 d32 2.03 / 2.25 at rank 8 and 2.31 / 2.29 at rank 16; B4 H16 L=4096 d64 1.57 / 1.64 at
+# rank 8, d128 2.95 / 4.03 at rank 8 and 3.12 / 4.05 at rank 16 (the dq kernel takes a vector mask
+# as a matrix, which is what the fold saves).  It is behind where the column makes another
+# rank bucket (rank 32: 3.03 / 2.43 at d32, 6.34 / 4.14 at d128), where the factors are shared by
+# the batch and the mask is not (768 x 4 rows of 768, rank 32: 5.96 / 2.47), and in a forward
+# alone (rank 8 as above: 0.53 / 0.52, 0.38 / 0.37, 0.62 / 0.64).
 _FOLD_MIN_PAIRS = 1 << 29
 
 

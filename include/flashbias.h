@@ -133,7 +133,7 @@ int fb_check(const fb_params *p, int pass);
  * swin_transformer_v2.py:178-203), where writing the full-shape factor gradients and summing them
  * afterwards costs more than the attention itself saves; then the largest of 8, 4, 2 (32, 16, ... for whole
  * sequences of at most 256 positions at head dim 32, which one workgroup per batch entry and head serves) that still
- * leaves every compute unit several workgroups.  Reads the sizes, the causal flag, the mask type and the factors' strides only.
+ * leaves every compute unit several workgroups.  Reads the sizes, the causal flag, the element types, the mask type and the factors' strides only.
  * No counterpart in the reference. */
 int fb_suggest_bias_grad_group(const fb_params *p);
 
