@@ -30,6 +30,12 @@ hipError_t launch_bwd_win_f16_2(const BwdArgs &a, hipStream_t stream);
 hipError_t launch_cosine(const fb_cosine *p, bool fp32, bool backward, hipStream_t stream);
 int64_t cosine_sweep(int64_t tokens, int H, int d);
 
+// weight and bias gradient of a projection (fb_wgrad.hip)
+size_t wgrad_workspace(int64_t tokens, int n, int k, bool bias);
+bool wgrad_recommended(int64_t tokens, int n, int k);
+hipError_t launch_wgrad(const void *dy, int64_t ldy, const void *x, int64_t ldx, void *dw, void *db, float *partial, int64_t tokens,
+                        int n, int k, bool bf16, hipStream_t stream);
+
 hipError_t launch_fwd(const FwdArgs &a, bool bf16, hipStream_t stream) {
     switch (nkd_of(a.d)) {
     case 1: return bf16 ? launch_fwd_bf16_1(a, stream) : launch_fwd_f16_1(a, stream);
@@ -299,6 +305,33 @@ int fb_cosine_bwd(const fb_cosine *p, void *stream) {
     const int rc = check_cosine(p, true);
     if (rc) return rc;
     return launched(fb::launch_cosine(p, cosine_fp32(p), true, static_cast<hipStream_t>(stream)), "fb_cosine_bwd");
+}
+
+static bool weight_grad_sizes(int64_t tokens, int n, int k) {
+    return tokens > 0 && tokens <= ((int64_t)1 << 40) && n > 0 && k > 0 && n <= (1 << 16) && k <= (1 << 16) && n % 8 == 0 && k % 8 == 0;
+}
+
+size_t fb_weight_grad_workspace_bytes(int64_t tokens, int n, int k, int with_bias) {
+    return weight_grad_sizes(tokens, n, k) ? fb::wgrad_workspace(tokens, n, k, with_bias != 0) : 0;
+}
+
+int fb_weight_grad_recommended(int64_t tokens, int n, int k) {
+    return weight_grad_sizes(tokens, n, k) && fb::wgrad_recommended(tokens, n, k) ? 1 : 0;
+}
+
+int fb_weight_grad(const void *dy, int64_t ldy, const void *x, int64_t ldx, void *dw, void *db, float *scratch, int dtype, int64_t tokens,
+                   int n, int k, void *stream) {
+    fb::api_clear_error();
+    if (!dy || !x || !dw || !scratch) return fb::api_fail(FB_ERR_NULL, "fb_weight_grad: null pointer");
+    if (dtype != FB_F16 && dtype != FB_BF16) return fb::api_fail(FB_ERR_DTYPE, "only fp16 and bf16 are supported");
+    if (!weight_grad_sizes(tokens, n, k))
+        return fb::api_fail(FB_ERR_SHAPE, "fb_weight_grad: tokens must be positive, n and k multiples of 8 up to 65536");
+    if (ldy < n || ldx < k || ldy % 8 != 0 || ldx % 8 != 0 || ldy >= (1 << 24) || ldx >= (1 << 24))
+        return fb::api_fail(FB_ERR_STRIDE, "fb_weight_grad: row strides must be multiples of 8 below 2^24 and hold a row");
+    for (const void *p : {dy, x, static_cast<const void *>(dw), static_cast<const void *>(scratch)})
+        if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return fb::api_fail(FB_ERR_STRIDE, "fb_weight_grad: tensors must be 16-byte aligned");
+    return launched(fb::launch_wgrad(dy, ldy, x, ldx, dw, db, scratch, tokens, n, k, dtype == FB_BF16, static_cast<hipStream_t>(stream)),
+                    "fb_weight_grad");
 }
 
 int fb_bwd_static(const fb_params *p, void *stream) {

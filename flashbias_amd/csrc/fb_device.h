@@ -44,6 +44,10 @@ struct BF16 {
     static __device__ __forceinline__ uint16_t from_float(float x) {
         return __builtin_bit_cast(uint16_t, (__bf16)x);
     }
+    static __device__ __forceinline__ float add2(uint32_t x, float acc) { // acc + both elements of x
+        const bf16x2_t one = {(__bf16)1.f, (__bf16)1.f};
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, x), one, acc, false);
+    }
     static constexpr uint16_t kOne = 0x3f80;
     static constexpr bool kWideRange = true; // the exponent range of fp32
 };
@@ -65,6 +69,10 @@ struct F16 {
     }
     static __device__ __forceinline__ uint16_t from_float(float x) {
         return __builtin_bit_cast(uint16_t, (_Float16)x);
+    }
+    static __device__ __forceinline__ float add2(uint32_t x, float acc) {
+        const f16x2_t one = {(_Float16)1.f, (_Float16)1.f};
+        return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, x), one, acc, false);
     }
     static constexpr uint16_t kOne = 0x3c00;
     static constexpr bool kWideRange = false;

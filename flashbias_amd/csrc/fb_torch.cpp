@@ -12,10 +12,13 @@
 #include <torch/extension.h>
 
 #include <ATen/FuncTorchTLS.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <cmath>
 #include <cstring>
@@ -341,6 +344,65 @@ std::pair<Tensor, Tensor> alibi_factors(int64_t Lq, int64_t Lk, int64_t heads, i
     return {qb, kb};
 }
 
+// A projection x w^T + b whose weight and bias gradients come from the library's kernel for long contractions
+// (fb_weight_grad); the forward and the input's gradient are the tensor library's products.
+struct LinearFn : public torch::autograd::Function<LinearFn> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &w, const c10::optional<Tensor> &b) {
+        ctx->save_for_backward({x, w});
+        ctx->saved_data["bias"] = b.has_value();
+        return at::linear(x, w, b);
+    }
+
+    static tensor_list backward(AutogradContext *ctx, tensor_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &w = saved[1];
+        const int64_t n = w.size(0), k = w.size(1);
+        const bool bias = ctx->saved_data["bias"].toBool();
+        const Tensor dy = grads[0].reshape({-1, n});
+        Tensor dx, dw, db;
+        if (ctx->needs_input_grad(0)) dx = dy.matmul(w).view(x.sizes());
+        const bool want_w = ctx->needs_input_grad(1), want_b = bias && ctx->needs_input_grad(2);
+        if (want_w && !c10::GradMode::is_enabled()) {
+            auto rows = [](const Tensor &t) { // rows of contiguous, 16-byte aligned elements
+                const bool ok = t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % 8 == 0 && t.stride(0) < (1 << 24) &&
+                                reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+                return ok ? t : t.clone(at::MemoryFormat::Contiguous);
+            };
+            const Tensor y2 = rows(dy), x2 = rows(x.reshape({-1, k}));
+            dw = fresh({n, k}, w.scalar_type(), w.device());
+            if (want_b) db = fresh({n}, w.scalar_type(), w.device());
+            const c10::hip::HIPGuardMasqueradingAsCUDA guard(w.device());
+            Tensor scratch = fresh({(int64_t)(fb_weight_grad_workspace_bytes(y2.size(0), (int)n, (int)k, want_b) / 4)}, torch::kFloat32, w.device());
+            check(fb_weight_grad(y2.data_ptr(), y2.stride(0), x2.data_ptr(), x2.stride(0), dw.data_ptr(), want_b ? db.data_ptr() : nullptr,
+                                 scratch.data_ptr<float>(), dtype_code(w.scalar_type()), y2.size(0), (int)n, (int)k, stream_of(w)));
+        } else { // (a gradient that is itself differentiated: tensor operations)
+            if (want_w) dw = dy.t().matmul(x.reshape({-1, k}));
+            if (want_b) db = dy.sum(0);
+        }
+        return {dx, dw, db};
+    }
+};
+
+// The projection where its weight gradient is asked for and the library's kernel for it is ahead, else nothing: the caller
+// then takes the tensor library's own operation, which is also what modes, transforms and tracers that look at operations see.
+c10::optional<Tensor> linear(const Tensor &x, const Tensor &w, const c10::optional<Tensor> &b) {
+    const auto type = x.scalar_type();
+    auto plain = [&](const Tensor &t) {
+        return t.is_cuda() && t.scalar_type() == type && t.device() == x.device() && !t.key_set().has(c10::DispatchKey::Python) &&
+               t.layout() == c10::kStrided && !t._fw_grad(/*level=*/0).defined();
+    };
+    const bool ready = c10::GradMode::is_enabled() && (type == torch::kFloat16 || type == torch::kBFloat16) && plain(x) && plain(w) &&
+                       w.requires_grad() && x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && x.numel() > 0 &&
+                       w.size(0) <= (1 << 16) && w.size(1) <= (1 << 16) &&
+                       fb_weight_grad_recommended(x.numel() / x.size(-1), (int)w.size(0), (int)w.size(1)) &&
+                       (!b.has_value() || (plain(*b) && b->dim() == 1 && b->size(0) == w.size(0))) &&
+                       !at::autocast::is_autocast_enabled(at::kCUDA) && !at::functorch::functorchTLSAccessor() &&
+                       !c10::impl::TorchDispatchModeTLS::any_modes_set() && !at::impl::torch_function_mode_enabled() &&
+                       !torch::jit::tracer::isTracing();
+    if (!ready) return c10::nullopt;
+    return LinearFn::apply(x, w, b);
+}
+
 // x (..., r) with its last dim zero-padded (or cut) to `rank` columns in one launch of the library; the gradient
 // is the same operation the other way.  For contiguous 16-bit GPU tensors (the caller checks).
 struct ResizeRankFn : public torch::autograd::Function<ResizeRankFn> {
@@ -410,6 +472,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("heads"), py::arg("dtype"));
     m.def("alibi_factors", &alibi_factors, py::arg("seqlen_q"), py::arg("seqlen_k"), py::arg("heads"), py::arg("rank"), py::arg("reference_sign"),
           py::arg("dtype"), py::arg("device"));
+    m.def("linear", &linear, py::arg("x"), py::arg("weight"), py::arg("bias"));
     m.def("resize_rank", &resize_rank, py::arg("x"), py::arg("rank"));
     m.def("flash_bias", &flash_bias, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("q_bias") = py::none(),
           py::arg("k_bias") = py::none(), py::arg("mask") = py::none(), py::arg("causal") = false,

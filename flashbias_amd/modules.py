@@ -11,6 +11,21 @@ from . import factors, interface
 from .interface import flash_bias_func
 
 
+def _project(layer, x):
+    """``layer(x)``.  A plain ``nn.Linear`` over many tokens gets its weight gradient from the library's own kernel for long
+    contractions (``ext.linear``, which says for which calls; a layer that something hooks into or replaces is called)."""
+    if (x.is_cuda and type(layer) is nn.Linear and torch.is_grad_enabled() and not torch.compiler.is_compiling()
+            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks)
+            and "forward" not in layer.__dict__ and layer._compiled_call_impl is None
+            and not nn.modules.module._has_any_global_hook()):
+        ext = interface._extension()
+        if ext is not None:
+            y = ext.linear(x, layer.weight, layer.bias)
+            if y is not None:
+                return y
+    return layer(x)
+
+
 class AttentionWithALiBiBias(nn.Module):
     """Causal multi-head self-attention with ALiBi as an exact rank-2 FlashBias.
 
@@ -35,7 +50,7 @@ class AttentionWithALiBiBias(nn.Module):
     def forward(self, x):
         b, n, _ = x.shape
         split = lambda t: t.view(b, n, self.heads, self.dim_head).to(self.dtype)
-        q, k, v = split(self.to_q(x)), split(self.to_k(x)), split(self.to_v(x))
+        q, k, v = split(_project(self.to_q, x)), split(_project(self.to_k, x)), split(_project(self.to_v, x))
         ext = interface._extension()
         if ext is not None and x.is_cuda and n <= 65536:
             # the same factors in one launch, with the zero columns the operator would append on every call
@@ -69,7 +84,7 @@ class WindowAttentionCore(nn.Module):
 
     def forward(self, x, mask=None):
         b_, n, c = x.shape
-        qkv = self.qkv(x)
+        qkv = _project(self.qkv, x)
         ext = interface._extension()
         if ext is not None and qkv.is_cuda:
             # normalisation, attention and the packed projection's gradient without passes in between (csrc/fb_torch.cpp)
@@ -80,7 +95,7 @@ class WindowAttentionCore(nn.Module):
                     m = m[None, :, None].expand(1, m.shape[0], 1, n, n)[0, :, 0]
             o = ext.window_attention(qkv, self.logit_scale, self.q_bias_pos, self.k_bias_pos, m, self.heads, self.dtype)
             if o is not None:
-                return self.proj(o.reshape(b_, n, c).to(x.dtype))
+                return _project(self.proj, o.reshape(b_, n, c).to(x.dtype))
         qkv = qkv.view(b_, n, 3, self.heads, c // self.heads)
         q, k, v = qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2]
         scale = torch.clamp(self.logit_scale, max=4.6052).exp().view(1, 1, self.heads, 1)
@@ -90,4 +105,4 @@ class WindowAttentionCore(nn.Module):
             nw = mask.shape[0]
             mask = mask.to(self.dtype)[None, :, None].expand(b_ // nw, nw, 1, n, n).reshape(b_, 1, n, n)
         o = flash_bias_func(q, k, v.to(self.dtype), self.q_bias_pos, self.k_bias_pos, mask, False, 1.0)
-        return self.proj(o.reshape(b_, n, c).to(x.dtype))
+        return _project(self.proj, o.reshape(b_, n, c).to(x.dtype))

@@ -247,6 +247,17 @@ size_t fb_cosine_workspace_bytes(const fb_cosine *p);
 int fb_cosine_fwd(const fb_cosine *p, void *stream);
 int fb_cosine_bwd(const fb_cosine *p, void *stream);
 
+/* Weight and bias gradient of a projection y = x w^T + b, the products around the attention of a block
+ * (swin_transformer_v2.py:155-207), for many tokens and a small weight: dw (n, k) = dy^T x and db (n) = the column sums
+ * of dy, both contiguous in the input dtype, accumulated in fp32 in a fixed order and rounded once; db NULL: not wanted.
+ * dy (tokens, n) and x (tokens, k) have contiguous rows at strides ldy, ldx (elements).  n, k, ldy and ldx are multiples
+ * of 8, dy, x, dw and scratch 16-byte aligned; scratch: fb_weight_grad_workspace_bytes() bytes.  Two launches.
+ * fb_weight_grad_recommended: 1 where this was measured ahead of the vendor library's product of the same shape. */
+size_t fb_weight_grad_workspace_bytes(int64_t tokens, int n, int k, int with_bias);
+int fb_weight_grad_recommended(int64_t tokens, int n, int k);
+int fb_weight_grad(const void *dy, int64_t ldy, const void *x, int64_t ldx, void *dw, void *db, float *scratch, int dtype, int64_t tokens,
+                   int n, int k, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -309,3 +309,65 @@ def test_window_block_against_float64(gpu_device, monkeypatch, dtype, param, win
         # y and dqkv: independent roundings of thousands of values, the two errors are measured to a percent or two; dscale:
         # `heads` values, each the rest of a sum that cancels, where two errors of one size differ by a factor
         assert torch.isfinite(g).all() and error(g) <= (3 if name == "dscale" else 1.05) * error(o), (name, error(g), error(o))
+
+
+# tiles of 256 and 128 and their ragged edges; fewer stages of 32 tokens than the pipeline is deep, a ragged last one, one
+# share and many; rows inside wider tensors
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens,n,k", [(1, 8, 8), (31, 264, 136), (64, 128, 384), (97, 248, 256), (129, 256, 504), (300, 1000, 248), (4100, 384, 128),
+                                        (20000, 768, 256)])
+def test_weight_gradient(gpu_device, dtype, tokens, n, k):
+    lib = _lib.load()
+    g = torch.Generator(device=gpu_device).manual_seed(tokens)
+    dy_all = torch.randn(tokens, n + 24, generator=g, device=gpu_device).to(dtype)
+    x_all = torch.randn(tokens, k + 8, generator=g, device=gpu_device).to(dtype)
+    dy, x = dy_all[:, 8:8 + n], x_all[:, :k]
+    # (nothing outside the rows may count: what lies beside them is not finite)
+    dy_all[:, :8] = dy_all[:, 8 + n:] = x_all[:, k:] = float("nan")
+    for bias in (True, False):
+        dw = torch.full((n, k), float("nan"), device=gpu_device, dtype=dtype)
+        db = torch.full((n,), float("nan"), device=gpu_device, dtype=dtype)
+        scratch = torch.full((lib.fb_weight_grad_workspace_bytes(tokens, n, k, bias) // 4,), float("nan"), device=gpu_device)
+        _lib.check_status(lib.fb_weight_grad(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), dw.data_ptr(), db.data_ptr() if bias else None,
+                                             scratch.data_ptr(), CODES[dtype], tokens, n, k, interface._stream()))
+        # rounded once to 8 / 11 significant bits: at most half a unit of the last place of every element, whose sums in
+        # 32 bits are far closer
+        bound = 1.01 * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)
+        want = dy.double().t().contiguous() @ x.double()
+        assert (dw.double() - want).norm() <= bound * want.norm()
+        if bias:
+            assert (db.double() - dy.double().sum(0)).norm() <= bound * dy.double().sum(0).norm()
+
+
+def test_projection_takes_the_kernel_and_leaves_the_rest(gpu_device):
+    torch.manual_seed(2)
+    layer = torch.nn.Linear(128, 136).to(gpu_device, torch.bfloat16)
+    x = torch.randn(5, 1300, 128, device=gpu_device, dtype=torch.bfloat16, requires_grad=True)
+    leaves = [x, layer.weight, layer.bias]
+    dy = torch.randn(5, 1300, 136, device=gpu_device, dtype=torch.bfloat16)
+    y, want_y = modules._project(layer, x), torch.nn.functional.linear(x, layer.weight, layer.bias)
+    assert "LinearFn" in type(y.grad_fn).__name__ + y.grad_fn.name() and torch.equal(y, want_y)
+    for out in (dy, dy[:1, :1].expand(5, 1300, 136), dy.transpose(0, 1).contiguous().transpose(0, 1)):
+        got = torch.autograd.grad(y, leaves, out, retain_graph=True)
+        want = torch.autograd.grad(want_y, leaves, out, retain_graph=True)
+        for g, w in zip(got, want):  # (the same products, rounded once each: two units of the last place in norm)
+            assert g.shape == w.shape and g.dtype == w.dtype and (g.float() - w.float()).norm() <= 2.0 ** -7 * w.float().norm()
+    # a gradient of a gradient is that of the tensor operations
+    for out in (y, want_y):
+        (gw,) = torch.autograd.grad((out.float() ** 2).sum(), [layer.weight], create_graph=True)
+        out.second = torch.autograd.grad(gw.float().square().sum(), [x], retain_graph=True)[0].float()
+    assert (y.second - want_y.second).norm() <= 2e-2 * want_y.second.norm()
+    # what else looks at or replaces the operation still does
+    seen = []
+    handle = layer.register_forward_hook(lambda *a: seen.append(1))
+    assert "LinearFn" not in modules._project(layer, x).grad_fn.name() and seen
+    handle.remove()
+    with torch.no_grad():
+        assert modules._project(layer, x).grad_fn is None
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert modules._project(layer, x).dtype == torch.float16
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        assert torch.autograd.forward_ad.unpack_dual(modules._project(layer, dual)).tangent is not None
+    per_sample = torch.func.vmap(lambda t: modules._project(layer, t))(x)
+    assert torch.allclose(per_sample.float(), want_y.float(), atol=2e-2)
