@@ -25,6 +25,8 @@ hipError_t launch_bwd_both_general_bf16_2(const BwdArgs &a, hipStream_t stream);
 hipError_t launch_bwd_both_general_f16_2(const BwdArgs &a, hipStream_t stream);
 hipError_t launch_bwd_win_bf16_2(const BwdArgs &a, hipStream_t stream);
 hipError_t launch_bwd_win_f16_2(const BwdArgs &a, hipStream_t stream);
+hipError_t launch_bwd_ring_bf16_2(const BwdArgs &a, hipStream_t stream);
+hipError_t launch_bwd_ring_f16_2(const BwdArgs &a, hipStream_t stream);
 
 // elementwise part of a cosine-attention window block (fb_cosine.hip)
 hipError_t launch_cosine(const fb_cosine *p, bool fp32, bool backward, hipStream_t stream);
@@ -73,6 +75,10 @@ hipError_t launch_bwd_both_general(const BwdArgs &a, bool bf16, hipStream_t stre
 // all five gradients of a short sequence in one workgroup (fb_bwd_win.hip; head dim 32)
 hipError_t launch_bwd_win(const BwdArgs &a, bool bf16, hipStream_t stream) {
     return bf16 ? launch_bwd_win_bf16_2(a, stream) : launch_bwd_win_f16_2(a, stream);
+}
+// the same without factor gradients, two workgroups per compute unit (fb_bwd_ring.hip; head dim 32)
+hipError_t launch_bwd_ring(const BwdArgs &a, bool bf16, hipStream_t stream) {
+    return bf16 ? launch_bwd_ring_bf16_2(a, stream) : launch_bwd_ring_f16_2(a, stream);
 }
 } // namespace fb
 
@@ -361,6 +367,8 @@ int fb_bwd(const fb_params *p, void *stream) {
     const int rc = fb_check(p, 1);
     if (rc) return rc;
     fb::BwdArgs a = bwd_args(p);
+    if (fb::ring_backward(a)) // ... without factor gradients
+        return launched(fb::launch_bwd_ring(a, p->dtype == FB_BF16, static_cast<hipStream_t>(stream)), "fb_bwd (ring)");
     if (fb::window_backward(a)) // whole sequences of at most 256 positions: one workgroup per (batch, head), one launch
         return launched(fb::launch_bwd_win(a, p->dtype == FB_BF16, static_cast<hipStream_t>(stream)), "fb_bwd (window)");
     const bool general_mix = p->dtype == FB_BF16 ? fb::mixed_general_backward<fb::BF16>(a) : fb::mixed_general_backward<fb::F16>(a);

@@ -149,6 +149,15 @@ inline bool window_backward(const BwdArgs &a) {
            (int64_t)((a.B + group - 1) / group) * a.H >= num_cus();
 }
 
+// Whether fb_bwd runs the ring kernel instead of the window kernel (fb_bwd_ring.hip: no factor gradients, ranks up to 16,
+// a matrix mask with rows of whole 16-byte chunks).
+inline bool ring_backward(const BwdArgs &a) {
+    if (!window_backward(a) || a.r > 16 || (a.r > 0 && a.dqb.ptr) || (int64_t)a.B * a.H < 4 * (int64_t)num_cus()) return false;
+    if (a.mask.type == kMatrixMask)
+        return a.Lk % 8 == 0 && a.mask.sm % 8 == 0 && a.mask.sb % 8 == 0 && a.mask.sh % 8 == 0 && reinterpret_cast<uintptr_t>(a.mask.ptr) % 16 == 0;
+    return true;
+}
+
 // What a launcher remembers about one kernel instantiation (one static object per instantiation;
 // the only mutable state of the library besides num_cus() and fb_bwd_static's scratch address:
 // write-once values, atomics, so concurrent first calls from several threads are fine).

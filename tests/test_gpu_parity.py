@@ -729,6 +729,44 @@ def test_window_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, group, grads
             assert errors(got, want)[1] <= max(tol, GRAD_TOL), name
 
 
+# waves without keys (64 keys each) and with half a block of them, a second half of 128 queries and none, its ragged last
+# block, one entry a workgroup and several (the last workgroup ragged), the scale folded and not
+@pytest.mark.parametrize("dtype,B,H,Lq,Lk,r,scale,shared", [
+    (torch.bfloat16, 263, 4, 256, 256, 16, None, True), (torch.bfloat16, 1029, 4, 129, 97, 8, None, True),
+    (torch.float16, 256, 4, 255, 193, 16, 1.0, False), (torch.float16, 1024, 1, 64, 144, 8, 0.3, False),
+    (torch.bfloat16, 128, 8, 144, 64, 0, None, False)])
+def test_ring_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, shared):
+    """Short sequences without factor gradients on grids of several workgroups per compute unit (fb_bwd_ring.hip): the
+    checks of test_window_backward."""
+    test_window_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, 2 if shared else 1, False)
+
+
+@pytest.mark.parametrize("kind,Lq,Lk,r,scale", [("matrix", 256, 256, 16, 1.0), ("matrix", 144, 144, 16, None), ("matrix", 130, 200, 8, None),
+                                                ("matrix", 200, 136, 0, None), ("matrix", 136, 130, 16, None), ("vector", 64, 250, 16, None),
+                                                ("vector", 256, 65, 8, 1.0)])
+def test_ring_backward_with_a_mask(gpu_device, monkeypatch, kind, Lq, Lk, r, scale):
+    """The same under additive masks (a key length without whole 16-byte chunks among them), against the oracle."""
+    from flashbias_amd import interface
+    monkeypatch.setattr(interface, "_FOLD_MIN_PAIRS", 1 << 62)
+    B, H, dtype = 258, 4, torch.bfloat16
+    q, k, v, qb, kb, do = make_inputs(B, Lq, Lk, H, 32, r, dtype, seed=Lq + Lk + r, bq=(True, False), bk=(True, False))
+    if scale == 1.0:
+        q = (q.float() / 6).to(dtype)
+    g = torch.Generator().manual_seed(3)
+    mask = torch.randn(B, 1, Lq if kind == "matrix" else 1, Lk, generator=g)
+    mask[..., Lk - Lk // 5:] = -100.0
+    if kind == "matrix":
+        mask[:, :, Lq // 2:, : Lk // 2] = float("-inf")
+    mask = mask.to(dtype)
+    ref = oracle(q, k, v, qb, kb, mask, False, scale, do)
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in (q, k, v)]
+    fac = [t.to(gpu_device) if r else None for t in (qb, kb)]
+    o = flash_bias_func(*leaves, *fac, mask.to(gpu_device), False, scale)
+    got = [t.float().cpu() for t in torch.autograd.grad(o, leaves, do.to(gpu_device))]
+    for name, a, want in zip(("dq", "dk", "dv"), got, ref[2:5]):
+        assert torch.isfinite(a).all() and errors(a, want)[1] <= GRAD_TOL, name
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,r_in,r_out", [(1000, 2, 16), (777, 5, 8), (300, 7, 16), (513, 16, 2), (129, 8, 5), (64, 20, 24),
                                              (50, 3, 6), (1, 1, 8)])
