@@ -17,6 +17,7 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
@@ -391,12 +392,14 @@ c10::optional<Tensor> linear(const Tensor &x, const Tensor &w, const c10::option
         return t.is_cuda() && t.scalar_type() == type && t.device() == x.device() && !t.key_set().has(c10::DispatchKey::Python) &&
                t.layout() == c10::kStrided && !t._fw_grad(/*level=*/0).defined();
     };
+    // (functorch's thread-local state outlives the thread's first transform; what a running one has included does not)
+    const bool transformed = c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
     const bool ready = c10::GradMode::is_enabled() && (type == torch::kFloat16 || type == torch::kBFloat16) && plain(x) && plain(w) &&
                        w.requires_grad() && x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && x.numel() > 0 &&
                        w.size(0) <= (1 << 16) && w.size(1) <= (1 << 16) &&
                        fb_weight_grad_recommended(x.numel() / x.size(-1), (int)w.size(0), (int)w.size(1)) &&
                        (!b.has_value() || (plain(*b) && b->dim() == 1 && b->size(0) == w.size(0))) &&
-                       !at::autocast::is_autocast_enabled(at::kCUDA) && !at::functorch::functorchTLSAccessor() &&
+                       !at::autocast::is_autocast_enabled(at::kCUDA) && !transformed &&
                        !c10::impl::TorchDispatchModeTLS::any_modes_set() && !at::impl::torch_function_mode_enabled() &&
                        !torch::jit::tracer::isTracing();
     if (!ready) return c10::nullopt;
