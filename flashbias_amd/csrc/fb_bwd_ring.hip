@@ -17,6 +17,11 @@
 //
 // Every query-side fragment (Q, Q_b, dO by rows and by columns) is read once per 64 keys, half of what 32 keys a
 // wave take.  All sums have a fixed order: the results are bit-reproducible.
+//
+// 4096 x 16 windows of 256 tokens, rank 16, bf16: 3.97 ms in the window kernel, 2.85 here; 1024 x 16 with shifted-window
+// masks 1.36 and 0.95.  Loads and stores alone take 1.9 ms (8.6 GB; the loads 1.08), the matrix pipe is busy for a
+// fifth of the time, the vector units for two: two waves per SIMD (240 registers) do not cover each other entirely, and
+// what would pipeline the blocks of one wave does not fit beside its operands.
 #include "fb_kernels.h"
 #include "fb_lean_tiles.h"
 
@@ -25,8 +30,11 @@ namespace fb {
 // NKR_: 16-wide steps of the rank (0, 1).  FOLD_: the scores are scale * (q k^T + q_b k_b^T), no multiply per score
 // for the scale (no factors, or a scale of exactly 1).  MASK_: an additive mask of the 16-bit type, a vector mask as
 // one value per lane (key) or a matrix mask as a 32 x 32 tile per block, copied to LDS by the wave that uses it.
-template <class T, int NKR_, bool FOLD_, int MASK_>
+// HIDE_: some wave's 64 keys are not all there, their scores are set to -inf (a branch on it inside the step cost 200
+// bytes of scratch).
+template <class T, int NKR_, bool FOLD_, int MASK_, bool HIDE_>
 struct RingCfg {
+    static constexpr bool HIDE = HIDE_;
     static constexpr bool FOLD = FOLD_, MASK = MASK_ == kMatrixMask, VMASK = MASK_ == kVectorMask;
     static constexpr int NKD = 2, NKR = NKR_, NK = NKD + NKR_;
     static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES, KBW = 2, LQ = 256, HALF = 128;
@@ -36,6 +44,28 @@ struct RingCfg {
                          STAT = DS + NWAVES * 2048, MT = STAT + 2 * LQ * 4, LDS_BYTES = MT + (MASK ? NWAVES * 2048 : 0);
     static_assert(LDS_BYTES <= 80 * 1024, "two workgroups per compute unit");
 };
+
+// A 32 x 32 accumulator block (lane = row, as store_acc_rows takes it) to rows [row0, row0 + 32) of a tensor through 2 KB
+// of LDS that only this wave touches: packed, written by rows, read back in the order of a copy (lean_copy_place), so
+// that four neighbouring lanes store a row of 64 bytes.
+template <class T>
+__device__ __forceinline__ void store_block_rows(const Tensor &t, int b, int h, int row0, int nrows, const f32x16_t &acc, float mul,
+                                                 uint8_t *buf, int lane) {
+    const int c = lane & 31, g = lane >> 5;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<u32x2_t *>(buf + lean_chunk_off<4>(c, j) + 8 * g) =
+            u32x2_t{T::pack2(acc[4 * j] * mul, acc[4 * j + 1] * mul), T::pack2(acc[4 * j + 2] * mul, acc[4 * j + 3] * mul)};
+    uint16_t *base = const_cast<uint16_t *>(t.ptr) + b * t.sb + h * t.sh;
+    int row, chunk;
+    lean_copy_place<4>(lane, row, chunk);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const u32x4_t x = *reinterpret_cast<const u32x4_t *>(buf + j * 1024 + lane * 16);
+        const int r = row0 + 16 * j + row;
+        if (r < nrows) *reinterpret_cast<u32x4_t *>(base + (int64_t)r * t.ss + 8 * chunk) = x;
+    }
+}
 
 template <class T, class C>
 __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_ring_kernel(const BwdArgs a) {
@@ -203,82 +233,153 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
                     da[t] = lds_load16(rows + C::DO + row_off[t]);
                 }
                 if constexpr (C::NKR > 0) qa[C::NKD] = lds_load16(qb_row + (r0 >> 5) * 1024);
+                f32x16_t lse2;
+                auto lses = [&]() { // register v <-> query r0 + 8 (v / 4) + 4 g + v % 4
 #pragma unroll
-                for (int kb = 0; kb < C::KBW; ++kb) {
-                    const int key = wk0 + 32 * kb + c;
-                    f32x16_t s, dp;
-                    u32x4_t mt[2];
+                    for (int j = 0; j < 4; ++j) {
+                        const f32x4_t x = *reinterpret_cast<const f32x4_t *>(smem + C::STAT + 4 * (r0 + 8 * j + 4 * g));
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) lse2[4 * j + e] = x[e];
+                    }
+                };
+                u32x4_t mt[2]; // mask values of the block, packed in the same order
+                auto mask_tile = [&](int kb) {
                     if constexpr (C::MASK) {
                         wait_vmcnt<0>();
 #pragma unroll
                         for (int t = 0; t < 2; ++t) mt[t] = lds_load_tr(lds_m + col_off[0] + t * 1024, lds_m + col_off[1] + t * 1024);
-                    }
-                    auto mask_at = [&](int v) { return T::to_float((uint16_t)(v & 1 ? mt[v >> 3][(v & 7) >> 1] >> 16 : mt[v >> 3][(v & 7) >> 1] & 0xffffu)); };
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) s[v] = C::FOLD ? (C::MASK ? mask_at(v) : C::VMASK ? mkey[kb] : 0.f) : 0.f;
-#pragma unroll
-                    for (int t = 0; t < C::NKD; ++t) s = T::mfma(qa[t], kr[kb][t], s);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) { // register v <-> query r0 + 8 (v / 4) + 4 g + v % 4
-                        const f32x4_t d4 = *reinterpret_cast<const f32x4_t *>(smem + C::STAT + 4 * (C::LQ + r0 + 8 * j + 4 * g));
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) dp[4 * j + e] = d4[e];
-                    }
-#pragma unroll
-                    for (int t = 0; t < C::NKD; ++t) dp = T::mfma(da[t], vr[kb][t], dp);
-                    if constexpr (!C::FOLD) { // the softmax scale multiplies q k^T only (flash_bias_triton.py:248)
-#pragma unroll
-                        for (int v = 0; v < 16; ++v)
-                            s[v] = C::MASK ? __builtin_fmaf(s[v], a.scale, mask_at(v)) : C::VMASK ? __builtin_fmaf(s[v], a.scale, mkey[kb]) : s[v] * a.scale;
-                    }
-                    if constexpr (C::MASK) { // the tile after this one: the other key block, then the next step's query block
-                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (its values have left LDS)
+                        // the tile after this one, once these values have left LDS: the other key block, then the next step's
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                         if (kb + 1 < C::KBW)
                             copy_mask(r0, wk0 + 32 * kb + 32);
                         else if (step + 1 < nsteps)
                             copy_mask(next_r0, wk0);
                     }
-                    if constexpr (C::NKR > 0) s = T::mfma(qa[C::NKD], kbr[kb][0], s);
-                    if (wk0 + 32 * kb + 32 > a.Lk) {
+                };
+                auto mask_at = [&](int v) { return T::to_float((uint16_t)(v & 1 ? mt[v >> 3][(v & 7) >> 1] >> 16 : mt[v >> 3][(v & 7) >> 1] & 0xffffu)); };
+                auto scores = [&](int kb, f32x16_t &s) { // q k^T
+                    mask_tile(kb);
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) s[v] = C::FOLD && C::MASK ? mask_at(v) : 0.f;
+#pragma unroll
+                    for (int t = 0; t < C::NKD; ++t) s = T::mfma(qa[t], kr[kb][t], s);
+                };
+                auto bias = [&](int kb, f32x16_t &s) { // the softmax scale multiplies q k^T only (flash_bias_triton.py:248)
+                    if constexpr (!C::FOLD) {
 #pragma unroll
                         for (int v = 0; v < 16; ++v)
-                            if (key >= a.Lk) s[v] = -INFINITY;
+                            s[v] = C::MASK ? __builtin_fmaf(s[v], a.scale, mask_at(v)) : C::VMASK ? __builtin_fmaf(s[v], a.scale, mkey[kb]) : s[v] * a.scale;
                     }
-                    asm volatile("s_nop 11" : "+v"(s), "+v"(dp)); // (fb_bwd_win.hip: wait states across the branch above)
-                    u32x4_t pp[2], pds[2]; // P and dS, packed, per 16-query step
+                    if constexpr (C::NKR > 0) s = T::mfma(qa[C::NKD], kbr[kb][0], s);
+                    if constexpr (C::HIDE) {
+                        const int key = wk0 + 32 * kb + c;
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) s[v] = key < a.Lk ? s[v] : -INFINITY;
+                    }
+                };
+                auto deltas = [&](f32x16_t &dp) { // dO V^T - delta: -delta is the initial value
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        const f32x4_t l4 = *reinterpret_cast<const f32x4_t *>(smem + C::STAT + 4 * (r0 + 8 * j + 4 * g));
+                        const f32x4_t x = *reinterpret_cast<const f32x4_t *>(smem + C::STAT + 4 * (C::LQ + r0 + 8 * j + 4 * g));
 #pragma unroll
-                        for (int e = 0; e < 4; e += 2) {
-                            const int v = 4 * j + e;
-                            const float p0 = fast_exp2(__builtin_fmaf(s[v], to_log2, -l4[e]));
-                            const float p1 = fast_exp2(__builtin_fmaf(s[v + 1], to_log2, -l4[e + 1]));
-                            pp[v >> 3][(v & 7) >> 1] = T::pack2(p0, p1);
-                            pds[v >> 3][(v & 7) >> 1] = T::pack2(p0 * dp[v], p1 * dp[v + 1]);
-                        }
+                        for (int e = 0; e < 4; ++e) dp[4 * j + e] = x[e];
                     }
-                    // dS of (this key, queries 16 t + 8 half + 4 g + 0..3) -> row c of the wave's dS block, read back column-wise
+                };
+                auto grads = [&](int kb, f32x16_t &dp) {
+#pragma unroll
+                    for (int t = 0; t < C::NKD; ++t) dp = T::mfma(da[t], vr[kb][t], dp);
+                };
+                // P and dS, packed per 16-query step; dS of (this key, queries 16 t + 8 half + 4 g + 0..3) also to row c of the
+                // wave's dS block, which comes back column-wise (lane = query)
+                const uint32_t ds = lds0 + C::DS + wave * 2048;
+                u32x4_t pp[2], pds[2], dsb[2];
+                auto probs = [&](const f32x16_t &s, const f32x16_t &dp) {
+#pragma unroll
+                    for (int v = 0; v < 16; v += 2) {
+                        const float p0 = fast_exp2(__builtin_fmaf(s[v], to_log2, -lse2[v]));
+                        const float p1 = fast_exp2(__builtin_fmaf(s[v + 1], to_log2, -lse2[v + 1]));
+                        pp[v >> 3][(v & 7) >> 1] = T::pack2(p0, p1);
+                        pds[v >> 3][(v & 7) >> 1] = T::pack2(p0 * dp[v], p1 * dp[v + 1]);
+                    }
 #pragma unroll
                     for (int t = 0; t < 2; ++t)
 #pragma unroll
                         for (int half = 0; half < 2; ++half)
                             *reinterpret_cast<u32x2_t *>(smem + C::DS + wave * 2048 + lean_chunk_off<4>(c, 2 * t + half) + 8 * g) =
                                 u32x2_t{pds[t][2 * half], pds[t][2 * half + 1]};
-                    // dV^T += dO^T P ; dK^T += Q^T dS  (contraction over this block's queries)
+                };
+                auto block_back = [&]() {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) dsb[t] = lds_load_tr(ds + col_off[0] + t * 1024, ds + col_off[1] + t * 1024);
+                };
+                u32x4_t dot[2], qt[2]; // dO^T and Q^T of the block, for both key blocks
+                auto sums = [&](int kb) { // dV^T += dO^T P ; dK^T += Q^T dS  (contraction over the block's queries)
 #pragma unroll
                     for (int t = 0; t < 2; ++t) {
-                        const u32x4_t dot = lds_load_tr(rows + C::DO + col_off[0] + t * 1024, rows + C::DO + col_off[1] + t * 1024);
-                        acc_dv[kb] = T::mfma(dot, pp[t], acc_dv[kb]);
-                        const u32x4_t qt = lds_load_tr(rows + C::Q + col_off[0] + t * 1024, rows + C::Q + col_off[1] + t * 1024);
-                        acc_dk[kb] = T::mfma(qt, pds[t], acc_dk[kb]);
+                        acc_dv[kb] = T::mfma(dot[t], pp[t], acc_dv[kb]);
+                        acc_dk[kb] = T::mfma(qt[t], pds[t], acc_dk[kb]);
                     }
-                    // dQ^T += K^T dS^T over these 32 keys
-                    const uint32_t dst = lds0 + C::DS + wave * 2048;
+                };
+                auto query_sums = [&](int kb) { // dQ^T += K^T dS^T over the 32 keys
 #pragma unroll
-                    for (int t = 0; t < 2; ++t)
-                        dq = T::mfma(kt[kb][t], lds_load_tr(dst + col_off[0] + t * 1024, dst + col_off[1] + t * 1024), dq);
+                    for (int t = 0; t < 2; ++t) dq = T::mfma(kt[kb][t], dsb[t], dq);
+                };
+                auto columns = [&]() {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        dot[t] = lds_load_tr(rows + C::DO + col_off[0] + t * 1024, rows + C::DO + col_off[1] + t * 1024);
+                        qt[t] = lds_load_tr(rows + C::Q + col_off[0] + t * 1024, rows + C::Q + col_off[1] + t * 1024);
+                    }
+                };
+                // The second block's first products stand between the first one's dS and its way back from LDS, and the
+                // wave that feeds the matrix pipe goes first.  4096 x 16 windows of 256 tokens, rank 16: block after block
+                // 3.10 ms, this order 2.95, with the priorities 2.89.  A matrix mask's values do not fit beside two blocks.
+                if constexpr (!C::MASK) {
+                    f32x16_t s0, dp0, s1, dp1;
+                    __builtin_amdgcn_s_setprio(1);
+                    lses();
+                    deltas(dp0);
+                    scores(0, s0);
+                    grads(0, dp0);
+                    bias(0, s0);
+                    columns();
+                    __builtin_amdgcn_s_setprio(0);
+                    probs(s0, dp0);
+                    __builtin_amdgcn_s_setprio(1);
+                    block_back();
+                    deltas(dp1);
+                    scores(1, s1);
+                    sums(0);
+                    grads(1, dp1);
+                    bias(1, s1);
+                    lses();
+                    query_sums(0);
+                    __builtin_amdgcn_s_setprio(0);
+                    probs(s1, dp1);
+                    __builtin_amdgcn_s_setprio(1);
+                    block_back();
+                    sums(1);
+                    query_sums(1);
+                } else {
+#pragma unroll
+                    for (int kb = 0; kb < C::KBW; ++kb) {
+                        f32x16_t s, dp;
+                        __builtin_amdgcn_s_setprio(1);
+                        scores(kb, s);
+                        deltas(dp);
+                        grads(kb, dp);
+                        bias(kb, s);
+                        lses();
+                        __builtin_amdgcn_s_setprio(0);
+                        probs(s, dp);
+                        __builtin_amdgcn_s_setprio(1);
+                        columns();
+                        block_back();
+                        sums(kb);
+                        query_sums(kb);
+                    }
                 }
+                __builtin_amdgcn_s_setprio(0);
             } else if (C::MASK && visible && step + 1 < nsteps) { // (a block past the end: its tile is replaced by the next step's)
                 wait_vmcnt<0>();
                 copy_mask(next_r0, wk0);
@@ -288,10 +389,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
 #pragma unroll
                 for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4_t *>(acc + 256 * j) = f32x4_t{dq[4 * j], dq[4 * j + 1], dq[4 * j + 2], dq[4 * j + 3]};
             } else {
-                const int query = r0 + c;
-                const bool ok = query < a.Lq;
-                uint16_t *row = const_cast<uint16_t *>(a.dq.ptr) + b * a.dq.sb + h * a.dq.sh + (int64_t)(ok ? query : 0) * a.dq.ss;
-                store_acc_rows<T, true>(row, ok, a.dq.vec_ok, dq, a.scale, a.d, g);
+                store_block_rows<T>(a.dq, b, h, r0, a.Lq, dq, a.scale, smem + C::DS + wave * 2048, lane);
             }
             barrier_lds(); // the accumulators are handed on
         }
@@ -299,27 +397,24 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
 #pragma unroll
         for (int kb = 0; kb < C::KBW; ++kb) {
             asm volatile("s_nop 11" : "+v"(acc_dv[kb]), "+v"(acc_dk[kb]));
-            int key = wk0 + 32 * kb + c;
-            asm volatile("" : "+v"(key));
-            const bool ok = key < a.Lk;
-            const int64_t krow = ok ? key : 0;
-            store_acc_rows<T, true>(const_cast<uint16_t *>(a.dv.ptr) + b * a.dv.sb + h * a.dv.sh + krow * a.dv.ss, ok, a.dv.vec_ok, acc_dv[kb], 1.f, a.d, g);
-            store_acc_rows<T, true>(const_cast<uint16_t *>(a.dk.ptr) + b * a.dk.sb + h * a.dk.sh + krow * a.dk.ss, ok, a.dk.vec_ok, acc_dk[kb], a.scale, a.d, g);
+            store_block_rows<T>(a.dv, b, h, wk0 + 32 * kb, a.Lk, acc_dv[kb], 1.f, smem + C::DS + wave * 2048, lane);
+            store_block_rows<T>(a.dk, b, h, wk0 + 32 * kb, a.Lk, acc_dk[kb], a.scale, smem + C::DS + wave * 2048, lane);
         }
     }
 }
 
-template <class T, int NKR, bool FOLD, int MASK>
+template <class T, int NKR, bool FOLD, int MASK, bool HIDE>
 static hipError_t launch_ring_cfg(const BwdArgs &a, hipStream_t stream) {
-    typedef RingCfg<T, NKR, FOLD, MASK> C;
+    typedef RingCfg<T, NKR, FOLD, MASK, HIDE> C;
     auto kern = bwd_ring_kernel<T, C>;
     static KernelOnce once;
     const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
     if (e != hipSuccess) return e;
     BwdArgs b = a;
     b.walk = 1;
-    // as many batch entries a workgroup as leave eight workgroups per compute unit
-    for (int w = 32; w > 1; w /= 2)
+    // Up to eight batch entries a workgroup (the factors and the cleared LDS are kept), as many as leave eight workgroups
+    // per compute unit: 4096 x 16 windows 2.96 ms with 32 entries, 2.90 with 16, 2.87 with 8, 2.86 with 4.
+    for (int w = 8; w > 1; w /= 2)
         if ((int64_t)((a.B + w - 1) / w) * a.H >= 8 * (int64_t)num_cus()) {
             b.walk = w;
             break;
@@ -327,16 +422,20 @@ static hipError_t launch_ring_cfg(const BwdArgs &a, hipStream_t stream) {
     return launch_flat(kern, (int64_t)((a.B + b.walk - 1) / b.walk) * a.H, C::NTHREADS, C::LDS_BYTES, stream, b);
 }
 
+template <class T, int NKR, int MASK>
+static hipError_t launch_ring_m(const BwdArgs &a, bool fold, hipStream_t stream) {
+    const bool hide = a.Lk % 64 != 0;
+    if constexpr (MASK != kVectorMask) // (there the mask rides on the scale's FMA)
+        if (fold) return hide ? launch_ring_cfg<T, NKR, true, MASK, true>(a, stream) : launch_ring_cfg<T, NKR, true, MASK, false>(a, stream);
+    return hide ? launch_ring_cfg<T, NKR, false, MASK, true>(a, stream) : launch_ring_cfg<T, NKR, false, MASK, false>(a, stream);
+}
+
 template <class T, int NKR>
 static hipError_t launch_ring_r(const BwdArgs &a, hipStream_t stream) {
-    const bool one = a.scale == 1.f;
     switch (a.mask.type) {
-    case kNoMask:
-        return one || a.r == 0 ? launch_ring_cfg<T, NKR, true, kNoMask>(a, stream) : launch_ring_cfg<T, NKR, false, kNoMask>(a, stream);
-    case kVectorMask: // (the mask is not divided by the scale)
-        return one ? launch_ring_cfg<T, NKR, true, kVectorMask>(a, stream) : launch_ring_cfg<T, NKR, false, kVectorMask>(a, stream);
-    default:
-        return one ? launch_ring_cfg<T, NKR, true, kMatrixMask>(a, stream) : launch_ring_cfg<T, NKR, false, kMatrixMask>(a, stream);
+    case kNoMask: return launch_ring_m<T, NKR, kNoMask>(a, a.r == 0 || a.scale == 1.f, stream);
+    case kVectorMask: return launch_ring_m<T, NKR, kVectorMask>(a, false, stream);
+    default: return launch_ring_m<T, NKR, kMatrixMask>(a, a.scale == 1.f, stream);
     }
 }
 

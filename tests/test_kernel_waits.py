@@ -63,3 +63,12 @@ def test_compiled_kernels():
             text = f.read()
         assert text.count("v_mfma_f32_32x32x16") > 100, unit
         assert waits.check(text) == [], unit
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None or shutil.which("make") is None, reason="needs hipcc and make")
+def test_compiled_ring_kernel():
+    unit = "build/asm/fb_bwd_ring_bf16_2.s"
+    subprocess.run(["make", unit], cwd=CSRC, check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    with open(os.path.join(CSRC, unit)) as f:
+        text = f.read()
+    assert text.count("v_mfma_f32_32x32x16") > 100 and waits.check(text) == []
