@@ -25,6 +25,8 @@ hipError_t launch_bwd_both_general_bf16_2(const BwdArgs &a, hipStream_t stream);
 hipError_t launch_bwd_both_general_f16_2(const BwdArgs &a, hipStream_t stream);
 hipError_t launch_bwd_win_bf16_2(const BwdArgs &a, hipStream_t stream);
 hipError_t launch_bwd_win_f16_2(const BwdArgs &a, hipStream_t stream);
+hipError_t launch_fwd_win_bf16_2(const FwdArgs &a, hipStream_t stream);
+hipError_t launch_fwd_win_f16_2(const FwdArgs &a, hipStream_t stream);
 hipError_t launch_bwd_ring_bf16_2(const BwdArgs &a, hipStream_t stream);
 hipError_t launch_bwd_ring_f16_2(const BwdArgs &a, hipStream_t stream);
 
@@ -39,6 +41,7 @@ hipError_t launch_wgrad(const void *dy, int64_t ldy, const void *x, int64_t ldx,
                         int n, int k, bool bf16, hipStream_t stream);
 
 hipError_t launch_fwd(const FwdArgs &a, bool bf16, hipStream_t stream) {
+    if (window_forward(a)) return bf16 ? launch_fwd_win_bf16_2(a, stream) : launch_fwd_win_f16_2(a, stream);
     switch (nkd_of(a.d)) {
     case 1: return bf16 ? launch_fwd_bf16_1(a, stream) : launch_fwd_f16_1(a, stream);
     case 2: return bf16 ? launch_fwd_bf16_2(a, stream) : launch_fwd_f16_2(a, stream);

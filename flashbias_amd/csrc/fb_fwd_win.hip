@@ -1,0 +1,240 @@
+// Forward for windows: head dim 32, Lq, Lk <= 256, rank up to 16, no mask or a 16-bit matrix mask, aligned tensors (the
+// window attention of 2_Vision_Transformer/swin_transformer_v2.py:178-203).  The arithmetic is that of fwd_kernel: one
+// query per lane, S^T = [K | K_b] [Q | Q_b]^T, online softmax against a lagging reference point, O^T += V^T P^T with P
+// from registers.
+//
+// The general kernel gives a window a workgroup that holds half of the compute unit's registers, and spends its life in
+// turn on the first tile's way from memory, eight 32-key blocks and the stores.  Here a window's K, K_b and V take 40 KB, a
+// wave works on one block of 32 queries at a time in 128 registers, and four workgroups (mask: three) share a
+// compute unit: nothing is pipelined by hand, whatever one waits for the others fill.
+#include "fb_kernels.h"
+#include "fb_lean_tiles.h"
+
+namespace fb {
+
+// FOLD_: the scores are scale * (q k^T + q_b k_b^T) in one chain (no factors, or a scale of exactly 1).
+// MASK_: a matrix mask, whose 32 x 32 blocks the wave that uses them copies to LDS one ahead.
+template <class T, int NKR_, bool FOLD_, bool MASK_>
+struct FwdWinCfg {
+    static constexpr bool FOLD = FOLD_, MASK = MASK_;
+    static constexpr int NKD = 2, NKR = NKR_, NK = NKD + NKR_;
+    static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES, LK = 256;
+    static constexpr int K = 0, V = K + LK * 64, KB = V + LK * 64, MT = KB + (NKR ? LK * 32 : 0), LDS_BYTES = MT + (MASK ? NWAVES * 2048 : 0);
+    static constexpr int WAVES_EU = MASK ? 3 : 4;
+    static_assert(WAVES_EU * LDS_BYTES <= 160 * 1024, "");
+};
+
+template <class T, class C>
+__global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::WAVES_EU, C::WAVES_EU))) void fwd_win_kernel(const FwdArgs a, int walk) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const uint32_t lds0 = lds_addr_of(smem);
+    const int lane = threadIdx.x & 63, c = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+
+    // a workgroup walks `walk` consecutive batch entries of its head
+    const int nbg = (a.B + walk - 1) / walk;
+    const int work = xcd_remap(blockIdx.x, nbg * a.H);
+    const int bg = work / a.H, h = work % a.H;
+    const int nqb = (a.Lq + 31) / 32, nkb = (a.Lk + 31) / 32;
+
+    if constexpr (C::NKR > 0) { // (the channel padding of a rank below 16 is never written)
+        for (int i = threadIdx.x; i < C::LK * 2; i += C::NTHREADS) reinterpret_cast<u32x4_t *>(smem + C::KB)[i] = u32x4_t{0u, 0u, 0u, 0u};
+        __syncthreads();
+    }
+    const float to_log2 = C::FOLD ? a.scale * kLog2e : kLog2e, lag = 8.f / to_log2;
+    const uint32_t row_off[2] = {lds0 + lean_row_addr<4>(c, g), lds0 + lean_row_addr<4>(c, 2 + g)};
+    const uint32_t col_off[2] = {lds0 + C::V + lean_tr_addr4(c, g, 0), lds0 + C::V + lean_tr_addr4(c, g, 1)};
+    const uint32_t kb_row = lds0 + C::KB + lean_row_addr<2>(c, g);
+    const uint32_t lds_m = lds0 + C::MT + wave * 2048;
+
+    for (int bi = 0; bi < walk; ++bi) {
+        const int b = __builtin_amdgcn_readfirstlane(bg * walk + bi);
+        if (b >= a.B) break;
+        {   // K and V: 16 rows a copy instruction, whole blocks of 32 keys (rows past the end: the last one again)
+            const uint8_t *kbase = reinterpret_cast<const uint8_t *>(a.k.ptr + b * a.k.sb + h * a.k.sh);
+            const uint8_t *vbase = reinterpret_cast<const uint8_t *>(a.v.ptr + b * a.v.sb + h * a.v.sh);
+            int row, chunk;
+            lean_copy_place<4>(lane, row, chunk);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = wave + C::NWAVES * j, r = min(16 * i + row, a.Lk - 1);
+                if (i < 2 * nkb) {
+                    lds_dma16_all((uint32_t)(r * (int)(a.k.ss * 2) + chunk * 16), kbase, lds0 + C::K + i * 1024);
+                    lds_dma16_all((uint32_t)(r * (int)(a.v.ss * 2) + chunk * 16), vbase, lds0 + C::V + i * 1024);
+                }
+            }
+            if constexpr (C::NKR > 0) {
+                if (bi == 0 || a.kb.sb != 0) {
+                    DenseCopy<C::LK / 2, 2> cb;
+                    cb.init(a.kb.ptr + b * a.kb.sb + h * a.kb.sh, a.kb.ss, a.r, false, wave, lane, 0);
+                    cb.issue(lds0 + C::KB, 0, a.Lk);
+                    // (only where it has rows: the copy's offsets count down from the half's first row, unsigned)
+                    if (a.Lk > C::LK / 2) cb.issue(lds0 + C::KB + C::LK * 16, C::LK / 2, a.Lk);
+                }
+            }
+        }
+        const uint16_t *qbase = a.q.ptr + b * a.q.sb + h * a.q.sh, *qbbase = C::NKR > 0 ? a.qb.ptr + b * a.qb.sb + h * a.qb.sh : nullptr;
+        u32x4_t qn[C::NK]; // the next block's query operand
+        auto load_q = [&](int qb) {
+            const int query = min(32 * qb + c, a.Lq - 1);
+#pragma unroll
+            for (int t = 0; t < C::NKD; ++t) qn[t] = *reinterpret_cast<const u32x4_t *>(qbase + (int64_t)query * a.q.ss + 16 * t + 8 * g);
+            if constexpr (C::NKR > 0) qn[C::NKD] = load_chunk<true>(qbbase, a.qb.ss, query, a.Lq, 8 * g, a.r);
+        };
+        if (wave < nqb) load_q(wave);
+        // Mask block (queries 32 qb .., keys 32 kb ..) as 32 rows of 64 bytes; rows and 16-byte chunks past the end re-read
+        // the last ones.
+        const uint8_t *mbase = nullptr;
+        if constexpr (C::MASK) mbase = reinterpret_cast<const uint8_t *>(a.mask.ptr) + mask_offset(a.mask, b, h) * 2;
+        auto copy_mask = [&](int qb, int kb) {
+            int row, chunk;
+            lean_copy_place<4>(lane, row, chunk);
+            const int col = min(32 * kb + 8 * chunk, a.Lk - 8);
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                lds_dma16_all((uint32_t)(min(32 * qb + 16 * j + row, a.Lq - 1) * (int)(a.mask.sm * 2) + col * 2), mbase, lds_m + j * 1024);
+        };
+        if constexpr (C::MASK) {
+            if (wave < nqb) copy_mask(wave, 0);
+        }
+        wait_vmcnt<0>();
+        barrier_lds();
+
+#pragma unroll 1
+        for (int qb = wave; qb < nqb; qb += C::NWAVES) {
+            u32x4_t q[C::NK];
+#pragma unroll
+            for (int t = 0; t < C::NK; ++t) q[t] = qn[t];
+            if (qb + C::NWAVES < nqb) load_q(qb + C::NWAVES);
+            f32x16_t o;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) o[v] = 0.f;
+            float m_ref = -INFINITY, m2 = 0.f, l_run = 0.f;
+#pragma unroll 1
+            for (int kb = 0; kb < nkb; ++kb) {
+                const uint32_t at = kb * 2048;
+                f32x16_t s, sb;
+                if constexpr (C::MASK) {
+                    wait_vmcnt<0>();
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) { // register v <-> key 32 kb + 8 (v / 4) + 4 g + v % 4 of the lane's row
+                        const u32x2_t x = *reinterpret_cast<const u32x2_t *>(smem + C::MT + wave * 2048 + lean_chunk_off<4>(c, j) + 8 * g);
+                        sb[4 * j + 0] = T::to_float((uint16_t)(x[0] & 0xffffu));
+                        sb[4 * j + 1] = T::to_float((uint16_t)(x[0] >> 16));
+                        sb[4 * j + 2] = T::to_float((uint16_t)(x[1] & 0xffffu));
+                        sb[4 * j + 3] = T::to_float((uint16_t)(x[1] >> 16));
+                    }
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (they have left LDS: the block after this one)
+                    if (kb + 1 < nkb)
+                        copy_mask(qb, kb + 1);
+                    else if (qb + C::NWAVES < nqb)
+                        copy_mask(qb + C::NWAVES, 0);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) sb[v] = 0.f;
+                }
+                // q k^T and q_b k_b^T: two chains joined by the FMA that applies the softmax scale to the first (:246-256),
+                // an additive mask the initial value of the second; folded, one chain
+                if constexpr (C::FOLD)
+                    s = sb;
+                else
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) s[v] = 0.f;
+#pragma unroll
+                for (int t = 0; t < C::NKD; ++t) s = T::mfma(lds_load16(row_off[t] + C::K + at), q[t], s);
+                if constexpr (C::NKR > 0) {
+                    const u32x4_t kf = lds_load16(kb_row + kb * 1024);
+                    if constexpr (C::FOLD)
+                        s = T::mfma(kf, q[C::NKD], s);
+                    else
+                        sb = T::mfma(kf, q[C::NKD], sb);
+                }
+                if constexpr (!C::FOLD) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) s[v] = __builtin_fmaf(s[v], a.scale, sb[v]);
+                }
+                u32x4_t vt[2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) vt[t] = lds_load_tr(col_off[0] + at + t * 1024, col_off[1] + at + t * 1024);
+                if (32 * kb + 32 > a.Lk) {
+                    const int key0 = 32 * kb + 4 * g;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v)
+                        if (key0 + 8 * (v >> 2) + (v & 3) >= a.Lk) s[v] = -INFINITY;
+                }
+                asm volatile("s_nop 11" : "+v"(s)); // (fb_bwd_win.hip: wait states across the branch above)
+                float mx = s[0];
+#pragma unroll
+                for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
+                mx = half_wave_max(mx);
+                const bool grow = mx > m_ref + lag; // also true for the first finite score of a row
+                if (__any(grow)) {
+                    const float m_new = grow ? mx : m_ref;
+                    const float alpha = grow ? fast_exp2((m_ref - m_new) * to_log2) : 1.f; // exp2(-inf) = 0
+                    l_run *= alpha;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) o[v] *= alpha;
+                    m_ref = m_new;
+                    m2 = (m_new == -INFINITY) ? 0.f : m_new * to_log2;
+                }
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    u32x4_t pb;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float p0 = fast_exp2(__builtin_fmaf(s[8 * t + 2 * e], to_log2, -m2));
+                        const float p1 = fast_exp2(__builtin_fmaf(s[8 * t + 2 * e + 1], to_log2, -m2));
+                        pb[e] = T::pack2(p0, p1);
+                        l_run += p0 + p1;
+                    }
+                    o = T::mfma(vt[t], pb, o);
+                }
+                asm volatile("s_nop 11" : "+v"(o)); // (across the loop's branches)
+            }
+            const float l = l_run + __shfl_xor(l_run, 32, 64);
+            const int query = 32 * qb + c;
+            const bool ok = query < a.Lq;
+            if (ok && g == 0) a.lse[((int64_t)b * a.H + h) * a.Lq + query] = m_ref * (C::FOLD ? a.scale : 1.f) + __builtin_amdgcn_logf(l) * kLn2;
+            uint16_t *orow = const_cast<uint16_t *>(a.o.ptr) + b * a.o.sb + h * a.o.sh + (int64_t)(ok ? query : 0) * a.o.ss;
+            store_acc_rows<T, true>(orow, ok, true, o, 1.f / l, a.d, g);
+        }
+        if (bi + 1 < walk) barrier_lds(); // everyone has read K and V
+    }
+}
+
+template <class T, int NKR, bool FOLD, bool MASK>
+static hipError_t launch_fwd_win_cfg(const FwdArgs &a, hipStream_t stream) {
+    typedef FwdWinCfg<T, NKR, FOLD, MASK> C;
+    auto kern = fwd_win_kernel<T, C>;
+    static KernelOnce once;
+    const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
+    if (e != hipSuccess) return e;
+    int walk = 1;
+    for (int w = 8; w > 1; w /= 2)
+        if ((int64_t)((a.B + w - 1) / w) * a.H >= 16 * (int64_t)num_cus()) {
+            walk = w;
+            break;
+        }
+    const int64_t total = (int64_t)((a.B + walk - 1) / walk) * a.H;
+    if (total <= 0 || total > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(C::NTHREADS), C::LDS_BYTES, stream, a, walk);
+    return hipGetLastError();
+}
+
+template <class T, int NKR>
+static hipError_t launch_fwd_win_r(const FwdArgs &a, hipStream_t stream) {
+    if (a.mask.type == kMatrixMask) // (the mask is not divided by the scale)
+        return a.scale == 1.f ? launch_fwd_win_cfg<T, NKR, true, true>(a, stream) : launch_fwd_win_cfg<T, NKR, false, true>(a, stream);
+    return a.r == 0 || a.scale == 1.f ? launch_fwd_win_cfg<T, NKR, true, false>(a, stream) : launch_fwd_win_cfg<T, NKR, false, false>(a, stream);
+}
+
+// Compiled once per element type for head dim 32 (see Makefile).  When fb_fwd takes this path is decided by
+// window_forward() in fb_kernels.h.
+#define FB_CAT2(a, b) a##b
+#define FB_CAT(a, b) FB_CAT2(a, b)
+hipError_t FB_CAT(launch_fwd_win_, FB_SUFFIX)(const FwdArgs &a, hipStream_t stream) {
+    return a.r == 0 ? launch_fwd_win_r<FB_T, 0>(a, stream) : launch_fwd_win_r<FB_T, 1>(a, stream);
+}
+
+} // namespace fb

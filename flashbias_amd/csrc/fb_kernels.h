@@ -149,6 +149,12 @@ inline bool window_backward(const BwdArgs &a) {
            (int64_t)((a.B + group - 1) / group) * a.H >= num_cus();
 }
 
+// A 16-bit matrix mask whose rows are whole, aligned 16-byte chunks: the window kernels copy its blocks to LDS.
+inline bool mask_in_chunks(const MaskDesc &m, int Lk) {
+    return !m.is_f32 && m.type == kMatrixMask && Lk % 8 == 0 && m.sm % 8 == 0 && m.sm < ((int64_t)1 << 22) && m.sb % 8 == 0 && m.sh % 8 == 0 &&
+           reinterpret_cast<uintptr_t>(m.ptr) % 16 == 0;
+}
+
 // Whether fb_bwd runs the ring kernel instead of the window kernel (fb_bwd_ring.hip: no factor gradients, ranks up to 16,
 // a matrix mask with rows of whole 16-byte chunks).  Ring against window kernel, rank 16, us: 640 pairs of 256 tokens 42 / 60,
 // 1024 54 / 82, 8192 x (144, 192, 224 tokens) 269 / 372, 313 / 418, 379 / 490, with a matrix mask 323 / 470, 371 / 528,
@@ -156,9 +162,23 @@ inline bool window_backward(const BwdArgs &a) {
 // the window kernel keeps dq, dk and dv bit for bit those of the call that computes the factor gradients too.
 inline bool ring_backward(const BwdArgs &a) {
     if (!window_backward(a) || a.r > 16 || (a.r > 0 && a.dqb.ptr) || (int64_t)a.B * a.H < 4 * (int64_t)num_cus()) return false;
-    if (a.mask.type == kMatrixMask)
-        return a.Lk % 8 == 0 && a.mask.sm % 8 == 0 && a.mask.sb % 8 == 0 && a.mask.sh % 8 == 0 && reinterpret_cast<uintptr_t>(a.mask.ptr) % 16 == 0;
-    return true;
+    return a.mask.type != kMatrixMask || mask_in_chunks(a.mask, a.Lk);
+}
+
+// Whether fb_fwd runs the forward for windows (fb_fwd_win.hip): whole sequences of at most 256 positions, head dim 32, a
+// rank up to 16, aligned tensors, no mask or a matrix mask of 16-byte chunks, a scale that keeps the order of the scores.
+// Against the general kernel, rank 16, us (window / general): 8192 pairs of 64 tokens 35 / 55, of 128 66 / 75, of 144
+// 107 / 183, with a matrix mask 47 / 84, 90 / 126, 149 / 318; 65536 of 256 1535 / 1572, masked 1904 / 2796; 512 pairs
+// of 144 14 / 16, masked 16 / 24; 512 of 256 21 / 19, masked 24 / 28; 1024 of 256 33 / 33.  Below two workgroups per compute unit
+// the general kernel's smaller workgroups spread better (256 of 256 16 / 13).
+inline bool window_forward(const FwdArgs &a) {
+    const int64_t lim = (int64_t)1 << 22; // (32-bit byte offsets of 256 rows)
+    if (a.d != 32 || a.r > 16 || a.r % 8 != 0 || a.Lq > 256 || a.Lk > 256 || a.causal || !(a.scale > 1e-6f && a.scale < 1e6f)) return false;
+    if (!(a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.o.vec_ok && a.k.ss < lim && a.v.ss < lim)) return false;
+    if (a.r > 0 && !(a.qb.vec_ok && a.kb.vec_ok && a.kb.ss < lim)) return false;
+    if (a.mask.type != kNoMask && !mask_in_chunks(a.mask, a.Lk)) return false;
+    const bool few = a.mask.type != kNoMask || a.Lq <= 224;
+    return (int64_t)a.B * a.H >= (few ? 2 : 4) * (int64_t)num_cus();
 }
 
 // What a launcher remembers about one kernel instantiation (one static object per instantiation;

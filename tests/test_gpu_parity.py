@@ -729,6 +729,39 @@ def test_window_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, group, grads
             assert errors(got, want)[1] <= max(tol, GRAD_TOL), name
 
 
+# a wave without queries, with two blocks of them, ragged last blocks on either side, ranks of one chunk and none
+@pytest.mark.parametrize("dtype,B,H,Lq,Lk,r,scale,shared,masked", [
+    (torch.bfloat16, 263, 4, 256, 256, 16, None, True, False), (torch.bfloat16, 1029, 4, 33, 97, 8, None, True, False),
+    (torch.float16, 256, 4, 160, 193, 16, 1.0, False, False), (torch.float16, 1024, 1, 1, 31, 8, 0.3, False, False),
+    (torch.bfloat16, 128, 8, 224, 129, 0, None, False, False), (torch.bfloat16, 260, 4, 256, 256, 16, 1.0, True, True),
+    (torch.float16, 130, 4, 144, 144, 16, None, True, True), (torch.bfloat16, 516, 1, 250, 8, 8, None, False, True),
+    (torch.bfloat16, 64, 8, 100, 136, 0, None, False, True)])
+def test_window_forward(gpu_device, dtype, B, H, Lq, Lk, r, scale, shared, masked):
+    """Forward of short sequences on grids of several workgroups per compute unit (fb_fwd_win.hip), o and lse against the
+    oracle; a mask of -100 and -inf blocks (rows that see one key block only) and random values."""
+    from flashbias_amd import _lib
+    from flashbias_amd.interface import _params, _stream, _tensor
+    q, k, v, qb, kb, do = make_inputs(B, Lq, Lk, H, 32, r, dtype, seed=Lq + Lk, bq=(shared, False), bk=(shared, False))
+    if scale == 1.0:
+        q = (q.float() / 6).to(dtype)
+    mask = None
+    if masked:
+        mask = torch.randn(B, 1, Lq, Lk, generator=torch.Generator().manual_seed(3))
+        mask[..., Lk - Lk // 5:] = -100.0
+        mask[:, :, Lq // 2:, : Lk // 2] = float("-inf")
+        mask = mask.to(dtype)
+    ref = oracle(q, k, v, qb, kb, mask, False, scale, do)
+    dev = [t.to(gpu_device) if t is not None else None for t in (q, k, v, qb if r else None, kb if r else None, mask)]
+    p, keep = _params(*dev, False, scale)
+    o, lse = torch.full_like(dev[0], float("nan")), torch.full((B, H, Lq), float("nan"), device=gpu_device)
+    p.o, p.lse = _tensor(o), lse.data_ptr()
+    _lib.check_status(_lib.load().fb_fwd(p, _stream()))
+    torch.cuda.synchronize()
+    del keep
+    assert errors(o.float().cpu(), ref[0])[0] <= O_TOL[dtype] * max(1.0, ref[0].abs().max().item())
+    assert errors(lse.cpu(), ref[1])[0] <= 1e-3 * max(1.0, ref[1].abs().max().item())  # (fp32 sums of 16-bit products)
+
+
 # waves without keys (64 keys each) and with half a block of them, a second half of 128 queries and none, its ragged last
 # block, one entry a workgroup and several (the last workgroup ragged), the scale folded and not
 @pytest.mark.parametrize("dtype,B,H,Lq,Lk,r,scale,shared", [
