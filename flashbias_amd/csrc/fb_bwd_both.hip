@@ -63,8 +63,8 @@ static hipError_t launch_both_lean(const BwdArgs &a0, hipStream_t stream) {
 // order (longest first within every XCD's share, work_order in fb_order.h).
 template <class T, int NKR, bool FOLD, bool BG>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void bwd_both_kernel(const BwdArgs a) {
-    typedef DqCfg<T, 2, NKR, true, false, false, FOLD, false, BG> Cq;
-    typedef DkvCfg<T, 2, NKR, 1, true, false, 0, FOLD, BG> Ck;
+    typedef DqCfg<T, 2, NKR, true, kNoMask, false, FOLD, false, BG> Cq;
+    typedef DkvCfg<T, 2, NKR, 1, true, kNoMask, 0, FOLD, BG> Ck;
     const int group = a.group > 1 ? a.group : 1;
     const int nbg = (a.B + group - 1) / group;
     const int ndq = a.ntiles_m * nbg * a.H, ndkv = a.ntiles_n * nbg * a.H;
@@ -78,8 +78,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 
 template <class T, int NKR, bool FOLD, bool BG>
 static hipError_t launch_both_general(const BwdArgs &a0, hipStream_t stream) {
-    typedef DqCfg<T, 2, NKR, true, false, false, FOLD, false, BG> Cq;
-    typedef DkvCfg<T, 2, NKR, 1, true, false, 0, FOLD, BG> Ck;
+    typedef DqCfg<T, 2, NKR, true, kNoMask, false, FOLD, false, BG> Cq;
+    typedef DkvCfg<T, 2, NKR, 1, true, kNoMask, 0, FOLD, BG> Ck;
     static_assert(Cq::NTHREADS == 256 && Ck::NTHREADS == 256 && Cq::BM == 128 && Ck::BN == 128, "128-row workgroups of four waves");
     BwdArgs a = a0;
     a.ntiles_m = (a.Lq + Cq::BM - 1) / Cq::BM;

@@ -29,26 +29,30 @@ namespace fb {
 // unmasked, rank <= 32: 16 + 2 or 4 chunks against 32), so that 64-key tiles in two stages fit two workgroups per CU.
 // BG_: also accumulate dq_bias (false: the caller does not want the factor gradients; the accumulator blocks that
 // hold nothing but dq_bias are then left out of the products).
-template <class T, int NKD_, int NKR_, bool VEC_, bool MASK_, bool QB2_ = true, bool FOLD_ = false, bool SPLIT_ = false,
+template <class T, int NKD_, int NKR_, bool VEC_, int MASK_, bool QB2_ = true, bool FOLD_ = false, bool SPLIT_ = false,
           bool BG_ = true>
 struct DqCfg {
     static constexpr bool FOLD = FOLD_;
-    static_assert(!FOLD_ || (VEC_ && !MASK_), "folded scale: direct loader, no additive mask");
+    // A vector mask is one fp32 value per key, all of them in LDS behind the stages: its instantiations (VMASK) are the
+    // unmasked ones otherwise; XMASK is every other masked one.
+    static constexpr bool MASK = MASK_ != kNoMask, VMASK = MASK_ == kVectorMask, XMASK = MASK_ == kMatrixMask;
+    static_assert(!VMASK || VEC_, "");
+    static_assert(!FOLD_ || (VEC_ && !MASK), "folded scale: direct loader, no additive mask");
     // folded scale with r <= 8: the K_b columns 8..15 of a tile hold a second copy of k_b, the
     // partner of the low parts of q_b / scale in the query operand
     static __device__ __forceinline__ bool low_parts(const BwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
     static constexpr int NKD = NKD_, NKR = NKR_;
     static constexpr bool SPLIT = SPLIT_;
-    static constexpr bool VEC = VEC_, MASK = MASK_;
+    static constexpr bool VEC = VEC_;
     static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES;
     static constexpr int NK = NKD + NKR;
     static constexpr int MB = (NK + 1) / 2; // 32-row blocks of [dQ | dQ_b]^T
     static constexpr int MBE = BG_ ? MB : (NKD + 1) / 2; // ... of which the key loop accumulates the first MBE
-    static constexpr int QBLK = (QB2_ && NK <= 3 && !MASK_) ? 2 : 1; // the mask values need the registers of the second block
+    static constexpr int QBLK = (QB2_ && NK <= 3 && !XMASK) ? 2 : 1; // the mask values need the registers of the second block
     static constexpr int BM = NWAVES * QBLK * 32;
     static constexpr int KBLK = 2, BN = 32 * KBLK;
     static constexpr int UNROLL = SPLIT ? 1 : KBLK; // key blocks computed together
-    static constexpr bool ONECHAIN = SPLIT_ && !MASK_; // scale between the d steps and the r steps of one MFMA chain
+    static constexpr bool ONECHAIN = SPLIT_ && !MASK; // scale between the d steps and the r steps of one MFMA chain
     // sK row: [K | K_b] of one key in ROWCH swizzled 16-byte chunks; the one copy is read
     // row-wise for S^T and column-wise for [dQ | dQ_b]^T
     static constexpr int ROWCH = SPLIT ? 2 * NKD : 2 * NK <= 8 ? 8 : 2 * NK <= 16 ? 16 : 32;
@@ -56,13 +60,13 @@ struct DqCfg {
     static constexpr int SK = BN * ROWCH * 8, SV = BN * ROWCHV * 8;
     static constexpr int CPR = 2 * (NKR > 0 ? NKR : 1), SKB = SPLIT && NKR > 0 ? BN * CPR * 8 : 0; // (after the V tile)
     // masked, aligned instantiations also stage the tile's BM x BN block of a 16-bit matrix mask
-    static constexpr bool MTILE = VEC_ && MASK_;
+    static constexpr bool MTILE = VEC_ && XMASK;
     static constexpr int MROWCH = BN / 8; // chunks per mask-tile row
     static constexpr int SM = MTILE ? BM * BN : 0;
     static constexpr int STAGE = SK + SV + SKB + SM;
     // direct loader: three stages, two tiles ahead; with a mask tile (or the element-wise loader)
     // two stages, one ahead
-    static constexpr int AHEAD = (VEC_ && !MASK_ && !SPLIT) ? 2 : 1;
+    static constexpr int AHEAD = (VEC_ && !XMASK && !SPLIT) ? 2 : 1;
     static constexpr int NSTAGE = AHEAD + 1;
     static constexpr int LDS_BYTES = NSTAGE * STAGE * 2;
     // loader: 8-channel chunks of K, K_b and V, one key row each
@@ -70,7 +74,7 @@ struct DqCfg {
     static constexpr int K_TASKS = BN * (CD + CR), V_TASKS = BN * CD;
     static constexpr int K_PT = (K_TASKS + NTHREADS - 1) / NTHREADS;
     static constexpr int V_PT = (V_TASKS + NTHREADS - 1) / NTHREADS;
-    static constexpr int WAVES_EU = (NK <= (MASK_ ? 6 : 8) || SPLIT_) ? 2 : 1;
+    static constexpr int WAVES_EU = (NK <= (XMASK ? 6 : 8) || SPLIT_) ? 2 : 1;
 };
 
 template <class C>
@@ -279,6 +283,11 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
     if constexpr (C::MASK)
         mbase = reinterpret_cast<const uint8_t *>(a.mask.ptr) +
                 mask_offset(a.mask, b, h) * (a.mask.is_f32 ? 4 : 2);
+    if constexpr (C::VMASK) { // (published by the barrier before the first tile; the tiles' scores past the end are set to -inf)
+        float *sM = reinterpret_cast<float *>(smem + C::LDS_BYTES);
+        for (int key = tid; key < a.Lk; key += C::NTHREADS)
+            sM[key] = a.mask.is_f32 ? reinterpret_cast<const float *>(mbase)[key] : T::to_float(reinterpret_cast<const uint16_t *>(mbase)[key]);
+    }
 
     // ---- query-side operands, resident in registers
     u32x4_t qr[C::QBLK][C::NKD];
@@ -447,7 +456,15 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
                     // initial value of the bias chain
                     if constexpr (C::NKR > 0 || C::MASK) {
                         f32x16_t sb;
-                        if constexpr (C::MASK) {
+                        if constexpr (C::VMASK) {
+                            const float *sM = reinterpret_cast<const float *>(smem + C::LDS_BYTES) + n0 + kb * 32 + 4 * g;
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) {
+                                const f32x4_t x = *reinterpret_cast<const f32x4_t *>(sM + 8 * j);
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) sb[4 * j + e] = x[e];
+                            }
+                        } else if constexpr (C::MASK) {
                             if (C::MTILE && direct.mtile) {
                                 // this lane's query row of the staged tile, keys in C-layout order
                                 const uint16_t *sM = sV + C::SV;
@@ -570,30 +587,34 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
 // (One query block per wave and at most four operand steps fit 168 registers: a third wave per SIMD, which the
 // upper bound of the attribute has to allow; 768 x 4 rows of 768 tokens at rank 32: 0.80 -> 0.71 ms.)
 template <class T, class C>
-__global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::WAVES_EU + (C::QBLK == 1 && C::NK <= 4 && C::VEC && !C::MASK ? 1 : 0), C::WAVES_EU + (C::QBLK == 1 && C::NK <= 4 ? 1 : 0)))) void
+__global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::WAVES_EU + (C::QBLK == 1 && C::NK <= 4 && C::VEC && (!C::MASK || (C::VMASK && C::NKD <= 2)) ? 1 : 0), C::WAVES_EU + (C::QBLK == 1 && C::NK <= 4 ? 1 : 0)))) void
 bwd_dq_kernel(const BwdArgs a) {
     bwd_dq_body<T, C>(a, blockIdx.x);
 }
 
-template <class T, int NKD, int NKR, bool VEC, bool MASK, bool QB2, bool FOLD, bool SPLIT, bool BG>
+// LDS of a vector mask's values: whole tiles of 64 keys.
+inline size_t vmask_lds(int Lk) { return (size_t)((Lk + 63) / 64) * 64 * sizeof(float); }
+
+template <class T, int NKD, int NKR, bool VEC, int MASK, bool QB2, bool FOLD, bool SPLIT, bool BG>
 static hipError_t launch_dq_qb_bg(const BwdArgs &a0, hipStream_t stream) {
     typedef DqCfg<T, NKD, NKR, VEC, MASK, QB2, FOLD, SPLIT, BG> C;
     BwdArgs a = a0;
     a.ntiles_m = (a.Lq + C::BM - 1) / C::BM;
     auto kern = bwd_dq_kernel<T, C>;
     static KernelOnce once;
-    const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
+    const size_t lds = C::LDS_BYTES + (C::VMASK ? vmask_lds(a.Lk) : 0);
+    const hipError_t e = allow_lds(kern, C::VMASK ? 80 * 1024 : C::LDS_BYTES, once); // (VMASK: at most that, see launch_dq_cfg)
     if (e != hipSuccess) return e;
     const int group = a.group > 1 ? a.group : 1;
     const int64_t total = (int64_t)a.ntiles_m * ((a.B + group - 1) / group) * a.H;
-    a.slots = slots_per_cu(kern, C::NTHREADS, C::LDS_BYTES, total, once);
-    return launch_flat(kern, total, C::NTHREADS, C::LDS_BYTES, stream, a);
+    a.slots = slots_per_cu(kern, C::NTHREADS, lds, total, once);
+    return launch_flat(kern, total, C::NTHREADS, lds, stream, a);
 }
 
-template <class T, int NKD, int NKR, bool VEC, bool MASK, bool QB2, bool FOLD, bool SPLIT = false>
+template <class T, int NKD, int NKR, bool VEC, int MASK, bool QB2, bool FOLD, bool SPLIT = false>
 static hipError_t launch_dq_qb(const BwdArgs &a, hipStream_t stream) {
     // head dim 32, aligned, unmasked, no dq_bias wanted: the instantiation without its products
-    if constexpr (NKD == 2 && NKR > 0 && NKR <= 2 && VEC && !MASK && !SPLIT) {
+    if constexpr (NKD == 2 && NKR > 0 && NKR <= 2 && VEC && MASK == kNoMask && !SPLIT) {
         if (!a.dqb.ptr) return launch_dq_qb_bg<T, NKD, NKR, VEC, MASK, QB2, FOLD, SPLIT, false>(a, stream);
     }
     return launch_dq_qb_bg<T, NKD, NKR, VEC, MASK, QB2, FOLD, SPLIT, true>(a, stream);
@@ -604,7 +625,7 @@ static hipError_t launch_dq_qb(const BwdArgs &a, hipStream_t stream) {
 // L=16384), 128-query workgroups below that and for short sequences whose last 256-query
 // workgroup would be half empty (8192 x 16 windows of 128 tokens: 2.59 -> 1.76 ms): as in the forward
 // launcher.
-template <class T, int NKD, int NKR, bool VEC, bool MASK, bool FOLD = false>
+template <class T, int NKD, int NKR, bool VEC, int MASK, bool FOLD = false>
 static hipError_t launch_dq_vec(const BwdArgs &a, hipStream_t stream) {
     if constexpr (DqCfg<T, NKD, NKR, VEC, MASK, true>::QBLK == 2) {
         const int64_t wgs = (int64_t)a.B * a.H * ((a.Lq + 255) / 256);
@@ -613,7 +634,7 @@ static hipError_t launch_dq_vec(const BwdArgs &a, hipStream_t stream) {
     }
     // head dims above 64, aligned, unmasked, rank <= 32: two workgroups per CU (larger ranks spill at 256 registers and
     // keep one wave per SIMD)
-    constexpr bool SPLIT = NKD > 4 && NKR <= 2 && VEC && !MASK;
+    constexpr bool SPLIT = NKD > 4 && NKR <= 2 && VEC && MASK == kNoMask;
     return launch_dq_qb<T, NKD, NKR, VEC, MASK, true, FOLD, SPLIT>(a, stream);
 }
 
@@ -628,8 +649,13 @@ static hipError_t launch_dq_cfg(const BwdArgs &a, hipStream_t stream) {
     const bool vec = a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.dout.vec_ok && a.d % 8 == 0 &&
                      (a.r == 0 || (a.qb.vec_ok && a.kb.vec_ok && a.r % 8 == 0)) && a.k.ss < lim && a.v.ss < lim &&
                      (a.r == 0 || a.kb.ss < lim) && (!a.stats_here || a.o.vec_ok);
+    if constexpr (NKD <= 4 && NKR <= 2) {
+        typedef DqCfg<T, NKD, NKR, true, kVectorMask, true> C;
+        if (vec && a.mask.type == kVectorMask && C::LDS_BYTES + vmask_lds(a.Lk) <= 80 * 1024)
+            return launch_dq_vec<T, NKD, NKR, true, kVectorMask>(a, stream);
+    }
     if (a.mask.type)
-        return vec ? launch_dq_vec<T, NKD, NKR, true, true>(a, stream) : launch_dq_vec<T, NKD, NKR, false, true>(a, stream);
+        return vec ? launch_dq_vec<T, NKD, NKR, true, kMatrixMask>(a, stream) : launch_dq_vec<T, NKD, NKR, false, kMatrixMask>(a, stream);
     if constexpr (NKD == 2 && NKR <= 1) {
         if (dq_streamlined(a)) {
             if constexpr (NKR > 0) {
@@ -639,9 +665,9 @@ static hipError_t launch_dq_cfg(const BwdArgs &a, hipStream_t stream) {
         }
     }
     if constexpr (NKR <= 2) {
-        if (vec && fold_scale_ok<T>(a.scale, a.r, a.Lk)) return launch_dq_vec<T, NKD, NKR, true, false, true>(a, stream);
+        if (vec && fold_scale_ok<T>(a.scale, a.r, a.Lk)) return launch_dq_vec<T, NKD, NKR, true, kNoMask, true>(a, stream);
     }
-    return vec ? launch_dq_vec<T, NKD, NKR, true, false>(a, stream) : launch_dq_vec<T, NKD, NKR, false, false>(a, stream);
+    return vec ? launch_dq_vec<T, NKD, NKR, true, kNoMask>(a, stream) : launch_dq_vec<T, NKD, NKR, false, kNoMask>(a, stream);
 }
 
 template <class T, int NKD>
