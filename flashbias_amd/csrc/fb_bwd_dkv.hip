@@ -155,8 +155,10 @@ __device__ __forceinline__ void dkv_load_step(DkvStage<C> &st, const BwdArgs &a,
         const int64_t ld = kind == 0 ? a.q.ss : kind == 1 ? a.qb.ss : a.dout.ss;
         const int ncols = kind == 1 ? a.r : a.d;
         st.x[i] = u32x4_t{0u, 0u, 0u, 0u};
+        // (queries past the end: the last one again, with P = 0, as the direct loader has it; zeros would meet an infinite
+        // entry of k_bias as 0 * inf)
         if (C::TASKS % C::NTHREADS == 0 || task < C::TASKS)
-            st.x[i] = load_chunk<false>(base, ld, m0 + row, a.Lq, ch * 8, ncols);
+            st.x[i] = load_chunk<false>(base, ld, min(m0 + row, a.Lq - 1), a.Lq, ch * 8, ncols);
     }
 }
 

@@ -191,6 +191,21 @@ def test_vector_mask_folded_into_factors(gpu_device, monkeypatch, r, bmask, hmas
     _gate(got2, ref, torch.bfloat16)
 
 
+@pytest.mark.parametrize("d", [32, 44, 100])
+def test_infinite_factor_entries_and_ragged_queries(gpu_device, d):
+    """Keys switched off by -inf in a factor column, tensors that are not 16-byte aligned, a last query tile that is not full."""
+    B, Lq, Lk, H, r = 1, 130, 75, 2, 9
+    q, k, v, qb, kb, do = make_inputs(B, Lq, Lk, H, d, r, torch.bfloat16, seed=5)
+    qb[..., -1], kb[..., -1] = 1.0, 0.0
+    kb[:, 40:, :, -1] = float("-inf")
+    ref = oracle(q, k, v, qb, kb, None, False, None, do)
+    wide = lambda t: torch.cat([t, t[..., :4]], dim=-1).to(gpu_device)[..., :d].requires_grad_(True)
+    leaves = [wide(t) for t in (q, k, v)] + [t.to(gpu_device).requires_grad_(True) for t in (qb, kb)]
+    o = flash_bias_func(*leaves, None, False, None)
+    got = [o.detach()] + list(torch.autograd.grad(o, leaves[:3], wide(do).detach()))
+    _gate([t.float().cpu() for t in got], ref[:5], torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d,r,B,Lq,Lk", [
     (32, 32, 2, 300, 520), (32, 8, 1, 65, 129), (32, 16, 160, 200, 130), (32, 0, 3, 64, 1), (64, 16, 2, 129, 257), (64, 0, 1, 31, 63),
