@@ -33,8 +33,9 @@ template <class T, int NKD_, int NKR_, bool VEC_, int MASK_, bool QB2_ = true, b
           bool BG_ = true>
 struct DqCfg {
     static constexpr bool FOLD = FOLD_;
-    // A vector mask is one fp32 value per key, all of them in LDS behind the stages: its instantiations (VMASK) are the
-    // unmasked ones otherwise; XMASK is every other masked one.
+    // A vector mask is one fp32 value per key: its instantiations (VMASK) are the unmasked ones otherwise; XMASK is every
+    // other masked one.  The values of VCH keys at a time are in LDS behind the stages, or (SPLIT, where a tile is waited for
+    // with everything in flight anyway) travel with their tile.
     static constexpr bool MASK = MASK_ != kNoMask, VMASK = MASK_ == kVectorMask, XMASK = MASK_ == kMatrixMask;
     static_assert(!VMASK || VEC_, "");
     static_assert(!FOLD_ || (VEC_ && !MASK), "folded scale: direct loader, no additive mask");
@@ -52,7 +53,7 @@ struct DqCfg {
     static constexpr int BM = NWAVES * QBLK * 32;
     static constexpr int KBLK = 2, BN = 32 * KBLK;
     static constexpr int UNROLL = SPLIT ? 1 : KBLK; // key blocks computed together
-    static constexpr bool ONECHAIN = SPLIT_ && !MASK; // scale between the d steps and the r steps of one MFMA chain
+    static constexpr bool ONECHAIN = SPLIT_ && !XMASK; // scale between the d steps and the r steps of one MFMA chain
     // sK row: [K | K_b] of one key in ROWCH swizzled 16-byte chunks; the one copy is read
     // row-wise for S^T and column-wise for [dQ | dQ_b]^T
     static constexpr int ROWCH = SPLIT ? 2 * NKD : 2 * NK <= 8 ? 8 : 2 * NK <= 16 ? 16 : 32;
@@ -63,12 +64,14 @@ struct DqCfg {
     static constexpr bool MTILE = VEC_ && XMASK;
     static constexpr int MROWCH = BN / 8; // chunks per mask-tile row
     static constexpr int SM = MTILE ? BM * BN : 0;
-    static constexpr int STAGE = SK + SV + SKB + SM;
+    static constexpr bool VROW = VMASK && !SPLIT_, VTILE = VMASK && SPLIT_;
+    static constexpr int STAGE = SK + SV + SKB + SM + (VTILE ? 2 * BN : 0);
     // direct loader: three stages, two tiles ahead; with a mask tile (or the element-wise loader)
     // two stages, one ahead
     static constexpr int AHEAD = (VEC_ && !XMASK && !SPLIT) ? 2 : 1;
     static constexpr int NSTAGE = AHEAD + 1;
-    static constexpr int LDS_BYTES = NSTAGE * STAGE * 2;
+    static constexpr int VCH = !VROW ? 0 : QBLK == 1 && NK <= 4 ? 1024 : 2048; // (three workgroups per compute unit, or two)
+    static constexpr int VBASE = NSTAGE * STAGE * 2, LDS_BYTES = VBASE + 4 * VCH;
     // loader: 8-channel chunks of K, K_b and V, one key row each
     static constexpr int CD = 2 * NKD, CR = 2 * NKR;
     static constexpr int K_TASKS = BN * (CD + CR), V_TASKS = BN * CD;
@@ -283,12 +286,6 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
     if constexpr (C::MASK)
         mbase = reinterpret_cast<const uint8_t *>(a.mask.ptr) +
                 mask_offset(a.mask, b, h) * (a.mask.is_f32 ? 4 : 2);
-    if constexpr (C::VMASK) { // (published by the barrier before the first tile; the tiles' scores past the end are set to -inf)
-        float *sM = reinterpret_cast<float *>(smem + C::LDS_BYTES);
-        for (int key = tid; key < a.Lk; key += C::NTHREADS)
-            sM[key] = a.mask.is_f32 ? reinterpret_cast<const float *>(mbase)[key] : T::to_float(reinterpret_cast<const uint16_t *>(mbase)[key]);
-    }
-
     // ---- query-side operands, resident in registers
     u32x4_t qr[C::QBLK][C::NKD];
     u32x4_t dor[C::QBLK][C::NKD];
@@ -380,6 +377,21 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
     // of tile t; element-wise loader: tile t + 1 goes through registers.  Keys past the end of a
     // ragged last tile hold copies of the last key; their scores are set to -inf below.
     constexpr int AHEAD = C::AHEAD;
+    // (thread `tid` carries the mask value of key n0 + tid of the tile that follows)
+    float mkey = 0.f;
+    auto load_vmask = [&](int n0) {
+        const int key = min(n0 + (tid & (C::BN - 1)), a.Lk - 1); // (past the end: the score is set to -inf below)
+        mkey = a.mask.is_f32 ? reinterpret_cast<const float *>(mbase)[key] : T::to_float(reinterpret_cast<const uint16_t *>(mbase)[key]);
+    };
+    auto store_vmask = [&](uint16_t *stage) {
+        if (tid < C::BN) reinterpret_cast<float *>(stage + C::SK + C::SV + C::SKB)[tid] = mkey;
+    };
+    auto vmask_chunk = [&](int n0) { // the values of keys [n0, n0 + VCH)
+        const int keys = min(a.Lk - n0, C::VCH);
+        for (int i = tid; i < keys; i += C::NTHREADS)
+            reinterpret_cast<float *>(smem + C::VBASE)[i] =
+                a.mask.is_f32 ? reinterpret_cast<const float *>(mbase)[n0 + i] : T::to_float(reinterpret_cast<const uint16_t *>(mbase)[n0 + i]);
+    };
     DqDirect<C> direct;
     DqStage<C> st;
     if constexpr (C::VEC) {
@@ -393,6 +405,11 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
 #pragma unroll
         for (int k = 0; k < AHEAD; ++k)
             if (k < ntiles_k) direct.issue(a, stage0 + k * C::STAGE, k * C::BN, a.Lk);
+        if constexpr (C::VROW) vmask_chunk(0);
+        if constexpr (C::VTILE) {
+            load_vmask(0);
+            store_vmask(stage0);
+        }
         if (AHEAD == 2 && 1 < ntiles_k)
             wait_vmcnt<DqDirect<C>::N>(); // the first tile has landed, the second may be in flight
         else
@@ -412,10 +429,17 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
         if constexpr (C::VEC) {
             if (it + AHEAD < ntiles_k)
                 direct.issue(a, stage0 + ((cur + AHEAD) % C::NSTAGE) * C::STAGE, n0 + AHEAD * C::BN, a.Lk);
+            if (C::VTILE && more) load_vmask(n0 + C::BN);
         } else if (more) {
             DqLoader<C>::load(st, a, kbase, kbbase, vbase, n0 + C::BN, tid);
         }
 
+        if constexpr (C::VROW) {
+            if (it > 0 && n0 % C::VCH == 0) { // (everyone has left the chunk before: the barrier that ended its last tile)
+                vmask_chunk(n0);
+                barrier_lds();
+            }
+        }
         const uint16_t *sK = stage0 + cur * C::STAGE, *sV = sK + C::SK;
         const uint8_t *sKb = reinterpret_cast<const uint8_t *>(sV + C::SV);
         const bool visible = !(a.causal && n0 > wq0 + 32 * C::QBLK - 1) && wq0 < a.Lq;
@@ -456,15 +480,17 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
                     // initial value of the bias chain
                     if constexpr (C::NKR > 0 || C::MASK) {
                         f32x16_t sb;
-                        if constexpr (C::VMASK) {
-                            const float *sM = reinterpret_cast<const float *>(smem + C::LDS_BYTES) + n0 + kb * 32 + 4 * g;
+                        // (the vector mask's values of this lane's registers, four at a time)
+                        const float *sM = !C::VMASK ? nullptr : (C::VROW ? reinterpret_cast<const float *>(smem + C::VBASE) + n0 % (C::VCH > 0 ? C::VCH : 1)
+                                                                         : reinterpret_cast<const float *>(sV + C::SV + C::SKB)) + kb * 32 + 4 * g;
+                        if constexpr (C::VROW) {
 #pragma unroll
                             for (int j = 0; j < 4; ++j) {
                                 const f32x4_t x = *reinterpret_cast<const f32x4_t *>(sM + 8 * j);
 #pragma unroll
                                 for (int e = 0; e < 4; ++e) sb[4 * j + e] = x[e];
                             }
-                        } else if constexpr (C::MASK) {
+                        } else if constexpr (C::XMASK) {
                             if (C::MTILE && direct.mtile) {
                                 // this lane's query row of the staged tile, keys in C-layout order
                                 const uint16_t *sM = sV + C::SV;
@@ -492,7 +518,16 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
                         for (int t = 0; t < C::NKD; ++t) s = T::mfma(ka[t], qr[qb][t], s);
                         if constexpr (C::ONECHAIN && !C::FOLD) { // (a second accumulator would spill here)
 #pragma unroll
-                            for (int v = 0; v < 16; ++v) s[v] *= a.scale;
+                            for (int j = 0; j < 4; ++j) {
+                                if constexpr (C::VMASK) {
+                                    const f32x4_t x = *reinterpret_cast<const f32x4_t *>(sM + 8 * j);
+#pragma unroll
+                                    for (int e = 0; e < 4; ++e) s[4 * j + e] = __builtin_fmaf(s[4 * j + e], a.scale, x[e]);
+                                } else {
+#pragma unroll
+                                    for (int e = 0; e < 4; ++e) s[4 * j + e] *= a.scale;
+                                }
+                            }
                         }
 #pragma unroll
                         for (int t = C::NKD; t < C::NK; ++t) {
@@ -558,6 +593,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
             }
         }
         if constexpr (C::VEC) {
+            if (C::VTILE && more) store_vmask(stage0 + nxt * C::STAGE);
             if (AHEAD == 2 && it + AHEAD < ntiles_k)
                 wait_vmcnt<DqDirect<C>::N>(); // the next tile has landed, the one after may be in flight
             else
@@ -592,9 +628,6 @@ bwd_dq_kernel(const BwdArgs a) {
     bwd_dq_body<T, C>(a, blockIdx.x);
 }
 
-// LDS of a vector mask's values: whole tiles of 64 keys.
-inline size_t vmask_lds(int Lk) { return (size_t)((Lk + 63) / 64) * 64 * sizeof(float); }
-
 template <class T, int NKD, int NKR, bool VEC, int MASK, bool QB2, bool FOLD, bool SPLIT, bool BG>
 static hipError_t launch_dq_qb_bg(const BwdArgs &a0, hipStream_t stream) {
     typedef DqCfg<T, NKD, NKR, VEC, MASK, QB2, FOLD, SPLIT, BG> C;
@@ -602,13 +635,12 @@ static hipError_t launch_dq_qb_bg(const BwdArgs &a0, hipStream_t stream) {
     a.ntiles_m = (a.Lq + C::BM - 1) / C::BM;
     auto kern = bwd_dq_kernel<T, C>;
     static KernelOnce once;
-    const size_t lds = C::LDS_BYTES + (C::VMASK ? vmask_lds(a.Lk) : 0);
-    const hipError_t e = allow_lds(kern, C::VMASK ? 80 * 1024 : C::LDS_BYTES, once); // (VMASK: at most that, see launch_dq_cfg)
+    const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
     if (e != hipSuccess) return e;
     const int group = a.group > 1 ? a.group : 1;
     const int64_t total = (int64_t)a.ntiles_m * ((a.B + group - 1) / group) * a.H;
-    a.slots = slots_per_cu(kern, C::NTHREADS, lds, total, once);
-    return launch_flat(kern, total, C::NTHREADS, lds, stream, a);
+    a.slots = slots_per_cu(kern, C::NTHREADS, C::LDS_BYTES, total, once);
+    return launch_flat(kern, total, C::NTHREADS, C::LDS_BYTES, stream, a);
 }
 
 template <class T, int NKD, int NKR, bool VEC, int MASK, bool QB2, bool FOLD, bool SPLIT = false>
@@ -634,7 +666,7 @@ static hipError_t launch_dq_vec(const BwdArgs &a, hipStream_t stream) {
     }
     // head dims above 64, aligned, unmasked, rank <= 32: two workgroups per CU (larger ranks spill at 256 registers and
     // keep one wave per SIMD)
-    constexpr bool SPLIT = NKD > 4 && NKR <= 2 && VEC && MASK == kNoMask;
+    constexpr bool SPLIT = NKD > 4 && NKR <= 2 && VEC && MASK != kMatrixMask;
     return launch_dq_qb<T, NKD, NKR, VEC, MASK, true, FOLD, SPLIT>(a, stream);
 }
 
@@ -649,9 +681,10 @@ static hipError_t launch_dq_cfg(const BwdArgs &a, hipStream_t stream) {
     const bool vec = a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.dout.vec_ok && a.d % 8 == 0 &&
                      (a.r == 0 || (a.qb.vec_ok && a.kb.vec_ok && a.r % 8 == 0)) && a.k.ss < lim && a.v.ss < lim &&
                      (a.r == 0 || a.kb.ss < lim) && (!a.stats_here || a.o.vec_ok);
-    if constexpr (NKD <= 4 && NKR <= 2) {
-        typedef DqCfg<T, NKD, NKR, true, kVectorMask, true> C;
-        if (vec && a.mask.type == kVectorMask && C::LDS_BYTES + vmask_lds(a.Lk) <= 80 * 1024)
+    if constexpr (NKR <= 2) {
+        // A vector mask on aligned tensors, against the instantiation that stages it as a matrix (training step, ms): B2 H4
+        // L=16384 d32 r16 2.27 / 2.35, d64 B4 H16 L=4096 r16 1.65 / 1.71, d128 3.09 / 4.04; the same bits.
+        if (vec && a.mask.type == kVectorMask)
             return launch_dq_vec<T, NKD, NKR, true, kVectorMask>(a, stream);
     }
     if (a.mask.type)

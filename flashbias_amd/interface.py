@@ -38,13 +38,7 @@ def _last_dim_contiguous(x):
 
 
 # A vector mask on a problem of at least this many (batch, head, query, key) pairs is folded into
-# the factors.  Forward + backward, folded against the kernels' own vector masks, in ms: B2 H4
-# L=16384 d32 2.03 / 2.25 at rank 8 and 2.31 / 2.29 at rank 16; B4 H16 L=4096 d64 1.57 / 1.64 at
-# rank 8, d128 2.95 / 4.03 at rank 8 and 3.12 / 4.05 at rank 16 (the dq kernel takes a vector mask
-# as a matrix, which is what the fold saves).  It is behind where the column makes another
-# rank bucket (rank 32: 3.03 / 2.43 at d32, 6.34 / 4.14 at d128), where the factors are shared by
-# the batch and the mask is not (768 x 4 rows of 768, rank 32: 5.96 / 2.47), and in a forward
-# alone (rank 8 as above: 0.53 / 0.52, 0.38 / 0.37, 0.62 / 0.64).
+# the factors where that pays (_fold_pays).
 _FOLD_MIN_PAIRS = 1 << 29
 
 
@@ -55,6 +49,20 @@ def _fold_keeps_rank_in_range(rank):
     """One more factor column, padded to the next multiple of 8, must still be a rank the library
     takes (rank 128 stays with the kernels' own vector-mask path)."""
     return rank is None or -(-(rank + 1) // 8) * 8 <= _MAX_RANK
+
+
+def _fold_pays(q, k, q_bias, k_bias, mask):
+    """Whether a large vector mask is ahead as one more factor column.  The kernels take a vector mask at the price of an
+    unmasked call (aligned tensors, ranks up to 32): forward + backward, the kernels' own / folded / without a mask, in ms:
+    B2 H4 L=16384 d32 2.00 / 2.01 / 1.64 at rank 8, 2.04 / 2.26 / 1.98 at 16, 2.32 / 2.99 / 2.25 at 32; B4 H16 L=4096 d64
+    1.53 / 1.54 / 1.50, 1.54 / 1.70 / 1.50, 1.62 / 2.98 / 1.57; 768 x 4 rows of 768 whose factors are shared, rank 32,
+    2.24 / 5.92 / 2.15.  What is left for the fold: head dims above 64 at ranks that stay in one 16-wide step, whose
+    unmasked kernels also fold the scale (d128 3.07 / 2.89 / 2.84 at rank 8, 3.12 / 3.07 at rank 16), unless the column
+    makes the key factor larger; and what the kernels have no vector-mask instantiation for."""
+    rank = 0 if q_bias is None else q_bias.shape[-1]
+    if q.shape[-1] % 8 or rank > 32 or any(t.storage_offset() % 8 or any(s % 8 for s in t.stride()[:3]) for t in (q, k)):
+        return True
+    return q.shape[-1] > 64 and 0 < rank < 16 and mask.shape[0] <= k_bias.shape[0] and mask.shape[1] <= k_bias.shape[2]
 
 
 def _fold_vector_mask(q, q_bias, k_bias, mask):
@@ -94,7 +102,8 @@ def _prepare_factors(q, k, q_bias, k_bias, mask):
     if (mask is not None and mask.dim() == 4 and mask.shape[2] == 1 and mask.shape[3] == seqlen_k
             and mask.dtype == q.dtype and mask.is_cuda
             and batch * nheads * seqlen_q * seqlen_k >= _FOLD_MIN_PAIRS
-            and _fold_keeps_rank_in_range(None if q_bias is None else q_bias.shape[-1])):
+            and _fold_keeps_rank_in_range(None if q_bias is None else q_bias.shape[-1])
+            and _fold_pays(q, k, q_bias, k_bias, mask)):
         q_bias, k_bias = _fold_vector_mask(q, q_bias, k_bias, mask)
         mask = None
     if q_bias is not None:

@@ -206,6 +206,37 @@ def test_infinite_factor_entries_and_ragged_queries(gpu_device, d):
     _gate([t.float().cpu() for t in got], ref[:5], torch.bfloat16)
 
 
+@pytest.mark.parametrize("d,r,bmask,hmask,folds", [(128, 8, True, True, True), (128, 15, False, False, True), (72, 8, True, False, True), (44, 8, True, True, True),
+                                                   (32, 40, False, True, True), (128, 16, True, True, False), (64, 8, True, True, False), (128, 0, True, True, False)])
+def test_where_a_vector_mask_is_folded(gpu_device, monkeypatch, d, r, bmask, hmask, folds):
+    """Which large calls still get the mask as a factor column, and both ways against the oracle; 2100 keys, more than
+    the dq kernel holds mask values of at a time."""
+    from flashbias_amd import interface
+    monkeypatch.setattr(interface, "_FOLD_MIN_PAIRS", 0)
+    B, Lq, Lk, H = 2, 130, 2100, 2
+    q, k, v, qb, kb, do = make_inputs(B, Lq, Lk, H, d, r, torch.bfloat16, seed=31)
+    g = torch.Generator().manual_seed(32)
+    mask = torch.randn(B if bmask else 1, H if hmask else 1, 1, Lk, generator=g).bfloat16()
+    mask[..., Lk - 100:] = float("-inf")
+    dev = [t.to(gpu_device) if t is not None else None for t in (q, k, qb, kb, mask)]
+    assert (interface._prepare_factors(*dev)[2] is None) == folds
+    ref = oracle(q, k, v, qb, kb, mask, False, None, do)
+    _gate(run_gpu(flash_bias_func, q, k, v, qb, kb, mask, False, None, do, gpu_device), ref, torch.bfloat16)
+
+
+@pytest.mark.parametrize("d,r", [(32, 8), (32, 0), (32, 32), (64, 16), (16, 16)])
+def test_vector_mask_over_many_keys(gpu_device, monkeypatch, d, r):
+    """dq refills its mask values every 1024 or 2048 keys: ragged ends behind the second refill, one and two query blocks per wave."""
+    from flashbias_amd import interface
+    monkeypatch.setattr(interface, "_FOLD_MIN_PAIRS", 1 << 62)
+    for B, H, Lq, Lk in ((1, 2, 70, 4130), (1, 128, 1040, 1030)):
+        q, k, v, qb, kb, do = make_inputs(B, Lq, Lk, H, d, r, torch.bfloat16, seed=Lk)
+        mask = torch.randn(B, 1, 1, Lk, generator=torch.Generator().manual_seed(5)).mul(3).bfloat16()
+        mask[..., Lk - 60:] = float("-inf")
+        ref = oracle(q, k, v, qb, kb, mask, False, None, do)
+        _gate(run_gpu(flash_bias_func, q, k, v, qb, kb, mask, False, None, do, gpu_device), ref, torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d,r,B,Lq,Lk", [
     (32, 32, 2, 300, 520), (32, 8, 1, 65, 129), (32, 16, 160, 200, 130), (32, 0, 3, 64, 1), (64, 16, 2, 129, 257), (64, 0, 1, 31, 63),
