@@ -670,17 +670,17 @@ static hipError_t launch_dkv_part(const BwdArgs &a0, hipStream_t stream) {
     return launch_flat(kern, (int64_t)a.ntiles_n * ((a.B + group - 1) / group) * a.H, C::NTHREADS, C::LDS_BYTES, stream, a);
 }
 
-// One pass, or (head dims above 64, aligned tensors) two or three passes that each keep a part
+} // namespace fb
+#include "fb_bwd_dkv_pair.h"
+namespace fb {
+
+// One pass, or (head dims above 64, aligned tensors) two waves a block of keys or three passes that each keep a part
 // of the accumulators.
 template <class T, int NKD, int NKR, int NDV, bool VEC, int MASK, bool FOLD = false>
 static hipError_t launch_dkv_vec(const BwdArgs &a, hipStream_t stream) {
     if constexpr (NKD > 4 && VEC) {
         if constexpr (NKR <= 2 && MASK != kMatrixMask) {
-            // two passes, dv and then all of [dk | dk_bias]: 44 MFMAs per 32 x 32 block (three passes: 61;
-            // dv with the lower half of dk, then the upper half: 52, measured 15-24 % slower than this)
-            const hipError_t e = launch_dkv_part<T, NKD, NKR, NDV, VEC, MASK, 1, FOLD>(a, stream);
-            if (e != hipSuccess) return e;
-            return launch_dkv_part<T, NKD, NKR, NDV, VEC, MASK, 2, FOLD>(a, stream);
+            return launch_dkv_pair<T, NKR, MASK, FOLD>(a, stream);
         } else { // larger ranks and matrix masks: all of dk would spill at 256 registers
             hipError_t e = launch_dkv_part<T, NKD, NKR, NDV, VEC, MASK, 1, FOLD>(a, stream);
             if (e != hipSuccess) return e;
