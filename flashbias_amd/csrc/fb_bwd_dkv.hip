@@ -26,11 +26,10 @@
 
 namespace fb {
 
-// PART: 0 = dv, dk and dk_bias in one pass; 1 = dv only; 2 = [dk | dk_bias] only; 3 / 4 = the
-// lower / upper half of the 32-row blocks of [dk | dk_bias] only.  Head dims above 64 run as two
-// launches (1, 2) while the accumulators of pass 2 fit 256 registers (ranks up to 32, no mask),
-// else as three (1, 3, 4), with 32-query steps: each pass keeps its accumulators in registers and
-// its LDS stages small enough for two waves per SIMD, which is worth recomputing S.
+// PART: 0 = dv, dk and dk_bias in one pass; 1 = dv only; 3 / 4 = the lower / upper half of the 32-row blocks of
+// [dk | dk_bias] only.  Head dims above 64 (where fb_bwd_dkv_pair.h does not take the call) run as three launches (1, 3, 4)
+// with 32-query steps: each pass keeps its accumulators in registers and its LDS stages small enough for two waves per
+// SIMD, which is worth recomputing S.
 // FOLD_: the scores are scale * (q k^T + q_b (k_b / scale)^T), no multiply per score for the scale
 // (the launcher says when that is exact).
 // BG_: also accumulate dk_bias (false: the caller does not want the factor gradients; the accumulator blocks that
@@ -56,30 +55,22 @@ struct DkvCfg {
     static constexpr int MB0 = PART_ == 4 ? MB / 2 : 0,
                          MB1 = PART_ == 1 ? 0 : PART_ == 3 ? MB / 2 : (BG_ ? MB : (NKD_ + 1) / 2);
     static_assert(BG_ || PART_ == 0, "");
-    // Q_b in a dense region of its own instead of the upper chunks of a padded Q row (head dims above 64: 16 + 2 or 4
-    // chunks against 32): steps of 64 queries in two stages then fit two workgroups per compute unit, where rows of
-    // 512 bytes allow 32 in three.  Half the barriers and, with TileAddr16, no scratch: a spilled address is a vector
-    // memory load whose wait also waits for the tile copies in flight.  B2 H8 L=4096 d128 r8, whole backward with the
-    // dq kernel's: 652 -> 566 us; causal B4 H32: 2714 -> 2510 us
-    static constexpr bool SPLIT = VEC_ && !XMASK && PART_ != 0 && NKR_ <= 2;
     static constexpr int KBW = 1; // key blocks per wave
     static constexpr int BN = 32 * KBW * NWAVES;              // keys per workgroup
-    static constexpr int QBLK = PART_ == 0 || SPLIT ? 2 : 1, BMQ = 32 * QBLK; // queries per step
-    static constexpr int UNROLL = SPLIT && DO_DK ? 1 : QBLK; // query blocks computed together
+    static constexpr int QBLK = PART_ == 0 ? 2 : 1, BMQ = 32 * QBLK; // queries per step
     // sQ row: [Q | Q_b] of one query, sdO row: dout of one query, both in swizzled 16-byte
     // chunks; each tile is kept once and read row-wise (S, dP) and column-wise (dK, dV)
-    static constexpr int ROWCH = SPLIT ? 2 * NKD : 2 * NK <= 8 ? 8 : 2 * NK <= 16 ? 16 : 32;
+    static constexpr int ROWCH = 2 * NK <= 8 ? 8 : 2 * NK <= 16 ? 16 : 32;
     static constexpr int ROWCHO = 2 * NKD <= 8 ? 8 : 16;
     static constexpr int SQ = BMQ * ROWCH * 8, SDO = BMQ * ROWCHO * 8;
-    static constexpr int CPR = 2 * (NKR > 0 ? NKR : 1), SQB = SPLIT && NKR > 0 ? BMQ * CPR * 8 : 0; // (after the dO tile)
     // masked, aligned instantiations also stage the step's 64 x 128 tile of a 16-bit matrix mask
     static constexpr bool MTILE = VEC_ && XMASK;
     static constexpr int MROWCH = BN / 8; // chunks per mask-tile row
     static constexpr int SM = MTILE ? BMQ * BN : 0;
-    static constexpr int STAGE_ELEMS = SQ + SDO + SQB + 4 * BMQ + SM; // + lse * log2(e), -delta as fp32
+    static constexpr int STAGE_ELEMS = SQ + SDO + 4 * BMQ + SM; // + lse * log2(e), -delta as fp32
     // direct loader: three stages, two steps ahead; with a mask tile (or the element-wise loader) two
     // stages, one step ahead
-    static constexpr int AHEAD = (VEC_ && !XMASK && !SPLIT) ? 2 : 1;
+    static constexpr int AHEAD = (VEC_ && !XMASK) ? 2 : 1;
     static constexpr int NSTAGE = AHEAD + 1;
     static constexpr int LDS_BYTES = NSTAGE * STAGE_ELEMS * 2;
     // loader tasks: 8-channel chunks of Q, Q_b and dout, one query row each
@@ -133,7 +124,7 @@ __device__ __forceinline__ void dkv_load_stats(DkvStage<C> &st, const float *lse
 
 template <class C>
 __device__ __forceinline__ void dkv_store_stats(const DkvStage<C> &st, uint16_t *stage, int tid) {
-    float *sStat = reinterpret_cast<float *>(stage + C::SQ + C::SDO + C::SQB);
+    float *sStat = reinterpret_cast<float *>(stage + C::SQ + C::SDO);
     if (tid < C::BMQ) {
         sStat[tid] = st.lse2;
         sStat[C::BMQ + tid] = st.negd;
@@ -184,8 +175,7 @@ __device__ __forceinline__ void dkv_store_step(const DkvStage<C> &st, const BwdA
 // tiles of a step plus its statistics rows, copied straight into an LDS stage.
 template <class C>
 struct DkvDirect {
-    TileDma<C::BMQ, C::ROWCH, C::NWAVES, (C::SQB == 0 && C::NKR > 0)> q;
-    DenseCopy<C::BMQ, C::CPR> qb; // Q_b where it has a region of its own
+    TileDma<C::BMQ, C::ROWCH, C::NWAVES, (C::NKR > 0)> q;
     TileDma<C::BMQ, C::ROWCHO, C::NWAVES, false> d;
     TileDma<C::BMQ, C::MROWCH, C::NWAVES, false> m; // mask tile (masked instantiations, 16-bit matrix masks)
     bool mtile;
@@ -205,7 +195,6 @@ struct DkvDirect {
         stat = wave == 0 ? lse2 : wave == 1 ? negd : nullptr;
         q.init(qbase, a.q.ss, a.d, 2 * C::NKD, C::NKR > 0 ? qbbase : nullptr, C::NKR > 0 ? a.qb.ss : 0, a.r, wave, lane, m0,
                C::low_parts(a));
-        if constexpr (C::SQB > 0) qb.init(qbbase, a.qb.ss, a.r, C::low_parts(a), wave, lane, m0);
         d.init(dobase, a.dout.ss, a.d, C::ROWCHO, nullptr, 0, 0, wave, lane, m0);
         mtile = false;
     }
@@ -220,12 +209,11 @@ struct DkvDirect {
     __device__ __forceinline__ void issue(const BwdArgs &a, uint16_t *stage, int m0, int Lq) {
         const uint32_t base = lds_addr_of(stage);
         q.issue(base, m0, Lq, a.q.ss, C::NKR > 0 ? a.qb.ss : 0, 2 * C::NKD);
-        if constexpr (C::SQB > 0) qb.issue(base + 2 * (C::SQ + C::SDO), m0, Lq);
         d.issue(base + 2 * C::SQ, m0, Lq, a.dout.ss, 0, C::ROWCHO);
         if (wave < 2 && lane < C::BMQ)
-            lds_dma4(stat + min(m0 + lane, Lq - 1), base + 2 * (C::SQ + C::SDO + C::SQB) + wave * (4 * C::BMQ));
+            lds_dma4(stat + min(m0 + lane, Lq - 1), base + 2 * (C::SQ + C::SDO) + wave * (4 * C::BMQ));
         if constexpr (C::MTILE) {
-            if (mtile) m.issue(base + 2 * (C::SQ + C::SDO + C::SQB + 4 * C::BMQ), m0, Lq, a.mask.sm, 0, C::MROWCH);
+            if (mtile) m.issue(base + 2 * (C::SQ + C::SDO + 4 * C::BMQ), m0, Lq, a.mask.sm, 0, C::MROWCH);
         }
     }
 
@@ -243,7 +231,7 @@ struct DkvDirect {
     // A last step that runs past the sequence fetched clamped rows: give them P = 0.
     __device__ __forceinline__ void fix_ragged(uint16_t *stage, int m0, int Lq, int tid) const {
         if (m0 + C::BMQ > Lq) {
-            float *sStat = reinterpret_cast<float *>(stage + C::SQ + C::SDO + C::SQB);
+            float *sStat = reinterpret_cast<float *>(stage + C::SQ + C::SDO);
             if (tid < C::BMQ && m0 + tid >= Lq) {
                 sStat[tid] = INFINITY;
                 sStat[C::BMQ + tid] = 0.f;
@@ -486,36 +474,19 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
         }
         const uint16_t *sQ = stage0 + cur * C::STAGE_ELEMS;
         const uint16_t *sdO = sQ + C::SQ;
-        const uint8_t *sQb = reinterpret_cast<const uint8_t *>(sdO + C::SDO);
-        const float *sStat = reinterpret_cast<const float *>(sdO + C::SDO + C::SQB);
-        const uint16_t *sM = sdO + C::SDO + C::SQB + 4 * C::BMQ;
+        const float *sStat = reinterpret_cast<const float *>(sdO + C::SDO);
+        const uint16_t *sM = sdO + C::SDO + 4 * C::BMQ;
 
         const bool visible = !(a.causal && wk0 > m0 + C::BMQ - 1) && wk0 < a.Lk;
         if (visible) {
-            // ([dK | dK_b] at head dims above 64: one block at a time, two at once would spill)
-#pragma unroll 1
-            for (int qo = 0; qo < C::QBLK; qo += C::UNROLL)
 #pragma unroll
-            for (int qi = 0; qi < C::UNROLL; ++qi) {
-                const int qb = qo + qi;
-                TileAddr16 ta(lds_addr_of(sQ) + qb * (32 * 256), c, g); // (SPLIT; the dO tile follows at + 2 SQ)
-                if constexpr (C::SPLIT) asm volatile("" : "+v"(ta.row), "+v"(ta.tr));
-                if (C::UNROLL == 1 && C::QBLK > 1 && a.causal && wk0 > m0 + qb * 32 + 31) continue; // hidden from every key of this wave
-                // (the wave that feeds the matrix pipe goes first: [dK | dK_b] at head dim 128, causal B4 H32 L=4096, 990 -> 970 us)
-                if (C::SPLIT && C::DO_DK) __builtin_amdgcn_s_setprio(1);
+            for (int qb = 0; qb < C::QBLK; ++qb) {
                 u32x4_t qa[C::NK], da[C::NKD];
 #pragma unroll
-                for (int t = 0; t < C::NK; ++t) {
-                    if (C::SQB > 0 && t >= C::NKD)
-                        qa[t] = *reinterpret_cast<const u32x4_t *>(sQb + qb * 32 * C::CPR * 16 + lean_row_addr<C::CPR>(c, 2 * (t - C::NKD) + g));
-                    else if constexpr (C::SPLIT)
-                        qa[t] = ta.load_row(t, 0);
-                    else
-                        qa[t] = *reinterpret_cast<const u32x4_t *>(sQ + swz_off<C::ROWCH>(qb * 32 + c, 2 * t + g));
-                }
+                for (int t = 0; t < C::NK; ++t) qa[t] = *reinterpret_cast<const u32x4_t *>(sQ + swz_off<C::ROWCH>(qb * 32 + c, 2 * t + g));
 #pragma unroll
                 for (int t = 0; t < (C::DO_DK ? C::NKD : 0); ++t)
-                    da[t] = C::SPLIT ? ta.load_row(t, 2 * C::SQ) : *reinterpret_cast<const u32x4_t *>(sdO + swz_off<C::ROWCHO>(qb * 32 + c, 2 * t + g));
+                    da[t] = *reinterpret_cast<const u32x4_t *>(sdO + swz_off<C::ROWCHO>(qb * 32 + c, 2 * t + g));
                 u32x4_t pp[C::KBW][2], pds[C::KBW][2]; // P and dS, packed, per 16-query step
 #pragma unroll
                 for (int kb = 0; kb < C::KBW; ++kb) {
@@ -570,7 +541,6 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
                     }
 #pragma unroll
                     for (int t = C::NKD; t < C::NK; ++t) s = T::mfma(qa[t], kreg[kb][t], s);
-                    if (C::SPLIT && C::DO_DK) __builtin_amdgcn_s_setprio(0);
                     const bool edge = (wk0 + kb * 32 + 32 > a.Lk) || (a.causal && wk0 + kb * 32 + 31 > m0 + qb * 32);
                     if (edge) {
                         int query0 = m0 + qb * 32 + 4 * g;
@@ -589,25 +559,18 @@ __device__ __forceinline__ void bwd_dkv_body(const BwdArgs &a, int wg) {
                         if constexpr (C::DO_DK) pds[kb][v >> 3][(v & 7) >> 1] = T::pack2(p0 * dp[v], p1 * dp[v + 1]);
                     }
                 }
-                if (C::SPLIT && C::DO_DK) __builtin_amdgcn_s_setprio(1);
                 // dV^T += dout^T P ; [dK|dK_b]^T += [Q|Q_b]^T dS  (contraction over this block's queries)
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
 #pragma unroll
                     for (int n = 0; n < (C::DO_DV ? C::NDV : 0); ++n) {
-                        const u32x4_t dot = C::SPLIT ? ta.load_tr(n, 2 * C::SQ + 16 * 256 * t) : lds_read_a_tr<C::ROWCHO>(sdO, qb * 32 + 16 * t, 32 * n, c, g);
+                        const u32x4_t dot = lds_read_a_tr<C::ROWCHO>(sdO, qb * 32 + 16 * t, 32 * n, c, g);
 #pragma unroll
                         for (int kb = 0; kb < C::KBW; ++kb) acc_dv[kb][n] = T::mfma(dot, pp[kb][t], acc_dv[kb][n]);
                     }
 #pragma unroll
                     for (int n = C::MB0; n < C::MB1; ++n) {
-                        u32x4_t qt;
-                        if (C::SQB > 0 && 2 * n >= C::NKD)
-                            qt = dense_read_a_tr<C::CPR>(sQb, qb * 32 + 16 * t, c, g);
-                        else if constexpr (C::SPLIT)
-                            qt = ta.load_tr(n, 16 * 256 * t);
-                        else
-                            qt = lds_read_a_tr<C::ROWCH>(sQ, qb * 32 + 16 * t, 32 * n, c, g);
+                        const u32x4_t qt = lds_read_a_tr<C::ROWCH>(sQ, qb * 32 + 16 * t, 32 * n, c, g);
 #pragma unroll
                         for (int kb = 0; kb < C::KBW; ++kb)
                             acc_dk[kb][n - C::MB0] = T::mfma(qt, pds[kb][t], acc_dk[kb][n - C::MB0]);
