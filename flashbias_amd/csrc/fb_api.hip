@@ -39,6 +39,10 @@ size_t wgrad_workspace(int64_t tokens, int n, int k, bool bias);
 bool wgrad_recommended(int64_t tokens, int n, int k);
 hipError_t launch_wgrad(const void *dy, int64_t ldy, const void *x, int64_t ldx, void *dw, void *db, float *partial, int64_t tokens,
                         int n, int k, bool bf16, hipStream_t stream);
+// projections of one input by up to three weights (fb_project.hip)
+bool project_recommended(int64_t tokens, const int *n, int count);
+hipError_t launch_project(const void *x, int64_t ldx, const void *const *w, void *const *y, const int *n, int count, int64_t tokens, int k, bool bf16,
+                          hipStream_t stream);
 
 hipError_t launch_fwd(const FwdArgs &a, bool bf16, hipStream_t stream) {
     if (window_forward(a)) return bf16 ? launch_fwd_win_bf16_2(a, stream) : launch_fwd_win_f16_2(a, stream);
@@ -341,6 +345,35 @@ int fb_weight_grad(const void *dy, int64_t ldy, const void *x, int64_t ldx, void
         if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return fb::api_fail(FB_ERR_STRIDE, "fb_weight_grad: tensors must be 16-byte aligned");
     return launched(fb::launch_wgrad(dy, ldy, x, ldx, dw, db, scratch, tokens, n, k, dtype == FB_BF16, static_cast<hipStream_t>(stream)),
                     "fb_weight_grad");
+}
+
+static bool project_sizes(int64_t tokens, int k, const int *n, int count) {
+    if (!n || count < 1 || count > 3 || tokens <= 0 || tokens > (1 << 24) || k <= 0 || k > (1 << 16) || k % 64 != 0) return false;
+    for (int i = 0; i < count; ++i)
+        if (n[i] <= 0 || n[i] > (1 << 16) || n[i] % 8 != 0) return false;
+    return true;
+}
+
+int fb_project_recommended(int64_t tokens, int k, const int *n, int count) {
+    return project_sizes(tokens, k, n, count) && fb::project_recommended(tokens, n, count) ? 1 : 0;
+}
+
+int fb_project(const void *x, int64_t ldx, const void *const *w, void *const *y, const int *n, int count, int dtype, int64_t tokens, int k,
+               void *stream) {
+    fb::api_clear_error();
+    if (!x || !w || !y || !n) return fb::api_fail(FB_ERR_NULL, "fb_project: null pointer");
+    if (dtype != FB_F16 && dtype != FB_BF16) return fb::api_fail(FB_ERR_DTYPE, "only fp16 and bf16 are supported");
+    if (!project_sizes(tokens, k, n, count))
+        return fb::api_fail(FB_ERR_SHAPE, "fb_project: one to three weights, tokens up to 2^24, k a multiple of 64 and n of 8, both up to 65536");
+    if (ldx < k || ldx % 8 != 0 || ldx >= (1 << 22))
+        return fb::api_fail(FB_ERR_STRIDE, "fb_project: the row stride must be a multiple of 8 below 2^22 and hold a row");
+    bool aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
+    for (int i = 0; i < count; ++i) {
+        if (!w[i] || !y[i]) return fb::api_fail(FB_ERR_NULL, "fb_project: null pointer");
+        aligned = aligned && reinterpret_cast<uintptr_t>(w[i]) % 16 == 0 && reinterpret_cast<uintptr_t>(y[i]) % 16 == 0;
+    }
+    if (!aligned) return fb::api_fail(FB_ERR_STRIDE, "fb_project: tensors must be 16-byte aligned");
+    return launched(fb::launch_project(x, ldx, w, y, n, count, tokens, k, dtype == FB_BF16, static_cast<hipStream_t>(stream)), "fb_project");
 }
 
 int fb_bwd_static(const fb_params *p, void *stream) {

@@ -384,26 +384,63 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
     }
 };
 
+// What a projection's own route needs of the call: nothing that looks at operations or replaces them is active.
+bool nothing_watches() {
+    // (functorch's thread-local state outlives the thread's first transform; what a running one has included does not)
+    return !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
+           !at::autocast::is_autocast_enabled(at::kCUDA) && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+           !at::impl::torch_function_mode_enabled() && !torch::jit::tracer::isTracing();
+}
+
+// ... and of a tensor
+bool plain_tensor(const Tensor &t, const Tensor &like) {
+    return t.is_cuda() && t.scalar_type() == like.scalar_type() && t.device() == like.device() && !t.key_set().has(c10::DispatchKey::Python) &&
+           t.layout() == c10::kStrided && !t._fw_grad(/*level=*/0).defined();
+}
+
 // The projection where its weight gradient is asked for and the library's kernel for it is ahead, else nothing: the caller
 // then takes the tensor library's own operation, which is also what modes, transforms and tracers that look at operations see.
 c10::optional<Tensor> linear(const Tensor &x, const Tensor &w, const c10::optional<Tensor> &b) {
     const auto type = x.scalar_type();
-    auto plain = [&](const Tensor &t) {
-        return t.is_cuda() && t.scalar_type() == type && t.device() == x.device() && !t.key_set().has(c10::DispatchKey::Python) &&
-               t.layout() == c10::kStrided && !t._fw_grad(/*level=*/0).defined();
-    };
-    // (functorch's thread-local state outlives the thread's first transform; what a running one has included does not)
-    const bool transformed = c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
-    const bool ready = c10::GradMode::is_enabled() && (type == torch::kFloat16 || type == torch::kBFloat16) && plain(x) && plain(w) &&
-                       w.requires_grad() && x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && x.numel() > 0 &&
+    const bool ready = c10::GradMode::is_enabled() && (type == torch::kFloat16 || type == torch::kBFloat16) && plain_tensor(x, x) &&
+                       plain_tensor(w, x) && w.requires_grad() && x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && x.numel() > 0 &&
                        w.size(0) <= (1 << 16) && w.size(1) <= (1 << 16) &&
                        fb_weight_grad_recommended(x.numel() / x.size(-1), (int)w.size(0), (int)w.size(1)) &&
-                       (!b.has_value() || (plain(*b) && b->dim() == 1 && b->size(0) == w.size(0))) &&
-                       !at::autocast::is_autocast_enabled(at::kCUDA) && !transformed &&
-                       !c10::impl::TorchDispatchModeTLS::any_modes_set() && !at::impl::torch_function_mode_enabled() &&
-                       !torch::jit::tracer::isTracing();
+                       (!b.has_value() || (plain_tensor(*b, x) && b->dim() == 1 && b->size(0) == w.size(0))) && nothing_watches();
     if (!ready) return c10::nullopt;
     return LinearFn::apply(x, w, b);
+}
+
+// x w^T for each of three weights in one launch of the library's kernel, where nothing is differentiated and that kernel is
+// ahead, else an empty list (the caller then takes the tensor library's operations, as with `linear`).
+std::vector<Tensor> project(const Tensor &x, const std::vector<Tensor> &w) {
+    const auto type = x.scalar_type();
+    const bool grad_mode = c10::GradMode::is_enabled();
+    auto takes = [&](const Tensor &t) {
+        return plain_tensor(t, x) && !(grad_mode && t.requires_grad()) && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+    };
+    if (!(type == torch::kFloat16 || type == torch::kBFloat16) || x.dim() < 2 || w.size() != 3 || !nothing_watches() || !takes(x) || x.numel() == 0)
+        return {};
+    const int64_t k = x.size(-1), tokens = x.numel() / k;
+    const void *ws[3];
+    void *ys[3];
+    int n[3];
+    for (int i = 0; i < 3; ++i) {
+        if (w[i].dim() != 2 || w[i].size(1) != k || w[i].size(0) > (1 << 16) || k > (1 << 16) || !takes(w[i])) return {};
+        n[i] = (int)w[i].size(0);
+        ws[i] = w[i].data_ptr();
+    }
+    if (!fb_project_recommended(tokens, (int)k, n, 3)) return {};
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    std::vector<Tensor> y(3);
+    auto shape = x.sizes().vec();
+    for (int i = 0; i < 3; ++i) {
+        shape.back() = n[i];
+        y[i] = fresh(shape, type, x.device());
+        ys[i] = y[i].data_ptr();
+    }
+    check(fb_project(x.data_ptr(), k, ws, ys, n, 3, dtype_code(type), tokens, (int)k, stream_of(x)));
+    return y;
 }
 
 // x (..., r) with its last dim zero-padded (or cut) to `rank` columns in one launch of the library; the gradient
@@ -476,6 +513,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("alibi_factors", &alibi_factors, py::arg("seqlen_q"), py::arg("seqlen_k"), py::arg("heads"), py::arg("rank"), py::arg("reference_sign"),
           py::arg("dtype"), py::arg("device"));
     m.def("linear", &linear, py::arg("x"), py::arg("weight"), py::arg("bias"));
+    m.def("project", &project, py::arg("x"), py::arg("weights"));
     m.def("resize_rank", &resize_rank, py::arg("x"), py::arg("rank"));
     m.def("flash_bias", &flash_bias, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("q_bias") = py::none(),
           py::arg("k_bias") = py::none(), py::arg("mask") = py::none(), py::arg("causal") = false,

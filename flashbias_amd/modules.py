@@ -11,19 +11,35 @@ from . import factors, interface
 from .interface import flash_bias_func
 
 
+def _plain(layer, x):
+    """Whether ``layer(x)`` is a GPU's plain ``nn.Linear`` that nothing hooks into or replaces."""
+    return (x.is_cuda and type(layer) is nn.Linear and not torch.compiler.is_compiling()
+            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks)
+            and "forward" not in layer.__dict__ and layer._compiled_call_impl is None
+            and not nn.modules.module._has_any_global_hook())
+
+
 def _project(layer, x):
     """``layer(x)``.  A plain ``nn.Linear`` over many tokens gets its weight gradient from the library's own kernel for long
     contractions (``ext.linear``, which says for which calls; a layer that something hooks into or replaces is called)."""
-    if (x.is_cuda and type(layer) is nn.Linear and torch.is_grad_enabled() and not torch.compiler.is_compiling()
-            and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks)
-            and "forward" not in layer.__dict__ and layer._compiled_call_impl is None
-            and not nn.modules.module._has_any_global_hook()):
+    if torch.is_grad_enabled() and _plain(layer, x):
         ext = interface._extension()
         if ext is not None:
             y = ext.linear(x, layer.weight, layer.bias)
             if y is not None:
                 return y
     return layer(x)
+
+
+def _project_all(layers, x):
+    """``[layer(x) for layer in layers]``.  Plain ``nn.Linear`` layers without bias, where nothing is differentiated, in one
+    launch of the library's own kernel (``ext.project``, which says for which calls)."""
+    if all(_plain(layer, x) and layer.bias is None for layer in layers):
+        ext = interface._extension()
+        y = [] if ext is None else ext.project(x, [layer.weight for layer in layers])
+        if y:
+            return y
+    return [_project(layer, x) for layer in layers]
 
 
 class AttentionWithALiBiBias(nn.Module):
@@ -50,7 +66,7 @@ class AttentionWithALiBiBias(nn.Module):
     def forward(self, x):
         b, n, _ = x.shape
         split = lambda t: t.view(b, n, self.heads, self.dim_head).to(self.dtype)
-        q, k, v = split(_project(self.to_q, x)), split(_project(self.to_k, x)), split(_project(self.to_v, x))
+        q, k, v = (split(t) for t in _project_all((self.to_q, self.to_k, self.to_v), x))
         ext = interface._extension()
         if ext is not None and x.is_cuda and n <= 65536:
             # the same factors in one launch, with the zero columns the operator would append on every call

@@ -258,6 +258,15 @@ int fb_weight_grad_recommended(int64_t tokens, int n, int k);
 int fb_weight_grad(const void *dy, int64_t ldy, const void *x, int64_t ldx, void *dw, void *db, float *scratch, int dtype, int64_t tokens,
                    int n, int k, void *stream);
 
+/* Up to three projections of one input in one launch (the q, k and v projections of an attention block,
+ * 1_Language_Model/attention_with_alibi_bias.py:26-28): y[i] (tokens, n[i]) = x (tokens, k) w[i]^T in the input dtype,
+ * accumulated in fp32 and rounded once.  w[i] (n[i], k) and y[i] are contiguous, x has contiguous rows at a stride of ldx elements.
+ * k is a multiple of 64, n[i] and ldx of 8, ldx below 2^22, n[i] and k at most 65536, tokens at most 2^24; all 16-byte aligned.
+ * fb_project_recommended: 1 where this was measured ahead of the vendor library's products of the same shape. */
+int fb_project_recommended(int64_t tokens, int k, const int *n, int count);
+int fb_project(const void *x, int64_t ldx, const void *const *w, void *const *y, const int *n, int count, int dtype, int64_t tokens,
+               int k, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

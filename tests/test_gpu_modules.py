@@ -339,6 +339,60 @@ def test_weight_gradient(gpu_device, dtype, tokens, n, k):
             assert (db.double() - dy.double().sum(0)).norm() <= bound * dy.double().sum(0).norm()
 
 
+# one step of 64 columns, fewer steps than the pipeline has stages, and many; both tiles (128 x 64 up to 512 of them, 256 x 128
+# beyond) with ragged edges along tokens and channels; one to three weights of different sizes; rows inside a wider tensor
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens,n,k", [(1, (8,), 64), (63, (136, 64), 128), (65, (128, 8, 264), 192), (300, (1000, 72, 512), 320),
+                                        (4099, (520, 136, 1288), 128), (2600, (776, 1032, 776), 1600)])
+def test_projections(gpu_device, dtype, tokens, n, k):
+    lib = _lib.load()
+    g = torch.Generator(device=gpu_device).manual_seed(tokens)
+    x_all = torch.randn(tokens, k + 24, generator=g, device=gpu_device).to(dtype)
+    x = x_all[:, 8:8 + k]
+    x_all[:, :8] = x_all[:, 8 + k:] = float("nan")  # (nothing outside the rows may count)
+    w = [torch.randn(m, k, generator=g, device=gpu_device).to(dtype) for m in n]
+    whole = [torch.full((tokens * m + 64,), 7.0, device=gpu_device, dtype=dtype) for m in n]  # (nor be written)
+    y = [t[:tokens * m].view(tokens, m) for t, m in zip(whole, n)]
+    pointers = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+    sizes = (ctypes.c_int * len(n))(*n)
+    _lib.check_status(lib.fb_project(x.data_ptr(), x.stride(0), pointers(w), pointers(y), sizes, len(n), CODES[dtype], tokens, k, interface._stream()))
+    # rounded once to 8 / 11 significant bits: at most half a unit of the last place of every element, plus its sum in 32 bits
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for got, weight, full, m in zip(y, w, whole, n):
+        want = x.double() @ weight.double().t().contiguous()
+        size = x.double().abs() @ weight.double().abs().t().contiguous()
+        assert ((got.double() - want).abs() <= 1.01 * unit * want.abs() + k * 2.0 ** -24 * size).all()
+        assert (full[tokens * m:] == 7.0).all()
+    assert lib.fb_project(x.data_ptr(), x.stride(0), pointers(w), pointers(y), sizes, len(n), CODES[dtype], tokens, k - 8, interface._stream()) != 0
+
+
+def test_block_projections_take_the_kernel_and_leave_the_rest(gpu_device):
+    torch.manual_seed(3)
+    layers = [torch.nn.Linear(128, 136, bias=False).to(gpu_device, torch.bfloat16) for _ in range(3)]
+    x = torch.randn(5, 130, 128, device=gpu_device, dtype=torch.bfloat16)
+    weights = [layer.weight for layer in layers]
+    exact = [x.double() @ w.detach().double().t().contiguous() for w in weights]
+    with torch.no_grad():
+        assert len(interface._extension().project(x, weights)) == 3
+        for got, want in zip(modules._project_all(layers, x), exact):
+            assert got.shape == want.shape and (got.double() - want).norm() <= 1.01 * 2.0 ** -8 * want.norm()
+        # no rows of 16-byte aligned chunks, another type, nothing to do, more work than the kernel is ahead for: not taken
+        assert not interface._extension().project(x.transpose(0, 1), weights) and not interface._extension().project(x[..., :72], weights)
+        assert not interface._extension().project(x.float(), weights) and not interface._extension().project(x[:0], weights)
+        big = torch.empty(1, 256 * 128 + 1, 128, device=gpu_device, dtype=torch.bfloat16)
+        assert not interface._extension().project(big, weights) and interface._extension().project(big[:, 1:], weights)
+        seen = []
+        handle = layers[1].register_forward_hook(lambda *a: seen.append(1))
+        modules._project_all(layers, x)
+        handle.remove()
+        assert seen
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert all(t.dtype == torch.float16 for t in modules._project_all(layers, x))
+        per_sample = torch.func.vmap(lambda t: modules._project_all(layers, t)[2])(x)
+        assert (per_sample.double() - exact[2]).norm() <= 1.01 * 2.0 ** -8 * exact[2].norm()
+    assert all(t.grad_fn is not None for t in modules._project_all(layers, x))
+
+
 def test_projection_takes_the_kernel_and_leaves_the_rest(gpu_device):
     torch.manual_seed(2)
     layer = torch.nn.Linear(128, 136).to(gpu_device, torch.bfloat16)
