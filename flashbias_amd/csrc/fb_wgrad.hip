@@ -317,6 +317,7 @@ size_t wgrad_workspace(int64_t tokens, int n, int k, bool bias) {
 //    16384      19 / 114     27 / 90       32 / 100    44 / 101     52 / 103     98 / 146     124 / 158    362 / 478
 //    32768      21 / 128     36 / 166      38 / 152    64 / 196     77 / 198     183 / 328    233 / 303    710 / 877
 //   262144      63 / 529     143 / 717     153 / 839   393 / 1102
+// (flashbias_amd/modules.py asks for the 6000 tokens before anything else.)
 // A bias gradient costs it 1-10 %; as a sum of its own it is another pass over dy (18 us at 4096 tokens, 75 at 262144 x 512).
 bool wgrad_recommended(int64_t tokens, int n, int k) {
     const int64_t nk = (int64_t)n * k;
