@@ -130,23 +130,27 @@ inline bool mixed_backward(const BwdArgs &a0) {
 template <class T>
 inline bool mixed_general_backward(const BwdArgs &a0);
 
-// Whether fb_bwd runs the window kernel (fb_bwd_win.hip: one workgroup per (batch, head) forms the per-query
-// statistics and all five gradients, dq summed inside the workgroup) instead of the dq and dk/dv launches: whole
-// sequences of at most 256 positions, head dim 32, rank a multiple of 8 up to 32, aligned tensors, no causal
-// mask, no fp32 mask (the mask is read element-wise, any strides), and at least one workgroup per compute unit (a workgroup fills a compute unit by itself).  Such
-// sequences are bound by memory traffic, and the two-kernel backward reads q, k, v, o and dO twice.
-// And sequences of more than one 128-row block: up to there the two kernels read nothing twice either, and most of
-// the window kernel's eight waves have no keys (512 x 16 windows, rank 16, two kernels against this one: 170 / 224 us
-// at 64 positions, 248 / 264 at 96, 290 / 303 at 128, 570 / 411 at 144; with a matrix mask 284 / 412, 450 / 481,
-// 442 / 535, 1188 / 713; with a vector mask, whose dq kernel stages it as a tile, 227 / 231, 346 / 274, 354 / 317, 835 / 422).
-inline bool window_backward(const BwdArgs &a) {
+// What the two one-launch backwards below share: whole sequences of at most 256 positions, head dim 32, rank a multiple of 8 up
+// to 32, aligned tensors, no causal mask, no fp32 mask (the mask is read element-wise, any strides), and at least one workgroup
+// per compute unit.  Such sequences are bound by memory traffic, and the two-kernel backward reads q, k, v, o and dO twice.
+inline bool short_sequences(const BwdArgs &a) {
     const int64_t lim = (int64_t)1 << 22; // (32-bit byte offsets of 256 tile rows)
     const int group = a.group > 1 ? a.group : 1;
-    if (a.Lq <= 128 && a.Lk <= 128 && a.mask.type != kVectorMask) return false;
     return (a.mask.type == 0 || (!a.mask.is_f32 && a.mask.sm < lim)) && !a.causal && a.d == 32 && a.r % 8 == 0 && a.r <= 32 && a.Lq <= 256 && a.Lk <= 256 &&
            a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.o.vec_ok && a.dout.vec_ok && (a.r == 0 || (a.qb.vec_ok && a.kb.vec_ok)) &&
            a.q.ss < lim && a.k.ss < lim && a.dout.ss < lim && (a.r == 0 || (a.qb.ss < lim && a.kb.ss < lim)) &&
            (int64_t)((a.B + group - 1) / group) * a.H >= num_cus();
+}
+
+// Whether fb_bwd runs the window kernel (fb_bwd_win.hip: one workgroup per (batch, head) forms the per-query
+// statistics and all five gradients, dq summed inside the workgroup; it fills a compute unit by itself) instead of the dq and
+// dk/dv launches: sequences of more than one 128-row block.  Up to there the two kernels read nothing twice either, and most of
+// the window kernel's eight waves have no keys (512 x 16 windows, rank 16, two kernels against this one: 170 / 224 us
+// at 64 positions, 248 / 264 at 96, 290 / 303 at 128, 570 / 411 at 144; with a matrix mask 284 / 412, 450 / 481,
+// 442 / 535, 1188 / 713; with a vector mask 166 / 199, 269 / 253, 314 / 295).
+inline bool window_backward(const BwdArgs &a) {
+    const int few = a.mask.type == kVectorMask ? 64 : 128;
+    return short_sequences(a) && !(a.Lq <= few && a.Lk <= few);
 }
 
 // A 16-bit matrix mask whose rows are whole, aligned 16-byte chunks: the window kernels copy its blocks to LDS.
@@ -158,10 +162,12 @@ inline bool mask_in_chunks(const MaskDesc &m, int Lk) {
 // Whether fb_bwd runs the ring kernel instead of the window kernel (fb_bwd_ring.hip: no factor gradients, ranks up to 16,
 // a matrix mask with rows of whole 16-byte chunks).  Ring against window kernel, rank 16, us: 640 pairs of 256 tokens 42 / 60,
 // 1024 54 / 82, 8192 x (144, 192, 224 tokens) 269 / 372, 313 / 418, 379 / 490, with a matrix mask 323 / 470, 371 / 528,
-// 434 / 596.  It is ahead on every grid; below four workgroups per compute unit, where that is some microseconds,
+// 434 / 596; and against the two kernels that 128 positions and fewer took before (512 x 16 windows of 64, 96, 128): 105 / 144,
+// 165 / 236, 183 / 275, with a matrix mask 124 / 193, 193 / 306, 222 / 338, with a vector mask 110 / 187, 168 / 237, 188 / 281;
+// 1024 x 16 of 16 157 / 238.  It is ahead on every grid; below four workgroups per compute unit, where that is some microseconds,
 // the window kernel keeps dq, dk and dv bit for bit those of the call that computes the factor gradients too.
 inline bool ring_backward(const BwdArgs &a) {
-    if (!window_backward(a) || a.r > 16 || (a.r > 0 && a.dqb.ptr) || (int64_t)a.B * a.H < 4 * (int64_t)num_cus()) return false;
+    if (!short_sequences(a) || a.r > 16 || (a.r > 0 && a.dqb.ptr) || (int64_t)a.B * a.H < 4 * (int64_t)num_cus()) return false;
     return a.mask.type != kMatrixMask || mask_in_chunks(a.mask, a.Lk);
 }
 

@@ -813,7 +813,9 @@ def test_window_forward(gpu_device, dtype, B, H, Lq, Lk, r, scale, shared, maske
 @pytest.mark.parametrize("dtype,B,H,Lq,Lk,r,scale,shared", [
     (torch.bfloat16, 263, 4, 256, 256, 16, None, True), (torch.bfloat16, 1029, 4, 129, 97, 8, None, True),
     (torch.float16, 256, 4, 255, 193, 16, 1.0, False), (torch.float16, 1024, 1, 64, 144, 8, 0.3, False),
-    (torch.bfloat16, 128, 8, 144, 64, 0, None, False)])
+    (torch.bfloat16, 128, 8, 144, 64, 0, None, False), (torch.bfloat16, 513, 2, 64, 64, 16, None, True),
+    (torch.float16, 263, 4, 49, 128, 16, None, True), (torch.bfloat16, 1030, 1, 3, 17, 8, None, False),
+    (torch.bfloat16, 258, 4, 128, 33, 0, 1.0, False)])
 def test_ring_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, shared):
     """Short sequences without factor gradients on grids of several workgroups per compute unit (fb_bwd_ring.hip): the
     checks of test_window_backward."""
@@ -822,7 +824,8 @@ def test_ring_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, shared):
 
 @pytest.mark.parametrize("kind,Lq,Lk,r,scale", [("matrix", 256, 256, 16, 1.0), ("matrix", 144, 144, 16, None), ("matrix", 130, 200, 8, None),
                                                 ("matrix", 200, 136, 0, None), ("matrix", 136, 130, 16, None), ("vector", 64, 250, 16, None),
-                                                ("vector", 256, 65, 8, 1.0)])
+                                                ("vector", 256, 65, 8, 1.0), ("matrix", 64, 64, 16, 1.0), ("matrix", 100, 8, 16, None),
+                                                ("matrix", 31, 128, 8, 1.0), ("vector", 64, 64, 16, None), ("vector", 3, 128, 0, 1.0)])
 def test_ring_backward_with_a_mask(gpu_device, monkeypatch, kind, Lq, Lk, r, scale):
     """The same under additive masks (a key length without whole 16-byte chunks among them), against the oracle."""
     from flashbias_amd import interface
