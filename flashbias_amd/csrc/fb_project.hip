@@ -3,19 +3,17 @@
 //
 // For a few thousand tokens one product of this kind does not fill the chip: 1500 x 1600 x 1600 is 84 tiles of 256 x 128.  The
 // three weights' tiles together are one round of workgroups (252).  Measured, three weights, against three products of
-// the vendor library (us): 1500 x 1600 x 1600 28.7 / 50.3, 600 x 1024 x 1024 11.3 / 22.6, 256 x 512 x 512 7.2 / 15.8,
-// 4096 x 512 x 512 12.7 / 23.4, 2048 x 2048 x 2048 64 / 69, 4096 x 1600 x 1600 88 / 96.  What bounds it: at one round, the
-// fill and drain of the pipeline around k / 64 steps of about 2000 cycles of matrix work a SIMD (750 TFLOP/s); the library is ahead
-// (238 / 278 at 4096 x 3200 x 3200) where many rounds of larger tiles hide both.
+// the vendor library (us): 1500 x 1600 x 1600 27.8 / 50.3, 600 x 1024 x 1024 9.8 / 22.6, 256 x 512 x 512 6.3 / 15.8,
+// 4096 x 512 x 512 12.1 / 23.4, 2048 x 1024 x 1024 18.5 / 31, 4096 x 1600 x 1600 83 / 96.  What bounds it: a wave's own
+// order of copies, LDS reads and products, about 1000 cycles a step where the products take 512 (more stages change nothing); the
+// library is ahead (238 / 278 at 4096 x 3200 x 3200) where many rounds of larger tiles hide it.
 //
 // A workgroup forms a tile of 64 WN channels x 64 WM tokens, a wave 64 x 64 of it (D = W X^T, so a lane holds a token and its
 // registers channels).  Both operands stream through three LDS stages of 64 columns (rows of 128 bytes, the dense regions of
-// fb_lean_tiles.h): one in use and two on their way.  Every wave issues the same number of copies in every step (past the
-// end: the last columns again), so the waits are constants.  Tiles of 256 x 128 with eight waves (144 KB, one workgroup a compute
-// unit) move the fewest bytes per product; where tiles of 128 x 64 with two waves (72 KB, two a unit) are no more than one
-// round, they are ahead by filling more of the chip (600 x 1024 x 1024: 11.3 against 16.1; 1024 x 1024 x 1024: 15.6 / 16.5;
-// just past a round, 1500 x 1024 x 1024, 23.4 against 17.9).  Tiles of 128 x 128 and 64 x 64 were ahead nowhere by more than
-// a few per cent; 32 columns a step in five stages took 37.1 for 1500 x 1600 x 1600.
+// fb_lean_tiles.h): one in use and two on their way.  The copies of a step are issued between its products (all of them ahead
+// of the fragment reads: 1600 channels 28.7, 600 x 1024 x 1024 11.0, one token 13.6 against 11.9).  Every wave issues the same
+// number of them in every step (past the end: the last columns again), so the waits are constants.  Four and five stages of the
+// 128 x 64 tile measured as three do; 32 columns a step in five stages took 37.1 for 1500 x 1600 x 1600.
 #include "fb_kernels.h"
 #include "fb_lean_tiles.h"
 
@@ -77,16 +75,20 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     }
     const uint8_t *wp = reinterpret_cast<const uint8_t *>(a.w[i]) + (int64_t)n0 * a.k * 2, *xp = reinterpret_cast<const uint8_t *>(a.x) + (int64_t)m0 * a.ldx * 2;
     const int nsteps = a.k / 64;
-    auto issue = [&](int step, int stage) {
+    auto issue = [&](int step, int stage, int part, int parts) { // (this part of the copies)
         const int at = min(step, nsteps - 1) * 128;
         const uint32_t dst = lds0 + stage * C::STAGE;
 #pragma unroll
-        for (int j = 0; j < C::CW; ++j) lds_dma16_all(off[j], wp + at, dst + (C::CW * wave + j) * 1024);
-#pragma unroll
-        for (int j = 0; j < C::CX; ++j) lds_dma16_all(off[C::CW + j], xp + at, dst + C::SW + (C::CX * wave + j) * 1024);
+        for (int j = 0; j < C::CW + C::CX; ++j)
+            if (j * parts / (C::CW + C::CX) == part) {
+                if (j < C::CW)
+                    lds_dma16_all(off[j], wp + at, dst + (C::CW * wave + j) * 1024);
+                else
+                    lds_dma16_all(off[j], xp + at, dst + C::SW + (C::CX * wave + j - C::CW) * 1024);
+            }
     };
-    issue(0, 0);
-    issue(1, 1);
+    issue(0, 0, 0, 1);
+    issue(1, 1, 0, 1);
 
     f32x16_t acc[2][2];
 #pragma unroll
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     int stage = 0;
 #pragma unroll 1
     for (int step = 0; step < nsteps; ++step) {
-        issue(step + 2, stage == 0 ? 2 : stage - 1); // (the stage of the step before: everyone has left it)
+        const int into = stage == 0 ? 2 : stage - 1; // (the stage of the step before: everyone has left it)
         const uint32_t aw = lds0 + stage * C::STAGE + 8192 * wn, ax = lds0 + stage * C::STAGE + C::SW + 8192 * wm;
         u32x4_t wf[2][4], xf[2][4];
 #pragma unroll
@@ -113,13 +115,17 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                 wf[p][t] = lds_load16(aw + 4096 * p + row_off[t]);
                 xf[p][t] = lds_load16(ax + 4096 * p + row_off[t]);
             }
+        __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < 4; ++t) {
 #pragma unroll
             for (int p = 0; p < 2; ++p)
 #pragma unroll
                 for (int q = 0; q < 2; ++q) acc[p][q] = T::mfma(wf[p][t], xf[q][t], acc[p][q]);
+            issue(step + 2, into, t, 4);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         __builtin_amdgcn_s_setprio(0);
         wait_vmcnt<C::CW + C::CX>(); // the next step's columns
         barrier_lds();
@@ -156,9 +162,9 @@ static int64_t project_tiles(int64_t tokens, const int *n, int count) {
     return channels * ((tokens + TM - 1) / TM);
 }
 
-// Up to three rounds of the large tile: at exactly three 38.7 us against the library's 47.1 (16384 x 512 x 512) and 62 / 64
-// (8192 x 1024 x 1024); four and more 123 / 107 (6144 x 1600 x 1600), 278 / 238 (4096 x 3200 x 3200), 50 / 50 (65536 x 256
-// x 256).  A single weight gains nothing from the shared launch (1500 x 1600 x 1600: 29.5 against 17.4).
+// Up to three rounds of the large tile: at exactly three 37.0 us against the library's 47.1 (16384 x 512 x 512); four and more
+// 116 / 107 (6144 x 1600 x 1600), 278 / 238 (4096 x 3200 x 3200), 47 / 50 (65536 x 256 x 256).  A single weight gains nothing from
+// the shared launch (1500 x 1600 x 1600: 29.5 against 17.4).
 bool project_recommended(int64_t tokens, const int *n, int count) {
     return count == 3 && project_tiles<256, 128>(tokens, n, count) <= 3 * (int64_t)num_cus();
 }
@@ -187,8 +193,15 @@ hipError_t launch_project(const void *x, int64_t ldx, const void *const *w, void
         a.y[i] = static_cast<uint16_t *>(y[i]);
         a.n[i] = n[i];
     }
-    if (project_tiles<128, 64>(tokens, n, count) <= 2 * (int64_t)num_cus())
-        return bf16 ? launch_project_t<BF16, 2, 1>(a, stream) : launch_project_t<F16, 2, 1>(a, stream);
+    // The tile that fills the chip in one round, us (256 x 128 with eight waves, 144 KB and one workgroup a compute unit / 128 x 128
+    // with four, 96 KB, one / 128 x 64 with two, 72 KB, two): 600 x 1024 x 1024 14.7 / 10.1 / 9.8 (240 of the small ones),
+    // 1024 x 1024 x 1024 15.5 / 10.7 / 14.7 (384 of them, 192 of 128 x 128), 2048 x 512 x 512 11.4 / 8.7 / 10.1 (the same),
+    // 777 x 1600 x 1600 22.9 / 27.0 / 20.2 (507, 273), 2048 x 768 x 768 14.5 / 16.7 / 16.9 (576, 288), 4096 x 512 x 512 12.1 /
+    // 13.3 / 15.0.  Tiles of 64 x 64 with one wave are ahead nowhere.
+    const int64_t cus = num_cus(), small = project_tiles<128, 64>(tokens, n, count);
+    if (small > cus && project_tiles<128, 128>(tokens, n, count) <= cus)
+        return bf16 ? launch_project_t<BF16, 2, 2>(a, stream) : launch_project_t<F16, 2, 2>(a, stream);
+    if (small <= 2 * cus) return bf16 ? launch_project_t<BF16, 2, 1>(a, stream) : launch_project_t<F16, 2, 1>(a, stream);
     return bf16 ? launch_project_t<BF16, 4, 2>(a, stream) : launch_project_t<F16, 4, 2>(a, stream);
 }
 

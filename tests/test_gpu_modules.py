@@ -339,11 +339,11 @@ def test_weight_gradient(gpu_device, dtype, tokens, n, k):
             assert (db.double() - dy.double().sum(0)).norm() <= bound * dy.double().sum(0).norm()
 
 
-# one step of 64 columns, fewer steps than the pipeline has stages, and many; both tiles (128 x 64 up to 512 of them, 256 x 128
-# beyond) with ragged edges along tokens and channels; one to three weights of different sizes; rows inside a wider tensor
+# one step of 64 columns, fewer steps than the pipeline has stages, and many; the three tiles (128 x 64 up to 512 of them, 128 x 128
+# where up to 256 of them are enough for more than 256 small ones, 256 x 128) with ragged edges along tokens and channels; one to three weights of different sizes; rows inside a wider tensor
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("tokens,n,k", [(1, (8,), 64), (63, (136, 64), 128), (65, (128, 8, 264), 192), (300, (1000, 72, 512), 320),
-                                        (4099, (520, 136, 1288), 128), (2600, (776, 1032, 776), 1600)])
+                                        (1500, (1000, 1032, 264), 192), (4099, (520, 136, 1288), 128), (2600, (776, 1032, 776), 1600)])
 def test_projections(gpu_device, dtype, tokens, n, k):
     lib = _lib.load()
     g = torch.Generator(device=gpu_device).manual_seed(tokens)
