@@ -168,6 +168,7 @@ inline bool mask_in_chunks(const MaskDesc &m, int Lk) {
 // the window kernel keeps dq, dk and dv bit for bit those of the call that computes the factor gradients too.
 inline bool ring_backward(const BwdArgs &a) {
     if (!short_sequences(a) || a.r > 16 || (a.r > 0 && a.dqb.ptr) || (int64_t)a.B * a.H < 4 * (int64_t)num_cus()) return false;
+    if (!(a.dq.vec_ok && a.dk.vec_ok && a.dv.vec_ok)) return false; // (it stores whole 16-byte chunks)
     return a.mask.type != kMatrixMask || mask_in_chunks(a.mask, a.Lk);
 }
 

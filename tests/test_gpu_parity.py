@@ -822,6 +822,49 @@ def test_ring_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, shared):
     test_window_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, 2 if shared else 1, False)
 
 
+# one output with a base of its own, one with a row pitch of its own: neither holds rows of aligned 16-byte chunks
+@pytest.mark.parametrize("which,offset,pad", [("dq", 1, 0), ("dk", 4, 0), ("dv", 0, 4), ("dq", 0, 1), ("dv", 1, 0), ("dk", 2, 6)])
+@pytest.mark.parametrize("Lq,Lk,r,mask", [(256, 256, 16, None), (100, 72, 8, None), (144, 136, 0, "matrix"), (64, 40, 16, "vector")])
+def test_short_sequences_with_unaligned_gradients(gpu_device, which, offset, pad, Lq, Lk, r, mask):
+    """The C ABI takes gradients of any base and row pitch: those of the call with aligned ones up to the rounding of other
+    summation orders, and nothing beside their rows is written."""
+    from flashbias_amd import _lib
+    from flashbias_amd.interface import _params, _stream, _tensor
+    dev, dtype, B, H = gpu_device, torch.bfloat16, 260, 4
+    q, k, v, qb, kb, do = [None if t is None else t.to(dev) for t in make_inputs(B, Lq, Lk, H, 32, r, dtype, seed=Lq + r, bq=(True, False), bk=(True, False))]
+    m = None
+    if mask:
+        m = (torch.rand(B, 1, Lq if mask == "matrix" else 1, Lk, generator=torch.Generator().manual_seed(2)) < 0.2).to(dev, dtype) * -100.0
+    lib = _lib.load()
+
+    def run(offset, pad):
+        p, keep = _params(q, k, v, qb, kb, m, False, None)
+        o, lse = torch.empty_like(q), torch.empty((B, H, Lq), device=dev)
+        scratch = torch.empty(lib.fb_bwd_workspace_bytes(p) // 4, device=dev)
+        out, whole = {}, {}
+        for name, like in (("dq", q), ("dk", k), ("dv", v)):
+            off, pitch = (offset, H * 32 + pad) if name == which else (0, H * 32)
+            rows = like.shape[0] * like.shape[1]
+            whole[name] = torch.full((off + rows * pitch + 8,), 7.0, device=dev, dtype=dtype)
+            out[name] = whole[name][off:off + rows * pitch].view(rows, pitch)[:, :H * 32].view(B, -1, H, 32)
+            setattr(p, name, _tensor(out[name]))
+        p.o, p.lse, p.dout, p.delta = _tensor(o), lse.data_ptr(), _tensor(do), scratch.data_ptr()
+        _lib.check_status(lib.fb_fwd(p, _stream()))
+        _lib.check_status(lib.fb_bwd(p, _stream()))
+        torch.cuda.synchronize()
+        del keep
+        return out, whole
+
+    (want, _), (got, whole) = run(0, 0), run(offset, pad)
+    for name in ("dq", "dk", "dv"):
+        a, b = got[name].float(), want[name].float()
+        assert (a - b).abs().max() <= 2.0 ** -6 * b.abs().max(), name  # (as test_window_backward)
+    rest = whole[which].clone()
+    rows = got[which].shape[0] * got[which].shape[1]
+    rest[offset:offset + rows * (H * 32 + pad)].view(rows, -1)[:, :H * 32] = 7.0
+    assert (rest == 7.0).all()
+
+
 @pytest.mark.parametrize("kind,Lq,Lk,r,scale", [("matrix", 256, 256, 16, 1.0), ("matrix", 144, 144, 16, None), ("matrix", 130, 200, 8, None),
                                                 ("matrix", 200, 136, 0, None), ("matrix", 136, 130, 16, None), ("vector", 64, 250, 16, None),
                                                 ("vector", 256, 65, 8, 1.0), ("matrix", 64, 64, 16, 1.0), ("matrix", 100, 8, 16, None),
