@@ -473,6 +473,18 @@ __device__ __forceinline__ float half_wave_max(float x) {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// m2 of the exponent fma(s, to_log2, -m2) for a row whose reference point is m (0 while it has seen no finite score).  Where
+// m is large (a block of keys that a mask of -1e9 or of the type's lowest value switches off) the rounding of the product can
+// leave the exponent of m itself at many powers of two, beyond what a probability holds, and a later block's 0 * inf is NaN: the next
+// number up is taken there, which leaves that block nothing (it is what the row's first visible key leaves it).
+template <class T>
+__device__ __forceinline__ float reference_log2(float m, float to_log2) {
+    const float m2 = m == -INFINITY ? 0.f : m * to_log2;
+    const bool over = __builtin_fmaf(m, to_log2, -m2) > (T::kWideRange ? 100.f : 15.f); // (at m = -inf: -inf)
+    const int bits = __builtin_bit_cast(int, m2);
+    return __builtin_bit_cast(float, over ? bits + (m2 < 0.f ? -1 : 1) : bits);
+}
+
 // Epilogue store of one 32 x 32 accumulator block whose lanes are rows: lane (c, g) holds, for
 // bq = 0..3, the channels ch0 + 8 bq + 4 g + {0..3} of row c in acc[4 bq .. 4 bq + 3] (what the
 // 32x32 MFMA leaves with the row operand as B).  `row` points at channel ch0 of this lane's row,

@@ -808,6 +808,28 @@ def test_window_forward(gpu_device, dtype, B, H, Lq, Lk, r, scale, shared, maske
     assert errors(lse.cpu(), ref[1])[0] <= 1e-3 * max(1.0, ref[1].abs().max().item())  # (fp32 sums of 16-bit products)
 
 
+@pytest.mark.parametrize("dtype,low", [(torch.bfloat16, torch.finfo(torch.bfloat16).min), (torch.bfloat16, -1e30), (torch.bfloat16, -1e9),
+                                       (torch.float16, torch.finfo(torch.float16).min)])
+@pytest.mark.parametrize("n,r,scale", [(64, 16, None), (64, 8, 1.0), (128, 16, None), (256, 0, None)])
+def test_windows_shifted_by_lowest_values(gpu_device, dtype, low, n, r, scale):
+    """Shifted windows whose mask switches keys off by the type's lowest value, or one near it, in the place of -100: the first
+    half of the keys for half of the queries, the second for the others (the result is that of -inf).  At 64 tokens the first
+    half is one block of the window forward's 32 keys."""
+    B, H = 520, 4
+    q, k, v, qb, kb, do = make_inputs(B, n, n, H, 32, r, dtype, seed=n + r, bq=(True, False), bk=(True, False))
+    if scale == 1.0:
+        q = (q.float() / 6).to(dtype)
+    mask = torch.zeros(B, 1, n, n)
+    mask[1::2, :, n // 2:, :n // 2] = low
+    mask[1::2, :, :n // 2, n // 2:] = low
+    ref = oracle(q, k, v, qb, kb, mask, False, scale, do)
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in (q, k, v)]
+    fac = [t.to(gpu_device) if r else None for t in (qb, kb)]
+    o = flash_bias_func(*leaves, *fac, mask.to(gpu_device, dtype), False, scale)
+    got = [o.detach().float().cpu()] + [t.float().cpu() for t in torch.autograd.grad(o, leaves, do.to(gpu_device))]
+    _gate(got + [None, None], ref[:5] + (None, None), dtype, o_by_magnitude=True)
+
+
 # waves without keys (64 keys each) and with half a block of them, a second half of 128 queries and none, its ragged last
 # block, one entry a workgroup and several (the last workgroup ragged), the scale folded and not
 @pytest.mark.parametrize("dtype,B,H,Lq,Lk,r,scale,shared", [
