@@ -109,7 +109,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             f32x16_t o;
 #pragma unroll
             for (int v = 0; v < 16; ++v) o[v] = 0.f;
-            float m_ref = -INFINITY, m2 = 0.f, l_run = 0.f;
+            float m_ref = -INFINITY, m2 = 0.f, l_run = 0.f, slack = lag;
 #pragma unroll 1
             for (int kb = 0; kb < nkb; ++kb) {
                 const uint32_t at = kb * 2048;
@@ -167,7 +167,10 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 #pragma unroll
                 for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
                 mx = half_wave_max(mx);
-                const bool grow = mx > m_ref + lag; // also true for the first finite score of a row
+                // After an even block that moved the reference the odd one moves it without a lag, so that it is the
+                // maximum of 64 keys, as in fwd_kernel: the probability 1 is the one that is not rounded.
+                const bool grow = mx > m_ref + slack; // also true for the first finite score of a row
+                slack = grow && !(kb & 1) ? 0.f : lag;
                 if (__any(grow)) {
                     const float m_new = grow ? mx : m_ref;
                     const float alpha = grow ? fast_exp2((m_ref - m_new) * to_log2) : 1.f; // exp2(-inf) = 0

@@ -830,6 +830,32 @@ def test_windows_shifted_by_lowest_values(gpu_device, dtype, low, n, r, scale):
     _gate(got + [None, None], ref[:5] + (None, None), dtype, o_by_magnitude=True)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,low", [(64, None), (128, float("-inf")), (128, -1e4), (200, None)])
+def test_window_forward_is_as_exact_as_the_general_kernel(gpu_device, dtype, n, low):
+    """Error of o against float64 beside that of the same windows in calls of a size that the general kernel serves."""
+    B, H, r = 512, 8, 16
+    q, k, v, qb, kb, _ = [t.to(gpu_device) for t in make_inputs(B, n, n, H, 32, r, dtype, seed=n, bq=(True, False), bk=(True, False))]
+    mask = None
+    if low is not None:
+        mask = torch.zeros(B, 1, n, n, device=gpu_device)
+        mask[1::2, :, n // 2:, :n // 2] = mask[1::2, :, :n // 2, n // 2:] = low
+        mask = mask.to(dtype)
+    bias = qb.double().transpose(1, 2).contiguous() @ kb.double().permute(0, 2, 3, 1).contiguous()
+    together = flash_bias_func(q, k, v, qb, kb, mask)
+    error = torch.zeros(2, dtype=torch.float64, device=gpu_device)
+    for at in range(0, B, 32):  # (256 pairs: less than one for every workgroup slot)
+        part = [t[at:at + 32] for t in (q, k, v)]
+        m = None if mask is None else mask[at:at + 32]
+        a = [t.double().transpose(1, 2).contiguous() for t in part]
+        logits = a[0] @ a[1].transpose(-1, -2).contiguous() / math.sqrt(32) + bias
+        exact = (torch.softmax(logits if m is None else logits + m.double(), -1) @ a[2]).transpose(1, 2)
+        for i, o in enumerate((together[at:at + 32], flash_bias_func(*part, qb, kb, m))):
+            error[i] += (o.double() - exact).square().sum()
+    # (millions of values with roundings of their own: the two errors are measured to a tenth of a percent)
+    assert error[0].sqrt() <= 1.01 * error[1].sqrt(), error.sqrt()
+
+
 # waves without keys (64 keys each) and with half a block of them, a second half of 128 queries and none, its ragged last
 # block, one entry a workgroup and several (the last workgroup ragged), the scale folded and not
 @pytest.mark.parametrize("dtype,B,H,Lq,Lk,r,scale,shared", [
