@@ -345,6 +345,20 @@ std::pair<Tensor, Tensor> alibi_factors(int64_t Lq, int64_t Lk, int64_t heads, i
     return {qb, kb};
 }
 
+// What a projection's own route needs of the call: nothing that looks at operations or replaces them is active.
+bool nothing_watches() {
+    // (functorch's thread-local state outlives the thread's first transform; what a running one has included does not)
+    return !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
+           !at::autocast::is_autocast_enabled(at::kCUDA) && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+           !at::impl::torch_function_mode_enabled() && !torch::jit::tracer::isTracing();
+}
+
+// ... and of a tensor: memory of its own that holds its values (a tensor that a transform wraps has none)
+bool plain_tensor(const Tensor &t, const Tensor &like) {
+    return t.is_cuda() && t.scalar_type() == like.scalar_type() && t.device() == like.device() && !t.key_set().has(c10::DispatchKey::Python) &&
+           t.layout() == c10::kStrided && t.has_storage() && !t.is_neg() && !t._is_zerotensor() && !t._fw_grad(/*level=*/0).defined();
+}
+
 // A projection x w^T + b whose weight and bias gradients come from the library's kernel for long contractions
 // (fb_weight_grad); the forward and the input's gradient are the tensor library's products.
 struct LinearFn : public torch::autograd::Function<LinearFn> {
@@ -361,9 +375,10 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
         const bool bias = ctx->saved_data["bias"].toBool();
         const Tensor dy = grads[0].reshape({-1, n});
         Tensor dx, dw, db;
-        if (ctx->needs_input_grad(0)) dx = dy.matmul(w).view(x.sizes());
+        if (ctx->needs_input_grad(0)) dx = dy.matmul(w).reshape(x.sizes());
         const bool want_w = ctx->needs_input_grad(1), want_b = bias && ctx->needs_input_grad(2);
-        if (want_w && !c10::GradMode::is_enabled()) {
+        // (a gradient that is itself differentiated, batched gradients, modes that look at the backward: tensor operations)
+        if (want_w && !c10::GradMode::is_enabled() && plain_tensor(dy, w) && plain_tensor(x, w) && plain_tensor(w, w) && nothing_watches()) {
             auto rows = [](const Tensor &t) { // rows of contiguous, 16-byte aligned elements
                 const bool ok = t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % 8 == 0 && t.stride(0) < (1 << 24) &&
                                 reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
@@ -376,27 +391,13 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
             Tensor scratch = fresh({(int64_t)(fb_weight_grad_workspace_bytes(y2.size(0), (int)n, (int)k, want_b) / 4)}, torch::kFloat32, w.device());
             check(fb_weight_grad(y2.data_ptr(), y2.stride(0), x2.data_ptr(), x2.stride(0), dw.data_ptr(), want_b ? db.data_ptr() : nullptr,
                                  scratch.data_ptr<float>(), dtype_code(w.scalar_type()), y2.size(0), (int)n, (int)k, stream_of(w)));
-        } else { // (a gradient that is itself differentiated: tensor operations)
+        } else {
             if (want_w) dw = dy.t().matmul(x.reshape({-1, k}));
             if (want_b) db = dy.sum(0);
         }
         return {dx, dw, db};
     }
 };
-
-// What a projection's own route needs of the call: nothing that looks at operations or replaces them is active.
-bool nothing_watches() {
-    // (functorch's thread-local state outlives the thread's first transform; what a running one has included does not)
-    return !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
-           !at::autocast::is_autocast_enabled(at::kCUDA) && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
-           !at::impl::torch_function_mode_enabled() && !torch::jit::tracer::isTracing();
-}
-
-// ... and of a tensor
-bool plain_tensor(const Tensor &t, const Tensor &like) {
-    return t.is_cuda() && t.scalar_type() == like.scalar_type() && t.device() == like.device() && !t.key_set().has(c10::DispatchKey::Python) &&
-           t.layout() == c10::kStrided && !t._fw_grad(/*level=*/0).defined();
-}
 
 // The projection where its weight gradient is asked for and the library's kernel for it is ahead, else nothing: the caller
 // then takes the tensor library's own operation, which is also what modes, transforms and tracers that look at operations see.

@@ -425,3 +425,31 @@ def test_projection_takes_the_kernel_and_leaves_the_rest(gpu_device):
         assert torch.autograd.forward_ad.unpack_dual(modules._project(layer, dual)).tangent is not None
     per_sample = torch.func.vmap(lambda t: modules._project(layer, t))(x)
     assert torch.allclose(per_sample.float(), want_y.float(), atol=2e-2)
+
+
+def _projection_case(dev):
+    torch.manual_seed(6)
+    layer = torch.nn.Linear(128, 136).to(dev, torch.bfloat16)
+    x = torch.randn(5, 1300, 128, device=dev, dtype=torch.bfloat16, requires_grad=True)
+    return layer, x, torch.randn(3, 5, 1300, 136, device=dev, dtype=torch.bfloat16)
+
+
+@pytest.mark.parametrize("what", ["batched gradients", "counted operations", "autocast"])
+def test_projection_backward_that_something_watches(gpu_device, what):
+    """What wraps the gradients or looks at the operations of a backward, around a forward that took the kernel's route."""
+    from torch.utils.flop_counter import FlopCounterMode
+    layer, x, dy = _projection_case(gpu_device)
+    leaves = [layer.weight, layer.bias, x]
+    results = []
+    for y in (modules._project(layer, x), layer(x)):
+        if what == "batched gradients":
+            results.append(torch.autograd.grad(y, leaves, dy, is_grads_batched=True))
+        elif what == "counted operations":
+            with FlopCounterMode(display=False) as counter:
+                torch.autograd.grad(y, leaves, dy[0])
+            results.append([torch.tensor(float(counter.get_total_flops()))])
+        else:
+            with torch.autocast("cuda", dtype=torch.float16):
+                results.append(torch.autograd.grad(y, leaves, dy[0]))
+    for got, want in zip(*results):  # (the same products, rounded once each: two units of the last place in norm)
+        assert got.shape == want.shape and got.dtype == want.dtype and (got.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
