@@ -363,7 +363,8 @@ bool plain_tensor(const Tensor &t, const Tensor &like) {
 // (fb_weight_grad); the forward and the input's gradient are the tensor library's products.
 struct LinearFn : public torch::autograd::Function<LinearFn> {
     static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &w, const c10::optional<Tensor> &b) {
-        ctx->save_for_backward({x, w});
+        // (the weight only where the input's gradient needs it: as long as it is saved nobody may change it before the backward)
+        ctx->save_for_backward({x, x.requires_grad() ? w : Tensor()});
         ctx->saved_data["bias"] = b.has_value();
         return at::linear(x, w, b);
     }
@@ -371,26 +372,26 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
     static tensor_list backward(AutogradContext *ctx, tensor_list grads) {
         const auto saved = ctx->get_saved_variables();
         const Tensor &x = saved[0], &w = saved[1];
-        const int64_t n = w.size(0), k = w.size(1);
+        const int64_t n = grads[0].size(-1), k = x.size(-1);
         const bool bias = ctx->saved_data["bias"].toBool();
         const Tensor dy = grads[0].reshape({-1, n});
         Tensor dx, dw, db;
         if (ctx->needs_input_grad(0)) dx = dy.matmul(w).reshape(x.sizes());
         const bool want_w = ctx->needs_input_grad(1), want_b = bias && ctx->needs_input_grad(2);
         // (a gradient that is itself differentiated, batched gradients, modes that look at the backward: tensor operations)
-        if (want_w && !c10::GradMode::is_enabled() && plain_tensor(dy, w) && plain_tensor(x, w) && plain_tensor(w, w) && nothing_watches()) {
+        if (want_w && !c10::GradMode::is_enabled() && plain_tensor(x, x) && plain_tensor(dy, x) && nothing_watches()) {
             auto rows = [](const Tensor &t) { // rows of contiguous, 16-byte aligned elements
                 const bool ok = t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % 8 == 0 && t.stride(0) < (1 << 24) &&
                                 reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
                 return ok ? t : t.clone(at::MemoryFormat::Contiguous);
             };
             const Tensor y2 = rows(dy), x2 = rows(x.reshape({-1, k}));
-            dw = fresh({n, k}, w.scalar_type(), w.device());
-            if (want_b) db = fresh({n}, w.scalar_type(), w.device());
-            const c10::hip::HIPGuardMasqueradingAsCUDA guard(w.device());
-            Tensor scratch = fresh({(int64_t)(fb_weight_grad_workspace_bytes(y2.size(0), (int)n, (int)k, want_b) / 4)}, torch::kFloat32, w.device());
+            dw = fresh({n, k}, x.scalar_type(), x.device());
+            if (want_b) db = fresh({n}, x.scalar_type(), x.device());
+            const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+            Tensor scratch = fresh({(int64_t)(fb_weight_grad_workspace_bytes(y2.size(0), (int)n, (int)k, want_b) / 4)}, torch::kFloat32, x.device());
             check(fb_weight_grad(y2.data_ptr(), y2.stride(0), x2.data_ptr(), x2.stride(0), dw.data_ptr(), want_b ? db.data_ptr() : nullptr,
-                                 scratch.data_ptr<float>(), dtype_code(w.scalar_type()), y2.size(0), (int)n, (int)k, stream_of(w)));
+                                 scratch.data_ptr<float>(), dtype_code(x.scalar_type()), y2.size(0), (int)n, (int)k, stream_of(x)));
         } else {
             if (want_w) dw = dy.t().matmul(x.reshape({-1, k}));
             if (want_b) db = dy.sum(0);

@@ -453,3 +453,21 @@ def test_projection_backward_that_something_watches(gpu_device, what):
                 results.append(torch.autograd.grad(y, leaves, dy[0]))
     for got, want in zip(*results):  # (the same products, rounded once each: two units of the last place in norm)
         assert got.shape == want.shape and got.dtype == want.dtype and (got.float() - want.float()).norm() <= 2.0 ** -7 * want.float().norm()
+
+
+def test_projection_of_an_input_without_gradient_keeps_no_weight(gpu_device):
+    """Nothing of the backward needs the weight then: it may change before it (an optimizer's step between two losses)."""
+    layer, x, dy = _projection_case(gpu_device)
+    x = x.detach()
+    want = torch.autograd.grad(layer(x), [layer.weight, layer.bias], dy[0])
+    y = modules._project(layer, x)
+    assert "LinearFn" in y.grad_fn.name()
+    with torch.no_grad():
+        layer.weight.mul_(0.5)
+    for got, w in zip(torch.autograd.grad(y, [layer.weight, layer.bias], dy[0]), want):
+        assert (got.float() - w.float()).norm() <= 2.0 ** -7 * w.float().norm()
+    y = modules._project(layer, x.requires_grad_(True))
+    with torch.no_grad():
+        layer.weight.mul_(0.5)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(y, [x], dy[0])
