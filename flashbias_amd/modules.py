@@ -16,9 +16,14 @@ from .interface import flash_bias_func
 _TOKENS_OF_A_LONG_CONTRACTION = 6000
 
 
+# (a subclass may see or replace operations by ``__torch_function__``, which a call into the extension is not)
+_TENSORS = (torch.Tensor, nn.Parameter)
+
+
 def _plain(layer):
-    """Whether ``layer`` is a plain ``nn.Linear`` that nothing hooks into or replaces."""
-    return (type(layer) is nn.Linear and not torch.compiler.is_compiling()
+    """Whether ``layer`` is a plain ``nn.Linear`` on plain tensors that nothing hooks into or replaces."""
+    return (type(layer) is nn.Linear and type(layer.weight) in _TENSORS and (layer.bias is None or type(layer.bias) in _TENSORS)
+            and not torch.compiler.is_compiling()
             and not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks)
             and "forward" not in layer.__dict__ and layer._compiled_call_impl is None
             and not nn.modules.module._has_any_global_hook())
@@ -27,7 +32,7 @@ def _plain(layer):
 def _project(layer, x):
     """``layer(x)``.  A plain ``nn.Linear`` over many tokens gets its weight gradient from the library's own kernel for long
     contractions (``ext.linear``, which says for which calls; a layer that something hooks into or replaces is called)."""
-    if x.is_cuda and torch.is_grad_enabled() and x.numel() >= _TOKENS_OF_A_LONG_CONTRACTION * x.shape[-1] and _plain(layer):
+    if type(x) in _TENSORS and x.is_cuda and torch.is_grad_enabled() and x.numel() >= _TOKENS_OF_A_LONG_CONTRACTION * x.shape[-1] and _plain(layer):
         ext = interface._extension()
         if ext is not None:
             y = ext.linear(x, layer.weight, layer.bias)
@@ -39,7 +44,7 @@ def _project(layer, x):
 def _project_all(layers, x):
     """``[layer(x) for layer in layers]``.  Plain ``nn.Linear`` layers without bias, with gradients off, in one launch of the
     library's own kernel (``ext.project``, which says for which calls)."""
-    if x.is_cuda and not torch.is_grad_enabled() and all(_plain(layer) and layer.bias is None for layer in layers):
+    if type(x) in _TENSORS and x.is_cuda and not torch.is_grad_enabled() and all(_plain(layer) and layer.bias is None for layer in layers):
         ext = interface._extension()
         y = None if ext is None else ext.project(x, [layer.weight for layer in layers])
         if y:

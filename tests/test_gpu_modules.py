@@ -471,3 +471,34 @@ def test_projection_of_an_input_without_gradient_keeps_no_weight(gpu_device):
         layer.weight.mul_(0.5)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         torch.autograd.grad(y, [x], dy[0])
+
+
+class Watching(torch.Tensor):
+    """A tensor type that sees operations without a dispatch key of its own."""
+    seen = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.seen.append(func)
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+@pytest.mark.parametrize("what", ["input", "weight"])
+@pytest.mark.parametrize("grad", [True, False])
+def test_projections_of_tensor_subclasses(gpu_device, what, grad):
+    """An input or a weight of a type that overrides operations sees its projection, as F.linear shows it."""
+    torch.manual_seed(7)
+    layers = [torch.nn.Linear(128, 136, bias=False).to(gpu_device, torch.bfloat16) for _ in range(3)]
+    x = torch.randn(5, 1300, 128, device=gpu_device, dtype=torch.bfloat16)
+    with torch.set_grad_enabled(grad):
+        want = modules._project_all(layers, x)
+        if what == "input":
+            x = x.as_subclass(Watching)
+        else:
+            layers[1].weight = torch.nn.Parameter(layers[1].weight.detach().as_subclass(Watching))
+        Watching.seen.clear()
+        got = modules._project_all(layers, x)
+    assert Watching.seen.count(torch.nn.functional.linear) == (3 if what == "input" else 1)
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert type(a) is (Watching if what == "input" or i == 1 else torch.Tensor)
+        assert (a.as_subclass(torch.Tensor).float() - b.float()).norm() <= 2.0 ** -7 * b.float().norm()
