@@ -77,10 +77,12 @@ int fb_suggest_bias_grad_group(const fb_params *p) {
     // Whole sequences of at most 256 positions at head dim 32 run one workgroup per (batch, head) pair, which fills a
     // compute unit by itself and pays for every start with an LDS clear and a first window whose loads nothing
     // overlaps (about 4.6 us: 4096 x 16 windows 5.33 ms ungrouped, 4.29 in groups of 8): groups of up to 32 there,
-    // as long as four workgroups per compute unit remain.
+    // as long as four workgroups per compute unit remain.  Up to 128 positions (64 under a vector mask) the two kernels
+    // serve them as others (window_backward() in fb_kernels.h): 4096 x 16 windows of 64, rank 16, groups of 4 / 8 / 16 / 32:
+    // 1.08 / 1.04 / 1.06 / 1.10 ms, with a vector mask 1.15 / 1.10 / 1.12 / 1.17.
+    const int few = p->mask_type == FB_MASK_VECTOR ? 64 : 128;
     const bool window = p->d == 32 && p->r % 8 == 0 && p->r <= 32 && p->Lq <= 256 && p->Lk <= 256 && !p->causal &&
-                        (p->mask_type == FB_MASK_NONE || p->mask_dtype == p->dtype) &&
-                        (p->Lq > 128 || p->Lk > 128 || p->mask_type == FB_MASK_VECTOR);
+                        (p->mask_type == FB_MASK_NONE || p->mask_dtype == p->dtype) && (p->Lq > few || p->Lk > few);
     for (int g = window ? 32 : 8; g > 1; g /= 2)
         if (((int64_t)p->B + g - 1) / g * p->H * ((lmin + 255) / 256) >= 1024) return g;
     return 1;

@@ -183,6 +183,12 @@ def test_grouped_factor_gradients_checks_and_suggestion():
     p.Lq, p.r = 256, 0
     assert lib.fb_suggest_bias_grad_group(p) == 1
     assert lib.fb_suggest_bias_grad_group(None) == 1
+    # ... and so do windows that the two kernels serve: up to 128 positions, 64 under a vector mask
+    p.r, p.mask_dtype = 16, p.dtype
+    for n, mask, group in ((128, 0, 8), (136, 0, 32), (64, 1, 8), (72, 1, 32), (64, 2, 8), (128, 2, 8), (136, 2, 32)):
+        p.Lq = p.Lk = n
+        p.mask_type = mask
+        assert lib.fb_suggest_bias_grad_group(p) == group, (n, mask)
 
 
 @pytest.mark.parametrize("args,code", [
