@@ -517,7 +517,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs &a) {
 #pragma unroll
                         for (int v = 0; v < 16; ++v) acc_o[qb][n][v] *= alpha;
                     m_ref[qb] = m_new;
-                    m2[qb] = (m_new == -INFINITY) ? 0.f : m_new * to_log2;
+                    m2[qb] = reference_log2<T>(m_new, to_log2);
                 }
                 // ---- P^T = exp(S^T - m_ref), row sums (of the fp32 values, :271), O^T += V^T P^T
 #pragma unroll

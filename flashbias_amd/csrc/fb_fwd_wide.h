@@ -193,7 +193,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 #pragma unroll
                     for (int v = 0; v < 16; ++v) acc_o[n][v] *= alpha;
                 m_ref = m_new;
-                m2 = (m_new == -INFINITY) ? 0.f : m_new * to_log2;
+                m2 = reference_log2<T>(m_new, to_log2);
             }
 #pragma unroll
             for (int kb = 0; kb < C::KBLK; ++kb)

@@ -270,6 +270,28 @@ def test_vector_mask_equals_its_matrix(gpu_device, monkeypatch, d, r, B, Lq, Lk,
             assert (x - y).abs().max() <= 2 * eps * max(1e-3, float(y.abs().max())), (name, mtype, causal)
 
 
+# 128 and 256 queries per workgroup, one and two groups of 64 keys a tile, the wide kernel, element-wise loaders
+@pytest.mark.parametrize("d,r,B,L,pad", [(32, 8, 2, 384, 70), (32, 16, 24, 1300, 200), (32, 0, 2, 300, 64), (16, 8, 2, 384, 130), (64, 16, 2, 384, 70),
+                                         (128, 8, 2, 384, 200), (44, 8, 2, 260, 64), (32, 32, 64, 512, 96)])
+@pytest.mark.parametrize("dtype,mdtype,low", [(torch.bfloat16, torch.bfloat16, torch.finfo(torch.bfloat16).min), (torch.bfloat16, torch.float32, -1e30),
+                                              (torch.float16, torch.float32, torch.finfo(torch.float32).min), (torch.float16, torch.float32, -1e9)])
+@pytest.mark.parametrize("kind", ["vector", "matrix"])
+def test_leading_keys_of_lowest_values(gpu_device, monkeypatch, d, r, B, L, pad, dtype, mdtype, low, kind):
+    """Padding at the front: whole key blocks that a mask switches off by the type's lowest value, or a number near it, before
+    the first visible key (the result is that of -inf)."""
+    from flashbias_amd import interface
+    monkeypatch.setattr(interface, "_FOLD_MIN_PAIRS", 1 << 62)
+    q, k, v, qb, kb, do = make_inputs(B, L, L, 2, d, r, dtype, seed=d + r)
+    mask = torch.zeros(B, 1, 1, L)
+    mask[1::2, ..., :pad] = low
+    if kind == "matrix":
+        mask = mask.expand(B, 1, L, L).contiguous()
+    mask = mask.to(mdtype)
+    ref = oracle(q, k, v, qb, kb, mask, False, None, do)
+    got = run_gpu(flash_bias_func, q, k, v, qb, kb, mask, False, None, do, gpu_device)
+    _gate(got, ref, dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d,r,Lq,Lk,scale", [
     (64, 8, 1, 1, None), (64, 16, 127, 63, None), (40, 8, 129, 64, None), (64, 0, 128, 65, None), (56, 24, 200, 600, 0.125),
