@@ -669,7 +669,11 @@ def test_small_grid_backward_in_one_launch(gpu_device, dtype, B, H, Lq, Lk, r, c
     (6, 130, 70, 2, 16, 16, 2, False, False),     # head dim 16: dq and dq_bias share an accumulator block
     (5, 96, 96, 2, 64, 32, 3, True, False),
     (4, 100, 100, 2, 24, 5, 2, False, False),     # unaligned rank: element-wise loaders and stores
-    (6, 64, 64, 4, 32, 16, 3, False, True)])      # additive matrix mask (the shifted windows of Swin)
+    (6, 64, 64, 4, 32, 16, 3, False, True),       # additive matrix mask (the shifted windows of Swin)
+    # head dims above 64: pairs of waves walk the entries; a ragged last group, key tiles past the last query (no step of
+    # their own), rank 32 in two steps, one step for all
+    (7, 200, 150, 2, 128, 8, 3, False, False), (5, 100, 300, 2, 96, 16, 4, True, False), (6, 130, 130, 2, 72, 32, 2, True, False),
+    (4, 64, 128, 3, 128, 16, 4, False, False)])
 def test_factor_gradients_summed_over_batch_groups(gpu_device, dtype, B, Lq, Lk, H, d, r, group, causal, mask):
     """fb_params.bias_grad_group = g: dq, dk, dv are those of the ungrouped call (bit for bit where both
     run the same kernels), and row

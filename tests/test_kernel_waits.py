@@ -72,3 +72,15 @@ def test_compiled_ring_kernel():
     with open(os.path.join(CSRC, unit)) as f:
         text = f.read()
     assert text.count("v_mfma_f32_32x32x16") > 100 and waits.check(text) == []
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None or shutil.which("make") is None, reason="needs hipcc and make")
+def test_compiled_window_and_projection_kernels():
+    """The window forward, the ring in fp16, the weight gradient and the projections."""
+    units = {f"build/asm/fb_{unit}.s": products for unit, products in (("fwd_win_bf16_2", 30), ("fwd_win_f16_2", 30), ("bwd_ring_f16_2", 100),
+                                                                     ("wgrad", 100), ("project", 90))}
+    subprocess.run(["make", "-j4"] + list(units), cwd=CSRC, check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    for unit, products in units.items():
+        with open(os.path.join(CSRC, unit)) as f:
+            text = f.read()
+        assert text.count("v_mfma_f32_32x32x16") > products and waits.check(text) == [], unit
