@@ -28,7 +28,7 @@
 namespace fb {
 
 // NKR_: 16-wide steps of the rank (0, 1).  FOLD_: the scores are scale * (q k^T + q_b k_b^T), no multiply per score
-// for the scale (no factors, or a scale of exactly 1).  MASK_: an additive mask of the 16-bit type, a vector mask as
+// for the scale (no factors and a positive scale, or a scale of exactly 1).  MASK_: an additive mask of the 16-bit type, a vector mask as
 // one value per lane (key) or a matrix mask as a 32 x 32 tile per block, copied to LDS by the wave that uses it.
 // HIDE_: some wave's 64 keys are not all there, their scores are set to -inf (a branch on it inside the step cost 200
 // bytes of scratch).
@@ -433,7 +433,8 @@ static hipError_t launch_ring_m(const BwdArgs &a, bool fold, hipStream_t stream)
 template <class T, int NKR>
 static hipError_t launch_ring_r(const BwdArgs &a, hipStream_t stream) {
     switch (a.mask.type) {
-    case kNoMask: return launch_ring_m<T, NKR, kNoMask>(a, a.r == 0 || a.scale == 1.f, stream);
+    // (a negative scale is not folded: it would turn the -inf of the keys past the end round)
+    case kNoMask: return launch_ring_m<T, NKR, kNoMask>(a, (a.r == 0 && a.scale > 0.f) || a.scale == 1.f, stream);
     case kVectorMask: return launch_ring_m<T, NKR, kVectorMask>(a, false, stream);
     default: return launch_ring_m<T, NKR, kMatrixMask>(a, a.scale == 1.f, stream);
     }

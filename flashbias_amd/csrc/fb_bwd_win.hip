@@ -31,7 +31,7 @@
 namespace fb {
 
 // NKR_: 16-wide steps of the rank (0, 1, 2).  FOLD_: the scores are scale * (q k^T + q_b k_b^T), no multiply per
-// score for the scale (no factors, or a scale of exactly 1).  BG_: also form dq_bias and dk_bias.  MASK_: an additive
+// score for the scale (no factors and a positive scale, or a scale of exactly 1).  BG_: also form dq_bias and dk_bias.  MASK_: an additive
 // mask of the 16-bit type.  A vector mask is one value per lane (key).  A matrix mask's 32 x 32 block is read element-wise, lane = key and register = query (a load instruction
 // asks for two 64-byte row pieces, and the heads of a window meet in one L2), requested as soon as the block before it
 // has used its 16 registers: there is no LDS left for a tile, and the copies are 1024 of a window's 34000 cycles.
@@ -445,7 +445,8 @@ template <class T, int NKR>
 static hipError_t launch_win_r(const BwdArgs &a, hipStream_t stream) {
     const bool bg = NKR > 0 && a.dqb.ptr;
     switch (a.mask.type) {
-    case kNoMask: return launch_win_m<T, NKR, kNoMask>(a, a.r == 0 || a.scale == 1.f, bg, stream);
+    // (a negative scale is not folded: it would turn the -inf of the keys past the end round)
+    case kNoMask: return launch_win_m<T, NKR, kNoMask>(a, (a.r == 0 && a.scale > 0.f) || a.scale == 1.f, bg, stream);
     case kVectorMask: return launch_win_m<T, NKR, kVectorMask>(a, a.scale == 1.f, bg, stream); // (the mask is not divided by the scale)
     default: return launch_win_m<T, NKR, kMatrixMask>(a, a.scale == 1.f, bg, stream);
     }

@@ -740,6 +740,8 @@ def test_factor_gradients_summed_over_batch_groups(gpu_device, dtype, B, Lq, Lk,
     (torch.float16, 256, 1, 129, 255, 0, None, 1, True),     # no factors
     (torch.bfloat16, 36, 8, 250, 250, 16, None, 1, False),   # constant factors: no dq_bias / dk_bias
     (torch.bfloat16, 64, 4, 256, 256, 8, None, 8, False),    # constant shared factors, groups
+    (torch.bfloat16, 66, 4, 200, 130, 0, -0.2, 1, False),    # a negative scale, a key block that is not all there
+    (torch.float16, 66, 4, 256, 249, 0, -0.3, 1, False),
     # enough (batch, head) pairs for a workgroup to walk several entries without summing their factor gradients
     (torch.bfloat16, 1101, 4, 200, 256, 16, None, 1, True),  # four per workgroup, the last workgroup ragged
     (torch.float16, 2100, 1, 129, 255, 0, None, 1, True),    # no factors, two per workgroup
@@ -889,7 +891,9 @@ def test_window_forward_is_as_exact_as_the_general_kernel(gpu_device, dtype, n, 
     (torch.float16, 256, 4, 255, 193, 16, 1.0, False), (torch.float16, 1024, 1, 64, 144, 8, 0.3, False),
     (torch.bfloat16, 128, 8, 144, 64, 0, None, False), (torch.bfloat16, 513, 2, 64, 64, 16, None, True),
     (torch.float16, 263, 4, 49, 128, 16, None, True), (torch.bfloat16, 1030, 1, 3, 17, 8, None, False),
-    (torch.bfloat16, 258, 4, 128, 33, 0, 1.0, False)])
+    (torch.bfloat16, 258, 4, 128, 33, 0, 1.0, False),
+    # a negative scale without factors, keys past the end (whose scores of -inf must not change sign)
+    (torch.bfloat16, 258, 4, 144, 100, 0, -0.2, False), (torch.float16, 1030, 1, 64, 49, 0, -0.3, False), (torch.bfloat16, 263, 4, 256, 200, 0, -0.1, False)])
 def test_ring_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, shared):
     """Short sequences without factor gradients on grids of several workgroups per compute unit (fb_bwd_ring.hip): the
     checks of test_window_backward."""
