@@ -40,7 +40,7 @@ bool wgrad_recommended(int64_t tokens, int n, int k);
 hipError_t launch_wgrad(const void *dy, int64_t ldy, const void *x, int64_t ldx, void *dw, void *db, float *partial, int64_t tokens,
                         int n, int k, bool bf16, hipStream_t stream);
 // projections of one input by up to three weights (fb_project.hip)
-bool project_recommended(int64_t tokens, const int *n, int count);
+bool project_recommended(int64_t tokens, int k, const int *n, int count);
 hipError_t launch_project(const void *x, int64_t ldx, const void *const *w, void *const *y, const int *n, int count, int64_t tokens, int k, bool bf16,
                           hipStream_t stream);
 
@@ -355,7 +355,7 @@ static bool project_sizes(int64_t tokens, int k, const int *n, int count) {
 }
 
 int fb_project_recommended(int64_t tokens, int k, const int *n, int count) {
-    return project_sizes(tokens, k, n, count) && fb::project_recommended(tokens, n, count) ? 1 : 0;
+    return project_sizes(tokens, k, n, count) && fb::project_recommended(tokens, k, n, count) ? 1 : 0;
 }
 
 int fb_project(const void *x, int64_t ldx, const void *const *w, void *const *y, const int *n, int count, int dtype, int64_t tokens, int k,

@@ -165,8 +165,12 @@ static int64_t project_tiles(int64_t tokens, const int *n, int count) {
 // Up to three rounds of the large tile: at exactly three 37.0 us against the library's 47.1 (16384 x 512 x 512); four and more
 // 116 / 107 (6144 x 1600 x 1600), 278 / 238 (4096 x 3200 x 3200), 47 / 50 (65536 x 256 x 256).  A single weight gains nothing from
 // the shared launch (1500 x 1600 x 1600: 29.5 against 17.4).
-bool project_recommended(int64_t tokens, const int *n, int count) {
-    return count == 3 && project_tiles<256, 128>(tokens, n, count) <= 3 * (int64_t)num_cus();
+// Up to 4096 columns of x: a workgroup walks all of them, 6.5 us per 1024 however few tiles there are, where the library splits
+// long sums.  Few tokens, weights from memory, this / library, us: 1 x 1024 x 1024 9.1 / 17.0, 1 x 2048 x 64 14.6 / 15.4,
+// 16 x 1600 x 1600 12.5 / 25.9, 1 x 4096 x 256 25.6 / 32.5 (32 tokens 26.0 / 25.4), 1 x 4096 x 4096 37.4 / 46.5 (32: 37.4 / 39.4);
+// 16 x 5120 x 512 36.7 / 23.8, 1 x 5120 x 5120 50.8 / 43.8, 1 x 8192 x 1024 59.4 / 35.1, 64 x 16384 x 256 123 / 55.
+bool project_recommended(int64_t tokens, int k, const int *n, int count) {
+    return count == 3 && k <= 4096 && project_tiles<256, 128>(tokens, n, count) <= 3 * (int64_t)num_cus();
 }
 
 template <class T, int WN, int WM>

@@ -381,6 +381,10 @@ def test_block_projections_take_the_kernel_and_leave_the_rest(gpu_device):
         assert not interface._extension().project(x.float(), weights) and not interface._extension().project(x[:0], weights)
         big = torch.empty(1, 256 * 128 + 1, 128, device=gpu_device, dtype=torch.bfloat16)
         assert not interface._extension().project(big, weights) and interface._extension().project(big[:, 1:], weights)
+        # (a sum of many columns is not split)
+        row, narrow = torch.randn(1, 3, 8192, device=gpu_device, dtype=torch.bfloat16), [torch.randn(64, 8192, device=gpu_device, dtype=torch.bfloat16)] * 3
+        short = row[..., :4096].contiguous(), [w[:, :4096].contiguous() for w in narrow]
+        assert not interface._extension().project(row, narrow) and len(interface._extension().project(*short)) == 3
         seen = []
         handle = layers[1].register_forward_hook(lambda *a: seen.append(1))
         modules._project_all(layers, x)
