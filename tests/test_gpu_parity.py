@@ -744,12 +744,15 @@ def test_factor_gradients_summed_over_batch_groups(gpu_device, dtype, B, Lq, Lk,
     (torch.float16, 66, 4, 256, 249, 0, -0.3, 1, False),
     # enough (batch, head) pairs for a workgroup to walk several entries without summing their factor gradients
     (torch.bfloat16, 1101, 4, 200, 256, 16, None, 1, True),  # four per workgroup, the last workgroup ragged
-    (torch.float16, 2100, 1, 129, 255, 0, None, 1, True),    # no factors, two per workgroup
-    (torch.bfloat16, 4100, 2, 64, 64, 8, 1.0, 1, False),     # constant factors, eight per workgroup
+    (torch.float16, 2101, 1, 144, 200, 24, None, 1, False),  # constant factors of a rank that the ring kernel does not take, two
+    (torch.bfloat16, 4100, 2, 130, 64, 32, 1.0, 1, False),   # ... eight per workgroup
+    # the ring kernel's: no factors, and constant factors of a rank up to 16
+    (torch.float16, 2100, 1, 129, 255, 0, None, 1, True),    # one per workgroup
+    (torch.bfloat16, 4100, 2, 64, 64, 8, 1.0, 1, False),     # four per workgroup
 ])
 def test_window_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, group, grads):
-    """Whole sequences of at most 256 positions at head dim 32 on grids that fill the chip: fb_bwd runs the
-    preprocess step and one kernel that forms all five gradients per (batch, head), dq summed inside the
+    """Whole sequences of at most 256 positions at head dim 32 on grids that fill the chip: fb_bwd runs one
+    kernel that forms the statistics and all gradients per (batch, head), dq summed inside the
     workgroup.  Checked through the C ABI against the oracle, against the three phases called one by one (other
     kernels, other summation orders: equal up to rounding) and against itself (bit-reproducible)."""
     from flashbias_amd import _lib
