@@ -453,7 +453,7 @@ static hipError_t launch_win_r(const BwdArgs &a, hipStream_t stream) {
 }
 
 // Compiled once per element type for head dim 32 (see Makefile).  When fb_bwd takes this path is decided by
-// window_backward() in fb_kernels.h; the statistics must be in the scratch buffer (preprocess step).
+// window_backward() in fb_kernels.h.
 #define FB_CAT2(a, b) a##b
 #define FB_CAT(a, b) FB_CAT2(a, b)
 hipError_t FB_CAT(launch_bwd_win_, FB_SUFFIX)(const BwdArgs &a, hipStream_t stream) {

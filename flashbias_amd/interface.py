@@ -52,8 +52,10 @@ def _fold_keeps_rank_in_range(rank):
 
 
 def _fold_pays(q, k, q_bias, k_bias, mask):
-    """Whether a large vector mask is ahead as one more factor column.  The kernels take a vector mask at the price of an
-    unmasked call (aligned tensors, ranks up to 32): forward + backward, the kernels' own / folded / without a mask, in ms:
+    """Whether a large vector mask is ahead as one more factor column.  On aligned tensors at ranks up to 32
+    the kernels take a vector mask at 2 to 4 % above the price of an unmasked call (head dims above 64: 8 %; head dim 32 at
+    rank 8: 22 %, whose unmasked calls have kernels of their own).  Forward + backward, the kernels' own / folded / without a
+    mask, in ms:
     B2 H4 L=16384 d32 2.00 / 2.01 / 1.64 at rank 8, 2.04 / 2.26 / 1.98 at 16, 2.32 / 2.99 / 2.25 at 32; B4 H16 L=4096 d64
     1.53 / 1.54 / 1.50, 1.54 / 1.70 / 1.50, 1.62 / 2.98 / 1.57; 768 x 4 rows of 768 whose factors are shared, rank 32,
     2.24 / 5.92 / 2.15.  What is left for the fold: head dims above 64 at ranks that stay in one 16-wide step, whose
