@@ -281,7 +281,7 @@ __device__ __forceinline__ void fwd_body(const FwdArgs &a) {
     u32x4_t qr[C::QB][C::NKD], qbr[C::QB][C::NKR > 0 ? C::NKR : 1];
     f32x16_t acc_o[C::QB][C::NDV];
     float m_ref[C::QB]; // reference of the exponentials (natural units), lags the true row max
-    float m2[C::QB];    // m_ref * log2(e), 0 while the row has seen no finite score
+    float m2[C::QB];    // m_ref * log2(e) (reference_log2; any finite number while the row has seen no finite score)
     float l_run[C::QB]; // per-lane partial row sum (the two lanes of a query are added at the end)
 #pragma unroll
     for (int qb = 0; qb < C::QB; ++qb) {
