@@ -577,6 +577,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 
 } // namespace fb
 #include "fb_fwd_lean.h"
+#include "fb_fwd_thin.h"
 #include "fb_fwd_wide.h"
 namespace fb {
 
@@ -624,14 +625,20 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
     // d64 r8 20.0 -> 17.3; fp16 d64 r16 8 x 8 x (1000 x 1500) with a vector mask 117 -> 49); a matrix mask needs its tile
     // in LDS, larger ranks more registers, and they stay with the general one.
     constexpr bool WIDE = NKD >= 4 && NKR <= 2;
+    // Head dim 32 exactly (its copies fill whole rows), ranks up to 32: fb_fwd_thin.h at every length and grid that the
+    // streamlined kernel does not take (both sides measured at the kernel).
+    constexpr bool THIN = NKD == 2 && NKR <= 2;
     if constexpr (WIDE) {
         if (vec && a.mask.type == kVectorMask) return launch_fwd_wide<T, NKD, NKR, NDV, kVectorMask, false>(a, stream);
         if (vec && a.mask.type == kNoMask)
             return fold_scale_ok<T>(a.scale, a.r, a.Lk) ? launch_fwd_wide<T, NKD, NKR, NDV, kNoMask, true>(a, stream)
                                                        : launch_fwd_wide<T, NKD, NKR, NDV, kNoMask, false>(a, stream);
     } else if (vec && a.mask.type == kVectorMask) {
-        // A vector mask on aligned tensors, against the general masked instantiation: 384 x 4 rows of 384 tokens, rank
-        // 32, 131 -> 114 us a call.  The outputs are bit for bit the same.
+        if constexpr (THIN) {
+            if (a.d == 32) return launch_fwd_thin<T, NKR, kVectorMask, false>(a, stream);
+        }
+        // A vector mask on aligned tensors, other head dims and larger ranks, against the general masked instantiation: 384 x
+        // 4 rows of 384 tokens, rank 32, 131 -> 114 us a call.  The outputs are bit for bit the same.
         return launch_fwd_vec<T, NKD, NKR, NDV, true, kVectorMask>(a, stream);
     }
     if (a.mask.type)
@@ -649,6 +656,11 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
             return wgs >= num_cus() && !half_empty_256(a.Lq) ? launch_fwd_lean<T, NKR, 2>(a, stream)
                                                              : launch_fwd_lean<T, NKR, 1>(a, stream);
         }
+    }
+    if constexpr (THIN) {
+        if (vec && a.d == 32)
+            return fold_scale_ok<T>(a.scale, a.r, a.Lk) ? launch_fwd_thin<T, NKR, kNoMask, true>(a, stream)
+                                                       : launch_fwd_thin<T, NKR, kNoMask, false>(a, stream);
     }
     if constexpr (NKR <= 2 && !WIDE) {
         if (vec && fold_scale_ok<T>(a.scale, a.r, a.Lk)) return launch_fwd_vec<T, NKD, NKR, NDV, true, kNoMask, true>(a, stream);

@@ -304,6 +304,22 @@ def test_wide_heads(gpu_device, d, r, Lq, Lk, scale, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("r,Lq,Lk,scale", [(16, 1, 1, None), (32, 127, 63, None), (24, 129, 64, None), (0, 128, 65, None), (8, 33, 640, 1.0), (32, 130, 129, 1.0),
+                                           (16, 257, 127, -0.2), (0, 31, 192, -0.1), (16, 64, 530, 0.0625), (8, 95, 100, None)])
+def test_thin_forward(gpu_device, r, Lq, Lk, scale, dtype):
+    """Forward of head dim 32 with four waves a SIMD at the edges of its tiles (128 queries, 64 keys, two stages), padded ranks,
+    the scale folded (a power of two, 1, low parts at rank 8, a negative one without factors) and not, causal, and vector masks of
+    both kinds whose last keys are off."""
+    for kind in (None, "causal", "mask"):
+        mask = None
+        if kind == "mask":
+            mask = torch.randn(2, 1, 1, Lk, generator=torch.Generator().manual_seed(Lk))
+            mask[1, ..., Lk - Lk // 4:] = float("-inf")
+            mask = mask.to(dtype if Lq % 2 else torch.float32)
+        _case(gpu_device, 2, Lq, Lk, 3, 32, r, dtype, kind == "causal", mask=mask, scale=scale, seed=r + Lk, o_by_magnitude=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind,Lq,Lk,r,scale,shared", [
     ("matrix", 256, 256, 16, 1.0, True), ("matrix", 144, 144, 16, None, True), ("matrix", 129, 200, 32, None, False),
     ("matrix", 200, 129, 0, None, False), ("matrix", 131, 250, 8, 1.0, False), ("vector", 64, 64, 16, None, True),
