@@ -102,75 +102,96 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 
 #pragma unroll 1
         for (int qb = wave; qb < nqb; qb += C::NWAVES) {
+            if (!C::MASK && qb != wave) load_q(qb); // (a block ahead, as with a mask, it takes registers that pairs of blocks need)
             u32x4_t q[C::NK];
 #pragma unroll
             for (int t = 0; t < C::NK; ++t) q[t] = qn[t];
-            if (qb + C::NWAVES < nqb) load_q(qb + C::NWAVES);
+            if (C::MASK && qb + C::NWAVES < nqb) load_q(qb + C::NWAVES);
             f32x16_t o;
 #pragma unroll
             for (int v = 0; v < 16; ++v) o[v] = 0.f;
             float m_ref = -INFINITY, m2 = 0.f, l_run = 0.f, slack = lag;
-#pragma unroll 1
-            for (int kb = 0; kb < nkb; ++kb) {
+            // N blocks of 32 keys from block kb on.  Without a mask two at a time (one row maximum, one test of the reference point and
+            // one set of addresses for 64 keys), the last of an odd number alone: 4096 x 16 windows of 256 tokens 1430 -> 1354 us,
+            // 769 x 16 of 144 148 -> 142, 64 x 16 of 256 28.7 -> 27.  Masked blocks alone: the copies of two would leave two
+            // workgroups a compute unit, and masks loaded to registers a pair ahead cost more (1024 x 16 of 256 473 -> 635).
+            auto group = [&](auto tag, int kb) __attribute__((always_inline)) {
+                constexpr int N = decltype(tag)::value;
                 const uint32_t at = kb * 2048;
-                f32x16_t s, sb;
-                if constexpr (C::MASK) {
-                    wait_vmcnt<0>();
+                f32x16_t s[N];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) { // register v <-> key 32 kb + 8 (v / 4) + 4 g + v % 4 of the lane's row
-                        const u32x2_t x = *reinterpret_cast<const u32x2_t *>(smem + C::MT + wave * 2048 + lean_chunk_off<4>(c, j) + 8 * g);
-                        sb[4 * j + 0] = T::to_float((uint16_t)(x[0] & 0xffffu));
-                        sb[4 * j + 1] = T::to_float((uint16_t)(x[0] >> 16));
-                        sb[4 * j + 2] = T::to_float((uint16_t)(x[1] & 0xffffu));
-                        sb[4 * j + 3] = T::to_float((uint16_t)(x[1] >> 16));
+                for (int n = 0; n < N; ++n) {
+                    f32x16_t sb;
+                    if constexpr (C::MASK) {
+                        static_assert(N == 1, "");
+                        wait_vmcnt<0>();
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) { // register v <-> key 32 kb + 8 (v / 4) + 4 g + v % 4 of the lane's row
+                            const u32x2_t x = *reinterpret_cast<const u32x2_t *>(smem + C::MT + wave * 2048 + lean_chunk_off<4>(c, j) + 8 * g);
+                            sb[4 * j + 0] = T::to_float((uint16_t)(x[0] & 0xffffu));
+                            sb[4 * j + 1] = T::to_float((uint16_t)(x[0] >> 16));
+                            sb[4 * j + 2] = T::to_float((uint16_t)(x[1] & 0xffffu));
+                            sb[4 * j + 3] = T::to_float((uint16_t)(x[1] >> 16));
+                        }
+                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (they have left LDS: the block after this one)
+                        if (kb + 1 < nkb)
+                            copy_mask(qb, kb + 1);
+                        else if (qb + C::NWAVES < nqb)
+                            copy_mask(qb + C::NWAVES, 0);
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) sb[v] = 0.f;
                     }
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (they have left LDS: the block after this one)
-                    if (kb + 1 < nkb)
-                        copy_mask(qb, kb + 1);
-                    else if (qb + C::NWAVES < nqb)
-                        copy_mask(qb + C::NWAVES, 0);
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) sb[v] = 0.f;
-                }
-                // q k^T and q_b k_b^T: two chains joined by the FMA that applies the softmax scale to the first (:246-256),
-                // an additive mask the initial value of the second; folded, one chain
-                if constexpr (C::FOLD)
-                    s = sb;
-                else
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) s[v] = 0.f;
-#pragma unroll
-                for (int t = 0; t < C::NKD; ++t) s = T::mfma(lds_load16(row_off[t] + C::K + at), q[t], s);
-                if constexpr (C::NKR > 0) {
-                    const u32x4_t kf = lds_load16(kb_row + kb * 1024);
+                    // q k^T and q_b k_b^T: two chains joined by the FMA that applies the softmax scale to the first (:246-256),
+                    // an additive mask the initial value of the second; folded, one chain
                     if constexpr (C::FOLD)
-                        s = T::mfma(kf, q[C::NKD], s);
+                        s[n] = sb;
                     else
-                        sb = T::mfma(kf, q[C::NKD], sb);
-                }
-                if constexpr (!C::FOLD) {
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) s[v] = __builtin_fmaf(s[v], a.scale, sb[v]);
+                        for (int v = 0; v < 16; ++v) s[n][v] = 0.f;
+#pragma unroll
+                    for (int t = 0; t < C::NKD; ++t) s[n] = T::mfma(lds_load16(row_off[t] + C::K + at + n * 2048), q[t], s[n]);
+                    if constexpr (C::NKR > 0) {
+                        const u32x4_t kf = lds_load16(kb_row + kb * 1024 + n * 1024);
+                        if constexpr (C::FOLD)
+                            s[n] = T::mfma(kf, q[C::NKD], s[n]);
+                        else
+                            sb = T::mfma(kf, q[C::NKD], sb);
+                    }
+                    if constexpr (!C::FOLD) {
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) s[n][v] = __builtin_fmaf(s[n][v], a.scale, sb[v]);
+                    }
+                    // (the second block's fragments are not requested ahead of the first block's scores: that spills)
+                    if constexpr (N > 1) __builtin_amdgcn_sched_barrier(0);
                 }
                 u32x4_t vt[2];
+                if constexpr (N == 1) {
 #pragma unroll
-                for (int t = 0; t < 2; ++t) vt[t] = lds_load_tr(col_off[0] + at + t * 1024, col_off[1] + at + t * 1024);
-                if (32 * kb + 32 > a.Lk) {
-                    const int key0 = 32 * kb + 4 * g;
-#pragma unroll
-                    for (int v = 0; v < 16; ++v)
-                        if (key0 + 8 * (v >> 2) + (v & 3) >= a.Lk) s[v] = -INFINITY;
+                    for (int t = 0; t < 2; ++t) vt[t] = lds_load_tr(col_off[0] + at + t * 1024, col_off[1] + at + t * 1024);
                 }
-                asm volatile("s_nop 11" : "+v"(s)); // (fb_bwd_win.hip: wait states across the branch above)
-                float mx = s[0];
+                if (32 * (kb + N) > a.Lk) {
 #pragma unroll
-                for (int v = 1; v < 16; ++v) mx = fmaxf(mx, s[v]);
+                    for (int n = 0; n < N; ++n) {
+                        int key0 = 32 * (kb + n) + 4 * g;
+                        asm volatile("" : "+v"(key0)); // (formed in the branch)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v)
+                            if (key0 + 8 * (v >> 2) + (v & 3) >= a.Lk) s[n][v] = -INFINITY;
+                    }
+                }
+#pragma unroll
+                for (int n = 0; n < N; ++n) asm volatile("s_nop 11" : "+v"(s[n])); // (fb_bwd_win.hip: wait states across the branch above)
+                float mx = s[0][0];
+#pragma unroll
+                for (int n = 0; n < N; ++n)
+#pragma unroll
+                    for (int v = n == 0; v < 16; ++v) mx = fmaxf(mx, s[n][v]);
                 mx = half_wave_max(mx);
-                // After an even block that moved the reference the odd one moves it without a lag, so that it is the
+                // Single blocks: after an even one that moved the reference the odd one moves it without a lag, so that it is the
                 // maximum of 64 keys, as in fwd_kernel: the probability 1 is the one that is not rounded.
                 const bool grow = mx > m_ref + slack; // also true for the first finite score of a row
-                slack = grow && !(kb & 1) ? 0.f : lag;
+                if constexpr (C::MASK) slack = grow && !(kb & 1) ? 0.f : lag;
                 if (__any(grow)) {
                     const float m_new = grow ? mx : m_ref;
                     const float alpha = grow ? fast_exp2((m_ref - m_new) * to_log2) : 1.f; // exp2(-inf) = 0
@@ -181,18 +202,29 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                     m2 = reference_log2<T>(m_new, to_log2);
                 }
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    u32x4_t pb;
+                for (int n = 0; n < N; ++n)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float p0 = fast_exp2(__builtin_fmaf(s[8 * t + 2 * e], to_log2, -m2));
-                        const float p1 = fast_exp2(__builtin_fmaf(s[8 * t + 2 * e + 1], to_log2, -m2));
-                        pb[e] = T::pack2(p0, p1);
-                        l_run += p0 + p1;
+                    for (int t = 0; t < 2; ++t) {
+                        if constexpr (N > 1) vt[t] = lds_load_tr(col_off[0] + at + n * 2048 + t * 1024, col_off[1] + at + n * 2048 + t * 1024);
+                        u32x4_t pb;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float p0 = fast_exp2(__builtin_fmaf(s[n][8 * t + 2 * e], to_log2, -m2));
+                            const float p1 = fast_exp2(__builtin_fmaf(s[n][8 * t + 2 * e + 1], to_log2, -m2));
+                            pb[e] = T::pack2(p0, p1);
+                            l_run += p0 + p1;
+                        }
+                        o = T::mfma(vt[t], pb, o);
                     }
-                    o = T::mfma(vt[t], pb, o);
-                }
                 asm volatile("s_nop 11" : "+v"(o)); // (across the loop's branches)
+            };
+            if constexpr (C::MASK) {
+#pragma unroll 1
+                for (int kb = 0; kb < nkb; ++kb) group(std::integral_constant<int, 1>{}, kb);
+            } else {
+#pragma unroll 1
+                for (int kb = 0; kb + 1 < nkb; kb += 2) group(std::integral_constant<int, 2>{}, kb);
+                if (nkb & 1) group(std::integral_constant<int, 1>{}, nkb - 1);
             }
             const float l = l_run + __shfl_xor(l_run, 32, 64);
             const int query = 32 * qb + c;

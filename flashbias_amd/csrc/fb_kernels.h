@@ -175,8 +175,8 @@ inline bool ring_backward(const BwdArgs &a) {
 // Whether fb_fwd runs the forward for windows (fb_fwd_win.hip): whole sequences of at most 256 positions, head dim 32, a
 // rank up to 16, aligned tensors, no mask or a matrix mask of 16-byte chunks, a scale that keeps the order of the scores.
 // Against the general kernel, rank 16, us (window / general): 8192 pairs of 64 tokens 35 / 55, of 128 66 / 75, of 144
-// 107 / 183, with a matrix mask 47 / 84, 90 / 126, 149 / 318; 65536 of 256 1535 / 1572, masked 1904 / 2796; 512 pairs
-// of 144 14 / 16, masked 16 / 24; 512 of 256 21 / 19, masked 24 / 28; 1024 of 256 33 / 33.  Below two workgroups per compute unit
+// 107 / 183, with a matrix mask 47 / 84, 90 / 126, 149 / 318; 65536 of 256 1354 / 1572, masked 1904 / 2796; 512 pairs
+// of 144 14 / 16, masked 16 / 24; 512 of 256 21 / 19, masked 24 / 28; 1024 of 256 26 / 33.  Below two workgroups per compute unit
 // the general kernel's smaller workgroups spread better (256 of 256 16 / 13).
 inline bool window_forward(const FwdArgs &a) {
     const int64_t lim = (int64_t)1 << 22; // (32-bit byte offsets of 256 rows)
