@@ -635,6 +635,7 @@ static hipError_t launch_dkv_part(const BwdArgs &a0, hipStream_t stream) {
 
 } // namespace fb
 #include "fb_bwd_dkv_pair.h"
+#include "fb_bwd_dkv_mid.h"
 namespace fb {
 
 // One pass, or (head dims above 64, aligned tensors) two waves a block of keys or three passes that each keep a part
@@ -651,6 +652,8 @@ static hipError_t launch_dkv_vec(const BwdArgs &a, hipStream_t stream) {
             if (e != hipSuccess) return e;
         }
         return launch_dkv_part<T, NKD, NKR, NDV, VEC, MASK, 4, FOLD>(a, stream);
+    } else if constexpr (NKD == 4 && VEC && NKR <= 2 && MASK != kMatrixMask) {
+        return launch_dkv_mid<T, NKR, MASK, FOLD>(a, stream); // (head dims 33 ... 64, at every length and grid: measured at the kernel)
     } else {
         // head dim 32, aligned, unmasked, no dk_bias wanted: the instantiation without its products
         if constexpr (NKD == 2 && NKR > 0 && NKR <= 2 && VEC && !MASK) {

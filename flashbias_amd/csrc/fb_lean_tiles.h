@@ -189,24 +189,27 @@ __device__ __forceinline__ u32x4_t dense_read_a_tr(const uint8_t *region, int ro
     }
 }
 
-// Reads of a swizzled tile with 16 chunks per row (swz_off<16>) from one address register per access pattern: the chunk of
-// contraction step t, or of column block n, differs from the first one's in address bits that are XORed in, one
-// vector instruction a read, where one register for each of the 8 + 8 addresses costs a kernel its last ones (what
-// the compiler keeps if it may; the values are made opaque where they are formed).
-struct TileAddr16 {
+// Reads of a swizzled tile with ROWCH (8 or 16) chunks per row (swz_off<ROWCH>) from one address register per access pattern: the
+// chunk of contraction step t, or of column block n, differs from the first one's in address bits that are XORed in, one
+// vector instruction a read, where one register for each of the addresses costs a kernel its last ones (what the
+// compiler keeps if it may; the values are made opaque where they are formed).
+template <int ROWCH>
+struct TileAddr {
+    static constexpr int RB = 16 * ROWCH; // bytes of a row
     uint32_t row, tr;
-    __device__ __forceinline__ TileAddr16(uint32_t tile, int c, int g) {
+    __device__ __forceinline__ TileAddr(uint32_t tile, int c, int g) {
         const int r = 4 * g + ((c & 15) >> 2), chunk = 2 * (c >> 4) + ((c & 3) >> 1);
-        row = tile + c * 256 + ((g ^ swz_of<16>(c)) << 4);
-        tr = tile + r * 256 + ((chunk ^ swz_of<16>(r)) << 4) + 8 * (c & 1);
+        row = tile + c * RB + ((g ^ swz_of<ROWCH>(c)) << 4);
+        tr = tile + r * RB + ((chunk ^ swz_of<ROWCH>(r)) << 4) + 8 * (c & 1);
     }
     // chunk 2 t + g of row c of the 32 rows that start at byte `at` of the tile
     __device__ __forceinline__ u32x4_t load_row(int t, int at) const { return lds_load16((row ^ (uint32_t)(32 * t)) + at); }
-    // lds_read_a_tr<16> for the 16 rows that start at byte `at`, columns [32 n, 32 n + 32)  (row + 8: swizzle bit 1)
+    // lds_read_a_tr<ROWCH> for the 16 rows that start at byte `at`, columns [32 n, 32 n + 32)  (row + 8: swizzle bit 1)
     __device__ __forceinline__ u32x4_t load_tr(int n, int at) const {
-        return lds_load_tr((tr ^ (uint32_t)(64 * n)) + at, (tr ^ (uint32_t)(64 * n + 32)) + at + 8 * 256);
+        return lds_load_tr((tr ^ (uint32_t)(64 * n)) + at, (tr ^ (uint32_t)(64 * n + 32)) + at + 8 * RB);
     }
 };
+typedef TileAddr<16> TileAddr16;
 
 // The kernel arguments as a function called by the kernel may read them: a function's pointer
 // argument arrives in vector registers, which would make every value loaded through it look

@@ -320,6 +320,33 @@ def test_thin_forward(gpu_device, r, Lq, Lk, scale, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,r,Lq,Lk,scale", [(64, 16, 1, 1, None), (64, 32, 63, 127, None), (40, 8, 64, 129, None), (64, 0, 65, 128, None), (56, 24, 600, 200, 0.125),
+                                             (48, 16, 129, 33, 1.0), (64, 8, 127, 96, -0.1), (64, 0, 530, 64, -0.2), (64, 32, 200, 31, 0.0625)])
+def test_key_gradients_of_middle_head_dims(gpu_device, d, r, Lq, Lk, scale, dtype):
+    """dk, dv and dk_bias of head dims 33 ... 64 at the edges of the kernel's tiles (64 queries a step, two blocks, 128 keys),
+    padded head dims and ranks, the scale folded and not, causal, vector masks, constant factors (without their gradients) and
+    factors shared by the batch (summed over groups of entries)."""
+    for kind in (None, "causal", "mask"):
+        mask = None
+        if kind == "mask":
+            mask = torch.randn(2, 1, 1, Lk, generator=torch.Generator().manual_seed(Lq))
+            mask[1, ..., Lk - Lk // 4:] = float("-inf")
+            mask = mask.to(dtype if Lk % 2 else torch.float32)
+        _case(gpu_device, 2, Lq, Lk, 3, d, r, dtype, kind == "causal", mask=mask, scale=scale, seed=d + r + Lq, o_by_magnitude=True)
+    if r:
+        q, k, v, qb, kb, do = [t.to(gpu_device) for t in make_inputs(33, Lq, Lk, 2, d, r, dtype, seed=7, bq=(True, False), bk=(True, False))]
+        leaves = [t.detach().requires_grad_(True) for t in (q, k, v, qb, kb)]
+        every = torch.autograd.grad(flash_bias_func(*leaves, None, False, scale), leaves, do)
+        few = torch.autograd.grad(flash_bias_func(*leaves[:3], qb, kb, None, False, scale), leaves[:3], do)
+        for name, x, y in zip(NAMES[1:4], every, few):
+            assert torch.equal(x, y), name
+        ref = oracle(*(t.cpu() for t in (q, k, v)), *(t.cpu().expand(33, -1, -1, -1) for t in (qb, kb)), None, False, scale, do.cpu())
+        got = every[4].float().cpu()
+        want = ref[6].sum(0, keepdim=True)
+        assert (got - want).abs().max() <= GRAD_TOL * max(1e-3, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind,Lq,Lk,r,scale,shared", [
     ("matrix", 256, 256, 16, 1.0, True), ("matrix", 144, 144, 16, None, True), ("matrix", 129, 200, 32, None, False),
     ("matrix", 200, 129, 0, None, False), ("matrix", 131, 250, 8, 1.0, False), ("vector", 64, 64, 16, None, True),
