@@ -17,8 +17,6 @@
 
 namespace fb {
 
-#define FB_HOLD __builtin_amdgcn_sched_barrier(0) // (nothing moves across)
-
 template <class T, int NKR_, int MASK_, bool FOLD_, bool BG_>
 struct DkvMidCfg {
     static constexpr int NKD = 4, NKR = NKR_, NK = NKD + NKR_, NDV = 2;
@@ -274,8 +272,6 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
         store_acc_rows<T, true>(row, ok, a.dkb.vec_ok, acc_b, 1.f, a.r, lane >> 5);
     }
 }
-
-#undef FB_HOLD
 
 template <class T, int NKR, int MASK, bool FOLD, bool BG>
 static hipError_t launch_dkv_mid_bg(const BwdArgs &a0, hipStream_t stream) {

@@ -19,19 +19,6 @@
 
 namespace fb {
 
-#define FB_HOLD __builtin_amdgcn_sched_barrier(0) // (nothing moves across)
-
-// The region since the last FB_HOLD as M times (one product, D LDS reads, V vector instructions).
-template <int M, int D, int V>
-__device__ __forceinline__ void mix() {
-#pragma unroll
-    for (int i = 0; i < M; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (D) __builtin_amdgcn_sched_group_barrier(0x100, D, 0);
-        if (V) __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
-    }
-}
-
 template <class T, int NKR_, int MASK_, bool FOLD_>
 struct DkvPairCfg {
     static constexpr int NKD = 8, NKR = NKR_, NK = NKD + NKR_, NDV = 4, MB = 4 + (NKR_ > 0 ? 1 : 0);
@@ -426,8 +413,6 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
     else
         walk(std::false_type{});
 }
-
-#undef FB_HOLD
 
 template <class T, int NKR, int MASK, bool FOLD>
 static hipError_t launch_dkv_pair(const BwdArgs &a0, hipStream_t stream) {

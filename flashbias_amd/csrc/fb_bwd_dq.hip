@@ -223,6 +223,52 @@ __device__ __forceinline__ void dq_store(const BwdArgs &a, const f32x16_t (&acc)
     }
 }
 
+// -delta and lse * log2(e) of this lane's query: formed here (stats_here) or as the preprocess step left them in the scratch buffer.
+template <class T, int NKD, bool VEC>
+__device__ __forceinline__ void dq_row_stats(const BwdArgs &a, const u32x4_t (&dor)[NKD], int b, int h, int bh, int query, int g, float &nd, float &l2) {
+    const bool ok = query < a.Lq;
+    const int64_t sidx = (int64_t)bh * a.Lq + (ok ? query : a.Lq - 1);
+    if (a.stats_here) {
+        // delta = rowsum(o * dO) of this lane's query (flash_bias_triton.py:358-400) from the dO
+        // chunks it holds and the same chunks of o; the other half of the channels is with lane ^ 32.
+        // -delta and lse * log2(e) also go to the scratch buffer, for the dk/dv kernel that follows.
+        const uint16_t *obase = a.o.ptr + b * a.o.sb + h * a.o.sh;
+        // (summed in the order of the preprocess kernel: per 8-channel chunk, then a pairwise tree
+        // over the chunks, so that both ways of running the backward give the same bits)
+        float cs[NKD];
+#pragma unroll
+        for (int t = 0; t < NKD; ++t) {
+            const u32x4_t oc = load_chunk<VEC>(obase, a.o.ss, query, a.Lq, 16 * t + 8 * g, a.d);
+            float acc1 = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc1 = __builtin_fmaf(T::to_float((uint16_t)(oc[e] & 0xffffu)),
+                                      T::to_float((uint16_t)(dor[t][e] & 0xffffu)), acc1);
+                acc1 = __builtin_fmaf(T::to_float((uint16_t)(oc[e] >> 16)), T::to_float((uint16_t)(dor[t][e] >> 16)),
+                                      acc1);
+            }
+            cs[t] = acc1 + __shfl_xor(acc1, 32, 64); // chunks 2t and 2t + 1
+        }
+#pragma unroll
+        for (int m = 1; m < NKD; m <<= 1)
+#pragma unroll
+            for (int t = 0; t + m < NKD; t += 2 * m) cs[t] += cs[t + m];
+        const float part = cs[0];
+        nd = ok ? -part : 0.f;
+        l2 = ok ? a.lse[sidx] * kLog2e : INFINITY;
+        if (ok && g == 0) {
+            const int64_t rows = (int64_t)a.B * a.H * a.Lq;
+            a.delta[sidx] = nd;
+            a.delta[rows + sidx] = l2;
+            if (a.stat_chunks) reinterpret_cast<u32x4_t *>(a.delta + stat_offset(rows))[sidx] = stat_chunk<T>(nd, l2);
+        }
+    } else {
+        // the preprocess step left -delta and lse * log2(e) in the scratch buffer
+        l2 = ok ? a.delta[(int64_t)a.B * a.H * a.Lq + sidx] : INFINITY;
+        nd = ok ? a.delta[sidx] : 0.f;
+    }
+}
+
 // The whole dq / dq_bias computation of one workgroup; the kernel below is nothing else.
 template <class T, class C>
 __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
@@ -313,48 +359,8 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
                 }
             }
         }
-        const bool ok = query < a.Lq;
-        const int64_t sidx = (int64_t)bh * a.Lq + (ok ? query : a.Lq - 1);
         float nd, l2;
-        if (a.stats_here) {
-            // delta = rowsum(o * dO) of this lane's query (flash_bias_triton.py:358-400) from the dO
-            // chunks it holds and the same chunks of o; the other half of the channels is with lane ^ 32.
-            // -delta and lse * log2(e) also go to the scratch buffer, for the dk/dv kernel that follows.
-            const uint16_t *obase = a.o.ptr + b * a.o.sb + h * a.o.sh;
-            // (summed in the order of the preprocess kernel: per 8-channel chunk, then a pairwise tree
-            // over the chunks, so that both ways of running the backward give the same bits)
-            float cs[C::NKD];
-#pragma unroll
-            for (int t = 0; t < C::NKD; ++t) {
-                const u32x4_t oc = load_chunk<C::VEC>(obase, a.o.ss, query, a.Lq, 16 * t + 8 * g, a.d);
-                float acc1 = 0.f;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    acc1 = __builtin_fmaf(T::to_float((uint16_t)(oc[e] & 0xffffu)),
-                                          T::to_float((uint16_t)(dor[qb][t][e] & 0xffffu)), acc1);
-                    acc1 = __builtin_fmaf(T::to_float((uint16_t)(oc[e] >> 16)), T::to_float((uint16_t)(dor[qb][t][e] >> 16)),
-                                          acc1);
-                }
-                cs[t] = acc1 + __shfl_xor(acc1, 32, 64); // chunks 2t and 2t + 1
-            }
-#pragma unroll
-            for (int m = 1; m < C::NKD; m <<= 1)
-#pragma unroll
-                for (int t = 0; t + m < C::NKD; t += 2 * m) cs[t] += cs[t + m];
-            const float part = cs[0];
-            nd = ok ? -part : 0.f;
-            l2 = ok ? a.lse[sidx] * kLog2e : INFINITY;
-            if (ok && g == 0) {
-                const int64_t rows = (int64_t)a.B * a.H * a.Lq;
-                a.delta[sidx] = nd;
-                a.delta[rows + sidx] = l2;
-                if (a.stat_chunks) reinterpret_cast<u32x4_t *>(a.delta + stat_offset(rows))[sidx] = stat_chunk<T>(nd, l2);
-            }
-        } else {
-            // the preprocess step left -delta and lse * log2(e) in the scratch buffer
-            l2 = ok ? a.delta[(int64_t)a.B * a.H * a.Lq + sidx] : INFINITY;
-            nd = ok ? a.delta[sidx] : 0.f;
-        }
+        dq_row_stats<T, C::NKD, C::VEC>(a, dor[qb], b, h, bh, query, g, nd, l2);
         lse2[qb] = l2; // rows past the end: P = exp2(-inf) = 0
 #pragma unroll
         for (int v = 0; v < 16; ++v) negd[qb][v] = C::SPLIT ? 0.f : nd;
@@ -628,9 +634,9 @@ bwd_dq_kernel(const BwdArgs a) {
     bwd_dq_body<T, C>(a, blockIdx.x);
 }
 
-template <class T, int NKD, int NKR, bool VEC, int MASK, bool QB2, bool FOLD, bool SPLIT, bool BG>
-static hipError_t launch_dq_qb_bg(const BwdArgs &a0, hipStream_t stream) {
-    typedef DqCfg<T, NKD, NKR, VEC, MASK, QB2, FOLD, SPLIT, BG> C;
+template <class T, int NKD, int NKR, bool VEC, int MASK, bool QB2, bool FOLD, bool SPLIT = false>
+static hipError_t launch_dq_qb(const BwdArgs &a0, hipStream_t stream) {
+    typedef DqCfg<T, NKD, NKR, VEC, MASK, QB2, FOLD, SPLIT> C;
     BwdArgs a = a0;
     a.ntiles_m = (a.Lq + C::BM - 1) / C::BM;
     auto kern = bwd_dq_kernel<T, C>;
@@ -641,15 +647,6 @@ static hipError_t launch_dq_qb_bg(const BwdArgs &a0, hipStream_t stream) {
     const int64_t total = (int64_t)a.ntiles_m * ((a.B + group - 1) / group) * a.H;
     a.slots = slots_per_cu(kern, C::NTHREADS, C::LDS_BYTES, total, once);
     return launch_flat(kern, total, C::NTHREADS, C::LDS_BYTES, stream, a);
-}
-
-template <class T, int NKD, int NKR, bool VEC, int MASK, bool QB2, bool FOLD, bool SPLIT = false>
-static hipError_t launch_dq_qb(const BwdArgs &a, hipStream_t stream) {
-    // head dim 32, aligned, unmasked, no dq_bias wanted: the instantiation without its products
-    if constexpr (NKD == 2 && NKR > 0 && NKR <= 2 && VEC && MASK == kNoMask && !SPLIT) {
-        if (!a.dqb.ptr) return launch_dq_qb_bg<T, NKD, NKR, VEC, MASK, QB2, FOLD, SPLIT, false>(a, stream);
-    }
-    return launch_dq_qb_bg<T, NKD, NKR, VEC, MASK, QB2, FOLD, SPLIT, true>(a, stream);
 }
 
 // 256-query workgroups (two blocks per wave) once every compute unit has two of them (three under
@@ -672,6 +669,7 @@ static hipError_t launch_dq_vec(const BwdArgs &a, hipStream_t stream) {
 
 } // namespace fb
 #include "fb_bwd_dq_lean.h"
+#include "fb_bwd_dq_mid.h"
 namespace fb {
 
 template <class T, int NKD, int NKR>
@@ -697,10 +695,18 @@ static hipError_t launch_dq_cfg(const BwdArgs &a, hipStream_t stream) {
             return launch_dq_lean<T, NKR>(a, stream);
         }
     }
-    if constexpr (NKR <= 2) {
-        if (vec && fold_scale_ok<T>(a.scale, a.r, a.Lk)) return launch_dq_vec<T, NKD, NKR, true, kNoMask, true>(a, stream);
+    constexpr int MID = dq_mid_use(NKD, NKR);
+    if constexpr (MID > 0) {
+        if (vec && (MID == 2 || !a.dqb.ptr))
+            return fold_scale_ok<T>(a.scale, a.r, a.Lk) ? launch_dq_mid<T, NKD, NKR, true>(a, stream) : launch_dq_mid<T, NKD, NKR, false>(a, stream);
     }
-    return vec ? launch_dq_vec<T, NKD, NKR, true, kNoMask>(a, stream) : launch_dq_vec<T, NKD, NKR, false, kNoMask>(a, stream);
+    if constexpr (MID < 2) {
+        if constexpr (NKR <= 2) {
+            if (vec && fold_scale_ok<T>(a.scale, a.r, a.Lk)) return launch_dq_vec<T, NKD, NKR, true, kNoMask, true>(a, stream);
+        }
+        if (vec) return launch_dq_vec<T, NKD, NKR, true, kNoMask>(a, stream);
+    }
+    return launch_dq_vec<T, NKD, NKR, false, kNoMask>(a, stream);
 }
 
 template <class T, int NKD>

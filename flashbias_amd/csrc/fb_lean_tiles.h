@@ -210,6 +210,28 @@ struct TileAddr {
     }
 };
 typedef TileAddr<16> TileAddr16;
+// The same for a dense region of 4-chunk rows (lean_chunk_off<4>: two rows a line, the swizzle in the same address bits).
+template <>
+struct TileAddr<4> {
+    static constexpr int RB = 64;
+    uint32_t row, tr;
+    __device__ __forceinline__ TileAddr(uint32_t tile, int c, int g) : row(tile + lean_row_addr<4>(c, g)), tr(tile + lean_tr_addr4(c, g, 0)) {}
+    __device__ __forceinline__ u32x4_t load_row(int t, int at) const { return lds_load16((row ^ (uint32_t)(32 * t)) + at); }
+    __device__ __forceinline__ u32x4_t load_tr(int, int at) const { return lds_load_tr(tr + at, (tr ^ 32u) + at + 8 * RB); }
+};
+
+#define FB_HOLD __builtin_amdgcn_sched_barrier(0) // (nothing moves across)
+
+// The region since the last FB_HOLD as M times (one product, D LDS reads, V vector instructions).
+template <int M, int D, int V>
+__device__ __forceinline__ void mix() {
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (D) __builtin_amdgcn_sched_group_barrier(0x100, D, 0);
+        if (V) __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
+    }
+}
 
 // The kernel arguments as a function called by the kernel may read them: a function's pointer
 // argument arrives in vector registers, which would make every value loaded through it look

@@ -347,6 +347,23 @@ def test_key_gradients_of_middle_head_dims(gpu_device, d, r, Lq, Lk, scale, dtyp
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,r,Lq,Lk,scale", [(32, 32, 1, 1, None), (32, 16, 127, 63, None), (24, 24, 129, 64, None), (32, 32, 128, 65, 1.0), (32, 8, 33, 600, None),
+                                             (32, 16, 130, 129, 0.125), (24, 16, 257, 127, -0.2), (64, 16, 127, 64, None), (40, 24, 129, 65, 0.3)])
+def test_query_gradients_one_block_a_wave(gpu_device, d, r, Lq, Lk, scale, dtype):
+    """dq and dq_bias of head dims up to 64 at the edges of the kernel's tiles (128 queries, 64 keys, two blocks), padded head dims and
+    ranks, the scale folded and not, causal, with and without dq_bias, factors of the batch's own and shared (summed over groups)."""
+    for causal in (False, True):
+        _case(gpu_device, 2, Lq, Lk, 3, d, r, dtype, causal, scale=scale, seed=d + r + Lk, o_by_magnitude=True)
+        for B, bc in ((2, False), (33, True)):
+            q, k, v, qb, kb, do = make_inputs(B, Lq, Lk, 2, d, r, dtype, seed=9, bq=(bc, False), bk=(bc, False))
+            ref = oracle(q, k, v, *(t.expand(B, -1, -1, -1) for t in (qb, kb)), None, causal, scale, do)
+            q, k, v, qb, kb, do = (t.to(gpu_device) for t in (q, k, v, qb, kb, do))
+            leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+            got = torch.autograd.grad(flash_bias_func(*leaves, qb, kb, None, causal, scale), leaves, do)
+            _gate([ref[0]] + [t.float().cpu() for t in got] + [None, None], ref[:5] + (None, None), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind,Lq,Lk,r,scale,shared", [
     ("matrix", 256, 256, 16, 1.0, True), ("matrix", 144, 144, 16, None, True), ("matrix", 129, 200, 32, None, False),
     ("matrix", 200, 129, 0, None, False), ("matrix", 131, 250, 8, 1.0, False), ("vector", 64, 64, 16, None, True),
