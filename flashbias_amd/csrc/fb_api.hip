@@ -75,7 +75,7 @@ hipError_t launch_bwd_dq(const BwdArgs &a, bool bf16, hipStream_t stream) {
 hipError_t launch_bwd_both(const BwdArgs &a, bool bf16, hipStream_t stream) {
     return bf16 ? launch_bwd_both_bf16_2(a, stream) : launch_bwd_both_f16_2(a, stream);
 }
-// the same for the general kernels with factors of rank 8 ... 32
+// the same for the calls with factors of rank 8 ... 32 that the streamlined kernels do not cover
 hipError_t launch_bwd_both_general(const BwdArgs &a, bool bf16, hipStream_t stream) {
     return bf16 ? launch_bwd_both_general_bf16_2(a, stream) : launch_bwd_both_general_f16_2(a, stream);
 }

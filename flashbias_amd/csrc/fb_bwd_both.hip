@@ -55,31 +55,32 @@ static hipError_t launch_both_lean(const BwdArgs &a0, hipStream_t stream) {
     return launch_flat(kern, total, 256, lds, stream, a);
 }
 
-// The same for the general kernels of head dim 32 with factors of rank 8 ... 32 (aligned, unmasked, 128-row
-// workgroups of one block per wave: fb_bwd_dq.hip, fb_bwd_dkv.hip), where the grid is small in another way: under
-// a causal mask a launch lasts at least as long as its longest workgroup, which at a few hundred workgroups per
-// kind is about twice what the work would need (B1 H50 L=2048: 800 workgroups of 1 to 16 tiles on 768 slots), and
-// the two kinds in one launch fill each other's tails.  The ids alternate as above, which keeps each kind's own
-// order (longest first within every XCD's share, work_order in fb_order.h).
+// The same for head dim 32 with factors of rank 8 ... 32 where the streamlined kernels do not go (aligned, unmasked: the bodies of
+// fb_bwd_dq_mid.h and fb_bwd_dkv_mid.h, three waves a SIMD), where the grid is small in another way: under a causal mask a launch lasts at
+// least as long as its longest workgroup, which at a few hundred workgroups per kind is about twice what the work
+// would need (B1 H50 L=2048: 800 workgroups of 1 to 16 tiles on 768 slots), and the two kinds in one launch fill each other's
+// tails.  The ids alternate as above, which keeps each kind's own order (longest first within every XCD's share,
+// work_order in fb_order.h).  With the general kernels' bodies before: training step causal r2 as 16 B1 H50 L=2048 147 -> 137 us, r16 B1
+// H24 L=4096 251 -> 232, r32 B1 H8 L=3000 205 -> 167.
 template <class T, int NKR, bool FOLD, bool BG>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void bwd_both_kernel(const BwdArgs a) {
-    typedef DqCfg<T, 2, NKR, true, kNoMask, false, FOLD, false, BG> Cq;
-    typedef DkvCfg<T, 2, NKR, 1, true, kNoMask, 0, FOLD, BG> Ck;
+    typedef DqMidCfg<T, 2, NKR, FOLD, BG> Cq;
+    typedef DkvMidCfg<T, 2, NKR, kNoMask, FOLD, BG> Ck;
     const int group = a.group > 1 ? a.group : 1;
     const int nbg = (a.B + group - 1) / group;
     const int ndq = a.ntiles_m * nbg * a.H, ndkv = a.ntiles_n * nbg * a.H;
     const int paired = min(ndq, ndkv); // (both counts are multiples of 8: the launcher checks)
     const int id = blockIdx.x;
     if (id < 2 * paired ? ((id >> 3) & 1) == 0 : ndq > ndkv)
-        bwd_dq_body<T, Cq>(a, id < 2 * paired ? (id >> 4) * 8 + (id & 7) : id - paired);
+        bwd_dq_mid_body<T, Cq>(a, id < 2 * paired ? (id >> 4) * 8 + (id & 7) : id - paired);
     else
-        bwd_dkv_body<T, Ck>(a, id < 2 * paired ? (id >> 4) * 8 + (id & 7) : id - paired);
+        bwd_dkv_mid_body<T, Ck>(a, id < 2 * paired ? (id >> 4) * 8 + (id & 7) : id - paired);
 }
 
 template <class T, int NKR, bool FOLD, bool BG>
 static hipError_t launch_both_general(const BwdArgs &a0, hipStream_t stream) {
-    typedef DqCfg<T, 2, NKR, true, kNoMask, false, FOLD, false, BG> Cq;
-    typedef DkvCfg<T, 2, NKR, 1, true, kNoMask, 0, FOLD, BG> Ck;
+    typedef DqMidCfg<T, 2, NKR, FOLD, BG> Cq;
+    typedef DkvMidCfg<T, 2, NKR, kNoMask, FOLD, BG> Ck;
     static_assert(Cq::NTHREADS == 256 && Ck::NTHREADS == 256 && Cq::BM == 128 && Ck::BN == 128, "128-row workgroups of four waves");
     BwdArgs a = a0;
     a.ntiles_m = (a.Lq + Cq::BM - 1) / Cq::BM;

@@ -32,9 +32,7 @@ namespace fb {
 // SIMD, which is worth recomputing S.
 // FOLD_: the scores are scale * (q k^T + q_b (k_b / scale)^T), no multiply per score for the scale
 // (the launcher says when that is exact).
-// BG_: also accumulate dk_bias (false: the caller does not want the factor gradients; the accumulator blocks that
-// hold nothing but dk_bias are then left out).
-template <class T, int NKD_, int NKR_, int NDV_, bool VEC_, int MASK_, int PART_ = 0, bool FOLD_ = false, bool BG_ = true>
+template <class T, int NKD_, int NKR_, int NDV_, bool VEC_, int MASK_, int PART_ = 0, bool FOLD_ = false>
 struct DkvCfg {
     static constexpr bool FOLD = FOLD_;
     static constexpr bool VEC = VEC_;
@@ -53,8 +51,7 @@ struct DkvCfg {
     static constexpr int MB = (NK + 1) / 2; // 32-row blocks of [dK | dK_b]^T
     // ... of which this instantiation accumulates [MB0, MB1)
     static constexpr int MB0 = PART_ == 4 ? MB / 2 : 0,
-                         MB1 = PART_ == 1 ? 0 : PART_ == 3 ? MB / 2 : (BG_ ? MB : (NKD_ + 1) / 2);
-    static_assert(BG_ || PART_ == 0, "");
+                         MB1 = PART_ == 1 ? 0 : PART_ == 3 ? MB / 2 : MB;
     static constexpr int KBW = 1; // key blocks per wave
     static constexpr int BN = 32 * KBW * NWAVES;              // keys per workgroup
     static constexpr int QBLK = PART_ == 0 ? 2 : 1, BMQ = 32 * QBLK; // queries per step
@@ -620,9 +617,9 @@ bwd_dkv_kernel(const BwdArgs a) {
     bwd_dkv_body<T, C>(a, blockIdx.x);
 }
 
-template <class T, int NKD, int NKR, int NDV, bool VEC, int MASK, int PART, bool FOLD, bool BG = true>
+template <class T, int NKD, int NKR, int NDV, bool VEC, int MASK, int PART, bool FOLD>
 static hipError_t launch_dkv_part(const BwdArgs &a0, hipStream_t stream) {
-    typedef DkvCfg<T, NKD, NKR, NDV, VEC, MASK, PART, FOLD, BG> C;
+    typedef DkvCfg<T, NKD, NKR, NDV, VEC, MASK, PART, FOLD> C;
     BwdArgs a = a0;
     a.ntiles_n = (a.Lk + C::BN - 1) / C::BN;
     auto kern = bwd_dkv_kernel<T, C>;
@@ -652,13 +649,9 @@ static hipError_t launch_dkv_vec(const BwdArgs &a, hipStream_t stream) {
             if (e != hipSuccess) return e;
         }
         return launch_dkv_part<T, NKD, NKR, NDV, VEC, MASK, 4, FOLD>(a, stream);
-    } else if constexpr (NKD == 4 && VEC && NKR <= 2 && MASK != kMatrixMask) {
-        return launch_dkv_mid<T, NKR, MASK, FOLD>(a, stream); // (head dims 33 ... 64, at every length and grid: measured at the kernel)
+    } else if constexpr ((NKD == 2 || NKD == 4) && VEC && NKR <= 2 && MASK != kMatrixMask) {
+        return launch_dkv_mid<T, NKD, NKR, MASK, FOLD>(a, stream); // (head dims 17 ... 64, at every length and grid: measured at the kernel)
     } else {
-        // head dim 32, aligned, unmasked, no dk_bias wanted: the instantiation without its products
-        if constexpr (NKD == 2 && NKR > 0 && NKR <= 2 && VEC && !MASK) {
-            if (!a.dkb.ptr) return launch_dkv_part<T, NKD, NKR, NDV, VEC, MASK, 0, FOLD, false>(a, stream);
-        }
         return launch_dkv_part<T, NKD, NKR, NDV, VEC, MASK, 0, FOLD>(a, stream);
     }
 }

@@ -1,8 +1,8 @@
-// dk, dv and dk_bias for head dims 33 ... 64 (aligned tensors, rank up to 32, no mask or a vector mask).  Included by
+// dk, dv and dk_bias for head dims 17 ... 64 (aligned tensors, rank up to 32, no mask or a vector mask).  Included by
 // fb_bwd_dkv.hip after the pair kernel; the arithmetic is that of the general kernel, operation by operation (lane = key,
 // register = query; the same bits).
 //
-// A 32 x 32 block takes 19 or 21 products (650 cycles), about 100 vector instructions (450) and 37 LDS reads.  Left to itself the
+// Head dims above 32.  A 32 x 32 block takes 19 or 21 products (650 cycles), about 100 vector instructions (450) and 37 LDS reads.  Left to itself the
 // compiler asks for each fragment where it is used and waits for it, sixteen times a block: 4000 cycles for a wave that has a SIMD
 // to itself.  Here the reads of a phase are requested beside the products of the phase before, tiles of 128-byte rows and a dense
 // region for Q_b take half the copy instructions, and two stages leave the reads' addresses in two registers.  What is left is
@@ -12,28 +12,40 @@
 // General kernel against this one, us: fp16 r16, 8 x 8 x (1000 x 1500) with a padding mask 118 -> 97 (training step 212 -> 190);
 // bf16 r16 B4 H16 L=2048 217 -> 190 (step 409 -> 387); r8 causal B2 H8 L=4096 147 -> 119 (306 -> 276); r2 as 16 without dk_bias,
 // causal B2 H16 L=2048 80 -> 59 (177 -> 156); r32 B1 H4 L=1000 54 -> 42 (106 -> 94).
+//
+// Head dim 32: three waves a SIMD (125 to 168 registers) cover for each other as in the general kernel; what counts is the dense
+// rows of 64 bytes, three or four copy instructions a wave and step for six or seven (the copies were a tenth of the cycles).
+// General kernel against this one, training step, us, bf16: r2 as 16 without dk_bias, causal B1 H50 L=4096 412 -> 399, L=8192 1448 ->
+// 1416, B2 H32 L=3000 306 -> 293; r16 B2 H4 L=8192 567 -> 555, B8 H16 L=700 100 -> 95; r32 768 x 4 rows of 768 2139 -> 2097, 301 x
+// 4 of 301 225 -> 213; r32 fp16 with a padding mask, 2 x 4 x (1000 x 3000) 170 -> 160.  Not kept: four waves without dk_bias (spills:
+// 399 -> 409).
 #pragma once
 #include "fb_lean_tiles.h"
 
 namespace fb {
 
-template <class T, int NKR_, int MASK_, bool FOLD_, bool BG_>
+template <class T, int NKD_, int NKR_, int MASK_, bool FOLD_, bool BG_>
 struct DkvMidCfg {
-    static constexpr int NKD = 4, NKR = NKR_, NK = NKD + NKR_, NDV = 2;
+    static constexpr int NKD = NKD_, NKR = NKR_, NK = NKD + NKR_, NDV = NKD / 2;
+    static_assert(NKD_ == 2 || NKD_ == 4, "");
     static constexpr bool FOLD = FOLD_, VMASK = MASK_ == kVectorMask, BG = BG_ && NKR_ > 0;
     static_assert(MASK_ != kMatrixMask && !(FOLD_ && VMASK) && NKR_ <= 2, "");
     static constexpr int MB = NDV + (BG ? 1 : 0); // 32-row blocks of [dK | dK_b]^T
     static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES, BN = 128, BMQ = 64;
     static constexpr int CPR = 2 * (NKR > 0 ? NKR : 1);
-    // a stage, bytes: Q and dO rows of 128, Q_b rows of 32 or 64, lse * log2(e) and -delta
-    static constexpr int SQ = BMQ * 128, SQB = NKR > 0 ? BMQ * CPR * 16 : 0, STAGE = 2 * SQ + SQB + 8 * BMQ, NSTAGE = 2;
+    static constexpr int ROWCH = 2 * NKD, RB = 16 * ROWCH; // chunks and bytes of a Q or dO row
+    static constexpr int NI = NKD / 2; // copy instructions per wave, tensor and step
+    // a stage, bytes: Q, dO, Q_b rows of 32 or 64, lse * log2(e) and -delta
+    static constexpr int SQ = BMQ * RB, SQB = NKR > 0 ? BMQ * CPR * 16 : 0, STAGE = 2 * SQ + SQB + 8 * BMQ, NSTAGE = 2;
     static constexpr int LDS_BYTES = NSTAGE * STAGE;
-    static_assert(2 * LDS_BYTES <= 160 * 1024, "");
+    static constexpr int WAVES_EU = NKD == 4 ? 2 : 3;
+    static_assert(WAVES_EU * LDS_BYTES <= 160 * 1024, "");
+    static constexpr bool ORDERED = NKD == 4; // two waves a SIMD: the order is fixed phase by phase
     static __device__ __forceinline__ bool low_parts(const BwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
 };
 
 template <class T, class C>
-__global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_dkv_mid_kernel(const BwdArgs a) {
+__device__ __forceinline__ void bwd_dkv_mid_body(const BwdArgs &a, int wg) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t lds0 = lds_addr_of(smem);
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -42,7 +54,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
     const int group = a.group > 1 ? a.group : 1;
     const int nbg = (a.B + group - 1) / group;
     int bgh, tile_n;
-    work_order(blockIdx.x, a.ntiles_n, a.ntiles_n * nbg * a.H, a.causal, bgh, tile_n);
+    work_order(wg, a.ntiles_n, a.ntiles_n * nbg * a.H, a.causal, bgh, tile_n);
     const int bg = bgh / a.H, h = bgh % a.H;
     const int n0 = tile_n * C::BN, wk0 = n0 + 32 * wave;
 
@@ -64,11 +76,19 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
         const int lane = tid_again & 63, c = lane & 31, g = lane >> 5;
         const int bh = b * a.H + h, key = wk0 + c;
 
-        // ---- copies: per step every wave issues sixteen rows of Q and of dO (two instructions each), the first waves Q_b, the last
-        // ones a row of the statistics.
-        const int crow = 16 * wave + (lane >> 3); // (and crow + 8, whose chunks the swizzle moves by two places)
-        const uint32_t chunk = (uint32_t)((lane & 7) ^ swz_of<8>(crow));
-        const uint64_t lanes_on[2] = {__builtin_amdgcn_ballot_w64((int)chunk * 8 < a.d), __builtin_amdgcn_ballot_w64((int)(chunk ^ 2) * 8 < a.d)};
+        // ---- copies: per step every wave issues sixteen rows of Q and of dO, the first waves Q_b, the last ones a row of the
+        // statistics.
+        int crow, cch;
+        if constexpr (C::NKD == 4) {
+            crow = 16 * wave + (lane >> 3); // (and crow + 8, whose chunks the swizzle moves by two places)
+            cch = (lane & 7) ^ swz_of<8>(crow);
+        } else {
+            lean_copy_place<4>(lane, crow, cch);
+            crow += 16 * wave;
+        }
+        uint64_t lanes_on[C::NI];
+#pragma unroll
+        for (int j = 0; j < C::NI; ++j) lanes_on[j] = __builtin_amdgcn_ballot_w64((cch ^ (2 * j)) * 8 < a.d);
         const uint32_t qpitch = (uint32_t)(a.q.ss * 2), dpitch = (uint32_t)(a.dout.ss * 2), bpitch = C::NKR > 0 ? (uint32_t)(a.qb.ss * 2) : 0u;
         const uint8_t *qbase = reinterpret_cast<const uint8_t *>(a.q.ptr + b * a.q.sb + h * a.q.sh);
         const uint8_t *dbase = reinterpret_cast<const uint8_t *>(a.dout.ptr + b * a.dout.sb + h * a.dout.sh);
@@ -84,10 +104,10 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
             const int r0 = step * C::BMQ, last = a.Lq - 1 - r0; // (a ragged last step: rows past the end are the last one again)
             const uint32_t at = lds0 + stage * C::STAGE;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const uint32_t row = (uint32_t)min(crow + 8 * j, last), ch = (chunk ^ (2u * j)) * 16;
-                lds_dma16_lanes(row * qpitch + ch, qbase + (int64_t)r0 * qpitch, at + (2 * wave + j) * 1024, lanes_on[j]);
-                lds_dma16_lanes(row * dpitch + ch, dbase + (int64_t)r0 * dpitch, at + C::SQ + (2 * wave + j) * 1024, lanes_on[j]);
+            for (int j = 0; j < C::NI; ++j) {
+                const uint32_t row = (uint32_t)min(crow + 8 * j, last), ch = (uint32_t)(cch ^ (2 * j)) * 16;
+                lds_dma16_lanes(row * qpitch + ch, qbase + (int64_t)r0 * qpitch, at + (C::NI * wave + j) * 1024, lanes_on[j]);
+                lds_dma16_lanes(row * dpitch + ch, dbase + (int64_t)r0 * dpitch, at + C::SQ + (C::NI * wave + j) * 1024, lanes_on[j]);
             }
             if (wave < QB_WAVES) lds_dma16_lanes((uint32_t)min(brow, last) * bpitch + bch * 16, bbase + (int64_t)r0 * bpitch, at + 2 * C::SQ + wave * 1024, lanes_b);
             if (wave >= 2) lds_dma4(stat + min(r0 + lane, a.Lq - 1), at + 2 * C::SQ + C::SQB + (wave & 1) * 4 * C::BMQ);
@@ -134,14 +154,14 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
             if (step + 1 < nsteps) issue(step + 1, stage ^ 1);
             const int r0 = step * C::BMQ;
             if (!(a.causal && wk0 > r0 + C::BMQ - 1) && wk0 < a.Lk) {
-                TileAddr<8> ta(lds_addr_of(st), c, g);
-                asm volatile("" : "+v"(ta.row), "+v"(ta.tr));
+                TileAddr<C::ROWCH> ta(lds_addr_of(st), c, g);
+                if constexpr (C::ORDERED) asm volatile("" : "+v"(ta.row), "+v"(ta.tr));
                 u32x4_t qa[C::NK], da[C::NKD];
                 auto rows = [&](int i) {
 #pragma unroll
                     for (int t = 0; t < C::NKD; ++t) {
-                        qa[t] = ta.load_row(t, 4096 * i);
-                        da[t] = ta.load_row(t, C::SQ + 4096 * i);
+                        qa[t] = ta.load_row(t, 32 * C::RB * i);
+                        da[t] = ta.load_row(t, C::SQ + 32 * C::RB * i);
                     }
 #pragma unroll
                     for (int t = 0; t < C::NKR; ++t)
@@ -166,9 +186,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
                 u32x4_t dot[C::NDV], qt[C::MB];
                 auto columns = [&](int i, int t) {
 #pragma unroll
-                    for (int n = 0; n < C::NDV; ++n) dot[n] = ta.load_tr(n, C::SQ + 4096 * i + 16 * 128 * t);
+                    for (int n = 0; n < C::NDV; ++n) dot[n] = ta.load_tr(n, C::SQ + 32 * C::RB * i + 16 * C::RB * t);
 #pragma unroll
-                    for (int n = 0; n < C::NDV; ++n) qt[n] = ta.load_tr(n, 4096 * i + 16 * 128 * t);
+                    for (int n = 0; n < C::NDV; ++n) qt[n] = ta.load_tr(n, 32 * C::RB * i + 16 * C::RB * t);
                     if constexpr (C::BG) qt[C::NDV] = dense_read_a_tr<C::CPR>(st + 2 * C::SQ, 32 * i + 16 * t, c, g);
                 };
                 u32x4_t pp[2], pds[2];
@@ -182,7 +202,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
                 constexpr int NSUM = C::NDV + C::MB;
                 rows(0);
                 deltas(0);
-                FB_HOLD;
+                if constexpr (C::ORDERED) FB_HOLD;
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
                     const int q0 = r0 + 32 * i;
@@ -199,8 +219,10 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
                     for (int t = 0; t < C::NKR; ++t) fac[t] = qa[C::NKD + t];
                     columns(i, 0);
                     lses(i);
-                    mix<8, 2, 0>();
-                    FB_HOLD;
+                    if constexpr (C::ORDERED) {
+                        mix<2 * C::NKD, 2, 0>();
+                        FB_HOLD;
+                    }
                     // the softmax scale multiplies the fp32 q k^T accumulator before the bias steps
                     if constexpr (!C::FOLD) {
 #pragma unroll
@@ -208,7 +230,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
                     }
 #pragma unroll
                     for (int t = 0; t < C::NKR; ++t) s = T::mfma(fac[t], kr[C::NKD + t], s);
-                    FB_HOLD;
+                    if constexpr (C::ORDERED) FB_HOLD;
                     // (bitwise on purpose, as in the dq kernel: no scalar block between the last MFMA and the branch)
                     const bool edge = (wk0 + 32 > a.Lk) | (q0 + 32 > a.Lq) | ((a.causal != 0) & (wk0 + 31 > q0));
                     if (edge) {
@@ -223,7 +245,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
                     asm volatile("s_nop 11" : "+v"(s)); // (fb_bwd_win.hip: wait states across the branch above)
                     if (i == 0) {
                         rows(1);
-                        FB_HOLD;
+                        if constexpr (C::ORDERED) FB_HOLD;
                     }
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
@@ -236,16 +258,20 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
                             pds[j >> 1][2 * (j & 1) + e] = T::pack2(p[2 * e] * dp[4 * j + 2 * e], p[2 * e + 1] * dp[4 * j + 2 * e + 1]);
                         }
                     }
-                    FB_HOLD;
+                    if constexpr (C::ORDERED) FB_HOLD;
                     // ---- dV^T += dO^T P, [dK | dK_b]^T += [Q | Q_b]^T dS
                     sums(0);
                     columns(i, 1);
-                    mix<NSUM, 2, 0>();
-                    FB_HOLD;
+                    if constexpr (C::ORDERED) {
+                        mix<NSUM, 2, 0>();
+                        FB_HOLD;
+                    }
                     sums(1);
                     if (i == 0) deltas(1);
-                    mix<NSUM, 1, 0>();
-                    FB_HOLD;
+                    if constexpr (C::ORDERED) {
+                        mix<NSUM, 1, 0>();
+                        FB_HOLD;
+                    }
                 }
             }
             wait_vmcnt<0>(); // the next step has landed
@@ -273,9 +299,14 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
     }
 }
 
-template <class T, int NKR, int MASK, bool FOLD, bool BG>
+template <class T, class C>
+__global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::WAVES_EU, C::WAVES_EU))) void bwd_dkv_mid_kernel(const BwdArgs a) {
+    bwd_dkv_mid_body<T, C>(a, blockIdx.x);
+}
+
+template <class T, int NKD, int NKR, int MASK, bool FOLD, bool BG>
 static hipError_t launch_dkv_mid_bg(const BwdArgs &a0, hipStream_t stream) {
-    typedef DkvMidCfg<T, NKR, MASK, FOLD, BG> C;
+    typedef DkvMidCfg<T, NKD, NKR, MASK, FOLD, BG> C;
     BwdArgs a = a0;
     a.ntiles_n = (a.Lk + C::BN - 1) / C::BN;
     auto kern = bwd_dkv_mid_kernel<T, C>;
@@ -287,12 +318,12 @@ static hipError_t launch_dkv_mid_bg(const BwdArgs &a0, hipStream_t stream) {
 }
 
 // (no dk_bias wanted: without its products)
-template <class T, int NKR, int MASK, bool FOLD>
+template <class T, int NKD, int NKR, int MASK, bool FOLD>
 static hipError_t launch_dkv_mid(const BwdArgs &a, hipStream_t stream) {
     if constexpr (NKR > 0) {
-        if (a.dkb.ptr) return launch_dkv_mid_bg<T, NKR, MASK, FOLD, true>(a, stream);
+        if (a.dkb.ptr) return launch_dkv_mid_bg<T, NKD, NKR, MASK, FOLD, true>(a, stream);
     }
-    return launch_dkv_mid_bg<T, NKR, MASK, FOLD, false>(a, stream);
+    return launch_dkv_mid_bg<T, NKD, NKR, MASK, FOLD, false>(a, stream);
 }
 
 } // namespace fb

@@ -27,10 +27,7 @@ namespace fb {
 // score for the scale (the launcher says when that is exact).
 // SPLIT_: K_b in a dense region of its own instead of the upper chunks of a padded K row (head dims above 64, aligned,
 // unmasked, rank <= 32: 16 + 2 or 4 chunks against 32), so that 64-key tiles in two stages fit two workgroups per CU.
-// BG_: also accumulate dq_bias (false: the caller does not want the factor gradients; the accumulator blocks that
-// hold nothing but dq_bias are then left out of the products).
-template <class T, int NKD_, int NKR_, bool VEC_, int MASK_, bool QB2_ = true, bool FOLD_ = false, bool SPLIT_ = false,
-          bool BG_ = true>
+template <class T, int NKD_, int NKR_, bool VEC_, int MASK_, bool QB2_ = true, bool FOLD_ = false, bool SPLIT_ = false>
 struct DqCfg {
     static constexpr bool FOLD = FOLD_;
     // A vector mask is one fp32 value per key: its instantiations (VMASK) are the unmasked ones otherwise; XMASK is every
@@ -48,7 +45,6 @@ struct DqCfg {
     static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES;
     static constexpr int NK = NKD + NKR;
     static constexpr int MB = (NK + 1) / 2; // 32-row blocks of [dQ | dQ_b]^T
-    static constexpr int MBE = BG_ ? MB : (NKD + 1) / 2; // ... of which the key loop accumulates the first MBE
     static constexpr int QBLK = (QB2_ && NK <= 3 && !XMASK) ? 2 : 1; // the mask values need the registers of the second block
     static constexpr int BM = NWAVES * QBLK * 32;
     static constexpr int KBLK = 2, BN = 32 * KBLK;
@@ -585,7 +581,7 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
-                    for (int n = 0; n < C::MBE; ++n) {
+                    for (int n = 0; n < C::MB; ++n) {
                         u32x4_t kt;
                         if (C::SKB > 0 && 2 * n >= C::NKD)
                             kt = dense_read_a_tr<C::CPR>(sKb, kb * 32 + 16 * t, c, g);

@@ -39,7 +39,7 @@ struct DqMidCfg {
 };
 
 template <class T, class C>
-__global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::WAVES_EU, C::WAVES_EU))) void bwd_dq_mid_kernel(const BwdArgs a) {
+__device__ __forceinline__ void bwd_dq_mid_body(const BwdArgs &a, int wg) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t lds0 = lds_addr_of(smem);
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -48,7 +48,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     const int group = a.group > 1 ? a.group : 1;
     const int nbg = (a.B + group - 1) / group;
     int bgh, tile_m;
-    work_order(blockIdx.x, a.ntiles_m, a.ntiles_m * nbg * a.H, a.causal, bgh, tile_m);
+    work_order(wg, a.ntiles_m, a.ntiles_m * nbg * a.H, a.causal, bgh, tile_m);
     if (a.causal) tile_m = a.ntiles_m - 1 - tile_m; // the last query tile sees the most keys
     const int bg = bgh / a.H, h = bgh % a.H;
     const int m0 = tile_m * C::BM, wq0 = m0 + 32 * wave;
@@ -257,6 +257,11 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         uint16_t *row = const_cast<uint16_t *>(a.dqb.ptr) + bg * a.dqb.sb + h * a.dqb.sh + (int64_t)(ok ? q : 0) * a.dqb.ss;
         store_acc_rows<T, true>(row, ok, a.dqb.vec_ok, acc_b, 1.f, a.r, lane >> 5);
     }
+}
+
+template <class T, class C>
+__global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::WAVES_EU, C::WAVES_EU))) void bwd_dq_mid_kernel(const BwdArgs a) {
+    bwd_dq_mid_body<T, C>(a, blockIdx.x);
 }
 
 template <class T, int NKD, int NKR, bool FOLD, bool BG>

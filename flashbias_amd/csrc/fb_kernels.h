@@ -121,12 +121,13 @@ inline bool mixed_backward(const BwdArgs &a0) {
     return ndq % 8 == 0 && ndkv % 8 == 0 && ndq <= num_cus() && ndkv <= num_cus();
 }
 
-// The same question for the general dq and dk/dv kernels of head dim 32 with factors (launch_both_general in
-// fb_bwd_both.hip): both kernels would run their aligned, unmasked 128-row instantiations with the same folding of
-// the scale, the counts of both kinds split evenly over the eight XCDs, and the grid is small: at most one
-// workgroup per compute unit and kind, or, under a causal mask, at most one and a half per workgroup slot (three
-// slots per compute unit), where a launch's length is that of its longest workgroup and the two kinds fill each
-// other's tails.  Declared after fold_scale_ok below.
+// The same question for the dq and dk/dv bodies of head dim 32 with factors that are not the streamlined ones (launch_both_general in
+// fb_bwd_both.hip): aligned, no mask, the same folding of the scale in both, the counts of both kinds split evenly over the
+// eight XCDs, and the grid is small: at most one and a half workgroups per compute unit and kind (training step, two launches / one,
+// us: r16 B2 H4 L=4096 201 / 169, L=5000 355 / 318, r32 B2 H8 L=3000 239 / 218; two of a kind: r16 L=8192 548 / 562, r32 B4 H8 L=2048 162 /
+// 170), or, under a causal mask, at most one and a half per workgroup slot (three slots per compute unit), where a launch's
+// length is that of its longest workgroup and the two kinds fill each other's tails (r2 as 16 B1 H16 L=4096 199 / 170, r16 B1 H24 L=4096
+// 254 / 232, r2 B1 H50 L=2048 138 / 137, L=3000 254 / 250, L=4096 404 / 417).  Declared after fold_scale_ok below.
 template <class T>
 inline bool mixed_general_backward(const BwdArgs &a0);
 
@@ -273,7 +274,7 @@ inline bool mixed_general_backward(const BwdArgs &a0) {
     const int64_t ndq = units * ((a.Lq + 127) / 128), ndkv = units * ((a.Lk + 127) / 128);
     if (ndq % 8 != 0 || ndkv % 8 != 0) return false;
     const int64_t most = ndq > ndkv ? ndq : ndkv;
-    return most <= num_cus() || (a.causal && 2 * most <= 9 * (int64_t)num_cus());
+    return 2 * most <= (a.causal ? 9 : 3) * (int64_t)num_cus();
 }
 
 } // namespace fb

@@ -671,7 +671,8 @@ def test_backward_phases_through_the_c_abi(gpu_device):
     (torch.bfloat16, 1, 4, 640, 700, 0, False),
     # the general kernels (ranks 16 ... 32): small grids, and causal grids of up to 1.5 workgroups per slot and kind
     (torch.bfloat16, 1, 48, 2048, 2048, 16, True), (torch.float16, 2, 4, 1024, 1024, 16, False),
-    (torch.bfloat16, 2, 8, 700, 1500, 32, True), (torch.float16, 1, 8, 1024, 1000, 24, False)])
+    (torch.bfloat16, 2, 8, 700, 1500, 32, True), (torch.float16, 1, 8, 1024, 1000, 24, False),
+    (torch.bfloat16, 6, 8, 1000, 900, 16, False)])  # (one and a half workgroups per compute unit and kind)
 def test_small_grid_backward_in_one_launch(gpu_device, dtype, B, H, Lq, Lk, r, causal):
     """On grids that give neither backward kernel more than one workgroup per compute unit (with factors of rank 16
     and more under a causal mask: up to one and a half per workgroup slot) fb_bwd runs

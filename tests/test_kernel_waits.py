@@ -56,7 +56,7 @@ def test_every_path_counts():
 
 @pytest.mark.skipif(shutil.which("hipcc") is None or shutil.which("make") is None, reason="needs hipcc and make")
 def test_compiled_kernels():
-    units = [f"build/asm/fb_{unit}.s" for unit in ("bwd_dkv_bf16_8", "bwd_dkv_bf16_4", "bwd_win_bf16_2", "bwd_dq_bf16_8", "fwd_bf16_8", "fwd_bf16_2", "bwd_dq_bf16_2", "bwd_dq_bf16_4")]
+    units = [f"build/asm/fb_{unit}.s" for unit in ("bwd_dkv_bf16_8", "bwd_dkv_bf16_4", "bwd_both_bf16_2", "bwd_win_bf16_2", "bwd_dq_bf16_8", "fwd_bf16_8", "fwd_bf16_2", "bwd_dq_bf16_2", "bwd_dq_bf16_4")]
     subprocess.run(["make", "-j4"] + units, cwd=CSRC, check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
     for unit in units:
         with open(os.path.join(CSRC, unit)) as f:
