@@ -14,7 +14,7 @@ FB_MASK_NONE, FB_MASK_VECTOR, FB_MASK_MATRIX = 0, 1, 2
 
 #: every symbol that include/flashbias.h declares
 EXPORTS = ("fb_version", "fb_init", "fb_last_error", "fb_bwd_workspace_bytes", "fb_suggest_bias_grad_group", "fb_check", "fb_fwd", "fb_bwd",
-           "fb_sum_over_batch", "fb_resize_rank", "fb_alibi_factors", "fb_cosine_workspace_bytes", "fb_cosine_fwd", "fb_cosine_bwd",
+           "fb_sum_over_batch", "fb_resize_rank", "fb_resize_ranks", "fb_alibi_factors", "fb_cosine_workspace_bytes", "fb_cosine_fwd", "fb_cosine_bwd",
            "fb_weight_grad_workspace_bytes", "fb_weight_grad_recommended", "fb_weight_grad",
            "fb_project_recommended", "fb_project",
            "fb_bwd_preprocess", "fb_bwd_dkv", "fb_bwd_dq", "fb_bwd_static")
@@ -79,6 +79,9 @@ def load():
     lib.fb_sum_over_batch.restype = ctypes.c_int
     lib.fb_resize_rank.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
     lib.fb_resize_rank.restype = ctypes.c_int
+    lib.fb_resize_ranks.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64,
+                                    ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+    lib.fb_resize_ranks.restype = ctypes.c_int
     lib.fb_weight_grad_workspace_bytes.argtypes = [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int]
     lib.fb_weight_grad_workspace_bytes.restype = ctypes.c_size_t
     lib.fb_weight_grad_recommended.argtypes = [ctypes.c_int64, ctypes.c_int, ctypes.c_int]

@@ -261,7 +261,17 @@ int fb_resize_rank(const void *in, void *out, int64_t rows, int r_in, int r_out,
     if (!in || !out) return fb::api_fail(FB_ERR_NULL, "fb_resize_rank: null pointer");
     if (rows <= 0 || r_in <= 0 || r_out <= 0 || r_in > 4096 || r_out > 4096 || (rows + 255) / 256 > 0x7fffffff)
         return fb::api_fail(FB_ERR_SHAPE, "fb_resize_rank: rows and both ranks must be positive (ranks up to 4096, rows below 2^39)");
-    return launched(fb::launch_resize_rank(in, out, rows, r_in, r_out, static_cast<hipStream_t>(stream)), "fb_resize_rank");
+    return launched(fb::launch_resize_rank(in, out, rows, nullptr, nullptr, 0, r_in, r_out, static_cast<hipStream_t>(stream)), "fb_resize_rank");
+}
+
+int fb_resize_ranks(const void *q_in, void *q_out, int64_t q_rows, const void *k_in, void *k_out, int64_t k_rows, int r_in, int r_out,
+                    void *stream) {
+    fb::api_clear_error();
+    if (!q_in || !q_out || !k_in || !k_out) return fb::api_fail(FB_ERR_NULL, "fb_resize_ranks: null pointer");
+    if (q_rows <= 0 || k_rows <= 0 || r_in <= 0 || r_out <= 0 || r_in > 4096 || r_out > 4096 || (q_rows + 255) / 256 > 0x3fffffff ||
+        (k_rows + 255) / 256 > 0x3fffffff)
+        return fb::api_fail(FB_ERR_SHAPE, "fb_resize_ranks: rows and both ranks must be positive (ranks up to 4096, rows below 2^38)");
+    return launched(fb::launch_resize_rank(q_in, q_out, q_rows, k_in, k_out, k_rows, r_in, r_out, static_cast<hipStream_t>(stream)), "fb_resize_ranks");
 }
 
 int fb_alibi_factors(void *q_bias, void *k_bias, int dtype, int Lq, int Lk, int H, int r, int reference_sign, void *stream) {

@@ -174,9 +174,20 @@ hipError_t launch_sum_over_batch(const void *full, void *out, bool bf16, bool ou
     return hipGetLastError();
 }
 
-// out[row][c] = c < min(r_in, r_out) ? in[row][c] : 0 for contiguous rows of 16-bit elements: one thread per row.
-__global__ __launch_bounds__(256) void resize_rank_kernel(const uint16_t *in, uint16_t *out, int64_t rows, int r_in, int r_out) {
-    const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
+// out[row][c] = c < min(r_in, r_out) ? in[row][c] : 0 for contiguous rows of 16-bit elements: one thread per row.  The
+// first `blocks` workgroups take the rows of `in`, the rest those of `in2`: both factors of a call in one launch, whose
+// start, end and way through the host cost more than the bytes (rank 2 to 16: a causal forward of 8 heads of 512 positions
+// 21.8 us with two launches and 15.6 with one, a training step of 50 heads of 4096 positions 390 and 386).
+__global__ __launch_bounds__(256) void resize_rank_kernel(const uint16_t *in, uint16_t *out, int64_t rows, unsigned blocks, const uint16_t *in2,
+                                                          uint16_t *out2, int64_t rows2, int r_in, int r_out) {
+    unsigned block = blockIdx.x;
+    if (block >= blocks) {
+        block -= blocks;
+        in = in2;
+        out = out2;
+        rows = rows2;
+    }
+    const int64_t row = (int64_t)block * 256 + threadIdx.x;
     if (row >= rows) return;
     const uint16_t *src = in + row * r_in;
     uint16_t *dst = out + row * r_out;
@@ -196,10 +207,12 @@ __global__ __launch_bounds__(256) void resize_rank_kernel(const uint16_t *in, ui
     for (int c = 0; c < r_out; ++c) dst[c] = c < keep ? src[c] : (uint16_t)0;
 }
 
-hipError_t launch_resize_rank(const void *in, void *out, int64_t rows, int r_in, int r_out, hipStream_t stream) {
+hipError_t launch_resize_rank(const void *in, void *out, int64_t rows, const void *in2, void *out2, int64_t rows2, int r_in, int r_out,
+                              hipStream_t stream) {
     (void)hipGetLastError();
-    hipLaunchKernelGGL(resize_rank_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, stream,
-                       static_cast<const uint16_t *>(in), static_cast<uint16_t *>(out), rows, r_in, r_out);
+    const unsigned blocks = (unsigned)((rows + 255) / 256), blocks2 = (unsigned)((rows2 + 255) / 256);
+    hipLaunchKernelGGL(resize_rank_kernel, dim3(blocks + blocks2), dim3(256), 0, stream, static_cast<const uint16_t *>(in), static_cast<uint16_t *>(out),
+                       rows, blocks, static_cast<const uint16_t *>(in2), static_cast<uint16_t *>(out2), rows2, r_in, r_out);
     return hipGetLastError();
 }
 

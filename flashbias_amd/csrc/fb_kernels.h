@@ -49,8 +49,10 @@ hipError_t launch_bwd_dq(const BwdArgs &a, bool bf16, hipStream_t stream);
 hipError_t launch_sum_over_batch(const void *full, void *out, bool bf16, bool out_f32, int64_t B, int64_t n, int64_t sb,
                                  hipStream_t stream);
 
-// out[row][c] = c < min(r_in, r_out) ? in[row][c] : 0: contiguous rows of 16-bit elements.
-hipError_t launch_resize_rank(const void *in, void *out, int64_t rows, int r_in, int r_out, hipStream_t stream);
+// out[row][c] = c < min(r_in, r_out) ? in[row][c] : 0: contiguous rows of 16-bit elements, and the same of a second
+// tensor (rows2 may be 0).  At most 0x7fffffff workgroups of 256 rows in all.
+hipError_t launch_resize_rank(const void *in, void *out, int64_t rows, const void *in2, void *out2, int64_t rows2, int r_in, int r_out,
+                              hipStream_t stream);
 
 // The exact rank-4 ALiBi factors, zero-padded to r columns (include/flashbias.h).
 hipError_t launch_alibi_factors(void *q_bias, void *k_bias, bool bf16, int Lq, int Lk, int H, int r, bool reference_sign, hipStream_t stream);

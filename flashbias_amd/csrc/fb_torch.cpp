@@ -468,6 +468,35 @@ struct ResizeRankFn : public torch::autograd::Function<ResizeRankFn> {
 
 Tensor resize_rank(const Tensor &x, int64_t rank) { return ResizeRankFn::apply(x, rank); }
 
+// An input that a derivative is wanted of.  A forward-mode tangent counts: tensors that carry one need not require a
+// gradient, and may do so with gradients off.
+bool differentiated(const Tensor &x) {
+    return x.defined() && ((c10::GradMode::is_enabled() && x.requires_grad()) || x._fw_grad(/*level=*/0).defined());
+}
+
+// Both factors of a call (contiguous 16-bit GPU tensors of one rank) resized: in one launch where neither asks for a
+// gradient and both are on one device (constant factors: ALiBi on every call), by one autograd node each otherwise.
+std::pair<Tensor, Tensor> resize_ranks(const Tensor &q_bias, const Tensor &k_bias, int64_t rank) {
+    if (differentiated(q_bias) || differentiated(k_bias) || q_bias.device() != k_bias.device() || q_bias.scalar_type() != k_bias.scalar_type())
+        return {ResizeRankFn::apply(q_bias, rank), ResizeRankFn::apply(k_bias, rank)};
+    if (const auto &transforms = at::functorch::functorchTLSAccessor()) transforms->checkSupportsCppAutogradFunction();
+    Tensor out[2];
+    const Tensor *const in[2] = {&q_bias, &k_bias};
+    for (int i = 0; i < 2; ++i) {
+        const Tensor &x = *in[i];
+        TORCH_CHECK(x.is_cuda() && x.is_contiguous() && x.element_size() == 2 && x.dim() >= 1 && x.numel() > 0 && rank > 0 &&
+                        x.size(-1) == q_bias.size(-1),
+                    "resize_ranks wants contiguous fp16 / bf16 GPU tensors of one rank");
+        auto shape = x.sizes().vec();
+        shape.back() = rank;
+        out[i] = fresh(shape, x.scalar_type(), x.device());
+    }
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(q_bias.device());
+    check(fb_resize_ranks(q_bias.data_ptr(), out[0].data_ptr(), out[0].numel() / rank, k_bias.data_ptr(), out[1].data_ptr(),
+                          out[1].numel() / rank, (int)q_bias.size(-1), (int)rank, stream_of(q_bias)));
+    return {out[0], out[1]};
+}
+
 Tensor flash_bias(const Tensor &q_in, const Tensor &k_in, const Tensor &v_in, const c10::optional<Tensor> &q_bias,
                   const c10::optional<Tensor> &k_bias, const c10::optional<Tensor> &mask, bool causal, double softmax_scale) {
     const Tensor q = channel_contiguous(q_in), k = channel_contiguous(k_in), v = channel_contiguous(v_in);
@@ -477,8 +506,6 @@ Tensor flash_bias(const Tensor &q_in, const Tensor &k_in, const Tensor &v_in, co
     // Nothing to differentiate: no graph node either.  What the autograd function refuses stays refused: inputs that
     // carry a forward-mode tangent (they need not require a gradient, and may do so with gradients off; without the
     // refusal their derivative would come out as zero) and calls under a function transform (torch.func).
-    const bool grad_mode = c10::GradMode::is_enabled();
-    auto differentiated = [&](const Tensor &x) { return x.defined() && ((grad_mode && x.requires_grad()) || x._fw_grad(/*level=*/0).defined()); };
     if (!(differentiated(q) || differentiated(k) || differentiated(v) || differentiated(qb) || differentiated(kb) || differentiated(m))) {
         if (const auto &transforms = at::functorch::functorchTLSAccessor()) transforms->checkSupportsCppAutogradFunction();
         return attend(Call{q, k, v, qb, kb, m, causal, scale, 0}).first;
@@ -517,6 +544,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("linear", &linear, py::arg("x"), py::arg("weight"), py::arg("bias"));
     m.def("project", &project, py::arg("x"), py::arg("weights"));
     m.def("resize_rank", &resize_rank, py::arg("x"), py::arg("rank"));
+    m.def("resize_ranks", &resize_ranks, py::arg("q_bias"), py::arg("k_bias"), py::arg("rank"));
     m.def("flash_bias", &flash_bias, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("q_bias") = py::none(),
           py::arg("k_bias") = py::none(), py::arg("mask") = py::none(), py::arg("causal") = false,
           py::arg("softmax_scale") = 0.0);

@@ -85,14 +85,16 @@ def _fold_vector_mask(q, q_bias, k_bias, mask):
     return q_new, k_new
 
 
-def _resize_rank(x, rank):
-    """`x` (..., r) with its last dim zero-padded to `rank`: one launch of the library (fb_resize_rank, through the
-    C++ extension's autograd function) for contiguous 16-bit GPU tensors, the tensor library's pad otherwise (a
-    permuted view keeps its permuted layout there)."""
+def _resize_ranks(q_bias, k_bias, rank):
+    """Both factors (..., r) with their last dim zero-padded to `rank`: by the library (fb_resize_rank through the C++
+    extension's autograd function, one launch for both where neither wants a gradient) for contiguous 16-bit GPU
+    tensors, by the tensor library's pad otherwise (a permuted view keeps its permuted layout there)."""
     ext = _extension()
-    if ext is not None and x.is_cuda and x.is_contiguous() and x.element_size() == 2 and x.numel() > 0:
-        return ext.resize_rank(x, rank)
-    return torch.nn.functional.pad(x, (0, rank - x.shape[-1]))
+    direct = [ext is not None and x.is_cuda and x.is_contiguous() and x.element_size() == 2 and x.numel() > 0 for x in (q_bias, k_bias)]
+    if all(direct):
+        return ext.resize_ranks(q_bias, k_bias, rank)
+    return tuple(ext.resize_rank(x, rank) if d else torch.nn.functional.pad(x, (0, rank - x.shape[-1]))
+                 for x, d in zip((q_bias, k_bias), direct))
 
 
 def _prepare_factors(q, k, q_bias, k_bias, mask):
@@ -125,7 +127,7 @@ def _prepare_factors(q, k, q_bias, k_bias, mask):
             # over points in a unit box) opts in to rank 8 by padding them itself, once
             # (factors.pad_rank): the choice depends on nothing but the shapes it passes.
             target = 16 if rank < 8 else -(-rank // 8) * 8
-            q_bias, k_bias = _resize_rank(q_bias, target), _resize_rank(k_bias, target)
+            q_bias, k_bias = _resize_ranks(q_bias, k_bias, target)
         # (padding a permuted view keeps its permuted layout)
         q_bias, k_bias = _last_dim_contiguous(q_bias), _last_dim_contiguous(k_bias)
     if mask is not None:

@@ -197,6 +197,10 @@ int fb_sum_over_batch(const void *full, void *out, int dtype, int out_dtype, int
  * of two of at least 16, with masked loads: flash_bias_triton.py:1137, :195-200). */
 int fb_resize_rank(const void *in, void *out, int64_t rows, int r_in, int r_out, void *stream);
 
+/* The same of two tensors of one rank, the two factors of a call, in one launch. */
+int fb_resize_ranks(const void *q_in, void *q_out, int64_t q_rows, const void *k_in, void *k_out, int64_t k_rows,
+                    int r_in, int r_out, void *stream);
+
 /* The exact ALiBi bias -m_h (i - j) as factors of rank 4, zero-padded to `r` columns (positions below 65536 in two
  * 8-bit digits, i = 256 a + b, so that every column is a whole number or a slope in 16 bits):
  *     q_bias[i] = [a_i, b_i, 256 m, m, 0 ...],   k_bias[j] = [-256 m, -m, a_j, b_j, 0 ...],

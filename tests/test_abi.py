@@ -217,6 +217,17 @@ def test_resize_rank_rejects(args, code):
     assert lib.fb_last_error() != b""
 
 
+@pytest.mark.parametrize("args,code", [
+    ((None, 0x2000, 10, 2, 16), -1), ((0x1000, None, 10, 2, 16), -1),
+    ((0x1000, 0x2000, 0, 2, 16), -2), ((0x1000, 0x2000, 10, 0, 16), -2), ((0x1000, 0x2000, 1 << 38, 2, 16), -2),
+])
+def test_resize_ranks_rejects(args, code):
+    lib = _lib.load()
+    other = (0x3000, 0x4000, 10)
+    assert lib.fb_resize_ranks(*args[:3], *other, *args[3:], None) == code
+    assert lib.fb_resize_ranks(*other, *args[:3], *args[3:], None) == code
+
+
 def test_null_params():
     lib = _lib.load()
     assert lib.fb_check(None, 0) == -1

@@ -1057,6 +1057,31 @@ def test_resize_rank(gpu_device, dtype, rows, r_in, r_out):
         assert torch.isnan(buf[offset + rows * r_out:].float()).all() and torch.isnan(buf[:offset].float()).all()
 
 
+@pytest.mark.parametrize("rows_q,rows_k,r_in,r_out", [(1000, 777, 2, 16), (256, 257, 2, 16), (1, 512, 5, 8), (255, 1, 16, 2), (64, 300, 20, 24)])
+def test_both_ranks_resized_in_one_launch(gpu_device, rows_q, rows_k, r_in, r_out):
+    """fb_resize_ranks at the edges of the two tensors' workgroups of 256 rows: the bits of two calls, nothing beyond
+    either output; the extension's entry gives the same with and without a gradient to carry."""
+    from flashbias_amd import _lib
+    from flashbias_amd.interface import _extension, _stream
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(6)
+    x = [torch.randn(n, r_in, generator=g).to(torch.bfloat16).to(gpu_device) for n in (rows_q, rows_k)]
+    keep = min(r_in, r_out)
+    want = [torch.nn.functional.pad(t[:, :keep], (0, r_out - keep)) for t in x]
+    buf = [torch.full((n * r_out + 16,), float("nan"), dtype=torch.bfloat16, device=gpu_device) for n in (rows_q, rows_k)]
+    out = [b[8:8 + n * r_out].view(n, r_out) for b, n in zip(buf, (rows_q, rows_k))]
+    _lib.check_status(lib.fb_resize_ranks(x[0].data_ptr(), out[0].data_ptr(), rows_q, x[1].data_ptr(), out[1].data_ptr(), rows_k,
+                                          r_in, r_out, _stream()))
+    torch.cuda.synchronize()
+    for t, w, b in zip(out, want, buf):
+        assert torch.equal(t, w) and torch.isnan(b[:8].float()).all() and torch.isnan(b[8 + w.numel():].float()).all()
+    for grads in ((False, False), (False, True), (True, True)):
+        leaves = [t.clone().requires_grad_(n) for t, n in zip(x, grads)]
+        got = _extension().resize_ranks(*leaves, r_out)
+        assert [t.requires_grad for t in got] == list(grads)
+        assert all(torch.equal(t, w) for t, w in zip(got, want))
+
+
 def test_rank_padding_inside_the_operator(gpu_device):
     """Factors of rank 5 through flash_bias_func (padded per call by the library's kernel, their gradients cut
     back by it) against the same factors padded by the tensor library beforehand: same bits."""
