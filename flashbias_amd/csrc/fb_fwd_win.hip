@@ -5,23 +5,27 @@
 //
 // The general kernel gives a window a workgroup that holds half of the compute unit's registers, and spends its life in
 // turn on the first tile's way from memory, eight 32-key blocks and the stores.  Here a window's K, K_b and V take 40 KB, a
-// wave works on one block of 32 queries at a time in 128 registers, and four workgroups (mask: three) share a
-// compute unit: nothing is pipelined by hand, whatever one waits for the others fill.
+// wave works on one block of 32 queries at a time in 128 registers, and four workgroups of four waves (mask: three) or two of
+// eight share a compute unit: nothing is pipelined by hand, whatever one waits for the others fill.
 #include "fb_kernels.h"
 #include "fb_lean_tiles.h"
 
 namespace fb {
 
 // FOLD_: the scores are scale * (q k^T + q_b k_b^T) in one chain (no factors, or a scale of exactly 1).
-// MASK_: a matrix mask, whose 32 x 32 blocks the wave that uses them copies to LDS one ahead.
-template <class T, int NKR_, bool FOLD_, bool MASK_>
+// MASK_: a matrix mask, whose blocks the wave that uses them copies to LDS one ahead.
+// NWAVES_: 4, or 8 for small grids of windows of more than 128 queries (launch_fwd_win_waves).
+template <class T, int NKR_, bool FOLD_, bool MASK_, int NWAVES_>
 struct FwdWinCfg {
     static constexpr bool FOLD = FOLD_, MASK = MASK_;
     static constexpr int NKD = 2, NKR = NKR_, NK = NKD + NKR_;
-    static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES, LK = 256;
-    static constexpr int K = 0, V = K + LK * 64, KB = V + LK * 64, MT = KB + (NKR ? LK * 32 : 0), LDS_BYTES = MT + (MASK ? NWAVES * 2048 : 0);
-    static constexpr int WAVES_EU = MASK ? 3 : 4;
-    static_assert(WAVES_EU * LDS_BYTES <= 160 * 1024, "");
+    static constexpr int NWAVES = NWAVES_, NTHREADS = 64 * NWAVES, LK = 256;
+    static constexpr bool PAIR = !MASK || NWAVES == 8; // two blocks of 32 keys at a time
+    static constexpr int TILE = PAIR ? 4096 : 2048;    // a wave's mask tile: 32 queries x 64 or 32 keys
+    static constexpr int K = 0, V = K + LK * 64, KB = V + LK * 64, MT = KB + (NKR ? LK * 32 : 0), LDS_BYTES = MT + (MASK ? NWAVES * TILE : 0);
+    static constexpr int WAVES_EU = PAIR ? 4 : 3;
+    static_assert(NWAVES == 4 || NWAVES == 8, "");
+    static_assert(WAVES_EU * 4 / NWAVES * LDS_BYTES <= 160 * 1024, "");
 };
 
 template <class T, class C>
@@ -42,10 +46,17 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         __syncthreads();
     }
     const float to_log2 = C::FOLD ? a.scale * kLog2e : kLog2e, lag = 8.f / to_log2;
-    const uint32_t row_off[2] = {lds0 + lean_row_addr<4>(c, g), lds0 + lean_row_addr<4>(c, 2 + g)};
-    const uint32_t col_off[2] = {lds0 + C::V + lean_tr_addr4(c, g, 0), lds0 + C::V + lean_tr_addr4(c, g, 1)};
-    const uint32_t kb_row = lds0 + C::KB + lean_row_addr<2>(c, g);
-    const uint32_t lds_m = lds0 + C::MT + wave * 2048;
+    // With a mask a row of [K | K_b] stands for the key whose bits 2 and 3 are swapped: register v of a lane is then key 16 (v / 8) + 8 g +
+    // v % 8, and its mask values come in chunks of 16 bytes.
+    const int krow = C::MASK ? (c & 19) | ((c & 4) << 1) | ((c & 8) >> 1) : c;
+    const uint32_t row_off[2] = {lds0 + lean_row_addr<4>(krow, g), lds0 + lean_row_addr<4>(krow, 2 + g)};
+    const uint32_t kb_row = lds0 + C::KB + lean_row_addr<2>(krow, g);
+    auto col_at = [&](int hi) { // (lean_tr_addr4, in that order of the keys)
+        if constexpr (C::MASK) return lean_chunk_off<4>(8 * g + ((c & 15) >> 2) + 4 * hi, 2 * (c >> 4) + ((c & 3) >> 1)) + 8 * (c & 1);
+        return lean_tr_addr4(c, g, hi);
+    };
+    const uint32_t col_off[2] = {lds0 + C::V + col_at(0), lds0 + C::V + col_at(1)};
+    const uint32_t lds_m = lds0 + C::MT + wave * C::TILE;
 
     for (int bi = 0; bi < walk; ++bi) {
         const int b = __builtin_amdgcn_readfirstlane(bg * walk + bi);
@@ -56,7 +67,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             int row, chunk;
             lean_copy_place<4>(lane, row, chunk);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < C::LK / 16 / C::NWAVES; ++j) {
                 const int i = wave + C::NWAVES * j, r = min(16 * i + row, a.Lk - 1);
                 if (i < 2 * nkb) {
                     lds_dma16_all((uint32_t)(r * (int)(a.k.ss * 2) + chunk * 16), kbase, lds0 + C::K + i * 1024);
@@ -65,11 +76,12 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             }
             if constexpr (C::NKR > 0) {
                 if (bi == 0 || a.kb.sb != 0) {
-                    DenseCopy<C::LK / 2, 2> cb;
+                    constexpr int ROWS = 32 * C::NWAVES; // a copy instruction of each wave
+                    DenseCopy<ROWS, 2> cb;
                     cb.init(a.kb.ptr + b * a.kb.sb + h * a.kb.sh, a.kb.ss, a.r, false, wave, lane, 0);
                     cb.issue(lds0 + C::KB, 0, a.Lk);
                     // (only where it has rows: the copy's offsets count down from the half's first row, unsigned)
-                    if (a.Lk > C::LK / 2) cb.issue(lds0 + C::KB + C::LK * 16, C::LK / 2, a.Lk);
+                    if (ROWS < C::LK && a.Lk > ROWS) cb.issue(lds0 + C::KB + ROWS * 32, ROWS, a.Lk);
                 }
             }
         }
@@ -82,17 +94,27 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             if constexpr (C::NKR > 0) qn[C::NKD] = load_chunk<true>(qbbase, a.qb.ss, query, a.Lq, 8 * g, a.r);
         };
         if (wave < nqb) load_q(wave);
-        // Mask block (queries 32 qb .., keys 32 kb ..) as 32 rows of 64 bytes; rows and 16-byte chunks past the end re-read
-        // the last ones.
+        // Mask tile (queries 32 qb .., keys 32 kb ..) as 32 rows of 128 (pairs of blocks) or 64 bytes; rows and 16-byte chunks
+        // past the end re-read the last ones.
         const uint8_t *mbase = nullptr;
         if constexpr (C::MASK) mbase = reinterpret_cast<const uint8_t *>(a.mask.ptr) + mask_offset(a.mask, b, h) * 2;
         auto copy_mask = [&](int qb, int kb) {
-            int row, chunk;
-            lean_copy_place<4>(lane, row, chunk);
-            const int col = min(32 * kb + 8 * chunk, a.Lk - 8);
+            constexpr int NI = C::TILE / 1024, ROWS = 32 / NI; // copy instructions and the rows of one
+            int l = lane, row, chunk;
+            if constexpr (C::PAIR) asm volatile("" : "+v"(l)); // (the addresses are formed here, not kept in registers)
+            lean_copy_place<4>(l, row, chunk);
+            if constexpr (C::PAIR) {
+                row = l >> 3;
+                chunk = (l & 7) ^ swz_of<8>(row); // (rows + 8: two places further)
+            }
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-                lds_dma16_all((uint32_t)(min(32 * qb + 16 * j + row, a.Lq - 1) * (int)(a.mask.sm * 2) + col * 2), mbase, lds_m + j * 1024);
+            for (int j = 0; j < NI; ++j) {
+                const int col = min(32 * kb + 8 * (C::PAIR && (j & 1) ? chunk ^ 2 : chunk), a.Lk - 8);
+                lds_dma16_all((uint32_t)(min(32 * qb + ROWS * j + row, a.Lq - 1) * (int)(a.mask.sm * 2) + col * 2), mbase, lds_m + j * 1024);
+            }
+        };
+        auto mask_chunk = [&](int i) { // chunk i of this lane's row
+            return lds_load16(lds_m + (C::PAIR ? 2 * swz_off<8>(c, i) : lean_chunk_off<4>(c, i)));
         };
         if constexpr (C::MASK) {
             if (wave < nqb) copy_mask(wave, 0);
@@ -102,19 +124,20 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 
 #pragma unroll 1
         for (int qb = wave; qb < nqb; qb += C::NWAVES) {
-            if (!C::MASK && qb != wave) load_q(qb); // (a block ahead, as with a mask, it takes registers that pairs of blocks need)
+            if (C::PAIR && qb != wave) load_q(qb); // (a block ahead, as with a mask, it takes registers that pairs of blocks need)
             u32x4_t q[C::NK];
 #pragma unroll
             for (int t = 0; t < C::NK; ++t) q[t] = qn[t];
-            if (C::MASK && qb + C::NWAVES < nqb) load_q(qb + C::NWAVES);
+            if (C::MASK && !C::PAIR && qb + C::NWAVES < nqb) load_q(qb + C::NWAVES);
             f32x16_t o;
 #pragma unroll
             for (int v = 0; v < 16; ++v) o[v] = 0.f;
             float m_ref = -INFINITY, m2 = 0.f, l_run = 0.f, slack = lag;
             // N blocks of 32 keys from block kb on.  Without a mask two at a time (one row maximum, one test of the reference point and
             // one set of addresses for 64 keys), the last of an odd number alone: 4096 x 16 windows of 256 tokens 1430 -> 1354 us,
-            // 769 x 16 of 144 148 -> 142, 64 x 16 of 256 28.7 -> 27.  Masked blocks alone: the copies of two would leave two
-            // workgroups a compute unit, and masks loaded to registers a pair ahead cost more (1024 x 16 of 256 473 -> 635).
+            // 769 x 16 of 144 148 -> 142, 64 x 16 of 256 28.7 -> 27.  Masked blocks alone with four waves: the copies of two
+            // would leave two workgroups a compute unit, and masks loaded to registers a pair ahead cost more (1024 x 16 of 256
+            // 473 -> 635).
             auto group = [&](auto tag, int kb) __attribute__((always_inline)) {
                 constexpr int N = decltype(tag)::value;
                 const uint32_t at = kb * 2048;
@@ -123,21 +146,23 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                 for (int n = 0; n < N; ++n) {
                     f32x16_t sb;
                     if constexpr (C::MASK) {
-                        static_assert(N == 1, "");
-                        wait_vmcnt<0>();
+                        if (n == 0) wait_vmcnt<0>();
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) { // register v <-> key 32 kb + 8 (v / 4) + 4 g + v % 4 of the lane's row
-                            const u32x2_t x = *reinterpret_cast<const u32x2_t *>(smem + C::MT + wave * 2048 + lean_chunk_off<4>(c, j) + 8 * g);
-                            sb[4 * j + 0] = T::to_float((uint16_t)(x[0] & 0xffffu));
-                            sb[4 * j + 1] = T::to_float((uint16_t)(x[0] >> 16));
-                            sb[4 * j + 2] = T::to_float((uint16_t)(x[1] & 0xffffu));
-                            sb[4 * j + 3] = T::to_float((uint16_t)(x[1] >> 16));
+                        for (int j = 0; j < 2; ++j) {
+                            const u32x4_t x = mask_chunk(4 * n + 2 * j + g);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                sb[8 * j + 2 * e] = T::to_float((uint16_t)(x[e] & 0xffffu));
+                                sb[8 * j + 2 * e + 1] = T::to_float((uint16_t)(x[e] >> 16));
+                            }
                         }
-                        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (they have left LDS: the block after this one)
-                        if (kb + 1 < nkb)
-                            copy_mask(qb, kb + 1);
-                        else if (qb + C::NWAVES < nqb)
-                            copy_mask(qb + C::NWAVES, 0);
+                        if (n == N - 1) {
+                            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (they have left LDS: the tile after this one)
+                            if (kb + N < nkb)
+                                copy_mask(qb, kb + N);
+                            else if (qb + C::NWAVES < nqb)
+                                copy_mask(qb + C::NWAVES, 0);
+                        }
                     } else {
 #pragma unroll
                         for (int v = 0; v < 16; ++v) sb[v] = 0.f;
@@ -173,11 +198,11 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                 if (32 * (kb + N) > a.Lk) {
 #pragma unroll
                     for (int n = 0; n < N; ++n) {
-                        int key0 = 32 * (kb + n) + 4 * g;
+                        int key0 = 32 * (kb + n) + (C::MASK ? 8 : 4) * g;
                         asm volatile("" : "+v"(key0)); // (formed in the branch)
 #pragma unroll
                         for (int v = 0; v < 16; ++v)
-                            if (key0 + 8 * (v >> 2) + (v & 3) >= a.Lk) s[n][v] = -INFINITY;
+                            if (key0 + (C::MASK ? 16 * (v >> 3) + (v & 7) : 8 * (v >> 2) + (v & 3)) >= a.Lk) s[n][v] = -INFINITY;
                     }
                 }
 #pragma unroll
@@ -191,7 +216,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                 // Single blocks: after an even one that moved the reference the odd one moves it without a lag, so that it is the
                 // maximum of 64 keys, as in fwd_kernel: the probability 1 is the one that is not rounded.
                 const bool grow = mx > m_ref + slack; // also true for the first finite score of a row
-                if constexpr (C::MASK) slack = grow && !(kb & 1) ? 0.f : lag;
+                if constexpr (!C::PAIR) slack = grow && !(kb & 1) ? 0.f : lag;
                 if (__any(grow)) {
                     const float m_new = grow ? mx : m_ref;
                     const float alpha = grow ? fast_exp2((m_ref - m_new) * to_log2) : 1.f; // exp2(-inf) = 0
@@ -218,7 +243,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                     }
                 asm volatile("s_nop 11" : "+v"(o)); // (across the loop's branches)
             };
-            if constexpr (C::MASK) {
+            if constexpr (!C::PAIR) {
 #pragma unroll 1
                 for (int kb = 0; kb < nkb; ++kb) group(std::integral_constant<int, 1>{}, kb);
             } else {
@@ -237,9 +262,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     }
 }
 
-template <class T, int NKR, bool FOLD, bool MASK>
+template <class T, int NKR, bool FOLD, bool MASK, int NWAVES>
 static hipError_t launch_fwd_win_cfg(const FwdArgs &a, hipStream_t stream) {
-    typedef FwdWinCfg<T, NKR, FOLD, MASK> C;
+    typedef FwdWinCfg<T, NKR, FOLD, MASK, NWAVES> C;
     auto kern = fwd_win_kernel<T, C>;
     static KernelOnce once;
     const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
@@ -257,11 +282,24 @@ static hipError_t launch_fwd_win_cfg(const FwdArgs &a, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// Eight waves, one block of queries each, where a grid leaves compute units with fewer than four workgroups: twice the waves a
+// SIMD, and half as long a walk.  Four waves against eight, rank 16, us: 512 windows of 256 tokens 15.5 / 14.4, of 196 15.5 / 12.7, of 144
+// 11.1 / 9.1, with a mask (144, 256) 12.9 / 10.9, 21.0 / 18.7; 1024 windows of 256 29.3 / 26.2, of 196 24.5 / 22.8, with a mask
+// 22.9 / 20.0, 35.6 / 31.3; 2048 of 256 47.1 / 45.4, with a mask 37.6 / 35.8, 57.0 / 54.6.  Without a mask and with at most six blocks of
+// queries the idle waves count from 512 windows on (1024 of 144 15.5 / 16.7, 2048 28.2 / 30.2), above 2048 windows they do
+// everywhere (3072 of 144 with a mask 49.6 / 51.1, 8192 of 256 241 / 245).
+template <class T, int NKR, bool FOLD, bool MASK>
+static hipError_t launch_fwd_win_waves(const FwdArgs &a, hipStream_t stream) {
+    const int64_t windows = (int64_t)a.B * a.H;
+    const bool wide = a.Lq > 128 && (windows <= 2 * (int64_t)num_cus() || ((MASK || a.Lq > 192) && windows <= 8 * (int64_t)num_cus()));
+    return wide ? launch_fwd_win_cfg<T, NKR, FOLD, MASK, 8>(a, stream) : launch_fwd_win_cfg<T, NKR, FOLD, MASK, 4>(a, stream);
+}
+
 template <class T, int NKR>
 static hipError_t launch_fwd_win_r(const FwdArgs &a, hipStream_t stream) {
     if (a.mask.type == kMatrixMask) // (the mask is not divided by the scale)
-        return a.scale == 1.f ? launch_fwd_win_cfg<T, NKR, true, true>(a, stream) : launch_fwd_win_cfg<T, NKR, false, true>(a, stream);
-    return a.r == 0 || a.scale == 1.f ? launch_fwd_win_cfg<T, NKR, true, false>(a, stream) : launch_fwd_win_cfg<T, NKR, false, false>(a, stream);
+        return a.scale == 1.f ? launch_fwd_win_waves<T, NKR, true, true>(a, stream) : launch_fwd_win_waves<T, NKR, false, true>(a, stream);
+    return a.r == 0 || a.scale == 1.f ? launch_fwd_win_waves<T, NKR, true, false>(a, stream) : launch_fwd_win_waves<T, NKR, false, false>(a, stream);
 }
 
 // Compiled once per element type for head dim 32 (see Makefile).  When fb_fwd takes this path is decided by

@@ -179,16 +179,19 @@ inline bool ring_backward(const BwdArgs &a) {
 // rank up to 16, aligned tensors, no mask or a matrix mask of 16-byte chunks, a scale that keeps the order of the scores.
 // Against the general kernel, rank 16, us (window / general): 8192 pairs of 64 tokens 35 / 55, of 128 66 / 75, of 144
 // 107 / 183, with a matrix mask 47 / 84, 90 / 126, 149 / 318; 65536 of 256 1354 / 1572, masked 1904 / 2796; 512 pairs
-// of 144 14 / 16, masked 16 / 24; 512 of 256 21 / 19, masked 24 / 28; 1024 of 256 26 / 33.  Below two workgroups per compute unit
-// the general kernel's smaller workgroups spread better (256 of 256 16 / 13).
+// of 144 14 / 16, masked 16 / 24; 1024 of 256 26 / 33.  Where the general kernel has two workgroups a window (more than 128
+// queries) and these no longer find a compute unit each: 192 windows of 144 7.0 / 8.9, of 196 8.3 / 9.9, masked (144, 256)
+// 8.1 / 10.6, 10.7 / 12.0; 384 of 144 8.8 / 11.4, masked 10.4 / 17.5, 16.8 / 21.7.  Unmasked windows of eight blocks fill the general
+// kernel's workgroups: 384 of 256 13.3 / 12.3, 512 14.4 / 15.5; at most 128 queries are one workgroup there too (equal).
 inline bool window_forward(const FwdArgs &a) {
     const int64_t lim = (int64_t)1 << 22; // (32-bit byte offsets of 256 rows)
     if (a.d != 32 || a.r > 16 || a.r % 8 != 0 || a.Lq > 256 || a.Lk > 256 || a.causal || !(a.scale > 1e-6f && a.scale < 1e6f)) return false;
     if (!(a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.o.vec_ok && a.k.ss < lim && a.v.ss < lim)) return false;
     if (a.r > 0 && !(a.qb.vec_ok && a.kb.vec_ok && a.kb.ss < lim)) return false;
     if (a.mask.type != kNoMask && !mask_in_chunks(a.mask, a.Lk)) return false;
-    const bool few = a.mask.type != kNoMask || a.Lq <= 224;
-    return (int64_t)a.B * a.H >= (few ? 2 : 4) * (int64_t)num_cus();
+    const int64_t windows = (int64_t)a.B * a.H;
+    if (a.Lq > 128 && (a.mask.type != kNoMask || a.Lq <= 224)) return 4 * windows >= 3 * (int64_t)num_cus();
+    return windows >= 2 * (int64_t)num_cus();
 }
 
 // What a launcher remembers about one kernel instantiation (one static object per instantiation;

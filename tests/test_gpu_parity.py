@@ -873,7 +873,12 @@ def test_window_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, group, grads
     (torch.float16, 256, 4, 160, 193, 16, 1.0, False, False), (torch.float16, 1024, 1, 1, 31, 8, 0.3, False, False),
     (torch.bfloat16, 128, 8, 224, 129, 0, None, False, False), (torch.bfloat16, 260, 4, 256, 256, 16, 1.0, True, True),
     (torch.float16, 130, 4, 144, 144, 16, None, True, True), (torch.bfloat16, 516, 1, 250, 8, 8, None, False, True),
-    (torch.bfloat16, 64, 8, 100, 136, 0, None, False, True)])
+    (torch.bfloat16, 64, 8, 100, 136, 0, None, False, True),
+    # eight waves a window (small grids) and four: single rows of a last block, an odd number of key blocks, one block
+    (torch.bfloat16, 64, 3, 129, 88, 16, None, True, True), (torch.float16, 48, 4, 224, 161, 8, 1.0, False, False),
+    (torch.float16, 64, 8, 193, 8, 16, None, False, True), (torch.bfloat16, 64, 8, 136, 256, 0, None, False, False),
+    (torch.bfloat16, 257, 8, 136, 120, 16, None, True, True), (torch.bfloat16, 257, 8, 250, 200, 16, None, True, False),
+    (torch.float16, 257, 8, 130, 40, 8, 1.0, False, True), (torch.float16, 256, 8, 256, 256, 8, None, True, False)])
 def test_window_forward(gpu_device, dtype, B, H, Lq, Lk, r, scale, shared, masked):
     """Forward of short sequences on grids of several workgroups per compute unit (fb_fwd_win.hip), o and lse against the
     oracle; a mask of -100 and -inf blocks (rows that see one key block only) and random values."""
@@ -936,13 +941,13 @@ def test_window_forward_is_as_exact_as_the_general_kernel(gpu_device, dtype, n, 
     bias = qb.double().transpose(1, 2).contiguous() @ kb.double().permute(0, 2, 3, 1).contiguous()
     together = flash_bias_func(q, k, v, qb, kb, mask)
     error = torch.zeros(2, dtype=torch.float64, device=gpu_device)
-    for at in range(0, B, 32):  # (256 pairs: less than one for every workgroup slot)
-        part = [t[at:at + 32] for t in (q, k, v)]
-        m = None if mask is None else mask[at:at + 32]
+    for at in range(0, B, 16):  # (128 pairs: half a workgroup a compute unit)
+        part = [t[at:at + 16] for t in (q, k, v)]
+        m = None if mask is None else mask[at:at + 16]
         a = [t.double().transpose(1, 2).contiguous() for t in part]
         logits = a[0] @ a[1].transpose(-1, -2).contiguous() / math.sqrt(32) + bias
         exact = (torch.softmax(logits if m is None else logits + m.double(), -1) @ a[2]).transpose(1, 2)
-        for i, o in enumerate((together[at:at + 32], flash_bias_func(*part, qb, kb, m))):
+        for i, o in enumerate((together[at:at + 16], flash_bias_func(*part, qb, kb, m))):
             error[i] += (o.double() - exact).square().sum()
     # (millions of values with roundings of their own: the two errors are measured to a tenth of a percent)
     assert error[0].sqrt() <= 1.01 * error[1].sqrt(), error.sqrt()
