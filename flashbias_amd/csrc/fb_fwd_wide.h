@@ -7,6 +7,14 @@
 // in few banks, its stage takes about 40 registers (at head dim 128 the kernel spilled at 256), and K fragments are
 // requested one MFMA ahead.  Here global_load_lds copies [K], [K_b] and [V] row-major into two stages, one tile ahead,
 // V^T fragments come from transposing LDS reads, and no register holds a tile.
+//
+// Left to itself the compiler asks for two K fragments and waits for them, once a contraction step: at head dim 128 nine times a
+// tile of 64 keys, whose 34 products take 1088 cycles.  Here the order is fixed: fragments two steps ahead of their
+// products, the first columns of V with the last of them, addresses from two registers (240 -> 212 of them at head dim
+// 128, 147 -> 134 at 64).  us, before and after: causal B4 H32 L=4096 d128 r8 625 -> 610, B2 H8 L=1500 d128 r16 37.0 -> 35.0, B1 H4 L=999
+// d128 27.1 -> 24.8; d64 causal B2 H8 L=4096 r8 68.3 -> 62.0, r2 as 16 B2 H16 L=2048 45.2 -> 40.8, B1 H4 L=1000 r32 19.7 -> 18.8, B4 H16
+// L=2048 r8 92.6 -> 89.3.  What is left is products and exponentials of two waves that overlap in part.  Not kept: four waves a SIMD
+// at head dim 64 (spills: causal 64 -> 78, masked 44 -> 84).
 #pragma once
 #include "fb_lean_tiles.h"
 
@@ -26,6 +34,10 @@ struct FwdWideCfg {
     static constexpr int LDS_BYTES = 2 * STAGE * 2;
     // head dim <= 64: three workgroups per compute unit (168 registers, 3 x 40 KB)
     static constexpr int WAVES_EU = NKD <= 4 ? 3 : 2;
+    // Exponentials before another wave's products.  us, against the products first: causal B4 H32 L=4096 d128 629 -> 610, fp16 d64
+    // r16 8 x 8 x (1000 x 1500) with a padding mask 44.6 -> 43.9; without a mask at head dim 64 neither (causal B2 H8 L=4096
+    // 62.0, products first 63.7, exponentials first 66.3).
+    static constexpr bool EXP_FIRST = NKD > 4 || VMASK;
     static __device__ __forceinline__ bool low_parts(const FwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
 };
 
@@ -121,47 +133,62 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         const uint8_t *sKb = reinterpret_cast<const uint8_t *>(sV + C::SK);
         // (a tile hidden from every query of this wave: so are all later ones, but the copies and barriers go on)
         if (!(a.causal && n0 > wq0 + 31) && wq0 < a.Lq) {
-            // (the wave that feeds the matrix pipe goes first, its neighbour's exponentials fill the gaps: 2-3 % over taking
-            // turns by tile, causal B4 H32 L=4096 d128 646 -> 628 us)
-            __builtin_amdgcn_s_setprio(1);
+            if constexpr (C::EXP_FIRST) __builtin_amdgcn_s_setprio(0);
             f32x16_t s[C::KBLK];
 #pragma unroll
             for (int kb = 0; kb < C::KBLK; ++kb)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) s[kb][v] = 0.f;
+            // Fragments are requested two contraction steps ahead, beside the products; those of the first 16 keys of V with the
+            // last ones.
+            TileAddr<C::ROWCH> ta(lds_addr_of(sK), c, g);
+            asm volatile("" : "+v"(ta.row), "+v"(ta.tr));
+            u32x4_t kf[C::NK][C::KBLK], vt[C::NDV];
+            auto request = [&](int t) {
 #pragma unroll
-            for (int t = 0; t < C::NKD; ++t)
+                for (int kb = 0; kb < C::KBLK; ++kb)
+                    kf[t][kb] = t < C::NKD ? ta.load_row(t, kb * 32 * C::ROWCH * 16)
+                                           : *reinterpret_cast<const u32x4_t *>(sKb + lean_row_addr<C::CPR ? C::CPR : 2>(c, 2 * (t - C::NKD) + g) + kb * 32 * C::CPR * 16);
+            };
+            auto columns = [&](int key) {
 #pragma unroll
-                for (int kb = 0; kb < C::KBLK; ++kb) {
-                    const u32x4_t kf = *reinterpret_cast<const u32x4_t *>(sK + swz_off<C::ROWCH>(kb * 32 + c, 2 * t + g));
-                    s[kb] = T::mfma(kf, qr[t], s[kb]);
-                }
+                for (int n = 0; n < C::NDV; ++n) vt[n] = ta.load_tr(n, 2 * C::SK + key * C::ROWCH * 16);
+            };
             // the softmax scale multiplies the fp32 q k^T accumulator before the bias steps (:246-256)
-            if constexpr (!C::FOLD) {
+            auto scale_scores = [&]() {
 #pragma unroll
                 for (int kb = 0; kb < C::KBLK; ++kb) {
-                    if constexpr (C::VMASK) {
-                        const float *sM = reinterpret_cast<const float *>(sV + C::SK + C::SKB) + kb * 32 + 4 * g;
+                    const float *sM = reinterpret_cast<const float *>(sV + C::SK + C::SKB) + kb * 32 + 4 * g;
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const f32x4_t x = *reinterpret_cast<const f32x4_t *>(sM + 8 * j);
+                    for (int j = 0; j < 4; ++j) {
+                        f32x4_t x;
+                        if constexpr (C::VMASK) x = *reinterpret_cast<const f32x4_t *>(sM + 8 * j);
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) s[kb][4 * j + e] = __builtin_fmaf(s[kb][4 * j + e], a.scale, x[e]);
-                        }
-                    } else {
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) s[kb][v] *= a.scale;
+                        for (int e = 0; e < 4; ++e) s[kb][4 * j + e] = C::VMASK ? __builtin_fmaf(s[kb][4 * j + e], a.scale, x[e]) : s[kb][4 * j + e] * a.scale;
                     }
+                }
+            };
+            request(0);
+            request(1);
+            FB_HOLD;
+#pragma unroll
+            for (int t = 0; t < C::NK; ++t) {
+                if (!C::FOLD && t == C::NKD) scale_scores();
+                if (t + 2 < C::NK)
+                    request(t + 2);
+                else if (t + 2 == C::NK)
+                    columns(0);
+#pragma unroll
+                for (int kb = 0; kb < C::KBLK; ++kb) s[kb] = T::mfma(kf[t][kb], qr[t], s[kb]);
+                if (!C::FOLD && t == C::NKD - 1) {
+                    mix<C::KBLK * C::NKD, 1, 0>();
+                    FB_HOLD;
                 }
             }
-            if constexpr (C::NKR > 0) {
-#pragma unroll
-                for (int t = 0; t < C::NKR; ++t)
-#pragma unroll
-                    for (int kb = 0; kb < C::KBLK; ++kb) {
-                        const u32x4_t kf = *reinterpret_cast<const u32x4_t *>(sKb + lean_row_addr<C::CPR>(c, 2 * t + g) + kb * 32 * C::CPR * 16);
-                        s[kb] = T::mfma(kf, qr[C::NKD + t], s[kb]);
-                    }
+            if constexpr (!C::FOLD && C::NKR == 0) scale_scores();
+            if constexpr (C::FOLD) {
+                mix<C::KBLK * C::NK, 1, 0>();
+                FB_HOLD;
             }
             // (bitwise on purpose, as in the dq kernel: no scalar block between the last MFMA and the branch)
             const bool edge = (n0 + C::BN > a.Lk) | ((a.causal != 0) & (n0 + C::BN - 1 > wq0));
@@ -176,7 +203,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                         if (key >= a.Lk || (a.causal && key > query)) s[kb][v] = -INFINITY;
                     }
             }
-            __builtin_amdgcn_s_setprio(0);
+            if constexpr (C::EXP_FIRST) __builtin_amdgcn_s_setprio(1);
             float mx = s[0][0];
 #pragma unroll
             for (int kb = 0; kb < C::KBLK; ++kb)
@@ -208,8 +235,8 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                         l_run += p0 + p1;
                     }
 #pragma unroll
-                    for (int n = 0; n < C::NDV; ++n)
-                        acc_o[n] = T::mfma(lds_read_a_tr<C::ROWCH>(sV, kb * 32 + 16 * t, 32 * n, c, g), pb, acc_o[n]);
+                    for (int n = 0; n < C::NDV; ++n) acc_o[n] = T::mfma(vt[n], pb, acc_o[n]);
+                    if (2 * kb + t + 1 < 2 * C::KBLK) columns(kb * 32 + 16 * t + 16);
                 }
         }
         if constexpr (C::VMASK) {
