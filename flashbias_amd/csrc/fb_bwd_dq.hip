@@ -49,7 +49,6 @@ struct DqCfg {
     static constexpr int BM = NWAVES * QBLK * 32;
     static constexpr int KBLK = 2, BN = 32 * KBLK;
     static constexpr int UNROLL = SPLIT ? 1 : KBLK; // key blocks computed together
-    static constexpr bool ONECHAIN = SPLIT_ && !XMASK; // scale between the d steps and the r steps of one MFMA chain
     // sK row: [K | K_b] of one key in ROWCH swizzled 16-byte chunks; the one copy is read
     // row-wise for S^T and column-wise for [dQ | dQ_b]^T
     static constexpr int ROWCH = SPLIT ? 2 * NKD : 2 * NK <= 8 ? 8 : 2 * NK <= 16 ? 16 : 32;
@@ -452,24 +451,103 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
 #pragma unroll
             for (int ki = 0; ki < C::UNROLL; ++ki) {
                 const int kb = ko + ki;
-                TileAddr16 ta(lds_addr_of(sK) + kb * (32 * 256), c, g); // (SPLIT; the V tile follows at + 2 SK)
-                if constexpr (C::SPLIT) asm volatile("" : "+v"(ta.row), "+v"(ta.tr));
                 if (C::UNROLL == 1 && a.causal && n0 + kb * 32 > wq0 + 31) break; // hidden from every query of this wave
-                // (the wave that feeds the matrix pipe goes first, instead of turns by tile: 994 -> 977 us causal B4 H32 L=4096 d128)
-                if (C::SPLIT) __builtin_amdgcn_s_setprio(1);
+                if constexpr (C::SPLIT) {
+                    // Head dims above 64.  Left to itself the compiler has one fragment on its way and waits for it at every product, 27
+                    // times a block at head dim 128 (half of the wave cycles).  Here the order is fixed, K, V, K_b, then the columns of
+                    // [K | K_b], three fragments (of columns two) ahead: what the 242 registers of operands, accumulators and one
+                    // block's scores leave.  Training step, us: B2 H8 L=1500 r16 step 164 -> 151, fp16 B1 H4 L=999 r8 114.5 -> 105.5,
+                    // B2 H16 (2048 x 1700) r32 with a padding mask 338 -> 332.8, causal B4 H32 L=4096,
+                    // where power sets the clock, 2805 -> 2785.
+                    static_assert(C::QBLK == 1, "");
+                    TileAddr16 ta(lds_addr_of(sK) + kb * (32 * 256), c, g); // (the V tile follows at + 2 SK)
+                    asm volatile("" : "+v"(ta.row), "+v"(ta.tr));
+                    // (the wave that feeds the matrix pipe goes first, instead of turns by tile: 994 -> 977 us causal B4 H32 L=4096 d128)
+                    __builtin_amdgcn_s_setprio(1);
+                    const int query = wq0 + c;
+                    constexpr int NF = C::NK + C::NKD, NC = 2 * C::MB, FA = 3, CA = 2;
+                    u32x4_t f[NF], kt[NC], dsp[2];
+                    auto request = [&](int i) {
+                        f[i] = i < C::NKD       ? ta.load_row(i, 0)
+                               : i < 2 * C::NKD ? ta.load_row(i - C::NKD, 2 * C::SK)
+                                                : *reinterpret_cast<const u32x4_t *>(sKb + kb * 32 * C::CPR * 16 + lean_row_addr<C::CPR>(c, 2 * (i - 2 * C::NKD) + g));
+                    };
+                    auto columns = [&](int j) {
+                        const int t = j / C::MB, n = j % C::MB;
+                        if (C::SKB > 0 && 2 * n >= C::NKD)
+                            kt[j] = dense_read_a_tr<C::CPR>(sKb, kb * 32 + 16 * t, c, g);
+                        else
+                            kt[j] = ta.load_tr(n, 16 * 256 * t);
+                    };
+                    f32x16_t s, dp;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) s[v] = dp[v] = 0.f;
+#pragma unroll
+                    for (int i = 0; i < FA; ++i) request(i);
+                    FB_HOLD;
+#pragma unroll
+                    for (int i = 0; i < 2 * C::NKD; ++i) {
+                        if (i + FA < NF) request(i + FA);
+                        if (i < C::NKD)
+                            s = T::mfma(f[i], qr[0][i], s);
+                        else
+                            dp = T::mfma(f[i], dor[0][i - C::NKD], dp);
+                    }
+                    mix<2 * C::NKD, 1, 0>();
+                    FB_HOLD;
+                    // the softmax scale multiplies the fp32 q k^T accumulator before the bias steps (:638-641)
+                    if constexpr (!C::FOLD) {
+                        const float *sM = reinterpret_cast<const float *>(sV + C::SV + C::SKB) + kb * 32 + 4 * g;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            f32x4_t x;
+                            if constexpr (C::VMASK) x = *reinterpret_cast<const f32x4_t *>(sM + 8 * j);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) s[4 * j + e] = C::VMASK ? __builtin_fmaf(s[4 * j + e], a.scale, x[e]) : s[4 * j + e] * a.scale;
+                        }
+                    }
+#pragma unroll
+                    for (int t = 0; t < C::NKR; ++t) s = T::mfma(f[2 * C::NKD + t], qbr[0][t], s);
+#pragma unroll
+                    for (int j = 0; j < CA; ++j) columns(j);
+                    __builtin_amdgcn_s_setprio(0);
+                    // (bitwise on purpose, as below)
+                    const bool edge = (n0 + kb * 32 + 32 > a.Lk) | ((a.causal != 0) & (n0 + kb * 32 + 31 > wq0));
+                    if (edge) {
+                        int key0 = n0 + kb * 32 + 4 * g;
+                        asm volatile("" : "+v"(key0)); // (computed here, not kept in 16 registers across the loop)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) {
+                            const int key = key0 + 8 * (v >> 2) + (v & 3);
+                            if (key >= a.Lk || (a.causal && key > query)) s[v] = -INFINITY;
+                        }
+                    }
+#pragma unroll
+                    for (int v = 0; v < 16; v += 2) {
+                        const float p0 = fast_exp2(__builtin_fmaf(s[v], to_log2, -lse2[0]));
+                        const float p1 = fast_exp2(__builtin_fmaf(s[v + 1], to_log2, -lse2[0]));
+                        dsp[v >> 3][(v & 7) >> 1] = T::pack2(p0 * (dp[v] + negd1[0]), p1 * (dp[v + 1] + negd1[0]));
+                    }
+                    __builtin_amdgcn_s_setprio(1);
+                    FB_HOLD;
+                    // [dQ | dQ_b]^T += [K | K_b]^T dS^T over this block's 32 keys
+#pragma unroll
+                    for (int j = 0; j < NC; ++j) {
+                        if (j + CA < NC) columns(j + CA);
+                        acc[0][j % C::MB] = T::mfma(kt[j], dsp[j / C::MB], acc[0][j % C::MB]);
+                    }
+                    mix<NC, 2, 0>();
+                    FB_HOLD;
+                    continue;
+                }
                 u32x4_t ka[C::NK], va[C::NKD];
 #pragma unroll
                 for (int t = 0; t < C::NK; ++t) {
-                    if (C::SKB > 0 && t >= C::NKD)
-                        ka[t] = *reinterpret_cast<const u32x4_t *>(sKb + kb * 32 * C::CPR * 16 + lean_row_addr<C::CPR>(c, 2 * (t - C::NKD) + g));
-                    else if constexpr (C::SPLIT)
-                        ka[t] = ta.load_row(t, 0);
-                    else
-                        ka[t] = *reinterpret_cast<const u32x4_t *>(sK + swz_off<C::ROWCH>(kb * 32 + c, 2 * t + g));
+                    ka[t] = *reinterpret_cast<const u32x4_t *>(sK + swz_off<C::ROWCH>(kb * 32 + c, 2 * t + g));
                 }
 #pragma unroll
                 for (int t = 0; t < C::NKD; ++t)
-                    va[t] = C::SPLIT ? ta.load_row(t, 2 * C::SK) : *reinterpret_cast<const u32x4_t *>(sV + swz_off<C::ROWCHV>(kb * 32 + c, 2 * t + g));
+                    va[t] = *reinterpret_cast<const u32x4_t *>(sV + swz_off<C::ROWCHV>(kb * 32 + c, 2 * t + g));
                 u32x4_t dsp[C::QBLK][2]; // dS^T, packed, per 16-key step
 #pragma unroll
                 for (int qb = 0; qb < C::QBLK; ++qb) {
@@ -482,10 +560,8 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
                     // initial value of the bias chain
                     if constexpr (C::NKR > 0 || C::MASK) {
                         f32x16_t sb;
-                        // (the vector mask's values of this lane's registers, four at a time)
-                        const float *sM = !C::VMASK ? nullptr : (C::VROW ? reinterpret_cast<const float *>(smem + C::VBASE) + n0 % (C::VCH > 0 ? C::VCH : 1)
-                                                                         : reinterpret_cast<const float *>(sV + C::SV + C::SKB)) + kb * 32 + 4 * g;
                         if constexpr (C::VROW) {
+                            const float *sM = reinterpret_cast<const float *>(smem + C::VBASE) + n0 % (C::VCH > 0 ? C::VCH : 1) + kb * 32 + 4 * g;
 #pragma unroll
                             for (int j = 0; j < 4; ++j) {
                                 const f32x4_t x = *reinterpret_cast<const f32x4_t *>(sM + 8 * j);
@@ -518,27 +594,14 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
                         }
 #pragma unroll
                         for (int t = 0; t < C::NKD; ++t) s = T::mfma(ka[t], qr[qb][t], s);
-                        if constexpr (C::ONECHAIN && !C::FOLD) { // (a second accumulator would spill here)
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) {
-                                if constexpr (C::VMASK) {
-                                    const f32x4_t x = *reinterpret_cast<const f32x4_t *>(sM + 8 * j);
-#pragma unroll
-                                    for (int e = 0; e < 4; ++e) s[4 * j + e] = __builtin_fmaf(s[4 * j + e], a.scale, x[e]);
-                                } else {
-#pragma unroll
-                                    for (int e = 0; e < 4; ++e) s[4 * j + e] *= a.scale;
-                                }
-                            }
-                        }
 #pragma unroll
                         for (int t = C::NKD; t < C::NK; ++t) {
-                            if constexpr (C::FOLD || C::ONECHAIN)
+                            if constexpr (C::FOLD)
                                 s = T::mfma(ka[t], qbr[qb][t - C::NKD], s);
                             else
                                 sb = T::mfma(ka[t], qbr[qb][t - C::NKD], sb);
                         }
-                        if constexpr (!C::FOLD && !C::ONECHAIN) {
+                        if constexpr (!C::FOLD) {
 #pragma unroll
                             for (int v = 0; v < 16; ++v) s[v] = __builtin_fmaf(s[v], a.scale, sb[v]);
                         }
@@ -552,7 +615,6 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
                     }
 #pragma unroll
                     for (int t = 0; t < C::NKD; ++t) dp = T::mfma(va[t], dor[qb][t], t == 0 ? negd[qb] : dp);
-                    if (C::SPLIT) __builtin_amdgcn_s_setprio(0);
                     // (bitwise on purpose: a short-circuit evaluation puts a small block of scalar code between the last
                     // MFMA and the branch, which the branch's other edge skips, and the compiler then counts the
                     // wait states between an MFMA and the first reader of its result along the longer path only)
@@ -570,25 +632,15 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
                     for (int v = 0; v < 16; v += 2) {
                         const float p0 = fast_exp2(__builtin_fmaf(s[v], to_log2, -lse2[qb]));
                         const float p1 = fast_exp2(__builtin_fmaf(s[v + 1], to_log2, -lse2[qb]));
-                        if constexpr (C::SPLIT)
-                            dsp[qb][v >> 3][(v & 7) >> 1] = T::pack2(p0 * (dp[v] + negd1[qb]), p1 * (dp[v + 1] + negd1[qb]));
-                        else
-                            dsp[qb][v >> 3][(v & 7) >> 1] = T::pack2(p0 * dp[v], p1 * dp[v + 1]);
+                        dsp[qb][v >> 3][(v & 7) >> 1] = T::pack2(p0 * dp[v], p1 * dp[v + 1]);
                     }
                 }
-                if (C::SPLIT) __builtin_amdgcn_s_setprio(1);
                 // [dQ | dQ_b]^T += [K | K_b]^T dS^T over this block's 32 keys
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
                     for (int n = 0; n < C::MB; ++n) {
-                        u32x4_t kt;
-                        if (C::SKB > 0 && 2 * n >= C::NKD)
-                            kt = dense_read_a_tr<C::CPR>(sKb, kb * 32 + 16 * t, c, g);
-                        else if constexpr (C::SPLIT)
-                            kt = ta.load_tr(n, 16 * 256 * t);
-                        else
-                            kt = lds_read_a_tr<C::ROWCH>(sK, kb * 32 + 16 * t, 32 * n, c, g);
+                        const u32x4_t kt = lds_read_a_tr<C::ROWCH>(sK, kb * 32 + 16 * t, 32 * n, c, g);
 #pragma unroll
                         for (int qb = 0; qb < C::QBLK; ++qb) acc[qb][n] = T::mfma(kt, dsp[qb][t], acc[qb][n]);
                     }
