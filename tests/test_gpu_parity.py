@@ -953,6 +953,30 @@ def test_window_forward_is_as_exact_as_the_general_kernel(gpu_device, dtype, n, 
     assert error[0].sqrt() <= 1.01 * error[1].sqrt(), error.sqrt()
 
 
+@pytest.mark.parametrize("dtype,n,masked", [(torch.float16, 64, False), (torch.bfloat16, 144, False), (torch.float16, 144, True), (torch.bfloat16, 256, True),
+                                            (torch.bfloat16, 64, True)])
+def test_window_forward_moves_its_reference_point_block_by_block(gpu_device, dtype, n, masked):
+    """Rows that see two keys, one in each of the first two blocks of 32, the second with the larger score; v is zero at the second.
+    The first key's probability is 1 when its block is done and is scaled in fp32 afterwards, so o is exact up to its own
+    rounding: the error against float64 is that of float64 rounded once.  A probability rounded to the element type against
+    the pair's maximum would make it sqrt(2) times as much."""
+    B, H = 128, 4
+    g = torch.Generator().manual_seed(n)
+    u = (1 + 1.5 * torch.rand(B, n, H, generator=g)).to(dtype)
+    qb, kb = torch.zeros(B, n, H, 8, dtype=dtype), torch.zeros(B, n, H, 8, dtype=dtype)
+    qb[..., 0] = u
+    kb[..., 0] = -200.0
+    kb[:, 5, :, 0], kb[:, 40, :, 0] = 0.0, 1.0
+    q = torch.zeros(B, n, H, 32, dtype=dtype)
+    v = torch.zeros(B, n, H, 32, dtype=dtype)
+    v[:, 5] = (1 + torch.rand(B, H, 32, generator=g)).to(dtype)
+    mask = torch.zeros(B, 1, n, n, dtype=dtype, device=gpu_device) if masked else None
+    o = flash_bias_func(*(t.to(gpu_device) for t in (q, q, v, qb, kb)), mask).cpu().double()
+    exact = v[:, 5].double()[:, None] / (1 + u.double().exp())[..., None]
+    error, rounding = (((x - exact) / exact).square().mean().sqrt() for x in (o, exact.to(dtype).double()))
+    assert error <= 1.1 * rounding, (error, rounding)
+
+
 # waves without keys (64 keys each) and with half a block of them, a second half of 128 queries and none, its ragged last
 # block, one entry a workgroup and several (the last workgroup ragged), the scale folded and not
 @pytest.mark.parametrize("dtype,B,H,Lq,Lk,r,scale,shared", [
