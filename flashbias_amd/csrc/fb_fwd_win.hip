@@ -20,6 +20,7 @@ struct FwdWinCfg {
     static constexpr bool FOLD = FOLD_, MASK = MASK_;
     static constexpr int NKD = 2, NKR = NKR_, NK = NKD + NKR_;
     static constexpr int NWAVES = NWAVES_, NTHREADS = 64 * NWAVES, LK = 256;
+    static constexpr bool ONE = 32 * NWAVES >= LK;     // one window a workgroup, one block of queries a wave: nothing is kept for the next
     static constexpr bool PAIR = !MASK || NWAVES == 8; // two blocks of 32 keys at a time
     static constexpr int TILE = PAIR ? 4096 : 2048;    // a wave's mask tile: 32 queries x 64 or 32 keys
     static constexpr int K = 0, V = K + LK * 64, KB = V + LK * 64, MT = KB + (NKR ? LK * 32 : 0), LDS_BYTES = MT + (MASK ? NWAVES * TILE : 0);
@@ -36,6 +37,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
 
     // a workgroup walks `walk` consecutive batch entries of its head
+    if constexpr (C::ONE) walk = 1;
     const int nbg = (a.B + walk - 1) / walk;
     const int work = xcd_remap(blockIdx.x, nbg * a.H);
     const int bg = work / a.H, h = work % a.H;
@@ -124,7 +126,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 
 #pragma unroll 1
         for (int qb = wave; qb < nqb; qb += C::NWAVES) {
-            if (C::PAIR && qb != wave) load_q(qb); // (a block ahead, as with a mask, it takes registers that pairs of blocks need)
+            if (C::PAIR && !C::ONE && qb != wave) load_q(qb); // (a block ahead, as with a mask, it takes registers that pairs of blocks need)
             u32x4_t q[C::NK];
 #pragma unroll
             for (int t = 0; t < C::NK; ++t) q[t] = qn[t];
@@ -160,7 +162,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (they have left LDS: the tile after this one)
                             if (kb + N < nkb)
                                 copy_mask(qb, kb + N);
-                            else if (qb + C::NWAVES < nqb)
+                            else if (!C::ONE && qb + C::NWAVES < nqb)
                                 copy_mask(qb + C::NWAVES, 0);
                         }
                     } else {
@@ -268,6 +270,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             if (ok && g == 0) a.lse[((int64_t)b * a.H + h) * a.Lq + query] = m_ref * (C::FOLD ? a.scale : 1.f) + __builtin_amdgcn_logf(l) * kLn2;
             uint16_t *orow = const_cast<uint16_t *>(a.o.ptr) + b * a.o.sb + h * a.o.sh + (int64_t)(ok ? query : 0) * a.o.ss;
             store_acc_rows<T, true>(orow, ok, true, o, 1.f / l, a.d, g);
+            if constexpr (C::ONE) break;
         }
         if (bi + 1 < walk) barrier_lds(); // everyone has read K and V
     }
@@ -281,7 +284,7 @@ static hipError_t launch_fwd_win_cfg(const FwdArgs &a, hipStream_t stream) {
     const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
     if (e != hipSuccess) return e;
     int walk = 1;
-    for (int w = 8; w > 1; w /= 2)
+    for (int w = C::ONE ? 1 : 8; w > 1; w /= 2)
         if ((int64_t)((a.B + w - 1) / w) * a.H >= 16 * (int64_t)num_cus()) {
             walk = w;
             break;

@@ -5,6 +5,7 @@ general dq kernel, where a short-circuit condition gave the block after the last
 units of head dim 128 (the wide forward, dq and dk/dv with factors in a region of their own)."""
 import importlib.util
 import os
+import re
 import shutil
 import subprocess
 
@@ -84,3 +85,14 @@ def test_compiled_window_and_projection_kernels():
         with open(os.path.join(CSRC, unit)) as f:
             text = f.read()
         assert text.count("v_mfma_f32_32x32x16") > products and waits.check(text) == [], unit
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None or shutil.which("make") is None, reason="needs hipcc and make")
+@pytest.mark.parametrize("unit,kernel", [("fwd_win_bf16_2", "fwd_win_kernel"), ("fwd_win_f16_2", "fwd_win_kernel")])
+def test_kernels_that_keep_to_their_registers(unit, kernel):
+    """Kernels written for a number of waves a SIMD whose registers just hold them: none of their instantiations spills."""
+    path = f"build/asm/fb_{unit}.s"
+    subprocess.run(["make", path], cwd=CSRC, check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    with open(os.path.join(CSRC, path)) as f:
+        scratch = {name: int(size) for name, size in re.findall(r"\.amdhsa_kernel (\S+)\n.*?\.amdhsa_private_segment_fixed_size (\d+)", f.read(), re.S) if kernel in name}
+    assert scratch and not any(scratch.values()), scratch
