@@ -48,16 +48,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         __syncthreads();
     }
     const float to_log2 = C::FOLD ? a.scale * kLog2e : kLog2e, lag = 8.f / to_log2;
-    // With a mask a row of [K | K_b] stands for the key whose bits 2 and 3 are swapped: register v of a lane is then key 16 (v / 8) + 8 g +
-    // v % 8, and its mask values come in chunks of 16 bytes.
-    const int krow = C::MASK ? (c & 19) | ((c & 4) << 1) | ((c & 8) >> 1) : c;
-    const uint32_t row_off[2] = {lds0 + lean_row_addr<4>(krow, g), lds0 + lean_row_addr<4>(krow, 2 + g)};
-    const uint32_t kb_row = lds0 + C::KB + lean_row_addr<2>(krow, g);
-    auto col_at = [&](int hi) { // (lean_tr_addr4, in that order of the keys)
-        if constexpr (C::MASK) return lean_chunk_off<4>(8 * g + ((c & 15) >> 2) + 4 * hi, 2 * (c >> 4) + ((c & 3) >> 1)) + 8 * (c & 1);
-        return lean_tr_addr4(c, g, hi);
-    };
-    const uint32_t col_off[2] = {lds0 + C::V + col_at(0), lds0 + C::V + col_at(1)};
+    const uint32_t row_off[2] = {lds0 + lean_row_addr<4>(c, g), lds0 + lean_row_addr<4>(c, 2 + g)};
+    const uint32_t col_off[2] = {lds0 + C::V + lean_tr_addr4(c, g, 0), lds0 + C::V + lean_tr_addr4(c, g, 1)};
+    const uint32_t kb_row = lds0 + C::KB + lean_row_addr<2>(c, g);
     const uint32_t lds_m = lds0 + C::MT + wave * C::TILE;
 
     for (int bi = 0; bi < walk; ++bi) {
@@ -115,9 +108,10 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                 lds_dma16_all((uint32_t)(min(32 * qb + ROWS * j + row, a.Lq - 1) * (int)(a.mask.sm * 2) + col * 2), mbase, lds_m + j * 1024);
             }
         };
-        auto mask_chunk = [&](int i) { // chunk i of this lane's row
-            return lds_load16(lds_m + (C::PAIR ? 2 * swz_off<8>(c, i) : lean_chunk_off<4>(c, i)));
-        };
+        // This half-wave's four keys of the eight from 8 i on, in this lane's row of the tile.  (Chunks differ in address bits that are
+        // XORed in; eight waves: from an opaque address, or each one's is kept and fp16 spills.)
+        uint32_t mrow = lds_m + (C::PAIR ? 2 * swz_off<8>(c, 0) : lean_chunk_off<4>(c, 0)) + 8 * g;
+        auto mask_run = [&](int i) { return *(const __attribute__((address_space(3))) u32x2_t *)(mrow ^ (uint32_t)(16 * i)); };
         if constexpr (C::MASK) {
             if (wave < nqb) copy_mask(wave, 0);
         }
@@ -149,13 +143,14 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                     f32x16_t sb;
                     if constexpr (C::MASK) {
                         if (n == 0) wait_vmcnt<0>();
+                        if constexpr (C::PAIR) asm volatile("" : "+v"(mrow));
 #pragma unroll
-                        for (int j = 0; j < 2; ++j) {
-                            const u32x4_t x = mask_chunk(4 * n + 2 * j + g);
+                        for (int j = 0; j < 4; ++j) { // register v <-> key 8 (v / 4) + 4 g + v % 4 of the block
+                            const u32x2_t x = mask_run(4 * n + j);
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                sb[8 * j + 2 * e] = T::to_float((uint16_t)(x[e] & 0xffffu));
-                                sb[8 * j + 2 * e + 1] = T::to_float((uint16_t)(x[e] >> 16));
+                            for (int e = 0; e < 2; ++e) {
+                                sb[4 * j + 2 * e] = T::to_float((uint16_t)(x[e] & 0xffffu));
+                                sb[4 * j + 2 * e + 1] = T::to_float((uint16_t)(x[e] >> 16));
                             }
                         }
                         if (n == N - 1) {
@@ -200,11 +195,11 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                 if (32 * (kb + N) > a.Lk) {
 #pragma unroll
                     for (int n = 0; n < N; ++n) {
-                        int key0 = 32 * (kb + n) + (C::MASK ? 8 : 4) * g;
+                        int key0 = 32 * (kb + n) + 4 * g;
                         asm volatile("" : "+v"(key0)); // (formed in the branch)
 #pragma unroll
                         for (int v = 0; v < 16; ++v)
-                            if (key0 + (C::MASK ? 16 * (v >> 3) + (v & 7) : 8 * (v >> 2) + (v & 3)) >= a.Lk) s[n][v] = -INFINITY;
+                            if (key0 + 8 * (v >> 2) + (v & 3) >= a.Lk) s[n][v] = -INFINITY;
                     }
                 }
 #pragma unroll

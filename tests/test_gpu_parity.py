@@ -977,6 +977,21 @@ def test_window_forward_moves_its_reference_point_block_by_block(gpu_device, dty
     assert error <= 1.1 * rounding, (error, rounding)
 
 
+@pytest.mark.parametrize("dtype,n,r,scale", [(torch.bfloat16, 64, 16, None), (torch.bfloat16, 144, 16, None), (torch.float16, 136, 8, 1.0), (torch.float16, 256, 0, 1.0),
+                                             (torch.bfloat16, 200, 16, 1.0)])
+def test_window_forward_is_one_arithmetic(gpu_device, dtype, n, r, scale):
+    """A mask of zeros gives the bits of no mask, and windows in a small call (eight waves a window above 128 tokens) those that
+    they have in a large one (four): the keys are summed in one order, block by block.  (Without factors and at another scale than 1
+    the scale is folded where there is no mask only.)"""
+    B, H = 520, 4
+    q, k, v, *fac, _ = [t if t is None else t.to(gpu_device) for t in make_inputs(B, n, n, H, 32, r, dtype, seed=n, bq=(True, False), bk=(True, False))]
+    zeros = torch.zeros(1, 1, n, n, device=gpu_device, dtype=dtype).expand(B, 1, n, n)
+    o = flash_bias_func(q, k, v, *fac, None, False, scale)
+    assert torch.equal(o, flash_bias_func(q, k, v, *fac, zeros, False, scale))
+    for mask in (None, zeros[:128]):
+        assert torch.equal(o[:128], flash_bias_func(q[:128], k[:128], v[:128], *fac, mask, False, scale))
+
+
 # waves without keys (64 keys each) and with half a block of them, a second half of 128 queries and none, its ragged last
 # block, one entry a workgroup and several (the last workgroup ragged), the scale folded and not
 @pytest.mark.parametrize("dtype,B,H,Lq,Lk,r,scale,shared", [
