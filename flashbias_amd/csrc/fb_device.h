@@ -285,6 +285,22 @@ __device__ __forceinline__ void lds_dma16_lanes(uint32_t off, const void *base, 
                  : "v"(off), "s"(ub), "s"(lds), "s"(lanes)
                  : "memory");
 }
+// Zeros at LDS byte address lds + 16 * lane for the lanes of `on`: rows of V past the end of a sequence.  Their probabilities are 0,
+// and 0 times an infinite value of the last row, read again in their place, would be NaN.  (LDS stores: barrier_lds waits.)
+__device__ __forceinline__ void lds_zero16(uint32_t lds, int lane, bool on) {
+    if (on) {
+        uint32_t zero = 0;
+        asm volatile("" : "+v"(lane), "+v"(zero)); // (formed here, not kept in registers across the caller's loop)
+        *(__attribute__((address_space(3))) u32x4_t *)(lds + 16 * lane) = u32x4_t{zero, zero, zero, zero};
+    }
+}
+// Copies by the lanes of `lanes` whose row is in range, zeros by those whose row is not.  A wave without a row in range issues no
+// copy: for kernels that wait for all of theirs.
+__device__ __forceinline__ void lds_dma16_or_zero(uint32_t off, const void *base, uint32_t lds, int lane, uint64_t lanes, bool in_range) {
+    const uint64_t some = lanes & __builtin_amdgcn_ballot_w64(in_range);
+    if (some) lds_dma16_lanes(off, base, lds, some);
+    lds_zero16(lds, lane, !in_range);
+}
 __device__ __forceinline__ void lds_dma4(const void *g, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(g) : "memory");
 }
@@ -340,6 +356,20 @@ struct TileDma {
             lanes_b[j] = HASB ? __builtin_amdgcn_ballot_w64(is_b && cc * 8 < ncols_b) : 0;
             off[j] = (uint32_t)r * (uint32_t)((is_b ? ldb : lda) * 2) + cc * 16;
         }
+    }
+
+    // A tile of one tensor with zeros in the rows past the end (lds_dma16_or_zero), for kernels that wait for all of their copies.
+    __device__ __forceinline__ void issue_or_zero(uint32_t lds_tile, int r0, int nrows, int64_t lda) {
+        static_assert(!HASB, "");
+        if (r0 + ROWS <= nrows) {
+#pragma unroll
+            for (int j = 0; j < NI; ++j) lds_dma16_lanes(off[j], pa, lds_tile + (wave * NI + j) * 1024, lanes_a[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < NI; ++j)
+                lds_dma16_or_zero(off[j], pa, lds_tile + (wave * NI + j) * 1024, lane, lanes_a[j], r0 + ((wave * NI + j) * 64 + lane) / ROWCH < nrows);
+        }
+        pa += lda * (2 * ROWS);
     }
 
     // Copies the next tile, rows [r0, r0 + ROWS) clamped to nrows - 1, and moves on to the one

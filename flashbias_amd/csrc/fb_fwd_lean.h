@@ -320,10 +320,17 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
             }
         }
         // the next tile must have landed before the barrier that lets it start
-        if (it + 2 < ntiles_k)
+        if (it + 2 < ntiles_k) {
             wait_vmcnt<C::NDMA>();
-        else
+        } else {
             wait_vmcnt<0>();
+            // (a ragged last tile: this wave's rows of V past the end become zeros, see lds_dma16_or_zero; Lk is at least BN)
+            const int left = a.Lk - n0 - C::BN;
+            if (it + 1 < ntiles_k && left < C::BN) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) lds_zero16(lds0 + ((STG + 1) % 3) * C::STAGE_BYTES + C::V_OFF + wave * 2048 + j * 1024, lane, 32 * wave + 16 * j + krow >= left);
+            }
+        }
         barrier_lds();
     };
 #pragma unroll 1

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         const uint32_t base = lds0 + buf * C::STAGE;
         kd.issue(kptr + (int64_t)n0 * kd.pitch, base + C::K, wave, lane, a.Lk - n0);
         if constexpr (C::NKR > 0) kbd.issue(base + C::KB, n0, a.Lk);
-        vd.issue(vptr + (int64_t)n0 * vd.pitch, base + C::V, wave, lane, a.Lk - n0);
+        vd.template issue<true>(vptr + (int64_t)n0 * vd.pitch, base + C::V, wave, lane, a.Lk - n0);
     };
     // Vector mask: thread `tid` carries the value of key n0 + tid of the tile that follows.
     float mkey = 0.f;

@@ -102,7 +102,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         const uint32_t base = lds_addr_of(stage0 + buf * C::STAGE);
         kd.issue(base, n0, a.Lk, a.k.ss, 0, C::ROWCH);
         if constexpr (C::NKR > 0) kbd.issue(base + 4 * C::SK, n0, a.Lk);
-        vd.issue(base + 2 * C::SK, n0, a.Lk, a.v.ss, 0, C::ROWCH);
+        vd.issue_or_zero(base + 2 * C::SK, n0, a.Lk, a.v.ss);
     };
     // Vector mask: thread `tid` carries the value of key n0 + tid of the tile that follows.
     float mkey = 0.f;

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     for (int bi = 0; bi < walk; ++bi) {
         const int b = __builtin_amdgcn_readfirstlane(bg * walk + bi);
         if (b >= a.B) break;
-        {   // K and V: 16 rows a copy instruction, whole blocks of 32 keys (rows past the end: the last one again)
+        {   // K and V: 16 rows a copy instruction, whole blocks of 32 keys (past the end K's last row again, zeros for V)
             const uint8_t *kbase = reinterpret_cast<const uint8_t *>(a.k.ptr + b * a.k.sb + h * a.k.sh);
             const uint8_t *vbase = reinterpret_cast<const uint8_t *>(a.v.ptr + b * a.v.sb + h * a.v.sh);
             int row, chunk;
@@ -66,7 +66,11 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                 const int i = wave + C::NWAVES * j, r = min(16 * i + row, a.Lk - 1);
                 if (i < 2 * nkb) {
                     lds_dma16_all((uint32_t)(r * (int)(a.k.ss * 2) + chunk * 16), kbase, lds0 + C::K + i * 1024);
-                    lds_dma16_all((uint32_t)(r * (int)(a.v.ss * 2) + chunk * 16), vbase, lds0 + C::V + i * 1024);
+                    const uint32_t voff = (uint32_t)(r * (int)(a.v.ss * 2) + chunk * 16);
+                    if (16 * i + 16 <= a.Lk)
+                        lds_dma16_all(voff, vbase, lds0 + C::V + i * 1024);
+                    else
+                        lds_dma16_or_zero(voff, vbase, lds0 + C::V + i * 1024, lane, ~0ull, 16 * i + row < a.Lk);
                 }
             }
             if constexpr (C::NKR > 0) {

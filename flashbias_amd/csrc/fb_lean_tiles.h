@@ -98,7 +98,8 @@ struct LeanCopy4 {
     }
     // tile = first row of the tile in the tensor (wave-uniform), region = LDS byte address of the
     // region; rows_left = rows of the tensor from the tile's first row on (>= 1): rows past the end
-    // re-read the last one
+    // re-read the last one or (ZERO) are zeros (lds_dma16_or_zero)
+    template <bool ZERO = false>
     __device__ __forceinline__ void issue(const uint8_t *tile, uint32_t region, int wave, int lane, int rows_left) const {
         if (rows_left >= ROWS) {
 #pragma unroll
@@ -109,7 +110,10 @@ struct LeanCopy4 {
 #pragma unroll
             for (int j = 0; j < NI; ++j) {
                 const int over = max((ROWS / 4) * wave + 16 * j + row - (rows_left - 1), 0);
-                lds_dma16_all(off[j] - (uint32_t)(over * pitch), tile, region + (NI * wave + j) * 1024);
+                if constexpr (ZERO)
+                    lds_dma16_or_zero(off[j], tile, region + (NI * wave + j) * 1024, lane, ~0ull, over == 0);
+                else
+                    lds_dma16_all(off[j] - (uint32_t)(over * pitch), tile, region + (NI * wave + j) * 1024);
             }
         }
     }

@@ -364,6 +364,31 @@ def test_query_gradients_one_block_a_wave(gpu_device, d, r, Lq, Lk, scale, dtype
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,Lq,Lk,d,r,kind", [
+    (2, 4, 200, 100, 32, 16, None), (2, 4, 200, 161, 32, 32, "vector"), (2, 4, 100, 33, 32, 16, "causal"),      # head dim 32: 64 keys a tile
+    (2, 4, 300, 300, 32, 8, None), (2, 4, 150, 130, 32, 0, None), (1, 4, 600, 600, 32, 8, "causal"),             # streamlined: 128
+    (2, 4, 200, 100, 64, 16, None), (2, 4, 200, 65, 40, 8, "vector"), (2, 4, 200, 127, 128, 8, "causal"),       # head dims above 32
+    (64, 4, 144, 140, 32, 16, None), (64, 4, 144, 136, 32, 16, "matrix"), (512, 4, 49, 49, 32, 16, None),       # windows
+    (1040, 4, 49, 40, 32, 16, "matrix"), (4100, 4, 20, 17, 32, 8, None),                                        # (several a workgroup)
+    (2, 4, 200, 100, 24, 16, None), (2, 4, 200, 100, 32, 64, None), (2, 4, 100, 90, 30, 5, None)])              # general
+def test_infinite_value_in_the_last_row_of_v(gpu_device, dtype, B, H, Lq, Lk, d, r, kind):
+    """Ragged lengths: nothing of V counts for keys past the end, the last row's infinity least of all.  o is infinite in its
+    channel wherever the last key is seen, and the other channels have the bits they have beside a finite value."""
+    q, k, v, qb, kb, _ = [t if t is None else t.to(gpu_device) for t in make_inputs(B, Lq, Lk, H, d, r, dtype, seed=Lk, bq=(True, False), bk=(True, False))]
+    mask = {"vector": (2, 1, 1, Lk), "matrix": (1, 1, Lq, Lk)}.get(kind)
+    mask = mask and torch.zeros(mask, device=gpu_device, dtype=dtype).expand(B, -1, -1, -1)
+    o = []
+    for x in (0.0, float("inf")):
+        v[:, -1, :, 3] = x
+        o.append(flash_bias_func(q, k, v, qb, kb, mask, kind == "causal"))
+    finite, infinite = o
+    rows = slice(Lk - 1, None) if kind == "causal" else slice(None)
+    assert torch.isposinf(infinite[:, rows, :, 3]).all()
+    infinite[..., 3] = finite[..., 3]
+    assert torch.equal(finite, infinite)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind,Lq,Lk,r,scale,shared", [
     ("matrix", 256, 256, 16, 1.0, True), ("matrix", 144, 144, 16, None, True), ("matrix", 129, 200, 32, None, False),
     ("matrix", 200, 129, 0, None, False), ("matrix", 131, 250, 8, 1.0, False), ("vector", 64, 64, 16, None, True),
