@@ -40,6 +40,10 @@ struct DkvMidCfg {
     static constexpr int LDS_BYTES = NSTAGE * STAGE;
     static constexpr int WAVES_EU = NKD == 4 ? 2 : 3;
     static_assert(WAVES_EU * LDS_BYTES <= 160 * 1024, "");
+    // Rank above 16 with dk_bias at head dims above 32: the places of the copies are formed where they are used.  Kept, they spill (24
+    // bytes), and a reload waits for the tile that has just been requested: training step, us, r32 causal B2 H8 L=4096 272 -> 265,
+    // B4 H16 L=2048 405 -> 400, B1 H4 L=1000 87.3 -> 85.  The others have the registers (r2 as 16 causal B2 H16 L=2048 136.5 -> 138).
+    static constexpr bool FRESH = NKD == 4 && NKR == 2 && BG;
     static constexpr bool ORDERED = NKD == 4; // two waves a SIMD: the order is fixed phase by phase
     static __device__ __forceinline__ bool low_parts(const BwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
 };
@@ -78,14 +82,17 @@ __device__ __forceinline__ void bwd_dkv_mid_body(const BwdArgs &a, int wg) {
 
         // ---- copies: per step every wave issues sixteen rows of Q and of dO, the first waves Q_b, the last ones a row of the
         // statistics.
+        auto row_place = [&](int lane, int &crow, int &cch) {
+            if constexpr (C::NKD == 4) {
+                crow = 16 * wave + (lane >> 3); // (and crow + 8, whose chunks the swizzle moves by two places)
+                cch = (lane & 7) ^ swz_of<8>(crow);
+            } else {
+                lean_copy_place<4>(lane, crow, cch);
+                crow += 16 * wave;
+            }
+        };
         int crow, cch;
-        if constexpr (C::NKD == 4) {
-            crow = 16 * wave + (lane >> 3); // (and crow + 8, whose chunks the swizzle moves by two places)
-            cch = (lane & 7) ^ swz_of<8>(crow);
-        } else {
-            lean_copy_place<4>(lane, crow, cch);
-            crow += 16 * wave;
-        }
+        row_place(lane, crow, cch);
         uint64_t lanes_on[C::NI];
 #pragma unroll
         for (int j = 0; j < C::NI; ++j) lanes_on[j] = __builtin_amdgcn_ballot_w64((cch ^ (2 * j)) * 8 < a.d);
@@ -94,15 +101,25 @@ __device__ __forceinline__ void bwd_dkv_mid_body(const BwdArgs &a, int wg) {
         const uint8_t *dbase = reinterpret_cast<const uint8_t *>(a.dout.ptr + b * a.dout.sb + h * a.dout.sh);
         const uint8_t *bbase = C::NKR > 0 ? reinterpret_cast<const uint8_t *>(a.qb.ptr + b * a.qb.sb + h * a.qb.sh) : nullptr;
         constexpr int QB_WAVES = C::NKR > 0 ? C::BMQ * C::CPR / 64 : 0;
-        int brow, bch; // (a rank of at most 8 folded with low parts: chunk 1 is a second copy of chunk 0)
-        lean_copy_place<C::CPR>(lane, brow, bch);
-        brow += (wave < QB_WAVES ? wave : 0) * (64 / C::CPR);
-        if (C::low_parts(a) && bch == 1) bch = 0;
+        // (a rank of at most 8 folded with low parts: chunk 1 is a second copy of chunk 0)
+        auto factor_place = [&](int lane, int &brow, int &bch) {
+            lean_copy_place<C::CPR>(lane, brow, bch);
+            brow += (wave < QB_WAVES ? wave : 0) * (64 / C::CPR);
+            if (C::low_parts(a) && bch == 1) bch = 0;
+        };
+        int brow, bch;
+        factor_place(lane, brow, bch);
         const uint64_t lanes_b = __builtin_amdgcn_ballot_w64(bch * 8 < a.r);
         const float *stat = a.delta + (((wave & 1) == 0 ? (int64_t)a.B * a.H : 0) + bh) * a.Lq;
         auto issue = [&](int step, int stage) {
             const int r0 = step * C::BMQ, last = a.Lq - 1 - r0; // (a ragged last step: rows past the end are the last one again)
             const uint32_t at = lds0 + stage * C::STAGE;
+            int l = lane; // (opaque: the places are formed here, not reloaded from scratch behind the copies)
+            if constexpr (C::FRESH) {
+                asm volatile("" : "+v"(l));
+                row_place(l, crow, cch);
+                factor_place(l, brow, bch);
+            }
 #pragma unroll
             for (int j = 0; j < C::NI; ++j) {
                 const uint32_t row = (uint32_t)min(crow + 8 * j, last), ch = (uint32_t)(cch ^ (2 * j)) * 16;
@@ -110,7 +127,7 @@ __device__ __forceinline__ void bwd_dkv_mid_body(const BwdArgs &a, int wg) {
                 lds_dma16_lanes(row * dpitch + ch, dbase + (int64_t)r0 * dpitch, at + C::SQ + (C::NI * wave + j) * 1024, lanes_on[j]);
             }
             if (wave < QB_WAVES) lds_dma16_lanes((uint32_t)min(brow, last) * bpitch + bch * 16, bbase + (int64_t)r0 * bpitch, at + 2 * C::SQ + wave * 1024, lanes_b);
-            if (wave >= 2) lds_dma4(stat + min(r0 + lane, a.Lq - 1), at + 2 * C::SQ + C::SQB + (wave & 1) * 4 * C::BMQ);
+            if (wave >= 2) lds_dma4(stat + min(r0 + l, a.Lq - 1), at + 2 * C::SQ + C::SQB + (wave & 1) * 4 * C::BMQ);
         };
         if (step0 < nsteps) issue(step0, 0);
 

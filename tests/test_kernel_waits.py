@@ -88,7 +88,9 @@ def test_compiled_window_and_projection_kernels():
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None or shutil.which("make") is None, reason="needs hipcc and make")
-@pytest.mark.parametrize("unit,kernel", [("fwd_win_bf16_2", "fwd_win_kernel"), ("fwd_win_f16_2", "fwd_win_kernel")])
+@pytest.mark.parametrize("unit,kernel", [("fwd_win_bf16_2", "fwd_win_kernel"), ("fwd_win_f16_2", "fwd_win_kernel"), ("fwd_bf16_2", "fwd_thin_kernel"),
+                                         ("bwd_dkv_bf16_4", "bwd_dkv_mid_kernel"), ("bwd_dkv_f16_4", "bwd_dkv_mid_kernel"),
+                                         ("bwd_dq_bf16_2", "bwd_dq_mid_kernel"), ("bwd_dq_bf16_4", "bwd_dq_mid_kernel")])
 def test_kernels_that_keep_to_their_registers(unit, kernel):
     """Kernels written for a number of waves a SIMD whose registers just hold them: none of their instantiations spills."""
     path = f"build/asm/fb_{unit}.s"
