@@ -90,7 +90,7 @@ def test_large_head_dim_and_rank_together(gpu_device, d, r, causal):
 @pytest.mark.parametrize("d,r,scale", [(32, 8, None), (32, 8, 0.25), (32, 8, 0.29), (32, 8, 3.0), (64, 16, None),
                                        (64, 32, 0.5), (64, 24, 0.3), (128, 8, None), (32, 0, None), (32, 0, 0.7),
                                        (32, 8, -0.2), (64, 0, -0.125), (32, 8, 1.0), (32, 16, 1.0), (64, 32, 1.0),
-                                       (128, 8, 1.0)])
+                                       (128, 8, 1.0), (64, 8, None), (40, 8, 0.3)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_scale_folded_into_the_contraction(gpu_device, d, r, scale, dtype):
     """Where it is exact (no factors; a scale of exactly 1, which leaves the factors as they are,
@@ -305,11 +305,12 @@ def test_wide_heads(gpu_device, d, r, Lq, Lk, scale, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("r,Lq,Lk,scale", [(16, 1, 1, None), (32, 127, 63, None), (24, 129, 64, None), (0, 128, 65, None), (8, 33, 640, 1.0), (32, 130, 129, 1.0),
-                                           (16, 257, 127, -0.2), (0, 31, 192, -0.1), (16, 64, 530, 0.0625), (8, 95, 100, None)])
+                                           (16, 257, 127, -0.2), (0, 31, 192, -0.1), (16, 64, 530, 0.0625), (8, 95, 100, None),
+                                           (8, 129, 520, 3.0)])
 def test_thin_forward(gpu_device, r, Lq, Lk, scale, dtype):
     """Forward of head dim 32 with four waves a SIMD at the edges of its tiles (128 queries, 64 keys, two stages), padded ranks,
-    the scale folded (a power of two, 1, low parts at rank 8, a negative one without factors) and not, causal, and vector masks of
-    both kinds whose last keys are off."""
+    the scale folded (a power of two, 1, low parts at rank 8 and 512 keys with a scale that the streamlined kernel refuses) and not (a
+    negative one, short loops), causal, and vector masks of both kinds whose last keys are off."""
     for kind in (None, "causal", "mask"):
         mask = None
         if kind == "mask":
@@ -321,11 +322,12 @@ def test_thin_forward(gpu_device, r, Lq, Lk, scale, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d,r,Lq,Lk,scale", [(64, 16, 1, 1, None), (64, 32, 63, 127, None), (40, 8, 64, 129, None), (64, 0, 65, 128, None), (56, 24, 600, 200, 0.125),
-                                             (48, 16, 129, 33, 1.0), (64, 8, 127, 96, -0.1), (64, 0, 530, 64, -0.2), (64, 32, 200, 31, 0.0625)])
+                                             (48, 16, 129, 33, 1.0), (64, 8, 127, 96, -0.1), (64, 0, 530, 64, -0.2), (64, 32, 200, 31, 0.0625),
+                                             (64, 8, 520, 97, None)])
 def test_key_gradients_of_middle_head_dims(gpu_device, d, r, Lq, Lk, scale, dtype):
     """dk, dv and dk_bias of head dims 33 ... 64 at the edges of the kernel's tiles (64 queries a step, two blocks, 128 keys),
-    padded head dims and ranks, the scale folded and not, causal, vector masks, constant factors (without their gradients) and
-    factors shared by the batch (summed over groups of entries)."""
+    padded head dims and ranks, the scale folded (low parts at rank 8 and 512 queries) and not, causal, vector masks, constant factors
+    (without their gradients) and factors shared by the batch (summed over groups of entries)."""
     for kind in (None, "causal", "mask"):
         mask = None
         if kind == "mask":
@@ -348,10 +350,12 @@ def test_key_gradients_of_middle_head_dims(gpu_device, d, r, Lq, Lk, scale, dtyp
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d,r,Lq,Lk,scale", [(32, 32, 1, 1, None), (32, 16, 127, 63, None), (24, 24, 129, 64, None), (32, 32, 128, 65, 1.0), (32, 8, 33, 600, None),
-                                             (32, 16, 130, 129, 0.125), (24, 16, 257, 127, -0.2), (64, 16, 127, 64, None), (40, 24, 129, 65, 0.3)])
+                                             (32, 16, 130, 129, 0.125), (24, 16, 257, 127, -0.2), (64, 16, 127, 64, None), (40, 24, 129, 65, 0.3),
+                                             (64, 8, 97, 520, None), (40, 8, 129, 513, 0.3), (24, 8, 130, 520, 0.5)])
 def test_query_gradients_one_block_a_wave(gpu_device, d, r, Lq, Lk, scale, dtype):
     """dq and dq_bias of head dims up to 64 at the edges of the kernel's tiles (128 queries, 64 keys, two blocks), padded head dims and
-    ranks, the scale folded and not, causal, with and without dq_bias, factors of the batch's own and shared (summed over groups)."""
+    ranks, the scale folded (low parts at rank 8 and 512 keys) and not, causal, with and without dq_bias, factors of the batch's own
+    and shared (summed over groups)."""
     for causal in (False, True):
         _case(gpu_device, 2, Lq, Lk, 3, d, r, dtype, causal, scale=scale, seed=d + r + Lk, o_by_magnitude=True)
         for B, bc in ((2, False), (33, True)):
@@ -700,7 +704,7 @@ def test_backward_phases_through_the_c_abi(gpu_device):
     (torch.bfloat16, 6, 8, 1000, 900, 16, False)])  # (one and a half workgroups per compute unit and kind)
 def test_small_grid_backward_in_one_launch(gpu_device, dtype, B, H, Lq, Lk, r, causal):
     """On grids that give neither backward kernel more than one workgroup per compute unit (with factors of rank 16
-    and more under a causal mask: up to one and a half per workgroup slot) fb_bwd runs
+    and more one and a half, under a causal mask one and a half per workgroup slot) fb_bwd runs
     the preprocess step and one launch that holds the dq and the dk/dv workgroups side by side: the
     gradients and the scratch buffer are bit for bit those of the three phases launched one by one,
     and the gradients pass the gate against the oracle (ragged and rectangular shapes, even and odd
@@ -932,12 +936,13 @@ def test_window_forward(gpu_device, dtype, B, H, Lq, Lk, r, scale, shared, maske
 
 @pytest.mark.parametrize("dtype,low", [(torch.bfloat16, torch.finfo(torch.bfloat16).min), (torch.bfloat16, -1e30), (torch.bfloat16, -1e9),
                                        (torch.float16, torch.finfo(torch.float16).min)])
-@pytest.mark.parametrize("n,r,scale", [(64, 16, None), (64, 8, 1.0), (128, 16, None), (256, 0, None)])
-def test_windows_shifted_by_lowest_values(gpu_device, dtype, low, n, r, scale):
+@pytest.mark.parametrize("n,r,scale,B", [(64, 16, None, 520), (64, 8, 1.0, 520), (128, 16, None, 520), (256, 0, None, 520),
+                                         (256, 16, None, 64), (144, 8, 1.0, 64), (192, 0, None, 50)])  # (eight waves a window)
+def test_windows_shifted_by_lowest_values(gpu_device, dtype, low, n, r, scale, B):
     """Shifted windows whose mask switches keys off by the type's lowest value, or one near it, in the place of -100: the first
     half of the keys for half of the queries, the second for the others (the result is that of -inf).  At 64 tokens the first
     half is one block of the window forward's 32 keys."""
-    B, H = 520, 4
+    H = 4
     q, k, v, qb, kb, do = make_inputs(B, n, n, H, 32, r, dtype, seed=n + r, bq=(True, False), bk=(True, False))
     if scale == 1.0:
         q = (q.float() / 6).to(dtype)
@@ -953,10 +958,11 @@ def test_windows_shifted_by_lowest_values(gpu_device, dtype, low, n, r, scale):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("n,low", [(64, None), (128, float("-inf")), (128, -1e4), (200, None)])
-def test_window_forward_is_as_exact_as_the_general_kernel(gpu_device, dtype, n, low):
+@pytest.mark.parametrize("n,low,B", [(64, None, 512), (128, float("-inf"), 512), (128, -1e4, 512), (200, None, 512),
+                                     (200, None, 64), (144, -1e4, 64), (256, float("-inf"), 128)])  # (eight waves a window)
+def test_window_forward_is_as_exact_as_the_general_kernel(gpu_device, dtype, n, low, B):
     """Error of o against float64 beside that of the same windows in calls of a size that the general kernel serves."""
-    B, H, r = 512, 8, 16
+    H, r = 8, 16
     q, k, v, qb, kb, _ = [t.to(gpu_device) for t in make_inputs(B, n, n, H, 32, r, dtype, seed=n, bq=(True, False), bk=(True, False))]
     mask = None
     if low is not None:
@@ -1294,13 +1300,19 @@ def test_long_ragged_sequences(gpu_device, Lq, Lk, causal):
                                                  (16, 16, 700, 520, 32, False), (40, 16, 520, 700, 24, True)])
 def test_large_grids_ragged(gpu_device, B, H, Lq, Lk, r, causal):
     """Grids of at least two (causal: three) 256-query workgroups per compute unit of an MI355X
-    (256 CUs): the launchers then pick the two-query-blocks-per-wave kernels, which the small
-    cases above never reach; ragged last tiles, rectangular and causal shapes.  The last two are
-    windows whose last 256-query workgroup would be half empty: they take 128-query workgroups on a
-    grid that would otherwise get the large ones.  Ranks 32 and 24: four operand steps per score, the
-    widest forward that keeps two query blocks per wave."""
+    (256 CUs), ragged last tiles, rectangular and causal shapes: the streamlined kernels with two query blocks a wave, the dq
+    kernel with two at rank 16, and the kernels with one block a wave over many workgroups a compute unit.  Two are
+    windows whose last 256-query workgroup would be half empty."""
     assert B * H * ((Lq + 255) // 256) >= (3 if causal else 2) * 256
     _case(gpu_device, B, Lq, Lk, H, 32, r, torch.bfloat16, causal, seed=13)
+
+
+@pytest.mark.parametrize("B,H,Lq,Lk,r,causal", [(16, 16, 500, 300, 0, False), (24, 16, 500, 500, 16, True), (16, 16, 511, 333, 32, False), (16, 16, 500, 600, 8, False)])
+def test_large_grids_of_other_head_dims(gpu_device, B, H, Lq, Lk, r, causal):
+    """The same for head dim 24, which the forward of head dim 32 leaves to the general kernel: two query blocks a wave, at every
+    rank bucket that has them, the scale folded and not."""
+    assert B * H * ((Lq + 255) // 256) >= (3 if causal else 2) * 256
+    _case(gpu_device, B, Lq, Lk, H, 24, r, torch.bfloat16, causal, seed=13)
 
 
 @pytest.mark.parametrize("B,H,Lq,Lk,d,r,causal,dtype", [
