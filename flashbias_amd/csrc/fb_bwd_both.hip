@@ -92,7 +92,6 @@ static hipError_t launch_both_general(const BwdArgs &a0, hipStream_t stream) {
     if (e != hipSuccess) return e;
     const int group = a.group > 1 ? a.group : 1;
     const int64_t total = ((int64_t)a.ntiles_m + a.ntiles_n) * ((a.B + group - 1) / group) * a.H;
-    a.slots = slots_per_cu(kern, 256, lds, total, once);
     return launch_flat(kern, total, 256, lds, stream, a);
 }
 

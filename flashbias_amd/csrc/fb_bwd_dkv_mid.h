@@ -6,14 +6,14 @@
 // compiler asks for each fragment where it is used and waits for it, sixteen times a block: 4000 cycles for a wave that has a SIMD
 // to itself.  Here the reads of a phase are requested beside the products of the phase before, tiles of 128-byte rows and a dense
 // region for Q_b take half the copy instructions, and two stages leave the reads' addresses in two registers.  What is left is
-// two waves a SIMD (the accumulators and operands of 32 keys take 250 registers) that overlap their products and exponentials in
+// two waves a SIMD (the accumulators and operands of 32 keys take 213 to 256 registers) that overlap their products and exponentials in
 // part, and the copies (14 % without them, a fifth of it the clock).
 //
 // General kernel against this one, us: fp16 r16, 8 x 8 x (1000 x 1500) with a padding mask 118 -> 97 (training step 212 -> 190);
 // bf16 r16 B4 H16 L=2048 217 -> 190 (step 409 -> 387); r8 causal B2 H8 L=4096 147 -> 119 (306 -> 276); r2 as 16 without dk_bias,
 // causal B2 H16 L=2048 80 -> 59 (177 -> 156); r32 B1 H4 L=1000 54 -> 42 (106 -> 94).
 //
-// Head dim 32: three waves a SIMD (125 to 168 registers) cover for each other as in the general kernel; what counts is the dense
+// Head dim 32: three waves a SIMD (129 to 167 registers) cover for each other as in the general kernel; what counts is the dense
 // rows of 64 bytes, three or four copy instructions a wave and step for six or seven (the copies were a tenth of the cycles).
 // General kernel against this one, training step, us, bf16: r2 as 16 without dk_bias, causal B1 H50 L=4096 412 -> 399, L=8192 1448 ->
 // 1416, B2 H32 L=3000 306 -> 293; r16 B2 H4 L=8192 567 -> 555, B8 H16 L=700 100 -> 95; r32 768 x 4 rows of 768 2139 -> 2097, 301 x

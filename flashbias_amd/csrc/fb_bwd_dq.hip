@@ -674,8 +674,9 @@ __device__ __forceinline__ void bwd_dq_body(const BwdArgs &a, int wg) {
     }
 }
 
-// (One query block per wave and at most four operand steps fit 168 registers: a third wave per SIMD, which the
-// upper bound of the attribute has to allow; 768 x 4 rows of 768 tokens at rank 32: 0.80 -> 0.71 ms.)
+// (One query block per wave and at most four operand steps fit 168 registers: a third wave per SIMD, which the upper bound of
+// the attribute has to allow.  Unmasked calls of head dim 32 gained by it, before fb_bwd_dq_mid.h took them at rank 32; on the
+// small grids and vector masks that are left it is level, rank 32 2 x 8 x 4096 319 / 318 us a step.)
 template <class T, class C>
 __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::WAVES_EU + (C::QBLK == 1 && C::NK <= 4 && C::VEC && (!C::MASK || (C::VMASK && C::NKD <= 2)) ? 1 : 0), C::WAVES_EU + (C::QBLK == 1 && C::NK <= 4 ? 1 : 0)))) void
 bwd_dq_kernel(const BwdArgs a) {
@@ -697,11 +698,10 @@ static hipError_t launch_dq_qb(const BwdArgs &a0, hipStream_t stream) {
     return launch_flat(kern, total, C::NTHREADS, C::LDS_BYTES, stream, a);
 }
 
-// 256-query workgroups (two blocks per wave) once every compute unit has two of them (three under
-// a causal mask: B1 H50 d32 r16 at L=4096 0.162 -> 0.153 ms with the large ones, equal at L=8192 and
-// L=16384), 128-query workgroups below that and for short sequences whose last 256-query
-// workgroup would be half empty (8192 x 16 windows of 128 tokens: 2.59 -> 1.76 ms): as in the forward
-// launcher.
+// 256-query workgroups (two blocks per wave) once every compute unit has two of them (three under a causal mask), 128-query
+// workgroups below that and for short sequences whose last 256-query workgroup would be half empty (8192 x 16 windows of 128
+// tokens: 2.59 -> 1.76 ms): as in the forward launcher.  Training step with dq_bias, d32 r16, one block / two, us: 4 x 32 x
+// 1024 154.5 / 146.7, 2 x 32 x 1024 82.8 / 86.6, causal B1 H50 L=4096 442 / 431, L=8192 1623 / 1563.
 template <class T, int NKD, int NKR, bool VEC, int MASK, bool FOLD = false>
 static hipError_t launch_dq_vec(const BwdArgs &a, hipStream_t stream) {
     if constexpr (DqCfg<T, NKD, NKR, VEC, MASK, true>::QBLK == 2) {

@@ -31,7 +31,7 @@ struct DqMidCfg {
     // a stage, bytes: K, V, K_b rows of 32 or 64
     static constexpr int SK = BN * RB, SKB = NKR > 0 ? BN * CPR * 16 : 0, STAGE = 2 * SK + SKB;
     static constexpr int LDS_BYTES = 2 * STAGE;
-    // (head dim 32: 121-127 registers without dq_bias at ranks up to 16; with it, or at rank 32, 141-161)
+    // (head dim 32: 121-127 registers without dq_bias at ranks up to 16; at rank 32 129-135, with it 139-155)
     static constexpr int WAVES_EU = NKD == 4 ? 2 : BG || NKR == 2 ? 3 : 4;
     static_assert(WAVES_EU * LDS_BYTES <= 160 * 1024, "");
     static constexpr bool ORDERED = NKD == 4; // two waves a SIMD: the order is fixed phase by phase

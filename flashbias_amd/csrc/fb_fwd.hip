@@ -50,8 +50,9 @@ struct FwdCfg {
     static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES;
     // query blocks (of 32) per wave: two where the registers allow (head dim <= 32, rank <= 32:
     // 219-247 registers at four operand steps), so that every key / value fragment read from LDS
-    // feeds two blocks and two waves per SIMD carry four softmax streams (768 x 4 rows of 768
-    // tokens at rank 32: 0.77 -> 0.64 ms)
+    // feeds two blocks and two waves per SIMD carry four softmax streams (head dim 24, 8 x 32 x 1024, one
+    // block / two, us: rank 16 78 / 70.8, rank 32 89 / 76; head dim 32 itself is faster with four waves of one
+    // block per SIMD, fb_fwd_thin.h)
     static constexpr int QB = (QB2_ && NKD_ + NKR_ <= 4 && NDV_ == 1 && VEC_ && !XMASK) ? 2 : 1;
     static constexpr int BM = NWAVES * 32 * QB;
     static constexpr int NK = NKD + NKR;
@@ -595,14 +596,12 @@ static hipError_t launch_fwd_qb(const FwdArgs &a0, hipStream_t stream) {
     return launch_flat(kern, total, C::NTHREADS, C::LDS_BYTES, stream, a);
 }
 
-// Two query blocks per wave (256 queries per workgroup) pay once every compute unit has two such
-// workgroups; below that, 128-query workgroups at three waves per SIMD fill the chip better
-// (measured: 35 % faster at a quarter of that grid, 10 % slower at twice it).  Under a causal mask the
-// workgroups differ in length; with every XCD's share started longest first (work_order, fb_order.h) three
-// per compute unit are enough (B1 H50 d32 r16: 0.453 -> 0.434 ms at L=8192, 0.127 -> 0.125 at L=4096; while the
-// grid was walked head by head the small workgroups stayed ahead up to seven per compute unit).
-// Short sequences whose last 256-query workgroup would be half
-// empty also take the small ones (8192 x 16 windows of 128 tokens: 1.94 -> 1.41 ms).
+// Two query blocks per wave (256 queries per workgroup) pay once every compute unit has two such workgroups; below that,
+// 128-query workgroups at three waves per SIMD fill the chip better.  Head dim 24, rank 16, one block / two, us: 32 heads of
+// 1024 17.3 / 25.6, 64 23.1 / 26.2, 128 (where the line lies) 42.3 / 37.3, 256 78 / 70.8.  Under a causal mask the workgroups
+// differ in length; with every XCD's share started longest first (work_order, fb_order.h) three per compute unit are enough for
+// long sequences (48 heads of 4096 119 / 112.8, of 8192 421 / 405), not for many short ones (192 of 1024 36.9 / 44.2).  Short
+// sequences whose last 256-query workgroup would be half empty also take the small ones (8192 x 16 of 128 1150 / 1660).
 template <class T, int NKD, int NKR, int NDV, bool VEC, int MASK, bool FOLD = false>
 static hipError_t launch_fwd_vec(const FwdArgs &a, hipStream_t stream) {
     if constexpr (FwdCfg<T, NKD, NKR, NDV, VEC, MASK, true>::QB == 2) {

@@ -9,7 +9,7 @@
 // and leaves two or three waves a SIMD, which wait for LDS, for their own chains and, where a workgroup walks a few key
 // tiles, for its first tile at the same time: 1200 cycles a block at 384 keys and rank 32.  Here global_load_lds copies tiles
 // of 64 keys row-major into two stages, one tile ahead, V^T fragments come from transposing LDS reads, and no register
-// holds a tile or a fragment that is not in use: 88 to 126 of them, four workgroups a compute unit.
+// holds a tile or a fragment that is not in use: 97 to 127 of them, four workgroups a compute unit.
 //
 // General kernel against this one, us, bf16: rank 32, 384 x 4 rows of 384 with a padding mask 101 -> 78, 301 x 4 of 301 80 -> 53,
 // 512 x 4 of 512 163 -> 159, 768 x 4 of 768 528 -> 508 (masked 570 -> 551); rank 16, causal B1 H50 L=4096 137 -> 121, L=8192
