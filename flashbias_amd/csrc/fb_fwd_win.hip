@@ -15,16 +15,17 @@ namespace fb {
 // FOLD_: the scores are scale * (q k^T + q_b k_b^T) in one chain (no factors, or a scale of exactly 1).
 // MASK_: a matrix mask, whose blocks the wave that uses them copies to LDS one ahead.
 // NWAVES_: 4, or 8 for small grids of windows of more than 128 queries (launch_fwd_win_waves).
-template <class T, int NKR_, bool FOLD_, bool MASK_, int NWAVES_>
+// PAIR_: two blocks of 32 keys at a time (eight waves, and four without a mask above 64 keys).
+template <class T, int NKR_, bool FOLD_, bool MASK_, int NWAVES_, bool PAIR_>
 struct FwdWinCfg {
     static constexpr bool FOLD = FOLD_, MASK = MASK_;
     static constexpr int NKD = 2, NKR = NKR_, NK = NKD + NKR_;
     static constexpr int NWAVES = NWAVES_, NTHREADS = 64 * NWAVES, LK = 256;
     static constexpr bool ONE = 32 * NWAVES >= LK;     // one window a workgroup, one block of queries a wave: nothing is kept for the next
-    static constexpr bool PAIR = !MASK || NWAVES == 8; // two blocks of 32 keys at a time
+    static constexpr bool PAIR = PAIR_;
     static constexpr int TILE = PAIR ? 4096 : 2048;    // a wave's mask tile: 32 queries x 64 or 32 keys
     static constexpr int K = 0, V = K + LK * 64, KB = V + LK * 64, MT = KB + (NKR ? LK * 32 : 0), LDS_BYTES = MT + (MASK ? NWAVES * TILE : 0);
-    static constexpr int WAVES_EU = PAIR ? 4 : 3;
+    static constexpr int WAVES_EU = !MASK || PAIR ? 4 : 3;
     static_assert(NWAVES == 4 || NWAVES == 8, "");
     static_assert(WAVES_EU * 4 / NWAVES * LDS_BYTES <= 160 * 1024, "");
 };
@@ -56,7 +57,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     for (int bi = 0; bi < walk; ++bi) {
         const int b = __builtin_amdgcn_readfirstlane(bg * walk + bi);
         if (b >= a.B) break;
-        {   // K and V: 16 rows a copy instruction, whole blocks of 32 keys (past the end K's last row again, zeros for V)
+        {   // K and V: 16 rows a copy instruction, whole blocks of 32 keys (rows past the end: the last one again)
             const uint8_t *kbase = reinterpret_cast<const uint8_t *>(a.k.ptr + b * a.k.sb + h * a.k.sh);
             const uint8_t *vbase = reinterpret_cast<const uint8_t *>(a.v.ptr + b * a.v.sb + h * a.v.sh);
             int row, chunk;
@@ -66,11 +67,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                 const int i = wave + C::NWAVES * j, r = min(16 * i + row, a.Lk - 1);
                 if (i < 2 * nkb) {
                     lds_dma16_all((uint32_t)(r * (int)(a.k.ss * 2) + chunk * 16), kbase, lds0 + C::K + i * 1024);
-                    const uint32_t voff = (uint32_t)(r * (int)(a.v.ss * 2) + chunk * 16);
-                    if (16 * i + 16 <= a.Lk)
-                        lds_dma16_all(voff, vbase, lds0 + C::V + i * 1024);
-                    else
-                        lds_dma16_or_zero(voff, vbase, lds0 + C::V + i * 1024, lane, ~0ull, 16 * i + row < a.Lk);
+                    lds_dma16_all((uint32_t)(r * (int)(a.v.ss * 2) + chunk * 16), vbase, lds0 + C::V + i * 1024);
                 }
             }
             if constexpr (C::NKR > 0) {
@@ -120,6 +117,16 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             if (wave < nqb) copy_mask(wave, 0);
         }
         wait_vmcnt<0>();
+        if (a.Lk & 31) { // V past the end: zeros in place of the last row (lds_zero16), by the waves that copied there
+            int l = lane, row, chunk;
+            asm volatile("" : "+v"(l)); // (formed here)
+            lean_copy_place<4>(l, row, chunk);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int i = 2 * nkb - 2 + e;
+                if ((i & (C::NWAVES - 1)) == wave) lds_zero16(lds0 + C::V + i * 1024, l, 16 * i + row >= a.Lk);
+            }
+        }
         barrier_lds();
 
 #pragma unroll 1
@@ -133,11 +140,11 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 #pragma unroll
             for (int v = 0; v < 16; ++v) o[v] = 0.f;
             float m_ref = -INFINITY, m2 = 0.f, l_run = 0.f, slack = lag;
-            // N blocks of 32 keys from block kb on.  Without a mask two at a time (one row maximum, one test of the reference point and
-            // one set of addresses for 64 keys), the last of an odd number alone: 4096 x 16 windows of 256 tokens 1430 -> 1354 us,
-            // 769 x 16 of 144 148 -> 142, 64 x 16 of 256 28.7 -> 27.  Masked blocks alone with four waves: the copies of two
-            // would leave two workgroups a compute unit, and masks loaded to registers a pair ahead cost more (1024 x 16 of 256
-            // 473 -> 635).
+            // N blocks of 32 keys from block kb on.  In pairs two at a time (one test of the reference point and one set of addresses for
+            // 64 keys), the last of an odd number alone: 4096 x 16 windows of 256 tokens 1430 -> 1368 us, 128 x 16 of 144 28.3 -> 27.6,
+            // of 256 48.5 -> 45.5.  Masked blocks alone with four waves: the copies of two would leave two workgroups a compute unit,
+            // and masks loaded to registers a pair ahead cost more (1024 x 16 of 256 473 -> 635).  Up to 64 keys alone too: the one
+            // pair always moves its reference point (128 x 16 of 64 11.0, in a pair 11.7).
             auto group = [&](auto tag, int kb) __attribute__((always_inline)) {
                 constexpr int N = decltype(tag)::value;
                 const uint32_t at = kb * 2048;
@@ -275,9 +282,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     }
 }
 
-template <class T, int NKR, bool FOLD, bool MASK, int NWAVES>
+template <class T, int NKR, bool FOLD, bool MASK, int NWAVES, bool PAIR>
 static hipError_t launch_fwd_win_cfg(const FwdArgs &a, hipStream_t stream) {
-    typedef FwdWinCfg<T, NKR, FOLD, MASK, NWAVES> C;
+    typedef FwdWinCfg<T, NKR, FOLD, MASK, NWAVES, PAIR> C;
     auto kern = fwd_win_kernel<T, C>;
     static KernelOnce once;
     const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
@@ -305,7 +312,11 @@ template <class T, int NKR, bool FOLD, bool MASK>
 static hipError_t launch_fwd_win_waves(const FwdArgs &a, hipStream_t stream) {
     const int64_t windows = (int64_t)a.B * a.H;
     const bool wide = a.Lq > 128 && (windows <= 2 * (int64_t)num_cus() || ((MASK || a.Lq > 192) && windows <= 8 * (int64_t)num_cus()));
-    return wide ? launch_fwd_win_cfg<T, NKR, FOLD, MASK, 8>(a, stream) : launch_fwd_win_cfg<T, NKR, FOLD, MASK, 4>(a, stream);
+    if (wide) return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 8, true>(a, stream);
+    if constexpr (!MASK) {
+        if (a.Lk > 64) return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 4, true>(a, stream);
+    }
+    return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 4, false>(a, stream);
 }
 
 template <class T, int NKR>

@@ -178,7 +178,7 @@ inline bool ring_backward(const BwdArgs &a) {
 // Whether fb_fwd runs the forward for windows (fb_fwd_win.hip): whole sequences of at most 256 positions, head dim 32, a
 // rank up to 16, aligned tensors, no mask or a matrix mask of 16-byte chunks, a scale that keeps the order of the scores.
 // Against the general kernel, rank 16, us (window / general): 8192 pairs of 64 tokens 35 / 55, of 128 66 / 75, of 144
-// 107 / 183, with a matrix mask 47 / 84, 90 / 126, 149 / 318; 65536 of 256 1354 / 1572, masked 1904 / 2796; 512 pairs
+// 107 / 183, with a matrix mask 47 / 84, 90 / 126, 149 / 318; 65536 of 256 1368 / 1572, masked 1904 / 2796; 512 pairs
 // of 144 14 / 16, masked 16 / 24; 1024 of 256 26 / 33.  Where the general kernel has two workgroups a window (more than 128
 // queries) and these no longer find a compute unit each: 192 windows of 144 7.0 / 8.9, of 196 8.3 / 9.9, masked (144, 256)
 // 8.1 / 10.6, 10.7 / 12.0; 384 of 144 8.8 / 11.4, masked 10.4 / 17.5, 16.8 / 21.7.  Unmasked windows of eight blocks fill the general
