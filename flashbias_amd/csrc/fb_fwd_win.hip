@@ -131,11 +131,11 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 
 #pragma unroll 1
         for (int qb = wave; qb < nqb; qb += C::NWAVES) {
-            if (C::PAIR && !C::ONE && qb != wave) load_q(qb); // (a block ahead, as with a mask, it takes registers that pairs of blocks need)
+            if (C::PAIR && !C::ONE && qb != wave) load_q(qb); // (a block ahead, as below, it takes registers that pairs of blocks need)
             u32x4_t q[C::NK];
 #pragma unroll
             for (int t = 0; t < C::NK; ++t) q[t] = qn[t];
-            if (C::MASK && !C::PAIR && qb + C::NWAVES < nqb) load_q(qb + C::NWAVES);
+            if (!C::PAIR && qb + C::NWAVES < nqb) load_q(qb + C::NWAVES);
             f32x16_t o;
 #pragma unroll
             for (int v = 0; v < 16; ++v) o[v] = 0.f;
