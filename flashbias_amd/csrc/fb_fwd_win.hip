@@ -118,12 +118,12 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         }
         wait_vmcnt<0>();
         if (a.Lk & 31) { // V past the end: zeros in place of the last row (lds_zero16), by the waves that copied there
-            int l = lane, row, chunk;
-            asm volatile("" : "+v"(l)); // (formed here)
+            int l = lane, row, chunk, last = 2 * nkb - 2;
+            asm volatile("" : "+v"(l), "+s"(last)); // (formed here: ahead of the loop they cost every window's start)
             lean_copy_place<4>(l, row, chunk);
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
-                const int i = 2 * nkb - 2 + e;
+                const int i = last + e;
                 if ((i & (C::NWAVES - 1)) == wave) lds_zero16(lds0 + C::V + i * 1024, l, 16 * i + row >= a.Lk);
             }
         }
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             // 64 keys), the last of an odd number alone: 4096 x 16 windows of 256 tokens 1430 -> 1368 us, 128 x 16 of 144 28.3 -> 27.6,
             // of 256 48.5 -> 45.5.  Masked blocks alone with four waves: the copies of two would leave two workgroups a compute unit,
             // and masks loaded to registers a pair ahead cost more (1024 x 16 of 256 473 -> 635).  Up to 64 keys alone too: the one
-            // pair always moves its reference point (128 x 16 of 64 11.0, in a pair 11.7).
+            // pair always moves its reference point (128 x 16 of 64 11.2, in a pair 11.7).
             auto group = [&](auto tag, int kb) __attribute__((always_inline)) {
                 constexpr int N = decltype(tag)::value;
                 const uint32_t at = kb * 2048;
