@@ -612,6 +612,18 @@ static hipError_t launch_fwd_vec(const FwdArgs &a, hipStream_t stream) {
     return launch_fwd_qb<T, NKD, NKR, NDV, VEC, MASK, true, FOLD>(a, stream);
 }
 
+// Whether a call of head dim 32 takes fb_fwd_thin.h.  At rank 32 it reads its fragments where they are used, so that four
+// waves a SIMD fit; up to one workgroup a compute unit (causal: two) there are no other waves to wait with, and the general
+// kernel, which has the registers to read ahead, is faster.  us, general / this one: B1 H8 L=2048 32.9 / 38.6, L=4096 64.7 /
+// 74.9, B2 H16 L=512 11.2 / 12.6, with a padding mask B2 H8 L=1600 33.2 / 35.6; 384 workgroups 37.7 / 36.6 (B2 H16 L=1500);
+// causal B1 H16 L=1024 18.8 / 21.9, 512 workgroups 21.4 / 22.7 (B4 H16 L=1024), 600 32.6 / 32.6, 768 18.4 / 17.0 (B4 H32 L=600).
+// Between 129 and 192 keys the general kernel's second tile of 128 is half empty: causal B1 H8 L=160 7.5 / 7.1.
+template <int NKR>
+static bool thin_grid(const FwdArgs &a) {
+    const int64_t wgs = (int64_t)a.B * a.H * ((a.Lq + 127) / 128);
+    return NKR < 2 || wgs > (a.causal ? 2 : 1) * (int64_t)num_cus() || (a.Lk > 128 && a.Lk <= 192);
+}
+
 template <class T, int NKD, int NKR, int NDV>
 static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
     // the fast loader keeps the element offset of a tile row in 32 bits
@@ -624,8 +636,8 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
     // d64 r8 20.0 -> 17.3; fp16 d64 r16 8 x 8 x (1000 x 1500) with a vector mask 117 -> 49); a matrix mask needs its tile
     // in LDS, larger ranks more registers, and they stay with the general one.
     constexpr bool WIDE = NKD >= 4 && NKR <= 2;
-    // Head dim 32 exactly (its copies fill whole rows), ranks up to 32: fb_fwd_thin.h at every length and grid that the
-    // streamlined kernel does not take (both sides measured at the kernel).
+    // Head dim 32 exactly (its copies fill whole rows), ranks up to 32: fb_fwd_thin.h at every length that the streamlined
+    // kernel does not take, at rank 32 on grids that fill the chip (both sides measured at the kernel and at thin_grid).
     constexpr bool THIN = NKD == 2 && NKR <= 2;
     if constexpr (WIDE) {
         if (vec && a.mask.type == kVectorMask) return launch_fwd_wide<T, NKD, NKR, NDV, kVectorMask, false>(a, stream);
@@ -634,7 +646,7 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
                                                        : launch_fwd_wide<T, NKD, NKR, NDV, kNoMask, false>(a, stream);
     } else if (vec && a.mask.type == kVectorMask) {
         if constexpr (THIN) {
-            if (a.d == 32) return launch_fwd_thin<T, NKR, kVectorMask, false>(a, stream);
+            if (a.d == 32 && thin_grid<NKR>(a)) return launch_fwd_thin<T, NKR, kVectorMask, false>(a, stream);
         }
         // A vector mask on aligned tensors, other head dims and larger ranks, against the general masked instantiation: 384 x
         // 4 rows of 384 tokens, rank 32, 131 -> 114 us a call.  The outputs are bit for bit the same.
@@ -657,7 +669,7 @@ static hipError_t launch_fwd_cfg(const FwdArgs &a, hipStream_t stream) {
         }
     }
     if constexpr (THIN) {
-        if (vec && a.d == 32)
+        if (vec && a.d == 32 && thin_grid<NKR>(a))
             return fold_scale_ok<T>(a.scale, a.r, a.Lk) ? launch_fwd_thin<T, NKR, kNoMask, true>(a, stream)
                                                        : launch_fwd_thin<T, NKR, kNoMask, false>(a, stream);
     }

@@ -321,6 +321,30 @@ def test_thin_forward(gpu_device, r, Lq, Lk, scale, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("r,Lq,Lk,scale", [(32, 1, 1, None), (32, 127, 63, None), (24, 128, 65, 0.3), (32, 129, 128, 1.0), (24, 33, 193, -0.2),
+                                           (32, 100, 530, 0.0625)])
+def test_thin_forward_at_rank_32(gpu_device, r, Lq, Lk, scale, dtype):
+    """Ranks 17 to 32 take the kernel with four waves a SIMD on grids of more than a workgroup a compute unit (causal: two) and the
+    general one below: entries of a large call have the bits that they have in a small one, which passes the gate."""
+    B, H = 260, 4
+    assert B * H * ((Lq + 127) // 128) > 2 * 256
+    q, k, v, qb, kb, do = make_inputs(B, Lq, Lk, H, 32, r, dtype, seed=r + Lk)
+    for kind in (None, "causal", "mask"):
+        mask = None
+        if kind == "mask":
+            mask = torch.randn(B, 1, 1, Lk, generator=torch.Generator().manual_seed(Lk))
+            mask[1, ..., Lk - Lk // 4:] = float("-inf")
+            mask = mask.to(dtype if Lq % 2 else torch.float32)
+        dev = [t if t is None else t.to(gpu_device) for t in (q, k, v, qb, kb, mask)]
+        large = flash_bias_func(*dev, kind == "causal", scale)
+        small = [t if t is None else t[:2].contiguous() for t in (q, k, v, qb, kb, mask, do)]
+        ref = oracle(*small[:6], kind == "causal", scale, small[6])
+        got = run_gpu(flash_bias_func, *small[:6], kind == "causal", scale, small[6], gpu_device)
+        _gate(got, ref, dtype, o_by_magnitude=True)
+        assert torch.equal(large[:2].float().cpu(), got[0].float().cpu())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d,r,Lq,Lk,scale", [(64, 16, 1, 1, None), (64, 32, 63, 127, None), (40, 8, 64, 129, None), (64, 0, 65, 128, None), (56, 24, 600, 200, 0.125),
                                              (48, 16, 129, 33, 1.0), (64, 8, 127, 96, -0.1), (64, 0, 530, 64, -0.2), (64, 32, 200, 31, 0.0625),
                                              (64, 8, 520, 97, None)])
