@@ -170,14 +170,20 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             // (bitwise on purpose, as in the dq kernel: no scalar block between the last MFMA and the branch)
             const bool edge = (n0 + C::BN > a.Lk) | ((a.causal != 0) & (n0 + C::BN - 1 > wq0));
             if (edge) {
-                int key0 = n0 + 4 * g;
-                asm volatile("" : "+v"(key0)); // (computed here, not kept in registers across the loop)
+                // (without a mask one comparison a score.  With two, us, rank 16: causal B1 H64 L=256 8.6 for 8.0, L=512 12.2 for 11.6, B1 H8
+                // L=1024 17.75 for 17.3; the general kernel 8.1, 12.0, 17.7.  With a mask a last key in a register makes the compiler
+                // order the loop so that B1 H12 L=2500 takes 55 for 51.6.)
+                int key0 = n0 + 4 * g, last = a.causal ? min(query, a.Lk - 1) : a.Lk - 1;
+                if constexpr (C::VMASK)
+                    asm volatile("" : "+v"(key0)); // (computed here, not kept in registers across the loop)
+                else
+                    asm volatile("" : "+v"(key0), "+v"(last));
 #pragma unroll
                 for (int kb = 0; kb < C::KBLK; ++kb)
 #pragma unroll
                     for (int v = 0; v < 16; ++v) {
                         const int key = key0 + kb * 32 + 8 * (v >> 2) + (v & 3);
-                        if (key >= a.Lk || (a.causal && key > query)) s[kb][v] = -INFINITY;
+                        if (C::VMASK ? key >= a.Lk || (a.causal && key > query) : key > last) s[kb][v] = -INFINITY;
                     }
             }
             // (exponentials before another workgroup's products, which evens out who gets ahead: B2 H4 L=16384 r16 513 -> 475 us;
