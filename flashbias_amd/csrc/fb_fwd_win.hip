@@ -143,8 +143,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             // N blocks of 32 keys from block kb on.  In pairs two at a time (one test of the reference point and one set of addresses for
             // 64 keys), the last of an odd number alone: 4096 x 16 windows of 256 tokens 1430 -> 1368 us, 128 x 16 of 144 28.3 -> 27.6,
             // of 256 48.5 -> 45.5.  Masked blocks alone with four waves: the copies of two would leave two workgroups a compute unit,
-            // and masks loaded to registers a pair ahead cost more (1024 x 16 of 256 473 -> 635).  Up to 64 keys alone too: the one
-            // pair always moves its reference point (128 x 16 of 64 11.2, in a pair 11.7).
+            // and masks loaded to registers a pair ahead cost more (1024 x 16 of 256 473 -> 635).  Up to 128 keys alone too: the
+            // first pair always moves its reference point (64 x 16 of 64 tokens 7.5, in a pair 7.9, of 100 11.3 / 11.9, of 72 9.6 / 9.8,
+            // of 128 equal, 256 x 16 of 100 36.0 / 36.6).
             auto group = [&](auto tag, int kb) __attribute__((always_inline)) {
                 constexpr int N = decltype(tag)::value;
                 const uint32_t at = kb * 2048;
@@ -182,14 +183,21 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                     else
 #pragma unroll
                         for (int v = 0; v < 16; ++v) s[n][v] = 0.f;
+                    // (single blocks: the other chain's product between the two of q k^T; in pairs that spills)
+                    if constexpr (!C::FOLD && C::NKR > 0 && !C::PAIR) {
+                        s[n] = T::mfma(lds_load16(row_off[0] + C::K + at + n * 2048), q[0], s[n]);
+                        sb = T::mfma(lds_load16(kb_row + kb * 1024 + n * 1024), q[C::NKD], sb);
+                        s[n] = T::mfma(lds_load16(row_off[1] + C::K + at + n * 2048), q[1], s[n]);
+                    } else {
 #pragma unroll
-                    for (int t = 0; t < C::NKD; ++t) s[n] = T::mfma(lds_load16(row_off[t] + C::K + at + n * 2048), q[t], s[n]);
-                    if constexpr (C::NKR > 0) {
-                        const u32x4_t kf = lds_load16(kb_row + kb * 1024 + n * 1024);
-                        if constexpr (C::FOLD)
-                            s[n] = T::mfma(kf, q[C::NKD], s[n]);
-                        else
-                            sb = T::mfma(kf, q[C::NKD], sb);
+                        for (int t = 0; t < C::NKD; ++t) s[n] = T::mfma(lds_load16(row_off[t] + C::K + at + n * 2048), q[t], s[n]);
+                        if constexpr (C::NKR > 0) {
+                            const u32x4_t kf = lds_load16(kb_row + kb * 1024 + n * 1024);
+                            if constexpr (C::FOLD)
+                                s[n] = T::mfma(kf, q[C::NKD], s[n]);
+                            else
+                                sb = T::mfma(kf, q[C::NKD], sb);
+                        }
                     }
                     if constexpr (!C::FOLD) {
 #pragma unroll
@@ -229,15 +237,16 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
                     for (int v = 1; v < 16; ++v) mx[n] = fmaxf(mx[n], s[n][v]);
                 }
                 const float top = half_wave_max(N == 1 ? mx[0] : fmaxf(mx[0], mx[N - 1]));
-                const bool move = __any(top > m_ref + slack); // also true for the first finite score of a row
-                if (N == 1 && !C::PAIR && !move) slack = lag;
+                const bool above = top > m_ref + slack; // also true for the first finite score of a row
+                const bool move = __any(above);
+                if constexpr (N == 1) slack = above && !(kb & 1) ? 0.f : lag;
 #pragma unroll
                 for (int n = 0; n < N; ++n) {
                     if (move) {
                         if (n > 0) asm volatile("s_nop 11" : "+v"(o)); // (the first block's products)
                         const float m = N == 1 ? top : half_wave_max(mx[n]);
-                        const bool grow = m > m_ref + slack;
-                        slack = grow && (N == 1 ? !(kb & 1) : n == 0) ? 0.f : lag;
+                        const bool grow = N == 1 ? above : m > m_ref + slack;
+                        if constexpr (N > 1) slack = grow && n == 0 ? 0.f : lag;
                         const float m_new = grow ? m : m_ref;
                         const float alpha = grow ? fast_exp2((m_ref - m_new) * to_log2) : 1.f; // exp2(-inf) = 0
                         l_run *= alpha;
@@ -314,7 +323,7 @@ static hipError_t launch_fwd_win_waves(const FwdArgs &a, hipStream_t stream) {
     const bool wide = a.Lq > 128 && (windows <= 2 * (int64_t)num_cus() || ((MASK || a.Lq > 192) && windows <= 8 * (int64_t)num_cus()));
     if (wide) return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 8, true>(a, stream);
     if constexpr (!MASK) {
-        if (a.Lk > 64) return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 4, true>(a, stream);
+        if (a.Lk > 128) return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 4, true>(a, stream);
     }
     return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 4, false>(a, stream);
 }

@@ -932,9 +932,11 @@ def test_window_backward(gpu_device, dtype, B, H, Lq, Lk, r, scale, group, grads
     (torch.float16, 64, 8, 193, 8, 16, None, False, True), (torch.bfloat16, 64, 8, 136, 256, 0, None, False, False),
     (torch.bfloat16, 257, 8, 136, 120, 16, None, True, True), (torch.bfloat16, 257, 8, 250, 200, 16, None, True, False),
     (torch.float16, 257, 8, 130, 40, 8, 1.0, False, True), (torch.float16, 256, 8, 256, 256, 8, None, True, False),
-    # two blocks of queries a wave against single blocks of keys (up to 64), and one
+    # two blocks of queries a wave against single blocks of keys, and one
     (torch.bfloat16, 128, 8, 144, 64, 0, None, False, False), (torch.float16, 257, 8, 250, 64, 16, None, True, False),
-    (torch.bfloat16, 257, 8, 256, 33, 8, 1.0, False, False), (torch.bfloat16, 257, 8, 129, 20, 16, None, True, False)])
+    (torch.bfloat16, 257, 8, 256, 33, 8, 1.0, False, False), (torch.bfloat16, 257, 8, 129, 20, 16, None, True, False),
+    # up to four single blocks
+    (torch.float16, 257, 8, 250, 128, 16, None, True, False), (torch.bfloat16, 128, 8, 100, 97, 16, None, False, False), (torch.float16, 128, 8, 65, 72, 0, 0.2, False, False)])
 def test_window_forward(gpu_device, dtype, B, H, Lq, Lk, r, scale, shared, masked):
     """Forward of short sequences on grids of several workgroups per compute unit (fb_fwd_win.hip), o and lse against the
     oracle; a mask of -100 and -inf blocks (rows that see one key block only) and random values."""
