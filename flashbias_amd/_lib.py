@@ -15,6 +15,7 @@ FB_MASK_NONE, FB_MASK_VECTOR, FB_MASK_MATRIX = 0, 1, 2
 #: every symbol that include/flashbias.h declares
 EXPORTS = ("fb_version", "fb_init", "fb_last_error", "fb_bwd_workspace_bytes", "fb_suggest_bias_grad_group", "fb_check", "fb_fwd", "fb_bwd",
            "fb_sum_over_batch", "fb_resize_rank", "fb_resize_ranks", "fb_alibi_factors", "fb_cosine_workspace_bytes", "fb_cosine_fwd", "fb_cosine_bwd",
+           "fb_window_ready", "fb_window_workspace_bytes", "fb_window_fwd", "fb_window_bwd",
            "fb_weight_grad_workspace_bytes", "fb_weight_grad_recommended", "fb_weight_grad",
            "fb_project_recommended", "fb_project",
            "fb_bwd_preprocess", "fb_bwd_dkv", "fb_bwd_dq", "fb_bwd_static")
@@ -82,6 +83,11 @@ def load():
     lib.fb_resize_ranks.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64,
                                     ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
     lib.fb_resize_ranks.restype = ctypes.c_int
+    for name in ("fb_window_ready", "fb_window_fwd", "fb_window_bwd"):
+        getattr(lib, name).argtypes = [ctypes.POINTER(FbParams), ctypes.c_void_p, ctypes.c_int if name == "fb_window_ready" else ctypes.c_void_p]
+        getattr(lib, name).restype = ctypes.c_int
+    lib.fb_window_workspace_bytes.argtypes = [ctypes.POINTER(FbParams)]
+    lib.fb_window_workspace_bytes.restype = ctypes.c_size_t
     lib.fb_weight_grad_workspace_bytes.argtypes = [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int]
     lib.fb_weight_grad_workspace_bytes.restype = ctypes.c_size_t
     lib.fb_weight_grad_recommended.argtypes = [ctypes.c_int64, ctypes.c_int, ctypes.c_int]

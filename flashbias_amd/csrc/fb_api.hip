@@ -32,6 +32,7 @@ hipError_t launch_bwd_ring_f16_2(const BwdArgs &a, hipStream_t stream);
 
 // elementwise part of a cosine-attention window block (fb_cosine.hip)
 hipError_t launch_cosine(const fb_cosine *p, bool fp32, bool backward, hipStream_t stream);
+hipError_t launch_cosine_scale_grad(const fb_cosine *p, int shares, hipStream_t stream);
 int64_t cosine_sweep(int64_t tokens, int H, int d);
 
 // weight and bias gradient of a projection (fb_wgrad.hip)
@@ -328,6 +329,59 @@ int fb_cosine_bwd(const fb_cosine *p, void *stream) {
     const int rc = check_cosine(p, true);
     if (rc) return rc;
     return launched(fb::launch_cosine(p, cosine_fp32(p), true, static_cast<hipStream_t>(stream)), "fb_cosine_bwd");
+}
+
+// A cosine block's attention with the normalisation inside: q, k, v (and dq, dk, dv) of p are the parts of the projection c.qkv.
+static bool window_block(const fb_params *p, const fb_cosine *c, bool backward) {
+    return p->scale == 1.f && c->size >= offsetof(fb_cosine, fp32) && c->dtype == p->dtype && c->in_dtype == p->dtype && !cosine_fp32(c) &&
+           c->scale_dtype >= FB_F16 && c->scale_dtype <= FB_F32 && c->logit_scale && c->H == p->H && c->d == p->d &&
+           (backward ? fb::ring_shape(bwd_args(p)) && p->mask_type != FB_MASK_VECTOR : fb::window_shape(fwd_args(p)));
+}
+
+static int check_window(const fb_params *p, const fb_cosine *c, bool backward) {
+    if (!backward || !p || !fb::known_size(p)) {
+        const int rc = fb_check(p, backward);
+        if (rc) return rc;
+    } else { // (the scratch buffer is not used: any address will do for the check)
+        fb_params q;
+        std::memset(&q, 0, sizeof(q));
+        std::memcpy(&q, p, p->size);
+        q.delta = p->lse;
+        const int rc = fb_check(&q, 1);
+        if (rc) return rc;
+    }
+    if (!c) return fb::api_fail(FB_ERR_NULL, "fb_window: null pointer");
+    if (!window_block(p, c, backward)) return fb::api_fail(FB_ERR_SHAPE, "fb_window: not a block that fb_window_ready takes");
+    return FB_OK;
+}
+
+int fb_window_ready(const fb_params *p, const fb_cosine *c, int pass) { return check_window(p, c, pass == 1) == FB_OK ? 1 : 0; }
+
+size_t fb_window_workspace_bytes(const fb_params *p) {
+    if (!p || p->B <= 0 || p->H <= 0) return 0;
+    return (size_t)p->B * p->H * 4 * sizeof(float); // (a share of each wave; workgroups that walk several entries leave fewer)
+}
+
+int fb_window_fwd(const fb_params *p, const fb_cosine *c, void *stream) {
+    const int rc = check_window(p, c, false);
+    if (rc) return rc;
+    fb::FwdArgs a = fwd_args(p);
+    a.cosine = {c->logit_scale, c->scale_dtype};
+    return launched((p->dtype == FB_BF16 ? fb::launch_fwd_win_bf16_2 : fb::launch_fwd_win_f16_2)(a, static_cast<hipStream_t>(stream)), "fb_window_fwd");
+}
+
+int fb_window_bwd(const fb_params *p, const fb_cosine *c, void *stream) {
+    const int rc = check_window(p, c, true);
+    if (rc) return rc;
+    if (!c->dlogit_scale || !c->partial) return fb::api_fail(FB_ERR_NULL, "fb_window_bwd: null pointer");
+    fb::BwdArgs a = bwd_args(p);
+    a.cosine = {c->logit_scale, c->scale_dtype};
+    a.cosine_partial = c->partial;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    const int rc2 = launched(fb::launch_bwd_ring(a, p->dtype == FB_BF16, s), "fb_window_bwd");
+    if (rc2) return rc2;
+    const int walk = fb::ring_walk(a.B, a.H);
+    return launched(fb::launch_cosine_scale_grad(c, 4 * ((a.B + walk - 1) / walk), s), "fb_window_bwd (logit scale)");
 }
 
 static bool weight_grad_sizes(int64_t tokens, int n, int k) {

@@ -32,16 +32,23 @@ namespace fb {
 // one value per lane (key) or a matrix mask as a 32 x 32 tile per block, copied to LDS by the wave that uses it.
 // HIDE_: some wave's 64 keys are not all there, their scores are set to -inf (a branch on it inside the step cost 200
 // bytes of scratch).
-template <class T, int NKR_, bool FOLD_, int MASK_, bool HIDE_>
+// COS_: q and k are rows of a cosine block's projection, normalised here as in the forward (fb_unit.h), and dq and dk become the
+// projection's gradients where they are stored.  The rows of a dq block come from memory a second time, copied to where the block's
+// accumulator was while its last step runs, the rows of K are this wave's operand, and a row's norm and reciprocal are kept in LDS
+// (16 x 64 x 16 windows of 256 tokens with masks: both formed again from rows loaded at the end 1074 us, norms and K kept 1037, rows copied ahead
+// and bf16 quotients without a correction 1000).
+template <class T, int NKR_, bool FOLD_, int MASK_, bool HIDE_, bool COS_ = false>
 struct RingCfg {
-    static constexpr bool HIDE = HIDE_;
+    static constexpr bool HIDE = HIDE_, COS = COS_;
+    static_assert(FOLD_ || !COS_, "a cosine block's scale is 1");
     static constexpr bool FOLD = FOLD_, MASK = MASK_ == kMatrixMask, VMASK = MASK_ == kVectorMask;
     static constexpr int NKD = 2, NKR = NKR_, NK = NKD + NKR_;
     static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES, KBW = 2, LQ = 256, HALF = 128;
     // LDS, bytes: dense regions of 64-byte rows (Q, dO) and 32-byte rows (Q_b), the four accumulators of a half, a
     // dS block per wave, statistics, a mask tile per wave
     static constexpr int Q = 0, DO = Q + LQ * 64, QB = DO + LQ * 64, ACC = QB + (NKR ? LQ * 32 : 0), DS = ACC + 4 * 4096,
-                         STAT = DS + NWAVES * 2048, MT = STAT + 2 * LQ * 4, LDS_BYTES = MT + (MASK ? NWAVES * 2048 : 0);
+                         STAT = DS + NWAVES * 2048, MT = STAT + 2 * LQ * 4,
+                         NORM = MT + (MASK ? NWAVES * 2048 : 0), LDS_BYTES = NORM + (COS ? 4 * LQ * 4 + NTHREADS * 4 : 0); // (NORM: of Q's rows, of K's, then a thread's sum(dq * unit q))
     static_assert(LDS_BYTES <= 80 * 1024, "two workgroups per compute unit");
 };
 
@@ -67,6 +74,68 @@ __device__ __forceinline__ void store_block_rows(const Tensor &t, int b, int h, 
     }
 }
 
+// The same for the gradient g of unit rows n = x / |x|, which becomes that of x: s (g - n (n . g)) / |x|, as cosine_bwd_kernel forms it
+// from the rounded g.  The rows' n: this wave's operand `unit` (UNIT: K), or from the block's rows of x in LDS at `raw`, in the order of a copy
+// (Q, whose tile holds the products with the scale); `norms`: |x| of the block's rows and, 256 floats on, what they are multiplied
+// by.  Returns this lane's share of sum(g n).
+template <class T, bool UNIT>
+__device__ __forceinline__ float store_block_rows_unit(const Tensor &t, const u32x4_t (&unit)[2], const uint8_t *raw, const float *norms, int b, int h, int row0,
+                                                       int nrows, const f32x16_t &acc, float s, uint8_t *buf, int lane) {
+    asm volatile("" : "+v"(lane)); // (what derives from it is formed here, not kept in registers across the steps)
+    const int c = lane & 31, g = lane >> 5;
+    uint16_t *base = const_cast<uint16_t *>(t.ptr) + b * t.sb + h * t.sh;
+    int row, chunk;
+    lean_copy_place<4>(lane, row, chunk);
+    u32x4_t x[2];
+    if constexpr (UNIT) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) *reinterpret_cast<u32x4_t *>(buf + lean_chunk_off<4>(c, 2 * k + g)) = unit[k];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) x[j] = *reinterpret_cast<const u32x4_t *>(buf + j * 1024 + lane * 16);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) x[j] = *reinterpret_cast<const u32x4_t *>(raw + j * 1024 + lane * 16);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<u32x2_t *>(buf + lean_chunk_off<4>(c, j) + 8 * g) =
+            u32x2_t{T::pack2(acc[4 * j], acc[4 * j + 1]), T::pack2(acc[4 * j + 2], acc[4 * j + 3])};
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        float gr[8], n[8];
+        chunk_floats<T>(*reinterpret_cast<const u32x4_t *>(buf + j * 1024 + lane * 16), gr);
+        const int at = row0 + 16 * j + row;
+        const bool ok = at < nrows;
+        RowNorm r;
+        r.norm = norms[16 * j + row];
+        r.inv = norms[256 + 16 * j + row];
+        r.template finish<T>();
+        if constexpr (!UNIT) x[j] = chunk_unit<T>(x[j], r);
+        chunk_floats<T>(x[j], n);
+        float dot = 0.f;
+        if constexpr (!UNIT) { // (the scale's own gradient; k has none)
+            float mine = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                mine = __builtin_fmaf(gr[e], n[e], mine);
+                gr[e] *= s;
+            }
+            sum += ok ? mine : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot = __builtin_fmaf(gr[e], n[e], dot);
+        dot = quad_sum(dot);
+        if (r.norm < round16<T>(kNormEps)) dot = 0.f; // (a row of zeros: the clamped denominator is a constant)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) gr[e] = (gr[e] - n[e] * dot) * r.inv;
+        if (ok)
+            *reinterpret_cast<u32x4_t *>(base + (int64_t)at * t.ss + 8 * chunk) =
+                u32x4_t{T::pack2(gr[0], gr[1]), T::pack2(gr[2], gr[3]), T::pack2(gr[4], gr[5]), T::pack2(gr[6], gr[7])};
+    }
+    return sum;
+}
+
 template <class T, class C>
 __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_ring_kernel(const BwdArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -87,6 +156,12 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
     }
     const float to_log2 = C::FOLD ? a.scale * kLog2e : kLog2e;
     u32x4_t kbr[C::KBW][C::NKR > 0 ? C::NKR : 1]; // (kept across entries when the batch shares the factor)
+    float cos_scale = 1.f;
+    float *sNorm = reinterpret_cast<float *>(smem + C::NORM);
+    if constexpr (C::COS) {
+        cos_scale = scale_of_head(a.cosine, h);
+        sNorm[4 * C::LQ + threadIdx.x] = 0.f;
+    }
 
     for (int bi = 0; bi < walk; ++bi) {
         const int b = __builtin_amdgcn_readfirstlane(bg * walk + bi);
@@ -162,6 +237,14 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
 #pragma unroll
             for (int j = 0; j < 4; ++j) so[j] = *reinterpret_cast<const u32x4_t *>(orow + 8 * j);
             const float slse = a.lse[((int64_t)b * a.H + h) * a.Lq + row];
+            if constexpr (C::COS) {
+#pragma unroll
+                for (int kb = 0; kb < C::KBW; ++kb) {
+                    const RowNorm r = unit_operand<T>(kr[kb]);
+                    sNorm[2 * C::LQ + wk0 + 32 * kb + c] = r.norm;
+                    sNorm[3 * C::LQ + wk0 + 32 * kb + c] = r.inv;
+                }
+            }
             // K^T: this wave's rows of K through the first 16 KB of the accumulators (free until step 0, and the block
             // that this wave writes first)
             const uint32_t kst = lds0 + C::ACC + wave * 4096;
@@ -175,7 +258,22 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
                     kt[kb][t] = lds_load_tr(kst + lean_tr_addr4(c, g, 0) + (2 * kb + t) * 1024, kst + lean_tr_addr4(c, g, 1) + (2 * kb + t) * 1024);
-            wait_vmcnt<0>(); // this wave's copies have landed, among them row `tid` of dO
+            wait_vmcnt<0>(); // this wave's copies have landed, among them row `tid` of Q and dO
+            if constexpr (C::COS) {
+                u32x4_t x[4];
+                float sq[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    x[j] = lds_load16(lds0 + C::Q + lean_chunk_off<4>(tid, j));
+                    sq[j] = chunk_squares<T>(x[j]);
+                }
+                const RowNorm r = RowNorm::of<T>((sq[0] + sq[1]) + (sq[2] + sq[3]));
+                sNorm[tid] = r.norm;
+                sNorm[C::LQ + tid] = r.inv;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    *(__attribute__((address_space(3))) u32x4_t *)(lds0 + C::Q + lean_chunk_off<4>(tid, j)) = chunk_times<T>(chunk_unit<T>(x[j], r), cos_scale);
+            }
             float sum[2];
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
@@ -222,6 +320,19 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
                     const f32x4_t x = *reinterpret_cast<const f32x4_t *>(acc + 256 * j);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) dq[4 * j + e] = x[e];
+                }
+            }
+            // The raw rows of the block that this step completes, for store_block_rows_unit, to where its accumulator was.
+            if constexpr (C::COS) {
+                if ((step & 3) == 3 && r0 < a.Lq) {
+                    int row, chunk, l = lane;
+                    asm volatile("" : "+v"(l));
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (the accumulator has left LDS)
+                    lean_copy_place<4>(l, row, chunk);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        lds_dma16_all((uint32_t)(min(r0 + 16 * j + row, a.Lq - 1) * (int)(a.q.ss * 2) + chunk * 16),
+                                      reinterpret_cast<const uint8_t *>(a.q.ptr + b * a.q.sb + h * a.q.sh), lds0 + C::ACC + blk * 4096 + j * 1024);
                 }
             }
             if (visible && r0 < a.Lq) {
@@ -388,6 +499,11 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
             if ((step & 3) < 3) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4_t *>(acc + 256 * j) = f32x4_t{dq[4 * j], dq[4 * j + 1], dq[4 * j + 2], dq[4 * j + 3]};
+            } else if constexpr (C::COS) {
+                if (r0 < a.Lq) {
+                    wait_vmcnt<0>();
+                    sNorm[4 * C::LQ + threadIdx.x] += store_block_rows_unit<T, false>(a.dq, kr[0], smem + C::ACC + blk * 4096, sNorm + r0, b, h, r0, a.Lq, dq, cos_scale, smem + C::DS + wave * 2048, lane);
+                }
             } else {
                 store_block_rows<T>(a.dq, b, h, r0, a.Lq, dq, a.scale, smem + C::DS + wave * 2048, lane);
             }
@@ -398,27 +514,31 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
         for (int kb = 0; kb < C::KBW; ++kb) {
             asm volatile("s_nop 11" : "+v"(acc_dv[kb]), "+v"(acc_dk[kb]));
             store_block_rows<T>(a.dv, b, h, wk0 + 32 * kb, a.Lk, acc_dv[kb], 1.f, smem + C::DS + wave * 2048, lane);
-            store_block_rows<T>(a.dk, b, h, wk0 + 32 * kb, a.Lk, acc_dk[kb], a.scale, smem + C::DS + wave * 2048, lane);
+            if constexpr (C::COS) {
+                if (wk0 + 32 * kb < a.Lk)
+                    store_block_rows_unit<T, true>(a.dk, kr[kb], nullptr, sNorm + 2 * C::LQ + wk0 + 32 * kb, b, h, wk0 + 32 * kb, a.Lk, acc_dk[kb], 1.f, smem + C::DS + wave * 2048, lane);
+            } else {
+                store_block_rows<T>(a.dk, b, h, wk0 + 32 * kb, a.Lk, acc_dk[kb], a.scale, smem + C::DS + wave * 2048, lane);
+            }
         }
+    }
+    if constexpr (C::COS) { // this wave's share of the head's sum(dq * unit q), in a fixed order
+        float cos_sum = quad_sum(sNorm[4 * C::LQ + threadIdx.x]);
+#pragma unroll
+        for (int m = 4; m < 64; m <<= 1) cos_sum += __shfl_xor(cos_sum, m, 64);
+        if ((threadIdx.x & 63) == 0) a.cosine_partial[((int64_t)h * nbg + bg) * C::NWAVES + wave] = cos_sum;
     }
 }
 
-template <class T, int NKR, bool FOLD, int MASK, bool HIDE>
+template <class T, int NKR, bool FOLD, int MASK, bool HIDE, bool COS = false>
 static hipError_t launch_ring_cfg(const BwdArgs &a, hipStream_t stream) {
-    typedef RingCfg<T, NKR, FOLD, MASK, HIDE> C;
+    typedef RingCfg<T, NKR, FOLD, MASK, HIDE, COS> C;
     auto kern = bwd_ring_kernel<T, C>;
     static KernelOnce once;
     const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
     if (e != hipSuccess) return e;
     BwdArgs b = a;
-    b.walk = 1;
-    // Up to eight batch entries a workgroup (the factors and the cleared LDS are kept), as many as leave eight workgroups
-    // per compute unit: 4096 x 16 windows 2.96 ms with 32 entries, 2.90 with 16, 2.87 with 8, 2.86 with 4.
-    for (int w = 8; w > 1; w /= 2)
-        if ((int64_t)((a.B + w - 1) / w) * a.H >= 8 * (int64_t)num_cus()) {
-            b.walk = w;
-            break;
-        }
+    b.walk = ring_walk(a.B, a.H);
     return launch_flat(kern, (int64_t)((a.B + b.walk - 1) / b.walk) * a.H, C::NTHREADS, C::LDS_BYTES, stream, b);
 }
 
@@ -432,6 +552,12 @@ static hipError_t launch_ring_m(const BwdArgs &a, bool fold, hipStream_t stream)
 
 template <class T, int NKR>
 static hipError_t launch_ring_r(const BwdArgs &a, hipStream_t stream) {
+    if (a.cosine.ptr) {
+        const bool hide = a.Lk % 64 != 0;
+        if (a.mask.type == kMatrixMask)
+            return hide ? launch_ring_cfg<T, NKR, true, kMatrixMask, true, true>(a, stream) : launch_ring_cfg<T, NKR, true, kMatrixMask, false, true>(a, stream);
+        return hide ? launch_ring_cfg<T, NKR, true, kNoMask, true, true>(a, stream) : launch_ring_cfg<T, NKR, true, kNoMask, false, true>(a, stream);
+    }
     switch (a.mask.type) {
     // (a negative scale is not folded: it would turn the -inf of the keys past the end round)
     case kNoMask: return launch_ring_m<T, NKR, kNoMask>(a, (a.r == 0 && a.scale > 0.f) || a.scale == 1.f, stream);

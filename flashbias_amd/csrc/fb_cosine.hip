@@ -19,6 +19,7 @@
 // multiplies by 10 and more.  The backward rounds its results only.
 #include "flashbias.h"
 #include "fb_kernels.h"
+#include "fb_unit.h"
 
 namespace fb {
 
@@ -73,9 +74,6 @@ struct CosineArgs {
     int H, d;
     int sweep; // tokens per step of the grid
 };
-
-constexpr float kLogitMax = 4.6052f; // (swin_transformer_v2.py:180: log of 100)
-constexpr float kNormEps = 1e-12f;   // (torch.nn.functional.normalize)
 
 __device__ __forceinline__ float sum_over(float x, int lanes) { // over aligned groups of `lanes` (a power of two)
     for (int m = 1; m < lanes; m <<= 1) x += __shfl_xor(x, m, 64);
@@ -259,6 +257,20 @@ hipError_t launch_cosine(const fb_cosine *p, bool fp32, bool backward, hipStream
     case FB_F16: return bf16 ? launch_cosine_s<F16, BF16>(a, p->scale_dtype, fp32, backward, stream) : launch_cosine_s<F16, F16>(a, p->scale_dtype, fp32, backward, stream);
     case FB_BF16: return bf16 ? launch_cosine_s<BF16, BF16>(a, p->scale_dtype, fp32, backward, stream) : launch_cosine_s<BF16, F16>(a, p->scale_dtype, fp32, backward, stream);
     default: return bf16 ? launch_cosine_s<F32, BF16>(a, p->scale_dtype, fp32, backward, stream) : launch_cosine_s<F32, F16>(a, p->scale_dtype, fp32, backward, stream);
+    }
+}
+
+// The logit scale's gradient from `shares` partial sums a head (the ring backward's).
+hipError_t launch_cosine_scale_grad(const fb_cosine *p, int shares, hipStream_t stream) {
+    CosineArgs a = {};
+    a.logit_scale = p->logit_scale;
+    a.dlogit_scale = p->dlogit_scale;
+    a.partial = p->partial;
+    a.sweep = shares;
+    switch (p->scale_dtype) {
+    case FB_F16: return launch_flat(cosine_scale_grad_kernel<F16, false>, p->H, 256, 0, stream, a);
+    case FB_BF16: return launch_flat(cosine_scale_grad_kernel<BF16, false>, p->H, 256, 0, stream, a);
+    default: return launch_flat(cosine_scale_grad_kernel<F32, false>, p->H, 256, 0, stream, a);
     }
 }
 

@@ -16,9 +16,12 @@ namespace fb {
 // MASK_: a matrix mask, whose blocks the wave that uses them copies to LDS one ahead.
 // NWAVES_: 4, or 8 for small grids of windows of more than 128 queries (launch_fwd_win_waves).
 // PAIR_: two blocks of 32 keys at a time (eight waves, and four without a mask above 64 keys).
-template <class T, int NKR_, bool FOLD_, bool MASK_, int NWAVES_, bool PAIR_>
+// COS_: q and k are rows of a cosine block's projection, normalised here (fb_unit.h): K where its copies have landed in LDS, by
+// the wave that copied it, Q in the registers of the block that uses it.
+template <class T, int NKR_, bool FOLD_, bool MASK_, int NWAVES_, bool PAIR_, bool COS_ = false>
 struct FwdWinCfg {
-    static constexpr bool FOLD = FOLD_, MASK = MASK_;
+    static constexpr bool FOLD = FOLD_, MASK = MASK_, COS = COS_;
+    static_assert(FOLD_ || !COS_, "a cosine block's scale is 1");
     static constexpr int NKD = 2, NKR = NKR_, NK = NKD + NKR_;
     static constexpr int NWAVES = NWAVES_, NTHREADS = 64 * NWAVES, LK = 256;
     static constexpr bool ONE = 32 * NWAVES >= LK;     // one window a workgroup, one block of queries a wave: nothing is kept for the next
@@ -53,6 +56,8 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     const uint32_t col_off[2] = {lds0 + C::V + lean_tr_addr4(c, g, 0), lds0 + C::V + lean_tr_addr4(c, g, 1)};
     const uint32_t kb_row = lds0 + C::KB + lean_row_addr<2>(c, g);
     const uint32_t lds_m = lds0 + C::MT + wave * C::TILE;
+    float cos_scale = 1.f;
+    if constexpr (C::COS) cos_scale = scale_of_head(a.cosine, h);
 
     for (int bi = 0; bi < walk; ++bi) {
         const int b = __builtin_amdgcn_readfirstlane(bg * walk + bi);
@@ -117,6 +122,30 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             if (wave < nqb) copy_mask(wave, 0);
         }
         wait_vmcnt<0>();
+        if constexpr (C::COS) { // a row of this wave's by 64 / ROWS lanes
+            constexpr int ROWS = C::LK / C::NWAVES, LPR = 64 / ROWS, CH = 4 / LPR;
+            int l = lane;
+            asm volatile("" : "+v"(l)); // (formed here, not kept in registers across the blocks)
+            const int row = 16 * (wave + C::NWAVES * (l / LPR / 16)) + (l / LPR & 15);
+            if (row < 32 * nkb) {
+                u32x4_t x[CH];
+                float sq[CH];
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    x[j] = lds_load16(lds0 + C::K + lean_chunk_off<4>(row, CH * (l % LPR) + j));
+                    sq[j] = chunk_squares<T>(x[j]);
+                }
+                float sum = sq[0] + sq[1];
+                if constexpr (CH == 4)
+                    sum += sq[2] + sq[3];
+                else
+                    sum += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, sum), 0xB1, 0xf, 0xf, true)); // lane ^ 1
+                const RowNorm r = RowNorm::of<T>(sum);
+#pragma unroll
+                for (int j = 0; j < CH; ++j)
+                    *(__attribute__((address_space(3))) u32x4_t *)(lds0 + C::K + lean_chunk_off<4>(row, CH * (l % LPR) + j)) = chunk_unit<T>(x[j], r);
+            }
+        }
         if (a.Lk & 31) { // V past the end: zeros in place of the last row (lds_zero16), by the waves that copied there
             int l = lane, row, chunk, last = 2 * nkb - 2;
             asm volatile("" : "+v"(l), "+s"(last)); // (formed here: ahead of the loop they cost every window's start)
@@ -136,6 +165,12 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 #pragma unroll
             for (int t = 0; t < C::NK; ++t) q[t] = qn[t];
             if (!C::PAIR && qb + C::NWAVES < nqb) load_q(qb + C::NWAVES);
+            if constexpr (C::COS) {
+                u32x4_t x[2] = {q[0], q[1]};
+                unit_operand<T>(x);
+                q[0] = chunk_times<T>(x[0], cos_scale);
+                q[1] = chunk_times<T>(x[1], cos_scale);
+            }
             f32x16_t o;
 #pragma unroll
             for (int v = 0; v < 16; ++v) o[v] = 0.f;
@@ -291,9 +326,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     }
 }
 
-template <class T, int NKR, bool FOLD, bool MASK, int NWAVES, bool PAIR>
+template <class T, int NKR, bool FOLD, bool MASK, int NWAVES, bool PAIR, bool COS>
 static hipError_t launch_fwd_win_cfg(const FwdArgs &a, hipStream_t stream) {
-    typedef FwdWinCfg<T, NKR, FOLD, MASK, NWAVES, PAIR> C;
+    typedef FwdWinCfg<T, NKR, FOLD, MASK, NWAVES, PAIR, COS> C;
     auto kern = fwd_win_kernel<T, C>;
     static KernelOnce once;
     const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
@@ -317,19 +352,21 @@ static hipError_t launch_fwd_win_cfg(const FwdArgs &a, hipStream_t stream) {
 // 22.9 / 20.0, 35.6 / 31.3; 2048 of 256 47.1 / 45.4, with a mask 37.6 / 35.8, 57.0 / 54.6.  Without a mask and with at most six blocks of
 // queries the idle waves count from 512 windows on (1024 of 144 15.5 / 16.7, 2048 28.2 / 30.2), above 2048 windows they do
 // everywhere (3072 of 144 with a mask 49.6 / 51.1, 8192 of 256 241 / 245).
-template <class T, int NKR, bool FOLD, bool MASK>
+template <class T, int NKR, bool FOLD, bool MASK, bool COS = false>
 static hipError_t launch_fwd_win_waves(const FwdArgs &a, hipStream_t stream) {
     const int64_t windows = (int64_t)a.B * a.H;
     const bool wide = a.Lq > 128 && (windows <= 2 * (int64_t)num_cus() || ((MASK || a.Lq > 192) && windows <= 8 * (int64_t)num_cus()));
-    if (wide) return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 8, true>(a, stream);
+    if (wide) return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 8, true, COS>(a, stream);
     if constexpr (!MASK) {
-        if (a.Lk > 128) return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 4, true>(a, stream);
+        if (a.Lk > 128) return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 4, true, COS>(a, stream);
     }
-    return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 4, false>(a, stream);
+    return launch_fwd_win_cfg<T, NKR, FOLD, MASK, 4, false, COS>(a, stream);
 }
 
 template <class T, int NKR>
 static hipError_t launch_fwd_win_r(const FwdArgs &a, hipStream_t stream) {
+    if (a.cosine.ptr)
+        return a.mask.type == kMatrixMask ? launch_fwd_win_waves<T, NKR, true, true, true>(a, stream) : launch_fwd_win_waves<T, NKR, true, false, true>(a, stream);
     if (a.mask.type == kMatrixMask) // (the mask is not divided by the scale)
         return a.scale == 1.f ? launch_fwd_win_waves<T, NKR, true, true>(a, stream) : launch_fwd_win_waves<T, NKR, false, true>(a, stream);
     return a.r == 0 || a.scale == 1.f ? launch_fwd_win_waves<T, NKR, true, false>(a, stream) : launch_fwd_win_waves<T, NKR, false, false>(a, stream);

@@ -8,6 +8,7 @@
 #include <stdint.h>
 
 #include "fb_device.h"
+#include "fb_unit.h"
 
 namespace fb {
 
@@ -20,6 +21,7 @@ struct FwdArgs {
     float scale;
     int ntiles_m; // query tiles per (batch, head)
     int slots;    // workgroups of this launch that share a compute unit (priority turn-taking)
+    LogitScale cosine; // window forward: q and k are a projection's, their rows are normalised here (scale 1)
 };
 
 struct BwdArgs {
@@ -38,6 +40,8 @@ struct BwdArgs {
     int stat_chunks; // writers of the scratch buffer: also store the statistics chunks (dkv_streamlined())
     int group; // > 1: a workgroup serves this many consecutive batch entries and sums their factor gradients (row b / group)
     int walk;  // window backward without such sums: batch entries a workgroup walks (set by its launcher)
+    LogitScale cosine;     // ring backward: as in the forward; dq and dk are the projection's gradients
+    float *cosine_partial; // (H, workgroups of a head, 4): shares of sum(dq * unit q)
 };
 
 // Each returns hipSuccess or the launch error.  `bf16` selects the element type.
@@ -136,13 +140,15 @@ inline bool mixed_general_backward(const BwdArgs &a0);
 // What the two one-launch backwards below share: whole sequences of at most 256 positions, head dim 32, rank a multiple of 8 up
 // to 32, aligned tensors, no causal mask, no fp32 mask (the mask is read element-wise, any strides), and at least one workgroup
 // per compute unit.  Such sequences are bound by memory traffic, and the two-kernel backward reads q, k, v, o and dO twice.
-inline bool short_sequences(const BwdArgs &a) {
+inline bool short_shape(const BwdArgs &a) {
     const int64_t lim = (int64_t)1 << 22; // (32-bit byte offsets of 256 tile rows)
-    const int group = a.group > 1 ? a.group : 1;
     return (a.mask.type == 0 || (!a.mask.is_f32 && a.mask.sm < lim)) && !a.causal && a.d == 32 && a.r % 8 == 0 && a.r <= 32 && a.Lq <= 256 && a.Lk <= 256 &&
            a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.o.vec_ok && a.dout.vec_ok && (a.r == 0 || (a.qb.vec_ok && a.kb.vec_ok)) &&
-           a.q.ss < lim && a.k.ss < lim && a.dout.ss < lim && (a.r == 0 || (a.qb.ss < lim && a.kb.ss < lim)) &&
-           (int64_t)((a.B + group - 1) / group) * a.H >= num_cus();
+           a.q.ss < lim && a.k.ss < lim && a.dout.ss < lim && (a.r == 0 || (a.qb.ss < lim && a.kb.ss < lim));
+}
+inline bool short_sequences(const BwdArgs &a) {
+    const int group = a.group > 1 ? a.group : 1;
+    return short_shape(a) && (int64_t)((a.B + group - 1) / group) * a.H >= num_cus();
 }
 
 // Whether fb_bwd runs the window kernel (fb_bwd_win.hip: one workgroup per (batch, head) forms the per-query
@@ -169,10 +175,19 @@ inline bool mask_in_chunks(const MaskDesc &m, int Lk) {
 // 165 / 236, 183 / 275, with a matrix mask 124 / 193, 193 / 306, 222 / 338, with a vector mask 110 / 187, 168 / 237, 188 / 281;
 // 1024 x 16 of 16 157 / 238.  It is ahead on every grid; below four workgroups per compute unit, where that is some microseconds,
 // the window kernel keeps dq, dk and dv bit for bit those of the call that computes the factor gradients too.
-inline bool ring_backward(const BwdArgs &a) {
-    if (!short_sequences(a) || a.r > 16 || (a.r > 0 && a.dqb.ptr) || (int64_t)a.B * a.H < 4 * (int64_t)num_cus()) return false;
+inline bool ring_shape(const BwdArgs &a) {
+    if (!short_shape(a) || a.r > 16 || (a.r > 0 && a.dqb.ptr)) return false;
     if (!(a.dq.vec_ok && a.dk.vec_ok && a.dv.vec_ok)) return false; // (it stores whole 16-byte chunks)
     return a.mask.type != kMatrixMask || mask_in_chunks(a.mask, a.Lk);
+}
+inline bool ring_backward(const BwdArgs &a) { return ring_shape(a) && short_sequences(a) && (int64_t)a.B * a.H >= 4 * (int64_t)num_cus(); }
+
+// Batch entries a workgroup of the ring kernel walks (the factors and the cleared LDS are kept): up to eight, as many as leave eight workgroups
+// per compute unit: 4096 x 16 windows 2.96 ms with 32 entries, 2.90 with 16, 2.87 with 8, 2.86 with 4.
+inline int ring_walk(int B, int H) {
+    for (int w = 8; w > 1; w /= 2)
+        if ((int64_t)((B + w - 1) / w) * H >= 8 * (int64_t)num_cus()) return w;
+    return 1;
 }
 
 // Whether fb_fwd runs the forward for windows (fb_fwd_win.hip): whole sequences of at most 256 positions, head dim 32, a
@@ -183,12 +198,15 @@ inline bool ring_backward(const BwdArgs &a) {
 // queries) and these no longer find a compute unit each: 192 windows of 144 7.0 / 8.9, of 196 8.3 / 9.9, masked (144, 256)
 // 8.1 / 10.6, 10.7 / 12.0; 384 of 144 8.8 / 11.4, masked 10.4 / 17.5, 16.8 / 21.7.  Unmasked windows of eight blocks fill the general
 // kernel's workgroups: 384 of 256 13.3 / 12.3, 512 14.4 / 15.5; at most 128 queries are one workgroup there too (equal).
-inline bool window_forward(const FwdArgs &a) {
+inline bool window_shape(const FwdArgs &a) {
     const int64_t lim = (int64_t)1 << 22; // (32-bit byte offsets of 256 rows)
     if (a.d != 32 || a.r > 16 || a.r % 8 != 0 || a.Lq > 256 || a.Lk > 256 || a.causal || !(a.scale > 1e-6f && a.scale < 1e6f)) return false;
     if (!(a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.o.vec_ok && a.k.ss < lim && a.v.ss < lim)) return false;
     if (a.r > 0 && !(a.qb.vec_ok && a.kb.vec_ok && a.kb.ss < lim)) return false;
-    if (a.mask.type != kNoMask && !mask_in_chunks(a.mask, a.Lk)) return false;
+    return a.mask.type == kNoMask || mask_in_chunks(a.mask, a.Lk);
+}
+inline bool window_forward(const FwdArgs &a) {
+    if (!window_shape(a)) return false;
     const int64_t windows = (int64_t)a.B * a.H;
     if (a.Lq > 128 && (a.mask.type != kNoMask || a.Lq <= 224)) return 4 * windows >= 3 * (int64_t)num_cus();
     return windows >= 2 * (int64_t)num_cus();

@@ -217,11 +217,13 @@ struct FlashBiasFn : public torch::autograd::Function<FlashBiasFn> {
     }
 };
 
-// The attention core of a cosine-attention window block on its packed projection qkv (windows, n, 3 H d): unit q and
-// k and the logit scale in one pass (fb_cosine_fwd), the operator on them and on v where it lies, and backward the
-// operator's gradients written into the packed gradient, where one more pass (fb_cosine_bwd) turns dq and dk into
-// those of the projection.  (As tensor operations: about 40 passes over tensors of that size, and the split of the
-// packed tensor comes back as three zero-filled copies added up.)  `mask` (nW, n, n) or none, one per window of an image.
+// The attention core of a cosine-attention window block on its packed projection qkv (windows, n, 3 H d).  Where the window kernels
+// take the call (fb_window_ready) they normalise q and k themselves and the backward writes the packed gradient: one launch
+// forward, one and a sum of the logit scale's shares backward.  Else unit q and k and the logit scale in one pass (fb_cosine_fwd),
+// the operator on them and on v where it lies, and backward the operator's gradients written into the packed gradient, where one
+// more pass (fb_cosine_bwd) turns dq and dk into those of the projection.  (As tensor operations: about 40 passes over tensors of
+// that size, and the split of the packed tensor comes back as three zero-filled copies added up.)  `mask` (nW, n, n) or none, one
+// per window of an image.
 struct WindowFn : public torch::autograd::Function<WindowFn> {
     static fb_cosine cosine(const Tensor &qkv, const Tensor &logit_scale, int64_t heads, c10::ScalarType type, bool autocast) {
         fb_cosine a;
@@ -244,6 +246,18 @@ struct WindowFn : public torch::autograd::Function<WindowFn> {
         return packed.as_strided({B, n, heads, dim / heads}, {n * 3 * dim, 3 * dim, dim / heads, 1}, packed.storage_offset() + which * dim);
     }
 
+    // c.q and c.k (and c.v, if allocated): the normalised rows in memory
+    static void unit_rows(fb_cosine a, Call &c, const Tensor &qkv, c10::ScalarType type, int64_t heads, bool convert) {
+        const int64_t B = qkv.size(0), n = qkv.size(1), d = qkv.size(2) / (3 * heads);
+        c.q = fresh({B, n, heads, d}, type, qkv.device());
+        c.k = fresh({B, n, heads, d}, type, qkv.device());
+        a.q = c.q.data_ptr();
+        a.k = c.k.data_ptr();
+        a.v = convert ? c.v.data_ptr() : nullptr;
+        const c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
+        check(fb_cosine_fwd(&a, stream_of(qkv)));
+    }
+
     static Tensor forward(AutogradContext *ctx, const Tensor &qkv, const Tensor &logit_scale, const Tensor &qb, const Tensor &kb,
                           const c10::optional<Tensor> &mask_in, int64_t heads, int64_t dtype) {
         const auto type = (c10::ScalarType)dtype;
@@ -252,8 +266,6 @@ struct WindowFn : public torch::autograd::Function<WindowFn> {
         const bool autocast = at::autocast::is_autocast_enabled(at::kCUDA);
         fb_cosine a = cosine(qkv, logit_scale, heads, type, autocast);
         Call c;
-        c.q = fresh({B, n, heads, d}, type, qkv.device());
-        c.k = fresh({B, n, heads, d}, type, qkv.device());
         const bool convert = qkv.scalar_type() != type;
         c.v = convert ? fresh({B, n, heads, d}, type, qkv.device()) : part(qkv, 2, heads);
         c.qb = qb;
@@ -266,17 +278,27 @@ struct WindowFn : public torch::autograd::Function<WindowFn> {
             TORCH_CHECK(c.mask.dim() == 4 && c.mask.size(0) > 0 && B % c.mask.size(0) == 0, "the windows must be a multiple of the mask's");
             c.mask_batches = (int)c.mask.size(0);
         }
-        a.q = c.q.data_ptr();
-        a.k = c.k.data_ptr();
-        a.v = convert ? c.v.data_ptr() : nullptr;
-        {
-            const c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
-            check(fb_cosine_fwd(&a, stream_of(qkv)));
-        }
-        const auto [o, lse] = attend(c);
-        ctx->save_for_backward({qkv, logit_scale, c.q, c.k, convert ? c.v : Tensor(), o, lse, qb, kb, c.mask});
         ctx->saved_data["heads"] = heads;
         ctx->saved_data["autocast"] = autocast;
+        ctx->saved_data["dtype"] = dtype;
+        // (constant factors: their gradients need the normalised rows in memory)
+        if (!convert && !autocast && !qb.requires_grad() && !kb.requires_grad()) {
+            c.q = part(qkv, 0, heads);
+            c.k = part(qkv, 1, heads);
+            fb_params p = block(c);
+            const Tensor o = fresh({B, n, heads, d}, type, qkv.device()), lse = fresh({B, heads, n}, torch::kFloat32, qkv.device());
+            p.o = t4(o);
+            p.lse = lse.data_ptr<float>();
+            if (fb_window_ready(&p, &a, 0)) {
+                const c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
+                check(fb_window_fwd(&p, &a, stream_of(qkv)));
+                ctx->save_for_backward({qkv, logit_scale, Tensor(), Tensor(), Tensor(), o, lse, qb, kb, c.mask});
+                return o;
+            }
+        }
+        unit_rows(a, c, qkv, type, heads, convert);
+        const auto [o, lse] = attend(c);
+        ctx->save_for_backward({qkv, logit_scale, c.q, c.k, convert ? c.v : Tensor(), o, lse, qb, kb, c.mask});
         return o;
     }
 
@@ -299,9 +321,29 @@ struct WindowFn : public torch::autograd::Function<WindowFn> {
             dk = part(dqkv, 1, heads);
             dv = part(dqkv, 2, heads);
         }
-        const auto [dqb, dkb] = attend_backward(c, saved[5], saved[6], grads[0], dq, dk, dv, ctx->needs_input_grad(2) || ctx->needs_input_grad(3));
-        fb_cosine a = cosine(qkv, logit_scale, heads, c.q.scalar_type(), ctx->saved_data["autocast"].toBool());
+        const auto type = (c10::ScalarType)ctx->saved_data["dtype"].toInt();
+        fb_cosine a = cosine(qkv, logit_scale, heads, type, ctx->saved_data["autocast"].toBool());
         Tensor dscale = fresh_like(logit_scale);
+        if (!c.q.defined()) {
+            c.q = part(qkv, 0, heads);
+            c.k = part(qkv, 1, heads);
+            const Tensor dout = channel_contiguous(grads[0]);
+            fb_params p = block(c);
+            p.o = t4(saved[5]);
+            p.lse = saved[6].data_ptr<float>();
+            p.dout = t4(dout);
+            p.dq = t4(dq); p.dk = t4(dk); p.dv = t4(dv);
+            if (fb_window_ready(&p, &a, 1)) {
+                const Tensor partial = fresh({(int64_t)(fb_window_workspace_bytes(&p) / 4)}, torch::kFloat32, qkv.device());
+                a.partial = partial.data_ptr<float>();
+                a.dlogit_scale = dscale.data_ptr();
+                const c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
+                check(fb_window_bwd(&p, &a, stream_of(qkv)));
+                return {dqkv, dscale, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+            }
+            unit_rows(a, c, qkv, type, heads, false); // (a gradient or a saved tensor in rows these kernels do not read)
+        }
+        const auto [dqb, dkb] = attend_backward(c, saved[5], saved[6], grads[0], dq, dk, dv, ctx->needs_input_grad(2) || ctx->needs_input_grad(3));
         Tensor partial = fresh({(int64_t)(fb_cosine_workspace_bytes(&a) / 4)}, torch::kFloat32, qkv.device());
         a.dq = dq.data_ptr();
         a.dk = dk.data_ptr();

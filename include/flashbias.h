@@ -253,6 +253,18 @@ size_t fb_cosine_workspace_bytes(const fb_cosine *p);
 int fb_cosine_fwd(const fb_cosine *p, void *stream);
 int fb_cosine_bwd(const fb_cosine *p, void *stream);
 
+/* The attention of such a block with the normalisation inside the attention kernels: q, k, v (and dq, dk, dv) of `p` are the
+ * parts of the packed projection c->qkv (c->dqkv) itself, o and lse those of the attention on the normalised rows, scale 1, no
+ * factor gradients.  The backward reads the projection again, writes the projection's gradient and dlogit_scale, and takes
+ * c->partial of fb_window_workspace_bytes() bytes; p->delta is not used, and neither are the other pointers of `c`.  The bits are those of fb_cosine_fwd, fb_fwd, the ring
+ * backward and fb_cosine_bwd one after the other (dlogit_scale: another order of the same sum).
+ * fb_window_ready (pass: 0 = forward, 1 = backward): 1 for the calls these take: head dim 32, at most 256 positions, rank up to
+ * 16, one 16-bit type, fp32 = 0, aligned tensors, no mask or a matrix mask of 16-byte chunks; the others return FB_ERR_SHAPE. */
+int fb_window_ready(const fb_params *p, const fb_cosine *c, int pass);
+size_t fb_window_workspace_bytes(const fb_params *p);
+int fb_window_fwd(const fb_params *p, const fb_cosine *c, void *stream);
+int fb_window_bwd(const fb_params *p, const fb_cosine *c, void *stream);
+
 /* Weight and bias gradient of a projection y = x w^T + b, the products around the attention of a block
  * (swin_transformer_v2.py:155-207), for many tokens and a small weight: dw (n, k) = dy^T x and db (n) = the column sums
  * of dy, both contiguous in the input dtype, accumulated in fp32 in a fixed order and rounded once; db NULL: not wanted.

@@ -145,6 +145,111 @@ def test_cosine_forward_has_the_bits_of_tensor_operations(gpu_device, in_dtype, 
             assert (g.float() - w.float()).abs().max() <= 2.0 ** -6 * w.float().abs().max(), name
 
 
+def _window_params(qkv, qb, kb, mask, heads, o, lse):
+    """fb_params of the attention of a window block whose q, k, v are the parts of the packed projection (windows, n, 3 H d)."""
+    windows, n, dim = qkv.shape[0], qkv.shape[1], qkv.shape[2] // 3
+    p = _lib.new_params()
+    p.dtype, p.B, p.H, p.Lq, p.Lk, p.d, p.r, p.scale = CODES[qkv.dtype], windows, heads, n, n, dim // heads, qb.shape[3], 1.0
+    packed = lambda t, i: _lib.FbTensor(t.data_ptr() + 2 * dim * i, 3 * n * dim, dim // heads, 3 * dim)
+    p.q, p.k, p.v = (packed(qkv, i) for i in range(3))
+    p.q_bias, p.k_bias = (_lib.FbTensor(t.data_ptr(), 0, t.stride(2), t.stride(1)) for t in (qb, kb))
+    if mask is not None:
+        p.mask_type, p.mask_dtype, p.mask_batches = 2, CODES[mask.dtype], mask.shape[0]
+        p.mask = _lib.FbTensor(mask.data_ptr(), n * n, 0, n)
+    p.o = _lib.FbTensor(o.data_ptr(), n * dim, dim // heads, dim)
+    p.lse = lse.data_ptr()
+    return p, packed
+
+
+# edges: one query, one block, blocks of 32 and of 64 keys with a remainder, one and two halves of 128 queries, workgroups that walk
+# several windows (2048 x 8), four waves and eight (up to 512 pairs), grids below those where the operator takes these kernels
+@pytest.mark.parametrize("dtype,scale_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32), (torch.bfloat16, torch.float16)])
+@pytest.mark.parametrize("windows,n,heads,rank,types", [(2048, 8, 1, 8, 0), (1030, 1, 1, 8, 0), (2050, 49, 8, 16, 0), (260, 64, 4, 16, 4), (130, 72, 8, 8, 2), (344, 144, 3, 16, 0),
+                                                        (512, 144, 2, 16, 8), (128, 256, 8, 8, 0), (1024, 256, 1, 16, 4), (520, 200, 2, 16, 1), (3, 256, 5, 16, 3)])
+def test_window_block_in_the_attention_kernels(gpu_device, dtype, scale_dtype, windows, n, heads, rank, types):
+    """fb_window_fwd and fb_window_bwd have the bits of the normalisation, the operator and the normalisation's backward one after
+    the other; the logit scale's gradient is another order of the same sum."""
+    lib, s = _lib.load(), ctypes.c_void_p(interface._stream())
+    g = torch.Generator(device=gpu_device).manual_seed(n)
+    dim = 32 * heads
+    rand = lambda *shape: torch.randn(*shape, generator=g, device=gpu_device)
+    qkv = (rand(windows, n, 3 * dim) * torch.exp2(rand(windows, n, 1))).to(dtype)
+    if dtype == torch.bfloat16:
+        qkv[1, 0, :dim] = 0  # a row without a direction (fp16: 0 / 0)
+        qkv[2, n // 2, dim:2 * dim] = 1e20  # a norm beyond fp32: zeros
+    qb, kb = (rand(1, n, heads, rank).to(dtype) * 0.3 for _ in range(2))
+    scale = (rand(heads) * 0.5 + 2).to(scale_dtype)
+    scale[-1] = 5.0  # clamped
+    mask = ((rand(types, n, n) < -0.5).to(dtype) * -100.0) if types else None
+    dout = rand(windows, n, dim).to(dtype)
+    full = lambda *shape, dt=dtype: torch.full(shape, float("nan"), device=gpu_device, dtype=dt)
+
+    def outputs():
+        return full(windows, n, dim), full(windows, heads, n, dt=torch.float32), full(windows, n, 3 * dim), full(heads, dt=scale_dtype)
+
+    def one():
+        o, lse, dqkv, dscale = outputs()
+        p, packed = _window_params(qkv, qb, kb, mask, heads, o, lse)
+        a = _cosine_block(qkv.view(windows * n, -1), scale, heads, dtype)
+        assert lib.fb_window_ready(ctypes.byref(p), ctypes.byref(a), 0), lib.fb_last_error()
+        _lib.check_status(lib.fb_window_fwd(ctypes.byref(p), ctypes.byref(a), s))
+        p.dout = _lib.FbTensor(dout.data_ptr(), n * dim, 32, dim)
+        p.dq, p.dk, p.dv = (packed(dqkv, i) for i in range(3))
+        partial = full(lib.fb_window_workspace_bytes(ctypes.byref(p)) // 4, dt=torch.float32)
+        a.partial, a.dlogit_scale = partial.data_ptr(), dscale.data_ptr()
+        assert lib.fb_window_ready(ctypes.byref(p), ctypes.byref(a), 1), lib.fb_last_error()
+        _lib.check_status(lib.fb_window_bwd(ctypes.byref(p), ctypes.byref(a), s))
+        return o, lse, dqkv, dscale
+
+    def parts():
+        o, lse, dqkv, dscale = outputs()
+        q, k = full(windows, n, dim), full(windows, n, dim)
+        a = _cosine_block(qkv.view(windows * n, -1), scale, heads, dtype)
+        a.q, a.k = q.data_ptr(), k.data_ptr()
+        _lib.check_status(lib.fb_cosine_fwd(ctypes.byref(a), s))
+        p, packed = _window_params(qkv, qb, kb, mask, heads, o, lse)
+        p.q, p.k = (_lib.FbTensor(t.data_ptr(), n * dim, 32, dim) for t in (q, k))
+        _lib.check_status(lib.fb_fwd(ctypes.byref(p), s))
+        p.dout = _lib.FbTensor(dout.data_ptr(), n * dim, 32, dim)
+        p.dq, p.dk, p.dv = (packed(dqkv, i) for i in range(3))
+        scratch = full(lib.fb_bwd_workspace_bytes(ctypes.byref(p)) // 4, dt=torch.float32)
+        p.delta = scratch.data_ptr()
+        _lib.check_status(lib.fb_bwd(ctypes.byref(p), s))
+        lib.fb_cosine_workspace_bytes.restype = ctypes.c_size_t
+        partial = full(lib.fb_cosine_workspace_bytes(ctypes.byref(a)) // 4, dt=torch.float32)
+        a.dq, a.dk, a.grad_stride = p.dq.ptr, p.dk.ptr, 3 * dim
+        a.dqkv, a.dlogit_scale, a.partial = dqkv.data_ptr(), dscale.data_ptr(), partial.data_ptr()
+        _lib.check_status(lib.fb_cosine_bwd(ctypes.byref(a), s))
+        return o, lse, dqkv, dscale
+
+    got, want = one(), parts()
+    torch.cuda.synchronize()
+    same = windows * heads >= 1024  # (below, the operator's backward is not the ring kernel: other summation orders)
+    for name, x, w in zip(("o", "lse", "dqkv", "dlogit_scale"), got, want):
+        assert torch.isfinite(x).all(), name
+        if name == "dlogit_scale":
+            # sums of 32 windows n products each, any order: 2^-24 sqrt(their number) of the root of their sum of squares, which
+            # is that of random signs, and one rounding to the parameter's type
+            terms = 32 * windows * n
+            eps = 2.0 ** -24 if scale_dtype == torch.float32 else 2.0 ** -8 if scale_dtype == torch.bfloat16 else 2.0 ** -11
+            big = float(w.float().abs().max())
+            assert (x.float() - w.float()).abs().max() <= (eps + 2.0 ** -24 * terms ** 0.5 * 8 + (0 if same else 2.0 ** -8)) * max(big, 1.0), name
+            assert float(x[-1]) == 0
+        elif name == "dqkv" and same and dtype == torch.float16:
+            # (the compiler sums products of fp16 pairs by v_dot2_f32_f16 in one of the two and by fma in the other: fp32 roundings of
+            # a row's sums, 2^-21 of its largest value, and what of them reaches the result's 11 bits)
+            row = w.float().abs().view(windows, n, 3 * heads, 32).amax(-1, keepdim=True).expand(-1, -1, -1, 32).reshape(w.shape)
+            off = x != w
+            assert int(off.sum()) <= x.numel() * 2.0 ** -12, name
+            assert ((x.float() - w.float()).abs() <= w.float().abs() * 2.0 ** -10 + row * 2.0 ** -20 + 2.0 ** -24).all(), name
+        elif same or (name == "o" and windows * heads >= 512):
+            assert torch.equal(x, w), name
+        else:
+            assert (x.float() - w.float()).norm() <= 2.0 ** -7 * w.float().norm(), name
+    again = one()
+    assert all(torch.equal(x, y) for x, y in zip(got, again))
+
+
 class Given(torch.nn.Module):
     """In the place of a projection: its result."""
 
