@@ -44,6 +44,9 @@ hipError_t launch_wgrad(const void *dy, int64_t ldy, const void *x, int64_t ldx,
 bool project_recommended(int64_t tokens, int k, const int *n, int count);
 hipError_t launch_project(const void *x, int64_t ldx, const void *const *w, void *const *y, const int *n, int count, int64_t tokens, int k, bool bf16,
                           hipStream_t stream);
+// a projection of many tokens (fb_linear.hip)
+bool linear_recommended(int64_t tokens, int n, int k);
+hipError_t launch_linear(const void *x, int64_t ldx, const void *w, const void *b, void *y, int64_t tokens, int n, int k, bool bf16, hipStream_t stream);
 
 hipError_t launch_fwd(const FwdArgs &a, bool bf16, hipStream_t stream) {
     if (window_forward(a)) return bf16 ? launch_fwd_win_bf16_2(a, stream) : launch_fwd_win_f16_2(a, stream);
@@ -438,6 +441,22 @@ int fb_project(const void *x, int64_t ldx, const void *const *w, void *const *y,
     }
     if (!aligned) return fb::api_fail(FB_ERR_STRIDE, "fb_project: tensors must be 16-byte aligned");
     return launched(fb::launch_project(x, ldx, w, y, n, count, tokens, k, dtype == FB_BF16, static_cast<hipStream_t>(stream)), "fb_project");
+}
+
+int fb_linear_recommended(int64_t tokens, int n, int k) { return project_sizes(tokens, k, &n, 1) && fb::linear_recommended(tokens, n, k) ? 1 : 0; }
+
+int fb_linear(const void *x, int64_t ldx, const void *w, const void *b, void *y, int dtype, int64_t tokens, int n, int k, void *stream) {
+    fb::api_clear_error();
+    if (!x || !w || !y) return fb::api_fail(FB_ERR_NULL, "fb_linear: null pointer");
+    if (dtype != FB_F16 && dtype != FB_BF16) return fb::api_fail(FB_ERR_DTYPE, "only fp16 and bf16 are supported");
+    if (!project_sizes(tokens, k, &n, 1))
+        return fb::api_fail(FB_ERR_SHAPE, "fb_linear: tokens up to 2^24, k a multiple of 64 and n of 8, both up to 65536");
+    if (ldx < k || ldx % 8 != 0 || ldx >= (1 << 22))
+        return fb::api_fail(FB_ERR_STRIDE, "fb_linear: the row stride must be a multiple of 8 below 2^22 and hold a row");
+    for (const void *p : {x, w, static_cast<const void *>(y)})
+        if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return fb::api_fail(FB_ERR_STRIDE, "fb_linear: tensors must be 16-byte aligned");
+    if (reinterpret_cast<uintptr_t>(b) % 4 != 0) return fb::api_fail(FB_ERR_STRIDE, "fb_linear: the bias must be 4-byte aligned");
+    return launched(fb::launch_linear(x, ldx, w, b, y, tokens, n, k, dtype == FB_BF16, static_cast<hipStream_t>(stream)), "fb_linear");
 }
 
 int fb_bwd_static(const fb_params *p, void *stream) {

@@ -401,14 +401,30 @@ bool plain_tensor(const Tensor &t, const Tensor &like) {
            t.layout() == c10::kStrided && t.has_storage() && !t.is_neg() && !t._is_zerotensor() && !t._fw_grad(/*level=*/0).defined();
 }
 
+// x w^T + b of plain tensors of one 16-bit type: by the library's kernel (fb_linear) where that is ahead and takes them, else nothing.
+Tensor many_tokens(const Tensor &x, const Tensor &w, const c10::optional<Tensor> &b) {
+    const int64_t k = x.size(-1), n = w.size(0), tokens = x.numel() / k;
+    auto takes = [](const Tensor &t, int align) { return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % align == 0; };
+    if (n > (1 << 16) || k > (1 << 16) || !fb_linear_recommended(tokens, (int)n, (int)k) || !takes(x, 16) || !takes(w, 16) || (b.has_value() && !takes(*b, 4)))
+        return Tensor();
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    auto shape = x.sizes().vec();
+    shape.back() = n;
+    Tensor y = fresh(shape, x.scalar_type(), x.device());
+    check(fb_linear(x.data_ptr(), k, w.data_ptr(), b.has_value() ? b->data_ptr() : nullptr, y.data_ptr(), dtype_code(x.scalar_type()), tokens, (int)n, (int)k,
+                    stream_of(x)));
+    return y;
+}
+
 // A projection x w^T + b whose weight and bias gradients come from the library's kernel for long contractions
-// (fb_weight_grad); the forward and the input's gradient are the tensor library's products.
+// (fb_weight_grad); the forward is the library's where it is ahead (many_tokens), the input's gradient the tensor library's product.
 struct LinearFn : public torch::autograd::Function<LinearFn> {
     static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &w, const c10::optional<Tensor> &b) {
         // (the weight only where the input's gradient needs it: as long as it is saved nobody may change it before the backward)
         ctx->save_for_backward({x, x.requires_grad() ? w : Tensor()});
         ctx->saved_data["bias"] = b.has_value();
-        return at::linear(x, w, b);
+        const Tensor y = many_tokens(x, w, b);
+        return y.defined() ? y : at::linear(x, w, b);
     }
 
     static tensor_list backward(AutogradContext *ctx, tensor_list grads) {
@@ -442,16 +458,22 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
     }
 };
 
-// The projection where its weight gradient is asked for and the library's kernel for it is ahead, else nothing: the caller
-// then takes the tensor library's own operation, which is also what modes, transforms and tracers that look at operations see.
+// The projection where its weight gradient is asked for and the library's kernel for it is ahead, or where nothing is differentiated and
+// the library's product is, else nothing: the caller then takes the tensor library's own operation, which is also what modes,
+// transforms and tracers that look at operations see.
 c10::optional<Tensor> linear(const Tensor &x, const Tensor &w, const c10::optional<Tensor> &b) {
     const auto type = x.scalar_type();
-    const bool ready = c10::GradMode::is_enabled() && (type == torch::kFloat16 || type == torch::kBFloat16) && plain_tensor(x, x) &&
-                       plain_tensor(w, x) && w.requires_grad() && x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && x.numel() > 0 &&
-                       w.size(0) <= (1 << 16) && w.size(1) <= (1 << 16) &&
-                       fb_weight_grad_recommended(x.numel() / x.size(-1), (int)w.size(0), (int)w.size(1)) &&
-                       (!b.has_value() || (plain_tensor(*b, x) && b->dim() == 1 && b->size(0) == w.size(0))) && nothing_watches();
+    const bool ready = (type == torch::kFloat16 || type == torch::kBFloat16) && plain_tensor(x, x) && plain_tensor(w, x) && x.dim() >= 2 && w.dim() == 2 &&
+                       x.size(-1) == w.size(1) && x.numel() > 0 && (!b.has_value() || (plain_tensor(*b, x) && b->dim() == 1 && b->size(0) == w.size(0))) &&
+                       nothing_watches();
     if (!ready) return c10::nullopt;
+    if (!c10::GradMode::is_enabled()) {
+        const Tensor y = many_tokens(x, w, b);
+        return y.defined() ? c10::optional<Tensor>(y) : c10::nullopt;
+    }
+    if (!w.requires_grad() || w.size(0) > (1 << 16) || w.size(1) > (1 << 16) ||
+        !fb_weight_grad_recommended(x.numel() / x.size(-1), (int)w.size(0), (int)w.size(1)))
+        return c10::nullopt;
     return LinearFn::apply(x, w, b);
 }
 

@@ -30,9 +30,9 @@ def _plain(layer):
 
 
 def _project(layer, x):
-    """``layer(x)``.  A plain ``nn.Linear`` over many tokens gets its weight gradient from the library's own kernel for long
-    contractions (``ext.linear``, which says for which calls; a layer that something hooks into or replaces is called)."""
-    if type(x) in _TENSORS and x.is_cuda and torch.is_grad_enabled() and x.numel() >= _TOKENS_OF_A_LONG_CONTRACTION * x.shape[-1] and _plain(layer):
+    """``layer(x)``.  A plain ``nn.Linear`` over many tokens is the library's own product and gets its weight gradient from the
+    library's own kernel (``ext.linear``, which says for which calls; a layer that something hooks into or replaces is called)."""
+    if type(x) in _TENSORS and x.is_cuda and x.numel() >= _TOKENS_OF_A_LONG_CONTRACTION * x.shape[-1] and _plain(layer):
         ext = interface._extension()
         if ext is not None:
             y = ext.linear(x, layer.weight, layer.bias)

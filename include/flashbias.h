@@ -285,6 +285,14 @@ int fb_project_recommended(int64_t tokens, int k, const int *n, int count);
 int fb_project(const void *x, int64_t ldx, const void *const *w, void *const *y, const int *n, int count, int dtype, int64_t tokens,
                int k, void *stream);
 
+/* A projection of many tokens (the layers of a window block, swin_transformer_v2.py:155-207): y (tokens, n) = x (tokens, k) w^T + b
+ * in the input dtype, accumulated in fp32 and rounded once; b (n) NULL: none.  w (n, k) and y are contiguous, x has contiguous rows at
+ * a stride of ldx elements.  k is a multiple of 64, n and ldx of 8, ldx below 2^22, n and k at most 65536, tokens at most 2^24; x, w
+ * and y 16-byte aligned, b 4-byte aligned.
+ * fb_linear_recommended: 1 where this was measured ahead of the vendor library's product of the same shape. */
+int fb_linear_recommended(int64_t tokens, int n, int k);
+int fb_linear(const void *x, int64_t ldx, const void *w, const void *b, void *y, int dtype, int64_t tokens, int n, int k, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -471,6 +471,56 @@ def test_projections(gpu_device, dtype, tokens, n, k):
     assert lib.fb_project(x.data_ptr(), x.stride(0), pointers(w), pointers(y), sizes, len(n), CODES[dtype], tokens, k - 8, interface._stream()) != 0
 
 
+# one step of 64 columns, fewer steps than a tile has stages, and many; tiles of 128 and of 256 channels, one and several a workgroup, results
+# through the caches and past them (64 MB and more), ragged edges along tokens and channels, a bias on 4 bytes, rows inside a wider tensor
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens,n,k", [(1, 8, 64), (257, 136, 128), (300, 1000, 1600), (9001, 1000, 192), (33000, 512, 64), (70144, 512, 128),
+                                        (140001, 264, 64), (20001, 776, 512)])
+def test_linear(gpu_device, dtype, tokens, n, k):
+    lib = _lib.load()
+    g = torch.Generator(device=gpu_device).manual_seed(tokens)
+    x_all = torch.randn(tokens, k + 24, generator=g, device=gpu_device).to(dtype)
+    x = x_all[:, 8:8 + k]
+    x_all[:, :8] = x_all[:, 8 + k:] = float("nan")  # (nothing outside the rows may count)
+    w = torch.randn(n, k, generator=g, device=gpu_device).to(dtype)
+    bias = torch.randn(n + 2, generator=g, device=gpu_device).to(dtype)[2:]
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for b in (bias, None):
+        whole = torch.full((tokens * n + 64,), 7.0, device=gpu_device, dtype=dtype)  # (nor be written)
+        y = whole[:tokens * n].view(tokens, n)
+        _lib.check_status(lib.fb_linear(x.data_ptr(), x.stride(0), w.data_ptr(), None if b is None else b.data_ptr(), y.data_ptr(), CODES[dtype], tokens,
+                                        n, k, interface._stream()))
+        for rows in torch.arange(tokens, device=gpu_device).split(32768):
+            part = x[rows].double()
+            want = part @ w.double().t().contiguous() + (0 if b is None else b.double())
+            size = part.abs() @ w.double().abs().t().contiguous() + (0 if b is None else b.double().abs())
+            # rounded once: at most half a unit of the last place of every element, plus its sum in 32 bits
+            assert ((y[rows].double() - want).abs() <= 1.01 * unit * want.abs() + (k + 1) * 2.0 ** -24 * size).all()
+        assert (whole[tokens * n:] == 7.0).all()
+    assert lib.fb_linear(x.data_ptr(), x.stride(0), w.data_ptr(), None, y.data_ptr(), CODES[dtype], tokens, n, k - 8, interface._stream()) != 0
+
+
+@pytest.mark.parametrize("n,bias", [(384, False), (128, True)])
+def test_projection_of_many_tokens_takes_the_product_and_leaves_the_rest(gpu_device, n, bias):
+    torch.manual_seed(4)
+    layer = torch.nn.Linear(128, n, bias=bias).to(gpu_device, torch.bfloat16)
+    x = torch.randn(1025, 128, 128, device=gpu_device, dtype=torch.bfloat16)
+    ext, many = interface._extension(), 1.01 * 2.0 ** -8
+    want = layer(x).double()
+    with torch.no_grad():
+        got = ext.linear(x, layer.weight, layer.bias)
+        assert got is not None and (got.double() - want).norm() <= 2 * many * want.norm()
+        assert torch.equal(got, modules._project(layer, x))
+        # few tokens, rows that are not contiguous, long rows and other types are left to the tensor library
+        assert ext.linear(x[:2], layer.weight, layer.bias) is None and ext.linear(x.transpose(0, 1), layer.weight, layer.bias) is None
+        assert ext.linear(x.view(-1, 1024), torch.zeros(n, 1024, device=gpu_device, dtype=torch.bfloat16), layer.bias) is None
+        assert ext.linear(x.float(), layer.weight.float(), None) is None
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert ext.linear(x, layer.weight, layer.bias) is None
+    y = modules._project(layer, x)
+    assert "LinearFn" in y.grad_fn.name() and torch.equal(y.detach(), got)
+
+
 def test_block_projections_take_the_kernel_and_leave_the_rest(gpu_device):
     torch.manual_seed(3)
     layers = [torch.nn.Linear(128, 136, bias=False).to(gpu_device, torch.bfloat16) for _ in range(3)]

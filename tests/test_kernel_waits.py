@@ -77,9 +77,9 @@ def test_compiled_ring_kernel():
 
 @pytest.mark.skipif(shutil.which("hipcc") is None or shutil.which("make") is None, reason="needs hipcc and make")
 def test_compiled_window_and_projection_kernels():
-    """The window forward, the ring in fp16, the weight gradient and the projections."""
+    """The window forward, the ring in fp16, the weight gradient and the projections, of few tokens and of many."""
     units = {f"build/asm/fb_{unit}.s": products for unit, products in (("fwd_win_bf16_2", 30), ("fwd_win_f16_2", 30), ("bwd_ring_f16_2", 100),
-                                                                     ("wgrad", 100), ("project", 90))}
+                                                                     ("wgrad", 100), ("project", 90), ("linear", 300))}
     subprocess.run(["make", "-j4"] + list(units), cwd=CSRC, check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
     for unit, products in units.items():
         with open(os.path.join(CSRC, unit)) as f:
@@ -90,7 +90,7 @@ def test_compiled_window_and_projection_kernels():
 @pytest.mark.skipif(shutil.which("hipcc") is None or shutil.which("make") is None, reason="needs hipcc and make")
 @pytest.mark.parametrize("unit,kernel", [("fwd_win_bf16_2", "fwd_win_kernel"), ("fwd_win_f16_2", "fwd_win_kernel"), ("fwd_bf16_2", "fwd_thin_kernel"),
                                          ("bwd_dkv_bf16_4", "bwd_dkv_mid_kernel"), ("bwd_dkv_f16_4", "bwd_dkv_mid_kernel"),
-                                         ("bwd_dq_bf16_2", "bwd_dq_mid_kernel"), ("bwd_dq_bf16_4", "bwd_dq_mid_kernel")])
+                                         ("bwd_dq_bf16_2", "bwd_dq_mid_kernel"), ("bwd_dq_bf16_4", "bwd_dq_mid_kernel"), ("linear", "linear_kernel")])
 def test_kernels_that_keep_to_their_registers(unit, kernel):
     """Kernels written for a number of waves a SIMD whose registers just hold them: none of their instantiations spills."""
     path = f"build/asm/fb_{unit}.s"
