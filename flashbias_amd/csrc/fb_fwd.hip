@@ -617,11 +617,12 @@ static hipError_t launch_fwd_vec(const FwdArgs &a, hipStream_t stream) {
 // kernel, which has the registers to read ahead, is faster.  us, general / this one: B1 H8 L=2048 32.9 / 38.6, L=4096 64.7 /
 // 74.9, B2 H16 L=512 11.2 / 12.6, with a padding mask B2 H8 L=1600 33.2 / 35.6; 384 workgroups 37.7 / 36.6 (B2 H16 L=1500);
 // causal B1 H16 L=1024 18.8 / 21.9, 512 workgroups 21.4 / 22.7 (B4 H16 L=1024), 600 32.6 / 32.6, 768 18.4 / 17.0 (B4 H32 L=600).
+// (One group of waves; with the keys split over two it is ahead on small grids too: thin_split.)
 // Between 129 and 192 keys the general kernel's second tile of 128 is half empty: causal B1 H8 L=160 7.5 / 7.1.
 template <int NKR>
 static bool thin_grid(const FwdArgs &a) {
     const int64_t wgs = (int64_t)a.B * a.H * ((a.Lq + 127) / 128);
-    return NKR < 2 || wgs > (a.causal ? 2 : 1) * (int64_t)num_cus() || (a.Lk > 128 && a.Lk <= 192);
+    return NKR < 2 || wgs > (a.causal ? 2 : 1) * (int64_t)num_cus() || (a.Lk > 128 && a.Lk <= 192) || thin_split(a);
 }
 
 template <class T, int NKD, int NKR, int NDV>

@@ -18,31 +18,37 @@
 // -> 95), three waves and all fragments of a tile ahead (rank 32 padded 80, masked 768 586), turns by tile (rank 8 masked 156 ->
 // 168), priority for the products (no gain), scores and bias in one chain (2 % at rank 32, but the bias product then starts from
 // q k^T instead of zero: closed-form factors in the thousands lose its low bits, dq_bias of the ALiBi workload 0.067 for 0.01).
+//
+// SPLIT: on small grids a second group of four waves takes the second half of the keys for the same queries, in stages of its own, and hands
+// its sums over in LDS.  One group alone has one wave a SIMD there, which waits for itself: 1150 cycles a block where four waves take 500
+// (B1 H16 L=1500, causal: 192 workgroups 24.3 -> 19.5 us; dispatch and figures at thin_split).
 #pragma once
 #include "fb_lean_tiles.h"
 
 namespace fb {
 
-template <class T, int NKR_, int MASK_, bool FOLD_>
+template <class T, int NKR_, int MASK_, bool FOLD_, int SPLIT_>
 struct FwdThinCfg {
     static constexpr int NKD = 2, NKR = NKR_, NK = NKD + NKR_;
     static constexpr bool VMASK = MASK_ == kVectorMask, FOLD = FOLD_;
     static_assert(MASK_ != kMatrixMask && NKR_ <= 2 && !(FOLD_ && VMASK), "");
-    static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES, BM = 32 * NWAVES;
+    static constexpr int SPLIT = SPLIT_, NWAVES = 4, NTHREADS = 64 * NWAVES * SPLIT, BM = 32 * NWAVES; // (NWAVES: of a group)
     static constexpr int KBLK = 2, BN = 32 * KBLK;
     static constexpr int CPR = NKR == 2 ? 4 : 2; // 16-byte chunks per row of K_b
     static constexpr int K = 0, V = K + BN * 64, KB = V + BN * 64, MK = KB + (NKR ? BN * CPR * 16 : 0), STAGE = MK + (VMASK ? BN * 4 : 0);
-    static constexpr int LDS_BYTES = 2 * STAGE;
+    static constexpr int LDS_BYTES = 2 * STAGE * SPLIT;
     static constexpr int WAVES_EU = 4;
-    static_assert(WAVES_EU * LDS_BYTES <= 160 * 1024, "");
+    static_assert(WAVES_EU * LDS_BYTES / SPLIT <= 160 * 1024 && (SPLIT == 1 || LDS_BYTES >= 4 * 4608), "");
     static __device__ __forceinline__ bool low_parts(const FwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
 };
 
 template <class T, class C>
 __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::WAVES_EU, C::WAVES_EU))) void fwd_thin_kernel(const FwdArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const uint32_t lds0 = lds_addr_of(smem);
-    const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, g = lane >> 5;
+    const int grp = C::SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8); // takes its share of the tiles of keys, in stages of its own
+    uint8_t *const stages = smem + grp * 2 * C::STAGE;
+    const uint32_t lds0 = lds_addr_of(stages);
+    const int tid = threadIdx.x & (64 * C::NWAVES - 1), lane = tid & 63, c = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     const int total = a.ntiles_m * a.B * a.H;
@@ -53,6 +59,10 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     const int m0 = tile_m * C::BM, wq0 = m0 + wave * 32;
     const int query = wq0 + c;
 
+    int k_end = a.Lk; // causal: keys past the last query of this workgroup are never visible
+    if (a.causal && m0 + C::BM < k_end) k_end = m0 + C::BM;
+    const int ntiles = (k_end + C::BN - 1) / C::BN;
+    const int walk = (ntiles + C::SPLIT - 1) / C::SPLIT, tile0 = grp * walk; // this group's tiles: from tile0 on, `walk` of them if there are so many
     const uint8_t *kptr = reinterpret_cast<const uint8_t *>(a.k.ptr + b * a.k.sb + h * a.k.sh);
     const uint8_t *vptr = reinterpret_cast<const uint8_t *>(a.v.ptr + b * a.v.sb + h * a.v.sh);
     LeanCopy4<C::BN> kd, vd;
@@ -60,9 +70,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     vd.init(wave, lane, a.v.ss);
     DenseCopy<C::BN, C::CPR> kbd;
     if constexpr (C::NKR > 0) {
-        kbd.init(a.kb.ptr + b * a.kb.sb + h * a.kb.sh, a.kb.ss, a.r, C::low_parts(a), wave, lane, 0);
+        kbd.init(a.kb.ptr + b * a.kb.sb + h * a.kb.sh, a.kb.ss, a.r, C::low_parts(a), wave, lane, tile0 * C::BN);
         if (a.r < 16 * C::NKR && !C::low_parts(a)) { // (the channel padding of the rank is never written)
-            for (int i = tid; i < C::LDS_BYTES / 16; i += C::NTHREADS) reinterpret_cast<u32x4_t *>(smem)[i] = u32x4_t{0u, 0u, 0u, 0u};
+            for (int i = threadIdx.x; i < C::LDS_BYTES / 16; i += C::NTHREADS) reinterpret_cast<u32x4_t *>(smem)[i] = u32x4_t{0u, 0u, 0u, 0u};
             __syncthreads();
         }
     }
@@ -80,10 +90,12 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         mkey = a.mask.is_f32 ? reinterpret_cast<const float *>(mbase)[key] : T::to_float(reinterpret_cast<const uint16_t *>(mbase)[key]);
     };
     auto store_vmask = [&](int buf) {
-        if (tid < C::BN) *reinterpret_cast<float *>(smem + buf * C::STAGE + C::MK + 4 * tid) = mkey;
+        if (tid < C::BN) *reinterpret_cast<float *>(stages + buf * C::STAGE + C::MK + 4 * tid) = mkey;
     };
-    issue(0, 0);
-    if constexpr (C::VMASK) load_vmask(0);
+    if (C::SPLIT == 1 || tile0 < ntiles) {
+        issue(0, tile0 * C::BN);
+        if constexpr (C::VMASK) load_vmask(tile0 * C::BN);
+    }
 
     u32x4_t qr[C::NK];
     const uint16_t *qbase = a.q.ptr + b * a.q.sb + h * a.q.sh;
@@ -105,10 +117,6 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     float m_ref = -INFINITY, m2 = 0.f, l_run = 0.f; // (as in fwd_body)
     const float to_log2 = C::FOLD ? a.scale * kLog2e : kLog2e, lag = 8.0f / to_log2;
 
-    int k_end = a.Lk; // causal: keys past the last query of this workgroup are never visible
-    if (a.causal && m0 + C::BM < k_end) k_end = m0 + C::BM;
-    const int ntiles = (k_end + C::BN - 1) / C::BN;
-
     // this lane's read addresses inside a stage (stage, key block and step are added)
     const uint32_t row_off[2] = {lds0 + C::K + lean_row_addr<4>(c, g), lds0 + C::K + lean_row_addr<4>(c, 2 + g)};
     const uint32_t col_off[2] = {lds0 + C::V + lean_tr_addr4(c, g, 0), lds0 + C::V + lean_tr_addr4(c, g, 1)};
@@ -121,16 +129,16 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     barrier_lds();
 
 #pragma unroll 1
-    for (int it = 0; it < ntiles; ++it) {
-        const int cur = it & 1, n0 = it * C::BN;
-        const bool more = it + 1 < ntiles;
+    for (int it = 0; it < walk; ++it) {
+        const int cur = it & 1, tile = tile0 + it, n0 = tile * C::BN;
+        const bool more = it + 1 < walk && tile + 1 < ntiles;
         if (more) {
             issue(cur ^ 1, n0 + C::BN);
             if constexpr (C::VMASK) load_vmask(n0 + C::BN);
         }
         const uint32_t at = cur * C::STAGE;
         // (a tile hidden from every query of this wave: so are all later ones, but the copies and barriers go on)
-        if (!(a.causal && n0 > wq0 + 31) && wq0 < a.Lq) {
+        if (!(a.causal && n0 > wq0 + 31) && wq0 < a.Lq && (C::SPLIT == 1 || tile < ntiles)) {
             f32x16_t s[C::KBLK];
             if (!a.causal) __builtin_amdgcn_s_setprio(0);
 #pragma unroll
@@ -141,7 +149,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[v] = accb[v] = 0.f;
                 if constexpr (C::VMASK) {
-                    const float *sM = reinterpret_cast<const float *>(smem + at + C::MK) + kb * 32 + 4 * g;
+                    const float *sM = reinterpret_cast<const float *>(stages + at + C::MK) + kb * 32 + 4 * g;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         const f32x4_t x = *reinterpret_cast<const f32x4_t *>(sM + 8 * j);
@@ -228,6 +236,29 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         barrier_lds();
     }
 
+    if constexpr (C::SPLIT == 2) { // the second group's sums to the first one's (the stages are free: the loop ends with a barrier)
+        asm volatile("s_nop 11" : "+v"(o));
+        uint8_t *ex = smem + wave * 4608 + lane * 16;
+        float *em = reinterpret_cast<float *>(smem + wave * 4608 + 4096) + lane;
+        if (grp == 1) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4_t *>(ex + j * 1024) = f32x4_t{o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]};
+            em[0] = m_ref;
+            em[64] = l_run;
+        }
+        barrier_lds();
+        if (grp == 1) return;
+        const float m_other = em[0], m = fmaxf(m_ref, m_other);
+        const float mine = m_ref == m ? 1.f : fast_exp2((m_ref - m) * to_log2), other = m_other == m ? 1.f : fast_exp2((m_other - m) * to_log2); // exp2(-inf) = 0
+        l_run = l_run * mine + em[64] * other;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const f32x4_t x = *reinterpret_cast<const f32x4_t *>(ex + j * 1024);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[4 * j + e] = o[4 * j + e] * mine + x[e] * other;
+        }
+        m_ref = m;
+    }
     int q = query;
     asm volatile("" : "+v"(q)); // (keeps the address arithmetic below the key loop)
     const float l = l_run + __shfl_xor(l_run, 32, 64);
@@ -237,9 +268,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     store_acc_rows<T, true>(orow, ok, true, o, 1.f / l, a.d, g);
 }
 
-template <class T, int NKR, int MASK, bool FOLD>
-static hipError_t launch_fwd_thin(const FwdArgs &a0, hipStream_t stream) {
-    typedef FwdThinCfg<T, NKR, MASK, FOLD> C;
+template <class T, int NKR, int MASK, bool FOLD, int SPLIT>
+static hipError_t launch_fwd_thin_split(const FwdArgs &a0, hipStream_t stream) {
+    typedef FwdThinCfg<T, NKR, MASK, FOLD, SPLIT> C;
     FwdArgs a = a0;
     a.ntiles_m = (a.Lq + C::BM - 1) / C::BM;
     auto kern = fwd_thin_kernel<T, C>;
@@ -247,6 +278,23 @@ static hipError_t launch_fwd_thin(const FwdArgs &a0, hipStream_t stream) {
     const hipError_t e = allow_lds(kern, C::LDS_BYTES, once);
     if (e != hipSuccess) return e;
     return launch_flat(kern, (int64_t)a.ntiles_m * a.B * a.H, C::NTHREADS, C::LDS_BYTES, stream, a);
+}
+
+// Two groups of waves where four leave a compute unit with too few: up to two workgroups on each, under a causal mask, where a launch lasts
+// as long as its longest workgroup, up to 2.4 if that one is long, and more than 256 keys.  us, one group / two, rank 16: 64 workgroups (B1 H8 L=1024)
+// 16.8 / 13.8, 192 24.5 / 19.9, 256 57.4 / 44.9 (B2 H4 L=4096), 400 22.5 / 22.1, 512 71.4 / 70.3 (B1 H16 L=4096) and 22.3 / 22.5 (B2 H32 L=1024), 600 40.1 /
+// 40.3; with a padding mask 64 19.8 / 16.5, 256 68.3 / 51.8, 512 77.9 / 74.7, 600 44.9 / 46.8; causal 64 17.3 / 14.2, 192 24.3 / 19.5, 400 19.1 / 16.9, 512
+// 59.0 / 47.9 (B1 H16 L=4096) and 18.9 / 17.9 (B2 H32 L=1024), 576 20.4 / 19.2, 600 26.3 / 25.5 (B1 H50 L=1500) but 16.7 / 17.8 (B2 H50 L=700), 640 21.4 /
+// 22.5, 800 39.3 / 38.9; rank 32 (one group: the general kernel up to 256) 64 18.2 / 14.9, 512 45.7 / 43.1, causal 69.7 / 52.2.
+// Up to 256 keys (640 at ranks above 16) an entry keeps the bits that it has in a larger call.
+inline bool thin_split(const FwdArgs &a) {
+    const int64_t wgs = (int64_t)a.B * a.H * ((a.Lq + 127) / 128);
+    return a.Lk > (a.r > 16 ? 640 : 256) && 10 * wgs <= (a.causal && a.Lk >= 1024 ? 24 : 20) * (int64_t)num_cus();
+}
+
+template <class T, int NKR, int MASK, bool FOLD>
+static hipError_t launch_fwd_thin(const FwdArgs &a, hipStream_t stream) {
+    return thin_split(a) ? launch_fwd_thin_split<T, NKR, MASK, FOLD, 2>(a, stream) : launch_fwd_thin_split<T, NKR, MASK, FOLD, 1>(a, stream);
 }
 
 } // namespace fb

@@ -321,6 +321,28 @@ def test_thin_forward(gpu_device, r, Lq, Lk, scale, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,r,Lq,Lk,scale", [(2, 16, 1, 257, None), (2, 0, 130, 320, 0.3), (2, 8, 300, 513, -0.2), (2, 32, 65, 641, None), (2, 24, 127, 705, 1.0),
+                                             (172, 16, 129, 258, None), (258, 8, 260, 321, 3.0)])
+def test_thin_forward_with_the_keys_split(gpu_device, dtype, B, r, Lq, Lk, scale):
+    """Two groups of waves for one query block from 257 keys (641 at ranks above 16) on small grids, one on large ones: an odd number of tiles, a second half
+    that is hidden (a causal mask: every row of a short query side) or that a mask switches off for a whole entry, and the first half alike; o, lse
+    and the gradients through them."""
+    H = 1 if B > 2 else 3
+    assert (B * H * ((Lq + 127) // 128) <= 512) == (B < 258)
+    for kind in (None, "causal", "first", "second"):
+        if B > 2 and kind in ("first", "second"):
+            continue
+        mask = None
+        if kind in ("first", "second"):
+            mask = torch.randn(B, 1, 1, Lk, generator=torch.Generator().manual_seed(Lk))
+            half = ((Lk + 63) // 64 + 1) // 2 * 64
+            mask[1, ..., half:] = float("-inf") if kind == "second" else mask[1, ..., half:]
+            mask[1, ..., :half] = float("-inf") if kind == "first" else mask[1, ..., :half]
+            mask = mask.to(dtype if Lq % 2 else torch.float32)
+        _case(gpu_device, B, Lq, Lk, H, 32, r, dtype, kind == "causal", mask=mask, scale=scale, seed=r + Lk, o_by_magnitude=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("r,Lq,Lk,scale", [(32, 1, 1, None), (32, 127, 63, None), (24, 128, 65, 0.3), (32, 129, 128, 1.0), (24, 33, 193, -0.2),
                                            (32, 100, 530, 0.0625)])
 def test_thin_forward_at_rank_32(gpu_device, r, Lq, Lk, scale, dtype):
