@@ -19,31 +19,34 @@
 // 1416, B2 H32 L=3000 306 -> 293; r16 B2 H4 L=8192 567 -> 555, B8 H16 L=700 100 -> 95; r32 768 x 4 rows of 768 2139 -> 2097, 301 x
 // 4 of 301 225 -> 213; r32 fp16 with a padding mask, 2 x 4 x (1000 x 3000) 170 -> 160.  Not kept: four waves without dk_bias (spills:
 // 399 -> 409).
+//
+// SPLIT (head dims above 32): on small grids a second group of four waves takes the second half of the queries for the same keys, in stages of its own,
+// and hands its sums over in LDS (mid_split).  At 1 x 8 x 1000 one group takes 2.6 us for a step of 64 queries, most of it waiting.
 #pragma once
 #include "fb_lean_tiles.h"
 
 namespace fb {
 
-template <class T, int NKD_, int NKR_, int MASK_, bool FOLD_, bool BG_>
+template <class T, int NKD_, int NKR_, int MASK_, bool FOLD_, bool BG_, int SPLIT_ = 1>
 struct DkvMidCfg {
     static constexpr int NKD = NKD_, NKR = NKR_, NK = NKD + NKR_, NDV = NKD / 2;
     static_assert(NKD_ == 2 || NKD_ == 4, "");
     static constexpr bool FOLD = FOLD_, VMASK = MASK_ == kVectorMask, BG = BG_ && NKR_ > 0;
     static_assert(MASK_ != kMatrixMask && !(FOLD_ && VMASK) && NKR_ <= 2, "");
     static constexpr int MB = NDV + (BG ? 1 : 0); // 32-row blocks of [dK | dK_b]^T
-    static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES, BN = 128, BMQ = 64;
+    static constexpr int SPLIT = SPLIT_, NWAVES = 4, NTHREADS = 64 * NWAVES * SPLIT, BN = 128, BMQ = 64; // (NWAVES: of a group)
     static constexpr int CPR = 2 * (NKR > 0 ? NKR : 1);
     static constexpr int ROWCH = 2 * NKD, RB = 16 * ROWCH; // chunks and bytes of a Q or dO row
     static constexpr int NI = NKD / 2; // copy instructions per wave, tensor and step
     // a stage, bytes: Q, dO, Q_b rows of 32 or 64, lse * log2(e) and -delta
     static constexpr int SQ = BMQ * RB, SQB = NKR > 0 ? BMQ * CPR * 16 : 0, STAGE = 2 * SQ + SQB + 8 * BMQ, NSTAGE = 2;
-    static constexpr int LDS_BYTES = NSTAGE * STAGE;
+    static constexpr int LDS_BYTES = NSTAGE * STAGE * SPLIT;
     static constexpr int WAVES_EU = NKD == 4 ? 2 : 3;
-    static_assert(WAVES_EU * LDS_BYTES <= 160 * 1024, "");
+    static_assert(WAVES_EU * LDS_BYTES / SPLIT <= 160 * 1024 && (SPLIT == 1 || (NKD == 4 && LDS_BYTES >= 4 * 16384)), "");
     // Rank above 16 with dk_bias at head dims above 32: the places of the copies are formed where they are used.  Kept, they spill (24
     // bytes), and a reload waits for the tile that has just been requested: training step, us, r32 causal B2 H8 L=4096 272 -> 265,
     // B4 H16 L=2048 405 -> 400, B1 H4 L=1000 87.3 -> 85.  The others have the registers (r2 as 16 causal B2 H16 L=2048 136.5 -> 138).
-    static constexpr bool FRESH = NKD == 4 && NKR == 2 && BG;
+    static constexpr bool FRESH = NKD == 4 && BG && (NKR == 2 || SPLIT == 2);
     static constexpr bool ORDERED = NKD == 4; // two waves a SIMD: the order is fixed phase by phase
     static __device__ __forceinline__ bool low_parts(const BwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
 };
@@ -51,8 +54,10 @@ struct DkvMidCfg {
 template <class T, class C>
 __device__ __forceinline__ void bwd_dkv_mid_body(const BwdArgs &a, int wg) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const uint32_t lds0 = lds_addr_of(smem);
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int grp = C::SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8); // takes its share of the steps, in stages of its own
+    uint8_t *const stages = smem + grp * C::NSTAGE * C::STAGE;
+    const uint32_t lds0 = lds_addr_of(stages);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & (64 * C::NWAVES - 1)) >> 6);
 
     // (one workgroup serves `group` consecutive batch entries of its (head, key tile), as the general kernel does)
     const int group = a.group > 1 ? a.group : 1;
@@ -67,7 +72,8 @@ __device__ __forceinline__ void bwd_dkv_mid_body(const BwdArgs &a, int wg) {
     __syncthreads();
 
     const float to_log2 = C::FOLD ? a.scale * kLog2e : kLog2e; // the scores are in units of 1 / scale when folded
-    const int step0 = a.causal ? n0 / C::BMQ : 0, nsteps = (a.Lq + C::BMQ - 1) / C::BMQ; // causal: the first step that sees a key
+    const int nsteps = (a.Lq + C::BMQ - 1) / C::BMQ, seen = a.causal ? n0 / C::BMQ : 0; // causal: the first step that sees a key
+    const int walk = (max(nsteps - seen, 0) + C::SPLIT - 1) / C::SPLIT, step0 = seen + grp * walk;
     f32x16_t acc_b; // dk_bias, summed over the group
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc_b[v] = 0.f;
@@ -166,11 +172,11 @@ __device__ __forceinline__ void bwd_dkv_mid_body(const BwdArgs &a, int wg) {
 
         int stage = 0;
 #pragma unroll 1
-        for (int step = step0; step < nsteps; ++step) {
-            const uint8_t *st = smem + stage * C::STAGE;
-            if (step + 1 < nsteps) issue(step + 1, stage ^ 1);
+        for (int step = step0; step < (C::SPLIT == 1 ? nsteps : step0 + walk); ++step) {
+            const uint8_t *st = stages + stage * C::STAGE;
+            if (step + 1 < nsteps && (C::SPLIT == 1 || step + 1 < step0 + walk)) issue(step + 1, stage ^ 1);
             const int r0 = step * C::BMQ;
-            if (!(a.causal && wk0 > r0 + C::BMQ - 1) && wk0 < a.Lk) {
+            if (!(a.causal && wk0 > r0 + C::BMQ - 1) && wk0 < a.Lk && (C::SPLIT == 1 || step < nsteps)) {
                 TileAddr<C::ROWCH> ta(lds_addr_of(st), c, g);
                 if constexpr (C::ORDERED) asm volatile("" : "+v"(ta.row), "+v"(ta.tr));
                 u32x4_t qa[C::NK], da[C::NKD];
@@ -296,6 +302,34 @@ __device__ __forceinline__ void bwd_dkv_mid_body(const BwdArgs &a, int wg) {
             stage ^= 1;
         }
 
+        if constexpr (C::SPLIT == 2) { // the second group's sums to the first one's (the stages are free: the loop ends with a barrier)
+            uint8_t *ex = smem + wave * 4096;
+#pragma unroll
+            for (int n = 0; n < C::NDV; ++n) asm volatile("s_nop 11" : "+v"(acc_dv[n]), "+v"(acc_dk[n]));
+            if constexpr (C::BG) asm volatile("s_nop 11" : "+v"(acc_b));
+            if (grp == 1) {
+#pragma unroll
+                for (int n = 0; n < C::NDV; ++n) {
+                    lds_put_block(ex + 2 * n * 16384, acc_dv[n], lane);
+                    lds_put_block(ex + (2 * n + 1) * 16384, acc_dk[n], lane);
+                }
+            }
+            barrier_lds();
+            if (grp == 0) {
+#pragma unroll
+                for (int n = 0; n < C::NDV; ++n) {
+                    lds_add_block(ex + 2 * n * 16384, acc_dv[n], lane);
+                    lds_add_block(ex + (2 * n + 1) * 16384, acc_dk[n], lane);
+                }
+            }
+            if constexpr (C::BG) { // (no room for a fifth block beside them)
+                barrier_lds();
+                if (grp == 1) lds_put_block(ex, acc_b, lane);
+                barrier_lds();
+                if (grp == 0) lds_add_block(ex, acc_b, lane);
+            }
+            if (grp == 1) return; // (one batch entry: launch_dkv_mid)
+        }
         const bool ok = key < a.Lk;
         uint16_t *dvrow = const_cast<uint16_t *>(a.dv.ptr) + b * a.dv.sb + h * a.dv.sh + (int64_t)(ok ? key : 0) * a.dv.ss;
         uint16_t *dkrow = const_cast<uint16_t *>(a.dk.ptr) + b * a.dk.sb + h * a.dk.sh + (int64_t)(ok ? key : 0) * a.dk.ss;
@@ -321,9 +355,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     bwd_dkv_mid_body<T, C>(a, blockIdx.x);
 }
 
-template <class T, int NKD, int NKR, int MASK, bool FOLD, bool BG>
-static hipError_t launch_dkv_mid_bg(const BwdArgs &a0, hipStream_t stream) {
-    typedef DkvMidCfg<T, NKD, NKR, MASK, FOLD, BG> C;
+template <class T, int NKD, int NKR, int MASK, bool FOLD, bool BG, int SPLIT = 1>
+static hipError_t launch_dkv_mid_split(const BwdArgs &a0, hipStream_t stream) {
+    typedef DkvMidCfg<T, NKD, NKR, MASK, FOLD, BG, SPLIT> C;
     BwdArgs a = a0;
     a.ntiles_n = (a.Lk + C::BN - 1) / C::BN;
     auto kern = bwd_dkv_mid_kernel<T, C>;
@@ -332,6 +366,14 @@ static hipError_t launch_dkv_mid_bg(const BwdArgs &a0, hipStream_t stream) {
     if (e != hipSuccess) return e;
     const int group = a.group > 1 ? a.group : 1;
     return launch_flat(kern, (int64_t)a.ntiles_n * ((a.B + group - 1) / group) * a.H, C::NTHREADS, C::LDS_BYTES, stream, a);
+}
+
+template <class T, int NKD, int NKR, int MASK, bool FOLD, bool BG>
+static hipError_t launch_dkv_mid_bg(const BwdArgs &a, hipStream_t stream) {
+    if constexpr (NKD == 4) {
+        if (mid_split(a, a.Lk, a.Lq)) return launch_dkv_mid_split<T, NKD, NKR, MASK, FOLD, BG, 2>(a, stream);
+    }
+    return launch_dkv_mid_split<T, NKD, NKR, MASK, FOLD, BG>(a, stream);
 }
 
 // (no dk_bias wanted: without its products)

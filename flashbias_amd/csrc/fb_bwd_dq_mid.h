@@ -13,27 +13,30 @@
 // L=4096 412 -> 399, L=8192 1428 -> 1397, B2 H32 L=3000 304 -> 294; d32 r32 768 x 4 rows of 768 2080 -> 2045, 301 x 4 of 301 229 -> 221.
 // With a vector mask it was behind (its values a tile at a time in the stage: fp16 d64 8 x 8 x (1000 x 1500) 194 -> 196, d32 r8 157.8 ->
 // 158.3), so those stay with the general kernel.
+//
+// SPLIT (head dims above 32): on small grids a second group of four waves takes the second half of the keys for the same queries, in stages of its own,
+// and hands its sums over in LDS (mid_split).
 #pragma once
 #include "fb_lean_tiles.h"
 
 namespace fb {
 
-template <class T, int NKD_, int NKR_, bool FOLD_, bool BG_>
+template <class T, int NKD_, int NKR_, bool FOLD_, bool BG_, int SPLIT_ = 1>
 struct DqMidCfg {
     static constexpr int NKD = NKD_, NKR = NKR_, NK = NKD + NKR_, NDQ = NKD / 2;
     static_assert(NKD_ == 2 || NKD_ == 4, "");
     static constexpr bool FOLD = FOLD_, BG = BG_ && NKR_ > 0;
     static_assert(NKR_ <= 2, "");
-    static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES, BM = 32 * NWAVES, BN = 64;
+    static constexpr int SPLIT = SPLIT_, NWAVES = 4, NTHREADS = 64 * NWAVES * SPLIT, BM = 32 * NWAVES, BN = 64; // (NWAVES: of a group)
     static constexpr int ROWCH = 2 * NKD, RB = 16 * ROWCH; // chunks and bytes of a K or V row
     static constexpr int CPR = 2 * (NKR > 0 ? NKR : 1);
     static constexpr int NI = NKD / 2; // copy instructions per wave, tensor and tile
     // a stage, bytes: K, V, K_b rows of 32 or 64
     static constexpr int SK = BN * RB, SKB = NKR > 0 ? BN * CPR * 16 : 0, STAGE = 2 * SK + SKB;
-    static constexpr int LDS_BYTES = 2 * STAGE;
+    static constexpr int LDS_BYTES = 2 * STAGE * SPLIT;
     // (head dim 32: 121-127 registers without dq_bias at ranks up to 16; at rank 32 129-135, with it 139-155)
     static constexpr int WAVES_EU = NKD == 4 ? 2 : BG || NKR == 2 ? 3 : 4;
-    static_assert(WAVES_EU * LDS_BYTES <= 160 * 1024, "");
+    static_assert(WAVES_EU * LDS_BYTES / SPLIT <= 160 * 1024 && (SPLIT == 1 || (NKD == 4 && LDS_BYTES >= (NDQ + 1) * 4 * 4096)), "");
     static constexpr bool ORDERED = NKD == 4; // two waves a SIMD: the order is fixed phase by phase
     static __device__ __forceinline__ bool low_parts(const BwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
 };
@@ -41,8 +44,10 @@ struct DqMidCfg {
 template <class T, class C>
 __device__ __forceinline__ void bwd_dq_mid_body(const BwdArgs &a, int wg) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    const uint32_t lds0 = lds_addr_of(smem);
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int grp = C::SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8); // takes its share of the tiles of keys, in stages of its own
+    uint8_t *const stages = smem + grp * 2 * C::STAGE;
+    const uint32_t lds0 = lds_addr_of(stages);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & (64 * C::NWAVES - 1)) >> 6);
 
     // (one workgroup serves `group` consecutive batch entries of its (head, query tile), as the general kernel does)
     const int group = a.group > 1 ? a.group : 1;
@@ -60,7 +65,7 @@ __device__ __forceinline__ void bwd_dq_mid_body(const BwdArgs &a, int wg) {
     const float to_log2 = C::FOLD ? a.scale * kLog2e : kLog2e; // the scores are in units of 1 / scale when folded
     int k_end = a.Lk;
     if (a.causal && m0 + C::BM < k_end) k_end = m0 + C::BM; // keys past the last query are hidden
-    const int ntiles = (k_end + C::BN - 1) / C::BN;
+    const int ntiles = (k_end + C::BN - 1) / C::BN, walk = (ntiles + C::SPLIT - 1) / C::SPLIT, tile0 = grp * walk;
     f32x16_t acc_b; // dq_bias, summed over the group
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc_b[v] = 0.f;
@@ -107,7 +112,7 @@ __device__ __forceinline__ void bwd_dq_mid_body(const BwdArgs &a, int wg) {
             }
             if (wave < KB_WAVES) lds_dma16_lanes((uint32_t)min(brow, last) * bpitch + bch * 16, bbase + (int64_t)n0 * bpitch, at + 2 * C::SK + wave * 1024, lanes_b);
         };
-        issue(0, 0);
+        if (C::SPLIT == 1 || tile0 < ntiles) issue(tile0 * C::BN, 0);
 
         // ---- query-side operands
         u32x4_t qr[C::NKD], dor[1][C::NKD];
@@ -141,11 +146,11 @@ __device__ __forceinline__ void bwd_dq_mid_body(const BwdArgs &a, int wg) {
         barrier_lds();
 
 #pragma unroll 1
-        for (int it = 0; it < ntiles; ++it) {
-            const int stage = it & 1, n0 = it * C::BN;
-            if (it + 1 < ntiles) issue(n0 + C::BN, stage ^ 1);
-            if (!(a.causal && n0 > wq0 + 31) && wq0 < a.Lq) {
-                const uint8_t *st = smem + stage * C::STAGE;
+        for (int it = 0; it < walk; ++it) {
+            const int stage = it & 1, n0 = (tile0 + it) * C::BN;
+            if (it + 1 < walk && (C::SPLIT == 1 || tile0 + it + 1 < ntiles)) issue(n0 + C::BN, stage ^ 1);
+            if (!(a.causal && n0 > wq0 + 31) && wq0 < a.Lq && (C::SPLIT == 1 || tile0 + it < ntiles)) {
+                const uint8_t *st = stages + stage * C::STAGE;
                 TileAddr<C::ROWCH> ta(lds_addr_of(st), c, g);
                 if constexpr (C::ORDERED) asm volatile("" : "+v"(ta.row), "+v"(ta.tr));
                 u32x4_t ka[C::NK], va[C::NKD];
@@ -239,6 +244,22 @@ __device__ __forceinline__ void bwd_dq_mid_body(const BwdArgs &a, int wg) {
             barrier_lds();
         }
 
+        if constexpr (C::SPLIT == 2) { // the second group's sums to the first one's (the stages are free: the loop ends with a barrier)
+            uint8_t *ex = smem + wave * 4096;
+#pragma unroll
+            for (int n = 0; n < C::NDQ; ++n) asm volatile("s_nop 11" : "+v"(acc[n]));
+            if constexpr (C::BG) asm volatile("s_nop 11" : "+v"(acc_b));
+            if (grp == 1) {
+#pragma unroll
+                for (int n = 0; n < C::NDQ; ++n) lds_put_block(ex + n * 16384, acc[n], lane);
+                if constexpr (C::BG) lds_put_block(ex + C::NDQ * 16384, acc_b, lane);
+            }
+            barrier_lds();
+            if (grp == 1) return; // (one batch entry: launch_dq_mid)
+#pragma unroll
+            for (int n = 0; n < C::NDQ; ++n) lds_add_block(ex + n * 16384, acc[n], lane);
+            if constexpr (C::BG) lds_add_block(ex + C::NDQ * 16384, acc_b, lane);
+        }
         int q = wq0 + c;
         asm volatile("" : "+v"(q)); // (keeps the address arithmetic below the key loop)
         const bool ok = q < a.Lq;
@@ -264,9 +285,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     bwd_dq_mid_body<T, C>(a, blockIdx.x);
 }
 
-template <class T, int NKD, int NKR, bool FOLD, bool BG>
-static hipError_t launch_dq_mid_bg(const BwdArgs &a0, hipStream_t stream) {
-    typedef DqMidCfg<T, NKD, NKR, FOLD, BG> C;
+template <class T, int NKD, int NKR, bool FOLD, bool BG, int SPLIT = 1>
+static hipError_t launch_dq_mid_split(const BwdArgs &a0, hipStream_t stream) {
+    typedef DqMidCfg<T, NKD, NKR, FOLD, BG, SPLIT> C;
     BwdArgs a = a0;
     a.ntiles_m = (a.Lq + C::BM - 1) / C::BM;
     auto kern = bwd_dq_mid_kernel<T, C>;
@@ -275,6 +296,14 @@ static hipError_t launch_dq_mid_bg(const BwdArgs &a0, hipStream_t stream) {
     if (e != hipSuccess) return e;
     const int group = a.group > 1 ? a.group : 1;
     return launch_flat(kern, (int64_t)a.ntiles_m * ((a.B + group - 1) / group) * a.H, C::NTHREADS, C::LDS_BYTES, stream, a);
+}
+
+template <class T, int NKD, int NKR, bool FOLD, bool BG>
+static hipError_t launch_dq_mid_bg(const BwdArgs &a, hipStream_t stream) {
+    if constexpr (NKD == 4) {
+        if (mid_split(a, a.Lq, a.Lk)) return launch_dq_mid_split<T, NKD, NKR, FOLD, BG, 2>(a, stream);
+    }
+    return launch_dq_mid_split<T, NKD, NKR, FOLD, BG>(a, stream);
 }
 
 // Whether aligned calls without a mask take this kernel: 2 all, 1 those that want no dq_bias, 0 none (measured above).  Head dims above

@@ -549,6 +549,28 @@ __device__ __forceinline__ void store_acc_rows(uint16_t *row, bool row_ok, bool 
     }
 }
 
+// One group of waves' 32 x 32 block of sums to another's, through 4 KB of LDS a wave.
+__device__ __forceinline__ void lds_put_block(uint8_t *at, const f32x16_t &x, int lane) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4_t *>(at + j * 1024 + lane * 16) = f32x4_t{x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3]};
+}
+__device__ __forceinline__ void lds_add_block(const uint8_t *at, f32x16_t &x, int lane, float times = 1.f) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const f32x4_t y = *reinterpret_cast<const f32x4_t *>(at + j * 1024 + lane * 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[4 * j + e] = __builtin_fmaf(y[e], times, x[4 * j + e]);
+    }
+}
+// Two shares of a row's softmax sums, relative to the reference points m and m_other: both onto the larger one, which becomes m, by the factors
+// `mine` and `other` (of a share that has seen no finite score, m = -inf: 0).
+__device__ __forceinline__ void join_references(float &m, float m_other, float to_log2, float &mine, float &other) {
+    const float top = fmaxf(m, m_other);
+    mine = m == top ? 1.f : fast_exp2((m - top) * to_log2);
+    other = m_other == top ? 1.f : fast_exp2((m_other - top) * to_log2);
+    m = top;
+}
+
 // Turn-taking between the workgroups that share a CU.  The instruction arbiter serves the oldest
 // wave of a SIMD first, so of two resident workgroups the older one runs at the speed it would
 // have alone and the younger one only fills its stalls: their progress differs by a third, and

@@ -300,4 +300,14 @@ inline bool mixed_general_backward(const BwdArgs &a0) {
     return 2 * most <= (a.causal ? 9 : 3) * (int64_t)num_cus();
 }
 
+// Whether dq (rows: queries, walked: keys) and dk/dv (the other way round) of head dims 33 to 64 take two groups of waves a workgroup, which
+// split what it walks and add up their sums in LDS: where four waves leave a SIMD with one, which waits for LDS and its own chains. Training step,
+// both kernels, us, one group / two, rank 8: 64 workgroups (B1 H8) of 1000 keys 83.8 / 70.1, causal 74.0 / 66.9, padded 94.0 / 84.4; 192 of
+// 1500 121.9 / 101.0, of 3000 (B2 H4) 221 / 165; 256 of 1024 (B2 H16) 77.0 / 73.5, of 4096 (B1 H8) 248 / 213; of 512 keys (B1 H8) 44.3 / 44.1, of 256
+// 30.3 / 33.0; 384 of 1500 (B1 H32) 167.5 / 172.5, causal 113.2 / 106.3, of 700 causal 67.5 / 77.2; 512 of 2048 (B2 H16) 224 / 227, causal 149.3 / 150.3.
+inline bool mid_split(const BwdArgs &a, int rows, int walked) {
+    const int64_t wgs = (int64_t)a.B * a.H * ((rows + 127) / 128);
+    return a.group <= 1 && walked > 512 && 2 * wgs <= (a.causal && walked >= 1024 ? 3 : 2) * (int64_t)num_cus();
+}
+
 } // namespace fb
