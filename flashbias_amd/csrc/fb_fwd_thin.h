@@ -238,26 +238,21 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
 
     if constexpr (C::SPLIT == 2) { // the second group's sums to the first one's (the stages are free: the loop ends with a barrier)
         asm volatile("s_nop 11" : "+v"(o));
-        uint8_t *ex = smem + wave * 4608 + lane * 16;
+        uint8_t *ex = smem + wave * 4608;
         float *em = reinterpret_cast<float *>(smem + wave * 4608 + 4096) + lane;
         if (grp == 1) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4_t *>(ex + j * 1024) = f32x4_t{o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]};
+            lds_put_block(ex, o, lane);
             em[0] = m_ref;
             em[64] = l_run;
         }
         barrier_lds();
         if (grp == 1) return;
-        const float m_other = em[0], m = fmaxf(m_ref, m_other);
-        const float mine = m_ref == m ? 1.f : fast_exp2((m_ref - m) * to_log2), other = m_other == m ? 1.f : fast_exp2((m_other - m) * to_log2); // exp2(-inf) = 0
+        float mine, other;
+        join_references(m_ref, em[0], to_log2, mine, other);
         l_run = l_run * mine + em[64] * other;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const f32x4_t x = *reinterpret_cast<const f32x4_t *>(ex + j * 1024);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[4 * j + e] = o[4 * j + e] * mine + x[e] * other;
-        }
-        m_ref = m;
+        for (int v = 0; v < 16; ++v) o[v] *= mine;
+        lds_add_block(ex, o, lane, other);
     }
     int q = query;
     asm volatile("" : "+v"(q)); // (keeps the address arithmetic below the key loop)

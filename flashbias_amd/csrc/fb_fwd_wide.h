@@ -20,20 +20,21 @@
 
 namespace fb {
 
-template <class T, int NKD_, int NKR_, int NDV_, int MASK_, bool FOLD_>
+template <class T, int NKD_, int NKR_, int NDV_, int MASK_, bool FOLD_, int SPLIT_>
 struct FwdWideCfg {
     static constexpr int NKD = NKD_, NKR = NKR_, NDV = NDV_, NK = NKD_ + NKR_;
     static constexpr bool VMASK = MASK_ == kVectorMask, FOLD = FOLD_;
     static_assert(MASK_ != kMatrixMask && !(FOLD_ && VMASK), "");
-    static constexpr int NWAVES = 4, NTHREADS = 64 * NWAVES;
+    static constexpr int SPLIT = SPLIT_, NWAVES = 4, NTHREADS = 64 * NWAVES * SPLIT; // (NWAVES: of a group)
     static constexpr int BM = 32 * NWAVES;
     static constexpr int KBLK = 2, BN = 32 * KBLK;
     static constexpr int ROWCH = 2 * NKD, CPR = 2 * NKR; // 16-byte chunks per row of K and V, of K_b
     static constexpr int SK = BN * ROWCH * 8, SKB = BN * CPR * 8, SM = VMASK ? 2 * BN : 0;
     static constexpr int STAGE = 2 * SK + SKB + SM; // elements: K, V, K_b, fp32 vector mask
-    static constexpr int LDS_BYTES = 2 * STAGE * 2;
+    static constexpr int LDS_BYTES = 2 * STAGE * 2 * SPLIT;
+    static_assert(LDS_BYTES <= 160 * 1024 && (SPLIT == 1 || LDS_BYTES >= NDV_ * 16384 + 4 * 512), "");
     // head dim <= 64: three workgroups per compute unit (168 registers, 3 x 40 KB)
-    static constexpr int WAVES_EU = NKD <= 4 ? 3 : 2;
+    static constexpr int WAVES_EU = NKD <= 4 && SPLIT == 1 ? 3 : 2;
     // Exponentials before another wave's products.  us, against the products first: causal B4 H32 L=4096 d128 629 -> 610, fp16 d64
     // r16 8 x 8 x (1000 x 1500) with a padding mask 44.6 -> 43.9; without a mask at head dim 64 neither (causal B2 H8 L=4096
     // 62.0, products first 63.7, exponentials first 66.3).
@@ -44,8 +45,9 @@ struct FwdWideCfg {
 template <class T, class C>
 __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::WAVES_EU, C::WAVES_EU))) void fwd_wide_kernel(const FwdArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    uint16_t *stage0 = reinterpret_cast<uint16_t *>(smem);
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int grp = C::SPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8); // takes its share of the tiles of keys, in stages of its own
+    uint16_t *stage0 = reinterpret_cast<uint16_t *>(smem) + grp * 2 * C::STAGE;
+    const int tid = threadIdx.x & (64 * C::NWAVES - 1), lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 31, g = lane >> 5;
 
@@ -61,6 +63,10 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     const uint16_t *kbase = a.k.ptr + b * a.k.sb + h * a.k.sh;
     const uint16_t *vbase = a.v.ptr + b * a.v.sb + h * a.v.sh;
 
+    int k_end = a.Lk;
+    if (a.causal && m0 + C::BM < k_end) k_end = m0 + C::BM;
+    const int ntiles = (k_end + C::BN - 1) / C::BN, walk = (ntiles + C::SPLIT - 1) / C::SPLIT, tile0 = grp * walk;
+
     u32x4_t qr[C::NK];
 #pragma unroll
     for (int t = 0; t < C::NKD; ++t) qr[t] = load_chunk<true>(qbase, a.q.ss, query, a.Lq, 16 * t + 8 * g, a.d);
@@ -74,7 +80,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
             if (C::FOLD && a.scale != 1.f) x = fold_scale_chunk<T>(x, 1.f / a.scale, C::low_parts(a), low);
             qr[C::NKD + t] = x;
         }
-        kbd.init(a.kb.ptr + b * a.kb.sb + h * a.kb.sh, a.kb.ss, a.r, C::low_parts(a), wave, lane, 0);
+        kbd.init(a.kb.ptr + b * a.kb.sb + h * a.kb.sh, a.kb.ss, a.r, C::low_parts(a), wave, lane, tile0 * C::BN);
     }
     f32x16_t acc_o[C::NDV];
 #pragma unroll
@@ -85,19 +91,15 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     const float to_log2 = C::FOLD ? a.scale * kLog2e : kLog2e;
     const float lag = 8.0f / to_log2;
 
-    int k_end = a.Lk;
-    if (a.causal && m0 + C::BM < k_end) k_end = m0 + C::BM;
-    const int ntiles = (k_end + C::BN - 1) / C::BN;
-
     {   // clear the stages once: the zero padding of the channel dimension is never rewritten
         u32x4_t *z = reinterpret_cast<u32x4_t *>(smem);
-        for (int i = tid; i < C::LDS_BYTES / 16; i += C::NTHREADS) z[i] = u32x4_t{0u, 0u, 0u, 0u};
+        for (int i = threadIdx.x; i < C::LDS_BYTES / 16; i += C::NTHREADS) z[i] = u32x4_t{0u, 0u, 0u, 0u};
     }
     __syncthreads();
 
     TileDma<C::BN, C::ROWCH, C::NWAVES, false> kd, vd;
-    kd.init(kbase, a.k.ss, a.d, C::ROWCH, nullptr, 0, 0, wave, lane, 0);
-    vd.init(vbase, a.v.ss, a.d, C::ROWCH, nullptr, 0, 0, wave, lane, 0);
+    kd.init(kbase, a.k.ss, a.d, C::ROWCH, nullptr, 0, 0, wave, lane, tile0 * C::BN);
+    vd.init(vbase, a.v.ss, a.d, C::ROWCH, nullptr, 0, 0, wave, lane, tile0 * C::BN);
     auto issue = [&](int buf, int n0) {
         const uint32_t base = lds_addr_of(stage0 + buf * C::STAGE);
         kd.issue(base, n0, a.Lk, a.k.ss, 0, C::ROWCH);
@@ -114,17 +116,19 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     auto store_vmask = [&](int buf) {
         if (tid < C::BN) reinterpret_cast<float *>(stage0 + buf * C::STAGE + 2 * C::SK + C::SKB)[tid] = mkey;
     };
-    issue(0, 0);
-    if constexpr (C::VMASK) {
-        load_vmask(0);
-        store_vmask(0);
+    if (C::SPLIT == 1 || tile0 < ntiles) {
+        issue(0, tile0 * C::BN);
+        if constexpr (C::VMASK) {
+            load_vmask(tile0 * C::BN);
+            store_vmask(0);
+        }
     }
     wait_vmcnt<0>();
     barrier_lds();
 
-    for (int it = 0; it < ntiles; ++it) {
-        const int cur = it & 1, n0 = it * C::BN;
-        const bool more = it + 1 < ntiles;
+    for (int it = 0; it < walk; ++it) {
+        const int cur = it & 1, n0 = (tile0 + it) * C::BN;
+        const bool more = it + 1 < walk && (C::SPLIT == 1 || tile0 + it + 1 < ntiles);
         if (more) {
             issue(cur ^ 1, n0 + C::BN);
             if constexpr (C::VMASK) load_vmask(n0 + C::BN);
@@ -132,7 +136,7 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         const uint16_t *sK = stage0 + cur * C::STAGE, *sV = sK + C::SK;
         const uint8_t *sKb = reinterpret_cast<const uint8_t *>(sV + C::SK);
         // (a tile hidden from every query of this wave: so are all later ones, but the copies and barriers go on)
-        if (!(a.causal && n0 > wq0 + 31) && wq0 < a.Lq) {
+        if (!(a.causal && n0 > wq0 + 31) && wq0 < a.Lq && (C::SPLIT == 1 || tile0 + it < ntiles)) {
             if constexpr (C::EXP_FIRST) __builtin_amdgcn_s_setprio(0);
             f32x16_t s[C::KBLK];
 #pragma unroll
@@ -246,6 +250,29 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
         barrier_lds();
     }
 
+    if constexpr (C::SPLIT == 2) { // the second group's sums to the first one's (the stages are free: the loop ends with a barrier)
+        uint8_t *ex = smem + wave * 4096;
+        float *em = reinterpret_cast<float *>(smem + C::NDV * 16384 + wave * 512) + lane;
+#pragma unroll
+        for (int n = 0; n < C::NDV; ++n) asm volatile("s_nop 11" : "+v"(acc_o[n]));
+        if (grp == 1) {
+#pragma unroll
+            for (int n = 0; n < C::NDV; ++n) lds_put_block(ex + n * 16384, acc_o[n], lane);
+            em[0] = m_ref;
+            em[64] = l_run;
+        }
+        barrier_lds();
+        if (grp == 1) return;
+        float mine, other;
+        join_references(m_ref, em[0], to_log2, mine, other);
+        l_run = l_run * mine + em[64] * other;
+#pragma unroll
+        for (int n = 0; n < C::NDV; ++n) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc_o[n][v] *= mine;
+            lds_add_block(ex + n * 16384, acc_o[n], lane, other);
+        }
+    }
     uint16_t *obase = const_cast<uint16_t *>(a.o.ptr) + b * a.o.sb + h * a.o.sh;
     int q = query;
     asm volatile("" : "+v"(q)); // (keeps the address arithmetic below the key loop)
@@ -258,9 +285,9 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(C::
     for (int n = 0; n < C::NDV; ++n) store_acc_rows<T, true>(orow + 32 * n, ok, true, acc_o[n], inv, a.d - 32 * n, g);
 }
 
-template <class T, int NKD, int NKR, int NDV, int MASK, bool FOLD>
-static hipError_t launch_fwd_wide(const FwdArgs &a0, hipStream_t stream) {
-    typedef FwdWideCfg<T, NKD, NKR, NDV, MASK, FOLD> C;
+template <class T, int NKD, int NKR, int NDV, int MASK, bool FOLD, int SPLIT>
+static hipError_t launch_fwd_wide_split(const FwdArgs &a0, hipStream_t stream) {
+    typedef FwdWideCfg<T, NKD, NKR, NDV, MASK, FOLD, SPLIT> C;
     FwdArgs a = a0;
     a.ntiles_m = (a.Lq + C::BM - 1) / C::BM;
     auto kern = fwd_wide_kernel<T, C>;
@@ -269,6 +296,21 @@ static hipError_t launch_fwd_wide(const FwdArgs &a0, hipStream_t stream) {
     if (e != hipSuccess) return e;
     const int64_t total = (int64_t)a.ntiles_m * a.B * a.H;
     return launch_flat(kern, total, C::NTHREADS, C::LDS_BYTES, stream, a);
+}
+
+// Two groups of waves, which split the keys and join their sums in LDS: up to one workgroup a compute unit, under a causal mask, where a launch
+// lasts as long as its longest workgroup, up to two if that one is long. us, one group / two, rank 8: head dim 64, 64 workgroups (B1 H8) of 1000
+// keys 19.1 / 16.8, causal 19.3 / 16.8, padded 22.8 / 18.9; 192 of 1500 27.6 / 23.9, of 3000 (B2 H4) 48.1 / 37.4; 256 of 1024 (B2 H16) 20.1 / 18.3, of 4096
+// (B1 H8) 59.8 / 49.4; of 512 keys (B1 H8) 11.6 / 11.1, of 256 7.66 / 7.75; 384 of 1500 (B1 H32) 37.4 / 43.2, causal 27.9 / 25.9, of 700 causal 16.7 / 21.0;
+// 512 causal of 2048 36.8 / 36.3, of 8192 128.6 / 105.7; head dim 128, 64 of 1000 26.2 / 24.0, 256 of 4096 86.7 / 78.0, 512 causal of 8192 196 / 158.
+inline bool wide_split(const FwdArgs &a) {
+    const int64_t wgs = (int64_t)a.B * a.H * ((a.Lq + 127) / 128);
+    return a.Lk >= 512 && wgs <= (a.causal && a.Lk >= 1024 ? 2 : 1) * (int64_t)num_cus();
+}
+
+template <class T, int NKD, int NKR, int NDV, int MASK, bool FOLD>
+static hipError_t launch_fwd_wide(const FwdArgs &a, hipStream_t stream) {
+    return wide_split(a) ? launch_fwd_wide_split<T, NKD, NKR, NDV, MASK, FOLD, 2>(a, stream) : launch_fwd_wide_split<T, NKD, NKR, NDV, MASK, FOLD, 1>(a, stream);
 }
 
 } // namespace fb

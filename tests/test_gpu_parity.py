@@ -304,6 +304,25 @@ def test_wide_heads(gpu_device, d, r, Lq, Lk, scale, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,r,Lq,Lk,scale", [(64, 8, 130, 577, None), (40, 24, 577, 513, 0.3), (128, 16, 65, 705, None), (64, 0, 1100, 1030, 1.0), (72, 8, 129, 512, -0.2),
+                                             (64, 16, 513, 641, 0.125), (64, 32, 700, 64, None), (64, 0, 1, 520, None)])
+def test_wide_heads_with_the_walk_split(gpu_device, d, r, Lq, Lk, scale, dtype):
+    """Two groups of waves for one block of queries (forward from 512 keys, dq at head dims 33 to 64 above 512) or of keys (dk/dv above 512
+    queries) on small grids: odd numbers of tiles, a half that a causal mask hides or that a mask switches off for a whole entry."""
+    for kind in (None, "causal", "first", "second"):
+        mask = None
+        if kind in ("first", "second"):
+            mask = torch.randn(2, 1, 1, Lk, generator=torch.Generator().manual_seed(Lk))
+            half = ((Lk + 63) // 64 + 1) // 2 * 64
+            if half >= Lk:
+                continue
+            mask[1, ..., half:] = float("-inf") if kind == "second" else mask[1, ..., half:]
+            mask[1, ..., :half] = float("-inf") if kind == "first" else mask[1, ..., :half]
+            mask = mask.to(dtype if Lq % 2 else torch.float32)
+        _case(gpu_device, 2, Lq, Lk, 3, d, r, dtype, kind == "causal", mask=mask, scale=scale, seed=d + r + Lk, o_by_magnitude=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("r,Lq,Lk,scale", [(16, 1, 1, None), (32, 127, 63, None), (24, 129, 64, None), (0, 128, 65, None), (8, 33, 640, 1.0), (32, 130, 129, 1.0),
                                            (16, 257, 127, -0.2), (0, 31, 192, -0.1), (16, 64, 530, 0.0625), (8, 95, 100, None),
                                            (8, 129, 520, 3.0)])
