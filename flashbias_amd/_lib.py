@@ -17,7 +17,7 @@ EXPORTS = ("fb_version", "fb_init", "fb_last_error", "fb_bwd_workspace_bytes", "
            "fb_sum_over_batch", "fb_resize_rank", "fb_resize_ranks", "fb_alibi_factors", "fb_cosine_workspace_bytes", "fb_cosine_fwd", "fb_cosine_bwd",
            "fb_window_ready", "fb_window_workspace_bytes", "fb_window_fwd", "fb_window_bwd",
            "fb_weight_grad_workspace_bytes", "fb_weight_grad_recommended", "fb_weight_grad",
-           "fb_project_recommended", "fb_project", "fb_linear_recommended", "fb_linear",
+           "fb_project_recommended", "fb_project", "fb_linear_recommended", "fb_linear", "fb_transpose",
            "fb_bwd_preprocess", "fb_bwd_dkv", "fb_bwd_dq", "fb_bwd_static")
 
 
@@ -105,6 +105,8 @@ def load():
     lib.fb_linear.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int64,
                               ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
     lib.fb_linear.restype = ctypes.c_int
+    lib.fb_transpose.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+    lib.fb_transpose.restype = ctypes.c_int
     _lib = lib
     return lib
 

@@ -47,6 +47,7 @@ hipError_t launch_project(const void *x, int64_t ldx, const void *const *w, void
 // a projection of many tokens (fb_linear.hip)
 bool linear_recommended(int64_t tokens, int n, int k);
 hipError_t launch_linear(const void *x, int64_t ldx, const void *w, const void *b, void *y, int64_t tokens, int n, int k, bool bf16, hipStream_t stream);
+hipError_t launch_transpose(const void *in, void *out, int rows, int cols, hipStream_t stream);
 
 hipError_t launch_fwd(const FwdArgs &a, bool bf16, hipStream_t stream) {
     if (window_forward(a)) return bf16 ? launch_fwd_win_bf16_2(a, stream) : launch_fwd_win_f16_2(a, stream);
@@ -457,6 +458,16 @@ int fb_linear(const void *x, int64_t ldx, const void *w, const void *b, void *y,
         if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return fb::api_fail(FB_ERR_STRIDE, "fb_linear: tensors must be 16-byte aligned");
     if (reinterpret_cast<uintptr_t>(b) % 4 != 0) return fb::api_fail(FB_ERR_STRIDE, "fb_linear: the bias must be 4-byte aligned");
     return launched(fb::launch_linear(x, ldx, w, b, y, tokens, n, k, dtype == FB_BF16, static_cast<hipStream_t>(stream)), "fb_linear");
+}
+
+int fb_transpose(const void *in, void *out, int rows, int cols, void *stream) {
+    fb::api_clear_error();
+    if (!in || !out) return fb::api_fail(FB_ERR_NULL, "fb_transpose: null pointer");
+    if (rows <= 0 || cols <= 0 || rows > (1 << 16) || cols > (1 << 16) || rows % 64 != 0 || cols % 64 != 0)
+        return fb::api_fail(FB_ERR_SHAPE, "fb_transpose: rows and columns must be multiples of 64 up to 65536");
+    for (const void *p : {in, static_cast<const void *>(out)})
+        if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return fb::api_fail(FB_ERR_STRIDE, "fb_transpose: matrices must be 16-byte aligned");
+    return launched(fb::launch_transpose(in, out, rows, cols, static_cast<hipStream_t>(stream)), "fb_transpose");
 }
 
 int fb_bwd_static(const fb_params *p, void *stream) {

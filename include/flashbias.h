@@ -292,6 +292,9 @@ int fb_project(const void *x, int64_t ldx, const void *const *w, void *const *y,
  * fb_linear_recommended: 1 where this was measured ahead of the vendor library's product of the same shape. */
 int fb_linear_recommended(int64_t tokens, int n, int k);
 int fb_linear(const void *x, int64_t ldx, const void *w, const void *b, void *y, int dtype, int64_t tokens, int n, int k, void *stream);
+/* out (cols, rows) = in (rows, cols)^T of 16-bit elements, both contiguous and 16-byte aligned, rows and cols multiples of 64 up to 65536: the
+ * weight of the product above where it contracts the other way (an input's gradient dy w). */
+int fb_transpose(const void *in, void *out, int rows, int cols, void *stream);
 
 #ifdef __cplusplus
 }

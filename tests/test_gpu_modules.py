@@ -500,6 +500,16 @@ def test_linear(gpu_device, dtype, tokens, n, k):
     assert lib.fb_linear(x.data_ptr(), x.stride(0), w.data_ptr(), None, y.data_ptr(), CODES[dtype], tokens, n, k - 8, interface._stream()) != 0
 
 
+@pytest.mark.parametrize("rows,cols", [(64, 64), (512, 1536), (192, 128)])
+def test_transpose(gpu_device, rows, cols):
+    lib = _lib.load()
+    x = torch.randint(0, 1 << 15, (rows, cols), device=gpu_device, dtype=torch.int16)
+    whole = torch.full((rows * cols + 64,), 7, device=gpu_device, dtype=torch.int16)
+    _lib.check_status(lib.fb_transpose(x.data_ptr(), whole.data_ptr(), rows, cols, interface._stream()))
+    assert torch.equal(whole[:rows * cols].view(cols, rows), x.t()) and (whole[rows * cols:] == 7).all()
+    assert lib.fb_transpose(x.data_ptr(), whole.data_ptr(), rows - 8, cols, interface._stream()) != 0
+
+
 @pytest.mark.parametrize("n,bias", [(384, False), (128, True)])
 def test_projection_of_many_tokens_takes_the_product_and_leaves_the_rest(gpu_device, n, bias):
     torch.manual_seed(4)
@@ -519,6 +529,14 @@ def test_projection_of_many_tokens_takes_the_product_and_leaves_the_rest(gpu_dev
             assert ext.linear(x, layer.weight, layer.bias) is None
     y = modules._project(layer, x)
     assert "LinearFn" in y.grad_fn.name() and torch.equal(y.detach(), got)
+    # the input's gradient, by the same kernel, from rows of a wider tensor and from rows that it has to copy
+    x.requires_grad_(True)
+    y = modules._project(layer, x)
+    wide = torch.randn(1025, 128, n + 8, device=gpu_device, dtype=torch.bfloat16)
+    for dy in (wide[..., :n].contiguous(), wide[..., 8:], wide[..., 4:n + 4], wide[:1, :1, :n].expand(1025, 128, n)):
+        (dx,) = torch.autograd.grad(y, [x], dy, retain_graph=True)
+        want = dy.double() @ layer.weight.double()
+        assert dx.shape == x.shape and (dx.double() - want).norm() <= many * want.norm()
 
 
 def test_block_projections_take_the_kernel_and_leave_the_rest(gpu_device):
