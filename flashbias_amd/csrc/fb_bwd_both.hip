@@ -62,10 +62,10 @@ static hipError_t launch_both_lean(const BwdArgs &a0, hipStream_t stream) {
 // tails.  The ids alternate as above, which keeps each kind's own order (longest first within every XCD's share,
 // work_order in fb_order.h).  With the general kernels' bodies before: training step causal r2 as 16 B1 H50 L=2048 147 -> 137 us, r16 B1
 // H24 L=4096 251 -> 232, r32 B1 H8 L=3000 205 -> 167.
-template <class T, int NKR, bool FOLD, bool BG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void bwd_both_kernel(const BwdArgs a) {
-    typedef DqMidCfg<T, 2, NKR, FOLD, BG> Cq;
-    typedef DkvMidCfg<T, 2, NKR, kNoMask, FOLD, BG> Ck;
+template <class T, int NKR, bool FOLD, bool BG, int SPLIT>
+__global__ __launch_bounds__(256 * SPLIT) __attribute__((amdgpu_waves_per_eu(SPLIT == 1 ? 3 : 2, SPLIT == 1 ? 3 : 2))) void bwd_both_kernel(const BwdArgs a) {
+    typedef DqMidCfg<T, 2, NKR, FOLD, BG, SPLIT> Cq;
+    typedef DkvMidCfg<T, 2, NKR, kNoMask, FOLD, BG, SPLIT> Ck;
     const int group = a.group > 1 ? a.group : 1;
     const int nbg = (a.B + group - 1) / group;
     const int ndq = a.ntiles_m * nbg * a.H, ndkv = a.ntiles_n * nbg * a.H;
@@ -77,22 +77,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         bwd_dkv_mid_body<T, Ck>(a, id < 2 * paired ? (id >> 4) * 8 + (id & 7) : id - paired);
 }
 
-template <class T, int NKR, bool FOLD, bool BG>
-static hipError_t launch_both_general(const BwdArgs &a0, hipStream_t stream) {
-    typedef DqMidCfg<T, 2, NKR, FOLD, BG> Cq;
-    typedef DkvMidCfg<T, 2, NKR, kNoMask, FOLD, BG> Ck;
-    static_assert(Cq::NTHREADS == 256 && Ck::NTHREADS == 256 && Cq::BM == 128 && Ck::BN == 128, "128-row workgroups of four waves");
+template <class T, int NKR, bool FOLD, bool BG, int SPLIT>
+static hipError_t launch_both_split(const BwdArgs &a0, hipStream_t stream) {
+    typedef DqMidCfg<T, 2, NKR, FOLD, BG, SPLIT> Cq;
+    typedef DkvMidCfg<T, 2, NKR, kNoMask, FOLD, BG, SPLIT> Ck;
+    static_assert(Cq::NTHREADS == 256 * SPLIT && Ck::NTHREADS == 256 * SPLIT && Cq::BM == 128 && Ck::BN == 128, "128 rows a workgroup, four waves a group");
     BwdArgs a = a0;
     a.ntiles_m = (a.Lq + Cq::BM - 1) / Cq::BM;
     a.ntiles_n = (a.Lk + Ck::BN - 1) / Ck::BN;
     constexpr int lds = Cq::LDS_BYTES > Ck::LDS_BYTES ? Cq::LDS_BYTES : Ck::LDS_BYTES;
-    auto kern = bwd_both_kernel<T, NKR, FOLD, BG>;
+    auto kern = bwd_both_kernel<T, NKR, FOLD, BG, SPLIT>;
     static KernelOnce once;
     const hipError_t e = allow_lds(kern, lds, once);
     if (e != hipSuccess) return e;
     const int group = a.group > 1 ? a.group : 1;
     const int64_t total = ((int64_t)a.ntiles_m + a.ntiles_n) * ((a.B + group - 1) / group) * a.H;
-    return launch_flat(kern, total, 256, lds, stream, a);
+    return launch_flat(kern, total, 256 * SPLIT, lds, stream, a);
+}
+
+template <class T, int NKR, bool FOLD, bool BG>
+static hipError_t launch_both_general(const BwdArgs &a, hipStream_t stream) {
+    return both_split(a) ? launch_both_split<T, NKR, FOLD, BG, 2>(a, stream) : launch_both_split<T, NKR, FOLD, BG, 1>(a, stream);
 }
 
 template <class T, int NKR>

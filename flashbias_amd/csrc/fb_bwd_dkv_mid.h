@@ -20,7 +20,7 @@
 // 4 of 301 225 -> 213; r32 fp16 with a padding mask, 2 x 4 x (1000 x 3000) 170 -> 160.  Not kept: four waves without dk_bias (spills:
 // 399 -> 409).
 //
-// SPLIT (head dims above 32): on small grids a second group of four waves takes the second half of the queries for the same keys, in stages of its own,
+// SPLIT: on small grids a second group of four waves takes the second half of the queries for the same keys, in stages of its own,
 // and hands its sums over in LDS (mid_split).  At 1 x 8 x 1000 one group takes 2.6 us for a step of 64 queries, most of it waiting.
 #pragma once
 #include "fb_lean_tiles.h"
@@ -41,8 +41,8 @@ struct DkvMidCfg {
     // a stage, bytes: Q, dO, Q_b rows of 32 or 64, lse * log2(e) and -delta
     static constexpr int SQ = BMQ * RB, SQB = NKR > 0 ? BMQ * CPR * 16 : 0, STAGE = 2 * SQ + SQB + 8 * BMQ, NSTAGE = 2;
     static constexpr int LDS_BYTES = NSTAGE * STAGE * SPLIT;
-    static constexpr int WAVES_EU = NKD == 4 ? 2 : 3;
-    static_assert(WAVES_EU * LDS_BYTES / SPLIT <= 160 * 1024 && (SPLIT == 1 || (NKD == 4 && LDS_BYTES >= 4 * 16384)), "");
+    static constexpr int WAVES_EU = NKD == 4 || SPLIT == 2 ? 2 : 3;
+    static_assert(WAVES_EU * LDS_BYTES / SPLIT <= 160 * 1024 && (SPLIT == 1 || LDS_BYTES >= 2 * NDV * 16384), "");
     // Rank above 16 with dk_bias at head dims above 32: the places of the copies are formed where they are used.  Kept, they spill (24
     // bytes), and a reload waits for the tile that has just been requested: training step, us, r32 causal B2 H8 L=4096 272 -> 265,
     // B4 H16 L=2048 405 -> 400, B1 H4 L=1000 87.3 -> 85.  The others have the registers (r2 as 16 causal B2 H16 L=2048 136.5 -> 138).
@@ -370,9 +370,7 @@ static hipError_t launch_dkv_mid_split(const BwdArgs &a0, hipStream_t stream) {
 
 template <class T, int NKD, int NKR, int MASK, bool FOLD, bool BG>
 static hipError_t launch_dkv_mid_bg(const BwdArgs &a, hipStream_t stream) {
-    if constexpr (NKD == 4) {
-        if (mid_split(a, a.Lk, a.Lq)) return launch_dkv_mid_split<T, NKD, NKR, MASK, FOLD, BG, 2>(a, stream);
-    }
+    if (mid_split(a, a.Lk, a.Lq)) return launch_dkv_mid_split<T, NKD, NKR, MASK, FOLD, BG, 2>(a, stream);
     return launch_dkv_mid_split<T, NKD, NKR, MASK, FOLD, BG>(a, stream);
 }
 

@@ -745,7 +745,7 @@ static hipError_t launch_dq_cfg(const BwdArgs &a, hipStream_t stream) {
     }
     constexpr int MID = dq_mid_use(NKD, NKR);
     if constexpr (MID > 0) {
-        if (vec && (MID == 2 || !a.dqb.ptr))
+        if (vec && (MID == 2 || !a.dqb.ptr || both_split(a)))
             return fold_scale_ok<T>(a.scale, a.r, a.Lk) ? launch_dq_mid<T, NKD, NKR, true>(a, stream) : launch_dq_mid<T, NKD, NKR, false>(a, stream);
     }
     if constexpr (MID < 2) {

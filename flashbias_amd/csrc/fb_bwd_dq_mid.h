@@ -14,7 +14,7 @@
 // With a vector mask it was behind (its values a tile at a time in the stage: fp16 d64 8 x 8 x (1000 x 1500) 194 -> 196, d32 r8 157.8 ->
 // 158.3), so those stay with the general kernel.
 //
-// SPLIT (head dims above 32): on small grids a second group of four waves takes the second half of the keys for the same queries, in stages of its own,
+// SPLIT: on small grids a second group of four waves takes the second half of the keys for the same queries, in stages of its own,
 // and hands its sums over in LDS (mid_split).
 #pragma once
 #include "fb_lean_tiles.h"
@@ -35,8 +35,8 @@ struct DqMidCfg {
     static constexpr int SK = BN * RB, SKB = NKR > 0 ? BN * CPR * 16 : 0, STAGE = 2 * SK + SKB;
     static constexpr int LDS_BYTES = 2 * STAGE * SPLIT;
     // (head dim 32: 121-127 registers without dq_bias at ranks up to 16; at rank 32 129-135, with it 139-155)
-    static constexpr int WAVES_EU = NKD == 4 ? 2 : BG || NKR == 2 ? 3 : 4;
-    static_assert(WAVES_EU * LDS_BYTES / SPLIT <= 160 * 1024 && (SPLIT == 1 || (NKD == 4 && LDS_BYTES >= (NDQ + 1) * 4 * 4096)), "");
+    static constexpr int WAVES_EU = NKD == 4 || SPLIT == 2 ? 2 : BG || NKR == 2 ? 3 : 4;
+    static_assert(WAVES_EU * LDS_BYTES / SPLIT <= 160 * 1024 && (SPLIT == 1 || LDS_BYTES >= (NDQ + 1) * 4 * 4096), "");
     static constexpr bool ORDERED = NKD == 4; // two waves a SIMD: the order is fixed phase by phase
     static __device__ __forceinline__ bool low_parts(const BwdArgs &a) { return FOLD_ && NKR_ == 1 && a.r <= 8 && a.scale != 1.f; }
 };
@@ -300,21 +300,22 @@ static hipError_t launch_dq_mid_split(const BwdArgs &a0, hipStream_t stream) {
 
 template <class T, int NKD, int NKR, bool FOLD, bool BG>
 static hipError_t launch_dq_mid_bg(const BwdArgs &a, hipStream_t stream) {
-    if constexpr (NKD == 4) {
-        if (mid_split(a, a.Lq, a.Lk)) return launch_dq_mid_split<T, NKD, NKR, FOLD, BG, 2>(a, stream);
-    }
+    if (mid_split(a, a.Lq, a.Lk)) return launch_dq_mid_split<T, NKD, NKR, FOLD, BG, 2>(a, stream);
     return launch_dq_mid_split<T, NKD, NKR, FOLD, BG>(a, stream);
 }
 
 // Whether aligned calls without a mask take this kernel: 2 all, 1 those that want no dq_bias, 0 none (measured above).  Head dims above
 // 32, and at head dim 32 ranks above 16 and calls that want no dq_bias; with it the general kernel's two query blocks a wave
-// share enough to stay level at ranks up to 16 (B2 H4 L=8192 r16 training step 537 / 538, B8 H16 L=700 100 / 99.5).
+// share enough to stay level at ranks up to 16, on grids where the walk is not split (B2 H4 L=8192 r16 training step 537 / 538, B8 H16 L=700 100 / 99.5).
 constexpr int dq_mid_use(int nkd, int nkr) { return nkr > 2 ? 0 : nkd == 4 || (nkd == 2 && nkr == 2) ? 2 : nkd == 2 && nkr == 1 ? 1 : 0; }
 
 template <class T, int NKD, int NKR, bool FOLD>
 static hipError_t launch_dq_mid(const BwdArgs &a, hipStream_t stream) {
     if constexpr (NKR > 0 && dq_mid_use(NKD, NKR) == 2) {
         if (a.dqb.ptr) return launch_dq_mid_bg<T, NKD, NKR, FOLD, true>(a, stream);
+    }
+    if constexpr (NKR > 0 && dq_mid_use(NKD, NKR) == 1) {
+        if (a.dqb.ptr) return launch_dq_mid_split<T, NKD, NKR, FOLD, true, 2>(a, stream); // (both_split)
     }
     return launch_dq_mid_bg<T, NKD, NKR, FOLD, false>(a, stream); // (no dq_bias wanted: without its products)
 }

@@ -300,14 +300,27 @@ inline bool mixed_general_backward(const BwdArgs &a0) {
     return 2 * most <= (a.causal ? 9 : 3) * (int64_t)num_cus();
 }
 
-// Whether dq (rows: queries, walked: keys) and dk/dv (the other way round) of head dims 33 to 64 take two groups of waves a workgroup, which
+// Whether dq and dk/dv of head dims 17 to 32 without a mask, in one launch or two (the same bits), take two groups of waves a workgroup, which split what
+// it walks (mid_split): up to one workgroup of either kind a compute unit, causal one and a half. Training
+// step, us, one group / two, rank 16: 128 workgroups (B1 H8) of 1000 positions 53.6 / 43.4, causal 42.7 / 38.5; 256 of 2000 (B1 H8) 96.1 / 76.1, of 2048 (B2
+// H4) 72.0 / 64.0, of 1000 (B1 H16) 55.7 / 46.2, of 512 (B2 H16) 28.5 / 28.0, of 256 (B8 H8) 21.6 / 22.3; 288 of 1100 67.6 / 69.3, causal 49.2 / 44.6; 384 of 1500 87.9 /
+// 88.6, causal 60.9 / 57.5; rank 32, 256 of 2000 100.3 / 79.7.
+inline bool both_split(const BwdArgs &a) {
+    const int64_t wgs = (int64_t)a.B * a.H * ((a.Lq + 127) / 128 + (a.Lk + 127) / 128);
+    return a.group <= 1 && a.Lq >= 512 && a.Lk >= 512 && 2 * wgs <= (a.causal ? 3 : 2) * (int64_t)num_cus();
+}
+
+// Whether dq (rows: queries, walked: keys) and dk/dv (the other way round) of head dims 17 to 64 take two groups of waves a workgroup, which
 // split what it walks and add up their sums in LDS: where four waves leave a SIMD with one, which waits for LDS and its own chains. Training step,
 // both kernels, us, one group / two, rank 8: 64 workgroups (B1 H8) of 1000 keys 83.8 / 70.1, causal 74.0 / 66.9, padded 94.0 / 84.4; 192 of
 // 1500 121.9 / 101.0, of 3000 (B2 H4) 221 / 165; 256 of 1024 (B2 H16) 77.0 / 73.5, of 4096 (B1 H8) 248 / 213; of 512 keys (B1 H8) 44.3 / 44.1, of 256
 // 30.3 / 33.0; 384 of 1500 (B1 H32) 167.5 / 172.5, causal 113.2 / 106.3, of 700 causal 67.5 / 77.2; 512 of 2048 (B2 H16) 224 / 227, causal 149.3 / 150.3.
+// Head dim 32 with a padding mask (dk/dv): 64 (B1 H8) of 1000 78.2 / 68.5, 192 of 3000 (B2 H4) 200 / 166, 256 of 1000 (B1 H32) 82.1 / 73.1, of 4096 (B1 H8) 228 / 215,
+// 384 of 1500 129.8 / 132.8.
 inline bool mid_split(const BwdArgs &a, int rows, int walked) {
+    if (a.d <= 32 && a.mask.type == kNoMask) return both_split(a);
     const int64_t wgs = (int64_t)a.B * a.H * ((rows + 127) / 128);
-    return a.group <= 1 && walked > 512 && 2 * wgs <= (a.causal && walked >= 1024 ? 3 : 2) * (int64_t)num_cus();
+    return a.group <= 1 && walked >= 512 && 2 * wgs <= (a.causal && walked >= 1024 ? 3 : 2) * (int64_t)num_cus();
 }
 
 } // namespace fb

@@ -305,10 +305,11 @@ def test_wide_heads(gpu_device, d, r, Lq, Lk, scale, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d,r,Lq,Lk,scale", [(64, 8, 130, 577, None), (40, 24, 577, 513, 0.3), (128, 16, 65, 705, None), (64, 0, 1100, 1030, 1.0), (72, 8, 129, 512, -0.2),
-                                             (64, 16, 513, 641, 0.125), (64, 32, 700, 64, None), (64, 0, 1, 520, None)])
+                                             (64, 16, 513, 641, 0.125), (64, 32, 700, 64, None), (64, 0, 1, 520, None), (32, 16, 512, 512, None),
+                                             (32, 32, 1000, 1024, 0.5), (24, 8, 577, 641, None), (32, 16, 530, 512, -0.2)])
 def test_wide_heads_with_the_walk_split(gpu_device, d, r, Lq, Lk, scale, dtype):
-    """Two groups of waves for one block of queries (forward from 512 keys, dq at head dims 33 to 64 above 512) or of keys (dk/dv above 512
-    queries) on small grids: odd numbers of tiles, a half that a causal mask hides or that a mask switches off for a whole entry."""
+    """Two groups of waves for one block of queries (forward, and dq at head dims up to 64, from 512 keys) or of keys (dk/dv from 512 queries; at head
+    dim 32 both kinds in one launch or in two) on small grids: odd numbers of tiles, a half that a causal mask hides or that a mask switches off for a whole entry."""
     for kind in (None, "causal", "first", "second"):
         mask = None
         if kind in ("first", "second"):
