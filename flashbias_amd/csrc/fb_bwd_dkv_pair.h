@@ -179,15 +179,17 @@ __global__ __launch_bounds__(C::NTHREADS) __attribute__((amdgpu_waves_per_eu(2, 
                     }
                 };
                 auto hide = [&](f32x16_t &s, int q0) {
+                    // (keys past the end stay: their columns end in no other and are not stored.  Hidden, they cost the wave that holds some of them its every step
+                    // and the launch of a small grid as much: fb_bwd_dkv_mid.h, step of B1 H8 L=1000 d64 70.1 -> 64.1 us.)
                     // (bitwise on purpose, as in the dq kernel: no scalar block between the last MFMA and the branch)
-                    const bool edge = (wk0 + 32 > a.Lk) | (q0 + 32 > a.Lq) | ((a.causal != 0) & (wk0 + 31 > q0));
+                    const bool edge = (q0 + 32 > a.Lq) | ((a.causal != 0) & (wk0 + 31 > q0));
                     if (edge) {
                         int query0 = q0 + 4 * g;
                         asm volatile("" : "+v"(query0)); // (computed here, not kept in registers across the loop)
 #pragma unroll
                         for (int v = 0; v < 16; ++v) {
                             const int query = query0 + 8 * (v >> 2) + (v & 3);
-                            if (key >= a.Lk || query >= a.Lq || (a.causal && key > query)) s[v] = -INFINITY;
+                            if (query >= a.Lq || (a.causal && key > query)) s[v] = -INFINITY;
                         }
                     }
                     asm volatile("s_nop 11" : "+v"(s)); // (fb_bwd_win.hip: wait states across the branch above)

@@ -304,6 +304,20 @@ def test_wide_heads(gpu_device, d, r, Lq, Lk, scale, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,r,Lk", [(32, 16, 33), (64, 8, 100), (64, 32, 161), (128, 8, 97), (128, 16, 300)])
+def test_dkv_of_rows_without_keys(gpu_device, d, r, Lk, dtype):
+    """A ragged last block of keys beside an entry whose mask hides every key that is there (lse = -inf: the block's lanes past the end compute
+    infinities, which must stay theirs): the other entry's gradients are those of a call of its own."""
+    q, k, v, qb, kb, do = [t.to(gpu_device) for t in make_inputs(2, 70, Lk, 2, d, r, dtype, seed=Lk)]
+    mask = torch.zeros(2, 1, 1, Lk, device=gpu_device, dtype=dtype)
+    mask[1] = float("-inf")
+    both = run_gpu(flash_bias_func, q.cpu(), k.cpu(), v.cpu(), qb.cpu(), kb.cpu(), mask.cpu(), False, None, do.cpu(), gpu_device)
+    one = run_gpu(flash_bias_func, *[t[:1].cpu() for t in (q, k, v, qb, kb)], mask[:1].cpu(), False, None, do[:1].cpu(), gpu_device)
+    for got, want in zip(both, one):
+        assert torch.isfinite(got[0]).all() and torch.equal(got[0], want[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d,r,Lq,Lk,scale", [(64, 8, 130, 577, None), (40, 24, 577, 513, 0.3), (128, 16, 65, 705, None), (64, 0, 1100, 1030, 1.0), (72, 8, 129, 512, -0.2),
                                              (64, 16, 513, 641, 0.125), (64, 32, 700, 64, None), (64, 0, 1, 520, None), (32, 16, 512, 512, None),
                                              (32, 32, 1000, 1024, 0.5), (24, 8, 577, 641, None), (32, 16, 530, 512, -0.2)])
