@@ -56,7 +56,7 @@ static hipError_t launch_both_lean(const BwdArgs &a0, hipStream_t stream) {
 }
 
 // The same for head dim 32 with factors of rank 8 ... 32 where the streamlined kernels do not go (aligned, unmasked: the bodies of
-// fb_bwd_dq_mid.h and fb_bwd_dkv_mid.h, three waves a SIMD), where the grid is small in another way: under a causal mask a launch lasts at
+// fb_bwd_dq_mid.h and fb_bwd_dkv_mid.h, three waves a SIMD, on the smallest grids in two groups: both_split), where the grid is small in another way: under a causal mask a launch lasts at
 // least as long as its longest workgroup, which at a few hundred workgroups per kind is about twice what the work
 // would need (B1 H50 L=2048: 800 workgroups of 1 to 16 tiles on 768 slots), and the two kinds in one launch fill each other's
 // tails.  The ids alternate as above, which keeps each kind's own order (longest first within every XCD's share,
