@@ -416,14 +416,17 @@ Tensor many_tokens(const Tensor &x, const Tensor &w, const c10::optional<Tensor>
     return y;
 }
 
-// dy w by the same kernel on the transposed weight, else nothing.  Vendor library / this with the 3 us of the transpose, us: 147456 tokens of 128 to 128
-// 22.7 / 20.1, of 256 to 256 38.5 / 33.6, of 512 to 512 134 / 92, 262144 of 512 to 512 196 / 147, of 384 to 128 59.6 / 44.7; 65536 of 512 to 512
-// 45.9 / 45.1, of 256 to 256 19.0 / 19.9, of 384 to 128 18.3 / 18.2.
+// Whether dy w is left to the same kernel on the transposed weight (asked before dy is copied into rows that it reads).  Vendor library / this with the 3 us
+// of the transpose, us: 147456 tokens of 128 to 128 22.7 / 20.1, of 256 to 256 38.5 / 33.6, of 512 to 512 134 / 92, 262144 of 512 to 512 196 / 147, of 384 to
+// 128 59.6 / 44.7; 65536 of 512 to 512 45.9 / 45.1, of 256 to 256 19.0 / 19.9, of 384 to 128 18.3 / 18.2.
+bool input_gradient_pays(int64_t tokens, const Tensor &w) {
+    const int64_t n = w.size(0), k = w.size(1);
+    return tokens >= 100000 && n % 64 == 0 && k % 64 == 0 && n <= (1 << 16) && k <= (1 << 16) && w.is_contiguous() &&
+           reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 && fb_linear_recommended(tokens, (int)k, (int)n);
+}
 Tensor input_gradient(const Tensor &dy, const Tensor &w) {
     const int64_t tokens = dy.size(0), n = w.size(0), k = w.size(1);
-    if (tokens < 100000 || dy.stride(0) >= (1 << 22) || n % 64 != 0 || k % 64 != 0 || n > (1 << 16) || k > (1 << 16) || !w.is_contiguous() ||
-        reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 != 0 || !fb_linear_recommended(tokens, (int)k, (int)n))
-        return Tensor();
+    if (dy.stride(0) >= (1 << 22)) return Tensor();
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(dy.device());
     const Tensor wt = fresh({k, n}, w.scalar_type(), w.device());
     Tensor dx = fresh({tokens, k}, dy.scalar_type(), dy.device());
@@ -458,10 +461,12 @@ struct LinearFn : public torch::autograd::Function<LinearFn> {
                             reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
             return ok ? t : t.clone(at::MemoryFormat::Contiguous);
         };
-        if (want_x && plain && plain_tensor(w, x)) dx = input_gradient(rows(dy), w);
+        Tensor y2; // dy in such rows, for whoever reads them: copied at most once, and not for a product of the tensor library
+        if (want_x && plain && plain_tensor(w, x) && input_gradient_pays(dy.size(0), w)) dx = input_gradient(y2 = rows(dy), w);
         if (want_x) dx = (dx.defined() ? dx : dy.matmul(w)).reshape(x.sizes());
         if (want_w && plain) {
-            const Tensor y2 = rows(dy), x2 = rows(x.reshape({-1, k}));
+            if (!y2.defined()) y2 = rows(dy);
+            const Tensor x2 = rows(x.reshape({-1, k}));
             dw = fresh({n, k}, x.scalar_type(), x.device());
             if (want_b) db = fresh({n}, x.scalar_type(), x.device());
             const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());

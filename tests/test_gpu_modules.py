@@ -539,6 +539,37 @@ def test_projection_of_many_tokens_takes_the_product_and_leaves_the_rest(gpu_dev
         assert dx.shape == x.shape and (dx.double() - want).norm() <= many * want.norm()
 
 
+# few tokens, whose input gradient is left to the tensor library, and many, which the library's product takes
+@pytest.mark.parametrize("tokens", [20000, 110000])
+def test_projection_backward_copies_a_gradient_once(gpu_device, tokens):
+    """A gradient in rows that the kernels do not read is copied where one of them takes it, and once for both."""
+    torch.manual_seed(7)
+    layer = torch.nn.Linear(256, 256).to(gpu_device, torch.bfloat16)
+    x = torch.randn(tokens, 256, device=gpu_device, dtype=torch.bfloat16, requires_grad=True)
+    wide = torch.randn(tokens, 256 + 8, device=gpu_device, dtype=torch.bfloat16)
+    aligned, shifted = wide[:, :256], wide[:, 4:260]
+    assert shifted.data_ptr() % 16
+    y = modules._project(layer, x)
+    assert "LinearFn" in y.grad_fn.name()
+
+    def allocated(dy, leaves):
+        for _ in range(2):  # (the first call may set up the tensor library)
+            torch.cuda.synchronize()
+            before = torch.cuda.memory_stats()["requested_bytes.all.allocated"]
+            grads = torch.autograd.grad(y, leaves, dy, retain_graph=True)
+            bytes_ = torch.cuda.memory_stats()["requested_bytes.all.allocated"] - before
+        return bytes_, grads
+    copy = tokens * 256 * 2
+    for leaves, copies in (([x], 1 if tokens >= 100000 else 0), ([layer.weight, layer.bias], 1), ([x, layer.weight, layer.bias], 1)):
+        few, _ = allocated(aligned, leaves)
+        more, grads = allocated(shifted, leaves)
+        assert more - few == copies * copy, (len(leaves), (more - few) / copy)
+        d = shifted.double()
+        for name, g in zip(("weight", "bias") if len(leaves) == 2 else ("x", "weight", "bias"), grads):
+            want = d @ layer.weight.double() if name == "x" else d.t().contiguous() @ x.detach().double() if name == "weight" else d.sum(0)
+            assert (g.double() - want).norm() <= 1.01 * 2.0 ** -8 * want.norm(), name
+
+
 def test_block_projections_take_the_kernel_and_leave_the_rest(gpu_device):
     torch.manual_seed(3)
     layers = [torch.nn.Linear(128, 136, bias=False).to(gpu_device, torch.bfloat16) for _ in range(3)]
