@@ -359,7 +359,10 @@ static int check_window(const fb_params *p, const fb_cosine *c, bool backward) {
     return FB_OK;
 }
 
-int fb_window_ready(const fb_params *p, const fb_cosine *c, int pass) { return check_window(p, c, pass == 1) == FB_OK ? 1 : 0; }
+int fb_window_ready(const fb_params *p, const fb_cosine *c, int pass) {
+    const fb::KeptError kept; // (a "no" is an answer, nothing has failed)
+    return check_window(p, c, pass == 1) == FB_OK ? 1 : 0;
+}
 
 size_t fb_window_workspace_bytes(const fb_params *p) {
     if (!p || p->B <= 0 || p->H <= 0) return 0;

@@ -5,13 +5,14 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <cstring>
 
 #include "fb_checks.h"
 #include "flashbias.h"
 
 namespace {
 
-thread_local char g_err[256] = "";
+thread_local char g_err[sizeof(fb::KeptError::text)] = "";
 
 int fail(int code, const char *fmt, const char *what = "") {
     std::snprintf(g_err, sizeof(g_err), fmt, what);
@@ -50,6 +51,9 @@ int api_fail(int code, const char *fmt, ...) {
 }
 
 void api_clear_error() { g_err[0] = 0; }
+
+KeptError::KeptError() { std::memcpy(text, g_err, sizeof(text)); }
+KeptError::~KeptError() { std::memcpy(g_err, text, sizeof(text)); }
 
 } // namespace fb
 

@@ -17,6 +17,13 @@ namespace fb {
 int api_fail(int code, const char *fmt, ...);
 void api_clear_error();
 
+// For an entry point that answers a question by the checks of another: the calling thread's last error stays what it was.
+struct KeptError {
+    char text[256];
+    KeptError();
+    ~KeptError();
+};
+
 // Sizes a caller's block may have, and its mask_batches (version 3's block has none; what follows it is the caller's).
 inline bool known_size(const fb_params *p) { return p->size == sizeof(fb_params) || p->size == FB_PARAMS_SIZE_3; }
 inline int mask_batches(const fb_params *p) { return p->size > FB_PARAMS_SIZE_3 ? p->mask_batches : 0; }

@@ -259,7 +259,8 @@ int fb_cosine_bwd(const fb_cosine *p, void *stream);
  * c->partial of fb_window_workspace_bytes() bytes; p->delta is not used, and neither are the other pointers of `c`.  The bits are those of fb_cosine_fwd, fb_fwd, the ring
  * backward and fb_cosine_bwd one after the other (dlogit_scale: another order of the same sum).
  * fb_window_ready (pass: 0 = forward, 1 = backward): 1 for the calls these take: head dim 32, at most 256 positions, rank up to
- * 16, one 16-bit type, fp32 = 0, aligned tensors, no mask or a matrix mask of 16-byte chunks; the others return FB_ERR_SHAPE. */
+ * 16, one 16-bit type, fp32 = 0, aligned tensors, no mask or a matrix mask of 16-byte chunks; the others return FB_ERR_SHAPE.
+ * It leaves fb_last_error as it was. */
 int fb_window_ready(const fb_params *p, const fb_cosine *c, int pass);
 size_t fb_window_workspace_bytes(const fb_params *p);
 int fb_window_fwd(const fb_params *p, const fb_cosine *c, void *stream);

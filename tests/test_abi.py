@@ -9,6 +9,7 @@ import pytest
 import torch
 
 from flashbias_amd import _lib, flash_bias_func
+from test_gpu_modules import FbCosine
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -226,6 +227,44 @@ def test_resize_ranks_rejects(args, code):
     other = (0x3000, 0x4000, 10)
     assert lib.fb_resize_ranks(*args[:3], *other, *args[3:], None) == code
     assert lib.fb_resize_ranks(*other, *args[:3], *args[3:], None) == code
+
+
+def _window_block(pass_):
+    """A window block that fb_window_ready takes: q, k, v (and their gradients) are the parts of one packed projection."""
+    p = _good(pass_)
+    p.Lq = p.Lk = 64
+    p.scale = 1.0
+    part = lambda i: _lib.FbTensor(0x10000 + 2 * 128 * i, 64 * 384, 32, 384)
+    p.q, p.k, p.v = part(0), part(1), part(2)
+    p.q_bias = p.k_bias = _lib.FbTensor(0x10000, 0, 8, 32)
+    p.o = _lib.FbTensor(0x10000, 64 * 128, 32, 128)
+    if pass_:
+        p.dout, p.dq, p.dk, p.dv = p.o, part(0), part(1), part(2)
+        p.dq_bias = p.dk_bias = _lib.FbTensor()
+    c = FbCosine()
+    c.size = ctypes.sizeof(FbCosine)
+    c.dtype = c.in_dtype = c.scale_dtype = p.dtype
+    c.H, c.d, c.tokens, c.qkv, c.logit_scale = p.H, p.d, p.B * 64, 0x10000, 0x10000
+    return p, c
+
+
+@pytest.mark.parametrize("pass_", [0, 1])
+def test_window_ready_is_a_question(pass_):
+    """A "no" is no failure: the last error of the thread is that of the call before."""
+    lib = _lib.load()
+    ready = lambda p, c: lib.fb_window_ready(ctypes.byref(p), ctypes.byref(c), pass_)
+    p, c = _window_block(pass_)
+    assert lib.fb_check(_good(0), 0) == 0
+    assert ready(p, c) == 1 and lib.fb_last_error() == b""
+    for change in (lambda p, c: setattr(p, "d", 64), lambda p, c: setattr(p, "size", 8), lambda p, c: setattr(c, "fp32", 1)):
+        p, c = _window_block(pass_)
+        change(p, c)
+        assert ready(p, c) == 0 and lib.fb_last_error() == b""
+    assert lib.fb_window_ready(None, None, pass_) == 0 and lib.fb_last_error() == b""
+    assert lib.fb_check(None, 0) == -1  # a failure stays one
+    text = lib.fb_last_error()
+    assert text and ready(*_window_block(pass_)) == 1 and lib.fb_last_error() == text
+    assert lib.fb_window_fwd(ctypes.byref(p), ctypes.byref(c), None) == -2 and b"fb_window" in lib.fb_last_error()  # (the call itself does fail)
 
 
 def test_null_params():
