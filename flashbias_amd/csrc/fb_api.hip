@@ -291,10 +291,13 @@ int fb_alibi_factors(void *q_bias, void *k_bias, int dtype, int Lq, int Lk, int 
                     "fb_alibi_factors");
 }
 
+// Sizes a caller's block may have (the shorter one: before there was `fp32`).
+static bool known_size(const fb_cosine *p) { return p->size == sizeof(fb_cosine) || p->size == offsetof(fb_cosine, fp32); }
+
 static int check_cosine(const fb_cosine *p, bool backward) {
     fb::api_clear_error();
     if (!p) return fb::api_fail(FB_ERR_NULL, "fb_cosine: null pointer");
-    if (p->size != sizeof(fb_cosine) && p->size != offsetof(fb_cosine, fp32))
+    if (!known_size(p))
         return fb::api_fail(FB_ERR_ABI, "fb_cosine.size does not match this library");
     if (p->dtype != FB_F16 && p->dtype != FB_BF16) return fb::api_fail(FB_ERR_DTYPE, "only fp16 and bf16 are supported");
     if (p->in_dtype < FB_F16 || p->in_dtype > FB_F32 || p->scale_dtype < FB_F16 || p->scale_dtype > FB_F32)
@@ -337,7 +340,7 @@ int fb_cosine_bwd(const fb_cosine *p, void *stream) {
 
 // A cosine block's attention with the normalisation inside: q, k, v (and dq, dk, dv) of p are the parts of the projection c.qkv.
 static bool window_block(const fb_params *p, const fb_cosine *c, bool backward) {
-    return p->scale == 1.f && c->size >= offsetof(fb_cosine, fp32) && c->dtype == p->dtype && c->in_dtype == p->dtype && !cosine_fp32(c) &&
+    return p->scale == 1.f && c->dtype == p->dtype && c->in_dtype == p->dtype && !cosine_fp32(c) &&
            c->scale_dtype >= FB_F16 && c->scale_dtype <= FB_F32 && c->logit_scale && c->H == p->H && c->d == p->d &&
            (backward ? fb::ring_shape(bwd_args(p)) && p->mask_type != FB_MASK_VECTOR : fb::window_shape(fwd_args(p)));
 }
@@ -355,6 +358,7 @@ static int check_window(const fb_params *p, const fb_cosine *c, bool backward) {
         if (rc) return rc;
     }
     if (!c) return fb::api_fail(FB_ERR_NULL, "fb_window: null pointer");
+    if (!known_size(c)) return fb::api_fail(FB_ERR_ABI, "fb_cosine.size does not match this library");
     if (!window_block(p, c, backward)) return fb::api_fail(FB_ERR_SHAPE, "fb_window: not a block that fb_window_ready takes");
     return FB_OK;
 }

@@ -267,6 +267,19 @@ def test_window_ready_is_a_question(pass_):
     assert lib.fb_window_fwd(ctypes.byref(p), ctypes.byref(c), None) == -2 and b"fb_window" in lib.fb_last_error()  # (the call itself does fail)
 
 
+@pytest.mark.parametrize("pass_", [0, 1])
+def test_window_block_of_another_version_is_refused(pass_):
+    lib = _lib.load()
+    for size, known in ((ctypes.sizeof(FbCosine), True), (FbCosine.fp32.offset, True), (FbCosine.fp32.offset - 8, False),
+                        (ctypes.sizeof(FbCosine) - 4, False), (ctypes.sizeof(FbCosine) + 8, False)):
+        p, c = _window_block(pass_)
+        c.size = size
+        assert lib.fb_window_ready(ctypes.byref(p), ctypes.byref(c), pass_) == known
+        if not known:
+            call = lib.fb_window_bwd if pass_ else lib.fb_window_fwd
+            assert call(ctypes.byref(p), ctypes.byref(c), None) == -7 and b"size" in lib.fb_last_error()
+
+
 def test_null_params():
     lib = _lib.load()
     assert lib.fb_check(None, 0) == -1
