@@ -13,7 +13,7 @@
 //     later go out beside the products of the fourth slice and of the next step's first.
 //   * Workgroups stay for as many tiles as they get, and the copies run on into the next tile.  What a tile's end still has to copy
 //     goes out ahead of its stores, so that the next waits, which count in order, can leave the stores in flight.
-//   * Results that no cache will hold until they are read go past them (490 MB and more: 426 -> 390 us at that size).
+//   * Results that no cache will hold until they are read go past them (kPastCaches: 805 MB 426 -> 390 us).
 // Vendor library / this, us: 262144 tokens, 512 to 1536 channels 482 / 393, 512 to 512 with bias 162 / 143, 256 to 768 161 / 111;
 // 147456 tokens, 512 to 1536 366 / 215, 256 to 768 103 / 67; 36864 tokens, 256 to 768 35 / 24; 16384, 256 to 768 19.9 / 13.8.
 // Not kept: a line of x touched two steps ahead of its copy (431 -> 443, the touches wait in the same queue), workgroups that
@@ -297,6 +297,13 @@ static hipError_t launch_linear_w(const LinearArgs &a, hipStream_t stream) {
     return a.b ? launch_linear_t<T, 4, 4, 2, true>(a, stream) : launch_linear_t<T, 4, 4, 2, false>(a, stream);
 }
 
+// Bytes of results from which they are stored past the caches.  The kernel alone is ahead from 40 MB on, but the next one reads them, and up to
+// about 200 MB from the memory side's 256 MB.  This and its reader, through the caches / past them, us: the window forward (256 tokens) on 70 MB of
+// 256 to 768 channels 67.1 / 70.6, 100 MB 84.5 / 91.7, 130 MB 113.1 / 115.9, 180 MB 151.4 / 156.4, 250 MB 215.0 / 208.2, 400 MB 332.7 / 325.6, 800 MB of 512
+// to 1536 805 / 786; windows of 64, 128 to 384, 180 MB 128.4 / 133.6, 250 MB 181.4 / 176.4; an addition on 100 MB of 512 to 512 102.3 / 105.5, 180 MB
+// 195.2 / 194.0, 250 MB 267.3 / 261.7.
+constexpr int64_t kPastCaches = (int64_t)200 << 20;
+
 hipError_t launch_linear(const void *x, int64_t ldx, const void *w, const void *b, void *y, int64_t tokens, int n, int k, bool bf16, hipStream_t stream) {
     LinearArgs a = {};
     a.x = static_cast<const uint16_t *>(x);
@@ -307,7 +314,7 @@ hipError_t launch_linear(const void *x, int64_t ldx, const void *w, const void *
     a.n = n;
     a.tokens = (int)tokens;
     a.k = k;
-    a.stream = tokens * n * 2 >= (int64_t)64 << 20;
+    a.stream = tokens * n * 2 >= kPastCaches;
     return bf16 ? launch_linear_w<BF16>(a, stream) : launch_linear_w<F16>(a, stream);
 }
 

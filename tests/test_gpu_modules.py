@@ -472,10 +472,10 @@ def test_projections(gpu_device, dtype, tokens, n, k):
 
 
 # one step of 64 columns, fewer steps than a tile has stages, and many; tiles of 128 and of 256 channels, one and several a workgroup, results
-# through the caches and past them (64 MB and more), ragged edges along tokens and channels, a bias on 4 bytes, rows inside a wider tensor
+# through the caches and past them (200 MiB and more), ragged edges along tokens and channels, a bias on 4 bytes, rows inside a wider tensor
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("tokens,n,k", [(1, 8, 64), (257, 136, 128), (300, 1000, 1600), (9001, 1000, 192), (33000, 512, 64), (70144, 512, 128),
-                                        (140001, 264, 64), (20001, 776, 512)])
+                                        (140001, 264, 64), (20001, 776, 512), (202001, 520, 64), (137000, 776, 128)])
 def test_linear(gpu_device, dtype, tokens, n, k):
     lib = _lib.load()
     g = torch.Generator(device=gpu_device).manual_seed(tokens)
