@@ -376,6 +376,42 @@ def test_window_block_takes_what_the_tensor_operations_take(gpu_device, monkeypa
         assert (a - b).norm() <= (3e-2 if name == "scale" else 2.0 ** -7) * b.norm(), name
 
 
+def _requested(fn):
+    """fn(), and the bytes that it asked the allocator for."""
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_stats()["requested_bytes.all.allocated"]
+    out = fn()
+    return out, torch.cuda.memory_stats()["requested_bytes.all.allocated"] - before
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("windows,window,heads,types", [(264, 16, 4, 0), (264, 12, 4, 4), (8, 16, 4, 2), (6, 8, 2, 0)])
+def test_window_block_with_a_gradient_in_unaligned_rows(gpu_device, dtype, windows, window, heads, types):
+    """The forward normalised q and k inside its kernel and kept neither, and the backward kernel that would do so again does not read these
+    rows: the normalised rows are formed then, and the gradients are those of the same gradient in aligned rows."""
+    torch.manual_seed(8)
+    n, dim = window * window, 32 * heads
+    mod = modules.WindowAttentionCore(dim, window, heads, rank=8, dtype=dtype).to(gpu_device, dtype)
+    qkv = torch.randn(windows, n, 3 * dim, device=gpu_device).to(dtype).requires_grad_(True)
+    mod.qkv, mod.proj = Given(qkv), torch.nn.Identity()
+    x = torch.zeros(windows, n, dim, device=gpu_device, dtype=dtype)
+    mask = (torch.rand(types, n, n, device=gpu_device) < 0.2).to(dtype) * -100.0 if types else None
+    dy = torch.zeros(windows, n, dim + 8, device=gpu_device, dtype=dtype)[..., 4:dim + 4].copy_(torch.randn(windows, n, dim, device=gpu_device))
+    assert dy.data_ptr() % 16
+    y, asked = _requested(lambda: mod(x, mask))
+    size = windows * n * dim * 2
+    assert asked == size + windows * heads * n * 4  # (o and lse alone)
+    gradients = lambda d: torch.autograd.grad(y, [qkv, mod.logit_scale], d, retain_graph=True)
+    gradients(dy)
+    want, few = _requested(lambda: gradients(dy.contiguous()))
+    got, more = _requested(lambda: gradients(dy))
+    assert more >= few - size + 2 * size  # (less the copy of dy, and q and k)
+    for name, g, w in zip(("dqkv", "scale"), got, want):
+        # other kernels with other orders of their sums, dq and dk rounded before the normalisation's part on both ways (the scale's
+        # gradient is a sum over all scores: as the module's other tests)
+        assert torch.isfinite(g).all() and (g.double() - w.double()).norm() <= (3e-2 if name == "scale" else 2.0 ** -7) * w.double().norm(), name
+
+
 @pytest.mark.parametrize("dtype,param", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32), (torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("window,heads,hd,windows,types", [(8, 2, 32, 6, 3), (7, 3, 128, 4, 0), (16, 8, 32, 64, 4), (12, 4, 32, 66, 6)])
 def test_window_block_against_float64(gpu_device, monkeypatch, dtype, param, window, heads, hd, windows, types):
