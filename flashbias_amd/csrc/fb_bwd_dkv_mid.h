@@ -1,6 +1,6 @@
 // dk, dv and dk_bias for head dims 17 ... 64 (aligned tensors, rank up to 32, no mask or a vector mask).  Included by
 // fb_bwd_dkv.hip after the pair kernel; the arithmetic is that of the general kernel, operation by operation (lane = key,
-// register = query; the same bits).
+// register = query; the same bits where one group of waves walks all queries).
 //
 // Head dims above 32.  A 32 x 32 block takes 19 or 21 products (650 cycles), about 100 vector instructions (450) and 37 LDS reads.  Left to itself the
 // compiler asks for each fragment where it is used and waits for it, sixteen times a block: 4000 cycles for a wave that has a SIMD

@@ -1,6 +1,6 @@
 // dq and dq_bias for head dims 17 ... 64 (aligned tensors, rank up to 32, no mask): one query block a wave.  Included by
 // fb_bwd_dq.hip after the general kernel; the arithmetic is that of the general kernel, operation by operation (lane = query,
-// register = key; the same bits).
+// register = key; the same bits where one group of waves walks all keys).
 //
 // Head dims above 32: as in the dk/dv kernel for them (fb_bwd_dkv_mid.h) the reads of a phase are requested beside the products of
 // the phase before; left to itself the compiler waits for each where it is used.  Head dim 32: tiles of dense 64-byte rows take half

@@ -137,15 +137,16 @@ inline bool mixed_backward(const BwdArgs &a0) {
 template <class T>
 inline bool mixed_general_backward(const BwdArgs &a0);
 
-// What the two one-launch backwards below share: whole sequences of at most 256 positions, head dim 32, rank a multiple of 8 up
-// to 32, aligned tensors, no causal mask, no fp32 mask (the mask is read element-wise, any strides), and at least one workgroup
-// per compute unit.  Such sequences are bound by memory traffic, and the two-kernel backward reads q, k, v, o and dO twice.
+// What the two one-launch backwards below take: whole sequences of at most 256 positions, head dim 32, rank a multiple of 8 up
+// to 32, aligned tensors, no causal mask, no fp32 mask (the mask is read element-wise, any strides).  Such sequences are bound
+// by memory traffic, and the two-kernel backward reads q, k, v, o and dO twice.
 inline bool short_shape(const BwdArgs &a) {
     const int64_t lim = (int64_t)1 << 22; // (32-bit byte offsets of 256 tile rows)
     return (a.mask.type == 0 || (!a.mask.is_f32 && a.mask.sm < lim)) && !a.causal && a.d == 32 && a.r % 8 == 0 && a.r <= 32 && a.Lq <= 256 && a.Lk <= 256 &&
            a.q.vec_ok && a.k.vec_ok && a.v.vec_ok && a.o.vec_ok && a.dout.vec_ok && (a.r == 0 || (a.qb.vec_ok && a.kb.vec_ok)) &&
            a.q.ss < lim && a.k.ss < lim && a.dout.ss < lim && (a.r == 0 || (a.qb.ss < lim && a.kb.ss < lim));
 }
+// ... and where fb_bwd uses them: at least one workgroup per compute unit.
 inline bool short_sequences(const BwdArgs &a) {
     const int group = a.group > 1 ? a.group : 1;
     return short_shape(a) && (int64_t)((a.B + group - 1) / group) * a.H >= num_cus();

@@ -6,6 +6,11 @@
 // windows of 256 tokens, 16 heads, bf16, bound by memory.  In the window forward it is 41 us of vector work (498 -> 539), in the ring
 // backward 133 (867 -> 1000): training step of the block 3641 -> 3205 us; windows of 64 tokens 918 -> 880, of 144 (256 x 16) 647 -> 593;
 // small grids, which lose two launches, 64 x 4 windows of 144 98 -> 81, 64 x 8 of 256 196 -> 153.
+// There is no smallest grid: the ring kernel takes a (window, head) pair a workgroup, where the general kernels take two or four for windows of
+// more than 128 tokens, but that is less than the passes and launches around them.  Normalisation, forward, backward and its normalisation,
+// separate / inside, us, rank 16: 16 windows x 2 heads of 64 tokens 21.0 / 17.7, of 144 27.0 / 25.9, of 256 31.4 / 28.5; 16 x 4 21.5 / 17.9, 29.4 / 26.3,
+// 34.2 / 29.4; 16 x 8 23.2 / 18.4, 35.1 / 27.2, 39.4 / 31.9; 32 x 4 24.0 / 18.3, 36.9 / 26.8, 43.0 / 31.3; with masks 16 x 4 31.1 / 19.8, 50.2 / 30.2, 54.2 / 34.8.
+// Behind only at 4 x 2 without a mask, 25.1 / 25.8 and 26.4 / 28.1 (64 tokens 19.8 / 17.5), in graphs; an eager step of that size is 190 to 260 us of host.
 #pragma once
 #include "fb_device.h"
 

@@ -256,8 +256,10 @@ int fb_cosine_bwd(const fb_cosine *p, void *stream);
 /* The attention of such a block with the normalisation inside the attention kernels: q, k, v (and dq, dk, dv) of `p` are the
  * parts of the packed projection c->qkv (c->dqkv) itself, o and lse those of the attention on the normalised rows, scale 1, no
  * factor gradients.  The backward reads the projection again, writes the projection's gradient and dlogit_scale, and takes
- * c->partial of fb_window_workspace_bytes() bytes; p->delta is not used, and neither are the other pointers of `c`.  The bits are those of fb_cosine_fwd, fb_fwd, the ring
- * backward and fb_cosine_bwd one after the other (dlogit_scale: another order of the same sum).
+ * c->partial of fb_window_workspace_bytes() bytes; p->delta is not used, and neither are the other pointers of `c`.  The bits are those of
+ * fb_cosine_fwd, the forward and the backward for windows (which fb_fwd and fb_bwd use on grids that fill the chip) and fb_cosine_bwd one after the other, but for
+ * dlogit_scale (another order of the same sum) and, in fp16, for some of the gradients of q and k: fb_cosine_bwd adds up products in pairs there, whose
+ * fp32 roundings differ (about 2^-20 of a row's largest value before the result is rounded, one element in 2^12).
  * fb_window_ready (pass: 0 = forward, 1 = backward): 1 for the calls these take: head dim 32, at most 256 positions, rank up to
  * 16, one 16-bit type, fp32 = 0, aligned tensors, no mask or a matrix mask of 16-byte chunks; the others return FB_ERR_SHAPE.
  * It leaves fb_last_error as it was. */
